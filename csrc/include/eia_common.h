@@ -72,3 +72,14 @@ template <> EIA_DEV float ld_f32<float>(const float* p, long i) { return p[i]; }
 template <typename T> EIA_DEV void st_f32(T* p, long i, float v);
 template <> EIA_DEV void st_f32<bf16_t>(bf16_t* p, long i, float v) { p[i] = (bf16_t)v; }
 template <> EIA_DEV void st_f32<float>(float* p, long i, float v) { p[i] = v; }
+
+// Four steps of an fp32 matrix-core product (16x16x4): lane l of an A operand holds row l % 16 and
+// contraction indices 4 (l / 16) + i, of a B operand column l % 16 and the same indices; the
+// accumulator holds rows 4 (l / 16) + i of column l % 16, so that an accumulator is, register by
+// register, the B operand of a product over its rows (and the A operand of one over its columns'
+// transpose).
+EIA_DEV f32x4 mfma_f32_k16(f32x4 a, f32x4 b, f32x4 c) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[i], c, 0, 0, 0);
+  return c;
+}

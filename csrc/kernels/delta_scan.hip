@@ -228,11 +228,7 @@ struct DeltaChunkArgs {
   float* cA; float* wsG;                    // [rows, H] running sums, [nchunk, H] their last
 };
 
-EIA_DEV f32x4 mm(f32x4 a, f32x4 b, f32x4 c) {          // four steps of a 16x16 product
-#pragma unroll
-  for (int i = 0; i < 4; ++i) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[i], c, 0, 0, 0);
-  return c;
-}
+EIA_DEV f32x4 mm(f32x4 a, f32x4 b, f32x4 c) { return mfma_f32_k16(a, b, c); }
 
 __global__ void __launch_bounds__(256)
 delta_chunk_solve_kernel(DeltaArgs a, DeltaChunkArgs c) {

@@ -72,6 +72,7 @@ struct WkvArgs {
   const int* slots; const int* cu; const int* positions; const int* seq_lens;
   void* y; long ldy;                        // [rows, H*D]
   float eps; int H, D;
+  int split;                                // rows from which a sequence takes the chunk-parallel form (0: never)
 };
 
 // One workgroup per (sequence, head), 4 x max(64, DMAX) threads: thread (q, j) owns rows
@@ -96,7 +97,7 @@ wkv_scan_kernel(WkvArgs a) {
   const int slot = a.slots[s];
   if (slot < 0 || (a.seq_lens && a.seq_lens[s] <= 0)) return;
   const int lo = a.cu ? a.cu[s] : s, hi = a.cu ? a.cu[s + 1] : s + 1;
-  if (hi <= lo) return;
+  if (hi <= lo || (a.split && hi - lo >= a.split)) return;
   const bool fresh = a.positions[lo] == 0;
   const bool live = j < D, mine = j < DMAX;
   float* Sg = a.S + ((long)slot * a.H + h) * D * D;
@@ -187,17 +188,18 @@ wkv_scan_kernel(WkvArgs a) {
   }
 }
 
+// split > 0: sequences of that many rows or more are left out (eia_wkv_scan_chunked takes them).
 EIA_API int eia_wkv_scan(const void* r, const void* k, const void* v, const void* g, long ld,
                          const float* dec, long ld_dec, const void* w0, const void* u,
                          const void* norm_w, float* S, float* prev, const float* x, int W,
                          const int* slots, const int* cu, const int* positions,
                          const int* seq_lens, void* y, long ldy, float eps, int nseq, int H, int D,
-                         int is_bf16, hipStream_t st) {
-  if (nseq < 0 || H < 1 || D < 1 || W < 1) return EIA_BAD_SHAPE;
+                         int split, int is_bf16, hipStream_t st) {
+  if (nseq < 0 || H < 1 || D < 1 || W < 1 || split < 0) return EIA_BAD_SHAPE;
   if (D > 256) return EIA_UNSUPPORTED;
   if (nseq == 0) return EIA_OK;
   WkvArgs a{r, k, v, g, ld, dec, ld_dec, w0, u, norm_w, S, prev, x, W, slots, cu, positions,
-            seq_lens, y, ldy, eps, H, D};
+            seq_lens, y, ldy, eps, H, D, split};
   dim3 grid(nseq, H);
 #define WKV_LAUNCH(TT, DM)                                                                 \
   hipLaunchKernelGGL((wkv_scan_kernel<TT, DM>), grid, dim3(4 * (DM < 64 ? 64 : DM)), 0, st, a)
@@ -213,5 +215,422 @@ EIA_API int eia_wkv_scan(const void* r, const void* k, const void* v, const void
     else WKV_LAUNCH(float, 256);
   }
 #undef WKV_LAUNCH
+  EIA_LAUNCH_CHECK();
+}
+
+// ---------------------------------------------------------------------------------------------
+// Chunk-parallel form for prompt portions (D <= 64).  The kernel above walks a sequence with one
+// workgroup per head (0.5 us a token); here a sequence's rows are cut into chunks of WC tokens and,
+// with l_t = log2 w_t = -exp(dec_t + w0) / ln 2 per channel, S the state before a chunk and sums over the
+// chunk's tokens,
+//
+//   U   = sum_s 2^(sum_(s<x) l_x) k_s v_s^T                            (1) per chunk, in parallel
+//   S' = 2^(sum_x l_x) S + U                                           (2) a sequence's chunks in order
+//   o_t = (r_t 2^(sum_(x<t) l_x)) S + sum_(s<t) P_ts v_s + (r_t . u . k_t) v_t
+//   P_ts = sum_channels r_t k_s 2^(sum_(s<x<t) l_x)                    (3) per chunk, in parallel
+//
+// All products are fp32 matrix-core products.  Exponents are formed as sums of the l_x that they
+// cover, never as differences of long running sums, so they are <= 0 and keep their precision; a
+// pair of tokens meets through the edges of the 8-token blocks between them,
+//   P_ts = (r_t 2^(block start .. t)) . (whole blocks between) . (k_s 2^(s .. block end)),
+// and only pairs inside one 8-token block take the difference of a running sum over that block
+// (there a token's l is cut at -40: a weight below 1e-12).
+//
+// Chunks are numbered without a list from the host: sequence s owns the numbers from
+// cu[s] / WC + s on, at least as many as it has chunks; numbers past its last chunk do nothing.
+//
+// Bound by instruction issue (exponentials, conversions, fp32 products; 31 us of vector and 15 us of
+// matrix issue in (3)), not by memory: one 4096-token prompt, 32 heads of 64, bf16 takes 26 + 14 +
+// 71 us on an MI355X, 2091 us token by token.  (3) took 125 us with 2-byte loads and a padded LDS
+// tile for each of r, k, v and the running sums (two workgroups per CU instead of three).
+constexpr int WC = 64;                      // tokens per chunk
+constexpr int WD = 64;                      // widest head
+constexpr int WKV_AHEAD = 8;                // chunks whose contributions are in flight in (2)
+
+struct WkvChunkArgs {
+  float* U;                                 // [numbers, H, WD, WD]: contribution, then state before
+  float* L;                                 // [numbers, H, WD]: sums of l
+  int nseq;
+};
+
+// The chunk of number x; false where there is none or the sequence is skipped.
+EIA_DEV bool wkv_chunk(const WkvArgs& a, int nseq, int x, int& s, int& row0, int& n) {
+  int lo = 0, hi = nseq - 1;                // largest s with cu[s] / WC + s <= x
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (a.cu[mid] / WC + mid <= x) lo = mid; else hi = mid - 1;
+  }
+  s = lo;
+  if (x < a.cu[s] / WC + s) return false;   // (rows before the first sequence)
+  row0 = a.cu[s] + (x - a.cu[s] / WC - s) * WC;
+  n = min(WC, a.cu[s + 1] - row0);
+  return n > 0 && a.cu[s + 1] - a.cu[s] >= a.split && a.slots[s] >= 0 && (!a.seq_lens || a.seq_lens[s] > 0);
+}
+
+// Place of (token, channel) in an LDS tile [WC][WD]: the 16-byte units of a row are turned by the
+// token, so that sixteen tokens' units of one channel group lie on different banks.
+EIA_DEV int wkv_at(int t, int i) { return t * WD + (i ^ ((t & 15) << 2)); }
+EIA_DEV f32x4 wkv_get(const float* tile, int t, int i) {         // channels i .. i + 3, i % 4 == 0
+  return *reinterpret_cast<const f32x4*>(tile + wkv_at(t, i));
+}
+
+// A chunk's [WC][WD] tile of r, k or v on its way to LDS, zero past the chunk and past D: requested
+// by load, stored as fp32 by store.  VEC: 16-byte loads (D == WD, rows on 16-byte addresses).
+template <typename T, bool VEC>
+struct WkvTile {
+  static constexpr int E = VEC ? 16 / sizeof(T) : 1, N = WC * WD / (256 * E);
+  T v[N][E];
+  EIA_DEV void load(const void* src, long ld, long hc, int row0, int n, int D) {
+#pragma unroll
+    for (int x = 0; x < N; ++x) {
+      const int u = threadIdx.x + 256 * x, t = u / (WD / E), i = E * (u % (WD / E));
+      const T* p = static_cast<const T*>(src) + (row0 + min(t, n - 1)) * ld + hc + (VEC ? i : min(i, D - 1));
+      if constexpr (VEC) *reinterpret_cast<f32x4*>(v[x]) = *reinterpret_cast<const f32x4*>(p);
+      else v[x][0] = *p;
+    }
+  }
+  EIA_DEV void store(float* tile, int n, int D) const {
+#pragma unroll
+    for (int x = 0; x < N; ++x) {
+      const int u = threadIdx.x + 256 * x, t = u / (WD / E), i = E * (u % (WD / E));
+      const bool ok = t < n && (VEC || i < D);
+      if constexpr (VEC) {
+#pragma unroll
+        for (int e = 0; e < E; e += 4)
+          *reinterpret_cast<f32x4*>(tile + wkv_at(t, i + e)) =
+              ok ? f32x4{(float)v[x][e], (float)v[x][e + 1], (float)v[x][e + 2], (float)v[x][e + 3]}
+                 : f32x4{0.f, 0.f, 0.f, 0.f};
+      } else {
+        tile[wkv_at(t, i)] = ok ? (float)v[x][0] : 0.f;
+      }
+    }
+  }
+};
+
+// Base-2 log decays of channel i, tokens t0 .. t0 + 15 (0 past the chunk and past D): a weight then
+// costs one v_exp_f32.
+template <typename T>
+EIA_DEV void wkv_decays(const WkvArgs& a, long hc, int row0, int n, int t0, int i, float (&l)[16]) {
+  const int ic = min(i, a.D - 1);
+  const float w0 = ld_f32<T>(static_cast<const T*>(a.w0), hc + ic);
+#pragma unroll
+  for (int t = 0; t < 16; ++t) l[t] = a.dec[(long)(row0 + min(t0 + t, n - 1)) * a.ld_dec + hc + ic];
+#pragma unroll
+  for (int t = 0; t < 16; ++t)
+    l[t] = (i < a.D && t0 + t < n) ? -1.4426950408889634f * expf(l[t] + w0) : 0.f;
+}
+
+// (1) Wave w forms rows 16 w .. of U.  A lane of a product over tokens holds value columns
+// 4 (lane % 16) + j in its j-th tile, here and in (3): U, S and v move in 16-byte units.
+template <typename T, bool VEC>
+__global__ void __launch_bounds__(256)
+wkv_chunk_state_kernel(WkvArgs a, WkvChunkArgs c) {
+  __shared__ __align__(16) float sk[WC * WD], sv[WC * WD];
+  __shared__ float stot[4][WD];
+  int s, row0, n;
+  if (!wkv_chunk(a, c.nseq, blockIdx.x, s, row0, n)) return;
+  const int h = blockIdx.y, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int l16 = lane & 15, g4 = lane >> 4;
+  const long hc = (long)h * a.D;
+  WkvTile<T, VEC> tk, tv;
+  tk.load(a.k, a.ld, hc, row0, n, a.D);
+  tv.load(a.v, a.ld, hc, row0, n, a.D);
+  float l[16];
+  wkv_decays<T>(a, hc, row0, n, 16 * w, lane, l);
+  float tot = 0.f;
+#pragma unroll
+  for (int t = 0; t < 16; ++t) tot += l[t];
+  stot[w][lane] = tot;
+  tk.store(sk, n, a.D);
+  tv.store(sv, n, a.D);
+  __syncthreads();
+  float after = 0.f;                                   // sum of l from the next token on
+  for (int b = 3; b > w; --b) after += stot[b][lane];
+#pragma unroll
+  for (int t = 15; t >= 0; --t) {
+    sk[wkv_at(16 * w + t, lane)] *= __builtin_amdgcn_exp2f(after);
+    after += l[t];
+  }
+  const long at = (long)blockIdx.x * a.H + h;
+  if (w == 0) c.L[at * WD + lane] = after;
+  __syncthreads();
+  f32x4 acc[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    if (16 * b >= n) break;
+    f32x4 ka, vb[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int t = 16 * b + 4 * g4 + e;
+      ka[e] = sk[wkv_at(t, 16 * w + l16)];
+      const f32x4 x = wkv_get(sv, t, 4 * l16);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) vb[j][e] = x[j];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[j] = mfma_f32_k16(ka, vb[j], acc[j]);
+  }
+  float* U = c.U + at * WD * WD + (long)(16 * w + 4 * g4) * WD + 4 * l16;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    *reinterpret_cast<f32x4*>(U + i * WD) = f32x4{acc[0][i], acc[1][i], acc[2][i], acc[3][i]};
+}
+
+// (2) Four columns of a state row per thread: U of a chunk turns into the state before it; the slot
+// receives the state after the last one.  A group's contributions are requested while the previous
+// group is summed.
+__global__ void __launch_bounds__(256)
+wkv_chunk_scan_kernel(WkvArgs a, WkvChunkArgs c) {
+  const int s = blockIdx.x, h = blockIdx.y;
+  const int slot = a.slots[s], lo = a.cu[s], hi = a.cu[s + 1];
+  if (slot < 0 || hi - lo < a.split || (a.seq_lens && a.seq_lens[s] <= 0)) return;
+  const int e = 4 * (blockIdx.z * 256 + threadIdx.x), i = e / WD, j = e % WD, D = a.D;
+  const long x0 = lo / WC + s;
+  const int nc = (hi - lo + WC - 1) / WC;
+  float* Sg = a.S + ((long)slot * a.H + h) * D * D + (long)i * D + j;
+  f32x4 S = {0.f, 0.f, 0.f, 0.f};
+  if (a.positions[lo] != 0 && i < D) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (j + k < D) S[k] = Sg[k];
+  }
+  float* U = c.U + (x0 * a.H + h) * WD * WD + e;
+  const float* L = c.L + (x0 * a.H + h) * WD + i;
+  const long us = (long)a.H * WD * WD, ls = (long)a.H * WD;
+  f32x4 u[WKV_AHEAD];
+  float d[WKV_AHEAD];
+  auto fetch = [&](int b, f32x4 (&u)[WKV_AHEAD], float (&d)[WKV_AHEAD]) {
+#pragma unroll
+    for (int k = 0; k < WKV_AHEAD; ++k) {
+      const int x = min(b + k, nc - 1);
+      u[k] = *reinterpret_cast<const f32x4*>(U + x * us);
+      d[k] = L[x * ls];
+    }
+  };
+  fetch(0, u, d);
+  for (int b = 0; b < nc; b += WKV_AHEAD) {
+    f32x4 un[WKV_AHEAD];
+    float dn[WKV_AHEAD];
+    fetch(b + WKV_AHEAD, un, dn);
+#pragma unroll
+    for (int k = 0; k < WKV_AHEAD; ++k) {
+      if (b + k < nc) {
+        *reinterpret_cast<f32x4*>(U + (b + k) * us) = S;
+        S = S * __builtin_amdgcn_exp2f(d[k]) + u[k];
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < WKV_AHEAD; ++k) {
+      u[k] = un[k];
+      d[k] = dn[k];
+    }
+  }
+  if (i < D) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (j + k < D) Sg[k] = S[k];
+  }
+  if (h == 0) {                                        // the last token's layer input
+    const float* last = a.x + (long)(hi - 1) * a.W;
+    float* p = a.prev + (long)slot * a.W;
+    for (int k = e / 4; k < a.W; k += WD * WD / 4) p[k] = last[k];
+  }
+}
+
+// (3) Wave w forms the outputs of tokens 16 w .. (later tokens meet more keys: which wave takes them
+// rotates with the chunk, so that no SIMD gets all of them).  50 KiB of LDS: three workgroups per CU.
+template <typename T, bool VEC>
+__global__ void __launch_bounds__(256, 3)
+wkv_chunk_out_kernel(WkvArgs a, WkvChunkArgs c) {
+  __shared__ __align__(16) float sr[WC * WD], sk[WC * WD], sAv[WC * WD];
+  __shared__ __align__(16) float se[8][WD], su[WD];    // decays over whole 8-token blocks; u
+  int s, row0, n;
+  if (!wkv_chunk(a, c.nseq, blockIdx.x, s, row0, n)) return;
+  const int h = blockIdx.y, lane = threadIdx.x & 63, w = ((threadIdx.x >> 6) + blockIdx.x) & 3;
+  const int D = a.D, l16 = lane & 15, g4 = lane >> 4, t0 = 16 * w;
+  const long hc = (long)h * D;
+  WkvTile<T, VEC> tr, tk, tv;
+  tr.load(a.r, a.ld, hc, row0, n, D);
+  tk.load(a.k, a.ld, hc, row0, n, D);
+  float l[16];
+  wkv_decays<T>(a, hc, row0, n, t0, lane, l);
+  tv.load(a.v, a.ld, hc, row0, n, D);
+  tr.store(sr, n, D);
+  tk.store(sk, n, D);
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    float A = 0.f, tot = 0.f;
+#pragma unroll
+    for (int t = 8 * b; t < 8 * b + 8; ++t) {
+      A += fmaxf(l[t], -40.f);
+      tot += l[t];
+      sAv[wkv_at(t0 + t, lane)] = A;
+    }
+    se[2 * w + b][lane] = __builtin_amdgcn_exp2f(tot);
+  }
+  if (w == 0) su[lane] = lane < D ? ld_f32<T>(static_cast<const T*>(a.u), hc + lane) : 0.f;
+  __syncthreads();
+  // weights inside the wave's two 8-token blocks: lane = pair s < t, then to the lane that holds
+  // them as an operand (query l16, keys 4 g4 + i)
+  f32x4 p = {0.f, 0.f, 0.f, 0.f};
+  if (t0 < n) {
+    float v = 0.f;
+    if (lane < 56) {
+      const int x = lane % 28;
+      int t = 1;
+      while (t * (t + 1) / 2 <= x) ++t;
+      const int q = t0 + 8 * (lane / 28), ks = x - t * (t - 1) / 2;
+#pragma unroll 4
+      for (int i = 0; i < WD; i += 4) {
+        const f32x4 y = wkv_get(sr, q + t, i) * wkv_get(sk, q + ks, i);
+        const f32x4 d = wkv_get(sAv, q + t - 1, i) - wkv_get(sAv, q + ks, i);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v += y[e] * __builtin_amdgcn_exp2f(d[e]);
+      }
+    }
+    float b = 0.f;                                     // r . u . k of token t0 + l16
+#pragma unroll
+    for (int i = 0; i < 16; i += 4) {
+      const int d = 16 * g4 + i;
+      const f32x4 x = wkv_get(sr, t0 + l16, d) * wkv_get(sk, t0 + l16, d) *
+                      *reinterpret_cast<const f32x4*>(&su[d]);
+      b += x[0] + x[1] + x[2] + x[3];
+    }
+    b += __shfl_xor(b, 16, 64);
+    b += __shfl_xor(b, 32, 64);
+    const int t8 = l16 & 7;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int ks = 4 * g4 + i;
+      const float x = __shfl(v, 28 * (l16 >> 3) + (t8 * (t8 - 1) >> 1) + (ks & 7), 64);
+      p[i] = ks == l16 ? b : (ks < l16 && ks >> 3 == l16 >> 3) ? x : 0.f;
+    }
+  }
+  __syncthreads();
+  // r_t <- r_t 2^(block start .. t), k_s <- k_s 2^(s .. block end), 8-token blocks; v moves in
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    float pre = 0.f, suf = 0.f;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      sr[wkv_at(t0 + 8 * b + t, lane)] *= __builtin_amdgcn_exp2f(pre);
+      pre += l[8 * b + t];
+      sk[wkv_at(t0 + 8 * b + 7 - t, lane)] *= __builtin_amdgcn_exp2f(suf);
+      suf += l[8 * b + 7 - t];
+    }
+  }
+  tv.store(sAv, n, D);
+  __syncthreads();
+  if (t0 >= n) return;
+  f32x4 rt[4], o[4], pq = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    const int i = 16 * b + 4 * g4;
+    rt[b] = wkv_get(sr, t0 + l16, i);
+    pq = mfma_f32_k16(wkv_get(sk, t0 + l16, i), rt[b], pq);
+    if (l16 >= 8) rt[b] *= *reinterpret_cast<const f32x4*>(&se[2 * w][i]);
+    o[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  // (weights are formed transposed, keys x queries: their registers are the A operand of P v)
+  if (l16 >= 8 && g4 < 2) p += pq;                     // second 8 queries, first 8 keys
+  for (int b = w;;) {
+    f32x4 vb[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const f32x4 x = wkv_get(sAv, 16 * b + 4 * g4 + e, 4 * l16);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) vb[j][e] = x[j];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[j] = mfma_f32_k16(p, vb[j], o[j]);
+    if (--b < 0) break;
+    p = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {                      // keys of block b; rt: from its end on
+      const int i = 16 * x + 4 * g4;
+      const f32x4 e1 = *reinterpret_cast<const f32x4*>(&se[2 * b + 1][i]);
+      f32x4 kk = wkv_get(sk, 16 * b + l16, i);
+      if (l16 < 8) kk *= e1;
+      p = mfma_f32_k16(kk, rt[x], p);
+      rt[x] *= e1 * *reinterpret_cast<const f32x4*>(&se[2 * b][i]);
+    }
+  }
+  if (row0 != a.cu[s] || a.positions[a.cu[s]] != 0) {  // (a fresh sequence's first chunk: S = 0)
+    const float* S = c.U + ((long)blockIdx.x * a.H + h) * WD * WD + (long)4 * g4 * WD + 4 * l16;
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      f32x4 sb[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const f32x4 q = *reinterpret_cast<const f32x4*>(S + (16 * x + e) * WD);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sb[j][e] = q[j];
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[j] = mfma_f32_k16(rt[x], sb[j], o[j]);
+    }
+  }
+  const T* G = static_cast<const T*>(a.g);
+  const T* NW = static_cast<const T*>(a.norm_w);
+  T* Y = static_cast<T*>(a.y);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {                        // head RMS norm (zeros past D), weight, gate
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) ss += o[j][i] * o[j][i];
+    ss += __shfl_xor(ss, 1, 64);
+    ss += __shfl_xor(ss, 2, 64);
+    ss += __shfl_xor(ss, 4, 64);
+    ss += __shfl_xor(ss, 8, 64);
+    const int tok = t0 + 4 * g4 + i;
+    if (tok >= n) continue;
+    const float inv = 1.0f / sqrtf(ss / (float)D + a.eps);
+    const long row = row0 + tok;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int d = 4 * l16 + j;
+      if (d < D) {
+        const float g = ld_f32<T>(G, row * a.ld + hc + d);
+        st_f32<T>(Y, row * a.ldy + hc + d,
+                  o[j][i] * inv * ld_f32<T>(NW, hc + d) *
+                      (sizeof(T) == 2 ? g * __builtin_amdgcn_rcpf(1.0f + __expf(-g))
+                                      : g / (1.0f + expf(-g))));
+      }
+    }
+  }
+}
+
+template <typename T, bool VEC>
+static void wkv_chunked(const WkvArgs& a, const WkvChunkArgs& c, int rows, hipStream_t st) {
+  const dim3 gc(rows / WC + c.nseq, a.H), gs(c.nseq, a.H, WD * WD / 1024);
+  hipLaunchKernelGGL((wkv_chunk_state_kernel<T, VEC>), gc, dim3(256), 0, st, a, c);
+  hipLaunchKernelGGL(wkv_chunk_scan_kernel, gs, dim3(256), 0, st, a, c);
+  hipLaunchKernelGGL((wkv_chunk_out_kernel<T, VEC>), gc, dim3(256), 0, st, a, c);
+}
+
+// As eia_wkv_scan for D <= 64 with cu given, for the sequences of split rows or more; rows: cu[nseq] at most; workspaces U
+// [rows / 64 + nseq, H, 64, 64] and L [rows / 64 + nseq, H, 64] fp32.
+EIA_API int eia_wkv_scan_chunked(const void* r, const void* k, const void* v, const void* g,
+                                 long ld, const float* dec, long ld_dec, const void* w0,
+                                 const void* u, const void* norm_w, float* S, float* prev,
+                                 const float* x, int W, const int* slots, const int* cu,
+                                 const int* positions, const int* seq_lens, void* y, long ldy,
+                                 float eps, int nseq, int rows, int H, int D, int split, float* U,
+                                 float* L, int is_bf16, hipStream_t st) {
+  if (nseq < 0 || rows < 0 || H < 1 || D < 1 || W < 1 || split < 1 || !cu || !U || !L)
+    return EIA_BAD_SHAPE;
+  if (D > WD || H > 65535) return EIA_UNSUPPORTED;
+  if (nseq == 0 || rows == 0) return EIA_OK;
+  WkvArgs a{r, k, v, g, ld, dec, ld_dec, w0, u, norm_w, S, prev, x, W, slots, cu, positions,
+            seq_lens, y, ldy, eps, H, D, split};
+  WkvChunkArgs c{U, L, nseq};
+  const uintptr_t any = (uintptr_t)r | (uintptr_t)k | (uintptr_t)v | (uintptr_t)(ld * (is_bf16 ? 2 : 4));
+  const bool vec = D == WD && any % 16 == 0;
+  if (is_bf16 && vec) wkv_chunked<bf16_t, true>(a, c, rows, st);
+  else if (is_bf16) wkv_chunked<bf16_t, false>(a, c, rows, st);
+  else if (vec) wkv_chunked<float, true>(a, c, rows, st);
+  else wkv_chunked<float, false>(a, c, rows, st);
   EIA_LAUNCH_CHECK();
 }

@@ -18,6 +18,19 @@ import torch
 from ._dispatch import check, lib, ptr, require, stream, use_hip
 
 
+CHUNK = 64                 # tokens per chunk of the chunk-parallel form (wkv.hip WC)
+CHUNK_DIM = 64             # ... and its widest head
+
+
+def chunk_rows(nseq: int, heads: int) -> int:
+    """Rows from which a sequence takes the chunk-parallel form.  The token-by-token kernel costs
+    0.5 us a token whatever the batch, until its workgroups share CUs; the other form about 23 us
+    for its launches and then work per chunk: 1.7 us per sequence at 32 heads, so that a step of
+    many sequences needs longer ones.  MI355X, 32 heads, token by token / chunks: 1 x 32 rows 20 /
+    24 us, 1 x 64 35 / 24, 16 x 32 25 / 51, 64 x 8 29 / 141, 1 x 4096 2091 / 112."""
+    return 48 + min(64, nseq * heads // 32)
+
+
 def _seq_bounds(cu: Optional[torch.Tensor], nseq: int):
     if cu is None:
         return [(s, s + 1) for s in range(nseq)]
@@ -99,9 +112,21 @@ def wkv_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor,
     for t in (w0, u, norm_w):
         require(t.dtype == r.dtype and t.is_contiguous() and t.numel() == HD, "per-channel params")
     y = torch.empty(T, HD, dtype=r.dtype, device=r.device)
-    check(lib().eia_wkv_scan(ptr(r), ptr(k), ptr(v), ptr(g), ld, ptr(dec), dec.stride(0), ptr(w0),
-                             ptr(u), ptr(norm_w), ptr(S), ptr(prev_state), ptr(x), x.shape[1],
-                             ptr(slots), ptr(cu), ptr(positions), ptr(seq_lens), ptr(y),
-                             y.stride(0), float(eps), nseq, heads, D, 1 if bf else 0, stream(r)),
-          "wkv_scan")
+    args = (ptr(r), ptr(k), ptr(v), ptr(g), ld, ptr(dec), dec.stride(0), ptr(w0), ptr(u),
+            ptr(norm_w), ptr(S), ptr(prev_state), ptr(x), x.shape[1], ptr(slots), ptr(cu),
+            ptr(positions), ptr(seq_lens), ptr(y), y.stride(0), float(eps), nseq)
+    # Only the device knows the sequences' lengths: both forms are launched where a long sequence is
+    # likely, and each takes its own ones.  (The three more launches are 15 us of host time: a step
+    # of 16 x 8 rows that made them for nothing took 30 us instead of 15.)
+    split = chunk_rows(nseq, heads) if cu is not None and D <= CHUNK_DIM else 0
+    if T - nseq + 1 < split or not (T >= 24 * nseq or T - nseq >= 160):
+        split = 0
+    if nseq > 1 or not split:
+        check(lib().eia_wkv_scan(*args, heads, D, split, 1 if bf else 0, stream(r)), "wkv_scan")
+    if split:
+        n = T // CHUNK + nseq
+        U = torch.empty(n, heads, CHUNK_DIM, CHUNK_DIM, dtype=torch.float32, device=r.device)
+        L = torch.empty(n, heads, CHUNK_DIM, dtype=torch.float32, device=r.device)
+        check(lib().eia_wkv_scan_chunked(*args, T, heads, D, split, ptr(U), ptr(L), 1 if bf else 0,
+                                         stream(r)), "wkv_scan_chunked")
     return y

@@ -25,6 +25,8 @@
 // step is position 0 starts from the initial state whatever its slot held, so slots are reused
 // without clearing.
 // Batch layout: sequence s owns rows [cu[s], cu[s+1]) (cu == nullptr: row s).
+#include <type_traits>
+
 #include "eia_common.h"
 
 struct ScanArgs {
@@ -291,20 +293,635 @@ EIA_API int eia_linear_scan(const void* x, long ld, int q_off, int k_off, int v_
 }
 
 // ---------------------------------------------------------------------------------------------
-// Chunk-parallel form for prompt portions (dk, dv <= 128).  The token-by-token kernel above walks
-// a sequence with one workgroup per head; here a step's rows are cut into chunks of LC tokens
-// (never across sequences) and, with A_t the running sum of log a inside a chunk,
+// Chunk-parallel form for prompt portions, one decay per head and token (modes 0 and 1), dk, dv <=
+// 128.  The token-by-token kernel above walks a sequence with one workgroup per head; here a
+// sequence's rows are cut into chunks of LK tokens and, with l_t = log2 a_t, m_t = log2 b_t,
 //
-//   U_c   = sum_s exp(A_end - A_s) b_s k_s v_s^T            (1) per chunk, in parallel
-//   S_c+1 = exp(A_end) S_c + U_c                            (2) a short scan over a sequence's chunks
-//   o_t   = exp(A_t) S_c^T q_t + sum_(s<=t) exp(A_t - A_s) b_s (q_t . k_s) v_s     (3) per chunk
+//   U   = sum_s 2^(m_s + sum_(x>s) l_x) k_s v_s^T                         (1) per chunk, in parallel
+//   S' = 2^(sum_x l_x) S + U                                              (2) a sequence's chunks in order
+//   o_t = 2^(sum_(x<=t) l_x) S^T q_t
+//         + sum_(s<=t) 2^(m_s + sum_(s<x<=t) l_x) (q_t . k_s) v_s         (3) per chunk, in parallel
 //
-// (with a decay per key channel, mode 2, exp(A) is a vector over the channels and acts inside the
-// products: k_s and q_t are scaled channel by channel)
-// (the normaliser n likewise; n_t . q_t is the row sum of the same weights).  Every exponent is
-// <= 0.  The log gates of the gated mode come from a pre-pass that carries the running maximum
-// through the sequence.  All of it fp32 FMA: the 32-bit mode needs it, and the work is small
-// beside the projections.
+// (the normaliser n is one more state column, n_t . q_t the row sum of the same weights).  Sums of l
+// run over 16-token blocks and over whole blocks; only inside one block is a sum the difference of
+// two running sums, so every exponent is <= 0 and keeps its precision.  The log gates of mode 1 come
+// from a pre-pass that carries the running maximum, angles of rotated heads from a table.
+// Chunks are numbered without a list from the host: sequence s owns the numbers from
+// cu[s] / LK + s on, at least as many as it has chunks; numbers past its last chunk do nothing.
+//
+// Products are fp32 matrix-core products, except q . k of unrotated bf16 rows, which is exact in
+// bf16 operands.  128-token chunks: the states between chunks are the larger part of the memory
+// traffic (4 passes over chunks x H x dk x dv floats), and halving their number costs less than the
+// longer sums inside a chunk add.
+// Four prompts of 1000 .. 2000 tokens (6688 rows), 16 heads of 128, mode 1, bf16 take 13 + 57 + 21 +
+// 122 us on an MI355X (gates, (1), (2), (3)); in 32-token chunks of vector FMAs with a thread per state
+// column it was 63 + 151 + 119 + 581 us.  (3) spends 33 us of it in matrix products and 28 us in
+// vector issue; the rest is waiting for the 64 KiB state that each wave reads.
+constexpr int LK = 128;                     // tokens per chunk
+constexpr int LS_AHEAD = 8;                 // chunks whose contributions are in flight in (2)
+constexpr float LS_LOG2E = 1.4426950408889634f;
+
+struct KChunkArgs {
+  float* U;                                 // [numbers, H, DP, UW]: contribution, then state before
+  float* G;                                 // [numbers, H]: sums of l
+  float* la; float* lb; float* nm;          // [rows, H] log a, log b, -m  (mode 1)
+  float2* rot;                              // [rows, rot_dims / 2]: cos, sin
+  int nseq, rows, DP, VP, UW;               // UW: VP, and in mode 1 four more (the normaliser, 0, 0, 0)
+};
+
+// The chunk of number x; false where there is none or the sequence is skipped.
+EIA_DEV bool ls_chunk(const ScanArgs& a, int nseq, int x, int& s, int& row0, int& n) {
+  int lo = 0, hi = nseq - 1;                // largest s with cu[s] / LK + s <= x
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (a.cu[mid] / LK + mid <= x) lo = mid; else hi = mid - 1;
+  }
+  s = lo;
+  if (x < a.cu[s] / LK + s) return false;   // (rows before the first sequence)
+  row0 = a.cu[s] + (x - a.cu[s] / LK - s) * LK;
+  n = min(LK, a.cu[s + 1] - row0);
+  return n > 0 && a.slots[s] >= 0;
+}
+
+// (A) log gates of mode 1: one workgroup per (sequence, head).  The running maximum m_t =
+// max(f_t + m_(t-1), i_t) is a scan over pairs (f, i); a thread walks four tokens, the pairs of the
+// threads before it come from a scan over lanes and waves.  Serially in one thread the longest of
+// four 2000-token prompts took 63 us.
+template <typename T>
+__global__ void __launch_bounds__(256)
+ls_gates_kernel(ScanArgs a, KChunkArgs c) {
+  __shared__ float2 wsum[4];
+  __shared__ float carry;
+  const int s = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int slot = a.slots[s];
+  if (slot < 0) return;
+  const int lo = a.cu[s], hi = a.cu[s + 1];
+  if (hi <= lo) return;
+  float m0 = a.positions[lo] == 0 ? 0.f : a.M[(long)slot * a.H + h];
+  const T* X = static_cast<const T*>(a.x);
+  for (int base = lo; base < hi; base += 1024) {
+    float gi[4], gf[4];
+    float2 p = {0.f, -INFINITY};                       // the thread's pair: sum of f, max with decays
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int row = base + 4 * tid + k;
+      const T* xr = X + (long)min(row, hi - 1) * a.ld;
+      const float xi = ld_f32<T>(xr, a.i_off + h), xf = ld_f32<T>(xr, a.f_off + h);
+      gi[k] = a.cap > 0.f ? a.cap * tanhf(xi / a.cap) : xi;
+      gf[k] = ls_logsigmoid(a.cap > 0.f ? a.cap * tanhf(xf / a.cap) : xf);
+      if (row < hi) p = {p.x + gf[k], fmaxf(p.y + gf[k], gi[k])};
+    }
+    float2 q = p;                                      // inclusive over the lanes
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const float ux = __shfl_up(q.x, o, 64), uy = __shfl_up(q.y, o, 64);
+      if (lane >= o) q = {ux + q.x, fmaxf(uy + q.x, q.y)};
+    }
+    if (lane == 63) wsum[w] = q;
+    __syncthreads();
+    float m = m0;                                      // m before the thread's first token
+    for (int k = 0; k < w; ++k) m = fmaxf(m + wsum[k].x, wsum[k].y);
+    const float ex = __shfl_up(q.x, 1, 64), ey = __shfl_up(q.y, 1, 64);
+    if (lane > 0) m = fmaxf(m + ex, ey);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int row = base + 4 * tid + k;
+      const float fm = gf[k] + m, mn = fmaxf(fm, gi[k]);
+      if (row < hi) {
+        const long o = (long)row * a.H + h;
+        c.la[o] = fm - mn;
+        c.lb[o] = gi[k] - mn;
+        c.nm[o] = -mn;
+        m = mn;
+      }
+    }
+    if (tid == 255) carry = m;
+    __syncthreads();
+    m0 = carry;
+    // (the thread that holds the last token knows the final maximum)
+    if (base + 1024 >= hi && (hi - 1 - base) >> 2 == tid) a.M[(long)slot * a.H + h] = m;
+  }
+}
+
+// Angles of the rotated channels, shared by all heads and by the q and k of (1) and (3).
+__global__ void __launch_bounds__(256)
+ls_angles_kernel(ScanArgs a, KChunkArgs c) {
+  const int hd = a.rot_dims >> 1;
+  const long u = (long)blockIdx.x * 256 + threadIdx.x;
+  if (u >= (long)c.rows * hd) return;
+  float sn, cs;
+  sincosf((float)a.positions[u / hd] * a.inv_freq[u % hd], &sn, &cs);
+  c.rot[u] = make_float2(cs, sn);
+}
+
+// Eight channels i .. i + 7 (i % 8 == 0) of a q or k head of one row, rotated, not scaled; zero past
+// D.  VEC: 16-byte loads (D, the rotated channels and every offset are multiples of eight).
+template <typename T, bool VEC, bool ROT>
+EIA_DEV void ls_head8(const ScanArgs& a, const KChunkArgs& c, long row, long off, int i, float (&v)[8]) {
+  const T* x = static_cast<const T*>(a.x) + row * a.ld + off;
+  auto get = [&](int j, float (&o)[8]) {
+    if constexpr (VEC) {
+      alignas(16) T t[8];
+      const f32x4* p = reinterpret_cast<const f32x4*>(x + (j < a.D ? j : 0));
+#pragma unroll
+      for (int e = 0; e < (int)(sizeof(T) / 2); ++e) *reinterpret_cast<f32x4*>(&t[e * 16 / sizeof(T)]) = p[e];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = j < a.D ? (float)t[e] : 0.f;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = j + e < a.D ? (float)x[j + e] : 0.f;
+    }
+  };
+  get(i, v);
+  if constexpr (ROT) {
+    const int rd = a.rot_dims, hd = rd >> 1;
+    const float2* r = c.rot + row * hd;
+    if (i >= rd) return;
+    if (a.rot_half) {
+      if (VEC) {
+        const bool second = i >= hd;
+        const int j = second ? i - hd : i;
+        float p[8];
+        get(second ? j : j + hd, p);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = v[e] * r[j + e].x + (second ? p[e] : -p[e]) * r[j + e].y;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int ch = i + e;
+          if (ch < rd) {
+            const bool second = ch >= hd;
+            const int j = second ? ch - hd : ch;
+            const float p = (float)x[second ? j : j + hd];
+            v[e] = v[e] * r[j].x + (second ? p : -p) * r[j].y;
+          }
+        }
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) {
+        if (VEC || i + e < rd) {
+          const float2 cs = r[(i + e) >> 1];
+          const float u = v[e], w = v[e + 1];
+          v[e] = u * cs.x - w * cs.y;
+          v[e + 1] = w * cs.x + u * cs.y;
+        }
+      }
+    }
+  }
+}
+
+// Places in LDS tiles [tokens][MX]: the 16-byte units of a row are turned by the token, so that
+// sixteen tokens' units of one channel group, or four tokens' runs of sixteen channels, lie on
+// different banks.  ls_at: fp32 rows; ls_kat: the key rows of (3), units of 16 / sizeof(KT) entries.
+template <int MX> EIA_DEV int ls_at(int t, int i) { return t * MX + (i ^ ((t & 15) << 2)); }
+template <int MX, typename KT> EIA_DEV int ls_kat(int t, int i) {
+  if constexpr (sizeof(KT) == 4) return ls_at<MX>(t, i);
+  else return t * MX + (i ^ (MX == 128 ? (t & 15) << 3 : ((t >> 1) & 7) << 3));
+}
+// value rows: four tokens' runs meet as rows 4 g + e
+template <int MX> EIA_DEV int ls_vat(int t, int i) { return t * MX + (i ^ (((t >> 2) & 1) * (MX / 2))); }
+
+// Four value columns of a staged row as fp32.
+template <typename T> EIA_DEV f32x4 ls_v4(const T* p) {
+  if constexpr (sizeof(T) == 4) return *reinterpret_cast<const f32x4*>(p);
+  else {
+    const bf16x4 v = *reinterpret_cast<const bf16x4*>(p);
+    return f32x4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
+  }
+}
+
+// Tokens t0 .. t0 + N - 1 of the chunk's values to LDS, zero past the chunk and past Dv.
+template <typename T, bool VEC, int MX, int N, int NT>
+EIA_DEV void ls_stage_v(const ScanArgs& a, int row0, int n, int h, int t0, T* sv) {
+  constexpr int E = VEC ? 16 / (int)sizeof(T) : 1;
+  const T* X = static_cast<const T*>(a.x) + a.v_off + (long)h * a.Dv;
+#pragma unroll
+  for (int u = threadIdx.x; u < N * MX / E; u += NT) {
+    const int t = u / (MX / E), i = E * (u % (MX / E));
+    const bool ok = t0 + t < n && i < a.Dv;
+    const T* p = X + (long)(row0 + (ok ? t0 + t : 0)) * a.ld + (ok ? i : 0);
+    if constexpr (VEC) {
+      const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+      const f32x4 v = *reinterpret_cast<const f32x4*>(p);
+      *reinterpret_cast<f32x4*>(sv + ls_vat<MX>(t, i)) = ok ? v : z;
+    } else {
+      sv[ls_vat<MX>(t, i)] = ok ? *p : (T)0.f;
+    }
+  }
+}
+
+// Sums of l over 16-token blocks: pre up to and with a token, suf behind it, tot of whole blocks;
+// mb: m.  Threads 0 .. LK - 1.
+EIA_DEV void ls_chunk_logs(const ScanArgs& a, const KChunkArgs& c, int row0, int n, int h, float* pre,
+                           float* suf, float* tot, float* mb) {
+  const int t = threadIdx.x;
+  if (t >= LK) return;
+  float l = 0.f, b = 0.f;
+  if (t < n) {
+    if (a.mode == 0) {
+      l = logf(a.decay[h]) * LS_LOG2E;
+    } else {
+      l = c.la[(long)(row0 + t) * a.H + h] * LS_LOG2E;
+      b = c.lb[(long)(row0 + t) * a.H + h] * LS_LOG2E;
+    }
+  }
+  l = fmaxf(l, -150.f);                                // (2^-150 is zero)
+  float p = l, s = l;
+  const int t16 = t & 15;
+#pragma unroll
+  for (int o = 1; o < 16; o <<= 1) {
+    const float up = __shfl_up(p, o, 16), dn = __shfl_down(s, o, 16);
+    if (t16 >= o) p += up;
+    if (t16 + o < 16) s += dn;
+  }
+  const float after = __shfl_down(s, 1, 16);
+  pre[t] = p;
+  suf[t] = t16 == 15 ? 0.f : after;
+  mb[t] = b;
+  if (t16 == 15) tot[t >> 4] = p;
+}
+
+// (1) Eight waves; wave w forms rows 16 w .. of U.  Tokens come in two halves of 64.  A lane of a
+// product over tokens holds columns 64 x + 4 (lane % 16) + j in tile 4 x + j, here and in (3).
+template <typename T, bool VEC, bool ROT, int MX>
+__global__ void __launch_bounds__(512)
+ls_chunk_state_kernel(ScanArgs a, KChunkArgs c) {
+  __shared__ __align__(16) float sk[64 * MX];
+  __shared__ __align__(16) T sv[64 * MX];
+  __shared__ float pre[LK], suf[LK], mb[LK], tot[LK / 16];
+  int s, row0, n;
+  if (!ls_chunk(a, c.nseq, blockIdx.x, s, row0, n)) return;
+  const int h = blockIdx.y, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int l16 = lane & 15, g4 = lane >> 4;
+  ls_chunk_logs(a, c, row0, n, h, pre, suf, tot, mb);
+  f32x4 acc[MX / 16];
+  float un = 0.f;                                      // normaliser row 16 w + l16
+#pragma unroll
+  for (int j = 0; j < MX / 16; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int half = 0; half < 2; ++half) {
+    const int t0 = 64 * half;
+    if (t0 >= n) break;
+    __syncthreads();                                   // logs are there; the first half was read
+    ls_stage_v<T, VEC, MX, 64, 512>(a, row0, n, h, t0, sv);
+#pragma unroll
+    for (int u = threadIdx.x; u < 64 * MX / 8; u += 512) {
+      const int t = u / (MX / 8), i = 8 * (u % (MX / 8)), tk = t0 + t;
+      float v[8];
+      ls_head8<T, VEC, ROT>(a, c, row0 + min(tk, n - 1), a.k_off + (long)h * a.D, i, v);
+      float e = mb[tk] + suf[tk];
+      for (int b = (tk >> 4) + 1; b < LK / 16; ++b) e += tot[b];
+      const float wt = a.kscale * __builtin_amdgcn_exp2f(e);
+#pragma unroll
+      for (int x = 0; x < 8; x += 4)
+        *reinterpret_cast<f32x4*>(sk + ls_at<MX>(t, i + x)) =
+            tk < n ? f32x4{v[x], v[x + 1], v[x + 2], v[x + 3]} * wt : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    __syncthreads();
+    if (16 * w >= c.DP) continue;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      if (t0 + 16 * b >= n) break;
+      f32x4 ka, vb[MX / 16];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int t = 16 * b + 4 * g4 + e;
+        ka[e] = sk[ls_at<MX>(t, 16 * w + l16)];
+#pragma unroll
+        for (int x = 0; x < MX / 64; ++x) {
+          const f32x4 v = ls_v4<T>(sv + ls_vat<MX>(t, 64 * x + 4 * l16));
+#pragma unroll
+          for (int j = 0; j < 4; ++j) vb[4 * x + j][e] = v[j];
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < MX / 16; ++j) acc[j] = mfma_f32_k16(ka, vb[j], acc[j]);
+      un += ka[0] + ka[1] + ka[2] + ka[3];
+    }
+  }
+  const long at = (long)blockIdx.x * a.H + h;
+  if (threadIdx.x == 0) {
+    float g = 0.f;
+    for (int b = 0; b < LK / 16; ++b) g += tot[b];
+    c.G[at] = g;
+  }
+  if (16 * w >= c.DP) return;
+  float* U = c.U + (at * c.DP + 16 * w + 4 * g4) * c.UW;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+#pragma unroll
+    for (int x = 0; x < MX / 64; ++x)
+      if (64 * x + 4 * l16 < c.VP)
+        *reinterpret_cast<f32x4*>(U + (long)i * c.UW + 64 * x + 4 * l16) =
+            f32x4{acc[4 * x][i], acc[4 * x + 1][i], acc[4 * x + 2][i], acc[4 * x + 3][i]};
+  }
+  if (a.mode == 1) {
+    un += __shfl_xor(un, 16, 64);
+    un += __shfl_xor(un, 32, 64);
+    if (g4 == 0)
+      *reinterpret_cast<f32x4*>(c.U + (at * c.DP + 16 * w + l16) * c.UW + c.VP) = f32x4{un, 0.f, 0.f, 0.f};
+  }
+}
+
+// (2) Four columns of a state row per thread: U of a chunk turns into the state before it; the slot
+// receives the state after the last one.  A group's contributions are requested while the previous
+// group is summed.
+__global__ void __launch_bounds__(256)
+ls_chunk_scan_kernel(ScanArgs a, KChunkArgs c) {
+  const int s = blockIdx.x, h = blockIdx.y;
+  const int slot = a.slots[s], lo = a.cu[s], hi = a.cu[s + 1];
+  const int u4 = blockIdx.z * 256 + threadIdx.x, q = c.UW / 4, i = u4 / q, j = 4 * (u4 % q);
+  if (slot < 0 || hi <= lo || i >= c.DP) return;
+  const long x0 = lo / LK + s;
+  const int nc = (hi - lo + LK - 1) / LK;
+  const bool norm = j >= c.VP;                         // the normaliser's columns
+  const int nj = norm ? 1 : a.Dv;
+  float* Sg = norm ? a.N + ((long)slot * a.H + h) * a.D + i
+                   : a.S + (((long)slot * a.H + h) * a.D + i) * a.Dv + j;
+  const int j0 = norm ? 0 : j;
+  f32x4 S = {0.f, 0.f, 0.f, 0.f};
+  if (a.positions[lo] != 0 && i < a.D) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (j0 + k < nj) S[k] = Sg[k];
+  }
+  const long us = (long)a.H * c.DP * c.UW;
+  float* U = c.U + (x0 * a.H + h) * c.DP * c.UW + (long)i * c.UW + j;
+  const float* G = c.G + x0 * a.H + h;
+  f32x4 u[LS_AHEAD];
+  float d[LS_AHEAD];
+  auto fetch = [&](int b, f32x4 (&u)[LS_AHEAD], float (&d)[LS_AHEAD]) {
+#pragma unroll
+    for (int k = 0; k < LS_AHEAD; ++k) {
+      const int x = min(b + k, nc - 1);
+      u[k] = *reinterpret_cast<const f32x4*>(U + x * us);
+      d[k] = G[(long)x * a.H];
+    }
+  };
+  fetch(0, u, d);
+  for (int b = 0; b < nc; b += LS_AHEAD) {
+    f32x4 un[LS_AHEAD];
+    float dn[LS_AHEAD];
+    fetch(b + LS_AHEAD, un, dn);
+#pragma unroll
+    for (int k = 0; k < LS_AHEAD; ++k) {
+      if (b + k < nc) {
+        *reinterpret_cast<f32x4*>(U + (b + k) * us) = S;
+        S = S * __builtin_amdgcn_exp2f(d[k]) + u[k];
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < LS_AHEAD; ++k) {
+      u[k] = un[k];
+      d[k] = dn[k];
+    }
+  }
+  if (i < a.D) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (j0 + k < nj) Sg[k] = S[k];
+  }
+}
+
+// (3) Eight waves; a wave forms the outputs of 16 tokens.  A later block meets more keys: waves i
+// and i + 4, which share a SIMD, take blocks that add up to the same work.
+template <typename T, bool VEC, bool ROT, int MX>
+__global__ void __launch_bounds__(512, 4)
+ls_chunk_out_kernel(ScanArgs a, KChunkArgs c) {
+  // unrotated bf16 keys and queries meet as they are; else both are fp32
+  constexpr bool BF = sizeof(T) == 2 && !ROT;
+  using KT = typename std::conditional<BF, T, float>::type;
+  __shared__ __align__(16) KT sk[LK * MX];
+  __shared__ __align__(16) T sv[LK * MX];
+  __shared__ float pre[LK], suf[LK], mb[LK], tot[LK / 16];
+  int s, row0, n;
+  if (!ls_chunk(a, c.nseq, blockIdx.x, s, row0, n)) return;
+  const int h = blockIdx.y, lane = threadIdx.x & 63, wv = threadIdx.x >> 6, D = a.D, Dv = a.Dv;
+  const int w = wv < 4 ? wv : 11 - wv, l16 = lane & 15, g4 = lane >> 4, t0 = 16 * w;
+  ls_chunk_logs(a, c, row0, n, h, pre, suf, tot, mb);
+  ls_stage_v<T, VEC, MX, LK, 512>(a, row0, n, h, 0, sv);
+#pragma unroll
+  for (int u = threadIdx.x; u < LK * MX / 8; u += 512) {
+    const int t = u / (MX / 8), i = 8 * (u % (MX / 8));
+    float v[8];
+    ls_head8<T, VEC, ROT>(a, c, row0 + min(t, n - 1), a.k_off + (long)h * D, i, v);
+    if constexpr (BF) {
+      bf16x8 b;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) b[e] = t < n ? (bf16_t)v[e] : (bf16_t)0.f;
+      *reinterpret_cast<bf16x8*>(sk + ls_kat<MX, KT>(t, i)) = b;
+    } else {
+#pragma unroll
+      for (int x = 0; x < 8; x += 4)
+        *reinterpret_cast<f32x4*>(sk + ls_kat<MX, KT>(t, i + x)) =
+            t < n ? f32x4{v[x], v[x + 1], v[x + 2], v[x + 3]} : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+  }
+  // this lane's query: channels 32 x + 8 g4 + e
+  const int tq = t0 + l16;
+  KT qf[MX / 32][8];
+#pragma unroll
+  for (int x = 0; x < MX / 32; ++x) {
+    float v[8];
+    ls_head8<T, VEC, ROT>(a, c, row0 + min(tq, n - 1), a.q_off + (long)h * D, 32 * x + 8 * g4, v);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) qf[x][e] = (KT)v[e];
+  }
+  __syncthreads();
+  if (t0 >= n) return;
+  const float qk = a.qscale * a.kscale;
+  f32x4 o[MX / 16];
+#pragma unroll
+  for (int j = 0; j < MX / 16; ++j) o[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float rs = 0.f;                                      // row sum of query l16 (this lane's keys)
+  float back = 0.f;                                    // l from the end of block b to the query's
+  const float pq = pre[tq];
+  for (int b = w; b >= 0; --b) {
+    // weights are formed transposed, keys x queries: their registers are the A operand of P v
+    f32x4 p = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int x = 0; x < MX / 32; ++x) {
+      if constexpr (BF) {
+        bf16x8 qb;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) qb[e] = qf[x][e];
+        const bf16x8 kb = *reinterpret_cast<const bf16x8*>(sk + ls_kat<MX, KT>(16 * b + l16, 32 * x + 8 * g4));
+        p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kb, qb, p, 0, 0, 0);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; e += 4)
+          p = mfma_f32_k16(*reinterpret_cast<const f32x4*>(sk + ls_kat<MX, KT>(16 * b + l16, 32 * x + 8 * g4 + e)),
+                           f32x4{qf[x][e], qf[x][e + 1], qf[x][e + 2], qf[x][e + 3]}, p);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int tk = 16 * b + 4 * g4 + i;
+      const float e = b == w ? pq - pre[tk] + mb[tk] : pq + back + suf[tk] + mb[tk];
+      p[i] = tk <= tq ? p[i] * qk * __builtin_amdgcn_exp2f(e) : 0.f;
+      rs += p[i];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int x = 0; x < MX / 64; ++x) {
+        const f32x4 v = ls_v4<T>(sv + ls_vat<MX>(16 * b + 4 * g4 + e, 64 * x + 4 * l16));
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          o[4 * x + j] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[e], v[j], o[4 * x + j], 0, 0, 0);
+      }
+    if (b < w) back += tot[b];
+  }
+  if (row0 != a.cu[s] || a.positions[a.cu[s]] != 0) {  // (a fresh sequence's first chunk: S = 0)
+    const float eq = a.qscale * __builtin_amdgcn_exp2f(pq + back);
+    const float* S = c.U + ((long)blockIdx.x * a.H + h) * c.DP * c.UW;
+    float nq = 0.f;
+#pragma unroll
+    for (int x = 0; x < MX / 32; ++x)
+#pragma unroll
+      for (int e = 0; e < 8; e += 4) {
+        const int i = 32 * x + 8 * g4 + e;
+        if (32 * x >= c.DP) break;
+        const f32x4 qa = f32x4{(float)qf[x][e], (float)qf[x][e + 1], (float)qf[x][e + 2],
+                               (float)qf[x][e + 3]} * eq;
+#pragma unroll
+        for (int y = 0; y < 4; ++y) {
+          const float* r = S + (long)(i < c.DP ? i + y : 0) * c.UW;
+          if (a.mode == 1) nq += qa[y] * r[c.VP];
+#pragma unroll
+          for (int z = 0; z < MX / 64; ++z) {
+            const int d = 64 * z + 4 * l16;
+            const f32x4 v = *reinterpret_cast<const f32x4*>(r + (d < c.VP ? d : 0));
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              o[4 * z + j] = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[y], v[j], o[4 * z + j], 0, 0, 0);
+          }
+        }
+      }
+    rs += nq;
+  }
+  rs += __shfl_xor(rs, 16, 64);                        // n_t . q_t of query l16
+  rs += __shfl_xor(rs, 32, 64);
+  const T* X = static_cast<const T*>(a.x);
+  const T* NW = static_cast<const T*>(a.norm_w);
+  T* Y = static_cast<T*>(a.y);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {                        // normaliser, head RMS norm, weight, gate
+    const int t = t0 + 4 * g4 + i;
+    const float nqi = __shfl(rs, 4 * g4 + i, 64);
+    const long row = row0 + min(t, n - 1);
+    float den = 1.f;
+    if (a.mode == 1) den = 1.0f / (fmaxf(fabsf(nqi), expf(c.nm[row * a.H + h])) + 1e-6f);
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < MX / 16; ++j) {
+      const bool col = 64 * (j >> 2) + 4 * l16 + (j & 3) < Dv;
+      o[j][i] = col ? o[j][i] * den : 0.f;             // (padded columns read column 0 of S)
+      ss += o[j][i] * o[j][i];
+    }
+    ss += __shfl_xor(ss, 1, 64);
+    ss += __shfl_xor(ss, 2, 64);
+    ss += __shfl_xor(ss, 4, 64);
+    ss += __shfl_xor(ss, 8, 64);
+    if (t >= n) continue;
+    const float inv = a.out_scale / sqrtf(ss / (float)Dv + a.eps);
+#pragma unroll
+    for (int x = 0; x < MX / 64; ++x) {
+      const int d = 64 * x + 4 * l16;
+      if (d >= Dv) continue;
+      const T* gp = X + row * a.ld + a.g_off + (long)h * Dv + d;
+      T* yp = Y + row * a.ldy + (long)h * Dv + d;
+      alignas(16) T g4v[4], y4[4];
+      if constexpr (VEC && sizeof(T) == 2) *reinterpret_cast<float2*>(g4v) = *reinterpret_cast<const float2*>(gp);
+      else if constexpr (VEC) *reinterpret_cast<f32x4*>(g4v) = *reinterpret_cast<const f32x4*>(gp);
+      else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) g4v[j] = gp[d + j < Dv ? j : 0];
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float g = (float)g4v[j];
+        const float sig = sizeof(T) == 2 ? __builtin_amdgcn_rcpf(1.0f + __expf(-g)) : 1.0f / (1.0f + expf(-g));
+        const float nw = (NW && d + j < Dv) ? ld_f32<T>(NW, (long)h * a.norm_h + d + j) : 1.f;
+        y4[j] = (T)(o[4 * x + j][i] * inv * nw * (a.gate_act == 0 ? g * sig : sig));
+      }
+      if constexpr (VEC && sizeof(T) == 2) *reinterpret_cast<float2*>(yp) = *reinterpret_cast<const float2*>(y4);
+      else if constexpr (VEC) *reinterpret_cast<f32x4*>(yp) = *reinterpret_cast<const f32x4*>(y4);
+      else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (d + j < Dv) yp[j] = y4[j];
+      }
+    }
+  }
+}
+
+template <typename T, bool VEC, bool ROT, int MX>
+static void ls_chunked(const ScanArgs& a, const KChunkArgs& c, hipStream_t st) {
+  const dim3 gc(c.rows / LK + c.nseq, a.H), gs(c.nseq, a.H);
+  const dim3 gz(c.nseq, a.H, (c.DP * c.UW / 4 + 255) / 256);
+  if (a.mode == 1) hipLaunchKernelGGL((ls_gates_kernel<T>), gs, dim3(256), 0, st, a, c);
+  if (ROT) {
+    const long u = (long)c.rows * (a.rot_dims >> 1);
+    hipLaunchKernelGGL(ls_angles_kernel, dim3((unsigned)((u + 255) / 256)), dim3(256), 0, st, a, c);
+  }
+  hipLaunchKernelGGL((ls_chunk_state_kernel<T, VEC, ROT, MX>), gc, dim3(512), 0, st, a, c);
+  hipLaunchKernelGGL(ls_chunk_scan_kernel, gz, dim3(256), 0, st, a, c);
+  hipLaunchKernelGGL((ls_chunk_out_kernel<T, VEC, ROT, MX>), gc, dim3(512), 0, st, a, c);
+}
+
+template <typename T>
+static void ls_chunked_forms(const ScanArgs& a, const KChunkArgs& c, hipStream_t st) {
+  constexpr int A = 16 / (int)sizeof(T), W = 8;        // elements in 16 bytes; channels of a unit
+  const int rot8 = a.rot_dims ? (a.rot_half ? a.rot_dims / 2 : a.rot_dims) : 0;
+  const bool vec = (reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.y)) % 16 == 0 &&
+                   (a.ld | a.ldy | a.q_off | a.k_off | a.v_off | a.g_off) % A == 0 && a.D % W == 0 &&
+                   a.Dv % W == 0 && rot8 % W == 0;
+  const bool wide = a.D > 64 || a.Dv > 64, rot = a.rot_dims > 0;
+#define LS_GO(V, R) \
+  do { if (wide) ls_chunked<T, V, R, 128>(a, c, st); else ls_chunked<T, V, R, 64>(a, c, st); } while (0)
+  if (vec) { if (rot) LS_GO(true, true); else LS_GO(true, false); }
+  else { if (rot) LS_GO(false, true); else LS_GO(false, false); }
+#undef LS_GO
+}
+
+// Modes 0 and 1 for steps with prompt portions (cu given; rows: at least cu[nseq]): fp32 workspaces
+// U [rows / 128 + nseq, H, DP, UW] and G [rows / 128 + nseq, H] with DP and VP = dk and dv rounded up
+// to 16, UW = VP + 4 mode; la, lb, nm [rows, H] (mode 1); rot [rows, rot_dims] (rotated heads).
+EIA_API int eia_linear_scan_chunked(const void* x, long ld, int q_off, int k_off, int v_off, int g_off,
+                                    int i_off, int f_off, const float* decay, const float* inv_freq,
+                                    int rot_dims, int rot_half, float qscale, float kscale, float cap,
+                                    float out_scale, const void* norm_w, float* S, float* N, float* M,
+                                    const int* slots, const int* cu, const int* positions, void* y,
+                                    long ldy, float eps, int nseq, int rows, int H, int D, int Dv,
+                                    int mode, int gate_act, int norm_h, float* U, float* G, float* la,
+                                    float* lb, float* nm, float* rot, int is_bf16, hipStream_t st) {
+  if (nseq < 0 || rows < 0 || H < 1 || D < 1 || Dv < 1 || !x || !y || !S || !slots || !cu ||
+      !positions || !U || !G || (mode != 0 && mode != 1) || (mode == 0 && !decay) ||
+      (mode == 1 && (!N || !M || cap < 0.f || !la || !lb || !nm)) || rot_dims < 0 || rot_dims > D ||
+      (rot_dims & 1) || (rot_dims && (!inv_freq || !rot)) || (gate_act != 0 && gate_act != 1))
+    return EIA_BAD_SHAPE;
+  if (D > 128 || Dv > 128 || H > 65535) return EIA_UNSUPPORTED;
+  if (nseq == 0 || rows == 0) return EIA_OK;
+  ScanArgs a{x, ld, q_off, k_off, v_off, g_off, i_off, f_off, decay, inv_freq, rot_dims, rot_half,
+             qscale, kscale, cap, out_scale, norm_w, S, N, M, slots, cu, positions, nullptr, y,
+             ldy, eps, H, D, Dv, mode, gate_act, 0, 0, nullptr, nullptr, 1.f, norm_h};
+  const int DP = (D + 15) / 16 * 16, VP = (Dv + 15) / 16 * 16;
+  KChunkArgs c{U, G, la, lb, nm, reinterpret_cast<float2*>(rot), nseq, rows, DP, VP, VP + 4 * mode};
+  if (is_bf16) ls_chunked_forms<bf16_t>(a, c, st); else ls_chunked_forms<float>(a, c, st);
+  EIA_LAUNCH_CHECK();
+}
+
+// ---------------------------------------------------------------------------------------------
+// Chunk-parallel form of mode 2 (a decay per key channel), dk, dv <= 128: a step's rows are cut into
+// chunks of LC tokens (never across sequences) and, with A_t the running sum of log a inside a chunk,
+// a vector over the key channels,
+//
+//   U_c   = sum_s (exp(A_end - A_s) k_s) v_s^T              (1) per chunk, in parallel
+//   S_c+1 = diag(exp(A_end)) S_c + U_c                      (2) a short scan over a sequence's chunks
+//   o_t   = S_c^T (exp(A_t) q_t) + sum_(s<=t) (q_t exp(A_t - A_s) . k_s) v_s       (3) per chunk
+//
+// Every exponent is <= 0.  All of it fp32 FMA.
 constexpr int LC = 32;                      // tokens per chunk
 constexpr int LD = 128;                     // largest dk / dv of this form
 constexpr int LP = LD + 4;                  // LDS row pitch: 16-byte rows that rotate the banks
@@ -312,12 +929,11 @@ constexpr int LP = LD + 4;                  // LDS row pitch: 16-byte rows that 
 struct ChunkArgs {
   const int* chunks;                        // [nchunk, 4]: sequence, first row, tokens, unused
   const int* seq_first;                     // [nseq + 1]: first chunk of every sequence
-  float* wsS; float* wsN; float* wsG;       // [nchunk, H, D, Dv], [nchunk, H, D], [nchunk, H]
-  float* la; float* lb; float* nm;          // [rows, H] log a, log b, -m  (mode 1)
-  float* cA;                                // [rows, H * D] running log decays of a chunk (mode 2)
-};                                          // (mode 2: wsG is [nchunk, H, D])
+  float* wsS; float* wsG;                   // [nchunk, H, D, Dv], [nchunk, H, D]
+  float* cA;                                // [rows, H * D] running log decays of a chunk
+};
 
-// (A') running log decays per key channel inside every chunk (mode 2), thread = channel.
+// (A') running log decays per key channel inside every chunk, thread = channel.
 template <typename T>
 __global__ void __launch_bounds__(128)
 ls_chan_decay_kernel(ScanArgs a, ChunkArgs c) {
@@ -331,50 +947,6 @@ ls_chan_decay_kernel(ScanArgs a, ChunkArgs c) {
     c.cA[((long)(row0 + t) * a.H + h) * a.D + j] = A;
   }
   c.wsG[((long)ch * a.H + h) * a.D + j] = A;
-}
-
-// (A) log gates of the gated mode: one workgroup per (sequence, head); the transcendentals of 256
-// tokens in parallel, the running maximum serially in one thread.
-template <typename T>
-__global__ void __launch_bounds__(256)
-ls_gates_kernel(ScanArgs a, ChunkArgs c) {
-  __shared__ float gi[256], gf[256], o1[256], o2[256], o3[256];
-  const int s = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
-  const int slot = a.slots[s];
-  if (slot < 0) return;
-  const int lo = a.cu ? a.cu[s] : s, hi = a.cu ? a.cu[s + 1] : s + 1;
-  if (hi <= lo) return;
-  float m = a.positions[lo] == 0 ? 0.f : a.M[(long)slot * a.H + h];
-  const T* X = static_cast<const T*>(a.x);
-  for (int base = lo; base < hi; base += 256) {
-    const int n = min(256, hi - base);
-    if (tid < n) {
-      const T* xr = X + (long)(base + tid) * a.ld;
-      const float xi = ld_f32<T>(xr, a.i_off + h), xf = ld_f32<T>(xr, a.f_off + h);
-      gi[tid] = a.cap > 0.f ? a.cap * tanhf(xi / a.cap) : xi;
-      gf[tid] = ls_logsigmoid(a.cap > 0.f ? a.cap * tanhf(xf / a.cap) : xf);
-    }
-    __syncthreads();
-    if (tid == 0) {
-      for (int t = 0; t < n; ++t) {
-        const float fm = gf[t] + m;
-        const float mn = fmaxf(fm, gi[t]);
-        o1[t] = fm - mn;
-        o2[t] = gi[t] - mn;
-        o3[t] = -mn;
-        m = mn;
-      }
-    }
-    __syncthreads();
-    if (tid < n) {
-      const long o = (long)(base + tid) * a.H + h;
-      c.la[o] = o1[tid];
-      c.lb[o] = o2[tid];
-      c.nm[o] = o3[tid];
-    }
-    __syncthreads();
-  }
-  if (tid == 0) a.M[(long)slot * a.H + h] = m;
 }
 
 // Stages rotated, scaled q or k rows ([LC][LD], zero beyond n tokens / D channels).
@@ -402,37 +974,12 @@ EIA_DEV void ls_stage_rot(const ScanArgs& a, const T* X, int row0, int n, long o
   }
 }
 
-// Running sums of log a inside the chunk (sA) and log b (sB) into LDS, by the first wave.
-EIA_DEV void ls_chunk_decay(const ScanArgs& a, const ChunkArgs& c, int row0, int n, int h,
-                            float* sA, float* sB) {
-  if (threadIdx.x < 64) {
-    const int t = threadIdx.x;
-    float la = 0.f, lb = 0.f;
-    if (t < n) {
-      if (a.mode == 0) {
-        la = logf(a.decay[h]);
-      } else {
-        la = c.la[(long)(row0 + t) * a.H + h];
-        lb = c.lb[(long)(row0 + t) * a.H + h];
-      }
-    }
-#pragma unroll
-    for (int o = 1; o < LC; o <<= 1) {                 // inclusive prefix sum over the lanes
-      const float up = __shfl_up(la, o, 64);
-      if (t >= o) la += up;
-    }
-    if (t < LC) { sA[t] = la; sB[t] = lb; }
-  }
-}
-
-// (1) a chunk's own contribution to the state: U = sum_s w_s k_s v_s^T, u_n = sum_s w_s k_s,
-// w_s = exp(A_end - A_s + log b_s), and the chunk's total log decay.  Thread (r, j): rows
+// (1) a chunk's own contribution to the state.  Thread (r, j): rows
 // [64 r, 64 r + 64) of column j.
-template <typename T, bool CH>
+template <typename T>
 __global__ void __launch_bounds__(256)
-ls_chunk_state_kernel(ScanArgs a, ChunkArgs c) {
+ls_chan_state_kernel(ScanArgs a, ChunkArgs c) {
   __shared__ __align__(16) float sk[LC][LP], sv[LC][LD];
-  __shared__ float sA[LC], sB[LC];
   const int ch = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
   const int s = c.chunks[4 * ch], row0 = c.chunks[4 * ch + 1], n = c.chunks[4 * ch + 2];
   if (a.slots[s] < 0) return;
@@ -444,18 +991,12 @@ ls_chunk_state_kernel(ScanArgs a, ChunkArgs c) {
     sv[t][j] = (t < n && j < Dv) ? ld_f32<T>(X + (long)(row0 + t) * a.ld, a.v_off + (long)h * Dv + j)
                                  : 0.f;
   }
-  if constexpr (!CH) ls_chunk_decay(a, c, row0, n, h, sA, sB);
   __syncthreads();
-  const float Aend = CH ? 0.f : sA[n - 1];
   for (int idx = tid; idx < LC * LD; idx += 256) {     // k_s <- w_s k_s
     const int t = idx / LD, j = idx % LD;
-    if constexpr (CH) {
-      if (t < n && j < D)
-        sk[t][j] *= expf(c.wsG[((long)ch * a.H + h) * D + j] -
-                         c.cA[((long)(row0 + t) * a.H + h) * D + j]);
-    } else {
-      if (t < n) sk[t][j] *= expf(Aend - sA[t] + sB[t]);
-    }
+    if (t < n && j < D)
+      sk[t][j] *= expf(c.wsG[((long)ch * a.H + h) * D + j] -
+                       c.cA[((long)(row0 + t) * a.H + h) * D + j]);
   }
   __syncthreads();
   const int r = tid >> 7, j = tid & 127;
@@ -473,18 +1014,12 @@ ls_chunk_state_kernel(ScanArgs a, ChunkArgs c) {
     for (int i = 0; i < 64; ++i)
       if (64 * r + i < D) U[(long)(64 * r + i) * Dv + j] = acc[i];
   }
-  if (a.mode == 1 && tid < D) {
-    float un = 0.f;
-    for (int t = 0; t < n; ++t) un += sk[t][tid];
-    c.wsN[((long)ch * a.H + h) * D + tid] = un;
-  }
-  if (!CH && tid == 0) c.wsG[(long)ch * a.H + h] = Aend;
 }
 
 // (2) the scan over a sequence's chunks, element by element: the workspace entry of a chunk turns
 // from its own contribution into the state BEFORE the chunk; the slot receives the final state.
 __global__ void __launch_bounds__(256)
-ls_chunk_scan_kernel(ScanArgs a, ChunkArgs c) {
+ls_chan_scan_kernel(ScanArgs a, ChunkArgs c) {
   const int s = blockIdx.x, h = blockIdx.y;
   const int slot = a.slots[s];
   if (slot < 0) return;
@@ -502,38 +1037,27 @@ ls_chunk_scan_kernel(ScanArgs a, ChunkArgs c) {
       float* w = c.wsS + ((long)ch * a.H + h) * n_el + e;
       const float U = *w;
       *w = S;
-      S = expf(a.mode == 2 ? c.wsG[((long)ch * a.H + h) * a.D + ei] : c.wsG[(long)ch * a.H + h]) * S + U;
+      S = expf(c.wsG[((long)ch * a.H + h) * a.D + ei]) * S + U;
     }
     Sg[e] = S;
-  }
-  if (a.mode == 1 && blockIdx.z == 0 && threadIdx.x < a.D) {
-    float* Ng = a.N + ((long)slot * a.H + h) * a.D;
-    float nn = fresh ? 0.f : Ng[threadIdx.x];
-    for (int ch = c0; ch < c1; ++ch) {
-      float* w = c.wsN + ((long)ch * a.H + h) * a.D + threadIdx.x;
-      const float U = *w;
-      *w = nn;
-      nn = expf(c.wsG[(long)ch * a.H + h]) * nn + U;
-    }
-    Ng[threadIdx.x] = nn;
   }
 }
 
 // (3) a chunk's outputs from the state before it and its own tokens.  Thread (r, j): tokens
 // r, r + 2, ... of column j.
-// CH (a decay per key channel): the pair weights sum q_t k_u exp(A_t - A_u) over the channels.  A
+// The pair weights sum q_t k_u exp(A_t - A_u) over the channels.  A
 // chunk is four blocks of eight tokens; pairs inside a block form their exponents one by one,
 // pairs of different blocks factor them through the block edges (E_b: A just before block b),
 //   exp(A_t - A_u) = exp(A_t - E_tb) exp(E_tb - E_(ub+1)) exp(E_(ub+1) - A_u),
 // so every exponent stays <= 0 whatever the decays.
-template <typename T, bool CH>
+template <typename T>
 __global__ void __launch_bounds__(256)
-ls_chunk_out_kernel(ScanArgs a, ChunkArgs c) {
+ls_chan_out_kernel(ScanArgs a, ChunkArgs c) {
   __shared__ __align__(16) float sq[LC][LP], sk[LC][LP], sv[LC][LD];
   __shared__ float P[LC][LC + 1];
-  __shared__ float sA[LC], sB[LC], snq[LC], red[LC][2];
-  __shared__ __align__(16) float sC[CH ? LC : 1][CH ? LP : 1];   // running log decays per channel
-  __shared__ __align__(16) float sE[CH ? 3 : 1][CH ? LP : 1];    // products over whole blocks
+  __shared__ float red[LC][2];
+  __shared__ __align__(16) float sC[LC][LP];           // running log decays per channel
+  __shared__ __align__(16) float sE[3][LP];            // products over whole blocks
   const int ch = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
   const int s = c.chunks[4 * ch], row0 = c.chunks[4 * ch + 1], n = c.chunks[4 * ch + 2];
   if (a.slots[s] < 0) return;
@@ -546,91 +1070,63 @@ ls_chunk_out_kernel(ScanArgs a, ChunkArgs c) {
     sv[t][j] = (t < n && j < Dv) ? ld_f32<T>(X + (long)(row0 + t) * a.ld, a.v_off + (long)h * Dv + j)
                                  : 0.f;
   }
-  if constexpr (CH) {
-    for (int idx = tid; idx < LC * LD; idx += 256) {
-      const int t = idx / LD, j = idx % LD;            // (past the chunk's end: the last token's)
-      sC[t][j] = j < D ? c.cA[((long)(row0 + min(t, n - 1)) * a.H + h) * D + j] : 0.f;
-    }
-    __syncthreads();
-    // pairs inside a block of eight
-    for (int idx = tid; idx < LC * 8; idx += 256) {
-      const int t = idx >> 3, u = (t & ~7) + (idx & 7);
-      float p = 0.f;
-      if (u <= t && t < n) {
-        const f32x4* qa = reinterpret_cast<const f32x4*>(sq[t]);
-        const f32x4* ka = reinterpret_cast<const f32x4*>(sk[u]);
-        const f32x4* At = reinterpret_cast<const f32x4*>(sC[t]);
-        const f32x4* Au = reinterpret_cast<const f32x4*>(sC[u]);
+  for (int idx = tid; idx < LC * LD; idx += 256) {
+    const int t = idx / LD, j = idx % LD;            // (past the chunk's end: the last token's)
+    sC[t][j] = j < D ? c.cA[((long)(row0 + min(t, n - 1)) * a.H + h) * D + j] : 0.f;
+  }
+  __syncthreads();
+  // pairs inside a block of eight
+  for (int idx = tid; idx < LC * 8; idx += 256) {
+    const int t = idx >> 3, u = (t & ~7) + (idx & 7);
+    float p = 0.f;
+    if (u <= t && t < n) {
+      const f32x4* qa = reinterpret_cast<const f32x4*>(sq[t]);
+      const f32x4* ka = reinterpret_cast<const f32x4*>(sk[u]);
+      const f32x4* At = reinterpret_cast<const f32x4*>(sC[t]);
+      const f32x4* Au = reinterpret_cast<const f32x4*>(sC[u]);
 #pragma unroll 4
-        for (int i = 0; i < (D + 3) / 4; ++i) {
-          const f32x4 x = qa[i] * ka[i], d = At[i] - Au[i];
-          p += x[0] * __expf(d[0]) + x[1] * __expf(d[1]) + x[2] * __expf(d[2]) + x[3] * __expf(d[3]);
-        }
+      for (int i = 0; i < (D + 3) / 4; ++i) {
+        const f32x4 x = qa[i] * ka[i], d = At[i] - Au[i];
+        p += x[0] * __expf(d[0]) + x[1] * __expf(d[1]) + x[2] * __expf(d[2]) + x[3] * __expf(d[3]);
       }
-      P[t][u] = p;
     }
-    __syncthreads();
-    // q_t <- q_t exp(A_t - E_tb), k_u <- k_u exp(E_(ub+1) - A_u); block products for the carry
-    for (int idx = tid; idx < LC * LD; idx += 256) {
-      const int t = idx / LD, j = idx % LD, b = t >> 3;
-      const float A = sC[t][j];
-      sq[t][j] *= expf(A - (b ? sC[8 * b - 1][j] : 0.f));
-      sk[t][j] *= expf(sC[8 * b + 7][j] - A);
-      if (t < 3) sE[t][j] = expf(sC[8 * t + 15][j] - sC[8 * t + 7][j]);   // over block t + 1
-    }
-    __syncthreads();
-    // pairs of different blocks: (t, u) with ub < tb, over the blocks between them
-    for (int idx = tid; idx < LC * LC; idx += 256) {
-      const int t = idx / LC, u = idx % LC, tb = t >> 3, ub = u >> 3;
-      if (ub == tb) continue;
-      float p = 0.f;
-      if (ub < tb && t < n) {
-        const f32x4* qa = reinterpret_cast<const f32x4*>(sq[t]);
-        const f32x4* ka = reinterpret_cast<const f32x4*>(sk[u]);
-        const f32x4* e0 = reinterpret_cast<const f32x4*>(sE[ub]);        // block ub + 1
-        const f32x4* e1 = reinterpret_cast<const f32x4*>(sE[ub < 1 ? 1 : ub]);   // block ub + 2
+    P[t][u] = p;
+  }
+  __syncthreads();
+  // q_t <- q_t exp(A_t - E_tb), k_u <- k_u exp(E_(ub+1) - A_u); block products for the carry
+  for (int idx = tid; idx < LC * LD; idx += 256) {
+    const int t = idx / LD, j = idx % LD, b = t >> 3;
+    const float A = sC[t][j];
+    sq[t][j] *= expf(A - (b ? sC[8 * b - 1][j] : 0.f));
+    sk[t][j] *= expf(sC[8 * b + 7][j] - A);
+    if (t < 3) sE[t][j] = expf(sC[8 * t + 15][j] - sC[8 * t + 7][j]);   // over block t + 1
+  }
+  __syncthreads();
+  // pairs of different blocks: (t, u) with ub < tb, over the blocks between them
+  for (int idx = tid; idx < LC * LC; idx += 256) {
+    const int t = idx / LC, u = idx % LC, tb = t >> 3, ub = u >> 3;
+    if (ub == tb) continue;
+    float p = 0.f;
+    if (ub < tb && t < n) {
+      const f32x4* qa = reinterpret_cast<const f32x4*>(sq[t]);
+      const f32x4* ka = reinterpret_cast<const f32x4*>(sk[u]);
+      const f32x4* e0 = reinterpret_cast<const f32x4*>(sE[ub]);        // block ub + 1
+      const f32x4* e1 = reinterpret_cast<const f32x4*>(sE[ub < 1 ? 1 : ub]);   // block ub + 2
 #pragma unroll 4
-        for (int i = 0; i < (D + 3) / 4; ++i) {
-          f32x4 x = qa[i] * ka[i];
-          if (tb - ub > 1) x *= e0[i];
-          if (tb - ub > 2) x *= e1[i];
-          p += x[0] + x[1] + x[2] + x[3];
-        }
+      for (int i = 0; i < (D + 3) / 4; ++i) {
+        f32x4 x = qa[i] * ka[i];
+        if (tb - ub > 1) x *= e0[i];
+        if (tb - ub > 2) x *= e1[i];
+        p += x[0] + x[1] + x[2] + x[3];
       }
-      P[t][u] = p;
     }
-    __syncthreads();
-    // the carry reads q_t exp(A_t)
-    for (int idx = tid; idx < (LC - 8) * LD; idx += 256) {
-      const int t = 8 + idx / LD, j = idx % LD;
-      sq[t][j] *= expf(sC[8 * (t >> 3) - 1][j]);
-    }
-  } else {
-    ls_chunk_decay(a, c, row0, n, h, sA, sB);
-    __syncthreads();
-    // weights of the chunk's own pairs: P[t][u] = (q_t . k_u) exp(A_t - A_u + log b_u), u <= t
-    for (int idx = tid; idx < LC * LC; idx += 256) {
-      const int t = idx / LC, u = idx % LC;
-      float p = 0.f;
-      if (u <= t && t < n) {
-        const f32x4* qa = reinterpret_cast<const f32x4*>(sq[t]);
-        const f32x4* ka = reinterpret_cast<const f32x4*>(sk[u]);
-  #pragma unroll 8
-        for (int i = 0; i < LD / 4; ++i) {
-          const f32x4 x = qa[i], y = ka[i];
-          p += x[0] * y[0] + x[1] * y[1] + x[2] * y[2] + x[3] * y[3];
-        }
-        p *= expf(sA[t] - sA[u] + sB[u]);
-      }
-      P[t][u] = p;
-    }
-    // n_before . q_t of the gated mode
-    if (a.mode == 1 && tid < n) {
-      const float* nb = c.wsN + ((long)ch * a.H + h) * D;
-      float d = 0.f;
-      for (int i = 0; i < D; ++i) d += nb[i] * sq[tid][i];
-      snq[tid] = d;
-    }
+    P[t][u] = p;
+  }
+  __syncthreads();
+  // the carry reads q_t exp(A_t)
+  for (int idx = tid; idx < (LC - 8) * LD; idx += 256) {
+    const int t = 8 + idx / LD, j = idx % LD;
+    sq[t][j] *= expf(sC[8 * (t >> 3) - 1][j]);
   }
   __syncthreads();
   const int r = tid >> 7, j = tid & 127;
@@ -657,13 +1153,7 @@ ls_chunk_out_kernel(ScanArgs a, ChunkArgs c) {
 #pragma unroll
   for (int tt = 0; tt < LC / 2; ++tt) {
     const int t = 2 * tt + r;
-    const float eA = CH ? 1.f : expf(sA[t < n ? t : 0]);
-    float o = (j < Dv && t < n) ? own[tt] + eA * carry[tt] : 0.f;
-    if (a.mode == 1 && t < n) {
-      float nq = eA * snq[t];
-      for (int u = 0; u <= t; ++u) nq += P[t][u];
-      o = o / (fmaxf(fabsf(nq), expf(c.nm[(long)(row0 + t) * a.H + h])) + 1e-6f);
-    }
+    const float o = (j < Dv && t < n) ? own[tt] + carry[tt] : 0.f;
     const float ss = wave_sum(o * o);
     if ((tid & 63) == 0) red[t][(tid >> 6) & 1] = ss;
     own[tt] = o;
@@ -682,48 +1172,39 @@ ls_chunk_out_kernel(ScanArgs a, ChunkArgs c) {
   }
 }
 
-// The same arguments as eia_linear_scan plus the step's chunk list (chunks int32 [nchunk, 4]:
-// sequence, first row, tokens (1 .. 32), 0; seq_first int32 [nseq + 1]) and fp32 workspaces
-// wsS [nchunk, H, D, Dv], wsN [nchunk, H, D], wsG [nchunk, H], la / lb / nm [rows, H].
-EIA_API int eia_linear_scan_chunked(const void* x, long ld, int q_off, int k_off, int v_off,
-                                    int g_off, int i_off, int f_off, const float* decay,
-                                    const float* inv_freq, int rot_dims, int rot_half,
-                                    float qscale, float kscale, float cap, float out_scale,
-                                    const void* norm_w, float* S, float* N, float* M,
-                                    const int* slots, const int* cu, const int* positions,
-                                    void* y, long ldy, float eps, int nseq, int H, int D, int Dv,
-                                    int mode, int gate_act, int is_bf16, const int* chunks,
-                                    const int* seq_first, int nchunk, float* wsS, float* wsN,
-                                    float* wsG, float* la, float* lb, float* nm, int lo_off, int R,
-                                    const float* a2t, const float* a2b, float inv_tau, int norm_h,
-                                    float* cA, hipStream_t st) {
+// Mode 2 with the step's chunk list (chunks int32 [nchunk, 4]: sequence, first row, tokens (1 .. 32),
+// 0; seq_first int32 [nseq + 1]) and fp32 workspaces wsS [nchunk, H, D, Dv], wsG [nchunk, H, D], cA
+// [rows, H * D].
+EIA_API int eia_linear_scan_channels(const void* x, long ld, int q_off, int k_off, int v_off,
+                                     int g_off, const float* inv_freq, int rot_dims, int rot_half,
+                                     float qscale, float kscale, float out_scale,
+                                     const void* norm_w, float* S, const int* slots, const int* cu,
+                                     const int* positions, void* y, long ldy, float eps, int nseq,
+                                     int H, int D, int Dv, int gate_act, int norm_h,
+                                     const int* chunks, const int* seq_first, int nchunk, float* wsS,
+                                     float* wsG, int lo_off, int R, const float* a2t,
+                                     const float* a2b, float inv_tau, float* cA, int is_bf16,
+                                     hipStream_t st) {
   if (nseq < 0 || nchunk < 0 || H < 1 || D < 1 || Dv < 1 || !x || !y || !S || !slots || !positions ||
-      !chunks || !seq_first || !wsS || !wsG || mode < 0 || mode > 2 || (mode == 0 && !decay) ||
-      (mode == 2 && (R < 1 || !a2t || !cA)) ||
-      (mode == 1 && (!N || !M || cap < 0.f || !wsN || !la || !lb || !nm)) || rot_dims < 0 ||
+      !chunks || !seq_first || !wsS || !wsG || R < 1 || !a2t || !cA || rot_dims < 0 ||
       rot_dims > D || (rot_dims & 1) || (rot_dims && !inv_freq) ||
       (gate_act != 0 && gate_act != 1))
     return EIA_BAD_SHAPE;
   if (D > LD || Dv > LD) return EIA_UNSUPPORTED;
   if (nseq == 0 || nchunk == 0) return EIA_OK;
-  ScanArgs a{x, ld, q_off, k_off, v_off, g_off, i_off, f_off, decay, inv_freq, rot_dims, rot_half,
-             qscale, kscale, cap, out_scale, norm_w, S, N, M, slots, cu, positions, nullptr, y,
-             ldy, eps, H, D, Dv, mode, gate_act, lo_off, R, a2t, a2b, inv_tau, norm_h};
-  ChunkArgs c{chunks, seq_first, wsS, wsN, wsG, la, lb, nm, cA};
-  const dim3 gs(nseq, H), gc(nchunk, H), gz(nseq, H, (D * Dv + 255) / 256);
-#define LS_CHUNKED(TT, CHN)                                                                   \
-  do {                                                                                        \
-    if (mode == 1) hipLaunchKernelGGL((ls_gates_kernel<TT>), gs, dim3(256), 0, st, a, c);     \
-    if (mode == 2) hipLaunchKernelGGL((ls_chan_decay_kernel<TT>), gc, dim3(128), 0, st, a, c); \
-    hipLaunchKernelGGL((ls_chunk_state_kernel<TT, CHN>), gc, dim3(256), 0, st, a, c);         \
-    hipLaunchKernelGGL(ls_chunk_scan_kernel, gz, dim3(256), 0, st, a, c);                     \
-    hipLaunchKernelGGL((ls_chunk_out_kernel<TT, CHN>), gc, dim3(256), 0, st, a, c);           \
+  ScanArgs a{x, ld, q_off, k_off, v_off, g_off, 0, 0, nullptr, inv_freq, rot_dims, rot_half,
+             qscale, kscale, 0.f, out_scale, norm_w, S, nullptr, nullptr, slots, cu, positions,
+             nullptr, y, ldy, eps, H, D, Dv, 2, gate_act, lo_off, R, a2t, a2b, inv_tau, norm_h};
+  ChunkArgs c{chunks, seq_first, wsS, wsG, cA};
+  const dim3 gc(nchunk, H), gz(nseq, H, (D * Dv + 255) / 256);
+#define LS_CHUNKED(TT)                                                              \
+  do {                                                                              \
+    hipLaunchKernelGGL((ls_chan_decay_kernel<TT>), gc, dim3(128), 0, st, a, c);     \
+    hipLaunchKernelGGL((ls_chan_state_kernel<TT>), gc, dim3(256), 0, st, a, c);     \
+    hipLaunchKernelGGL(ls_chan_scan_kernel, gz, dim3(256), 0, st, a, c);            \
+    hipLaunchKernelGGL((ls_chan_out_kernel<TT>), gc, dim3(256), 0, st, a, c);       \
   } while (0)
-  if (is_bf16) {
-    if (mode == 2) LS_CHUNKED(bf16_t, true); else LS_CHUNKED(bf16_t, false);
-  } else {
-    if (mode == 2) LS_CHUNKED(float, true); else LS_CHUNKED(float, false);
-  }
+  if (is_bf16) LS_CHUNKED(bf16_t); else LS_CHUNKED(float);
 #undef LS_CHUNKED
   EIA_LAUNCH_CHECK();
 }

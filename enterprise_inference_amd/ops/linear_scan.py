@@ -26,7 +26,7 @@ slot held, so freed slots are reused without clearing.  Batch layout: sequence `
 state slot (< 0: padding row, skipped).
 
 Prompt portions run a chunk-parallel form on the GPU (``chunk_plan``): the step's rows are cut
-into chunks of 32 tokens, every chunk's own contribution to the state is formed in parallel, a
+into chunks of 128 tokens (32 with a decay per key channel), every chunk's own contribution to the state is formed in parallel, a
 short scan over a sequence's chunks yields the state before each chunk, and the outputs of all
 chunks are formed in parallel from that state and the chunk's own tokens.  The token-by-token
 kernel serves decode steps (also inside captured graphs) and heads wider than 128.
@@ -95,7 +95,8 @@ class ScanState:
         return 4 * per
 
 
-CHUNK = 32                 # tokens per chunk of the chunk-parallel form (linear_scan.hip LC)
+CHUNK = 32                 # tokens per chunk of the chunk-parallel form ("channel", linear_scan.hip LC)
+HEAD_CHUNK = 128           # ... with one decay per head and token (linear_scan.hip LK)
 CHUNK_MAX_DIM = 128        # ... and its largest dk / dv
 CHUNK_MIN_ROWS = 48        # a sequence with at least this many rows in the step selects it
 # tests and measurements: take the chunk-parallel form whenever a plan is handed over
@@ -113,14 +114,22 @@ class ChunkPlan:
         self.chunks, self.seq_first, self.n, self.rows = chunks, seq_first, n, rows
         self.nseq, self.longest = nseq, longest
 
-    def pays(self, heads: int, dim: int, cus: int = 256) -> bool:
+    def pays(self, heads: int, dim: int, cus: int = 256, channel: bool = False) -> bool:
         """Whether the chunk-parallel form beats the token-by-token one for a layer of ``heads``
-        heads up to ``dim`` wide: the latter walks the longest sequence with one workgroup per
-        (sequence, head) at about 0.5 us a token (0.85 us above 64), the former costs about 5 ns
-        (7 ns) per token and head over all rows (MI355X, measured on 4096-token prompts)."""
+        heads up to ``dim`` wide.  The latter walks the longest sequence at about 0.5 us a token
+        (0.85 us above 64) while its workgroups, one per (sequence, head), do not share CUs.  The
+        former costs 30 us for its launches and 0.7 ns (2 ns) per row and head, a short sequence
+        counting as 96 rows; with a decay per key channel 5 ns (7 ns).  MI355X, 16 heads of 128,
+        exponential gates, token by token / chunks: 1 x 48 rows 62 / 29 us, 1 x 4096 4793 / 145,
+        16 x 64 84 / 63, 16 x 512 599 / 196; 32 heads of 64, fixed decays: 1 x 48 24 / 27, 16 x 64
+        34 / 47, 16 x 128 75 / 68, 1 x 4096 2035 / 104."""
         wide = dim > 64
-        serial = self.longest * (0.85 if wide else 0.5) * -(-self.nseq * heads // cus)
-        return self.rows * heads * (0.0072 if wide else 0.0052) < serial
+        if channel:
+            serial = self.longest * (0.85 if wide else 0.5) * -(-self.nseq * heads // cus)
+            return self.rows * heads * (0.0072 if wide else 0.0052) < serial
+        busy = self.nseq * heads / (cus if wide else 2.7 * cus)
+        serial = self.longest * (0.85 if wide else 0.5) * max(1.0, busy)
+        return 30 + max(self.rows, 96 * self.nseq) * heads * (0.002 if wide else 0.0007) < serial
 
 
 def chunk_plan(host_lens, device, chunk: int = CHUNK, min_rows: int = CHUNK_MIN_ROWS,
@@ -270,23 +279,35 @@ def linear_scan(fused: torch.Tensor, q_off: int, k_off: int, v_off: int, g_off: 
     chan = (lo_off, R, ptr(spec.a2t), ptr(spec.a2b), 1.0 / float(spec.tau),
             0 if spec.norm_shared else Dv)
     if (plan is not None and plan.n and max(D, Dv) <= CHUNK_MAX_DIM and cu is not None
-            and plan.rows == T and (FORCE_CHUNKED or plan.pays(H, max(D, Dv)))
+            and plan.rows == T and (FORCE_CHUNKED or plan.pays(H, max(D, Dv), channel=channel))
             and not torch.cuda.is_current_stream_capturing()):
         dev = fused.device
         f32 = lambda *shape: torch.empty(*shape, dtype=torch.float32, device=dev)
-        wsS, wsG = f32(plan.n, H, D, Dv), f32(plan.n, H, D if channel else 1)
-        cA = f32(T, H, D) if channel else None
-        wsN = f32(plan.n, H, D) if exp_gates else None
+        act = 0 if spec.gate_act == "silu" else 1
+        if channel:
+            wsS, wsG, cA = f32(plan.n, H, D, Dv), f32(plan.n, H, D), f32(T, H, D)
+            check(lib().eia_linear_scan_channels(
+                ptr(fused), fused.stride(0), q_off, k_off, v_off, g_off, ptr(spec.inv_freq),
+                spec.rot_dims, 1 if spec.rot_half else 0, float(spec.qscale), float(spec.kscale),
+                float(spec.out_scale), ptr(norm_w), ptr(state.S), ptr(slots), ptr(cu),
+                ptr(positions), ptr(out), out.stride(0), float(spec.eps), nseq, H, D, Dv, act,
+                chan[-1], ptr(plan.chunks), ptr(plan.seq_first), plan.n, ptr(wsS), ptr(wsG),
+                *chan[:-1], ptr(cA), 1 if bf else 0, stream(fused)), "linear_scan_channels")
+            return out
+        # (these chunks are longer than the plan's and found on the device)
+        n, up16 = T // HEAD_CHUNK + nseq, lambda v: -(-v // 16) * 16
+        U = f32(n, H, up16(D), up16(Dv) + (4 if exp_gates else 0))
+        G = f32(n, H)
         la, lb, nm = (f32(T, H), f32(T, H), f32(T, H)) if exp_gates else (None, None, None)
+        rot = f32(T, spec.rot_dims) if spec.rot_dims else None
         check(lib().eia_linear_scan_chunked(
             ptr(fused), fused.stride(0), q_off, k_off, v_off, g_off, i_off, f_off,
             ptr(spec.decay), ptr(spec.inv_freq), spec.rot_dims, 1 if spec.rot_half else 0,
             float(spec.qscale), float(spec.kscale), float(spec.cap), float(spec.out_scale),
             ptr(norm_w), ptr(state.S), ptr(state.n), ptr(state.m), ptr(slots), ptr(cu),
-            ptr(positions), ptr(out), out.stride(0), float(spec.eps), nseq, H, D, Dv,
-            mode, 0 if spec.gate_act == "silu" else 1, 1 if bf else 0,
-            ptr(plan.chunks), ptr(plan.seq_first), plan.n, ptr(wsS), ptr(wsN), ptr(wsG), ptr(la),
-            ptr(lb), ptr(nm), *chan, ptr(cA), stream(fused)), "linear_scan_chunked")
+            ptr(positions), ptr(out), out.stride(0), float(spec.eps), nseq, T, H, D, Dv, mode, act,
+            chan[-1], ptr(U), ptr(G), ptr(la), ptr(lb), ptr(nm), ptr(rot), 1 if bf else 0,
+            stream(fused)), "linear_scan_chunked")
         return out
     check(lib().eia_linear_scan(
         ptr(fused), fused.stride(0), q_off, k_off, v_off, g_off, i_off, f_off, ptr(spec.decay),

@@ -50,3 +50,45 @@ def test_wkv_chunks(lens, H, D, dtype):
     assert _rel(z.cpu()[live], y[live]) < (1e-5 if dtype == torch.float32 else 4e-3)
     assert _rel(dev[8], S) < 2e-6
     assert torch.equal(dev[9].cpu(), prev)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("mode,rot,half", [("exp_gates", 0, True), ("decay", 64, True),
+                                           ("decay", 12, False), ("exp_gates", 20, True)])
+@pytest.mark.parametrize("H,D,Dv", [(2, 128, 128), (3, 64, 64), (2, 72, 40)])
+@pytest.mark.parametrize("lens", [[1, 128, 127, 129, 300], [500], [16, 15, 17, 144, 3]])
+def test_linear_chunks(lens, H, D, Dv, mode, rot, half, dtype, monkeypatch):
+    from enterprise_inference_amd.ops import linear_scan as ls
+    monkeypatch.setattr(ls, "FORCE_CHUNKED", True)
+    g = torch.Generator().manual_seed(sum(lens) + D + rot)
+    rnd = lambda *s: torch.randn(*s, generator=g)
+    n, T = len(lens), sum(lens)
+    cu, pos, slots = _step(lens, [0 if s % 2 == 0 else 5 for s in range(n)], n > 3)
+    at = [0, H * D, 2 * H * D, 2 * H * D + H * Dv, 2 * H * (D + Dv), 2 * H * (D + Dv) + H]
+    x = rnd(T, at[-1] + H)
+    x[:, at[-1]:] += 3.0
+    x = x.to(dtype)
+    inv = 10000.0 ** (-torch.arange(rot // 2) / max(1, rot // 2))
+
+    def run(dev):
+        spec = ls.ScanSpec(H, D, Dv, mode, cap=15.0, kscale=D ** -0.5, qscale=1.5, eps=1e-5,
+                           rot_dims=rot, rot_half=half, inv_freq=inv.to(dev), out_scale=0.7,
+                           decay=torch.linspace(0.999, 0.2, H).to(dev))
+        st = ls.ScanState.allocate(n, spec, "cpu")
+        gs = torch.Generator().manual_seed(1)
+        for t in (st.S, st.n, st.m):
+            if t is not None:
+                t.copy_(torch.randn(t.shape, generator=gs))
+        st = ls.ScanState(*(None if t is None else t.to(dev) for t in (st.S, st.n, st.m)))
+        plan = ls.chunk_plan(lens, dev) if dev == "cuda" else None
+        nw = torch.linspace(0.8, 1.2, H * Dv).to(dtype).to(dev)
+        y = ls.linear_scan(x.to(dev), at[0], at[1], at[2], at[3], spec, st, slots.to(dev),
+                           cu.to(dev), n, pos.to(dev), None, nw, at[4], at[5], plan=plan)
+        return y.cpu(), st
+
+    (y, a), (z, b) = run("cpu"), run("cuda")
+    live = torch.cat([torch.full((m,), int(s) >= 0) for m, s in zip(lens, slots)])
+    # fp32 sums over at most 128 products; bf16 adds one rounding and at times one step more
+    assert _rel(z[live], y[live]) < (1e-5 if dtype == torch.float32 else 4e-3)
+    for u, v in ((a.S, b.S), (a.n, b.n), (a.m, b.m)):
+        assert u is None or _rel(v, u) < 2e-6

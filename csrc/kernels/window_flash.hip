@@ -1,0 +1,472 @@
+// Windowed attention over prompt portions (bf16), for layers without head mixing or a distance term:
+// the caches, masks, weights and epilogues of window_attention.hip, on v_mfma_f32_32x32x16_bf16 with
+// keys and values shared through LDS.
+//
+// A workgroup of four waves owns HPW heads of one kv head (4, 2 or 1: as many as divide the group) and
+// 128 / HPW queries of one sequence; wave w takes head w % HPW and 32 queries, so that a 64-key tile
+// of K and V^T staged once in LDS feeds 128 (query, head) rows.  (The 16-query form in
+// window_attention.hip reads every operand of every head from the caches: 64 bytes of operand loads
+// per matrix instruction and lane, which bound it at 77 .. 127 TFLOP/s.)
+//
+// Per wave and tile: S^T[key, q] = K Q^T with Q^T in registers; a lane owns one query column, so the
+// softmax is lane-local but for one exchange with lane ^ 32; key rows are fed with bits 2 and 3 of
+// their number swapped, which makes a lane's accumulators eight consecutive keys, the operand of
+// O^T += V^T P^T.  The weights stay fp32: they enter the second product as a bf16 high part plus a
+// bf16 remainder, and the normaliser sums the fp32 values.  The running maximum moves only when a
+// tile exceeds it by 2^8.  Tile i + 1 is fetched into registers before tile i is multiplied and
+// written to the other LDS buffer behind it; one barrier per tile.  Rows are padded by 16 bytes, so
+// that the sixteen rows of an operand read lie on different banks.
+//
+// Four ragged prompts of up to 2048 tokens, 16 heads of 128 on 4, window 1024, soft-capped: 74 us on an
+// MI355X (249 us in the 16-query form); one 4096-token causal prompt, 8 heads on 2: 79 + 16 us in
+// parts (459 us), 126 us uncut -- a tile takes a lone workgroup 2.0 us, of which its matrix products
+// are 0.64 us; where two workgroups share a CU their products and exponentials overlap.
+#include "eia_common.h"
+
+namespace {
+
+typedef __attribute__((ext_vector_type(16))) float f32x16_t;
+
+constexpr int WF_KEYS = 64;                 // keys per tile
+constexpr int WF_ROWS = 128;                // (query, head) rows per workgroup
+constexpr float WF_LOG2E = 1.4426950408889634f;
+constexpr float WF_DEFER = 8.f;             // log2 by which a tile may exceed the running maximum
+
+struct FlashArgs {
+  const bf16_t* q; long ldq;                // [rows, H * P * D]
+  const bf16_t* kc; const bf16_t* vc;       // [blocks, bs, G * P * D], [blocks, G * Dv, bs]
+  const int* bt; int ldbt;
+  const int* positions; const int* cu; const int* work;
+  const float* mult; const float* bias; const float* sink; const float* lam;
+  const bf16_t* gate; long ldg;
+  bf16_t* out; long ldo;
+  int H, G, D, Dv, bs, window, keep, gate_heads, hpw;
+  float cap, eps, post;
+  int per, nparts;                          // tiles of a part, parts the workspace has room for
+  float* part;
+};
+
+EIA_DEV float wf_pair_max(float v) {        // with lane ^ 32
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+EIA_DEV float wf_pair_sum(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+EIA_DEV bf16x2 wf_pack(float a, float b) {  // one v_cvt_pk_bf16_f32
+  typedef __attribute__((ext_vector_type(2))) float f32x2_t;
+  return __builtin_convertvector(f32x2_t{a, b}, bf16x2);
+}
+
+// What the lanes of a workgroup work on; qn <= 0: nothing.
+struct WfRows {
+  int s, h, qn;                             // sequence, this wave's head, queries of the workgroup
+  bool live, mine;                          // the wave has a query; so has the lane
+  long row;                                 // the lane's query (the last one where it has none)
+  int p_last, w_first, w_last;              // last position of the workgroup; of the wave
+  // tiles: those of the kept first tokens that lie before the window's (nkeep), then the window's
+  // from key lo on
+  int lo, nkeep, ntile;
+};
+EIA_DEV WfRows wf_rows(const FlashArgs& a, int w, int r32) {
+  WfRows r;
+  r.s = a.work[2 * blockIdx.y];
+  const int q0 = a.work[2 * blockIdx.y + 1], qbeg = a.cu[r.s], qlen = a.cu[r.s + 1] - qbeg;
+  r.qn = min(WF_ROWS / a.hpw, qlen - q0);
+  r.h = blockIdx.x * a.hpw + w % a.hpw;
+  if (r.qn <= 0) return r;
+  const int wq0 = q0 + 32 * (w / a.hpw);
+  r.live = wq0 < qlen;
+  r.mine = wq0 + r32 < qlen;
+  r.row = qbeg + min(wq0 + r32, qlen - 1);
+  const int p_first = a.positions[qbeg + q0];
+  r.p_last = a.positions[qbeg + q0 + r.qn - 1];
+  r.w_first = a.positions[qbeg + min(wq0, qlen - 1)];
+  r.w_last = a.positions[qbeg + min(wq0 + 31, qlen - 1)];
+  const int lo_min = a.window > 0 ? max(0, p_first - a.window + 1) : 0;
+  r.lo = lo_min & ~(WF_KEYS - 1);
+  r.nkeep = min((min(a.keep, lo_min) + WF_KEYS - 1) / WF_KEYS, r.lo / WF_KEYS);
+  r.ntile = r.nkeep + (r.p_last - r.lo) / WF_KEYS + 1;
+  return r;
+}
+
+// Wave w's place for part z of the workgroup's rows: 4 NDV + 1 units of 64 lanes x 4 floats.
+EIA_DEV float* wf_part(const FlashArgs& a, int z, int w, int ndv) {
+  const long wg = (long)blockIdx.y * gridDim.x + blockIdx.x;
+  return a.part + ((wg * a.nparts + z) * 4 + w) * (4 * ndv + 1) * 256;
+}
+
+// From a lane's sums to its outputs: columns 32 dt + 8 j + 4 hh + i of its query.
+template <int P, int NDV>
+EIA_DEV void wf_finish(const FlashArgs& a, const WfRows& rw, int hh, const f32x16_t (&o)[NDV], float lsum) {
+  const int Dv = a.Dv, h = rw.h;
+  const long row = rw.row;
+  float inv = a.post / lsum;
+  if constexpr (P == 2) {                   // root mean square of the head (columns past Dv are zero)
+    float ss = 0.f;
+#pragma unroll
+    for (int dt = 0; dt < NDV; ++dt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) ss += o[dt][i] * o[dt][i];
+    inv = a.post / sqrtf(wf_pair_sum(ss) / (float)Dv + a.eps);
+  } else if (a.gate && a.gate_heads) {
+    inv *= 1.0f / (1.0f + __expf(-bf2f(a.gate[row * a.ldg + h])));
+  }
+  if (!rw.mine) return;
+  bf16_t* op = a.out + row * a.ldo + (long)h * Dv + 4 * hh;
+#pragma unroll
+  for (int dt = 0; dt < NDV; ++dt)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int c = 32 * dt + 8 * j;
+      if (c >= Dv) continue;                // (Dv % 16 == 0)
+      bf16x4 o4;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float v = o[dt][4 * j + i] * inv;
+        if (P == 1 && a.gate && !a.gate_heads)
+          v *= 1.0f / (1.0f + __expf(-bf2f(a.gate[row * a.ldg + (long)h * Dv + 4 * hh + c + i])));
+        o4[i] = f2bf(v);
+      }
+      *reinterpret_cast<bf16x4*>(op + c) = o4;
+    }
+}
+
+// P: score maps per head (2: a differential pair).  ND: 16-channel steps of a map (D <= 16 ND), NDV:
+// 32-column tiles of the values (Dv <= 32 NDV).  SIG: sigmoid weights, not normalised.
+// With P == 2 there are eight waves, four for each map of the same rows; the first four finish them.
+// SPLIT: a row block of more than a.per tiles is cut over grid.z, the parts meet in
+// window_flash_merge_kernel.
+template <int P, int ND, int NDV, bool SIG, bool SPLIT>
+__global__ void __launch_bounds__(256 * P, 2)
+window_flash_kernel(FlashArgs a) {
+  constexpr int NT = 256 * P;
+  constexpr int KW = P * 16 * ND, KS = KW + 8, VS = WF_KEYS + 8;
+  constexpr int KBUF = WF_KEYS * KS, BUF = KBUF + 32 * NDV * VS;
+  constexpr int NKU = WF_KEYS * KW / 8 / NT, NVU = 32 * NDV * WF_KEYS / 8 / NT;   // 16-byte units per thread
+  extern __shared__ __align__(16) bf16_t wf_lds[];      // 2 * BUF
+  const int tid = threadIdx.x, lane = tid & 63, grp = tid >> 8, w = (tid >> 6) & 3;
+  const int r32 = lane & 31, hh = lane >> 5, map = P == 2 ? grp : 0;
+  const WfRows rw = wf_rows(a, w, r32);
+  if (rw.qn <= 0) return;                               // (whole workgroup)
+  const int D = a.D, Dv = a.Dv, bs = a.bs, kvh = blockIdx.x * a.hpw / (a.H / a.G), h = rw.h;
+  const long row = rw.row;
+  const int qpos = a.positions[row], p_last = rw.p_last, w_first = rw.w_first, w_last = rw.w_last;
+  const bool live = rw.live;
+  const int lo = rw.lo, nkeep = rw.nkeep;
+  const int parts = SPLIT ? min(a.nparts, (rw.ntile + a.per - 1) / a.per) : 1;
+  if (SPLIT && (int)blockIdx.z >= parts) return;        // (whole workgroup)
+  // (equal parts)
+  const int it0 = SPLIT ? rw.ntile * blockIdx.z / parts : 0;
+  const int it1 = SPLIT ? rw.ntile * (blockIdx.z + 1) / parts : rw.ntile;
+  auto tile_key = [&](int it) { return it < nkeep ? it * WF_KEYS : lo + (it - nkeep) * WF_KEYS; };
+
+  bf16x8 qf[ND];
+  const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+  for (int t = 0; t < ND; ++t) {
+    const int d = 16 * t + 8 * hh;
+    const bf16x8 v = *reinterpret_cast<const bf16x8*>(a.q + row * a.ldq + (long)(h * P + map) * D + (d < D ? d : 0));
+    qf[t] = d < D ? v : zero8;
+  }
+  // base-2 scores are raw * ml (a negative multiplier changes the sign of the query instead, so that
+  // the largest raw score is the largest score); soft-capped scores are formed in base 2 at once
+  float ml = a.mult[h * P + map] * WF_LOG2E;
+  if (ml < 0.f) {
+    ml = -ml;
+#pragma unroll
+    for (int t = 0; t < ND; ++t) qf[t] = -qf[t];
+  }
+  const float capl = a.cap * WF_LOG2E, icap = a.cap > 0.f ? 2.f * ml / a.cap : 0.f;
+  const float sc = a.cap > 0.f ? 1.f : fmaxf(ml, 1e-30f);
+
+  const int* bt = a.bt + (long)rw.s * a.ldbt;
+  const long krow = (long)a.G * P * D, vpage = (long)a.G * Dv * bs;
+  bf16x8 kst[NKU], vst[NVU];
+  // (nothing may look at the values before stash: the loads are in flight during a whole tile)
+  auto fetch = [&](int kb) {
+    const long page = bt[kb / bs];
+    const bf16_t* kp = a.kc + (page * bs + kb % bs) * krow + (long)kvh * P * D;
+    const bf16_t* vp = a.vc + page * vpage + (long)kvh * Dv * bs + kb % bs;
+#pragma unroll
+    for (int i = 0; i < NKU; ++i) {
+      const int u = tid + NT * i, m = u % (KW / 8) / (2 * ND), d = 8 * (u % (KW / 8) % (2 * ND));
+      kst[i] = *reinterpret_cast<const bf16x8*>(kp + u / (KW / 8) * krow + m * D + (d < D ? d : 0));
+    }
+#pragma unroll
+    for (int i = 0; i < NVU; ++i) {
+      const int u = tid + NT * i, c = u >> 3;
+      vst[i] = *reinterpret_cast<const bf16x8*>(vp + (long)(c < Dv ? c : 0) * bs + 8 * (u & 7));
+    }
+  };
+  auto stash = [&](int buf, int kb) {
+    bf16_t* kl = wf_lds + buf * BUF;
+#pragma unroll
+    for (int i = 0; i < NKU; ++i) {
+      const int u = tid + NT * i;
+      *reinterpret_cast<bf16x8*>(kl + u / (KW / 8) * KS + 8 * (u % (KW / 8))) =
+          8 * (u % (KW / 8) % (2 * ND)) < D ? kst[i] : zero8;
+    }
+    if (kb + WF_KEYS > p_last + 1) {        // (slots behind the last key may hold anything: 0 x inf)
+#pragma unroll
+      for (int i = 0; i < NVU; ++i)
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (kb + 8 * ((tid + NT * i) & 7) + e > p_last) vst[i][e] = (bf16_t)0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < NVU; ++i) {
+      const int u = tid + NT * i;
+      *reinterpret_cast<bf16x8*>(kl + KBUF + (u >> 3) * VS + 8 * (u & 7)) = u >> 3 < Dv ? vst[i] : zero8;
+    }
+  };
+
+  f32x16_t oacc[NDV];
+#pragma unroll
+  for (int dt = 0; dt < NDV; ++dt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) oacc[dt][i] = 0.f;
+  const bool snk = !SIG && a.sink && it0 == 0;
+  float m_run = snk ? a.sink[h * P + map] * WF_LOG2E : -1e30f;
+  float l_run = snk && hh == 0 ? 1.f : 0.f;
+  const float bl = SIG && a.bias ? a.bias[h] * WF_LOG2E : 0.f;
+  const int krow0 = (r32 & ~12) | ((r32 & 4) << 1) | ((r32 & 8) >> 1);
+
+  auto compute = [&](int buf, int kb) {
+    const bf16_t* kf0 = wf_lds + buf * BUF + krow0 * KS + map * 16 * ND + 8 * hh;
+    const bf16_t* vf0 = wf_lds + buf * BUF + KBUF + r32 * VS + 8 * hh;
+    f32x16_t sacc[2];
+#pragma unroll
+    for (int sh = 0; sh < 2; ++sh)
+#pragma unroll
+      for (int t = 0; t < ND; ++t) {
+        const bf16x8 kf = *reinterpret_cast<const bf16x8*>(kf0 + 32 * KS * sh + 16 * t);
+        sacc[sh] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[t], t == 0 ? f32x16_t{} : sacc[sh], 0, 0, 0);
+      }
+    // element i of half sh is key kb + 32 sh + 16 (i >> 3) + 8 hh + (i & 7)
+    if (a.cap > 0.f) {                      // cap tanh(s / cap) = cap - 2 cap / (exp(2 s / cap) + 1)
+#pragma unroll
+      for (int sh = 0; sh < 2; ++sh)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          sacc[sh][i] = fmaf(-2.f * capl, __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(sacc[sh][i] * icap) + 1.f), capl);
+    }
+    // every query of the wave sees every key of the tile?
+    if (kb + WF_KEYS - 1 > w_first ||
+        (a.window > 0 && w_last - kb >= a.window && kb + WF_KEYS > a.keep)) {
+      const int d0 = qpos - kb - 8 * hh;
+      const int win = a.window > 0 ? a.window : 0x7fffffff, kp = a.keep - kb - 8 * hh;
+#pragma unroll
+      for (int sh = 0; sh < 2; ++sh)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int j = 32 * sh + 16 * (i >> 3) + (i & 7);
+          sacc[sh][i] = d0 >= j && (d0 - j < win || j < kp) ? sacc[sh][i] : -INFINITY;
+        }
+    }
+    float muse = 0.f;
+    if constexpr (!SIG) {
+      float mx4[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        mx4[c] = sacc[c >> 1][8 * (c & 1)];
+#pragma unroll
+        for (int j = 1; j < 8; ++j) mx4[c] = fmaxf(mx4[c], sacc[c >> 1][8 * (c & 1) + j]);
+      }
+      const float mt = wf_pair_max(fmaxf(fmaxf(mx4[0], mx4[1]), fmaxf(mx4[2], mx4[3]))) * sc;
+      const bool grow = mt > m_run + WF_DEFER;
+      if (__any(grow)) {
+        const float m_new = grow ? mt : m_run;
+        const float alpha = grow ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.f;
+        m_run = m_new;
+        l_run *= alpha;
+#pragma unroll
+        for (int dt = 0; dt < NDV; ++dt) oacc[dt] *= alpha;
+      }
+      muse = m_run;
+    }
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      bf16x8 ph, pl;
+      float ps = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; j += 2) {
+        float p[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const float x = sacc[ks >> 1][8 * (ks & 1) + j + e];
+          if constexpr (SIG) p[e] = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(fmaf(-x, sc, -bl)));
+          else p[e] = __builtin_amdgcn_exp2f(fmaf(x, sc, -muse));
+        }
+        ps += p[0] + p[1];
+        const bf16x2 hi = wf_pack(p[0], p[1]);
+        const unsigned hb = __builtin_bit_cast(unsigned, hi);
+        const bf16x2 lw = wf_pack(p[0] - __uint_as_float(hb << 16), p[1] - __uint_as_float(hb & 0xffff0000u));
+        ph[j] = hi[0]; ph[j + 1] = hi[1];
+        pl[j] = lw[0]; pl[j + 1] = lw[1];
+      }
+      l_run += ps;
+#pragma unroll
+      for (int dt = 0; dt < NDV; ++dt) {
+        const bf16x8 vf = *reinterpret_cast<const bf16x8*>(vf0 + 32 * VS * dt + 16 * ks);
+        oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, ph, oacc[dt], 0, 0, 0);
+        oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pl, oacc[dt], 0, 0, 0);
+      }
+    }
+  };
+
+  fetch(tile_key(it0));
+  stash(0, tile_key(it0));
+  __syncthreads();
+  for (int it = it0; it < it1; ++it) {
+    const int kb = tile_key(it);
+    const bool more = it + 1 < it1;
+    if (more) fetch(tile_key(it + 1));
+    // does any query of the wave see a key of the tile?
+    if (live && kb <= w_last && (a.window <= 0 || w_first - (kb + WF_KEYS - 1) < a.window || kb < a.keep))
+      compute((it - it0) & 1, kb);
+    if (more) stash((it - it0 + 1) & 1, tile_key(it + 1));
+    __syncthreads();
+  }
+  float lsum = SIG ? 1.f : wf_pair_sum(l_run);
+  if (SPLIT && parts > 1) {
+    float* x = wf_part(a, blockIdx.z, w, NDV) + 4 * lane;
+#pragma unroll
+    for (int dt = 0; dt < NDV; ++dt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<f32x4*>(x + (4 * dt + i) * 256) =
+            f32x4{oacc[dt][4 * i], oacc[dt][4 * i + 1], oacc[dt][4 * i + 2], oacc[dt][4 * i + 3]};
+    *reinterpret_cast<f32x4*>(x + 4 * NDV * 256) = f32x4{m_run, lsum, 0.f, 0.f};
+    return;
+  }
+  if constexpr (P == 2) {                               // a1 - lam a2
+    float* x = reinterpret_cast<float*>(wf_lds) + (w * 16 * NDV) * 64 + lane;
+    if (grp == 1) {
+      const float w1 = -a.lam[0] / lsum;
+#pragma unroll
+      for (int dt = 0; dt < NDV; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) x[(16 * dt + i) * 64] = oacc[dt][i] * w1;
+    }
+    __syncthreads();
+    if (grp == 1) return;
+    const float w0 = 1.f / lsum;
+    lsum = 1.f;
+#pragma unroll
+    for (int dt = 0; dt < NDV; ++dt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) oacc[dt][i] = oacc[dt][i] * w0 + x[(16 * dt + i) * 64];
+  }
+  wf_finish<P, NDV>(a, rw, hh, oacc, lsum);
+}
+
+// The parts of a row block put together: the workgroups, lanes and registers of the kernel above.
+template <int NDV, bool SIG>
+__global__ void __launch_bounds__(256)
+window_flash_merge_kernel(FlashArgs a) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const WfRows rw = wf_rows(a, w, lane & 31);
+  const int parts = min(a.nparts, (rw.ntile + a.per - 1) / a.per);
+  if (rw.qn <= 0 || parts <= 1 || !rw.live) return;
+  float m = -INFINITY, lsum = 0.f;
+  f32x16_t oacc[NDV];
+#pragma unroll
+  for (int dt = 0; dt < NDV; ++dt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) oacc[dt][i] = 0.f;
+  for (int z = 0; z < parts; ++z) {
+    const float* x = wf_part(a, z, w, NDV) + 4 * lane;
+    const f32x4 ml = *reinterpret_cast<const f32x4*>(x + 4 * NDV * 256);
+    float w0 = 1.f, w1 = 1.f;
+    if constexpr (!SIG) {
+      const float mn = fmaxf(m, ml[0]);
+      w0 = __builtin_amdgcn_exp2f(m - mn);
+      w1 = __builtin_amdgcn_exp2f(ml[0] - mn);
+      m = mn;
+    }
+    lsum = SIG ? 1.f : lsum * w0 + ml[1] * w1;
+#pragma unroll
+    for (int dt = 0; dt < NDV; ++dt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(x + (4 * dt + i) * 256);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) oacc[dt][4 * i + e] = oacc[dt][4 * i + e] * w0 + v[e] * w1;
+      }
+  }
+  wf_finish<1, NDV>(a, rw, lane >> 5, oacc, lsum);
+}
+
+template <int P, int ND, int NDV, bool SIG, bool SPLIT>
+static void wf_launch(const FlashArgs& a, int n_items, int parts, hipStream_t st) {
+  constexpr int BYTES = 4 * (WF_KEYS * (P * 16 * ND + 8) + 32 * NDV * (WF_KEYS + 8));
+  static_assert(P == 1 || BYTES >= 4 * 4 * 64 * 16 * NDV, "room to hand rows over");
+  auto* f = &window_flash_kernel<P, ND, NDV, SIG, SPLIT>;
+  if (BYTES > 64 * 1024)
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(f), hipFuncAttributeMaxDynamicSharedMemorySize, BYTES);
+  hipLaunchKernelGGL(f, dim3(a.H / a.hpw, n_items, parts), dim3(256 * P), BYTES, st, a);
+  if (SPLIT)
+    hipLaunchKernelGGL((window_flash_merge_kernel<NDV, SIG>), dim3(a.H / a.hpw, n_items), dim3(256), 0, st, a);
+}
+
+template <int P, int ND, int NDV, bool SIG>
+static void wf_go(const FlashArgs& a, int n_items, int parts, hipStream_t st) {
+  if constexpr (P == 1) {
+    if (parts > 1) {
+      wf_launch<P, ND, NDV, SIG, true>(a, n_items, parts, st);
+      return;
+    }
+  }
+  wf_launch<P, ND, NDV, SIG, false>(a, n_items, 1, st);
+}
+
+}  // namespace
+
+// Queries per work item of eia_window_flash, 0 where it does not take the shape.
+EIA_API int eia_window_flash_queries(int H, int G, int P, int D, int Dv, int bs) {
+  if (G < 1 || H < 1 || H % G || (P != 1 && P != 2) || D < 8 || D % 8 || Dv < 16 || Dv % 16 ||
+      D > (P == 2 ? 64 : 128) || Dv > 128 || bs < 64 || bs % 64)
+    return 0;
+  const int rep = H / G;
+  return WF_ROWS / (rep % 4 == 0 ? 4 : rep % 2 == 0 ? 2 : 1);
+}
+
+// Prompt portions of window attention without head mixing or slopes; the arguments are those of
+// eia_window_attn_mfma, work holds blocks of eia_window_flash_queries queries.  nparts > 1 (P == 1):
+// row blocks of more than per 64-key tiles are cut into parts of at most that many (nparts * per
+// tiles cover the longest), which meet in part [n_items * H / hpw, nparts, 4, 4 ceil(Dv / 32) + 1,
+// 256] fp32, hpw = 128 / queries (Dv counted as 128 where D > 96 or Dv > 96 or D <= 64 < Dv).
+EIA_API int eia_window_flash(const void* q, long ldq, const void* kc, const void* vc, const int* bt,
+                             int ldbt, const int* positions, const int* cu, const int* work,
+                             int n_items, const float* mult, const void* gate, long ldg, void* out,
+                             long ldo, int H, int G, int P, int D, int Dv, int bs, int window,
+                             int keep, const float* lam, float eps, float post, int wmode,
+                             const float* bias, const float* sink, float cap, int gate_heads,
+                             int nparts, int per, float* part, hipStream_t st) {
+  if (n_items < 0 || keep < 0 || cap < 0.f || !q || !kc || !vc || !bt || !positions || !cu || !work ||
+      !mult || !out || (P == 2) != (lam != nullptr) || (P == 2 && gate) ||
+      (wmode != 0 && wmode != 1) || (wmode == 1 && (P != 1 || sink)) || ldq % 8 || ldo % 4 ||
+      nparts < 1 || (nparts > 1 && (P != 1 || per < 1 || !part)))
+    return EIA_BAD_SHAPE;
+  const int qb = eia_window_flash_queries(H, G, P, D, Dv, bs);
+  if (!qb) return EIA_UNSUPPORTED;
+  if (n_items == 0) return EIA_OK;
+  FlashArgs a{(const bf16_t*)q, ldq, (const bf16_t*)kc, (const bf16_t*)vc, bt, ldbt, positions, cu,
+              work, mult, bias, sink, lam, (const bf16_t*)gate, ldg, (bf16_t*)out, ldo, H, G, D, Dv,
+              bs, window, keep, gate_heads, WF_ROWS / qb, cap, eps, post, per, nparts, part};
+#define WF_SIZES(SG)                                                    \
+  do {                                                                  \
+    if (D <= 64 && Dv <= 64) wf_go<1, 4, 2, SG>(a, n_items, nparts, st);  \
+    else if (D <= 64) wf_go<1, 4, 4, SG>(a, n_items, nparts, st);         \
+    else if (D <= 96 && Dv <= 96) wf_go<1, 6, 3, SG>(a, n_items, nparts, st); \
+    else wf_go<1, 8, 4, SG>(a, n_items, nparts, st);                      \
+  } while (0)
+  if (P == 2) wf_go<2, 4, 4, false>(a, n_items, nparts, st);
+  else if (wmode == 1) WF_SIZES(true);
+  else WF_SIZES(false);
+#undef WF_SIZES
+  EIA_LAUNCH_CHECK();
+}

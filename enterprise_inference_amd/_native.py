@@ -103,6 +103,9 @@ _SIGNATURES = {
                         I, I, I, I, I, P, F, F, I, P, P, F, I, I, I, S],
     "eia_window_attn_mfma": [P, L, P, P, IP, I, IP, IP, IP, IP, I, P, P, P, P, L, P, L, I, I, I, I,
                              I, I, I, I, I, P, F, F, I, P, I, P, P, P, F, I, S],
+    "eia_window_flash": [P, L, P, P, IP, I, IP, IP, IP, I, P, P, L, P, L, I, I, I, I, I, I, I, I, P,
+                         F, F, I, P, P, F, I, I, I, P, S],
+    "eia_window_flash_queries": [I, I, I, I, I, I],
     "eia_head_mix_attn": [P, L, P, P, IP, I, IP, IP, IP, IP, I, I, P, P, P, L, I, I, I, I, I, I, F,
                           F, I, P, P, S],
     "eia_head_mix_attn_ok": [I, I, I, I, I],

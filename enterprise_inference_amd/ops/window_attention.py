@@ -124,10 +124,48 @@ def head_mix_partitions(batch: int, spec: WindowSpec, cus: int = 256) -> int:
     return p
 
 
+def flash_queries(spec: WindowSpec, block_size: int) -> int:
+    """Queries per work item of the LDS-shared prefill kernel (window_flash.hip), 0 where a layer
+    with an MFMA form does not take it: head mixing, a distance term, a differential pair wider
+    than 64, pages that are no multiple of 64 tokens."""
+    if spec.talk is not None or spec.slope is not None:
+        return 0
+    return lib().eia_window_flash_queries(spec.heads, spec.kv_heads, spec.maps, spec.dim,
+                                          spec.vdim, block_size)
+
+
+def flash_parts(n_items: int, spec: WindowSpec, queries: int, longest: int, context: int,
+                cus: int = 256):
+    """(parts, 64-key tiles per part) of a flash prefill launch whose longest portion has
+    ``longest`` queries and whose block tables reach ``context`` tokens.  Two workgroups fit a CU.
+    Where there is not even one for each, row blocks are cut along the keys: where they are about
+    equally long (a window, or a portion behind a long context) into as many parts as there is room
+    for, from three on; where they grow from nothing (causal) so that a part is about 1/640 of all
+    tiles.  Fewer than twelve tiles are not worth the second launch.  MI355X, 8 heads of 128 on 2,
+    one portion, uncut / cut: 4096 tokens causal 126 / 99 us, 2048 62 / 43, 1000 34 / 29, 500 23 /
+    28, 96 behind 2000 64 / 32; 16 heads on 4: 4096 causal (512 workgroups) 147 / 158, 1000 behind
+    1900 88 / 58, 500 behind 1000 with a window of 1024 47 / 30, 2000 with it (252) 51 / 56."""
+    wgs = max(1, n_items * (spec.heads * queries // 128))
+    tiles = -(-context // 64)
+    if spec.window > 0:
+        tiles = min(tiles, (spec.window + queries + 62) // 64 + 1 + (spec.keep + 63) // 64)
+    mean = tiles if spec.window > 0 else max(1, tiles - longest // 128)
+    if spec.maps == 2 or wgs > cus or tiles < 12:
+        return 1, tiles
+    if 4 * mean >= 3 * tiles:
+        per = -(-tiles // (2 * cus // wgs)) if 3 * wgs <= 2 * cus else tiles
+    else:
+        per = -(-wgs * mean // 640)
+    per = max(6, per)
+    return -(-tiles // per), per
+
+
 def query_block(spec: WindowSpec, dtype: torch.dtype, block_size: int) -> int:
     if not mfma_ok(spec, dtype, block_size):
         return SCALAR_QB
-    return HEAD_MIX_QB if spec.talk_post else MFMA_QB
+    if spec.talk_post:
+        return HEAD_MIX_QB
+    return flash_queries(spec, block_size) or MFMA_QB
 
 
 def _rms(v: torch.Tensor, eps: float) -> torch.Tensor:
@@ -538,6 +576,22 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
                 ptr(spec.mult), ptr(spec.talk), ptr(o), o.stride(0), H, spec.kv_heads, D, Dv, bs,
                 spec.window, float(spec.cap), float(spec.post), NP, ptr(acc), ptr(ml), stream(q)),
                 "head_mix_attn")
+            return
+        if mfma and cu is not None and flash_queries(spec, bs):
+            NP, per = flash_parts(n_items, spec, qb, max(md.prefill_q_lens or [T]), bt.shape[1] * bs)
+            pa = None
+            if NP > 1:
+                vt = 4 if max(D, Dv) > 96 or D <= 64 < Dv else -(-max(D, Dv) // 32)
+                pa = torch.empty(n_items * (H * qb // 128) * NP * 4 * (4 * vt + 1) * 256,
+                                 dtype=torch.float32, device=q.device)
+            check(lib().eia_window_flash(
+                ptr(qa), qa.stride(0), ptr(k_cache), ptr(v_cache), ptr(bt), bt.stride(0),
+                ptr(md.positions[lo:]), ptr(cu), ptr(work), n_items, ptr(spec.mult), ptr(g),
+                g.stride(0) if g is not None else 0, ptr(o), o.stride(0), H, spec.kv_heads, P, D,
+                Dv, bs, spec.window, spec.keep, ptr(spec.lam) if P == 2 else None,
+                float(spec.eps), float(spec.post), spec.weights, ptr(spec.bias), ptr(spec.sink),
+                float(spec.cap), 1 if spec.gate_heads else 0, NP, per, ptr(pa), stream(q)),
+                "window_flash")
             return
         if mfma:
             NP = decode_partitions(n_items, spec) if cu is None else 1

@@ -1,0 +1,80 @@
+"""The LDS-shared prefill form of window attention against the op's own plain CPU path: group sizes,
+padded head sizes, windows and kept tokens on both sides of a 64-key tile, prompts that continue."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _spec(wa, kind, H, G, D, Dv, window, dev):
+    g = torch.Generator().manual_seed(3)
+    P = 2 if kind == "pair" else 1
+    s = wa.WindowSpec(H, G, P, D, Dv, window, 0, mult=torch.linspace(0.5, 1.5, H * P) * D ** -0.5)
+    if kind == "cap":
+        s.cap, s.sink, s.post = 5.0, torch.randn(H, generator=g), 0.8
+    elif kind == "sigmoid":
+        s.weights, s.bias = 1, torch.randn(H, generator=g) - 3.0
+    elif kind == "pair":
+        s.keep, s.epilogue, s.eps, s.post, s.lam = 70, 1, 1e-5, 0.7, torch.tensor([0.4])
+    elif kind == "keep":
+        s.keep = 4
+    for f in ("mult", "sink", "bias", "lam"):
+        t = getattr(s, f)
+        if t is not None:
+            setattr(s, f, t.to(dev))
+    return s
+
+
+@pytest.mark.parametrize("kind", ["plain", "cap", "sigmoid", "pair", "keep"])
+@pytest.mark.parametrize("H,G,D,Dv,bs", [(4, 1, 128, 128, 64), (6, 3, 72, 48, 128), (3, 1, 64, 64, 64),
+                                         (8, 2, 96, 96, 64), (2, 2, 64, 112, 64)])
+@pytest.mark.parametrize("window,new,past", [(0, [1, 200, 33, 65], [0, 0, 190, 63]),
+                                             (50, [1, 200, 33, 65], [0, 0, 190, 63]),
+                                             (130, [1, 200, 33, 65], [0, 0, 190, 63]),
+                                             (0, [40, 7], [1000, 130])])
+def test_window_flash(window, new, past, H, G, D, Dv, bs, kind):
+    from enterprise_inference_amd.ops import attention as A
+    from enterprise_inference_amd.ops import window_attention as wa
+    if kind == "pair":
+        D = 64 if D > 64 else 40
+    g = torch.Generator().manual_seed(H + D + window)
+    P = 2 if kind == "pair" else 1
+    pages = [-(-(a + b) // bs) for a, b in zip(new, past)]
+    order = torch.randperm(sum(pages), generator=g).to(torch.int32)
+    bt = torch.zeros(len(new), max(pages), dtype=torch.int32)
+    at = 0
+    for s, n in enumerate(pages):
+        bt[s, :n] = order[at:at + n]
+        at += n
+    cu = torch.tensor([0] + new).cumsum(0).to(torch.int32)
+    pos = torch.cat([torch.arange(n) + f for n, f in zip(new, past)]).to(torch.int32)
+    T = int(cu[-1])
+    bf = torch.bfloat16
+    rnd = lambda *s: torch.randn(*s, generator=g).to(bf)
+    q, k, v = rnd(T, H * P * D), rnd(sum(pages), bs, G * P * D), rnd(sum(pages), G * Dv, bs)
+    for s, (a, b) in enumerate(zip(new, past)):              # slots behind a sequence hold anything
+        last, used = int(bt[s, pages[s] - 1]), (a + b - 1) % bs + 1
+        k[last, used:] = float("nan")
+        v[last, :, used:] = float("nan")
+    gate = None if kind == "pair" else rnd(T, H if kind == "cap" else H * Dv)
+
+    def run(dev):
+        md = A.AttentionMetadata(
+            num_decode=0, num_prefill_tokens=T, slot_mapping=pos.to(dev), positions=pos.to(dev),
+            prefill_block_tables=bt.to(dev), prefill_cu_q=cu.to(dev), prefill_q_lens=new)
+        spec = _spec(wa, kind, H, G, D, Dv, window, dev)
+        spec.gate_heads = kind == "cap"
+        if dev == "cuda":
+            qb = wa.query_block(spec, bf, bs)
+            assert qb == 128 // {1: 1, 2: 2, 3: 1, 4: 4}[H // G]
+            n = sum(-(-a // qb) for a in new)           # (the long context is cut into parts)
+            assert (wa.flash_parts(n, spec, qb, max(new), bt.shape[1] * bs)[0] > 1) == (
+                max(past) > 900 and P == 1)
+        return wa.window_attention(q.to(dev), k.to(dev), v.to(dev), md, spec,
+                                   None if gate is None else gate.to(dev)).cpu()
+
+    a, b = run("cpu").double(), run("cuda").double()
+    # both sides sum in fp32 and round once to bf16 (2^-9): neighbouring roundings at most
+    assert float((a - b).norm() / a.norm()) < 4e-3
+    assert float(((a - b).abs() / (a.abs() + 0.05 * a.abs().mean())).max()) < 2 ** -6

@@ -653,41 +653,30 @@ latent_merge_kernel(const float* __restrict__ part_acc, const float* __restrict_
   }
 }
 
-// Rows per work item of the MFMA form: NW waves x 16; HB = min(H, 16) heads, QB = rows / HB
-// queries.  Returns QB for (H, prefill) so the host builds its work list with the same number.
-EIA_API int eia_latent_attn_mfma_qb(int H, int decode) {
-  const int HB = H < 16 ? H : 16;
-  return decode ? 1 : (64 / HB);
-}
-
+// Decode rows (one query each); prompt portions: latent_flash.hip.
 EIA_API int eia_latent_attn_mfma(const void* qa, long qa_st, long qa_sh, const void* qr,
                                  long qr_st, long qr_sh, const float* inv_freq, int rot_dims,
                                  const void* cache, long cache_row, const int* block_table,
-                                 int bt_stride, const int* seq_lens, const int* cu_q,
-                                 const int* work, int n_items, const int* positions,
-                                 const void* gate, long gate_st, void* out, long out_st,
-                                 long out_sh, float scale, int H, int R, int rd, int bs, int QB,
+                                 int bt_stride, const int* seq_lens, int n_items,
+                                 const int* positions, const void* gate, long gate_st, void* out,
+                                 long out_st, long out_sh, float scale, int H, int R, int rd, int bs,
                                  int window, const float* sink, int rot_half, float rot_amp,
                                  int nparts, float* part_acc, float* part_ml, hipStream_t st) {
-  if (H < 1 || R < 1 || rd < 0 || bs < 1 || QB < 1 || rot_dims > rd || (rot_dims & 1) ||
-      cache_row < R + rd || (cu_q && !work))
+  if (H < 1 || R < 1 || rd < 0 || bs < 1 || rot_dims > rd || (rot_dims & 1) || cache_row < R + rd)
     return EIA_BAD_SHAPE;
   const int Dk = R + rd;
   // 16-byte chunks must not straddle the latent / rotary boundary or the row end
   if ((R & 7) || (Dk & 7) || (cache_row & 7) || Dk > 640 || R > 512) return EIA_UNSUPPORTED;
   if (n_items <= 0) return EIA_OK;
   const int HB = H < 16 ? H : 16;
-  const bool decode = cu_q == nullptr;
-  if (QB != eia_latent_attn_mfma_qb(H, decode ? 1 : 0)) return EIA_BAD_SHAPE;
-  if (nparts < 1 || nparts > 64 || (nparts > 1 && (!decode || !part_acc || !part_ml)))
-    return EIA_BAD_SHAPE;
+  if (nparts < 1 || nparts > 64 || (nparts > 1 && (!part_acc || !part_ml))) return EIA_BAD_SHAPE;
   const int nk = (Dk + 31) / 32, Dkp = nk * 32, nc = (R + 15) / 16;
   const int ldk = ((Dkp / 8) & 1) ? Dkp : Dkp + 8;       // odd number of 16-byte units per row
-  // K tile, V^T tile, and the rotated rotary query parts of up to 64 rows
-  const size_t lds = ((size_t)32 * ldk + (size_t)nc * 16 * 40 + (size_t)64 * rd) * 2;
+  // K tile, V^T tile, and the rotated rotary query parts of up to 16 rows
+  const size_t lds = ((size_t)32 * ldk + (size_t)nc * 16 * 40 + (size_t)16 * rd) * 2;
   LatentAttnArgs a{qa, qa_st, qa_sh, qr, qr_st, qr_sh, inv_freq, rot_dims, cache, cache_row,
-                   block_table, bt_stride, seq_lens, cu_q, work, n_items, positions, gate, gate_st,
-                   out, out_st, out_sh, scale, H, R, rd, bs, QB, HB, 32, ldk, window, sink, rot_half,
+                   block_table, bt_stride, seq_lens, nullptr, nullptr, n_items, positions, gate, gate_st,
+                   out, out_st, out_sh, scale, H, R, rd, bs, 1, HB, 32, ldk, window, sink, rot_half,
                    rot_amp, nparts, part_acc, part_ml};
   dim3 grid(n_items, (H + HB - 1) / HB, nparts);
 #define LAT_MFMA(NK, NC, SV)                                                                \
@@ -698,15 +687,9 @@ EIA_API int eia_latent_attn_mfma(const void* qa, long qa_st, long qa_sh, const v
           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);                            \
     hipLaunchKernelGGL((latent_attn_mfma_kernel<NK, NC, 4, SV>), grid, dim3(256), lds, st, a); \
   } while (0)
-  if (decode) {
-    if (nk <= 6 && nc <= 8) LAT_MFMA(6, 8, true);
-    else if (nk <= 12 && nc <= 16) LAT_MFMA(12, 16, true);
-    else LAT_MFMA(20, 32, true);
-  } else {
-    if (nk <= 6 && nc <= 8) LAT_MFMA(6, 8, false);
-    else if (nk <= 12 && nc <= 16) LAT_MFMA(12, 16, false);
-    else LAT_MFMA(20, 32, false);
-  }
+  if (nk <= 6 && nc <= 8) LAT_MFMA(6, 8, true);
+  else if (nk <= 12 && nc <= 16) LAT_MFMA(12, 16, true);
+  else LAT_MFMA(20, 32, true);
 #undef LAT_MFMA
   if (nparts > 1)
     hipLaunchKernelGGL(latent_merge_kernel, dim3(n_items, H), dim3(128), 0, st, part_acc, part_ml,

@@ -21,16 +21,12 @@
 // MI355X (249 us in the 16-query form); one 4096-token causal prompt, 8 heads on 2: 79 + 16 us in
 // parts (459 us), 126 us uncut -- a tile takes a lone workgroup 2.0 us, of which its matrix products
 // are 0.64 us; where two workgroups share a CU their products and exponentials overlap.
-#include "eia_common.h"
+#include "eia_flash.h"
 
 namespace {
 
-typedef __attribute__((ext_vector_type(16))) float f32x16_t;
-
 constexpr int WF_KEYS = 64;                 // keys per tile
 constexpr int WF_ROWS = 128;                // (query, head) rows per workgroup
-constexpr float WF_LOG2E = 1.4426950408889634f;
-constexpr float WF_DEFER = 8.f;             // log2 by which a tile may exceed the running maximum
 
 struct FlashArgs {
   const bf16_t* q; long ldq;                // [rows, H * P * D]
@@ -45,20 +41,6 @@ struct FlashArgs {
   int per, nparts;                          // tiles of a part, parts the workspace has room for
   float* part;
 };
-
-EIA_DEV float wf_pair_max(float v) {        // with lane ^ 32
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-EIA_DEV float wf_pair_sum(float v) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
-EIA_DEV bf16x2 wf_pack(float a, float b) {  // one v_cvt_pk_bf16_f32
-  typedef __attribute__((ext_vector_type(2))) float f32x2_t;
-  return __builtin_convertvector(f32x2_t{a, b}, bf16x2);
-}
 
 // What the lanes of a workgroup work on; qn <= 0: nothing.
 struct WfRows {
@@ -110,7 +92,7 @@ EIA_DEV void wf_finish(const FlashArgs& a, const WfRows& rw, int hh, const f32x1
     for (int dt = 0; dt < NDV; ++dt)
 #pragma unroll
       for (int i = 0; i < 16; ++i) ss += o[dt][i] * o[dt][i];
-    inv = a.post / sqrtf(wf_pair_sum(ss) / (float)Dv + a.eps);
+    inv = a.post / sqrtf(flash_pair_sum(ss) / (float)Dv + a.eps);
   } else if (a.gate && a.gate_heads) {
     inv *= 1.0f / (1.0f + __expf(-bf2f(a.gate[row * a.ldg + h])));
   }
@@ -173,13 +155,13 @@ window_flash_kernel(FlashArgs a) {
   }
   // base-2 scores are raw * ml (a negative multiplier changes the sign of the query instead, so that
   // the largest raw score is the largest score); soft-capped scores are formed in base 2 at once
-  float ml = a.mult[h * P + map] * WF_LOG2E;
+  float ml = a.mult[h * P + map] * FLASH_LOG2E;
   if (ml < 0.f) {
     ml = -ml;
 #pragma unroll
     for (int t = 0; t < ND; ++t) qf[t] = -qf[t];
   }
-  const float capl = a.cap * WF_LOG2E, icap = a.cap > 0.f ? 2.f * ml / a.cap : 0.f;
+  const float capl = a.cap * FLASH_LOG2E, icap = a.cap > 0.f ? 2.f * ml / a.cap : 0.f;
   const float sc = a.cap > 0.f ? 1.f : fmaxf(ml, 1e-30f);
 
   const int* bt = a.bt + (long)rw.s * a.ldbt;
@@ -229,9 +211,9 @@ window_flash_kernel(FlashArgs a) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) oacc[dt][i] = 0.f;
   const bool snk = !SIG && a.sink && it0 == 0;
-  float m_run = snk ? a.sink[h * P + map] * WF_LOG2E : -1e30f;
+  float m_run = snk ? a.sink[h * P + map] * FLASH_LOG2E : -1e30f;
   float l_run = snk && hh == 0 ? 1.f : 0.f;
-  const float bl = SIG && a.bias ? a.bias[h] * WF_LOG2E : 0.f;
+  const float bl = SIG && a.bias ? a.bias[h] * FLASH_LOG2E : 0.f;
   const int krow0 = (r32 & ~12) | ((r32 & 4) << 1) | ((r32 & 8) >> 1);
 
   auto compute = [&](int buf, int kb) {
@@ -275,8 +257,8 @@ window_flash_kernel(FlashArgs a) {
 #pragma unroll
         for (int j = 1; j < 8; ++j) mx4[c] = fmaxf(mx4[c], sacc[c >> 1][8 * (c & 1) + j]);
       }
-      const float mt = wf_pair_max(fmaxf(fmaxf(mx4[0], mx4[1]), fmaxf(mx4[2], mx4[3]))) * sc;
-      const bool grow = mt > m_run + WF_DEFER;
+      const float mt = flash_pair_max(fmaxf(fmaxf(mx4[0], mx4[1]), fmaxf(mx4[2], mx4[3]))) * sc;
+      const bool grow = mt > m_run + FLASH_DEFER;
       if (__any(grow)) {
         const float m_new = grow ? mt : m_run;
         const float alpha = grow ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.f;
@@ -301,11 +283,7 @@ window_flash_kernel(FlashArgs a) {
           else p[e] = __builtin_amdgcn_exp2f(fmaf(x, sc, -muse));
         }
         ps += p[0] + p[1];
-        const bf16x2 hi = wf_pack(p[0], p[1]);
-        const unsigned hb = __builtin_bit_cast(unsigned, hi);
-        const bf16x2 lw = wf_pack(p[0] - __uint_as_float(hb << 16), p[1] - __uint_as_float(hb & 0xffff0000u));
-        ph[j] = hi[0]; ph[j + 1] = hi[1];
-        pl[j] = lw[0]; pl[j + 1] = lw[1];
+        flash_split(p[0], p[1], j, ph, pl);
       }
       l_run += ps;
 #pragma unroll
@@ -330,7 +308,7 @@ window_flash_kernel(FlashArgs a) {
     if (more) stash((it - it0 + 1) & 1, tile_key(it + 1));
     __syncthreads();
   }
-  float lsum = SIG ? 1.f : wf_pair_sum(l_run);
+  float lsum = SIG ? 1.f : flash_pair_sum(l_run);
   if (SPLIT && parts > 1) {
     float* x = wf_part(a, blockIdx.z, w, NDV) + 4 * lane;
 #pragma unroll

@@ -69,8 +69,8 @@ _SIGNATURES = {
     "eia_latent_prep": [P, L, I, I, P, P, L, I, I, P, I, I, I, P, IP, IP, P, L, F, I, F, I, I, S],
     "eia_latent_attn": [P, L, L, P, L, L, P, I, P, L, IP, I, IP, IP, IP, I, IP, P, L, P, L, L, F,
                         I, I, I, I, I, I, P, I, F, I, S],
-    "eia_latent_attn_mfma": [P, L, L, P, L, L, P, I, P, L, IP, I, IP, IP, IP, I, IP, P, L, P, L, L,
-                             F, I, I, I, I, I, I, P, I, F, I, P, P, S],
+    "eia_latent_attn_mfma": [P, L, L, P, L, L, P, I, P, L, IP, I, IP, I, IP, P, L, P, L, L, F, I, I,
+                             I, I, I, P, I, F, I, P, P, S],
     "eia_token_shift_mix": [P, P, I, P, IP, IP, I, IP, P, L, I, I, I, S],
     "eia_wkv_scan": [P, P, P, P, L, P, L, P, P, P, P, P, P, I, IP, IP, IP, IP, P, L, F, I, I, I,
                      I, I, S],
@@ -103,6 +103,11 @@ _SIGNATURES = {
                         I, I, I, I, I, P, F, F, I, P, P, F, I, I, I, S],
     "eia_window_attn_mfma": [P, L, P, P, IP, I, IP, IP, IP, IP, I, P, P, P, P, L, P, L, I, I, I, I,
                              I, I, I, I, I, P, F, F, I, P, I, P, P, P, F, I, S],
+    "eia_latent_flash": [P, L, L, P, L, L, P, I, P, L, IP, I, IP, IP, I, IP, P, L, P, L, L, F, I, I, I,
+                         I, I, P, I, F, I, I, P, S],
+    "eia_latent_flash_queries": [I, I, I],
+    "eia_latent_flash_keys": [I, I],
+    "eia_latent_flash_columns": [I, I],
     "eia_window_flash": [P, L, P, P, IP, I, IP, IP, IP, I, P, P, L, P, L, I, I, I, I, I, I, I, I, P,
                          F, F, I, P, P, F, I, I, I, P, S],
     "eia_window_flash_queries": [I, I, I, I, I, I],

@@ -98,6 +98,23 @@ def build_prefill_work(q_lens: Sequence[int], qblock: int) -> List[int]:
     return work
 
 
+def split_keys(wgs: int, tiles: int, mean: int, slots: int, least: int = 12):
+    """(parts, tiles per part) of a prefill launch of ``wgs`` workgroups that walk up to ``tiles`` and
+    on average ``mean`` key tiles, ``slots`` of which run at a time.  Where there is not one for each
+    of half the slots, row blocks are cut along the keys: where they are about equally long into as
+    many parts as there is room for, from three on; else so that a part is about 0.8 of a slot's
+    share.  Fewer than ``least`` tiles are not worth the second launch."""
+    wgs, mean = max(1, wgs), max(1, mean)
+    if 2 * wgs > slots or tiles < least:
+        return 1, tiles
+    if 4 * mean >= 3 * tiles:
+        per = -(-tiles // (slots // wgs)) if 3 * wgs <= slots else tiles
+    else:
+        per = -(-wgs * mean * 4 // (slots * 5))
+    per = max(least // 2, per)
+    return -(-tiles // per), per
+
+
 def decode_partitions(batch: int, num_kv_heads: int, num_heads: int, max_len: int,
                       cus: int = 256, max_parts: int = 8) -> int:
     """Context partitions (flash-decoding split) for a decode batch.

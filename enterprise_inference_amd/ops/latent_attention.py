@@ -18,6 +18,7 @@ from typing import List, Optional
 import torch
 
 from ._dispatch import check, lib, ptr, require, stream, use_hip
+from .attention import split_keys
 
 ACC_ROWS = 256 * 32        # csrc/kernels/latent_attention.hip: QB * HB * R <= 256 * LAT_ACC_MAX
 
@@ -41,12 +42,12 @@ _MFMA_ENV = os.environ.get("EIA_LATENT_MFMA", "1") != "0"
 
 def query_block(num_heads: int, kv_rank: int, rot_dim: int = 0,
                 dtype: torch.dtype = torch.float32) -> int:
-    """Queries per prefill work item.  MFMA form: 64 (query, head) rows per workgroup in slices
-    of min(heads, 16) heads.  Scalar form: as many queries as the per-thread accumulators and
+    """Queries per prefill work item.  MFMA form: 128 (query, head) rows per workgroup (64 of
+    wide latents) in slices of min(heads, 16) heads (latent_flash.hip).  Scalar form: as many queries as the per-thread accumulators and
     48 KiB of LDS for the staged queries allow for a 16-head slice."""
     hb = min(num_heads, 16)
     if mfma_ok(kv_rank, rot_dim, dtype):
-        return 64 // hb
+        return lib().eia_latent_flash_queries(num_heads, kv_rank, rot_dim)
     return max(1, min(16, ACC_ROWS // (hb * kv_rank), 12288 // (hb * (kv_rank + rot_dim))))
 
 
@@ -220,8 +221,29 @@ def latent_attention(q_abs: torch.Tensor, q_rot: torch.Tensor, inv_freq: torch.T
         qa, qr, o = q_abs[lo:], q_rot[lo:], out[lo:]
         g = None if gate is None else gate[lo:]
         require(bt.dtype == torch.int32 and bt.stride(1) == 1, "block tables int32")
+        if mfma and cu is not None:
+            KT = lib().eia_latent_flash_keys(R, rd)
+            hg = -(-H // 16)
+            tiles = -(-bt.shape[1] * bs // KT)
+            longest = max(md.prefill_q_lens or [T])
+            if window > 0:
+                tiles = min(tiles, (window + qb + KT - 2) // KT + 1)
+            P, per = split_keys(n_items * hg, tiles, tiles if window else tiles - longest // (2 * KT),
+                                512 if R <= 128 and R + rd <= 160 else 256, 12 * 64 // KT)
+            pa = None
+            if P > 1:
+                pa = torch.empty(n_items * hg * P * 4 * (4 * lib().eia_latent_flash_columns(R, rd) + 1) * 256,
+                                 dtype=torch.float32, device=q_abs.device)
+            check(lib().eia_latent_flash(
+                ptr(qa), qa.stride(0), qa.stride(1), ptr(qr), qr.stride(0), qr.stride(1),
+                ptr(inv_freq), rot_dims, ptr(cache), cache.shape[-1], ptr(bt), bt.stride(0), ptr(cu),
+                ptr(work), n_items, ptr(md.positions[lo:]), ptr(g),
+                g.stride(0) if g is not None else 0, ptr(o), o.stride(0), o.stride(1), float(scale),
+                H, R, rd, bs, window, ptr(sink), rh, amp, P, per, ptr(pa), stream(q_abs)),
+                "latent_flash")
+            return
         if mfma:
-            P = decode_partitions(n_items, H, window=window) if cu is None else 1
+            P = decode_partitions(n_items, H, window=window)
             pa = pm = None
             if P > 1:
                 pa = torch.empty(n_items * H * P * R, dtype=torch.float32, device=q_abs.device)
@@ -229,9 +251,9 @@ def latent_attention(q_abs: torch.Tensor, q_rot: torch.Tensor, inv_freq: torch.T
             check(lib().eia_latent_attn_mfma(
                 ptr(qa), qa.stride(0), qa.stride(1), ptr(qr), qr.stride(0), qr.stride(1),
                 ptr(inv_freq), rot_dims, ptr(cache), cache.shape[-1], ptr(bt), bt.stride(0),
-                ptr(lens), ptr(cu), ptr(work), n_items, ptr(md.positions[lo:]), ptr(g),
+                ptr(lens), n_items, ptr(md.positions[lo:]), ptr(g),
                 g.stride(0) if g is not None else 0, ptr(o), o.stride(0), o.stride(1),
-                float(scale), H, R, rd, bs, qb, window, ptr(sink), rh, amp, P, ptr(pa), ptr(pm),
+                float(scale), H, R, rd, bs, window, ptr(sink), rh, amp, P, ptr(pa), ptr(pm),
                 stream(q_abs)), "latent_attn_mfma")
             return
         check(lib().eia_latent_attn(

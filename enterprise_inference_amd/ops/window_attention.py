@@ -30,7 +30,7 @@ from typing import List, Optional
 import torch
 
 from ._dispatch import check, lib, ptr, require, stream, use_hip
-from .attention import build_prefill_work
+from .attention import build_prefill_work, split_keys
 
 SCALAR_QB = 4            # queries per prefill work item of the scalar-FMA kernel
 MFMA_QB = 16             # ... and of the MFMA kernel (one 16-row tile)
@@ -137,27 +137,18 @@ def flash_queries(spec: WindowSpec, block_size: int) -> int:
 def flash_parts(n_items: int, spec: WindowSpec, queries: int, longest: int, context: int,
                 cus: int = 256):
     """(parts, 64-key tiles per part) of a flash prefill launch whose longest portion has
-    ``longest`` queries and whose block tables reach ``context`` tokens.  Two workgroups fit a CU.
-    Where there is not even one for each, row blocks are cut along the keys: where they are about
-    equally long (a window, or a portion behind a long context) into as many parts as there is room
-    for, from three on; where they grow from nothing (causal) so that a part is about 1/640 of all
-    tiles.  Fewer than twelve tiles are not worth the second launch.  MI355X, 8 heads of 128 on 2,
-    one portion, uncut / cut: 4096 tokens causal 126 / 99 us, 2048 62 / 43, 1000 34 / 29, 500 23 /
-    28, 96 behind 2000 64 / 32; 16 heads on 4: 4096 causal (512 workgroups) 147 / 158, 1000 behind
-    1900 88 / 58, 500 behind 1000 with a window of 1024 47 / 30, 2000 with it (252) 51 / 56."""
-    wgs = max(1, n_items * (spec.heads * queries // 128))
+    ``longest`` queries and whose block tables reach ``context`` tokens; two workgroups fit a CU.
+    MI355X, 8 heads of 128 on 2, one portion, uncut / cut: 4096 tokens causal 126 / 99 us, 2048 62 /
+    43, 1000 34 / 29, 500 23 / 28, 96 behind 2000 64 / 32; 16 heads on 4: 4096 causal (512
+    workgroups) 147 / 158, 1000 behind 1900 88 / 58, 500 behind 1000 with a window of 1024 47 / 30,
+    2000 with it (252) 51 / 56."""
     tiles = -(-context // 64)
     if spec.window > 0:
         tiles = min(tiles, (spec.window + queries + 62) // 64 + 1 + (spec.keep + 63) // 64)
-    mean = tiles if spec.window > 0 else max(1, tiles - longest // 128)
-    if spec.maps == 2 or wgs > cus or tiles < 12:
+    if spec.maps == 2:
         return 1, tiles
-    if 4 * mean >= 3 * tiles:
-        per = -(-tiles // (2 * cus // wgs)) if 3 * wgs <= 2 * cus else tiles
-    else:
-        per = -(-wgs * mean // 640)
-    per = max(6, per)
-    return -(-tiles // per), per
+    return split_keys(n_items * (spec.heads * queries // 128), tiles,
+                      tiles if spec.window > 0 else tiles - longest // 128, 2 * cus)
 
 
 def query_block(spec: WindowSpec, dtype: torch.dtype, block_size: int) -> int:

@@ -14,7 +14,7 @@
 //
 //   eia_latent_prep : RMS-norm of the query latent, RMS-norm of c, rotation of k_rot, cache write
 //   eia_latent_attn : rotation of q_rot, tiled online-softmax attention, sigmoid head gate
-#include "eia_common.h"
+#include "eia_flash.h"
 
 // Entry d (< rot_dims) of a vector after the rotation by position pos: src holds the unrotated
 // vector; pairs are (2i, 2i+1), or (i, i + rot_dims/2) when half; cos and sin are times amp.
@@ -100,9 +100,11 @@ EIA_API int eia_latent_prep(const void* fused, long ld, int q_off, int q_rank, c
 }
 
 // ------------------------------------------------------------------------------------- attention
-// Key partitions a decode row uses out of the launch's grid.z: at least two 32-key units each.
+constexpr int LAT_UNIT = 64;       // keys per tile of the decode form, cut at multiples of it
+
+// Key partitions a decode row uses out of the launch's grid.z: at least one tile each.
 EIA_DEV int lat_parts(int nparts, int kmin, int kmax) {
-  return min(nparts, max(1, ((kmax - kmin + 31) >> 5) >> 1));
+  return min(nparts, (kmax - kmin + LAT_UNIT - 1) / LAT_UNIT);
 }
 
 #define LAT_ACC_MAX 32     // fp32 accumulators per thread: QB * HB * R <= 256 * LAT_ACC_MAX
@@ -335,261 +337,198 @@ EIA_API int eia_latent_attn(const void* qa, long qa_st, long qa_sh, const void* 
   EIA_LAUNCH_CHECK();
 }
 
-// --------------------------------------------------------------------------- MFMA form (bf16)
-// Flash-style kernel on v_mfma_f32_16x16x32_bf16.  A workgroup of NW waves owns NW x 16 rows
-// (row = (query, head) pair; every row reads the same keys) and walks the keys in units of 32.
-// Per unit the workgroup stages the 32 cache rows in LDS twice: row-major ("K tile", the A
-// operand of S^T = K Q^T) and transposed ("V^T tile", latent columns only, the A operand of
-// O^T = V^T P^T).  The K tile rows are stored in the order the two S^T tiles read them, so that
-// their accumulators hold, per lane, one row's scores of keys 8g..8g+7 -- exactly the B operand
-// of the second product (no shuffle, no LDS round trip for P).  Softmax weights stay fp32: P
-// is fed as a bf16 high part plus a bf16 remainder (two MFMAs), and the normaliser sums the
-// fp32 weights.  The next unit's cache rows are prefetched into registers during the products.
-// SPLITV (decode, one query): all NW waves own the SAME 16 rows (the heads of one query) and
-// each takes every NW-th latent column tile of the second product; the first product is
-// repeated per wave (decode is bound by the cache stream, not by MFMA issue), which buys NW
-// times the loading threads (so the prefetch fits) and a quarter of the accumulators.
-template <int NKMAX, int NCMAX, int NW, bool SPLITV>
-__global__ void __launch_bounds__(NW * 64)
-latent_attn_mfma_kernel(LatentAttnArgs a) {
+// ------------------------------------------------------------------------- decode rows, MFMA (bf16)
+// One workgroup of four waves per (decode row, 16 heads, key partition), v_mfma_f32_16x16x32_bf16.
+// 64 cache rows at a time are staged in LDS as they are; wave w forms the scores of keys 16 w .. + 15
+// (S^T: keys x heads), the waves exchange them through LDS, every wave forms the softmax weights of
+// all 64 keys and takes a quarter of the latent columns in O^T += C^T P^T, whose operand comes from the
+// same rows through the transposing LDS read.  Weights stay fp32: a bf16 high part plus a bf16
+// remainder (two products), and the normaliser sums the fp32 weights.  The next rows are in flight
+// during the products, the first ones during the rotation of the queries.
+//
+// Bound by latency: a row's 64-key tiles are a chain of cache loads and two barriers, and the launch
+// lasts as long as the longest partition.  MI355X, 48 rows at up to 4096 tokens, window 1024, 16
+// heads, R 512 + 64: 25 + 5 us in five partitions.  (32-key units that went through LDS twice, the
+// second time as transposed 2-byte stores, with the scores formed by every wave and sixteen
+// partitions: 91 + 21 us.)
+constexpr int lat_bufs(int NK) { return NK <= 18 ? 2 : 1; }       // tiles that fit 160 KB of LDS
+
+template <int NK, int NCW>                  // 32-entry steps of a cache row; column tiles of a wave
+__global__ void __launch_bounds__(256)
+latent_decode_kernel(LatentAttnArgs a) {
+  constexpr int NB = lat_bufs(NK), KT = LAT_UNIT;
+  constexpr int KS = 32 * NK + 8;                       // 4 NK + 1 units of 16 bytes per row
+  constexpr int SP = KT + 4;                            // pitch of the exchanged scores
   extern __shared__ __align__(16) unsigned char smem[];
-  constexpr int NT = NW * 64;
-  constexpr int PRE = (32 * NKMAX * 4 + NT - 1) / NT;      // 16-byte chunks per thread per unit
-  constexpr bool PREFETCH = PRE <= 12;                     // else the registers go to Q and O
-  const int Dk = a.R + a.rd;
-  const int nk = (Dk + 31) >> 5, Dkp = nk << 5;            // k-steps of 32
-  const int nc = (a.R + 15) >> 4;                          // latent column tiles of 16
-  const int ldk = a.ldk;                                   // K tile row stride (elements)
-  constexpr int LDV = 40;                                  // V^T tile row stride (elements)
-  bf16_t* kt = reinterpret_cast<bf16_t*>(smem);            // [32][ldk]
-  bf16_t* vt = kt + 32 * ldk;                              // [nc * 16][LDV]
-
-  int seq, row0, ntok;
-  if (a.cu_q) {
-    seq = a.work[2 * blockIdx.x];
-    const int q0 = a.work[2 * blockIdx.x + 1];
-    row0 = a.cu_q[seq] + q0;
-    ntok = min(a.QB, a.cu_q[seq + 1] - row0);
-  } else {
-    seq = blockIdx.x;
-    row0 = seq;
-    ntok = 1;
-  }
-  if (ntok <= 0 || (a.seq_lens && a.seq_lens[seq] <= 0)) return;
-  {   // a partition beyond the ones this row's context uses has nothing to do (whole workgroup)
-    const int kmax0 = a.positions[row0 + ntok - 1] + 1;
-    const int kmin0 = a.window > 0 ? (max(0, a.positions[row0] - a.window + 1) & ~31) : 0;
-    if ((int)blockIdx.z >= lat_parts(a.nparts, kmin0, kmax0)) return;
-  }
-  const int h0 = blockIdx.y * a.HB;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int c = lane & 15, g = lane >> 4;
+  bf16_t* tiles = reinterpret_cast<bf16_t*>(smem);      // [NB][KT][KS]
+  float* sS = reinterpret_cast<float*>(tiles + NB * KT * KS);      // [16][SP]
+  float2* rot = reinterpret_cast<float2*>(sS + 16 * SP);          // [rot_dims / 2]
+  const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int l16 = lane & 15, g4 = lane >> 4;
+  if (a.seq_lens && a.seq_lens[row] <= 0) return;
+  const int qpos = a.positions[row], kmax = qpos + 1;
+  const int wlo = a.window > 0 ? max(0, kmax - a.window) : 0, kmin = wlo & ~(KT - 1);
+  const int np = lat_parts(a.nparts, kmin, kmax);
+  if ((int)blockIdx.z >= np) return;                    // (whole workgroup)
+  const int units = (kmax - kmin + KT - 1) / KT;        // (equal parts)
+  const int k_begin = kmin + units * (int)blockIdx.z / np * KT;
+  const int k_end = min(kmax, kmin + units * ((int)blockIdx.z + 1) / np * KT);
+  const int R = a.R, Dk = R + a.rd, bs = a.bs, h0 = blockIdx.y * a.HB, nh = min(a.HB, a.H - h0);
   const bf16_t* cache = static_cast<const bf16_t*>(a.cache);
-  const int* bt = a.block_table + (long)seq * a.bt_stride;
-
-  // this lane's row (B operand column / accumulator column)
-  const int m = SPLITV ? c : wave * 16 + c;
-  const int t = m / a.HB, h = h0 + (m - t * a.HB);
-  const bool row_ok = t < ntok && h < a.H && m < a.QB * a.HB;
-  const long row = row0 + (row_ok ? t : 0);
-  const int qpos = row_ok ? a.positions[row] : -1;
-  // the rotary query parts of the workgroup's rows, rotated once into LDS: a thread takes whole
-  // pairs (one sine / cosine each, independent loads), not the entries of its own operand
-  bf16_t* qrs = vt + nc * 16 * LDV;                        // [rows][rd]
-  {
-    constexpr int NROWS = SPLITV ? 16 : NW * 16;
-    const bf16_t* qrb = static_cast<const bf16_t*>(a.qr);
-    const int hp = a.rot_dims >> 1, npass = a.rd - a.rot_dims;
-    for (int e = tid; e < NROWS * hp; e += NT) {
-      const int mm = e / hp, i = e - mm * hp;
-      const int tt = mm / a.HB, hh = h0 + (mm - tt * a.HB);
-      if (tt < ntok && hh < a.H && mm < a.QB * a.HB) {
-        const bf16_t* src = qrb + (long)(row0 + tt) * a.qr_st + (long)hh * a.qr_sh;
-        const int ia = a.rot_half ? i : 2 * i, ib = a.rot_half ? i + hp : 2 * i + 1;
-        const float u = bf2f(src[ia]), w = bf2f(src[ib]);
-        float sn, cs;
-        sincosf((float)a.positions[row0 + tt] * a.inv_freq[i], &sn, &cs);
-        sn *= a.rot_amp;
-        cs *= a.rot_amp;
-        qrs[mm * a.rd + ia] = f2bf(u * cs - w * sn);
-        qrs[mm * a.rd + ib] = f2bf(w * cs + u * sn);
-      }
-    }
-    for (int e = tid; e < NROWS * npass; e += NT) {        // entries past rot_dims pass unchanged
-      const int mm = e / npass, d = a.rot_dims + (e - mm * npass);
-      const int tt = mm / a.HB, hh = h0 + (mm - tt * a.HB);
-      if (tt < ntok && hh < a.H && mm < a.QB * a.HB)
-        qrs[mm * a.rd + d] = qrb[(long)(row0 + tt) * a.qr_st + (long)hh * a.qr_sh + d];
-    }
-    __syncthreads();
-  }
-  bf16x8 qf[NKMAX];
-  {
-    const bf16_t* qa = static_cast<const bf16_t*>(a.qa) + row * a.qa_st + (long)h * a.qa_sh;
-    // R % 8 == 0 and rd % 8 == 0: a lane's 8-entry chunk lies wholly in the absorbed part (one
-    // 16-byte load when the rows are aligned) or wholly in the rotary part (one LDS read)
-    const bool qvec = ((reinterpret_cast<uintptr_t>(a.qa) | (uintptr_t)(a.qa_st * 2) |
-                        (uintptr_t)(a.qa_sh * 2)) & 15) == 0;
+  const int* bt = a.block_table + (long)row * a.bt_stride;
+  const bool paged = bs % KT == 0;                      // a tile lies in one page
+  const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+  bf16x8 kst[NK];
+  // (nothing may look at the values before stash)
+  auto fetch = [&](int k0) {
+    const long base = paged ? (long)bt[k0 / bs] * bs + k0 % bs : 0;
 #pragma unroll
-    for (int s = 0; s < NKMAX; ++s) {
-      const int d0 = s * 32 + 8 * g;
-      bf16x8 v = {0, 0, 0, 0, 0, 0, 0, 0};
-      if (row_ok && s < nk && d0 < Dk) {
-        if (d0 >= a.R) {
-          v = *reinterpret_cast<const bf16x8*>(qrs + m * a.rd + (d0 - a.R));
-        } else if (qvec) {
-          v = *reinterpret_cast<const bf16x8*>(qa + d0);
+    for (int i = 0; i < NK; ++i) {
+      const int u = tid + 256 * i, j = u / (4 * NK), d = 8 * (u % (4 * NK));
+      const int kp = min(k0 + j, kmax - 1);
+      const long slot = paged ? base + j : (long)bt[kp / bs] * bs + kp % bs;
+      kst[i] = *reinterpret_cast<const bf16x8*>(cache + slot * a.cache_row + (d < Dk ? d : 0));
+    }
+  };
+  auto stash = [&](int buf, int k0) {       // (slots behind the last key may hold anything: 0 x inf)
+#pragma unroll
+    for (int i = 0; i < NK; ++i) {
+      const int u = tid + 256 * i, j = u / (4 * NK), d = 8 * (u % (4 * NK));
+      *reinterpret_cast<bf16x8*>(tiles + (buf * KT + j) * KS + d) = d < Dk && k0 + j < k_end ? kst[i] : zero8;
+    }
+  };
+  fetch(k_begin);
+
+  // the rotary query parts, rotated once into LDS: the heads of a row turn by the same angles
+  const int hp = a.rot_dims >> 1, npass = a.rd - a.rot_dims;
+  for (int i = tid; i < hp; i += 256) {
+    float sn, cs;
+    sincosf((float)qpos * a.inv_freq[i], &sn, &cs);
+    rot[i] = make_float2(cs * a.rot_amp, sn * a.rot_amp);
+  }
+  __syncthreads();
+  bf16_t* qrs = tiles;                                  // [16][rd]
+  const bf16_t* qrb = static_cast<const bf16_t*>(a.qr) + (long)row * a.qr_st;
+  for (int e = tid; e < nh * hp; e += 256) {
+    const int m = e / hp, i = e - m * hp;
+    const bf16_t* src = qrb + (long)(h0 + m) * a.qr_sh;
+    const int ia = a.rot_half ? i : 2 * i, ib = a.rot_half ? i + hp : 2 * i + 1;
+    const float u = bf2f(src[ia]), v = bf2f(src[ib]);
+    const float2 cs = rot[i];
+    qrs[m * a.rd + ia] = f2bf(u * cs.x - v * cs.y);
+    qrs[m * a.rd + ib] = f2bf(v * cs.x + u * cs.y);
+  }
+  for (int e = tid; e < nh * npass; e += 256) {         // entries past rot_dims pass unchanged
+    const int m = e / npass, d = a.rot_dims + e - m * npass;
+    qrs[m * a.rd + d] = qrb[(long)(h0 + m) * a.qr_sh + d];
+  }
+  __syncthreads();
+  const bool ok = l16 < nh;                             // this lane's head
+  const int h = h0 + (ok ? l16 : 0);
+  bf16x8 qf[NK];
+  {
+    // R % 8 == 0 and rd % 8 == 0: a lane's eight entries lie wholly in one of the two parts
+    const bf16_t* qa = static_cast<const bf16_t*>(a.qa) + (long)row * a.qa_st + (long)h * a.qa_sh;
+    const bool vec = ((reinterpret_cast<uintptr_t>(a.qa) | (uintptr_t)(a.qa_st * 2) | (uintptr_t)(a.qa_sh * 2)) & 15) == 0;
+#pragma unroll
+    for (int s = 0; s < NK; ++s) {
+      const int d = 32 * s + 8 * g4;
+      bf16x8 v = zero8;
+      if (ok && d < Dk) {
+        if (d >= R) {
+          v = *reinterpret_cast<const bf16x8*>(qrs + l16 * a.rd + (d - R));
+        } else if (vec) {
+          v = *reinterpret_cast<const bf16x8*>(qa + d);
         } else {
 #pragma unroll
-          for (int e = 0; e < 8; ++e) v[e] = qa[d0 + e];
+          for (int e = 0; e < 8; ++e) v[e] = qa[d + e];
         }
       }
       qf[s] = v;
     }
   }
-  constexpr int NACC = SPLITV ? (NCMAX + NW - 1) / NW : NCMAX;   // column tiles of this wave
-  const int ct0 = SPLITV ? wave : 0, ctstep = SPLITV ? NW : 1;   // tile i -> ct0 + i * ctstep
-  f32x4 acc[NACC];
+  __syncthreads();                                      // the rotary parts make room for tiles
+  stash(0, k_begin);
+  f32x4 acc[NCW];
 #pragma unroll
-  for (int i = 0; i < NACC; ++i) acc[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < NCW; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
   float mrun = -INFINITY, lrun = 0.f;
   const float scale_log2 = a.scale * 1.4426950408889634f;
-  const int kmax = a.positions[row0 + ntok - 1] + 1;
-  // first 32-key unit that holds a key some row of the tile sees
-  const int kmin = a.window > 0 ? (max(0, a.positions[row0] - a.window + 1) & ~31) : 0;
-  int k_begin = kmin, k_end = kmax;
-  // partitions this row really uses: at least two 32-key units each (decided here and, the same
-  // way, in the merge kernel), so short contexts do not pay for idle partitions
-  const int np = lat_parts(a.nparts, kmin, kmax);
-  if (np > 1) {                                            // this partition's run of 32-key units
-    const int units = (kmax - kmin + 31) >> 5;
-    const int per = (units + np - 1) / np;
-    k_begin = kmin + (min((int)blockIdx.z * per, units) << 5);
-    k_end = min(kmax, kmin + (((int)blockIdx.z + 1) * per << 5));
-  }
-  const int wlo = a.window > 0 ? qpos - a.window + 1 : 0;   // first key this lane's row sees
-  const int cpr = Dkp >> 3;                                // 16-byte chunks per (padded) key row
-  const int nchunk = 32 * cpr;
-
-  auto load_chunk = [&](int k0, int ch) {
-    bf16x8 v = {0, 0, 0, 0, 0, 0, 0, 0};
-    const int j = ch / cpr, d = (ch - j * cpr) << 3;
-    const int kp = k0 + j;
-    if (kp < k_end && d < Dk) {                            // Dk % 8 == 0: whole chunk inside
-      const long slot = (long)bt[kp / a.bs] * a.bs + (kp % a.bs);
-      v = *reinterpret_cast<const bf16x8*>(cache + slot * a.cache_row + d);
-    }
-    return v;
-  };
-  // key j = 8G + i lands in K tile row 4G + i (i < 4) or 16 + 4G + i - 4
-  auto store_chunk = [&](int ch, bf16x8 v) {
-    const int j = ch / cpr, d = (ch - j * cpr) << 3;
-    const int r = ((j & 4) ? 16 : 0) + 4 * (j >> 3) + (j & 3);
-    *reinterpret_cast<bf16x8*>(kt + r * ldk + d) = v;
-  };
-  bf16x8 pre[PREFETCH ? PRE : 1];
-  auto fetch = [&](int k0) {
-    if constexpr (PREFETCH) {
-#pragma unroll
-      for (int i = 0; i < PRE; ++i) {
-        const int ch = tid + i * NT;
-        if (ch < nchunk) pre[i] = load_chunk(k0, ch);
-      }
-    }
-  };
-  fetch(k_begin);
-  for (int k0 = k_begin; k0 < k_end; k0 += 32) {
-    if constexpr (PREFETCH) {
-#pragma unroll
-      for (int i = 0; i < PRE; ++i) {
-        const int ch = tid + i * NT;
-        if (ch < nchunk) store_chunk(ch, pre[i]);
-      }
-    } else {
-      for (int ch = tid; ch < nchunk; ch += NT) store_chunk(ch, load_chunk(k0, ch));
-    }
+  // transposing read: lane l of sixteen addresses row l / 4, entries 4 (l % 4), and receives column l
+  const int c0 = 16 * NCW * w, vrow = 8 * g4 + (l16 >> 2), vcol = c0 + 4 * (l16 & 3);
+  for (int k0 = k_begin, buf = 0; k0 < k_end; k0 += KT, buf ^= NB - 1) {
+    const bf16_t* t = tiles + buf * KT * KS;
     __syncthreads();
-    // K tile -> V^T tile (latent columns; rows past R are zero from the padded chunks)
-    for (int ch = tid; ch < 32 * nc * 2; ch += NT) {
-      const int j = ch & 31, d = (ch >> 5) << 3;
-      const int r = ((j & 4) ? 16 : 0) + 4 * (j >> 3) + (j & 3);
-      bf16x8 v = {0, 0, 0, 0, 0, 0, 0, 0};
-      if (d < a.R) v = *reinterpret_cast<const bf16x8*>(kt + r * ldk + d);   // R % 8 == 0
+    if (k0 + KT < k_end) fetch(k0 + KT);
+    f32x4 sc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int e = 0; e < 8; ++e) vt[(d + e) * LDV + j] = v[e];
-    }
+    for (int s = 0; s < NK; ++s)
+      sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+          *reinterpret_cast<const bf16x8*>(t + (16 * w + l16) * KS + 32 * s + 8 * g4), qf[s], sc, 0, 0, 0);
+    *reinterpret_cast<f32x4*>(sS + l16 * SP + 16 * w + 4 * g4) = sc * scale_log2;
     __syncthreads();
-    if (k0 + 32 < k_end) fetch(k0 + 32);
-    // S^T tiles: keys (rows) x this wave's 16 rows (columns)
-    f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+    // head l16, keys 32 x + 8 g4 + e
+    float v[2][8];
+    float mloc = -INFINITY;
 #pragma unroll
-    for (int s = 0; s < NKMAX; ++s) {
-      if (s < nk) {
-        const bf16x8 ka = *reinterpret_cast<const bf16x8*>(kt + c * ldk + s * 32 + 8 * g);
-        const bf16x8 kb = *reinterpret_cast<const bf16x8*>(kt + (16 + c) * ldk + s * 32 + 8 * g);
-        s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka, qf[s], s0, 0, 0, 0);
-        s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kb, qf[s], s1, 0, 0, 0);
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int e = 0; e < 8; e += 4) {
+        const f32x4 q = *reinterpret_cast<const f32x4*>(sS + l16 * SP + 32 * x + 8 * g4 + e);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int key = k0 + 32 * x + 8 * g4 + e + i;
+          v[x][e + i] = key >= wlo && key < k_end ? q[i] : -INFINITY;
+          mloc = fmaxf(mloc, v[x][e + i]);
+        }
       }
-    }
-    float v[8];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int ka = k0 + 8 * g + i, kb = ka + 4;
-      v[i] = (ka <= qpos && ka >= wlo) ? s0[i] * scale_log2 : -INFINITY;
-      v[4 + i] = (kb <= qpos && kb >= wlo) ? s1[i] * scale_log2 : -INFINITY;
-    }
-    float mloc = v[0];
-#pragma unroll
-    for (int i = 1; i < 8; ++i) mloc = fmaxf(mloc, v[i]);
     mloc = fmaxf(mloc, __shfl_xor(mloc, 16, 64));
     mloc = fmaxf(mloc, __shfl_xor(mloc, 32, 64));
-    const float mnew = fmaxf(mrun, mloc);
-    const float muse = (mnew == -INFINITY) ? 0.f : mnew;
-    const float alpha = exp2f(mrun - muse);                // mrun = -inf: 0 (nothing summed yet)
-    bf16x8 ph, pl;
+    const float mnew = fmaxf(mrun, mloc), muse = mnew == -INFINITY ? 0.f : mnew;
+    const float alpha = exp2f(mrun - muse);             // mrun = -inf: 0 (nothing summed yet)
+    bf16x8 ph[2], pl[2];
     float psum = 0.f;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float p = exp2f(v[i] - muse);
-      const bf16_t hi = f2bf(p);
-      ph[i] = hi;
-      pl[i] = f2bf(p - bf2f(hi));
-      psum += p;
-    }
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) {
+        const float p0 = exp2f(v[x][e] - muse), p1 = exp2f(v[x][e + 1] - muse);
+        psum += p0 + p1;
+        flash_split(p0, p1, e, ph[x], pl[x]);
+      }
     psum += __shfl_xor(psum, 16, 64);
     psum += __shfl_xor(psum, 32, 64);
     lrun = lrun * alpha + psum;
     mrun = mnew;
-    const bool rescale = !__all(alpha == 1.f);
 #pragma unroll
-    for (int ai = 0; ai < NACC; ++ai) {
-      const int ct = ct0 + ai * ctstep;
-      if (ct < nc) {
-        const bf16x8 vf = *reinterpret_cast<const bf16x8*>(vt + (ct * 16 + c) * LDV + 8 * g);
-        f32x4 o = acc[ai];
-        if (rescale) o *= alpha;
-        o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, ph, o, 0, 0, 0);
-        acc[ai] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pl, o, 0, 0, 0);
+    for (int i = 0; i < NCW; ++i) acc[i] *= alpha;
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int i = 0; i < NCW; ++i) {
+        typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+        const bf16_t* p = t + (32 * x + vrow) * KS + vcol + 16 * i;
+        const s16x4 a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p);
+        const s16x4 a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p + 4 * KS));
+        const bf16x8 vf = __builtin_bit_cast(bf16x8, __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7));
+        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, ph[x], acc[i], 0, 0, 0);
+        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pl[x], acc[i], 0, 0, 0);
       }
+    if (k0 + KT < k_end) {
+      if (NB == 1) __syncthreads();                     // the tile was read
+      stash(buf ^ (NB - 1), k0 + KT);
     }
-    __syncthreads();
   }
-  if (!row_ok) return;
+  if (!ok) return;
+  // the lane holds columns c0 + 16 i + 4 g4 .. + 3 of its head (R % 8 == 0)
   if (np > 1) {
     const long pr = ((long)row * a.H + h) * a.nparts + blockIdx.z;
-    float* pa = a.part_acc + pr * a.R;
 #pragma unroll
-    for (int ai = 0; ai < NACC; ++ai) {
-      const int ct = ct0 + ai * ctstep;
-      if (ct < nc) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int col = ct * 16 + 4 * g + i;
-          if (col < a.R) pa[col] = acc[ai][i];
-        }
-      }
+    for (int i = 0; i < NCW; ++i) {
+      const int c = c0 + 16 * i + 4 * g4;
+      if (c < R) *reinterpret_cast<f32x4*>(a.part_acc + pr * R + c) = acc[i];
     }
-    if (g == 0 && (!SPLITV || wave == 0)) {
+    if (g4 == 0 && w == 0) {
       a.part_ml[2 * pr] = mrun;
       a.part_ml[2 * pr + 1] = lrun;
     }
@@ -597,28 +536,23 @@ latent_attn_mfma_kernel(LatentAttnArgs a) {
   }
   if (a.sink) lrun += exp2f(a.sink[h] * 1.4426950408889634f - mrun);
   float f = 1.0f / lrun;
-  if (a.gate) {
-    const bf16_t* gate = static_cast<const bf16_t*>(a.gate);
-    f *= 1.0f / (1.0f + expf(-bf2f(gate[row * a.gate_st + h])));
-  }
+  if (a.gate) f *= 1.0f / (1.0f + expf(-bf2f(static_cast<const bf16_t*>(a.gate)[row * a.gate_st + h])));
   bf16_t* out = static_cast<bf16_t*>(a.out) + row * a.out_st + (long)h * a.out_sh;
 #pragma unroll
-  for (int ai = 0; ai < NACC; ++ai) {
-    const int ct = ct0 + ai * ctstep;
-    if (ct < nc) {
+  for (int i = 0; i < NCW; ++i) {
+    const int c = c0 + 16 * i + 4 * g4;
+    if (c >= R) continue;
+    bf16x4 o;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int col = ct * 16 + 4 * g + i;
-        if (col < a.R) out[col] = f2bf(acc[ai][i] * f);
-      }
-    }
+    for (int e = 0; e < 4; ++e) o[e] = f2bf(acc[i][e] * f);
+    *reinterpret_cast<bf16x4*>(out + c) = o;
   }
 }
 
 // Merge of the decode partitions: out = sum_p acc_p 2^(m_p - M) / sum_p l_p 2^(m_p - M), times
 // the head gate.  One workgroup per (row, head); lane p first turns partition p's (max, sum) into
-// its weight, then the threads sum the latent columns over the partitions with independent loads
-// (nparts <= 64).  Rows whose context is too short for two partitions were finished by the
+// its weight, then the threads sum four latent columns each over the partitions with independent
+// loads (nparts <= 64).  Rows whose context is too short for two partitions were finished by the
 // attention kernel itself.
 __global__ void __launch_bounds__(128)
 latent_merge_kernel(const float* __restrict__ part_acc, const float* __restrict__ part_ml,
@@ -629,7 +563,7 @@ latent_merge_kernel(const float* __restrict__ part_acc, const float* __restrict_
   const int row = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63;
   if (seq_lens && seq_lens[row] <= 0) return;
   const int kmax = positions[row] + 1;
-  const int kmin = window > 0 ? (max(0, kmax - window) & ~31) : 0;
+  const int kmin = window > 0 ? max(0, kmax - window) & ~(LAT_UNIT - 1) : 0;
   const int np = lat_parts(nparts, kmin, kmax);
   if (np == 1) return;
   const long pr = ((long)row * H + h) * nparts;
@@ -641,15 +575,20 @@ latent_merge_kernel(const float* __restrict__ part_acc, const float* __restrict_
   if (sink && M != -INFINITY) L += exp2f(sink[h] * 1.4426950408889634f - M);
   float f = L > 0.f ? 1.0f / L : 0.f;
   if (gate) f *= 1.0f / (1.0f + expf(-bf2f(gate[row * gate_st + h])));
-  for (int c0 = 0; c0 < R; c0 += blockDim.x) {
-    const int c = c0 + threadIdx.x;
-    float v = 0.f;
+  for (int c0 = 0; c0 < R; c0 += 4 * blockDim.x) {      // (R % 8 == 0; every lane takes part)
+    const int c = c0 + 4 * threadIdx.x;
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
     for (int p = 0; p < np; ++p) {
       const float w = __shfl(wp, p, 64);
-      if (c < R) v += part_acc[(pr + p) * R + c] * w;
+      if (c < R) v += *reinterpret_cast<const f32x4*>(part_acc + (pr + p) * R + c) * w;
     }
-    if (c < R) out[row * out_st + h * out_sh + c] = f2bf(v * f);
+    if (c < R) {
+      bf16x4 o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = f2bf(v[e] * f);
+      *reinterpret_cast<bf16x4*>(out + row * out_st + h * out_sh + c) = o;
+    }
   }
 }
 
@@ -666,31 +605,31 @@ EIA_API int eia_latent_attn_mfma(const void* qa, long qa_st, long qa_sh, const v
     return EIA_BAD_SHAPE;
   const int Dk = R + rd;
   // 16-byte chunks must not straddle the latent / rotary boundary or the row end
-  if ((R & 7) || (Dk & 7) || (cache_row & 7) || Dk > 640 || R > 512) return EIA_UNSUPPORTED;
+  if ((R & 7) || (Dk & 7) || (cache_row & 7) || Dk > 640 || R > 512 || out_sh % 4 || out_st % 4)
+    return EIA_UNSUPPORTED;
   if (n_items <= 0) return EIA_OK;
   const int HB = H < 16 ? H : 16;
   if (nparts < 1 || nparts > 64 || (nparts > 1 && (!part_acc || !part_ml))) return EIA_BAD_SHAPE;
-  const int nk = (Dk + 31) / 32, Dkp = nk * 32, nc = (R + 15) / 16;
-  const int ldk = ((Dkp / 8) & 1) ? Dkp : Dkp + 8;       // odd number of 16-byte units per row
-  // K tile, V^T tile, and the rotated rotary query parts of up to 16 rows
-  const size_t lds = ((size_t)32 * ldk + (size_t)nc * 16 * 40 + (size_t)16 * rd) * 2;
   LatentAttnArgs a{qa, qa_st, qa_sh, qr, qr_st, qr_sh, inv_freq, rot_dims, cache, cache_row,
-                   block_table, bt_stride, seq_lens, nullptr, nullptr, n_items, positions, gate, gate_st,
-                   out, out_st, out_sh, scale, H, R, rd, bs, 1, HB, 32, ldk, window, sink, rot_half,
-                   rot_amp, nparts, part_acc, part_ml};
-  dim3 grid(n_items, (H + HB - 1) / HB, nparts);
-#define LAT_MFMA(NK, NC, SV)                                                                \
-  do {                                                                                      \
-    if (lds > 48 * 1024)                                                                    \
-      (void)hipFuncSetAttribute(                                                            \
-          reinterpret_cast<const void*>(&latent_attn_mfma_kernel<NK, NC, 4, SV>),           \
-          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);                            \
-    hipLaunchKernelGGL((latent_attn_mfma_kernel<NK, NC, 4, SV>), grid, dim3(256), lds, st, a); \
+                   block_table, bt_stride, seq_lens, nullptr, nullptr, n_items, positions, gate,
+                   gate_st, out, out_st, out_sh, scale, H, R, rd, bs, 1, HB, 0, 0, window, sink,
+                   rot_half, rot_amp, nparts, part_acc, part_ml};
+  const dim3 grid(n_items, (H + HB - 1) / HB, nparts);
+#define LAT_DECODE(NK, NCW)                                                                        \
+  do {                                                                                             \
+    const int lds = 2 * lat_bufs(NK) * LAT_UNIT * (32 * NK + 8) +                                  \
+                    4 * 16 * (LAT_UNIT + 4) + 4 * rot_dims;                                        \
+    if (lds > 64 * 1024)                                                                           \
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&latent_decode_kernel<NK, NCW>),     \
+                                hipFuncAttributeMaxDynamicSharedMemorySize, lds);                  \
+    hipLaunchKernelGGL((latent_decode_kernel<NK, NCW>), grid, dim3(256), lds, st, a);              \
   } while (0)
-  if (nk <= 6 && nc <= 8) LAT_MFMA(6, 8, true);
-  else if (nk <= 12 && nc <= 16) LAT_MFMA(12, 16, true);
-  else LAT_MFMA(20, 32, true);
-#undef LAT_MFMA
+  if (Dk <= 160 && R <= 128) LAT_DECODE(5, 2);
+  else if (Dk <= 288 && R <= 256) LAT_DECODE(9, 4);
+  else if (Dk <= 320 && R <= 256) LAT_DECODE(10, 4);
+  else if (Dk <= 576) LAT_DECODE(18, 8);
+  else LAT_DECODE(20, 8);
+#undef LAT_DECODE
   if (nparts > 1)
     hipLaunchKernelGGL(latent_merge_kernel, dim3(n_items, H), dim3(128), 0, st, part_acc, part_ml,
                        nparts, seq_lens, positions, window, static_cast<const bf16_t*>(gate),

@@ -51,21 +51,19 @@ def query_block(num_heads: int, kv_rank: int, rot_dim: int = 0,
     return max(1, min(16, ACC_ROWS // (hb * kv_rank), 12288 // (hb * (kv_rank + rot_dim))))
 
 
-def decode_partitions(batch: int, num_heads: int, cus: int = 256, window: int = 0) -> int:
-    """Key partitions (grid.z) of a decode launch of the MFMA form: a decode row is one
-    single-wave workgroup per 16-head slice, so small batches split every row's keys until about
-    four workgroups per CU exist (a power of two, at most 32, and no more than the 32-key units
-    a sliding window can hold); the partials are merged by a second kernel.  Depends on the
-    batch and the layer's constants only, so a captured decode graph keeps its grid."""
+def decode_partitions(batch: int, num_heads: int, cus: int = 256, window: int = 0,
+                      wide: bool = True) -> int:
+    """Key partitions (grid.z) of a decode launch of the MFMA form: a decode row is one workgroup
+    per 16-head slice, so small batches split every row's 64-key tiles until the chip's slots are
+    taken -- one workgroup per CU with ``wide`` rows (LDS), two otherwise -- at most 64 and no more
+    than the tiles a sliding window can hold; the partials are merged by a second kernel.  Depends
+    on the batch and the layer's constants only, so a captured decode graph keeps its grid."""
     forced = int(os.environ.get("EIA_LATENT_DECODE_P", "0"))
     if forced > 0:
         return min(forced, 64)
     wgs = max(1, batch * ((num_heads + 15) // 16))
-    limit = 32 if window <= 0 else max(1, min(32, (window + 31) // 32 + 1))
-    p = 1
-    while p * 2 <= limit and wgs * p * 2 <= 4 * cus:
-        p *= 2
-    return p
+    limit = 64 if window <= 0 else max(1, min(64, (window + 63) // 64 + 1))
+    return max(1, min(limit, (cus if wide else 2 * cus) // wgs))
 
 
 def build_work(q_lens: List[int], qblock: int) -> List[int]:
@@ -243,7 +241,7 @@ def latent_attention(q_abs: torch.Tensor, q_rot: torch.Tensor, inv_freq: torch.T
                 "latent_flash")
             return
         if mfma:
-            P = decode_partitions(n_items, H, window=window)
+            P = decode_partitions(n_items, H, window=window, wide=R + rd > 320)
             pa = pm = None
             if P > 1:
                 pa = torch.empty(n_items * H * P * R, dtype=torch.float32, device=q_abs.device)

@@ -59,3 +59,33 @@ def test_latent_flash(window, bs, new, past, H, R, rd):
                                    (R + rd) ** -0.5, window, d(sink), bool(window), 1.1).cpu()
 
     _check(run("cpu"), run("cuda"))
+
+
+@pytest.mark.parametrize("H,R,rd", [(8, 128, 32), (3, 48, 16), (20, 40, 8), (16, 256, 32), (8, 256, 64),
+                                    (16, 512, 64), (2, 512, 128)])
+@pytest.mark.parametrize("window,bs,parts", [(0, 64, 1), (0, 64, 3), (70, 128, 2), (0, 16, 64), (200, 48, 5)])
+def test_latent_decode(window, bs, parts, H, R, rd, monkeypatch):
+    from enterprise_inference_amd.ops import attention as A
+    from enterprise_inference_amd.ops import latent_attention as la
+    monkeypatch.setenv("EIA_LATENT_DECODE_P", str(parts))
+    g = torch.Generator().manual_seed(H + R + window)
+    total = [1, 64, 65, 300, 129]
+    bt, n = _pages(g, total, bs)
+    pos = torch.tensor(total, dtype=torch.int32) - 1
+    T, bf = len(total), torch.bfloat16
+    rnd = lambda *s: torch.randn(*s, generator=g).to(bf)
+    qa, qr, cache = rnd(T, H, R), rnd(T, H, rd), rnd(n, bs, R + rd)
+    for s, k in enumerate(total):
+        cache[int(bt[s, -(-k // bs) - 1]), (k - 1) % bs + 1:] = float("nan")
+    gate, sink = (rnd(T, H), None) if window == 0 else (None, torch.randn(H, generator=g))
+    inv = la.inv_frequencies(rd, 100.0, "cpu")
+
+    def run(dev):
+        d = lambda t: None if t is None else t.to(dev)
+        md = A.AttentionMetadata(
+            num_decode=T, num_prefill_tokens=0, slot_mapping=d(pos), positions=d(pos),
+            decode_block_tables=d(bt), decode_seq_lens=d(pos + 1))
+        return la.latent_attention(d(qa), d(qr), d(inv), rd - 8, d(cache), md, d(gate),
+                                   (R + rd) ** -0.5, window, d(sink), bool(window), 1.1).cpu()
+
+    _check(run("cpu"), run("cuda"))

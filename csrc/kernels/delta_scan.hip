@@ -205,74 +205,117 @@ EIA_API int eia_delta_scan(const float* q, const float* k, const float* v, const
 //
 //   u_t + sum_(s<t) L_ts u_s = b_t v_t - b_t exp(A_t) S^T k_t,    L_ts = b_t exp(A_t - A_s) k_t . k_s
 //
-// whose right side is linear in S:  u = X - Y S  with (I + L) X = diag(b) V and
-// (I + L) Y = diag(b exp(A)) K.
-//   (1) X, Y of every chunk, in parallel (block forward substitution, 16-token blocks whose diagonal
-//       inverses are formed first)
-//   (2) a sequence's chunks in order, in parallel over heads and 16-column slices of the state:
+// whose right side is linear in S:  with T = (I + L)^-1,  u = X - Y S,  X = T diag(b) V,
+// Y = T diag(b exp(A)) K.
+//   (1) T, X, Y of every chunk, in parallel (T by 16-token blocks, diagonal inverses first)
+//   (2) a sequence's chunks in order, in parallel over heads and slices of the state's columns:
 //       u = X - Y S (replaces X), S <- exp(A_end) S + sum_t exp(A_end - A_t) k_t u_t^T
 //   (3) outputs of every chunk, in parallel:
 //       o_t = exp(A_t) S^T q_t + sum_(s<=t) exp(A_t - A_s) (q_t . k_s) u_s
 // Every exponent is <= 0.  All products are fp32 matrix-core products (16x16x4): an accumulator's
 // registers (row 4 (lane / 16) + i, column lane % 16) are, step i, the B operand of a product over
-// its rows, so X, Y, u and S go from one product to the next in registers; an A operand's lane reads
-// four consecutive k as one 16-byte access.
+// its rows; an A operand's lane holds four consecutive k of row lane % 16.
+//
+// Layout.  With row-major workspaces most operands were 4-byte accesses, and issuing them took longer
+// than the products.  So everything that passes between the kernels lies as the lanes of the next
+// product take it, 16 bytes per lane and 1 KB per access: a fragment [64 lanes][4].  The row and
+// column order inside a head is free as long as all products agree, and is chosen so that rows of q, k and v are
+// read 8 or 16 bytes at a time: tile j of a group of 64 holds entries 64 g + 4 x + j; its column r is
+// x = r, its row r (dk only) x = 4 (r % 4) + r / 4, the order in which an A operand's rows are read.
+//   Y  [chunk, H, 4 token tiles, DP tiles]   A operand, rows tokens
+//   X  [chunk, H, 4 token tiles, VP tiles]   B operand, rows tokens (u after the scan)
+//   Kt [chunk, G, DP tiles, 4 token tiles]   A operand, rows dk
+//   S  [chunk, H, DP tiles, VP tiles]        B operand, rows dk
+// with DP and VP rounded up to 64.  MI355X, 16 heads of 128 x 128, three prompts of 750 to 1500
+// tokens: 48 + 77 + 83 us (row-major: 87 + 138 + 129), of which the products alone are 14 + 46 + 26.
 constexpr int DC = 64;                      // tokens per chunk
 constexpr int DL = DC + 4;                  // LDS row pitch of the triangular blocks
 
 struct DeltaChunkArgs {
   const int* chunks;                        // [nchunk, 4]: sequence, first row, tokens, unused
   const int* seq_first;                     // [nseq + 1]: first chunk of every sequence
-  float* Y; float* X;                       // [rows, H, DP], [rows, H, VP]
-  float* wsS;                               // [nchunk, H, DP, VP]: the state before each chunk
-  float* cA; float* wsG;                    // [rows, H] running sums, [nchunk, H] their last
+  float* Y; float* X; float* Kt; float* wsS;   // fragments, as above (wsS: the state before each chunk)
+  float* cA;                                // [nchunk, H, DC] running sums of la, constant past the end
+  int ncg;                                  // groups of 64 state columns
+  int vec;                                  // out, gate and weight rows can be taken 4 at a time
 };
 
 EIA_DEV f32x4 mm(f32x4 a, f32x4 b, f32x4 c) { return mfma_f32_k16(a, b, c); }
+EIA_DEV int dl_row(int r) { return 4 * (r & 3) + (r >> 2); }
+EIA_DEV f32x4 frag(const float* p, long tile, int lane) {
+  return *reinterpret_cast<const f32x4*>(p + tile * 256 + 4 * lane);
+}
+EIA_DEV void put_frag(float* p, long tile, int lane, f32x4 v) {
+  *reinterpret_cast<f32x4*>(p + tile * 256 + 4 * lane) = v;
+}
 
+// (1) one workgroup per (chunk, head).  K is staged in LDS: the triangle takes it by rows, Y by
+// columns.  Y and X are made in units of 32 columns, 8-byte reads; a wave has at most one unit of
+// each, and the rows of v for its unit are on their way from the start.
+template <int NDG>                                     // groups of 64 dk
 __global__ void __launch_bounds__(256)
 delta_chunk_solve_kernel(DeltaArgs a, DeltaChunkArgs c) {
-  __shared__ __align__(16) float Ls[DC][DL];           // -L
-  __shared__ __align__(16) float Ts[4][16][20];        // inverses of the diagonal blocks
+  constexpr int KP = 64 * NDG + 4;
+  __shared__ __align__(16) float ks[DC][KP];
+  __shared__ __align__(16) float Ls[DC][DL];           // -L, then T
   __shared__ float sA[DC], sb[DC];
-  const int ch = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int ch = blockIdx.y, h = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int s = c.chunks[4 * ch], row0 = c.chunks[4 * ch + 1], n = c.chunks[4 * ch + 2];
   if (a.slots[s] < 0) return;
   const int H = a.H, G = a.G, DP = a.DP, VP = a.VP, kh = h / (H / G);
   const int g4 = lane >> 4, l16 = lane & 15;
+  const long ldk = (long)G * DP, ldv = (long)H * VP;
+  const float* K = a.k + (long)row0 * ldk + (long)kh * DP;
+  f32x4 kst[4 * NDG];
+#pragma unroll
+  for (int i = 0; i < 4 * NDG; ++i) {
+    const int e = tid + 256 * i, r = e / (16 * NDG), d = 4 * (e % (16 * NDG));
+    kst[i] = *reinterpret_cast<const f32x4*>(K + min(r, n - 1) * ldk + min(d, DP - 4));
+  }
+  const int xu = wave >= 2 * NDG ? wave - 2 * NDG : wave + 4 - 2 * NDG;     // this wave's unit of X
+  const bool hasx = xu < 2 * c.ncg;
+  float2 vf[4][4];
+  if (hasx) {
+    const int col = min(64 * (xu >> 1) + 4 * l16 + 2 * (xu & 1), VP - 2);   // past VP: unused columns
+    const float* V = a.v + (long)row0 * ldv + (long)h * VP + col;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        vf[k][i] = *reinterpret_cast<const float2*>(V + min(16 * k + 4 * g4 + i, n - 1) * ldv);
+  }
   if (wave == 0) {                                     // running sums of the log decays
     float la = lane < n ? a.la[(long)(row0 + lane) * H + h] : 0.f;
+    const float b = lane < n ? a.beta[(long)(row0 + lane) * H + h] : 0.f;
 #pragma unroll
     for (int o = 1; o < DC; o <<= 1) {
       const float up = __shfl_up(la, o, 64);
       if (lane >= o) la += up;
     }
     sA[lane] = la;
-    sb[lane] = lane < n ? a.beta[(long)(row0 + lane) * H + h] : 0.f;
-    if (lane < n) c.cA[(long)(row0 + lane) * H + h] = la;
-    if (lane == n - 1) c.wsG[(long)ch * H + h] = la;
+    sb[lane] = b;
+    c.cA[((long)ch * H + h) * DC + lane] = la;
+  }
+#pragma unroll
+  for (int i = 0; i < 4 * NDG; ++i) {
+    const int e = tid + 256 * i, r = e / (16 * NDG), d = 4 * (e % (16 * NDG));
+    *reinterpret_cast<f32x4*>(&ks[r][d]) = d < DP ? kst[i] : f32x4{0.f, 0.f, 0.f, 0.f};
   }
   __syncthreads();
-  const long ldk = (long)G * DP, ldv = (long)H * VP, ldx = (long)H * DP;
-  const float* K = a.k + (long)kh * DP;
-  const int nb = DP >> 4;
-  {                                                    // rows 16 wave .. of -L
-    const float* ka = K + (long)(row0 + min(16 * wave + l16, n - 1)) * ldk + 4 * g4;
-    f32x4 kf[8];
+  // the ten blocks of -L, two or three per wave: block p is row tile t, column tile u
+  for (int p = wave; p < 10; p += 4) {
+    const int t = p >= 6 ? 3 : p >= 3 ? 2 : p >= 1 ? 1 : 0, u = p - t * (t + 1) / 2;
+    f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-    for (int b = 0; b < 8; ++b)
-      if (b < nb) kf[b] = *reinterpret_cast<const f32x4*>(ka + 16 * b);
-    for (int st = 0; st <= wave; ++st) {
-      const float* kb = K + (long)(row0 + min(16 * st + l16, n - 1)) * ldk + 4 * g4;
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int b = 0; b < 4 * NDG; ++b)
+      acc[b & 1] = mm(*reinterpret_cast<const f32x4*>(&ks[16 * t + l16][16 * b + 4 * g4]),
+                      *reinterpret_cast<const f32x4*>(&ks[16 * u + l16][16 * b + 4 * g4]), acc[b & 1]);
 #pragma unroll
-      for (int b = 0; b < 8; ++b)
-        if (b < nb) acc = mm(kf[b], *reinterpret_cast<const f32x4*>(kb + 16 * b), acc);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int t = 16 * wave + 4 * g4 + i, u = 16 * st + l16;
-        Ls[t][u] = u < t ? -sb[t] * expf(sA[t] - sA[u]) * acc[i] : 0.f;
-      }
+    for (int i = 0; i < 4; ++i) {
+      const int tr = 16 * t + 4 * g4 + i, tc = 16 * u + l16;
+      const float z = acc[0][i] + acc[1][i];
+      Ls[tr][tc] = tc < tr ? -sb[tr] * expf(sA[tr] - sA[tc]) * z : 0.f;
     }
   }
   __syncthreads();
@@ -285,274 +328,383 @@ delta_chunk_solve_kernel(DeltaArgs a, DeltaChunkArgs c) {
       for (int u = 0; u < r; ++u) v += Ls[16 * wave + r][16 * wave + u] * x[u];
       x[r] = v;
     }
-    if (lane < 16) {
+    if (lane < 16) {                                   // after every lane's reads: one wave, in order
 #pragma unroll
-      for (int r = 0; r < 16; ++r) Ts[wave][r][l16] = x[r];
+      for (int r = 0; r < 16; ++r) Ls[16 * wave + r][16 * wave + l16] = x[r];
     }
   }
   __syncthreads();
-  f32x4 lf[4][4], tf[4];                               // A operands: blocks of -L, inverses
+  // block column `wave` of T:  T_ij = T_ii sum_(j<=k<i) (-L_ik) T_kj
+  f32x4 tc[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    tf[i] = *reinterpret_cast<const f32x4*>(&Ts[i][l16][4 * g4]);
+  for (int e = 0; e < 4; ++e) tc[0][e] = Ls[16 * wave + 4 * g4 + e][16 * wave + l16];
 #pragma unroll
-    for (int k = 0; k < i; ++k) lf[i][k] = *reinterpret_cast<const f32x4*>(&Ls[16 * i + l16][16 * k + 4 * g4]);
-  }
-  float eb[4][4], bb[4][4];
+  for (int i = 1; i < 4; ++i)
+    if (wave + i < 4) {
+      f32x4 r = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < i; ++k)
+        r = mm(*reinterpret_cast<const f32x4*>(&Ls[16 * (wave + i) + l16][16 * (wave + k) + 4 * g4]),
+               tc[k], r);
+      tc[i] = mm(*reinterpret_cast<const f32x4*>(&Ls[16 * (wave + i) + l16][16 * (wave + i) + 4 * g4]),
+                 r, f32x4{0.f, 0.f, 0.f, 0.f});
+    }
+  __syncthreads();
+#pragma unroll
+  for (int i = 1; i < 4; ++i)
+    if (wave + i < 4) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) Ls[16 * (wave + i) + 4 * g4 + e][16 * wave + l16] = tc[i][e];
+    }
+  __syncthreads();
+  f32x4 tf[4][4];                                      // row l16 of token tile i, tokens 16 k + 4 g4 ..
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int t = 16 * i + 4 * g4 + e;
-      bb[i][e] = sb[t];
-      eb[i][e] = sb[t] * expf(sA[t]);
+    for (int k = 0; k <= i; ++k)
+      tf[i][k] = *reinterpret_cast<const f32x4*>(&Ls[16 * i + l16][16 * k + 4 * g4]);
+  const long blk = ((long)ch * H + h) * 4;
+  if (wave < 2 * NDG) {                                // Y^T = (diag(b exp A) K)^T T^T
+    f32x4 o[2][4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      f32x4 kt[2], fs;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int t = 16 * k + 4 * g4 + i;
+        const float f = sb[t] * expf(sA[t]);
+        const int d = 64 * (wave >> 1) + 4 * dl_row(l16) + 2 * (wave & 1);
+        const float2 z = *reinterpret_cast<const float2*>(&ks[t][d]);
+        kt[0][i] = z.x;
+        kt[1][i] = z.y;
+        fs[i] = f;
+      }
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        if (h == kh * (H / G))
+          put_frag(c.Kt, (((long)ch * G + kh) * (4 * NDG) + 2 * wave + j) * 4 + k, lane, kt[j]);
+        kt[j] *= fs;
+      }
+#pragma unroll
+      for (int i = k; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          o[j][i] = mm(kt[j], tf[i][k], k ? o[j][i] : f32x4{0.f, 0.f, 0.f, 0.f});
     }
-  const int nct = nb + (VP >> 4);
-  for (int ct = wave; ct < nct; ct += 4) {             // 16 columns of Y, then of X
-    const bool isy = ct < nb;
-    const float* src = isy ? K + 16 * ct : a.v + (long)h * VP + 16 * (ct - nb);
-    float* dst = isy ? c.Y + (long)h * DP + 16 * ct : c.X + (long)h * VP + 16 * (ct - nb);
-    const long lds_ = isy ? ldk : ldv, ldd = isy ? ldx : ldv;
-    f32x4 B[4], X[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int t = 16 * i + 4 * g4 + e;
-        B[i][e] = src[(long)(row0 + min(t, n - 1)) * lds_ + l16] * (isy ? eb[i][e] : bb[i][e]);
+      for (int j = 0; j < 2; ++j)
+        put_frag(c.Y, (blk + i) * (4 * NDG) + 2 * wave + j, lane, o[j][i]);
+  }
+  if (hasx) {                                          // X = T diag(b) V
+    f32x4 o[2][4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      f32x4 vt[2];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float f = sb[16 * k + 4 * g4 + i];
+        vt[0][i] = vf[k][i].x * f;
+        vt[1][i] = vf[k][i].y * f;
       }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      f32x4 r = B[i];
+      for (int i = k; i < 4; ++i)
 #pragma unroll
-      for (int k = 0; k < i; ++k) r = mm(lf[i][k], X[k], r);
-      X[i] = mm(tf[i], r, f32x4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int t = 16 * i + 4 * g4 + e;
-        if (t < n) dst[(long)(row0 + t) * ldd + l16] = X[i][e];
-      }
+        for (int j = 0; j < 2; ++j)
+          o[j][i] = mm(tf[i][k], vt[j], k ? o[j][i] : f32x4{0.f, 0.f, 0.f, 0.f});
     }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        put_frag(c.X, (blk + i) * (4 * c.ncg) + 2 * xu + j, lane, o[j][i]);
   }
 }
 
-// (2) one workgroup per (sequence, head, 16 state columns).  Wave w owns tokens 16 w .. of u and state
-// row tiles w and w + 4; u and S pass between the waves through LDS.  The next chunk's operands are
-// in flight while this one is worked on.
-template <int NB>                                      // row tiles of the state (DP / 16 <= NB)
+// (2) one workgroup per (sequence, head, tile of 16 state columns).  Wave w owns tokens 16 w .. of u and
+// NDG row tiles of the state; u and S pass between the waves through LDS.  The next chunk's operands
+// are fetched between this one's products: issued in one go they held every wave up for 2800 to 6100
+// cycles of the 9400 that a chunk took, 5800 now.  Two tiles per workgroup halve the reads but leave
+// a quarter of the CUs idle here: 93 us instead of 77.
+template <int NDG>
 __global__ void __launch_bounds__(256)
 delta_chunk_scan_kernel(DeltaArgs a, DeltaChunkArgs c) {
-  constexpr int OWN = (NB + 3) / 4;
+  constexpr int NB = 4 * NDG;                          // row tiles
   __shared__ __align__(16) f32x4 Ss[NB][64];
   __shared__ __align__(16) f32x4 Us[4][64];
-  const int s = blockIdx.x, h = blockIdx.y, cb = blockIdx.z;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g4 = lane >> 4, l16 = lane & 15;
+  const int s = blockIdx.x, h = blockIdx.y, ct = blockIdx.z;
+  const int tid = threadIdx.x, lane = tid & 63, g4 = lane >> 4, l16 = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int slot = a.slots[s];
   if (slot < 0) return;
   const int c0 = c.seq_first[s], c1 = c.seq_first[s + 1];
   if (c1 <= c0) return;
-  const int H = a.H, G = a.G, D = a.D, Dv = a.Dv, DP = a.DP, VP = a.VP, kh = h / (H / G);
-  const int nb = DP >> 4, col = 16 * cb + l16;
+  const int H = a.H, G = a.G, D = a.D, Dv = a.Dv, kh = h / (H / G), nct = 4 * c.ncg;
   const bool fresh = a.positions[c.chunks[4 * c0 + 1]] == 0;
+  const int tile0 = NDG * wave;                        // tiles tile0 .. + NDG - 1, one group's
+  const int d0 = 64 * (tile0 >> 2) + (tile0 & 3);      // entries d0 + 4 x + o
+  const int col = 64 * (ct >> 2) + 4 * l16 + (ct & 3);
   float* Sg = a.S + ((long)slot * H + h) * D * Dv;
-  f32x4 S[OWN];
+  f32x4 S[NDG];
 #pragma unroll
-  for (int o = 0; o < OWN; ++o) {
-    const int tl = wave + 4 * o;
+  for (int o = 0; o < NDG; ++o) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int r = 16 * tl + 4 * g4 + i;
+      const int r = d0 + 4 * (4 * i + g4) + o;
       S[o][i] = (!fresh && r < D && col < Dv) ? Sg[(long)r * Dv + col] : 0.f;
     }
-    if (tl < nb) Ss[tl][lane] = S[o];
+    Ss[tile0 + o][lane] = S[o];
   }
-  const long ldk = (long)G * DP, ldv = (long)H * VP, ldx = (long)H * DP;
-  const float* K = a.k + (long)kh * DP;
-  struct Op { f32x4 y[NB], x; float k[OWN][16]; float ca[4], ga; int row0, n; };
+  struct Op { f32x4 y[NB], x, k[NDG][4], ca; float ga; };
   auto load = [&](int ch, Op& p) {
-    p.row0 = c.chunks[4 * ch + 1];
-    p.n = c.chunks[4 * ch + 2];
-    p.ga = c.wsG[(long)ch * H + h];
-    const float* yp = c.Y + (long)(p.row0 + min(16 * wave + l16, p.n - 1)) * ldx + (long)h * DP + 4 * g4;
+    const long hb = (long)ch * H + h, gb = (long)ch * G + kh;
+    p.ca = *reinterpret_cast<const f32x4*>(c.cA + hb * DC + 16 * wave + 4 * g4);
+    p.ga = c.cA[hb * DC + DC - 1];
 #pragma unroll
-    for (int b = 0; b < NB; ++b)
-      p.y[b] = *reinterpret_cast<const f32x4*>(yp + 16 * (b < nb ? b : 0));
+    for (int b = 0; b < NB; ++b) p.y[b] = frag(c.Y, (hb * 4 + wave) * NB + b, lane);
+    p.x = frag(c.X, (hb * 4 + wave) * nct + ct, lane);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const long r = p.row0 + min(16 * wave + 4 * g4 + i, p.n - 1);
-      p.x[i] = c.X[r * ldv + (long)h * VP + col];
-      p.ca[i] = c.cA[r * H + h];
-    }
+    for (int o = 0; o < NDG; ++o)
 #pragma unroll
-    for (int o = 0; o < OWN; ++o) {
-      const int d = 16 * (wave + 4 * o < nb ? wave + 4 * o : 0) + l16;
-#pragma unroll
-      for (int t = 0; t < 16; ++t)                     // token 16 (t / 4) + 4 g4 + t % 4
-        p.k[o][t] = K[(long)(p.row0 + min(16 * (t >> 2) + 4 * g4 + (t & 3), p.n - 1)) * ldk + d];
-    }
+      for (int t = 0; t < 4; ++t) p.k[o][t] = frag(c.Kt, (gb * NB + tile0 + o) * 4 + t, lane);
   };
-  Op cur, nxt;
-  load(c0, cur);
-  __syncthreads();
-  for (int ch = c0; ch < c1; ++ch) {
-    load(ch + 1 < c1 ? ch + 1 : ch, nxt);
-    // the state before the chunk, for the outputs
-    float* w = c.wsS + ((long)ch * H + h) * DP * VP;
+  auto step = [&](int ch, const Op& p) {
+    const long hb = (long)ch * H + h;
 #pragma unroll
-    for (int o = 0; o < OWN; ++o)
-      if (wave + 4 * o < nb) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) w[(long)(16 * (wave + 4 * o) + 4 * g4 + i) * VP + col] = S[o][i];
-      }
+    for (int o = 0; o < NDG; ++o)                      // the state before the chunk, for the outputs
+      put_frag(c.wsS, (hb * NB + tile0 + o) * nct + ct, lane, S[o]);
     f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-    for (int b = 0; b < NB; ++b)
-      if (b < nb) acc[b & 1] = mm(cur.y[b], Ss[b][lane], acc[b & 1]);
-    f32x4 us;
+    for (int b = 0; b < NB; ++b) acc[b & 1] = mm(p.y[b], Ss[b][lane], acc[b & 1]);
+    f32x4 us = p.x - acc[0] - acc[1];
+    put_frag(c.X, (hb * 4 + wave) * nct + ct, lane, us);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int t = 16 * wave + 4 * g4 + i;
-      const float u = cur.x[i] - acc[0][i] - acc[1][i];
-      if (t < cur.n) c.X[(long)(cur.row0 + t) * ldv + (long)h * VP + col] = u;
-      us[i] = t < cur.n ? u * expf(cur.ga - cur.ca[i]) : 0.f;
-    }
+    for (int i = 0; i < 4; ++i) us[i] *= expf(p.ga - p.ca[i]);
     Us[wave][lane] = us;
-    __syncthreads();
-    const float eg = expf(cur.ga);
 #pragma unroll
-    for (int o = 0; o < OWN; ++o) {
-      f32x4 v0 = S[o] * eg, v1 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int tt = 0; tt < 4; ++tt) {
-        const f32x4 kv = {cur.k[o][4 * tt], cur.k[o][4 * tt + 1], cur.k[o][4 * tt + 2],
-                          cur.k[o][4 * tt + 3]};
-        if (tt & 1) v1 = mm(kv, Us[tt][lane], v1); else v0 = mm(kv, Us[tt][lane], v0);
-      }
-      S[o] = v0 + v1;
-      if (wave + 4 * o < nb) Ss[wave + 4 * o][lane] = S[o];
+    for (int i = 0; i < NB + 4 * NDG + 3; ++i) {       // one load per product
+      __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
     }
     __syncthreads();
-    cur = nxt;
+    const float eg = expf(p.ga);
+#pragma unroll
+    for (int o = 0; o < NDG; ++o) {
+      f32x4 v[2] = {S[o] * eg, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+      for (int tt = 0; tt < 4; ++tt) v[tt & 1] = mm(p.k[o][tt], Us[tt][lane], v[tt & 1]);
+      S[o] = v[0] + v[1];
+      Ss[tile0 + o][lane] = S[o];
+    }
+    __syncthreads();
+  };
+  Op p0, p1;
+  load(c0, p0);
+  __syncthreads();
+  for (int ch = c0; ch < c1; ch += 2) {
+    load(min(ch + 1, c1 - 1), p1);
+    step(ch, p0);
+    if (ch + 1 >= c1) break;
+    load(min(ch + 2, c1 - 1), p0);
+    step(ch + 1, p1);
   }
 #pragma unroll
-  for (int o = 0; o < OWN; ++o)
+  for (int o = 0; o < NDG; ++o)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int r = 16 * (wave + 4 * o) + 4 * g4 + i;
+      const int r = d0 + 4 * (4 * i + g4) + o;
       if (r < D && col < Dv) Sg[(long)r * Dv + col] = S[o][i];
     }
 }
 
-// (3) one workgroup per (chunk, head); wave w owns queries 16 w ..
-template <typename T, int NV>                          // value column tiles (VP / 16 <= NV)
-__global__ void __launch_bounds__(256)
+// (3) one workgroup per (chunk, head).  A wave owns one query tile and 64 columns; the waves of the same
+// queries share the weights P through LDS, key tiles in turn.  The state is read once, straight to LDS,
+// while the weights are formed.  Bound by the reads of a round of workgroups, which all come at its start.
+template <typename T, int NDG, int NCG>
+__global__ void __launch_bounds__(256 * NCG)
 delta_chunk_out_kernel(DeltaArgs a, DeltaChunkArgs c) {
-  __shared__ float sA[DC];
-  const int ch = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int NB = 4 * NDG, NCT = 4 * NCG;
+  __shared__ __align__(16) f32x4 Ss[NB * NCT][64];
+  __shared__ __align__(16) f32x4 Ps[10][64];
+  __shared__ float red[NCG][DC];
+  const int ch = blockIdx.y, h = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int s = c.chunks[4 * ch], row0 = c.chunks[4 * ch + 1], n = c.chunks[4 * ch + 2];
   if (a.slots[s] < 0) return;
-  const int H = a.H, G = a.G, Dv = a.Dv, DP = a.DP, VP = a.VP, kh = h / (H / G);
-  const int g4 = lane >> 4, l16 = lane & 15, nb = DP >> 4, nv = VP >> 4;
-  if (tid < DC) sA[tid] = c.cA[(long)(row0 + min(tid, n - 1)) * H + h];
-  __syncthreads();
-  if (16 * wave >= n) return;
-  const long ldk = (long)G * DP, ldv = (long)H * VP;
-  const int tq = 16 * wave + l16;                      // this lane's query
-  const float* qp = a.q + (long)(row0 + min(tq, n - 1)) * ldk + (long)kh * DP + 4 * g4;
-  f32x4 qf[8];
+  const int H = a.H, G = a.G, Dv = a.Dv, DP = a.DP, kh = h / (H / G);
+  const int g4 = lane >> 4, l16 = lane & 15, cg = wave % NCG, qt = wave / NCG;
+  const long ldk = (long)G * DP, hb = (long)ch * H + h;
+  // entries 64 g + 4 (4 i + g4) + j of a row, i = 0 .. 3: the k of tile j's fragment
+  auto rows = [&](const float* base, int tile, f32x4 (&f)[NDG][4]) {
+    const float* p = base + (long)(row0 + min(16 * tile + l16, n - 1)) * ldk + (long)kh * DP;
 #pragma unroll
-  for (int b = 0; b < 8; ++b)
-    if (b < nb) qf[b] = *reinterpret_cast<const f32x4*>(qp + 16 * b);
-  f32x4 o[NV];
+    for (int g = 0; g < NDG; ++g)
 #pragma unroll
-  for (int t = 0; t < NV; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // weights of the chunk's own tokens: P^T = K Q^T, so that its registers are the A operand of P u
-  for (int kt = 0; kt <= wave; ++kt) {
-    const float* kp = a.k + (long)(row0 + min(16 * kt + l16, n - 1)) * ldk + (long)kh * DP + 4 * g4;
-    f32x4 p = {0.f, 0.f, 0.f, 0.f};
+      for (int i = 0; i < 4; ++i) {
+        const f32x4 z = *reinterpret_cast<const f32x4*>(p + min(64 * g + 16 * i + 4 * g4, DP - 4));
 #pragma unroll
-    for (int b = 0; b < 8; ++b)
-      if (b < nb) p = mm(*reinterpret_cast<const f32x4*>(kp + 16 * b), qf[b], p);
-    const float* up[4];
+        for (int j = 0; j < 4; ++j) f[g][j][i] = z[j];
+      }
+  };
+  f32x4 qf[NDG][4], kf[NDG][4];
+  rows(a.q, qt, qf);
+  rows(a.k, cg, kf);
+  const float* cA = c.cA + hb * DC;
+  const int tq = 16 * qt + l16;
+  const float aq = cA[tq];
+  const f32x4 ar = *reinterpret_cast<const f32x4*>(cA + 16 * qt + 4 * g4);
+  f32x4 ak = *reinterpret_cast<const f32x4*>(cA + 16 * cg + 4 * g4);
+  // the state goes to LDS while the weights are formed; nothing reads LDS until it is there
+#pragma unroll
+  for (int t = 0; t < NB; ++t) {
+    const int tile = wave + 4 * NCG * t;
+    __builtin_amdgcn_global_load_lds(
+        (const __attribute__((address_space(1))) void*)(c.wsS + (hb * NB * NCT + tile) * 256 + 4 * lane),
+        (__attribute__((address_space(3))) void*)&Ss[tile][0], 16, 0, 0);
+  }
+  if (DP & 63) {                                       // entries past DP are not the row's
+#pragma unroll
+    for (int g = 0; g < NDG; ++g)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (64 * g + 16 * i + 4 * g4 >= DP) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) qf[g][j][i] = 0.f;
+        }
+  }
+  // P^T = K Q^T: its registers are the A operand of P u
+  for (int kt = cg; kt <= qt; kt += NCG) {
+    if (kt != cg) {
+      rows(a.k, kt, kf);
+      ak = *reinterpret_cast<const f32x4*>(cA + 16 * kt + 4 * g4);
+    }
+    f32x4 p[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int b = 0; b < NB; ++b) p[b & 1] = mm(kf[b >> 2][b & 3], qf[b >> 2][b & 3], p[b & 1]);
+    f32x4 w;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int tk = 16 * kt + 4 * g4 + i;
-      p[i] = tk <= tq && tk < n ? p[i] * expf(sA[tq] - sA[tk]) : 0.f;
-      up[i] = c.X + (long)(row0 + min(tk, n - 1)) * ldv + (long)h * VP + l16;
+      w[i] = tk <= tq && tk < n ? (p[0][i] + p[1][i]) * expf(aq - ak[i]) : 0.f;
     }
-#pragma unroll
-    for (int t = 0; t < NV; ++t) {
-      const int ct = t < nv ? t : 0;
-      o[t] = mm(p, f32x4{up[0][16 * ct], up[1][16 * ct], up[2][16 * ct], up[3][16 * ct]}, o[t]);
-    }
+    Ps[qt * (qt + 1) / 2 + kt][lane] = w;
   }
-  const float eA = expf(sA[tq]);
-  const float* Sb = c.wsS + ((long)ch * H + h) * DP * VP + (long)4 * g4 * VP + l16;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  f32x4 z[4], o[4];
 #pragma unroll
-  for (int b = 0; b < 8; ++b) {
-    if (b >= nb) break;
-    const f32x4 qa = qf[b] * eA;
-    const float* sp = Sb + (long)16 * b * VP;
+  for (int j = 0; j < 4; ++j) z[j] = frag(c.X, hb * 4 * NCT + 4 * cg + j, lane);
 #pragma unroll
-    for (int t = 0; t < NV; ++t) {
-      const int ct = 16 * (t < nv ? t : 0);
-      o[t] = mm(qa, f32x4{sp[ct], sp[VP + ct], sp[2 * VP + ct], sp[3 * VP + ct]}, o[t]);
-    }
+  for (int j = 0; j < 4; ++j) o[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      o[j] = mm(qf[b >> 2][b & 3], Ss[b * NCT + 4 * cg + j][lane], o[j]);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float e = expf(ar[i]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[j][i] *= e;
   }
-  // head RMS norm (columns past Dv are zero), weight, gate
+  for (int kt = 0; kt <= qt; ++kt) {
+    f32x4 zn[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) zn[j] = frag(c.X, (hb * 4 + min(kt + 1, qt)) * NCT + 4 * cg + j, lane);
+    const f32x4 w = Ps[qt * (qt + 1) / 2 + kt][lane];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[j] = mm(w, z[j], o[j]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) z[j] = zn[j];
+  }
+  // head RMS norm, weight, gate
+  const int col = 64 * cg + 4 * l16;
+  float ss[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float z = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) z += col + j < Dv ? o[j][i] * o[j][i] : 0.f;
+    z += __shfl_xor(z, 1, 64);
+    z += __shfl_xor(z, 2, 64);
+    z += __shfl_xor(z, 4, 64);
+    z += __shfl_xor(z, 8, 64);
+    ss[i] = z;
+    if (NCG == 2 && l16 == 0) red[cg][16 * qt + 4 * g4 + i] = z;
+  }
+  if (NCG == 2) __syncthreads();
   const T* NW = static_cast<const T*>(a.norm_w);
   const T* GT = static_cast<const T*>(a.g);
   T* Yo = static_cast<T*>(a.y);
+  if (col >= Dv) return;
+  float nw[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) nw[j] = ld_f32<T>(NW, min(col + j, Dv - 1)) * a.out_scale;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    float ss = 0.f;
-#pragma unroll
-    for (int t = 0; t < NV; ++t) ss += t < nv ? o[t][i] * o[t][i] : 0.f;
-    ss += __shfl_xor(ss, 1, 64);
-    ss += __shfl_xor(ss, 2, 64);
-    ss += __shfl_xor(ss, 4, 64);
-    ss += __shfl_xor(ss, 8, 64);
-    const int tr = 16 * wave + 4 * g4 + i;
+    const int tr = 16 * qt + 4 * g4 + i;
     if (tr >= n) continue;
-    const float inv = a.out_scale / sqrtf(ss / (float)Dv + a.eps);
+    const float sq = NCG == 2 ? ss[i] + red[NCG - 1 - cg][tr] : ss[i];
+    const float inv = 1.0f / sqrtf(sq / (float)Dv + a.eps);
     const long r = row0 + tr;
+    const T* gp = GT + r * a.ldg + (long)h * Dv + col;
+    T* yp = Yo + r * a.ldy + (long)h * Dv + col;
+    if (c.vec) {
+      typedef T T4 __attribute__((ext_vector_type(4)));
+      const T4 gz = *reinterpret_cast<const T4*>(gp);
+      T4 yz;
 #pragma unroll
-    for (int t = 0; t < NV; ++t) {
-      const int d = 16 * t + l16;
-      if (d < Dv)
-        st_f32<T>(Yo + r * a.ldy, (long)h * Dv + d,
-                  o[t][i] * inv * ld_f32<T>(NW, d) * dl_silu(ld_f32<T>(GT + r * a.ldg, (long)h * Dv + d)));
+      for (int j = 0; j < 4; ++j) {
+        const T gj = gz[j];
+        T v;
+        st_f32<T>(&v, 0, o[j][i] * inv * nw[j] * dl_silu(ld_f32<T>(&gj, 0)));
+        yz[j] = v;
+      }
+      *reinterpret_cast<T4*>(yp) = yz;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (col + j < Dv) st_f32<T>(yp, j, o[j][i] * inv * nw[j] * dl_silu(ld_f32<T>(gp, j)));
     }
   }
 }
 
 // As eia_delta_scan for sequences whose chunk list is given (chunks int32 [nchunk, 4]: sequence,
 // first row, tokens (1 .. 64), 0; seq_first int32 [nseq + 1], indexed by sequence), with fp32
-// workspaces Y [rows, H, DP], X [rows, H, VP], wsS [nchunk, H, DP, VP], cA [rows, H],
-// wsG [nchunk, H]; DP and VP multiples of 16, at most 128.
+// workspaces Y [nchunk, H, 64, DQ], X [nchunk, H, 64, VQ], Kt [nchunk, G, DQ, 64], wsS [nchunk, H, DQ,
+// VQ], cA [nchunk, H, 64], 16-byte aligned; DP and VP multiples of 16, at most 128, DQ and VQ the
+// same rounded up to 64.
 EIA_API int eia_delta_scan_chunked(const float* q, const float* k, const float* v, const float* la,
                                    const float* beta, int H, int G, int D, int Dv, int DP, int VP,
                                    const void* g, long ldg, const void* norm_w, float out_scale,
                                    float eps, float* S, const int* slots, const int* positions,
                                    void* y, long ldy, int nseq, const int* chunks,
-                                   const int* seq_first, int nchunk, float* Y, float* X, float* wsS,
-                                   float* cA, float* wsG, int is_bf16, hipStream_t st) {
+                                   const int* seq_first, int nchunk, float* Y, float* X, float* Kt,
+                                   float* wsS, float* cA, int is_bf16, hipStream_t st) {
   DeltaArgs a{q, k, v, la, beta, H, G, D, Dv, DP, VP, g, ldg, norm_w, out_scale, eps, S, slots,
               nullptr, positions, nullptr, y, ldy};
-  if (!delta_args_ok(a, nseq) || nchunk < 0 || !chunks || !seq_first || !Y || !X || !wsS || !cA ||
-      !wsG || DP % 16 || VP % 16)
+  if (!delta_args_ok(a, nseq) || nchunk < 0 || !chunks || !seq_first || !Y || !X || !Kt || !wsS || !cA ||
+      DP % 16 || VP % 16)
     return EIA_BAD_SHAPE;
   if (DP > 128 || VP > 128) return EIA_UNSUPPORTED;
   if (nseq == 0 || nchunk == 0) return EIA_OK;
-  DeltaChunkArgs c{chunks, seq_first, Y, X, wsS, cA, wsG};
-  const dim3 gc(nchunk, H), gs(nseq, H, VP / 16);
-  hipLaunchKernelGGL(delta_chunk_solve_kernel, gc, dim3(256), 0, st, a, c);
-  if (DP <= 64) hipLaunchKernelGGL((delta_chunk_scan_kernel<4>), gs, dim3(256), 0, st, a, c);
-  else hipLaunchKernelGGL((delta_chunk_scan_kernel<8>), gs, dim3(256), 0, st, a, c);
-#define DO_GO(TT, NV) \
-  hipLaunchKernelGGL((delta_chunk_out_kernel<TT, NV>), gc, dim3(256), 0, st, a, c)
-  if (is_bf16) { if (VP <= 64) DO_GO(bf16_t, 4); else DO_GO(bf16_t, 8); }
-  else { if (VP <= 64) DO_GO(float, 4); else DO_GO(float, 8); }
+  const int ndg = (DP + 63) / 64, ncg = (VP + 63) / 64, es = is_bf16 ? 2 : 4;
+  const bool vec = Dv % 4 == 0 && ldy % 4 == 0 && ldg % 4 == 0 &&
+                   (reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(g)) % (4 * es) == 0;
+  DeltaChunkArgs c{chunks, seq_first, Y, X, Kt, wsS, cA, ncg, vec};
+  const dim3 gc(H, nchunk), b(256);
+#define DO_GO(TT, A, B) \
+  hipLaunchKernelGGL((delta_chunk_out_kernel<TT, A, B>), gc, dim3(256 * B), 0, st, a, c)
+#define DO_DIMS(A, B)                                                                              \
+  do {                                                                                             \
+    hipLaunchKernelGGL(delta_chunk_solve_kernel<A>, gc, b, 0, st, a, c);                           \
+    hipLaunchKernelGGL(delta_chunk_scan_kernel<A>, dim3(nseq, H, 4 * ncg), b, 0, st, a, c);        \
+    if (is_bf16) DO_GO(bf16_t, A, B); else DO_GO(float, A, B);                                     \
+  } while (0)
+  if (ndg == 2) { if (ncg == 2) DO_DIMS(2, 2); else DO_DIMS(2, 1); }
+  else { if (ncg == 2) DO_DIMS(1, 2); else DO_DIMS(1, 1); }
+#undef DO_DIMS
 #undef DO_GO
   EIA_LAUNCH_CHECK();
 }

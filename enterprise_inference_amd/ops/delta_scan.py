@@ -343,10 +343,11 @@ def delta_scan(rows: DeltaRows, spec: DeltaSpec, state: DeltaState, md, norm_w: 
     step(0, nd)
     dev = out.device
     f32 = lambda *s: torch.empty(*s, dtype=torch.float32, device=dev)
-    Y, X, wsS = f32(T, H, DP), f32(T, H, VP), f32(plan.n, H, DP, VP)
-    cA, wsG = f32(T, H), f32(plan.n, H)
+    DQ, VQ, n = -(-DP // 64) * 64, -(-VP // 64) * 64, plan.n
+    Y, X = f32(n, H, CHUNK, DQ), f32(n, H, CHUNK, VQ)
+    Kt, wsS, cA = f32(n, G, DQ, CHUNK), f32(n, H, DQ, VQ), f32(n, H, CHUNK)
     check(lib().eia_delta_scan_chunked(
         *common, ptr(md.seq_slots[nd:]), ptr(md.positions), ptr(out), out.stride(0), plan.nseq,
-        ptr(plan.chunks), ptr(plan.seq_first), plan.n, ptr(Y), ptr(X), ptr(wsS), ptr(cA), ptr(wsG),
-        1 if bf else 0, stream(out)), "delta_scan_chunked")
+        ptr(plan.chunks), ptr(plan.seq_first), n, ptr(Y), ptr(X), ptr(Kt), ptr(wsS),
+        ptr(cA), 1 if bf else 0, stream(out)), "delta_scan_chunked")
     return out

@@ -92,3 +92,42 @@ def test_linear_chunks(lens, H, D, Dv, mode, rot, half, dtype, monkeypatch):
     assert _rel(z[live], y[live]) < (1e-5 if dtype == torch.float32 else 4e-3)
     for u, v in ((a.S, b.S), (a.n, b.n), (a.m, b.m)):
         assert u is None or _rel(v, u) < 2e-6
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,G,D,Dv", [(4, 2, 128, 128), (2, 2, 64, 64), (3, 1, 72, 40),
+                                      (2, 1, 16, 120), (2, 2, 112, 6)])
+@pytest.mark.parametrize("lens", [[1, 64, 63, 65, 130], [200], [15, 16, 17, 129, 3]])
+def test_delta_chunks(lens, H, G, D, Dv, dtype, monkeypatch):
+    from types import SimpleNamespace
+    from enterprise_inference_amd.ops import delta_scan as ds
+    monkeypatch.setattr(ds, "FORCE_CHUNKED", True)
+    g = torch.Generator().manual_seed(sum(lens) + D)
+    rnd = lambda *s: torch.randn(*s, generator=g)
+    n, T = len(lens), sum(lens)
+    cu, pos, slots = _step(lens, [0 if s % 2 == 0 else 5 for s in range(n)], n > 3)
+    pad = lambda t, m: torch.nn.functional.pad(t, (0, -(-m // 16) * 16 - m))
+    unit = lambda t: t / t.norm(dim=-1, keepdim=True)
+    rows = [pad(unit(rnd(T, G, D)), D), pad(unit(rnd(T, G, D)), D), pad(rnd(T, H, Dv), Dv),
+            -torch.rand(T, H, generator=g) ** 4, torch.sigmoid(2.0 * rnd(T, H)),
+            rnd(T, H * Dv).to(dtype)]
+    S0, nw = rnd(n, H, D, Dv), (1 + 0.1 * rnd(Dv)).to(dtype)
+
+    def run(dev):
+        md = SimpleNamespace(seq_cu=cu.to(dev), seq_slots=slots.to(dev), positions=pos.to(dev),
+                             num_seqs=n, num_decode=0, num_prefill_tokens=T, prefill_q_lens=lens,
+                             decode_seq_lens=None, work_cache={})
+        st = ds.DeltaState(S0.clone().to(dev), None)
+        spec = ds.DeltaSpec(H, G, D, Dv, 1, eps=1e-6, out_scale=0.7)
+        plan = ds.prefill_plan(md, torch.device(dev)) if dev == "cuda" else None
+        wide = torch.empty(T, H * Dv + 1, dtype=dtype, device=dev)      # rows of any alignment
+        y = ds.delta_scan(ds.DeltaRows(*(t.to(dev) for t in rows)), spec, st, md, nw.to(dev),
+                          wide[:, 1:] if D == 128 and n == 1 else None, plan)
+        return y.cpu(), st.S.cpu()
+
+    (y, S), (z, Z) = run("cpu"), run("cuda")
+    live = torch.cat([torch.full((m,), int(s) >= 0) for m, s in zip(lens, slots)])
+    # fp32 sums over at most 128 products and a 64-row triangular solve; bf16 adds one rounding and
+    # at times one step more
+    assert _rel(z[live], y[live]) < (1e-5 if dtype == torch.float32 else 4e-3)
+    assert _rel(Z, S) < 4e-6

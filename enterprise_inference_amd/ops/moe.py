@@ -2,16 +2,14 @@
 
 Both regimes run entirely on the device with no host synchronisation: top-k routing,
 on-device expert alignment (offsets + sorted token list), grouped gate_up GEMM with the
-SwiGLU epilogue, grouped down GEMM, weighted combine.  Decode-sized batches (<= 96 rows per
-expert on average) use the weight-streaming grouped skinny GEMM (gemm_skinny.hip); prefill-
-sized batches use the MFMA grouped GEMM (moe_gemm.hip), whose grid is an upper bound that
-each workgroup maps to (expert, M tile) from the device-side offsets (graph-capturable).  Past
-128 rows per expert hipBLASLt's tiles are faster (Mixtral-8x7B, profiles/moe_bench_r2.log:
-512 / 2048 / 8192 tokens = 0.98 / 1.89 / 5.19 ms against 1.08 / 2.42 / 8.13 ms for the
-grouped MFMA kernel), so that regime reads the E+1 offsets back once per layer and runs one
-GEMM pair per expert on contiguous slices of the sorted rows (the old path synchronised once
-per expert through nonzero() and scattered with fp32 index_add: 1.43 ms at 65 tokens,
-profiles/moe_bench_r2.log first run).
+SwiGLU epilogue, grouped down GEMM, weighted combine.  Decode-sized batches use the
+weight-streaming grouped skinny GEMM (gemm_skinny.hip); from a few dozen rows per expert the
+MFMA grouped GEMM (moe_gemm.hip) is faster, whose grid is an upper bound that each workgroup maps
+to (expert, tile) from the device-side offsets (graph-capturable).  Past GROUPED_MAX_ROWS rows per
+expert hipBLASLt's larger tiles are level with it, so that regime reads the E+1 offsets back once
+per layer and runs one GEMM pair per expert on contiguous slices of the sorted rows (the old path
+synchronised once per expert through nonzero() and scattered with fp32 index_add: 1.43 ms at 65
+tokens, profiles/moe_bench_r2.log first run).
 
 Expert parallelism (``--enable-expert-parallel``, core/helm-charts/vllm/gaudi3-values.yaml:492):
 rank r owns experts [e_lo, e_hi); tokens routed elsewhere contribute zero locally
@@ -183,13 +181,14 @@ def fused_moe(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, topk_w: torc
         return ref.fused_moe(x, w13, w2, tw, ids.clamp(0, El - 1).to(torch.int32), act)
     avg = T * k / max(1, El)
     capturable = capturable or torch.cuda.is_current_stream_capturing()
-    if act == "silu" and avg <= 96 and _grouped_ok(x, w13, w2):
+    if act == "silu" and _grouped_ok(x, w13, w2) and not (
+            _mfma_ok(x, w13, w2) and _mfma_pays(avg, El, w13.shape[1] // 2, H)) and avg <= 96:
         return _fused_moe_grouped(x, w13, w2, topk_w, topk_ids, e_lo, e_hi,
                                   defer_combine=defer_combine)
     # (small experts stay on the grouped MFMA kernel at any row count: their per-expert library
     # GEMMs are launch- and read-back-bound, not MFMA-bound)
     if act == "silu" and _mfma_ok(x, w13, w2) and (
-            avg <= MFMA_MAX_ROWS or capturable
+            avg <= GROUPED_MAX_ROWS or capturable
             or (w13.shape[1] // 2) * H <= UNGATED_SMALL_EXPERT):
         return _fused_moe_grouped(x, w13, w2, topk_w, topk_ids, e_lo, e_hi, mfma=True)
     if capturable:
@@ -203,13 +202,32 @@ def fused_moe(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, topk_w: torc
     return _fused_moe_per_expert(x, w13, w2, topk_w, topk_ids, e_lo, act)
 
 
-MFMA_MAX_ROWS = 128      # rows per expert above which the per-expert hipBLASLt GEMMs win
+# rows per expert above which the per-expert hipBLASLt GEMMs win: ungated experts, and SwiGLU ones
+# (Mixtral-8x7B, grouped against per expert: 256 rows 1149 / 1256 us, 512 rows 1822 / 1839 us)
+MFMA_MAX_ROWS = 128
+GROUPED_MAX_ROWS = 384
+
+
+def _mfma_pays(avg: float, El: int, I: int, H: int) -> bool:
+    """Whether the MFMA grouped GEMM beats the weight-streaming skinny one at ``avg`` rows per expert.
+    The skinny kernel goes over the weights once per 16 to 128 rows, the MFMA kernel once per 128.
+    us, skinny / MFMA: 8 experts of 4096 x 14336, 40 rows 546 / 545, 65 rows 672 / 551; 8 of 1024 x
+    512 (64 workgroups: half the chip idles), 50 rows 28.4 / 29.1, 95 rows 40 / 31.  Experts that
+    fill the chip and whose weights stay in the 256 MB cache gain sooner: 16 of 2048 x 1024, 25 rows
+    56 / 45, 50 rows 73 / 46."""
+    return avg > 48 or (avg > 24 and El * (I // 64) >= 256 and 6 * El * I * H <= 1 << 28)
 
 
 def _mfma_ok(x, w13, w2) -> bool:
     H, I = x.shape[1], w13.shape[1] // 2
     return (x.dtype == torch.bfloat16 and H % 128 == 0 and I % 64 == 0
-            and w13.is_contiguous() and w2.is_contiguous() and x.stride(1) == 1)
+            and w13.is_contiguous() and w2.is_contiguous() and x.stride(1) == 1
+            and x.stride(0) % 8 == 0)
+
+
+def _aligned16(t):
+    """The MFMA grouped GEMM's operands go straight to LDS, 16 bytes at a time."""
+    return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
 def _fused_moe_grouped(x, w13, w2, topk_w, topk_ids, e_lo, e_hi, mfma: bool = False,
@@ -225,6 +243,7 @@ def _fused_moe_grouped(x, w13, w2, topk_w, topk_ids, e_lo, e_hi, mfma: bool = Fa
     h1 = torch.empty(max(1, n), I, dtype=x.dtype, device=dev)
     h2 = torch.empty(max(1, n), H, dtype=x.dtype, device=dev)
     if mfma:
+        x, w13, w2 = _aligned16(x), _aligned16(w13), _aligned16(w2)
         check(lib().eia_moe_grouped_gemm(ptr(x), x.stride(0), ptr(row_idx), ptr(w13), I2, H, El,
                                          ptr(offs), n, 1, ptr(h1), h1.stride(0), st),
               "moe_grouped_gemm_gate_up")
@@ -475,6 +494,7 @@ def ungated_moe(x: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor, topk_
             avg <= MFMA_MAX_ROWS or capturing or I * H <= UNGATED_SMALL_EXPERT):
         h1 = torch.empty(max(1, n), I, dtype=x.dtype, device=dev)
         h2 = torch.empty(max(1, n), H, dtype=x.dtype, device=dev)
+        x, w_up, w_down = _aligned16(x), _aligned16(w_up), _aligned16(w_down)
         check(lib().eia_moe_grouped_gemm(ptr(x), x.stride(0), ptr(row_idx), ptr(w_up), I, H, E,
                                          ptr(offs), n, 2, ptr(h1), h1.stride(0), st),
               "moe_grouped_gemm_up_relu2")

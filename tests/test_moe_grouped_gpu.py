@@ -1,0 +1,53 @@
+"""The MFMA grouped expert GEMM: K steps around the length of its LDS ring, slices around its row
+tiles, and the sizes at which fused_moe turns to it."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+BF = torch.bfloat16
+
+
+@pytest.mark.parametrize("form", [0, 1, 2])
+@pytest.mark.parametrize("K", [64, 128, 192, 320, 640])
+@pytest.mark.parametrize("counts", [[1, 0, 127, 128, 129, 65], [0] * 65 + [200, 0, 3]])
+def test_grouped_gemm(counts, K, form):
+    from enterprise_inference_amd._native import kernels as lib
+    from enterprise_inference_amd.ops._dispatch import ptr, stream
+    g = torch.Generator().manual_seed(K + form)
+    E, n, N = len(counts), sum(counts), 384
+    X = torch.randn(300, K, generator=g).to("cuda", BF)
+    row_idx = torch.randint(0, 300, (n,), generator=g).to("cuda", torch.int32)
+    offs = torch.tensor([0] + counts).cumsum(0).to("cuda", torch.int32)
+    W = (torch.randn(E, N, K, generator=g) * K ** -0.5).to("cuda", BF)
+    out = torch.full((n, N // 2 if form == 1 else N), float("nan"), device="cuda", dtype=BF)
+    assert lib().eia_moe_grouped_gemm(ptr(X), X.stride(0), ptr(row_idx), ptr(W), N, K, E, ptr(offs),
+                                      n, form, ptr(out), out.stride(0), stream(X)) == 0
+    xs = X.double()[row_idx.long()]
+    for e, (a, b) in enumerate(zip(offs.tolist(), offs.tolist()[1:])):
+        y = xs[a:b] @ W[e].double().t()
+        if form == 1:
+            y = torch.nn.functional.silu(y[:, :N // 2]) * y[:, N // 2:]
+        elif form == 2:
+            y = torch.relu(y) ** 2
+        # fp32 sums of K exact products, one bf16 rounding (2^-9) and a fast exponential
+        assert a == b or ((out[a:b].double() - y).norm() / y.norm()) < 3e-3
+
+
+@pytest.mark.parametrize("T,E,H,I", [(100, 4, 512, 256), (96, 4, 512, 256), (200, 16, 1024, 1024),
+                                     (600, 4, 512, 4352)])
+@pytest.mark.parametrize("shift", [0, 4])
+def test_fused_moe_rows_per_expert(T, E, H, I, shift):
+    from enterprise_inference_amd.ops import moe
+    from enterprise_inference_amd.ops import reference as ref
+    g = torch.Generator().manual_seed(T)
+    x = torch.randn(T * H + shift, generator=g).to(BF)[shift:].view(T, H)
+    w13 = (torch.randn(E, 2 * I, H, generator=g) * H ** -0.5).to(BF)
+    w2 = (torch.randn(E, H, I, generator=g) * I ** -0.5).to(BF)
+    w, ids = torch.topk(torch.softmax(torch.randn(T, E, generator=g), -1), 2, -1)
+    ids = ids.to(torch.int32)
+    xd = torch.empty(T * H + shift, dtype=BF, device="cuda")[shift:].view(T, H).copy_(x)
+    out = moe.fused_moe(xd, *(t.cuda() for t in (w13, w2, w, ids))).double().cpu()
+    r = ref.fused_moe(x, w13, w2, w, ids).double()
+    # hidden rows, expert outputs and sums are rounded to bf16 on both sides: 3 x 1.7e-3 each
+    assert (out - r).norm() / r.norm() < 1.1e-2

@@ -314,9 +314,11 @@ EIA_API int eia_linear_scan(const void* x, long ld, int q_off, int k_off, int v_
 // traffic (4 passes over chunks x H x dk x dv floats), and halving their number costs less than the
 // longer sums inside a chunk add.
 // Four prompts of 1000 .. 2000 tokens (6688 rows), 16 heads of 128, mode 1, bf16 take 13 + 57 + 21 +
-// 122 us on an MI355X (gates, (1), (2), (3)); in 32-token chunks of vector FMAs with a thread per state
-// column it was 63 + 151 + 119 + 581 us.  (3) spends 33 us of it in matrix products and 28 us in
-// vector issue; the rest is waiting for the 64 KiB state that each wave reads.
+// 103 us on an MI355X (gates, (1), (2), (3)); in 32-token chunks of vector FMAs with a thread per state
+// column it was 63 + 151 + 119 + 581 us.  (3) spends 40 us of it in matrix products and 28 us in
+// vector issue; the rest is waiting for reads, which a round of workgroups makes all at its start.
+// The 64 KB state goes through the LDS that the keys and values take after it: read by every wave for
+// itself (3) took 122 us.
 constexpr int LK = 128;                     // tokens per chunk
 constexpr int LS_AHEAD = 8;                 // chunks whose contributions are in flight in (2)
 constexpr float LS_LOG2E = 1.4426950408889634f;
@@ -691,35 +693,36 @@ ls_chunk_out_kernel(ScanArgs a, KChunkArgs c) {
   // unrotated bf16 keys and queries meet as they are; else both are fp32
   constexpr bool BF = sizeof(T) == 2 && !ROT;
   using KT = typename std::conditional<BF, T, float>::type;
-  __shared__ __align__(16) KT sk[LK * MX];
-  __shared__ __align__(16) T sv[LK * MX];
-  __shared__ float pre[LK], suf[LK], mb[LK], tot[LK / 16];
+  constexpr bool PRE = BF && VEC;            // keys fetched while the state is used
+  constexpr int KV = LK * MX * (int)(sizeof(KT) + sizeof(T));
+  __shared__ __align__(16) unsigned char tiles[KV > MX * MX * 4 ? KV : MX * MX * 4];
+  float* sS = reinterpret_cast<float*>(tiles);         // [MX][MX] the state, then keys and values
+  KT* sk = reinterpret_cast<KT*>(tiles);
+  T* sv = reinterpret_cast<T*>(sk + LK * MX);
+  __shared__ float pre[LK], suf[LK], mb[LK], tot[LK / 16], sn[MX];
   int s, row0, n;
   if (!ls_chunk(a, c.nseq, blockIdx.x, s, row0, n)) return;
   const int h = blockIdx.y, lane = threadIdx.x & 63, wv = threadIdx.x >> 6, D = a.D, Dv = a.Dv;
   const int w = wv < 4 ? wv : 11 - wv, l16 = lane & 15, g4 = lane >> 4, t0 = 16 * w;
-  ls_chunk_logs(a, c, row0, n, h, pre, suf, tot, mb);
-  ls_stage_v<T, VEC, MX, LK, 512>(a, row0, n, h, 0, sv);
+  const bool state = row0 != a.cu[s] || a.positions[a.cu[s]] != 0;   // (else a fresh sequence: S = 0)
+  if (state) {                                         // straight to LDS, 1 KB per access
+    const float* S = c.U + ((long)blockIdx.x * a.H + h) * c.DP * c.UW;
 #pragma unroll
-  for (int u = threadIdx.x; u < LK * MX / 8; u += 512) {
-    const int t = u / (MX / 8), i = 8 * (u % (MX / 8));
-    float v[8];
-    ls_head8<T, VEC, ROT>(a, c, row0 + min(t, n - 1), a.k_off + (long)h * D, i, v);
-    if constexpr (BF) {
-      bf16x8 b;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) b[e] = t < n ? (bf16_t)v[e] : (bf16_t)0.f;
-      *reinterpret_cast<bf16x8*>(sk + ls_kat<MX, KT>(t, i)) = b;
-    } else {
-#pragma unroll
-      for (int x = 0; x < 8; x += 4)
-        *reinterpret_cast<f32x4*>(sk + ls_kat<MX, KT>(t, i + x)) =
-            t < n ? f32x4{v[x], v[x + 1], v[x + 2], v[x + 3]} : f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int u = 0; u < MX * MX / 256 / 8; ++u) {
+      const int at = 256 * (8 * u + wv), r = (at + 4 * lane) / MX, d = (at + 4 * lane) % MX;
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) void*)(S + (long)min(r, c.DP - 1) * c.UW +
+                                                          (d < c.VP ? d : 0)),
+          (__attribute__((address_space(3))) void*)(sS + __builtin_amdgcn_readfirstlane(at)), 16, 0, 0);
     }
+    if (a.mode == 1 && threadIdx.x < MX)
+      sn[threadIdx.x] = S[(long)min((int)threadIdx.x, c.DP - 1) * c.UW + c.VP];
   }
+  ls_chunk_logs(a, c, row0, n, h, pre, suf, tot, mb);
   // this lane's query: channels 32 x + 8 g4 + e
   const int tq = t0 + l16;
-  KT qf[MX / 32][8];
+  typedef KT KT8 __attribute__((ext_vector_type(8)));
+  KT8 qf[MX / 32];
 #pragma unroll
   for (int x = 0; x < MX / 32; ++x) {
     float v[8];
@@ -727,26 +730,90 @@ ls_chunk_out_kernel(ScanArgs a, KChunkArgs c) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) qf[x][e] = (KT)v[e];
   }
+  constexpr int NU = LK * MX / 8 / 512;                // units of 8 channels per thread
+  f32x4 kp[PRE ? NU : 1];                              // (the values too: 84 bytes spilled, 109 us)
+  const T* X0 = static_cast<const T*>(a.x) + (long)row0 * a.ld;
+  if constexpr (PRE) {
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      const int at = threadIdx.x + 512 * u, t = min(at / (MX / 8), n - 1), i = 8 * (at % (MX / 8));
+      const T* r = X0 + (long)t * a.ld;
+      kp[u] = *reinterpret_cast<const f32x4*>(r + a.k_off + (long)h * D + (i < D ? i : 0));
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  if (t0 >= n) return;
-  const float qk = a.qscale * a.kscale;
   f32x4 o[MX / 16];
 #pragma unroll
   for (int j = 0; j < MX / 16; ++j) o[j] = f32x4{0.f, 0.f, 0.f, 0.f};
   float rs = 0.f;                                      // row sum of query l16 (this lane's keys)
-  float back = 0.f;                                    // l from the end of block b to the query's
   const float pq = pre[tq];
+  if (state && t0 < n) {
+    float front = 0.f;                                 // l of the blocks before the query's
+    for (int b = 0; b < w; ++b) front += tot[b];
+    const float eq = a.qscale * __builtin_amdgcn_exp2f(pq + front);
+#pragma unroll
+    for (int x = 0; x < MX / 32; ++x)
+#pragma unroll
+      for (int e = 0; e < 8; e += 4) {
+        const int i = 32 * x + 8 * g4 + e;
+        if (32 * x >= c.DP) break;
+        const f32x4 qa = f32x4{(float)qf[x][e], (float)qf[x][e + 1], (float)qf[x][e + 2],
+                               (float)qf[x][e + 3]} * eq;
+#pragma unroll
+        for (int y = 0; y < 4; ++y) {
+          if (a.mode == 1) rs += qa[y] * sn[i + y];
+#pragma unroll
+          for (int z = 0; z < MX / 64; ++z) {
+            const f32x4 v = *reinterpret_cast<const f32x4*>(sS + (i + y) * MX + 64 * z + 4 * l16);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              o[4 * z + j] = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[y], v[j], o[4 * z + j], 0, 0, 0);
+          }
+        }
+      }
+  }
+  __syncthreads();                                     // the state was read
+  if constexpr (PRE) {
+    ls_stage_v<T, VEC, MX, LK, 512>(a, row0, n, h, 0, sv);
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      const int at = threadIdx.x + 512 * u, t = at / (MX / 8), i = 8 * (at % (MX / 8));
+      *reinterpret_cast<f32x4*>(sk + ls_kat<MX, KT>(t, i)) = t < n && i < D ? kp[u] : zero;
+    }
+  } else {
+    ls_stage_v<T, VEC, MX, LK, 512>(a, row0, n, h, 0, sv);
+#pragma unroll
+    for (int u = threadIdx.x; u < LK * MX / 8; u += 512) {
+      const int t = u / (MX / 8), i = 8 * (u % (MX / 8));
+      float v[8];
+      ls_head8<T, VEC, ROT>(a, c, row0 + min(t, n - 1), a.k_off + (long)h * a.D, i, v);
+      if constexpr (BF) {
+        bf16x8 b;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) b[e] = t < n ? (bf16_t)v[e] : (bf16_t)0.f;
+        *reinterpret_cast<bf16x8*>(sk + ls_kat<MX, KT>(t, i)) = b;
+      } else {
+#pragma unroll
+        for (int x = 0; x < 8; x += 4)
+          *reinterpret_cast<f32x4*>(sk + ls_kat<MX, KT>(t, i + x)) =
+              t < n ? f32x4{v[x], v[x + 1], v[x + 2], v[x + 3]} : f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+    }
+  }
+  __syncthreads();
+  if (t0 >= n) return;
+  const float qk = a.qscale * a.kscale;
+  float back = 0.f;                                    // l from the end of block b to the query's
   for (int b = w; b >= 0; --b) {
     // weights are formed transposed, keys x queries: their registers are the A operand of P v
     f32x4 p = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int x = 0; x < MX / 32; ++x) {
       if constexpr (BF) {
-        bf16x8 qb;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) qb[e] = qf[x][e];
         const bf16x8 kb = *reinterpret_cast<const bf16x8*>(sk + ls_kat<MX, KT>(16 * b + l16, 32 * x + 8 * g4));
-        p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kb, qb, p, 0, 0, 0);
+        p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kb, qf[x], p, 0, 0, 0);
       } else {
 #pragma unroll
         for (int e = 0; e < 8; e += 4)
@@ -771,34 +838,6 @@ ls_chunk_out_kernel(ScanArgs a, KChunkArgs c) {
           o[4 * x + j] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[e], v[j], o[4 * x + j], 0, 0, 0);
       }
     if (b < w) back += tot[b];
-  }
-  if (row0 != a.cu[s] || a.positions[a.cu[s]] != 0) {  // (a fresh sequence's first chunk: S = 0)
-    const float eq = a.qscale * __builtin_amdgcn_exp2f(pq + back);
-    const float* S = c.U + ((long)blockIdx.x * a.H + h) * c.DP * c.UW;
-    float nq = 0.f;
-#pragma unroll
-    for (int x = 0; x < MX / 32; ++x)
-#pragma unroll
-      for (int e = 0; e < 8; e += 4) {
-        const int i = 32 * x + 8 * g4 + e;
-        if (32 * x >= c.DP) break;
-        const f32x4 qa = f32x4{(float)qf[x][e], (float)qf[x][e + 1], (float)qf[x][e + 2],
-                               (float)qf[x][e + 3]} * eq;
-#pragma unroll
-        for (int y = 0; y < 4; ++y) {
-          const float* r = S + (long)(i < c.DP ? i + y : 0) * c.UW;
-          if (a.mode == 1) nq += qa[y] * r[c.VP];
-#pragma unroll
-          for (int z = 0; z < MX / 64; ++z) {
-            const int d = 64 * z + 4 * l16;
-            const f32x4 v = *reinterpret_cast<const f32x4*>(r + (d < c.VP ? d : 0));
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-              o[4 * z + j] = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[y], v[j], o[4 * z + j], 0, 0, 0);
-          }
-        }
-      }
-    rs += nq;
   }
   rs += __shfl_xor(rs, 16, 64);                        // n_t . q_t of query l16
   rs += __shfl_xor(rs, 32, 64);

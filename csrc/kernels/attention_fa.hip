@@ -1,8 +1,11 @@
 // K2 (long prompts): paged flash-attention prefill on v_mfma_f32_32x32x16_bf16, D = 128.
 //
-// Work split: a workgroup of 8 waves owns one 64-query block of one sequence for FOUR query
-// heads of one KV group (wave w: head 4*hg + (w & 3), queries q0 + 32*(w >> 2) + [0, 32)), so
-// every 64-key K/V tile staged in LDS feeds 256 query rows (the GQA group shares it).
+// Work split: a workgroup of 8 waves owns HPW query heads of one KV group -- 4, 2 or 1, as many as
+// divide the group -- and 256 / HPW queries of one sequence (wave w: head HPW*hg + w % HPW, queries
+// q0 + 32*(w / HPW) + [0, 32)), so every 64-key K/V tile staged in LDS feeds 256 query rows.
+// One 4096-token causal prompt, 40 heads on 8 (one head per workgroup): 205 us on an MI355X, 16 on 8
+// (two): 129 us, against 749 and 381 us in the 16-query register form (attention.hip), which reads
+// every K/V unit once per head and 48 or 96 queries; equal below about 100 tokens.
 //
 // Per wave and tile (swapped products, guide §3 "An accumulator tile as the next MFMA's
 // operand"):
@@ -44,7 +47,7 @@ typedef __attribute__((ext_vector_type(16))) float f32x16_t;
 
 constexpr int FD = 128;        // head dim
 constexpr int FKB = 64;        // keys per tile
-constexpr int FQB = 64;        // queries per workgroup and head
+constexpr int FROWS = 256;     // (query, head) rows per workgroup
 constexpr int FTHREADS = 512;  // 8 waves
 constexpr int KS = FD + 8;           // K row stride (elements)
 constexpr int VS = FKB + 8;          // V^T row stride (elements)
@@ -63,6 +66,7 @@ EIA_DEV float pair_sum(float v) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+template <int HPW>
 __global__ void __launch_bounds__(FTHREADS, 1)
 paged_prefill_fa_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __restrict__ out,
                         long out_stride, const bf16_t* __restrict__ kc,
@@ -78,10 +82,11 @@ paged_prefill_fa_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __r
   // the work list is latest-block-first, so the dispatch order is longest-first over the
   // whole grid (causal blocks grow with their position), not per head
   const int s = work[2 * blockIdx.y], q0 = work[2 * blockIdx.y + 1];
-  const int G = Hq / Hkv, NHG = G / 4;
+  constexpr int FQB = FROWS / HPW;
+  const int G = Hq / Hkv, NHG = G / HPW;
   const int kvh = blockIdx.x / NHG, hg = blockIdx.x % NHG;
-  const int hq = kvh * G + hg * 4 + (w & 3);
-  const int qsub = w >> 2;
+  const int hq = kvh * G + hg * HPW + w % HPW;
+  const int qsub = w / HPW;
   const int qbeg = cu_q[s], qlen = cu_q[s + 1] - qbeg;
   if (q0 >= qlen) return;                                  // workgroup-uniform
   const int L = seq_lens[s], ctx = L - qlen;
@@ -169,6 +174,8 @@ paged_prefill_fa_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __r
     }
     // element i of half sh is key kb + 32 sh + 16 (i >> 3) + 8 h + (i & 7)
     const bool whole = !window && kb + FKB <= L && (!causal || kb + FKB - 1 <= ctx + wq0);
+    // the branch must not carry a reader of the last product past the wait states it needs
+    asm volatile("s_nop 5" : "+v"(sacc[1]));
     if (!whole) {
       // key kp is visible iff q_lo <= kp <= kmax: one unsigned compare per score, no branches
       const int kmax = causal ? min(L - 1, qa) : L - 1;
@@ -283,8 +290,8 @@ paged_prefill_fa_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __r
 
 }  // namespace
 
-// work = [seq, first query] pairs with 64-query blocks (attention.prefill_query_block);
-// grid (Hkv * G/4, n_work).  Requires D = 128, G % 4 == 0, block size % 64 == 0.
+// work = [seq, first query] pairs with blocks of 256 / HPW queries (attention.prefill_query_block);
+// grid (Hkv * G / HPW, n_work).  Requires D = 128, block size % 64 == 0.
 EIA_API int eia_paged_prefill_fa(const void* q, long q_stride, void* out, long out_stride,
                                  const void* k_cache, const void* v_cache,
                                  const int* block_tables, int bt_stride, const int* seq_lens,
@@ -292,19 +299,20 @@ EIA_API int eia_paged_prefill_fa(const void* q, long q_stride, void* out, long o
                                  int Hkv, int D, int bs, int causal, int sliding_window,
                                  int chunk_size, hipStream_t st) {
   if (Hkv <= 0 || Hq % Hkv != 0) return EIA_BAD_SHAPE;
-  if (D != FD || (Hq / Hkv) % 4 != 0 || bs % FKB != 0 || out_stride % 8 != 0)
-    return EIA_UNSUPPORTED;                                 // (16-B output stores)
+  if (D != FD || bs % FKB != 0 || out_stride % 8 != 0) return EIA_UNSUPPORTED;   // (16-B output stores)
   if (n_work == 0) return EIA_OK;
-  static bool attr = false;   // > 64 KiB of dynamic LDS must be opted into
-  if (!attr) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(paged_prefill_fa_kernel),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, FA_LDS_BYTES);
-    attr = true;
-  }
-  dim3 grid(Hkv * ((Hq / Hkv) / 4), n_work);
-  hipLaunchKernelGGL(paged_prefill_fa_kernel, grid, dim3(FTHREADS), FA_LDS_BYTES, st, (const bf16_t*)q,
-                     q_stride, (bf16_t*)out, out_stride, (const bf16_t*)k_cache,
-                     (const bf16_t*)v_cache, block_tables, bt_stride, seq_lens, cu_q, work,
-                     scale * 1.4426950408889634f, Hq, Hkv, bs, causal, sliding_window, chunk_size);
+  const int G = Hq / Hkv, hpw = G % 4 == 0 ? 4 : G % 2 == 0 ? 2 : 1;
+#define FA_GO(HPW)                                                                                  \
+  do {                                                                                              \
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(paged_prefill_fa_kernel<HPW>),          \
+                              hipFuncAttributeMaxDynamicSharedMemorySize, FA_LDS_BYTES);            \
+    hipLaunchKernelGGL(paged_prefill_fa_kernel<HPW>, dim3(Hq / HPW, n_work), dim3(FTHREADS),        \
+                       FA_LDS_BYTES, st, (const bf16_t*)q, q_stride, (bf16_t*)out, out_stride,      \
+                       (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, bt_stride,     \
+                       seq_lens, cu_q, work, scale * 1.4426950408889634f, Hq, Hkv, bs, causal,      \
+                       sliding_window, chunk_size);                                                 \
+  } while (0)
+  if (hpw == 4) FA_GO(4); else if (hpw == 2) FA_GO(2); else FA_GO(1);
+#undef FA_GO
   EIA_LAUNCH_CHECK();
 }

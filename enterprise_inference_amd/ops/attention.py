@@ -50,17 +50,17 @@ PREFILL_LDS_QT = {64: 1, 128: 2}
 
 
 # Flash-attention form (csrc/kernels/attention_fa.hip): 8 waves, 64 queries x 4 heads of one KV
-# group per workgroup, 64-key K/V tiles in swizzled LDS, v_mfma_f32_32x32x16_bf16 with P^T fed
-# from the S^T accumulators.  D = 128, G % 4 == 0, block size % 64 == 0.
+# group per workgroup (128 x 2, 256 x 1 where 4 do not divide the group), 64-key K/V tiles in
+# LDS, v_mfma_f32_32x32x16_bf16 with P^T fed from the S^T accumulators.  D = 128, block size % 64
+# == 0.
 PREFILL_FA = 32
 _FA_ENV = os.environ.get("EIA_PREFILL_FA", "1") != "0"
-PREFILL_FA_QB = 64
+PREFILL_FA_QB = 64           # with 4 heads per workgroup
 
 
 def fa_supported(num_heads: int, num_kv_heads: int, head_dim: int,
                  block_size: Optional[int]) -> bool:
-    return (_FA_ENV and head_dim == 128 and (num_heads // num_kv_heads) % 4 == 0
-            and block_size is not None and block_size % 64 == 0)
+    return (_FA_ENV and head_dim == 128 and block_size is not None and block_size % 64 == 0)
 
 
 def prefill_variant(num_heads: int, num_kv_heads: int, head_dim: int,
@@ -79,10 +79,10 @@ def prefill_variant(num_heads: int, num_kv_heads: int, head_dim: int,
 def prefill_query_block(num_heads: int, num_kv_heads: int, head_dim: int = 128,
                         qt: Optional[int] = None, block_size: Optional[int] = None) -> int:
     """Queries covered by one prefill workgroup (4 waves x QT x 16 columns / heads-per-WG;
-    64 for the flash form)."""
+    64 x 4 / heads-per-WG for the flash form)."""
     code = qt or prefill_variant(num_heads, num_kv_heads, head_dim, block_size)
     if code & PREFILL_FA:
-        return PREFILL_FA_QB
+        return PREFILL_FA_QB * (4 // heads_per_workgroup(num_heads, num_kv_heads))
     return 16 * (code & 15) * (4 // heads_per_workgroup(num_heads, num_kv_heads))
 
 
@@ -287,8 +287,9 @@ def paged_prefill(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
         if rc != EIA_UNSUPPORTED:
             check(rc, "paged_prefill_fa")
             return o
-        code = PREFILL_LDS | (PREFILL_FA_QB // 16)   # same query blocks (HPW 4 x QT x 16)
-        require(hpw == 4, "paged_prefill: flash work list needs 4 heads per workgroup")
+        code = PREFILL_FA_QB // 16                   # same query blocks (QT x 16 x 4 / HPW)
+        if hpw == 4:
+            code |= PREFILL_LDS
     check(lib().eia_paged_prefill(
         ptr(q), q.stride(0), ptr(o), o.stride(0), ptr(k_cache), ptr(v_cache), ptr(block_tables),
         block_tables.stride(0), ptr(seq_lens), ptr(cu_q), ptr(work), n_work, float(scale), Hq, Hkv,

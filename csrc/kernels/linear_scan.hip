@@ -1247,3 +1247,491 @@ EIA_API int eia_linear_scan_channels(const void* x, long ld, int q_off, int k_of
 #undef LS_CHUNKED
   EIA_LAUNCH_CHECK();
 }
+
+// ---------------------------------------------------------------------------------------------
+// Mode 2 for dk <= 64 on matrix cores: the chunks of GC tokens, the block edges and the cut at 2^-40
+// of wkv.hip's chunk-parallel form, with the token itself among its keys,
+//
+//   U   = sum_s 2^(sum_(s<x) l_x) k_s v_s^T                            (1) per chunk, in parallel
+//   S' = 2^(sum_x l_x) S + U                                           (2) a sequence's chunks in order
+//   o_t = (q_t 2^(sum_(x<=t) l_x)) S + sum_(s<=t) P_ts v_s
+//   P_ts = sum_channels q_t k_s 2^(sum_(s<x<=t) l_x)                   (3) per chunk, in parallel
+//
+// where l_x = log2 a_x per key channel, formed by a pass of its own for all rows and heads (its
+// low-rank product and logarithms are the same for (1) and (3)).  Exponents are sums of the l_x that
+// they cover; pairs of different 8-token blocks meet through the edges of the blocks between them, and
+// only pairs inside a block take the difference of a running sum over that block.  Products are fp32
+// matrix-core products.  Bound by instruction issue (exponentials, operand rows through LDS), as there.
+// Four prompts of 490 to 977 tokens, 16 heads of 64 x 128, bf16: 21 + 22 + 11 + 60 us on an MI355X (l, (1),
+// (2), (3)); in the 32-token chunks of vector FMAs above 38 + 71 + 21 + 235 us, which remain for keys
+// wider than 64.
+constexpr int GC = 64;                      // tokens per chunk
+constexpr int GD = 64;                      // widest key head
+
+EIA_DEV bool gl_chunk(const ScanArgs& a, int nseq, int x, int& s, int& row0, int& n) {
+  int lo = 0, hi = nseq - 1;                // largest s with cu[s] / GC + s <= x
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (a.cu[mid] / GC + mid <= x) lo = mid; else hi = mid - 1;
+  }
+  s = lo;
+  if (x < a.cu[s] / GC + s) return false;   // (rows before the first sequence)
+  row0 = a.cu[s] + (x - a.cu[s] / GC - s) * GC;
+  n = min(GC, a.cu[s + 1] - row0);
+  return n > 0 && a.slots[s] >= 0;
+}
+
+// Place of (token, channel) in an fp32 tile [GC][W]: units of four channels turned by the token.
+template <int W> EIA_DEV int gl_at(int t, int i) { return t * W + (i ^ ((t & 15) << 2)); }
+template <int W> EIA_DEV f32x4 gl_get(const float* tile, int t, int i) {
+  return *reinterpret_cast<const f32x4*>(tile + gl_at<W>(t, i));
+}
+
+// l of all rows: thread = channel of one head and 16 rows.
+template <typename T>
+__global__ void __launch_bounds__(256)
+gl_logs_kernel(ScanArgs a, KChunkArgs c) {
+  constexpr int RB = 32;
+  __shared__ float lo[64][RB + 1];
+  const int h = blockIdx.y, j = threadIdx.x & 63, g = threadIdx.x >> 6, r0 = blockIdx.x * 64;
+  const long HD = (long)a.H * a.D, hc = (long)h * a.D + min(j, a.D - 1);
+  const T* X = static_cast<const T*>(a.x) + a.lo_off;
+  float z[16];
+  const float b = a.a2b ? a.a2b[hc] : 0.f;
+#pragma unroll
+  for (int t = 0; t < 16; ++t) z[t] = b;
+  for (int k0 = 0; k0 < a.R; k0 += RB) {
+    const int kn = min(RB, a.R - k0);
+    __syncthreads();
+    for (int u = threadIdx.x; u < 64 * kn; u += 256) {
+      const int t = u / kn, k = u % kn;
+      lo[t][k] = ld_f32<T>(X + (long)min(r0 + t, c.rows - 1) * a.ld, k0 + k);
+    }
+    __syncthreads();
+#pragma unroll 8
+    for (int k = 0; k < kn; ++k) {
+      const float w = a.a2t[(k0 + k) * HD + hc];
+#pragma unroll
+      for (int t = 0; t < 16; ++t) z[t] += lo[16 * g + t][k] * w;
+    }
+  }
+  if (j >= a.D) return;
+#pragma unroll
+  for (int t = 0; t < 16; ++t) {
+    const int r = r0 + 16 * g + t;
+    if (r < c.rows) c.la[r * HD + hc] = ls_logsigmoid(z[t]) * a.inv_tau * LS_LOG2E;
+  }
+}
+
+// l of channel i, tokens t0 .. t0 + 15 of the chunk (0 past its end and past D).
+EIA_DEV void gl_decays(const ScanArgs& a, const KChunkArgs& c, int h, int row0, int n, int t0, int i,
+                       float (&l)[16]) {
+  const float* p = c.la + (long)h * a.D + min(i, a.D - 1);
+#pragma unroll
+  for (int t = 0; t < 16; ++t) l[t] = p[(long)(row0 + min(t0 + t, n - 1)) * a.H * a.D];
+#pragma unroll
+  for (int t = 0; t < 16; ++t) l[t] = (i < a.D && t0 + t < n) ? l[t] : 0.f;
+}
+
+// A chunk's [GC][GD] tile of q or k, rotated and scaled, on its way to LDS.
+template <typename T, bool VEC, bool ROT>
+struct GlTile {
+  float v[2][8];
+  EIA_DEV void load(const ScanArgs& a, const KChunkArgs& c, int row0, int n, long off) {
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      const int u = threadIdx.x + 256 * x;
+      ls_head8<T, VEC, ROT>(a, c, row0 + min(u >> 3, n - 1), off, 8 * (u & 7), v[x]);
+    }
+  }
+  EIA_DEV void store(float* tile, int n, float scale) const {
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      const int u = threadIdx.x + 256 * x, t = u >> 3, i = 8 * (u & 7);
+#pragma unroll
+      for (int e = 0; e < 8; e += 4)
+        *reinterpret_cast<f32x4*>(tile + gl_at<GD>(t, i + e)) =
+            t < n ? f32x4{v[x][e], v[x][e + 1], v[x][e + 2], v[x][e + 3]} * scale
+                  : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+  }
+};
+
+// ... and of v, GC x 64 NV, zero past the chunk and past Dv.
+template <typename T, bool VEC, int NV>
+struct GlValues {
+  static constexpr int E = VEC ? 16 / (int)sizeof(T) : 1, W = 64 * NV, N = GC * W / (256 * E);
+  T v[N][E];
+  EIA_DEV void load(const ScanArgs& a, int row0, int n, int h) {
+    const T* X = static_cast<const T*>(a.x) + a.v_off + (long)h * a.Dv;
+#pragma unroll
+    for (int x = 0; x < N; ++x) {
+      const int u = threadIdx.x + 256 * x, t = u / (W / E), i = E * (u % (W / E));
+      const T* p = X + (long)(row0 + min(t, n - 1)) * a.ld + (i < a.Dv ? i : 0);
+      if constexpr (VEC) *reinterpret_cast<f32x4*>(v[x]) = *reinterpret_cast<const f32x4*>(p);
+      else v[x][0] = *p;
+    }
+  }
+  EIA_DEV void store(float* tile, int n, int Dv) const {
+#pragma unroll
+    for (int x = 0; x < N; ++x) {
+      const int u = threadIdx.x + 256 * x, t = u / (W / E), i = E * (u % (W / E));
+      const bool ok = t < n && i < Dv;
+      if constexpr (VEC) {
+#pragma unroll
+        for (int e = 0; e < E; e += 4)
+          *reinterpret_cast<f32x4*>(tile + gl_at<W>(t, i + e)) =
+              ok ? f32x4{(float)v[x][e], (float)v[x][e + 1], (float)v[x][e + 2], (float)v[x][e + 3]}
+                 : f32x4{0.f, 0.f, 0.f, 0.f};
+      } else {
+        tile[gl_at<W>(t, i)] = ok ? (float)v[x][0] : 0.f;
+      }
+    }
+  }
+};
+
+// (1) Wave w forms rows 16 w .. of U [GD][64 NV].  A lane holds value columns 64 z + 4 (lane % 16) + j
+// in its tile 4 z + j, here and in (3).
+template <typename T, bool VEC, bool ROT, int NV>
+__global__ void __launch_bounds__(256)
+gl_state_kernel(ScanArgs a, KChunkArgs c) {
+  constexpr int W = 64 * NV;
+  __shared__ __align__(16) float sk[GC * GD], sv[GC * W];
+  __shared__ float stot[4][GD];
+  int s, row0, n;
+  if (!gl_chunk(a, c.nseq, blockIdx.x, s, row0, n)) return;
+  const int h = blockIdx.y, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int l16 = lane & 15, g4 = lane >> 4;
+  GlTile<T, VEC, ROT> tk;
+  GlValues<T, VEC, NV> tv;
+  tk.load(a, c, row0, n, a.k_off + (long)h * a.D);
+  tv.load(a, row0, n, h);
+  float l[16];
+  gl_decays(a, c, h, row0, n, 16 * w, lane, l);
+  float tot = 0.f;
+#pragma unroll
+  for (int t = 0; t < 16; ++t) tot += l[t];
+  stot[w][lane] = tot;
+  tk.store(sk, n, a.kscale);
+  tv.store(sv, n, a.Dv);
+  __syncthreads();
+  float after = 0.f;                                   // sum of l from the next token on
+  for (int b = 3; b > w; --b) after += stot[b][lane];
+#pragma unroll
+  for (int t = 15; t >= 0; --t) {
+    sk[gl_at<GD>(16 * w + t, lane)] *= __builtin_amdgcn_exp2f(after);
+    after += l[t];
+  }
+  const long at = (long)blockIdx.x * a.H + h;
+  if (w == 0) c.G[at * GD + lane] = after;
+  __syncthreads();
+  f32x4 acc[4 * NV];
+#pragma unroll
+  for (int j = 0; j < 4 * NV; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    if (16 * b >= n) break;
+    f32x4 ka, vb[4 * NV];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int t = 16 * b + 4 * g4 + e;
+      ka[e] = sk[gl_at<GD>(t, 16 * w + l16)];
+#pragma unroll
+      for (int z = 0; z < NV; ++z) {
+        const f32x4 x = gl_get<W>(sv, t, 64 * z + 4 * l16);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) vb[4 * z + j][e] = x[j];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4 * NV; ++j) acc[j] = mfma_f32_k16(ka, vb[j], acc[j]);
+  }
+  float* U = c.U + at * GD * W + (long)(16 * w + 4 * g4) * W + 4 * l16;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int z = 0; z < NV; ++z)
+      *reinterpret_cast<f32x4*>(U + i * W + 64 * z) =
+          f32x4{acc[4 * z][i], acc[4 * z + 1][i], acc[4 * z + 2][i], acc[4 * z + 3][i]};
+}
+
+// (2) Four columns of a state row per thread: U of a chunk turns into the state before it; the slot
+// receives the state after the last one.  A group's contributions are requested while the previous
+// group is summed.
+template <int NV>
+__global__ void __launch_bounds__(256)
+gl_scan_kernel(ScanArgs a, KChunkArgs c) {
+  constexpr int W = 64 * NV;
+  const int s = blockIdx.x, h = blockIdx.y;
+  const int slot = a.slots[s], lo = a.cu[s], hi = a.cu[s + 1];
+  if (slot < 0 || hi <= lo) return;
+  const int e = 4 * (blockIdx.z * 256 + threadIdx.x), i = e / W, j = e % W, D = a.D, Dv = a.Dv;
+  const long x0 = lo / GC + s;
+  const int nc = (hi - lo + GC - 1) / GC;
+  float* Sg = a.S + ((long)slot * a.H + h) * D * Dv + (long)i * Dv + j;
+  f32x4 S = {0.f, 0.f, 0.f, 0.f};
+  if (a.positions[lo] != 0 && i < D) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (j + k < Dv) S[k] = Sg[k];
+  }
+  float* U = c.U + (x0 * a.H + h) * GD * W + e;
+  const float* L = c.G + (x0 * a.H + h) * GD + i;
+  const long us = (long)a.H * GD * W, ls = (long)a.H * GD;
+  f32x4 u[LS_AHEAD];
+  float d[LS_AHEAD];
+  auto fetch = [&](int b, f32x4 (&u)[LS_AHEAD], float (&d)[LS_AHEAD]) {
+#pragma unroll
+    for (int k = 0; k < LS_AHEAD; ++k) {
+      const int x = min(b + k, nc - 1);
+      u[k] = *reinterpret_cast<const f32x4*>(U + x * us);
+      d[k] = L[x * ls];
+    }
+  };
+  fetch(0, u, d);
+  for (int b = 0; b < nc; b += LS_AHEAD) {
+    f32x4 un[LS_AHEAD];
+    float dn[LS_AHEAD];
+    fetch(b + LS_AHEAD, un, dn);
+#pragma unroll
+    for (int k = 0; k < LS_AHEAD; ++k) {
+      if (b + k < nc) {
+        *reinterpret_cast<f32x4*>(U + (b + k) * us) = S;
+        S = S * __builtin_amdgcn_exp2f(d[k]) + u[k];
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < LS_AHEAD; ++k) {
+      u[k] = un[k];
+      d[k] = dn[k];
+    }
+  }
+  if (i < D) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (j + k < Dv) Sg[k] = S[k];
+  }
+}
+
+// (3) Wave w forms the outputs of tokens 16 w .. (which wave takes which rotates with the chunk).  The
+// running sums of l share their LDS with the values, which move in after them.
+template <typename T, bool VEC, bool ROT, int NV>
+__global__ void __launch_bounds__(256, 2)
+gl_out_kernel(ScanArgs a, KChunkArgs c) {
+  constexpr int W = 64 * NV;
+  __shared__ __align__(16) float sq[GC * GD], sk[GC * GD], sAv[GC * W];
+  __shared__ __align__(16) float se[8][GD];            // decays over whole 8-token blocks
+  int s, row0, n;
+  if (!gl_chunk(a, c.nseq, blockIdx.x, s, row0, n)) return;
+  const int h = blockIdx.y, lane = threadIdx.x & 63, w = ((threadIdx.x >> 6) + blockIdx.x) & 3;
+  const int Dv = a.Dv, l16 = lane & 15, g4 = lane >> 4, t0 = 16 * w;
+  GlTile<T, VEC, ROT> tq, tk;
+  GlValues<T, VEC, NV> tv;
+  tq.load(a, c, row0, n, a.q_off + (long)h * a.D);
+  tk.load(a, c, row0, n, a.k_off + (long)h * a.D);
+  float l[16];
+  gl_decays(a, c, h, row0, n, t0, lane, l);
+  tv.load(a, row0, n, h);
+  tq.store(sq, n, a.qscale);
+  tk.store(sk, n, a.kscale);
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    float A = 0.f, tot = 0.f;
+#pragma unroll
+    for (int t = 8 * b; t < 8 * b + 8; ++t) {
+      A += fmaxf(l[t], -40.f);
+      tot += l[t];
+      sAv[gl_at<GD>(t0 + t, lane)] = A;
+    }
+    se[2 * w + b][lane] = __builtin_amdgcn_exp2f(tot);
+  }
+  __syncthreads();
+  // weights inside the wave's two 8-token blocks: lane = pair s < t, then to the lane that holds
+  // them as an operand (query l16, keys 4 g4 + i)
+  f32x4 p = {0.f, 0.f, 0.f, 0.f};
+  if (t0 < n) {
+    float v = 0.f;
+    if (lane < 56) {
+      const int x = lane % 28;
+      int t = 1;
+      while (t * (t + 1) / 2 <= x) ++t;
+      const int q = t0 + 8 * (lane / 28), ks = x - t * (t - 1) / 2;
+#pragma unroll 4
+      for (int i = 0; i < GD; i += 4) {
+        const f32x4 y = gl_get<GD>(sq, q + t, i) * gl_get<GD>(sk, q + ks, i);
+        const f32x4 d = gl_get<GD>(sAv, q + t, i) - gl_get<GD>(sAv, q + ks, i);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v += y[e] * __builtin_amdgcn_exp2f(d[e]);
+      }
+    }
+    float b = 0.f;                                     // q . k of token t0 + l16
+#pragma unroll
+    for (int i = 0; i < 16; i += 4) {
+      const int d = 16 * g4 + i;
+      const f32x4 x = gl_get<GD>(sq, t0 + l16, d) * gl_get<GD>(sk, t0 + l16, d);
+      b += x[0] + x[1] + x[2] + x[3];
+    }
+    b += __shfl_xor(b, 16, 64);
+    b += __shfl_xor(b, 32, 64);
+    const int t8 = l16 & 7;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int ks = 4 * g4 + i;
+      const float x = __shfl(v, 28 * (l16 >> 3) + (t8 * (t8 - 1) >> 1) + (ks & 7), 64);
+      p[i] = ks == l16 ? b : (ks < l16 && ks >> 3 == l16 >> 3) ? x : 0.f;
+    }
+  }
+  __syncthreads();
+  // q_t <- q_t 2^(block start .. t], k_s <- k_s 2^(s .. block end), 8-token blocks; v moves in
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    float pre = 0.f, suf = 0.f;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      pre += l[8 * b + t];
+      sq[gl_at<GD>(t0 + 8 * b + t, lane)] *= __builtin_amdgcn_exp2f(pre);
+      sk[gl_at<GD>(t0 + 8 * b + 7 - t, lane)] *= __builtin_amdgcn_exp2f(suf);
+      suf += l[8 * b + 7 - t];
+    }
+  }
+  tv.store(sAv, n, Dv);
+  __syncthreads();
+  if (t0 >= n) return;
+  f32x4 rt[4], o[4 * NV], pq = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    const int i = 16 * b + 4 * g4;
+    rt[b] = gl_get<GD>(sq, t0 + l16, i);
+    pq = mfma_f32_k16(gl_get<GD>(sk, t0 + l16, i), rt[b], pq);
+    if (l16 >= 8) rt[b] *= *reinterpret_cast<const f32x4*>(&se[2 * w][i]);
+  }
+#pragma unroll
+  for (int j = 0; j < 4 * NV; ++j) o[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // (weights are formed transposed, keys x queries: their registers are the A operand of P v)
+  if (l16 >= 8 && g4 < 2) p += pq;                     // second 8 queries, first 8 keys
+  for (int b = w;;) {
+    f32x4 vb[4 * NV];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int z = 0; z < NV; ++z) {
+        const f32x4 x = gl_get<W>(sAv, 16 * b + 4 * g4 + e, 64 * z + 4 * l16);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) vb[4 * z + j][e] = x[j];
+      }
+#pragma unroll
+    for (int j = 0; j < 4 * NV; ++j) o[j] = mfma_f32_k16(p, vb[j], o[j]);
+    if (--b < 0) break;
+    p = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {                      // keys of block b; rt: from its end on
+      const int i = 16 * x + 4 * g4;
+      const f32x4 e1 = *reinterpret_cast<const f32x4*>(&se[2 * b + 1][i]);
+      f32x4 kk = gl_get<GD>(sk, 16 * b + l16, i);
+      if (l16 < 8) kk *= e1;
+      p = mfma_f32_k16(kk, rt[x], p);
+      rt[x] *= e1 * *reinterpret_cast<const f32x4*>(&se[2 * b][i]);
+    }
+  }
+  if (row0 != a.cu[s] || a.positions[a.cu[s]] != 0) {  // (a fresh sequence's first chunk: S = 0)
+    const float* S = c.U + ((long)blockIdx.x * a.H + h) * GD * W + (long)4 * g4 * W + 4 * l16;
+#pragma unroll
+    for (int x = 0; x < 4; ++x)
+#pragma unroll
+      for (int z = 0; z < NV; ++z) {
+        f32x4 sb[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const f32x4 q = *reinterpret_cast<const f32x4*>(S + (16 * x + e) * W + 64 * z);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) sb[j][e] = q[j];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[4 * z + j] = mfma_f32_k16(rt[x], sb[j], o[4 * z + j]);
+      }
+  }
+  const T* X = static_cast<const T*>(a.x);
+  const T* NW = static_cast<const T*>(a.norm_w);
+  T* Y = static_cast<T*>(a.y);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {                        // head RMS norm (zeros past Dv), weight, gate
+    const int t = t0 + 4 * g4 + i;
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4 * NV; ++j) ss += o[j][i] * o[j][i];
+    ss += __shfl_xor(ss, 1, 64);
+    ss += __shfl_xor(ss, 2, 64);
+    ss += __shfl_xor(ss, 4, 64);
+    ss += __shfl_xor(ss, 8, 64);
+    if (t >= n) continue;
+    const float inv = a.out_scale / sqrtf(ss / (float)Dv + a.eps);
+    const long row = row0 + t;
+#pragma unroll
+    for (int z = 0; z < NV; ++z)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int d = 64 * z + 4 * l16 + j;
+        if (d < Dv) {
+          const float g = ld_f32<T>(X + row * a.ld, a.g_off + (long)h * Dv + d);
+          const float sig = sizeof(T) == 2 ? __builtin_amdgcn_rcpf(1.0f + __expf(-g))
+                                           : 1.0f / (1.0f + expf(-g));
+          const float nw = NW ? ld_f32<T>(NW, (long)h * a.norm_h + d) : 1.f;
+          st_f32<T>(Y + row * a.ldy, (long)h * Dv + d,
+                    o[4 * z + j][i] * inv * nw * (a.gate_act == 0 ? g * sig : sig));
+        }
+      }
+  }
+}
+
+template <typename T, bool VEC, bool ROT, int NV>
+static void gl_launch(const ScanArgs& a, const KChunkArgs& c, hipStream_t st) {
+  const dim3 gc(c.rows / GC + c.nseq, a.H), gs(c.nseq, a.H, GD * 64 * NV / 1024);
+  hipLaunchKernelGGL((gl_logs_kernel<T>), dim3((c.rows + 63) / 64, a.H), dim3(256), 0, st, a, c);
+  if (ROT) {
+    const long u = (long)c.rows * (a.rot_dims >> 1);
+    hipLaunchKernelGGL(ls_angles_kernel, dim3((unsigned)((u + 255) / 256)), dim3(256), 0, st, a, c);
+  }
+  hipLaunchKernelGGL((gl_state_kernel<T, VEC, ROT, NV>), gc, dim3(256), 0, st, a, c);
+  hipLaunchKernelGGL((gl_scan_kernel<NV>), gs, dim3(256), 0, st, a, c);
+  hipLaunchKernelGGL((gl_out_kernel<T, VEC, ROT, NV>), gc, dim3(256), 0, st, a, c);
+}
+
+template <typename T>
+static void gl_forms(const ScanArgs& a, const KChunkArgs& c, hipStream_t st) {
+  constexpr int A = 16 / (int)sizeof(T);               // elements in 16 bytes
+  const int rot8 = a.rot_dims ? (a.rot_half ? a.rot_dims / 2 : a.rot_dims) : 0;
+  const bool vec = reinterpret_cast<uintptr_t>(a.x) % 16 == 0 &&
+                   (a.ld | a.q_off | a.k_off | a.v_off) % A == 0 && a.D % 8 == 0 && a.Dv % 8 == 0 &&
+                   rot8 % 8 == 0;
+  const bool wide = a.Dv > 64, rot = a.rot_dims > 0;
+#define GL_GO(V, R) \
+  do { if (wide) gl_launch<T, V, R, 2>(a, c, st); else gl_launch<T, V, R, 1>(a, c, st); } while (0)
+  if (vec) { if (rot) GL_GO(true, true); else GL_GO(true, false); }
+  else { if (rot) GL_GO(false, true); else GL_GO(false, false); }
+#undef GL_GO
+}
+
+// As eia_linear_scan_channels for D <= 64, Dv <= 128, chunks found on the device (rows: at least
+// cu[nseq]): fp32 workspaces U [rows / 64 + nseq, H, 64, Dv rounded up to 64], L [rows / 64 + nseq, H,
+// 64], l [rows, H, D] and, with rotated heads, rot [rows, rot_dims].
+EIA_API int eia_linear_scan_channels64(const void* x, long ld, int q_off, int k_off, int v_off, int g_off,
+                                       const float* inv_freq, int rot_dims, int rot_half, float qscale,
+                                       float kscale, float out_scale, const void* norm_w, float* S,
+                                       const int* slots, const int* cu, const int* positions, void* y,
+                                       long ldy, float eps, int nseq, int rows, int H, int D, int Dv,
+                                       int gate_act, int norm_h, int lo_off, int R, const float* a2t,
+                                       const float* a2b, float inv_tau, float* U, float* L, float* l,
+                                       float* rot, int is_bf16, hipStream_t st) {
+  if (nseq < 0 || rows < 0 || H < 1 || D < 1 || Dv < 1 || !x || !y || !S || !slots || !cu ||
+      !positions || !U || !L || !l || R < 1 || !a2t || rot_dims < 0 || rot_dims > D ||
+      (rot_dims & 1) || (rot_dims && (!inv_freq || !rot)) || (gate_act != 0 && gate_act != 1))
+    return EIA_BAD_SHAPE;
+  if (D > GD || Dv > 128 || H > 65535) return EIA_UNSUPPORTED;
+  if (nseq == 0 || rows == 0) return EIA_OK;
+  ScanArgs a{x, ld, q_off, k_off, v_off, g_off, 0, 0, nullptr, inv_freq, rot_dims, rot_half,
+             qscale, kscale, 0.f, out_scale, norm_w, S, nullptr, nullptr, slots, cu, positions,
+             nullptr, y, ldy, eps, H, D, Dv, 2, gate_act, lo_off, R, a2t, a2b, inv_tau, norm_h};
+  KChunkArgs c{U, L, l, nullptr, nullptr, reinterpret_cast<float2*>(rot), nseq, rows, GD, Dv, Dv};
+  if (is_bf16) gl_forms<bf16_t>(a, c, st); else gl_forms<float>(a, c, st);
+  EIA_LAUNCH_CHECK();
+}

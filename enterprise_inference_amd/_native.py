@@ -84,6 +84,8 @@ _SIGNATURES = {
                                 IP, P, L, F, I, I, I, I, I, I, I, I, P, P, P, P, P, P, I, S],
     "eia_linear_scan_channels": [P, L, I, I, I, I, P, I, I, F, F, F, P, P, IP, IP, IP, P, L, F, I,
                                  I, I, I, I, I, IP, IP, I, P, P, I, I, P, P, F, P, I, S],
+    "eia_linear_scan_channels64": [P, L, I, I, I, I, P, I, I, F, F, F, P, P, IP, IP, IP, P, L, F, I,
+                                   I, I, I, I, I, I, I, I, P, P, F, P, P, P, P, I, S],
     "eia_hyper_step": [P, I, I, P, L, P, I, P, P, P, F, P, P, F, P, L, F, I, I, S],
     "eia_bigram_embed": [IP, P, F, P, I, L, L, IP, IP, IP, I, IP, P, I, I, I, I, I, S],
     "eia_relu2": [P, L, P, I, P, L, I, I, I, S],

@@ -97,6 +97,7 @@ class ScanState:
 
 CHUNK = 32                 # tokens per chunk of the chunk-parallel form ("channel", linear_scan.hip LC)
 HEAD_CHUNK = 128           # ... with one decay per head and token (linear_scan.hip LK)
+KEY_CHUNK64, KEY_DIM64 = 64, 64     # ... of the form with a decay per key channel, and its widest dk
 CHUNK_MAX_DIM = 128        # ... and its largest dk / dv
 CHUNK_MIN_ROWS = 48        # a sequence with at least this many rows in the step selects it
 # tests and measurements: take the chunk-parallel form whenever a plan is handed over
@@ -114,16 +115,24 @@ class ChunkPlan:
         self.chunks, self.seq_first, self.n, self.rows = chunks, seq_first, n, rows
         self.nseq, self.longest = nseq, longest
 
-    def pays(self, heads: int, dim: int, cus: int = 256, channel: bool = False) -> bool:
+    def pays(self, heads: int, dim: int, cus: int = 256, channel: bool = False,
+             key_dim: int = 0) -> bool:
         """Whether the chunk-parallel form beats the token-by-token one for a layer of ``heads``
         heads up to ``dim`` wide.  The latter walks the longest sequence at about 0.5 us a token
         (0.85 us above 64) while its workgroups, one per (sequence, head), do not share CUs.  The
         former costs 30 us for its launches and 0.7 ns (2 ns) per row and head, a short sequence
-        counting as 96 rows; with a decay per key channel 5 ns (7 ns).  MI355X, 16 heads of 128,
+        counting as 96 rows; with a decay per key channel 0.8 ns (1.7 ns, 64 rows), and 5 ns (7 ns)
+        for keys above KEY_DIM64, against 0.6 us (1.0 us) a token.  MI355X, 16 heads of 128,
         exponential gates, token by token / chunks: 1 x 48 rows 62 / 29 us, 1 x 4096 4793 / 145,
         16 x 64 84 / 63, 16 x 512 599 / 196; 32 heads of 64, fixed decays: 1 x 48 24 / 27, 16 x 64
-        34 / 47, 16 x 128 75 / 68, 1 x 4096 2035 / 104."""
+        34 / 47, 16 x 128 75 / 68, 1 x 4096 2035 / 104; 16 heads of 64 x 128, a decay per channel: 1 x
+        48 52 / 36, 16 x 64 70 / 60, 16 x 512 536 / 185, 1 x 4096 4307 / 122; 32 of 32 x 64: 1 x 48
+        33 / 31, 16 x 64 48 / 56, 16 x 128 93 / 87, 64 x 64 128 / 142."""
         wide = dim > 64
+        if channel and key_dim <= KEY_DIM64:
+            busy = self.nseq * heads / (cus if wide else 2.7 * cus)
+            serial = self.longest * (1.0 if wide else 0.6) * max(1.0, busy)
+            return 32 + max(self.rows, 64 * self.nseq) * heads * (0.0017 if wide else 0.0008) < serial
         if channel:
             serial = self.longest * (0.85 if wide else 0.5) * -(-self.nseq * heads // cus)
             return self.rows * heads * (0.0072 if wide else 0.0052) < serial
@@ -279,11 +288,24 @@ def linear_scan(fused: torch.Tensor, q_off: int, k_off: int, v_off: int, g_off: 
     chan = (lo_off, R, ptr(spec.a2t), ptr(spec.a2b), 1.0 / float(spec.tau),
             0 if spec.norm_shared else Dv)
     if (plan is not None and plan.n and max(D, Dv) <= CHUNK_MAX_DIM and cu is not None
-            and plan.rows == T and (FORCE_CHUNKED or plan.pays(H, max(D, Dv), channel=channel))
+            and plan.rows == T and
+            (FORCE_CHUNKED or plan.pays(H, max(D, Dv), channel=channel, key_dim=D))
             and not torch.cuda.is_current_stream_capturing()):
         dev = fused.device
         f32 = lambda *shape: torch.empty(*shape, dtype=torch.float32, device=dev)
         act = 0 if spec.gate_act == "silu" else 1
+        if channel and D <= KEY_DIM64:
+            n, W = T // KEY_CHUNK64 + nseq, -(-Dv // 64) * 64
+            U, L, l = f32(n, H, KEY_DIM64, W), f32(n, H, KEY_DIM64), f32(T, H, D)
+            rot = f32(T, spec.rot_dims) if spec.rot_dims else None
+            check(lib().eia_linear_scan_channels64(
+                ptr(fused), fused.stride(0), q_off, k_off, v_off, g_off, ptr(spec.inv_freq),
+                spec.rot_dims, 1 if spec.rot_half else 0, float(spec.qscale), float(spec.kscale),
+                float(spec.out_scale), ptr(norm_w), ptr(state.S), ptr(slots), ptr(cu),
+                ptr(positions), ptr(out), out.stride(0), float(spec.eps), nseq, T, H, D, Dv, act,
+                chan[-1], *chan[:-1], ptr(U), ptr(L), ptr(l), ptr(rot), 1 if bf else 0,
+                stream(fused)), "linear_scan_channels64")
+            return out
         if channel:
             wsS, wsG, cA = f32(plan.n, H, D, Dv), f32(plan.n, H, D), f32(T, H, D)
             check(lib().eia_linear_scan_channels(

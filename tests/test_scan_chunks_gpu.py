@@ -131,3 +131,39 @@ def test_delta_chunks(lens, H, G, D, Dv, dtype, monkeypatch):
     # at times one step more
     assert _rel(z[live], y[live]) < (1e-5 if dtype == torch.float32 else 4e-3)
     assert _rel(Z, S) < 4e-6
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,D,Dv,R,rot", [(2, 64, 128, 16, 0), (3, 32, 64, 33, 0), (2, 64, 64, 8, 64),
+                                          (2, 24, 40, 5, 8), (1, 20, 126, 16, 6)])
+@pytest.mark.parametrize("lens", [[1, 64, 63, 65, 130], [200], [7, 8, 9, 50, 129, 3]])
+def test_channel_chunks(lens, H, D, Dv, R, rot, dtype, monkeypatch):
+    from enterprise_inference_amd.ops import linear_scan as ls
+    monkeypatch.setattr(ls, "FORCE_CHUNKED", True)
+    g = torch.Generator().manual_seed(sum(lens) + D + R)
+    rnd = lambda *s: torch.randn(*s, generator=g)
+    n, T = len(lens), sum(lens)
+    cu, pos, slots = _step(lens, [0 if s % 2 == 0 else 5 for s in range(n)], n > 3)
+    at = [0, H * D, 2 * H * D, 2 * H * D + H * Dv, 2 * H * (D + Dv)]
+    x = rnd(T, at[-1] + R).to(dtype)
+    a2t, a2b = rnd(R, H * D), torch.linspace(-8.0, 8.0, H * D)     # from forgetting to keeping
+    inv = 10000.0 ** (-torch.arange(rot // 2) / max(1, rot // 2))
+    S0, nw = rnd(n, H, D, Dv), (1 + 0.1 * rnd(Dv)).to(dtype)
+
+    def run(dev):
+        spec = ls.ScanSpec(H, D, Dv, "channel", kscale=0.5, qscale=1.5, eps=1e-5, rot_dims=rot,
+                           rot_half=rot != 8, inv_freq=inv.to(dev), out_scale=0.7, norm_shared=True,
+                           a2t=a2t.to(dev), a2b=a2b.to(dev), tau=2.0)
+        st = ls.ScanState.allocate(n, spec, "cpu")
+        st = ls.ScanState(S0.clone().to(dev), None, None)
+        plan = ls.chunk_plan(lens, dev) if dev == "cuda" else None
+        y = ls.linear_scan(x.to(dev), at[0], at[1], at[2], at[3], spec, st, slots.to(dev),
+                           cu.to(dev), n, pos.to(dev), None, nw.to(dev), lo_off=at[4], plan=plan)
+        return y.cpu(), st.S.cpu()
+
+    (y, S), (z, Z) = run("cpu"), run("cuda")
+    live = torch.cat([torch.full((m,), int(s) >= 0) for m, s in zip(lens, slots)])
+    # fp32 sums over at most 64 products, logarithms of decays summed over at most 64 tokens; bf16
+    # adds one rounding and at times one step more
+    assert _rel(z[live], y[live]) < (2e-5 if dtype == torch.float32 else 4e-3)
+    assert _rel(Z, S) < 4e-6

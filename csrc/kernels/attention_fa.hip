@@ -3,9 +3,11 @@
 // Work split: a workgroup of 8 waves owns HPW query heads of one KV group -- 4, 2 or 1, as many as
 // divide the group -- and 256 / HPW queries of one sequence (wave w: head HPW*hg + w % HPW, queries
 // q0 + 32*(w / HPW) + [0, 32)), so every 64-key K/V tile staged in LDS feeds 256 query rows.
-// One 4096-token causal prompt, 40 heads on 8 (one head per workgroup): 205 us on an MI355X, 16 on 8
-// (two): 129 us, against 749 and 381 us in the 16-query register form (attention.hip), which reads
-// every K/V unit once per head and 48 or 96 queries; equal below about 100 tokens.
+// One 4096-token causal prompt, 40 heads on 8 (one head per workgroup): 225 us on an MI355X, 16 on 8
+// (two): 143 us, against 749 and 381 us in the 16-query register form (attention.hip), which reads
+// every K/V unit once per head and 48 or 96 queries; equal below about 100 tokens.  These groups keep
+// that form's exact running maximum and normalise by the weights as rounded, which keeps their error
+// against 64 bits (1.94e-3 to 1.93e-3; deferred and unrounded, as with four heads, 2.0e-3 and 205 us).
 //
 // Per wave and tile (swapped products, guide §3 "An accumulator tile as the next MFMA's
 // operand"):
@@ -199,7 +201,7 @@ paged_prefill_fa_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __r
     }
     const float mx = fmaxf(fmaxf(mx4[0], mx4[1]), fmaxf(mx4[2], mx4[3]));
     const float mt = pair_max(mx) * scale_log2;
-    const bool grow = mt > m_run + DEFER_LOG2;
+    const bool grow = mt > m_run + (HPW == 4 ? DEFER_LOG2 : 0.f);
     if (__any(grow)) {                                     // wave-uniform
       const float m_new = grow ? mt : m_run;
       const float alpha = grow ? exp2f(m_run - m_new) : 1.f;
@@ -220,7 +222,7 @@ paged_prefill_fa_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __r
       for (int j = 0; j < 8; ++j) {
         const float p = __builtin_amdgcn_exp2f(fmaf(sacc[ks >> 1][8 * (ks & 1) + j], scale_log2, -muse));
         pb[ks][j] = f2bf(p);
-        ps4[ks] += p;
+        ps4[ks] += HPW == 4 ? p : bf2f(pb[ks][j]);
       }
     };
     auto pv = [&](int ks0) {

@@ -265,6 +265,7 @@ struct WinAttnArgs {
   float cap;                        // > 0: scores soft-capped, cap * tanh(s / cap)
   int talk_post;                    // talk mixes the softmax weights, not the scores (scalar form)
   int gate_heads;                   // gate [rows, H]: one value per head
+  int part_min;                     // blocks that a key partition holds at least
 };
 
 // The visible keys of a 16-query tile as absolute 32-key blocks: the blocks of the kept first
@@ -284,7 +285,9 @@ EIA_DEV float wa_softcap(float s, float cap, float icap2) {
 // loads, products and the exchange is microseconds long, so a lone workgroup should walk few),
 // so short contexts use few partitions whatever the launch's grid.z (the same on both sides of
 // the merge).
-EIA_DEV int wa_parts(int nparts, int nblocks) { return min(nparts, max(1, nblocks >> 1)); }
+EIA_DEV int wa_parts(const WinAttnArgs& a, int nblocks) {
+  return min(a.nparts, max(1, nblocks / a.part_min));
+}
 
 constexpr int WA_KT = 64;           // keys per tile = lanes of a wave
 constexpr int WA_PAGES = 256;       // MFMA form: block -> page entries kept in LDS
@@ -569,7 +572,7 @@ window_attn_mfma_kernel(const WinAttnArgs a) {
   const int pos_first = a.positions[row0], pos_last = a.positions[row0 + nq - 1];
   const WaBlocks kbs = wa_blocks(pos_first, pos_last, a.window, a.keep);
   const int wb0 = kbs.wb0, nsink = kbs.nsink, nblocks = kbs.nblocks;
-  const int np = wa_parts(a.nparts, nblocks);
+  const int np = wa_parts(a, nblocks);
   if ((int)blockIdx.z >= np) return;                                // (whole workgroup)
 
   // Q^T operands of this wave's maps: column = query c, rows = d 32 s + 8 g .. + 8
@@ -890,37 +893,11 @@ window_attn_mfma_kernel(const WinAttnArgs a) {
   }
 }
 
-// Merge of key partitions and the row's epilogue: one wave per (row, head).  Lane z first turns
-// partition z's (max, sum) into its weight; the value columns are then summed over the partitions
-// with independent loads (nparts <= 64).
-__global__ void __launch_bounds__(64)
-window_attn_merge_kernel(const WinAttnArgs a) {
-  const int H = a.H, P = a.P, Dv = a.Dv, M = H * P, NP = a.nparts;
-  const long row = blockIdx.x;
-  const int h = blockIdx.y, lane = threadIdx.x;
+// Epilogue of one head: o[map][0, 1] are value columns lane and lane + 64, normalised.
+template <int P>
+EIA_DEV void wa_finish_head(const WinAttnArgs& a, long row, int h, int lane, const float (&o)[P][2]) {
+  const int Dv = a.Dv;
   bf16_t* out = (bf16_t*)a.out + row * a.ldo + h * Dv;
-  if (a.lens && a.lens[row] <= 0) return;           // padding row: the partition kernel wrote zeros
-  const int pos = a.positions[row];
-  const int np = wa_parts(NP, wa_blocks(pos, pos, a.window, a.keep).nblocks);
-  if (np == 1) return;                              // a whole row: already finished and written
-  float o[2][2];                                    // [map][column lane, lane + 64]
-  for (int pm = 0; pm < P; ++pm) {
-    const long pr = (row * M + h * P + pm) * NP;
-    const float mz = lane < np ? a.part_ml[(pr + lane) * 2] : -1e30f;
-    const float lz = lane < np ? a.part_ml[(pr + lane) * 2 + 1] : 0.f;
-    // sigmoid weights: the partitions' sums simply add up
-    const float wz = a.wmode == 1 ? (lane < np ? 1.f : 0.f) : __expf(mz - wave_max(mz));
-    const float inv = a.wmode == 1 ? 1.f : 1.0f / wave_sum(wz * lz);
-    float v0 = 0.f, v1 = 0.f;
-#pragma unroll 4
-    for (int z = 0; z < np; ++z) {
-      const float w = __shfl(wz, z, 64);
-      if (lane < Dv) v0 += w * a.part_acc[(pr + z) * Dv + lane];
-      if (lane + 64 < Dv) v1 += w * a.part_acc[(pr + z) * Dv + lane + 64];
-    }
-    o[pm][0] = v0 * inv;
-    o[pm][1] = v1 * inv;
-  }
   float r0, r1;
   if (a.epilogue == 0) {
     const bf16_t* gate = (const bf16_t*)a.gate;
@@ -936,14 +913,261 @@ window_attn_merge_kernel(const WinAttnArgs a) {
     }
   } else {
     const float lam = a.lam[0];
-    r0 = lane < Dv ? o[0][0] - lam * o[1][0] : 0.f;
-    r1 = lane + 64 < Dv ? o[0][1] - lam * o[1][1] : 0.f;
+    r0 = lane < Dv ? o[0][0] - lam * o[P - 1][0] : 0.f;
+    r1 = lane + 64 < Dv ? o[0][1] - lam * o[P - 1][1] : 0.f;
     const float inv = a.post / sqrtf(wave_sum(r0 * r0 + r1 * r1) / (float)Dv + a.eps);
     r0 *= inv;
     r1 *= inv;
   }
   if (lane < Dv) out[lane] = f2bf(r0);
   if (lane + 64 < Dv) out[lane + 64] = f2bf(r1);
+}
+
+// Decode rows without head mixing: one workgroup per (row, kv head, key partition).  The heads of the
+// kv head are the columns of the 16-query tile, so a block's K and V^T operands are loaded once for
+// all of them (a wave per head loaded them once per head, with fifteen idle columns); the four waves
+// take every fourth 32-key block of the partition and meet in LDS, so that a partition holds four
+// times the blocks and most batches need none.  Products, masks and weights as above.
+//
+// Bound by latency: a wave's blocks are a chain of loads, two products and a softmax, 1 us each.
+// MI355X, window 1024, 8 heads on 2, 3 rows: 15.5 us in four partitions (7 of them the merge's launch),
+// 64 rows: 22, 128 rows: 28 us; a wave per head took 21, 45 and 72 us.
+template <int P, int ND, int NDV, bool SIG>
+__global__ void __launch_bounds__(256, 2)
+window_decode_kernel(const WinAttnArgs a) {
+  constexpr float LOG2E = 1.4426950408889634f;
+  constexpr bool PIPE = P == 1;                         // the next block's operands are in flight
+  extern __shared__ float so[];                         // [4][P][rep][Dv]
+  __shared__ float sm[4][P][16], sl[4][P][16];
+  __shared__ int page_s[WA_PAGES];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, c = lane & 15, g = lane >> 4;
+  const int H = a.H, D = a.D, Dv = a.Dv, M = H * P, rep = H / a.G, bs = a.bs, kvh = blockIdx.y;
+  const long row = blockIdx.x;
+  const int h0 = kvh * rep;
+  bf16_t* out = (bf16_t*)a.out + row * a.ldo + (long)h0 * Dv;
+  if (a.lens && a.lens[row] <= 0) {                     // padding row: zeros
+    for (int i = tid; i < rep * Dv; i += 256) out[i] = f2bf(0.f);
+    return;
+  }
+  const int qpos = a.positions[row];
+  const WaBlocks kbs = wa_blocks(qpos, qpos, a.window, a.keep);
+  const int wb0 = kbs.wb0, nsink = kbs.nsink, nblocks = kbs.nblocks;
+  const int np = wa_parts(a, nblocks);
+  if ((int)blockIdx.z >= np) return;                    // (whole workgroup)
+  const int per = (nblocks + np - 1) / np;
+  const int b_lo = blockIdx.z * per, b_hi = min(nblocks, b_lo + per);
+  const int* bt = a.bt + row * a.ldbt;
+  for (int i = tid; i < min(b_hi - b_lo, WA_PAGES); i += 256) {
+    const int bb = b_lo + i;
+    page_s[i] = bt[((bb < nsink ? bb : wb0 + bb - nsink) << 5) / bs];
+  }
+  const bf16_t* q = (const bf16_t*)a.q;
+  const bf16_t* kc = (const bf16_t*)a.kc;
+  const bf16_t* vc = (const bf16_t*)a.vc;
+  const long krow = (long)a.G * P * D, vpage = (long)a.G * Dv * bs;
+  const int hd = h0 + min(c, rep - 1);                  // this lane's head
+  const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+  bf16x8 qf[P][ND];
+  float mult[P], slope[P], bias[P], mrun[P], lrun[P];
+  f32x4 acc[P][NDV];
+#pragma unroll
+  for (int m = 0; m < P; ++m) {
+#pragma unroll
+    for (int s = 0; s < ND; ++s) {
+      const int d = 32 * s + 8 * g;
+      const bf16x8 v = *reinterpret_cast<const bf16x8*>(q + row * a.ldq + (hd * P + m) * D +
+                                                        (d < D ? d : 0));
+      qf[m][s] = d < D ? v : zero8;
+    }
+    mult[m] = a.mult[hd * P + m];
+    slope[m] = a.slope ? a.slope[hd * P + m] : 0.f;
+    bias[m] = (SIG && a.bias) ? a.bias[hd * P + m] : 0.f;
+    const bool snk = !SIG && a.sink && blockIdx.z == 0 && w == 0;
+    mrun[m] = snk ? a.sink[hd * P + m] : -1e30f;
+    lrun[m] = snk ? 1.f : 0.f;
+#pragma unroll
+    for (int t = 0; t < NDV; ++t) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  const float cap = a.cap, icap2 = cap > 0.f ? 2.f * LOG2E / cap : 0.f;
+  const int r0 = 8 * (c >> 2) + (c & 3), dq = 8 * g, ndv = Dv >> 4;
+  __syncthreads();
+  struct Ops { bf16x8 k[P][2][ND], v[NDV]; };
+  auto load = [&](int b, Ops& o) {
+    const int key0 = (b < nsink ? b : wb0 + b - nsink) << 5;
+    const long page = b - b_lo < WA_PAGES ? page_s[b - b_lo] : bt[key0 / bs];
+    const bf16_t* kp = kc + (page * bs + key0 % bs + r0) * krow + (long)kvh * P * D;
+#pragma unroll
+    for (int m = 0; m < P; ++m)
+#pragma unroll
+      for (int s = 0; s < ND; ++s) {                    // (past D the queries are zero)
+        const int d = min(32 * s + dq, D - 8);
+        o.k[m][0][s] = *reinterpret_cast<const bf16x8*>(kp + m * D + d);
+        o.k[m][1][s] = *reinterpret_cast<const bf16x8*>(kp + 4 * krow + m * D + d);
+      }
+    const bf16_t* vp = vc + page * vpage + ((long)kvh * Dv + c) * bs + key0 % bs + dq;
+#pragma unroll
+    for (int t = 0; t < NDV; ++t)
+      o.v[t] = *reinterpret_cast<const bf16x8*>(vp + (long)(t < ndv ? t : 0) * 16 * bs);
+  };
+  auto block = [&](int b, const Ops& o) {
+    const int key0 = (b < nsink ? b : wb0 + b - nsink) << 5;
+    bool vis[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int key = key0 + 8 * g + e;
+      vis[e] = key <= qpos && (a.window <= 0 || qpos - key < a.window || key < a.keep);
+    }
+#pragma unroll
+    for (int m = 0; m < P; ++m) {
+      f32x4 sc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+      for (int s = 0; s < ND; ++s) {
+        sc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.k[m][0][s], qf[m][s], sc[0], 0, 0, 0);
+        sc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.k[m][1][s], qf[m][s], sc[1], 0, 0, 0);
+      }
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        v[e] = sc[e >> 2][e & 3] * mult[m] - slope[m] * (float)(qpos - key0 - 8 * g - e);
+      if (cap > 0.f) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = wa_softcap(v[e], cap, icap2);
+      }
+      bf16x8 ph, pl;
+      float alpha = 1.f;
+      if constexpr (SIG) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float p = vis[e] ? __builtin_amdgcn_rcpf(1.0f + exp2f(-(v[e] + bias[m]) * LOG2E)) : 0.f;
+          ph[e] = f2bf(p);
+          pl[e] = f2bf(p - bf2f(ph[e]));
+        }
+        lrun[m] = 1.f;
+      } else {
+        float mloc = -1e30f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (vis[e]) mloc = fmaxf(mloc, v[e]);
+        mloc = fmaxf(mloc, __shfl_xor(mloc, 16, 64));
+        mloc = fmaxf(mloc, __shfl_xor(mloc, 32, 64));
+        const float mnew = fmaxf(mrun[m], mloc);
+        alpha = exp2f((mrun[m] - mnew) * LOG2E);
+        float psum = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float p = vis[e] ? exp2f((v[e] - mnew) * LOG2E) : 0.f;
+          ph[e] = f2bf(p);
+          pl[e] = f2bf(p - bf2f(ph[e]));
+          psum += p;
+        }
+        psum += __shfl_xor(psum, 16, 64);
+        psum += __shfl_xor(psum, 32, 64);
+        lrun[m] = lrun[m] * alpha + psum;
+        mrun[m] = mnew;
+      }
+#pragma unroll
+      for (int t = 0; t < NDV; ++t) {
+        f32x4 x = SIG ? acc[m][t] : acc[m][t] * alpha;
+        x = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.v[t], ph, x, 0, 0, 0);
+        acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.v[t], pl, x, 0, 0, 0);
+      }
+    }
+  };
+  if constexpr (PIPE) {
+    Ops o0, o1;
+    if (b_lo + w < b_hi) load(b_lo + w, o0);
+    for (int b = b_lo + w; b < b_hi; b += 8) {
+      if (b + 4 < b_hi) load(b + 4, o1);
+      block(b, o0);
+      if (b + 4 >= b_hi) break;
+      if (b + 8 < b_hi) load(b + 8, o0);
+      block(b + 4, o1);
+    }
+  } else {
+    Ops o;
+    for (int b = b_lo + w; b < b_hi; b += 4) {
+      load(b, o);
+      block(b, o);
+    }
+  }
+  // the waves' sums meet: this lane holds, per map and tile t, value columns 16 t + 4 g + i of head c
+  if (c < rep) {
+#pragma unroll
+    for (int m = 0; m < P; ++m) {
+      if (g == 0) {
+        sm[w][m][c] = mrun[m];
+        sl[w][m][c] = lrun[m];
+      }
+#pragma unroll
+      for (int t = 0; t < NDV; ++t)
+        if (t < ndv)
+          *reinterpret_cast<f32x4*>(so + ((w * P + m) * rep + c) * Dv + 16 * t + 4 * g) = acc[m][t];
+    }
+  }
+  __syncthreads();
+  for (int x = w; x < rep; x += 4) {                    // wave per head, columns lane and lane + 64
+    float o[P][2];
+#pragma unroll
+    for (int m = 0; m < P; ++m) {
+      float mx = sm[0][m][x], ls = 0.f, v0 = 0.f, v1 = 0.f;
+#pragma unroll
+      for (int z = 1; z < 4; ++z) mx = fmaxf(mx, sm[z][m][x]);
+#pragma unroll
+      for (int z = 0; z < 4; ++z) {
+        const float wz = SIG ? 1.f : exp2f((sm[z][m][x] - mx) * LOG2E);
+        const float* p = so + ((z * P + m) * rep + x) * Dv;
+        ls += wz * sl[z][m][x];
+        if (lane < Dv) v0 += wz * p[lane];
+        if (lane + 64 < Dv) v1 += wz * p[lane + 64];
+      }
+      if (np > 1) {                                     // window_attn_merge_kernel finishes the row
+        const long pr = (row * M + (h0 + x) * P + m) * a.nparts + blockIdx.z;
+        if (lane == 0) {
+          a.part_ml[pr * 2] = mx;
+          a.part_ml[pr * 2 + 1] = ls;
+        }
+        if (lane < Dv) a.part_acc[pr * Dv + lane] = v0;
+        if (lane + 64 < Dv) a.part_acc[pr * Dv + lane + 64] = v1;
+      }
+      const float inv = SIG ? 1.f : 1.0f / ls;
+      o[m][0] = v0 * inv;
+      o[m][1] = v1 * inv;
+    }
+    if (np == 1) wa_finish_head(a, row, h0 + x, lane, o);
+  }
+}
+
+// Merge of key partitions and the row's epilogue: one wave per (row, head).  Lane z first turns
+// partition z's (max, sum) into its weight; the value columns are then summed over the partitions
+// with independent loads (nparts <= 64).
+__global__ void __launch_bounds__(64)
+window_attn_merge_kernel(const WinAttnArgs a) {
+  const int H = a.H, P = a.P, Dv = a.Dv, M = H * P, NP = a.nparts;
+  const long row = blockIdx.x;
+  const int h = blockIdx.y, lane = threadIdx.x;
+  if (a.lens && a.lens[row] <= 0) return;           // padding row: the partition kernel wrote zeros
+  const int pos = a.positions[row];
+  const int np = wa_parts(a, wa_blocks(pos, pos, a.window, a.keep).nblocks);
+  if (np == 1) return;                              // a whole row: already finished and written
+  float o[2][2];                                    // [map][column lane, lane + 64]
+  for (int pm = 0; pm < P; ++pm) {
+    const long pr = (row * M + h * P + pm) * NP;
+    const float mz = lane < np ? a.part_ml[(pr + lane) * 2] : -1e30f;
+    const float lz = lane < np ? a.part_ml[(pr + lane) * 2 + 1] : 0.f;
+    // sigmoid weights: the partitions' sums simply add up
+    const float wz = a.wmode == 1 ? (lane < np ? 1.f : 0.f) : __expf(mz - wave_max(mz));
+    const float inv = a.wmode == 1 ? 1.f : 1.0f / wave_sum(wz * lz);
+    float v0 = 0.f, v1 = 0.f;
+#pragma unroll 8
+    for (int z = 0; z < np; ++z) {
+      const float w = __shfl(wz, z, 64);
+      if (lane < Dv) v0 += w * a.part_acc[(pr + z) * Dv + lane];
+      if (lane + 64 < Dv) v1 += w * a.part_acc[(pr + z) * Dv + lane + 64];
+    }
+    o[pm][0] = v0 * inv;
+    o[pm][1] = v1 * inv;
+  }
+  wa_finish_head(a, row, h, lane, o);
 }
 
 // Heads per wave of the MFMA form for (H, P), 0 when the shape runs the scalar form: with head
@@ -956,6 +1180,9 @@ static int wa_mfma_hw(int H, int P, int talk) {
   if (H <= 16 && H % 2 == 0) return 2;
   return 0;
 }
+
+// Whether decode rows take the form that packs the heads of a kv head into one query tile.
+EIA_API int eia_window_decode_packed(int H, int G) { return G > 0 && H % G == 0 && H / G <= 16; }
 
 EIA_API int eia_window_attn_mfma_ok(int H, int G, int P, int D, int Dv, int bs, int talk) {
   const int hw = wa_mfma_hw(H, P, talk);
@@ -988,6 +1215,8 @@ EIA_API int eia_window_attn_mfma(const void* q, long ldq, const void* kc, const 
   WinAttnArgs a{q, ldq, kc, vc, bt, ldbt, positions, cu, work, lens, mult, slope, talk, gate, ldg,
                 out, ldo, H, G, P, D, Dv, bs, window, keep, 16, epilogue, lam, eps, post, nparts,
                 2, part_acc, part_ml, wmode, bias, sink, cap, 0, gate_heads};
+  const bool packed = !cu && !talk && eia_window_decode_packed(H, G);
+  a.part_min = packed ? 8 : 2;
   // raw-score buffers of the head-mixing form: two (one barrier per block) while they fit 48 KiB
   if (talk) a.raw_bufs = (size_t)2 * H * P * 128 * sizeof(f32x4) > 48 * 1024 ? 1 : 2;
   // sigmoid weights: a wave takes two heads of one kv head where the grouping allows it, so the
@@ -1025,6 +1254,28 @@ EIA_API int eia_window_attn_mfma(const void* q, long ldq, const void* kc, const 
       hipLaunchKernelGGL((window_attn_mfma_kernel<1, 1, false, true, NDX, NDVX, true>), grid,   \
                          block, lds, st, a);                                                    \
   } while (0)
+  if (packed) {
+    const dim3 dg(n_items, G, nparts), db(256);
+    const size_t dl = sizeof(float) * 4 * P * (H / G) * Dv;
+#define WD_GO(PV, NDX, NDVX, SG)                                                                \
+  do {                                                                                          \
+    if (dl > 48 * 1024)                                                                         \
+      (void)hipFuncSetAttribute(                                                                \
+          reinterpret_cast<const void*>(&window_decode_kernel<PV, NDX, NDVX, SG>),              \
+          hipFuncAttributeMaxDynamicSharedMemorySize, (int)dl);                                 \
+    hipLaunchKernelGGL((window_decode_kernel<PV, NDX, NDVX, SG>), dg, db, dl, st, a);           \
+  } while (0)
+#define WD_DIMS(PV, SG)                                                                         \
+  do {                                                                                          \
+    if (D > 64) WD_GO(PV, 4, 8, SG); else if (Dv > 64) WD_GO(PV, 2, 8, SG); else WD_GO(PV, 2, 4, SG); \
+  } while (0)
+    if (P == 2) WD_DIMS(2, false); else if (wmode == 1) WD_DIMS(1, true); else WD_DIMS(1, false);
+#undef WD_DIMS
+#undef WD_GO
+    if (nparts > 1)
+      hipLaunchKernelGGL(window_attn_merge_kernel, dim3(n_items, H), dim3(64), 0, st, a);
+    EIA_LAUNCH_CHECK();
+  }
   // without head mixing the key width may be half the value width (a differential pair)
   const bool narrow_k = !talk && D <= 64 && Dv > 64;
   if (talk) {

@@ -130,6 +130,7 @@ _SIGNATURES = {
     "eia_xielu": [P, L, P, I, L, P, P, L, I, I, I, S],
     "eia_sigmoid_gate": [P, L, L, I, P, L, P, L, I, I, I, S],
     "eia_window_attn_mfma_ok": [I, I, I, I, I, I, I],
+    "eia_window_decode_packed": [I, I],
     "eia_ar_alloc": [P, L],
     "eia_moe_splitk_norm_route": [P, I, I, I, P, P, F, P, L, P, I, I, I, I, P, P, P, S],
     "eia_moe_combine_norm": [P, I, I, P, P, I, I, I, P, P, F, P, L, S],

@@ -78,3 +78,45 @@ def test_window_flash(window, new, past, H, G, D, Dv, bs, kind):
     # both sides sum in fp32 and round once to bf16 (2^-9): neighbouring roundings at most
     assert float((a - b).norm() / a.norm()) < 4e-3
     assert float(((a - b).abs() / (a.abs() + 0.05 * a.abs().mean())).max()) < 2 ** -6
+
+
+@pytest.mark.parametrize("kind", ["plain", "cap", "sigmoid", "pair", "keep"])
+@pytest.mark.parametrize("H,G,D,Dv,bs", [(4, 1, 128, 128, 64), (6, 2, 72, 48, 32), (16, 1, 64, 64, 64),
+                                         (3, 3, 96, 96, 64), (10, 2, 64, 112, 128)])
+@pytest.mark.parametrize("window", [0, 50, 600])
+@pytest.mark.parametrize("parts", [1, 3, 16])
+def test_window_decode(parts, window, H, G, D, Dv, bs, kind, monkeypatch):
+    from enterprise_inference_amd.ops import attention as A
+    from enterprise_inference_amd.ops import window_attention as wa
+    monkeypatch.setenv("EIA_WINDOW_DECODE_P", str(parts))
+    if kind == "pair":
+        D = 64 if D > 64 else 40
+    g = torch.Generator().manual_seed(H + D + window)
+    P = 2 if kind == "pair" else 1
+    lens = [1, 32, 33, 0, 257, 700]                          # (0: a padding row)
+    pages = [max(1, -(-n // bs)) for n in lens]
+    order = torch.randperm(sum(pages), generator=g).to(torch.int32)
+    bt = torch.zeros(len(lens), max(pages), dtype=torch.int32)
+    at = 0
+    for s, n in enumerate(pages):
+        bt[s, :n] = order[at:at + n]
+        at += n
+    pos = torch.tensor([max(0, n - 1) for n in lens], dtype=torch.int32)
+    bf, T = torch.bfloat16, len(lens)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(bf)
+    q, k, v = rnd(T, H * P * D), rnd(sum(pages), bs, G * P * D), rnd(sum(pages), G * Dv, bs)
+    gate = None if kind == "pair" else rnd(T, H if kind == "cap" else H * Dv)
+
+    def run(dev):
+        md = A.AttentionMetadata(
+            num_decode=T, num_prefill_tokens=0, slot_mapping=pos.to(dev), positions=pos.to(dev),
+            decode_block_tables=bt.to(dev),
+            decode_seq_lens=torch.tensor(lens, dtype=torch.int32, device=dev))
+        spec = _spec(wa, kind, H, G, D, Dv, window, dev)
+        spec.gate_heads = kind == "cap"
+        return wa.window_attention(q.to(dev), k.to(dev), v.to(dev), md, spec,
+                                   None if gate is None else gate.to(dev)).cpu()
+
+    a, b = run("cpu").double(), run("cuda").double()
+    live = torch.tensor(lens) > 0
+    assert float((a - b)[live].norm() / a[live].norm()) < 4e-3   # as above

@@ -566,8 +566,10 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
 
     def launch(lo, n_items, bt, lens, cu, work, qb):
         require(bt.dtype == torch.int32 and bt.stride(1) == 1, "block tables int32")
-        qa, o = q[lo:], out[lo:]
-        g = None if gate is None else gate[lo:]
+        qa, o, g, pos = q, out, gate, md.positions
+        if lo:
+            qa, o, pos = q[lo:], out[lo:], pos[lo:]
+            g = None if gate is None else gate[lo:]
         if mfma and spec.talk_post:
             rows = n_items if cu is None else T - lo
             NP = head_mix_partitions(n_items, spec) if cu is None else 1
@@ -576,7 +578,7 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
             ml = torch.empty(rows * NP * H * 2, dtype=torch.float32, device=q.device)
             check(lib().eia_head_mix_attn(
                 ptr(qa), qa.stride(0), ptr(k_cache), ptr(v_cache), ptr(bt), bt.stride(0),
-                ptr(md.positions[lo:]), ptr(cu), ptr(work), ptr(lens), n_items, rows,
+                ptr(pos), ptr(cu), ptr(work), ptr(lens), n_items, rows,
                 ptr(spec.mult), ptr(spec.talk), ptr(o), o.stride(0), H, spec.kv_heads, D, Dv, bs,
                 spec.window, float(spec.cap), float(spec.post), NP, ptr(acc), ptr(ml), stream(q)),
                 "head_mix_attn")
@@ -590,7 +592,7 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
                                  dtype=torch.float32, device=q.device)
             check(lib().eia_window_flash(
                 ptr(qa), qa.stride(0), ptr(k_cache), ptr(v_cache), ptr(bt), bt.stride(0),
-                ptr(md.positions[lo:]), ptr(cu), ptr(work), n_items, ptr(spec.mult), ptr(g),
+                ptr(pos), ptr(cu), ptr(work), n_items, ptr(spec.mult), ptr(g),
                 g.stride(0) if g is not None else 0, ptr(o), o.stride(0), H, spec.kv_heads, P, D,
                 Dv, bs, spec.window, spec.keep, ptr(spec.lam) if P == 2 else None,
                 float(spec.eps), float(spec.post), spec.weights, ptr(spec.bias), ptr(spec.sink),
@@ -601,20 +603,22 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
             NP = decode_partitions(n_items, spec) if cu is None else 1
             pa = pm = None
             if NP > 1:
-                pa = torch.empty(n_items * H * P * NP * Dv, dtype=torch.float32, device=q.device)
-                pm = torch.empty(n_items * H * P * NP * 2, dtype=torch.float32, device=q.device)
+                n = n_items * H * P * NP
+                ws = torch.empty(n * (Dv + 2), dtype=torch.float32, device=q.device)
+                pa = ws.data_ptr()
+                pm = pa + 4 * n * Dv
             check(lib().eia_window_attn_mfma(
                 ptr(qa), qa.stride(0), ptr(k_cache), ptr(v_cache), ptr(bt), bt.stride(0),
-                ptr(md.positions[lo:]), ptr(cu), ptr(work), ptr(lens), n_items, ptr(spec.mult),
+                ptr(pos), ptr(cu), ptr(work), ptr(lens), n_items, ptr(spec.mult),
                 ptr(spec.slope), ptr(spec.talk), ptr(g), g.stride(0) if g is not None else 0,
                 ptr(o), o.stride(0), H, spec.kv_heads, P, D, Dv, bs, spec.window, spec.keep,
                 spec.epilogue, ptr(spec.lam), float(spec.eps), float(spec.post), spec.weights,
-                ptr(spec.bias), NP, ptr(pa), ptr(pm), ptr(spec.sink), float(spec.cap),
+                ptr(spec.bias), NP, pa, pm, ptr(spec.sink), float(spec.cap),
                 1 if spec.gate_heads else 0, stream(q)), "window_attn_mfma")
             return
         check(lib().eia_window_attn(
             ptr(qa), qa.stride(0), ptr(k_cache), ptr(v_cache), ptr(bt), bt.stride(0),
-            ptr(md.positions[lo:]), ptr(cu), ptr(work), ptr(lens), n_items, ptr(spec.mult),
+            ptr(pos), ptr(cu), ptr(work), ptr(lens), n_items, ptr(spec.mult),
             ptr(spec.slope), ptr(spec.talk), ptr(g), g.stride(0) if g is not None else 0, ptr(o),
             o.stride(0), H, spec.kv_heads, P, D, Dv, bs, spec.window, spec.keep, qb,
             spec.epilogue, ptr(spec.lam), float(spec.eps), float(spec.post), spec.weights,

@@ -265,7 +265,6 @@ struct WinAttnArgs {
   float cap;                        // > 0: scores soft-capped, cap * tanh(s / cap)
   int talk_post;                    // talk mixes the softmax weights, not the scores (scalar form)
   int gate_heads;                   // gate [rows, H]: one value per head
-  int part_min;                     // blocks that a key partition holds at least
 };
 
 // The visible keys of a 16-query tile as absolute 32-key blocks: the blocks of the kept first
@@ -285,9 +284,9 @@ EIA_DEV float wa_softcap(float s, float cap, float icap2) {
 // loads, products and the exchange is microseconds long, so a lone workgroup should walk few),
 // so short contexts use few partitions whatever the launch's grid.z (the same on both sides of
 // the merge).
-EIA_DEV int wa_parts(const WinAttnArgs& a, int nblocks) {
-  return min(a.nparts, max(1, nblocks / a.part_min));
-}
+EIA_DEV int wa_parts(int nparts, int nblocks) { return min(nparts, max(1, nblocks >> 1)); }
+// (of window_decode_kernel: two blocks for each of its four waves)
+EIA_DEV int wd_parts(int nparts, int nblocks) { return min(nparts, max(1, nblocks >> 3)); }
 
 constexpr int WA_KT = 64;           // keys per tile = lanes of a wave
 constexpr int WA_PAGES = 256;       // MFMA form: block -> page entries kept in LDS
@@ -572,7 +571,7 @@ window_attn_mfma_kernel(const WinAttnArgs a) {
   const int pos_first = a.positions[row0], pos_last = a.positions[row0 + nq - 1];
   const WaBlocks kbs = wa_blocks(pos_first, pos_last, a.window, a.keep);
   const int wb0 = kbs.wb0, nsink = kbs.nsink, nblocks = kbs.nblocks;
-  const int np = wa_parts(a, nblocks);
+  const int np = wa_parts(a.nparts, nblocks);
   if ((int)blockIdx.z >= np) return;                                // (whole workgroup)
 
   // Q^T operands of this wave's maps: column = query c, rows = d 32 s + 8 g .. + 8
@@ -952,7 +951,7 @@ window_decode_kernel(const WinAttnArgs a) {
   const int qpos = a.positions[row];
   const WaBlocks kbs = wa_blocks(qpos, qpos, a.window, a.keep);
   const int wb0 = kbs.wb0, nsink = kbs.nsink, nblocks = kbs.nblocks;
-  const int np = wa_parts(a, nblocks);
+  const int np = wd_parts(a.nparts, nblocks);
   if ((int)blockIdx.z >= np) return;                    // (whole workgroup)
   const int per = (nblocks + np - 1) / np;
   const int b_lo = blockIdx.z * per, b_hi = min(nblocks, b_lo + per);
@@ -1140,6 +1139,7 @@ window_decode_kernel(const WinAttnArgs a) {
 // Merge of key partitions and the row's epilogue: one wave per (row, head).  Lane z first turns
 // partition z's (max, sum) into its weight; the value columns are then summed over the partitions
 // with independent loads (nparts <= 64).
+template <bool PACKED>
 __global__ void __launch_bounds__(64)
 window_attn_merge_kernel(const WinAttnArgs a) {
   const int H = a.H, P = a.P, Dv = a.Dv, M = H * P, NP = a.nparts;
@@ -1147,7 +1147,8 @@ window_attn_merge_kernel(const WinAttnArgs a) {
   const int h = blockIdx.y, lane = threadIdx.x;
   if (a.lens && a.lens[row] <= 0) return;           // padding row: the partition kernel wrote zeros
   const int pos = a.positions[row];
-  const int np = wa_parts(a, wa_blocks(pos, pos, a.window, a.keep).nblocks);
+  const int nblocks = wa_blocks(pos, pos, a.window, a.keep).nblocks;
+  const int np = PACKED ? wd_parts(NP, nblocks) : wa_parts(NP, nblocks);
   if (np == 1) return;                              // a whole row: already finished and written
   float o[2][2];                                    // [map][column lane, lane + 64]
   for (int pm = 0; pm < P; ++pm) {
@@ -1158,7 +1159,7 @@ window_attn_merge_kernel(const WinAttnArgs a) {
     const float wz = a.wmode == 1 ? (lane < np ? 1.f : 0.f) : __expf(mz - wave_max(mz));
     const float inv = a.wmode == 1 ? 1.f : 1.0f / wave_sum(wz * lz);
     float v0 = 0.f, v1 = 0.f;
-#pragma unroll 8
+#pragma unroll 4
     for (int z = 0; z < np; ++z) {
       const float w = __shfl(wz, z, 64);
       if (lane < Dv) v0 += w * a.part_acc[(pr + z) * Dv + lane];
@@ -1216,7 +1217,6 @@ EIA_API int eia_window_attn_mfma(const void* q, long ldq, const void* kc, const 
                 out, ldo, H, G, P, D, Dv, bs, window, keep, 16, epilogue, lam, eps, post, nparts,
                 2, part_acc, part_ml, wmode, bias, sink, cap, 0, gate_heads};
   const bool packed = !cu && !talk && eia_window_decode_packed(H, G);
-  a.part_min = packed ? 8 : 2;
   // raw-score buffers of the head-mixing form: two (one barrier per block) while they fit 48 KiB
   if (talk) a.raw_bufs = (size_t)2 * H * P * 128 * sizeof(f32x4) > 48 * 1024 ? 1 : 2;
   // sigmoid weights: a wave takes two heads of one kv head where the grouping allows it, so the
@@ -1273,7 +1273,7 @@ EIA_API int eia_window_attn_mfma(const void* q, long ldq, const void* kc, const 
 #undef WD_DIMS
 #undef WD_GO
     if (nparts > 1)
-      hipLaunchKernelGGL(window_attn_merge_kernel, dim3(n_items, H), dim3(64), 0, st, a);
+      hipLaunchKernelGGL(window_attn_merge_kernel<true>, dim3(n_items, H), dim3(64), 0, st, a);
     EIA_LAUNCH_CHECK();
   }
   // without head mixing the key width may be half the value width (a differential pair)
@@ -1297,6 +1297,6 @@ EIA_API int eia_window_attn_mfma(const void* q, long ldq, const void* kc, const 
 #undef WA_LAUNCH
 #undef WA_LAUNCH1
   if (nparts > 1)
-    hipLaunchKernelGGL(window_attn_merge_kernel, dim3(n_items, H), dim3(64), 0, st, a);
+    hipLaunchKernelGGL(window_attn_merge_kernel<false>, dim3(n_items, H), dim3(64), 0, st, a);
   EIA_LAUNCH_CHECK();
 }

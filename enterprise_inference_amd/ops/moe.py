@@ -181,8 +181,8 @@ def fused_moe(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, topk_w: torc
         return ref.fused_moe(x, w13, w2, tw, ids.clamp(0, El - 1).to(torch.int32), act)
     avg = T * k / max(1, El)
     capturable = capturable or torch.cuda.is_current_stream_capturing()
-    if act == "silu" and _grouped_ok(x, w13, w2) and not (
-            _mfma_ok(x, w13, w2) and _mfma_pays(avg, El, w13.shape[1] // 2, H)) and avg <= 96:
+    if act == "silu" and avg <= 96 and _grouped_ok(x, w13, w2) and not (
+            _mfma_pays(avg, El, w13.shape[1] // 2, H) and _mfma_ok(x, w13, w2)):
         return _fused_moe_grouped(x, w13, w2, topk_w, topk_ids, e_lo, e_hi,
                                   defer_combine=defer_combine)
     # (small experts stay on the grouped MFMA kernel at any row count: their per-expert library

@@ -244,6 +244,132 @@ linear_scan_kernel(ScanArgs a) {
   }
 }
 
+// Decode rows (one token per sequence, dk and dv up to 128): one workgroup per (row, head).  The state
+// is requested first, 16 bytes per access, and everything else -- q, k, v, the gates or the decays,
+// each by threads of its own -- is formed while it is on its way; it is scaled, used and stored from the
+// registers that it arrives in.  Thread (rg, cg) holds rows rg, rg + RG, ... of columns 4 cg ..
+//
+// Bound by the state's traffic (64 rows, 16 heads of 128 x 128, exponential gates: 22 us for 134 MB on an
+// MI355X) and, at a few rows, by one round of dependent loads (6 us).  The kernel above, made to walk
+// tokens, took 61 and 15 us: 4-byte state accesses, the gates and decays in a chain of their own behind
+// barriers, and with dk < dv half of its threads without rows.
+template <typename T, int DM, int W, bool NRM, bool CH>       // dk <= DM, dv <= W
+__global__ void __launch_bounds__(256)
+linear_decode_kernel(ScanArgs a) {
+  constexpr int CG = W / 4, RG = 256 / CG, NR = DM / RG;
+  __shared__ float sq[DM], sk[DM], sal[CH ? DM : 1];
+  __shared__ __align__(16) float sv[W], po[RG][W];
+  __shared__ float sgate[3], red[4], rn[4];
+  const int s = blockIdx.x, h = blockIdx.y, D = a.D, Dv = a.Dv, tid = threadIdx.x;
+  const int slot = a.slots[s];
+  if (slot < 0 || (a.seq_lens && a.seq_lens[s] <= 0)) return;
+  const bool fresh = a.positions[s] == 0;
+  const int cg = tid % CG, rg = tid / CG, c0 = min(4 * cg, Dv - 4);     // (Dv % 4 == 0)
+  float* Sg = a.S + ((long)slot * a.H + h) * D * Dv;
+  f32x4 S[NR];
+#pragma unroll
+  for (int i = 0; i < NR; ++i)
+    S[i] = *reinterpret_cast<const f32x4*>(Sg + (long)min(rg + RG * i, D - 1) * Dv + c0);
+  const T* xr = static_cast<const T*>(a.x) + (long)s * a.ld;
+  const bool chan = tid < D, col = tid < Dv;
+  float n = 0.f, q = 0.f, k = 0.f;
+  if (tid < DM) {
+    if (chan) {
+      if (NRM && !fresh) n = a.N[((long)slot * a.H + h) * D + tid];
+      const long qc = a.q_off + (long)h * D, kc = a.k_off + (long)h * D;
+      q = ld_f32<T>(xr, qc + tid);
+      k = ld_f32<T>(xr, kc + tid);
+      if (tid < a.rot_dims) {
+        const int hd = a.rot_dims >> 1;
+        const bool second = a.rot_half ? tid >= hd : (tid & 1);
+        const int pi = a.rot_half ? (second ? tid - hd : tid) : (tid >> 1);
+        const int jp = a.rot_half ? (second ? tid - hd : tid + hd) : (tid ^ 1);
+        const float sgn = second ? 1.f : -1.f;
+        float sn, cs;
+        sincosf((float)a.positions[s] * a.inv_freq[pi], &sn, &cs);
+        q = q * cs + sgn * ld_f32<T>(xr, qc + jp) * sn;
+        k = k * cs + sgn * ld_f32<T>(xr, kc + jp) * sn;
+      }
+      q *= a.qscale;
+      k *= a.kscale;
+    }
+    sq[tid] = q;
+    sk[tid] = k;
+  }
+  if (tid < W) sv[tid] = col ? ld_f32<T>(xr, a.v_off + (long)h * Dv + tid) : 0.f;
+  if constexpr (CH) {
+    const int j = tid - 128;
+    if (j >= 0 && j < DM) sal[j] = j < D ? expf(ls_chan_log<T>(a, xr, h, j)) : 1.f;
+  } else if (NRM && tid == 255) {
+    const float xi = ld_f32<T>(xr, a.i_off + h), xf = ld_f32<T>(xr, a.f_off + h);
+    const float gi = a.cap > 0.f ? a.cap * tanhf(xi / a.cap) : xi;
+    const float gf = ls_logsigmoid(a.cap > 0.f ? a.cap * tanhf(xf / a.cap) : xf);
+    const float fm = gf + (fresh ? 0.f : a.M[(long)slot * a.H + h]), m = fmaxf(fm, gi);
+    sgate[0] = expf(fm - m);
+    sgate[1] = expf(gi - m);
+    sgate[2] = expf(-m);
+    a.M[(long)slot * a.H + h] = m;
+  }
+  const float g = (tid < W && col) ? ld_f32<T>(xr, a.g_off + (long)h * Dv + tid) : 0.f;
+  const T* NW = static_cast<const T*>(a.norm_w);
+  const float nw = (NW && tid < W && col) ? ld_f32<T>(NW, (long)h * a.norm_h + tid) : 1.f;
+  __syncthreads();
+  const float at = NRM ? sgate[0] : CH ? 1.f : a.decay[h], bt = NRM ? sgate[1] : 1.f;
+  if constexpr (NRM) {
+    n = at * n + bt * k;
+    if (chan) a.N[((long)slot * a.H + h) * D + tid] = n;
+    const float nq = wave_sum(chan ? q * n : 0.f);
+    if ((tid & 63) == 0) rn[tid >> 6] = nq;
+  }
+  const f32x4 v = *reinterpret_cast<const f32x4*>(&sv[c0]);
+  f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < NR; ++i) {
+    const int r = rg + RG * i;
+    if (r < D) {
+      const f32x4 z = fresh ? f32x4{0.f, 0.f, 0.f, 0.f} : S[i];
+      const f32x4 u = (CH ? sal[r] : at) * z + (bt * sk[r]) * v;
+      o += sq[r] * u;
+      if (4 * cg < Dv) *reinterpret_cast<f32x4*>(Sg + (long)r * Dv + c0) = u;
+    }
+  }
+  if (4 * cg < Dv) *reinterpret_cast<f32x4*>(&po[rg][4 * cg]) = o;
+  __syncthreads();
+  float y = 0.f;
+  if (tid < W && col) {
+#pragma unroll
+    for (int x = 0; x < RG; ++x) y += po[x][tid];
+    if constexpr (NRM) y = y / (fmaxf(fabsf(rn[0] + rn[1] + rn[2] + rn[3]), sgate[2]) + 1e-6f);
+  }
+  const float ss = wave_sum(y * y);
+  if ((tid & 63) == 0) red[tid >> 6] = ss;
+  __syncthreads();
+  if (tid < W && col) {
+    const float sig = 1.0f / (1.0f + expf(-g));
+    const float all = W == 64 ? red[0] : red[0] + red[1];
+    st_f32<T>(static_cast<T*>(a.y), (long)s * a.ldy + (long)h * Dv + tid,
+              y / sqrtf(all * (1.0f / (float)Dv) + a.eps) * nw * (a.gate_act == 0 ? g * sig : sig) *
+                  a.out_scale);
+  }
+}
+
+template <typename T>
+static void linear_decode(const ScanArgs& a, int nseq, hipStream_t st) {
+  const dim3 grid(nseq, a.H), block(256);
+#define LD_GO(DM, W, N, C) \
+  hipLaunchKernelGGL((linear_decode_kernel<T, DM, W, N, C>), grid, block, 0, st, a)
+#define LD_MODES(DM, W)                                                                             \
+  do {                                                                                              \
+    if (a.mode == 1) LD_GO(DM, W, true, false);                                                     \
+    else if (a.mode == 2) LD_GO(DM, W, false, true);                                                \
+    else LD_GO(DM, W, false, false);                                                                \
+  } while (0)
+  if (a.D <= 64) { if (a.Dv <= 64) LD_MODES(64, 64); else LD_MODES(64, 128); }
+  else { if (a.Dv <= 64) LD_MODES(128, 64); else LD_MODES(128, 128); }
+#undef LD_MODES
+#undef LD_GO
+}
+
 // x: fused rows (bf16 when is_bf16, else fp32) holding the q [H*D], k [H*D], v [H*Dv] and gate
 // [H*Dv] columns at the given offsets (mode 1: also the H input-gate and H forget-gate
 // pre-activations at i_off / f_off); y [rows, >= H*Dv] of the same type.
@@ -268,6 +394,10 @@ EIA_API int eia_linear_scan(const void* x, long ld, int q_off, int k_off, int v_
   ScanArgs a{x, ld, q_off, k_off, v_off, g_off, i_off, f_off, decay, inv_freq, rot_dims, rot_half,
              qscale, kscale, cap, out_scale, norm_w, S, N, M, slots, cu, positions, seq_lens, y,
              ldy, eps, H, D, Dv, mode, gate_act, lo_off, R, a2t, a2b, inv_tau, norm_h};
+  if (!cu && D <= 128 && Dv <= 128 && Dv % 4 == 0 && reinterpret_cast<uintptr_t>(S) % 16 == 0) {
+    if (is_bf16) linear_decode<bf16_t>(a, nseq, st); else linear_decode<float>(a, nseq, st);
+    EIA_LAUNCH_CHECK();
+  }
   dim3 grid(nseq, H);
 #define LS_LAUNCH(TT, DM, NR, CHN)                                                                  \
   hipLaunchKernelGGL((linear_scan_kernel<TT, DM, NR, CHN>), grid, dim3(4 * (DM < 64 ? 64 : DM)), 0, \

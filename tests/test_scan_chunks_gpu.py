@@ -167,3 +167,44 @@ def test_channel_chunks(lens, H, D, Dv, R, rot, dtype, monkeypatch):
     # adds one rounding and at times one step more
     assert _rel(z[live], y[live]) < (2e-5 if dtype == torch.float32 else 4e-3)
     assert _rel(Z, S) < 4e-6
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("mode", ["decay", "exp_gates", "channel"])
+@pytest.mark.parametrize("H,D,Dv,rot", [(2, 64, 64, 0), (3, 64, 128, 64), (2, 128, 128, 0),
+                                        (1, 72, 40, 12), (2, 17, 100, 0), (2, 64, 6, 0)])
+def test_linear_decode_rows(H, D, Dv, rot, mode, dtype):
+    from enterprise_inference_amd.ops import linear_scan as ls
+    g = torch.Generator().manual_seed(D + Dv)
+    rnd = lambda *s: torch.randn(*s, generator=g)
+    n, R = 5, 9
+    pos = torch.tensor([0, 7, 300, 4, 0], dtype=torch.int32)
+    slots = torch.tensor([3, 0, -1, 4, 1], dtype=torch.int32)
+    lens = torch.tensor([1, 8, 301, 0, 1], dtype=torch.int32)      # (0: a padding row)
+    at = [0, H * D, 2 * H * D, 2 * H * D + H * Dv, 2 * H * (D + Dv), 2 * H * (D + Dv) + H]
+    x = rnd(n, at[-1] + H + R).to(dtype)
+    inv = 10000.0 ** (-torch.arange(rot // 2) / max(1, rot // 2))
+    S0, N0, M0, nw = rnd(n, H, D, Dv), rnd(n, H, D), rnd(n, H), (1 + 0.1 * rnd(H * Dv)).to(dtype)
+    a2t, a2b = rnd(R, H * D), rnd(H * D)
+
+    def run(dev):
+        spec = ls.ScanSpec(H, D, Dv, mode, cap=15.0, kscale=D ** -0.5, qscale=1.5, eps=1e-5,
+                           rot_dims=rot, rot_half=rot != 12, inv_freq=inv.to(dev), out_scale=0.7,
+                           decay=torch.linspace(0.999, 0.2, H).to(dev), a2t=a2t.to(dev),
+                           a2b=a2b.to(dev), tau=2.0)
+        st = ls.ScanState(*(t.clone().to(dev) if i == 0 or mode == "exp_gates" else None
+                            for i, t in enumerate((S0, N0, M0))))
+        y = ls.linear_scan(x.to(dev), at[0], at[1], at[2], at[3], spec, st, slots.to(dev), None, n,
+                           pos.to(dev), lens.to(dev), nw.to(dev), at[4], at[5], lo_off=at[5] + H)
+        return y.cpu(), st
+
+    (y, a), (z, b) = run("cpu"), run("cuda")
+    live = (slots >= 0) & (lens > 0)
+    # fp32 sums over at most 128 products; bf16 adds one rounding and at times one step more
+    assert _rel(z[live], y[live]) < (1e-5 if dtype == torch.float32 else 4e-3)
+    for u, v in ((a.S, b.S), (a.n, b.n), (a.m, b.m)):
+        if u is not None:                  # (a padding row leaves its slot alone on the GPU)
+            kept = slots[live].long()
+            assert _rel(v.cpu()[kept], u[kept]) < 2e-6
+            if dtype == torch.float32 and u is a.S:
+                assert torch.equal(v.cpu()[4], S0[4])

@@ -82,7 +82,7 @@ struct WkvArgs {
 // recurrence runs TC steps on LDS broadcasts leaving four partial outputs per token and column,
 // and the partials are then summed, RMS-normed per head, weighted and gated -- so a token costs
 // a quarter pass over dk per thread instead of a global-memory round trip.
-template <typename T, int DMAX>
+template <typename T, int DMAX, bool SPLIT>
 __global__ void __launch_bounds__(4 * (DMAX < 64 ? 64 : DMAX))
 wkv_scan_kernel(WkvArgs a) {
   constexpr int DP = DMAX < 64 ? 64 : DMAX;          // threads per quarter
@@ -97,7 +97,7 @@ wkv_scan_kernel(WkvArgs a) {
   const int slot = a.slots[s];
   if (slot < 0 || (a.seq_lens && a.seq_lens[s] <= 0)) return;
   const int lo = a.cu ? a.cu[s] : s, hi = a.cu ? a.cu[s + 1] : s + 1;
-  if (hi <= lo || (a.split && hi - lo >= a.split)) return;
+  if (hi <= lo || (SPLIT && hi - lo >= a.split)) return;
   const bool fresh = a.positions[lo] == 0;
   const bool live = j < D, mine = j < DMAX;
   float* Sg = a.S + ((long)slot * a.H + h) * D * D;
@@ -202,7 +202,11 @@ EIA_API int eia_wkv_scan(const void* r, const void* k, const void* v, const void
             seq_lens, y, ldy, eps, H, D, split};
   dim3 grid(nseq, H);
 #define WKV_LAUNCH(TT, DM)                                                                 \
-  hipLaunchKernelGGL((wkv_scan_kernel<TT, DM>), grid, dim3(4 * (DM < 64 ? 64 : DM)), 0, st, a)
+  do {                                                                                     \
+    const dim3 block(4 * (DM < 64 ? 64 : DM));                                             \
+    if (split) hipLaunchKernelGGL((wkv_scan_kernel<TT, DM, true>), grid, block, 0, st, a); \
+    else hipLaunchKernelGGL((wkv_scan_kernel<TT, DM, false>), grid, block, 0, st, a);      \
+  } while (0)
   if (is_bf16) {
     if (D <= 32) WKV_LAUNCH(bf16_t, 32);
     else if (D <= 64) WKV_LAUNCH(bf16_t, 64);

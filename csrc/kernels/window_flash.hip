@@ -211,8 +211,11 @@ window_flash_kernel(FlashArgs a) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) oacc[dt][i] = 0.f;
   const bool snk = !SIG && a.sink && it0 == 0;
-  float m_run = snk ? a.sink[h * P + map] * FLASH_LOG2E : -1e30f;
-  float l_run = snk && hh == 0 ? 1.f : 0.f;
+  // (never below -1e30: a sink that weighs nothing must not make the maximum -inf, which a tile of
+  // which the lane sees no key would keep, and -inf - -inf is no number)
+  const float sinkl = snk ? a.sink[h * P + map] * FLASH_LOG2E : 0.f;
+  float m_run = snk ? fmaxf(sinkl, -1e30f) : -1e30f;
+  float l_run = snk && hh == 0 ? __builtin_amdgcn_exp2f(sinkl - m_run) : 0.f;
   const float bl = SIG && a.bias ? a.bias[h] * FLASH_LOG2E : 0.f;
   const int krow0 = (r32 & ~12) | ((r32 & 4) << 1) | ((r32 & 8) >> 1);
 

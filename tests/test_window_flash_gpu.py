@@ -26,6 +26,18 @@ def _spec(wa, kind, H, G, D, Dv, window, dev):
     return s
 
 
+def _pages(g, total, bs):
+    """Random pages for sequences of ``total`` tokens: block tables and the page count."""
+    pages = [max(1, -(-n // bs)) for n in total]
+    order = torch.randperm(sum(pages), generator=g).to(torch.int32)
+    bt = torch.zeros(len(total), max(pages), dtype=torch.int32)
+    at = 0
+    for s, n in enumerate(pages):
+        bt[s, :n] = order[at:at + n]
+        at += n
+    return bt, sum(pages)
+
+
 @pytest.mark.parametrize("kind", ["plain", "cap", "sigmoid", "pair", "keep"])
 @pytest.mark.parametrize("H,G,D,Dv,bs", [(4, 1, 128, 128, 64), (6, 3, 72, 48, 128), (3, 1, 64, 64, 64),
                                          (8, 2, 96, 96, 64), (2, 2, 64, 112, 64)])
@@ -120,3 +132,38 @@ def test_window_decode(parts, window, H, G, D, Dv, bs, kind, monkeypatch):
     a, b = run("cpu").double(), run("cuda").double()
     live = torch.tensor(lens) > 0
     assert float((a - b)[live].norm() / a[live].norm()) < 4e-3   # as above
+
+
+@pytest.mark.parametrize("sink", [float("-inf"), torch.finfo(torch.float32).min, -1e31])
+@pytest.mark.parametrize("cap", [0.0, 5.0])
+@pytest.mark.parametrize("window,new,past,cut", [(50, [1, 200, 33, 65], [0, 0, 190, 63], False),
+                                                 (1000, [300, 40], [1500, 900], True)])
+def test_window_flash_heads_without_a_sink(window, new, past, cut, cap, sink):
+    """A sink that weighs nothing beside ones that do, behind a window: a wave's later queries meet
+    tiles of which they see no key, before and between the ones that they do see."""
+    from enterprise_inference_amd.ops import attention as A
+    from enterprise_inference_amd.ops import window_attention as wa
+    H, G, D, bs, bf = 4, 1, 128, 64, torch.bfloat16
+    g = torch.Generator().manual_seed(window)
+    bt, n = _pages(g, [a + b for a, b in zip(new, past)], bs)
+    cu = torch.tensor([0] + new).cumsum(0).to(torch.int32)
+    pos = torch.cat([torch.arange(k) + f for k, f in zip(new, past)]).to(torch.int32)
+    T = int(cu[-1])
+    rnd = lambda *s: torch.randn(*s, generator=g).to(bf)
+    q, k, v = rnd(T, H * D), rnd(n, bs, G * D), rnd(n, G * D, bs)
+
+    def run(dev):
+        md = A.AttentionMetadata(
+            num_decode=0, num_prefill_tokens=T, slot_mapping=pos.to(dev), positions=pos.to(dev),
+            prefill_block_tables=bt.to(dev), prefill_cu_q=cu.to(dev), prefill_q_lens=new)
+        spec = wa.WindowSpec(H, G, 1, D, D, window, 0, mult=torch.full((H,), D ** -0.5).to(dev),
+                             sink=torch.tensor([sink, 0.3, sink, -2.0]).to(dev), cap=cap)
+        if dev == "cuda":
+            qb = wa.query_block(spec, bf, bs)
+            items = sum(-(-a // qb) for a in new)
+            assert (wa.flash_parts(items, spec, qb, max(new), bt.shape[1] * bs)[0] > 1) == cut
+        return wa.window_attention(q.to(dev), k.to(dev), v.to(dev), md, spec, None).cpu()
+
+    a, b = run("cpu").double(), run("cuda").double()
+    assert torch.isfinite(b).all()
+    assert float((a - b).norm() / a.norm()) < 4e-3           # one bf16 rounding (2^-9) on each side

@@ -127,6 +127,7 @@ def wkv_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor,
         n = T // CHUNK + nseq
         U = torch.empty(n, heads, CHUNK_DIM, CHUNK_DIM, dtype=torch.float32, device=r.device)
         L = torch.empty(n, heads, CHUNK_DIM, dtype=torch.float32, device=r.device)
-        check(lib().eia_wkv_scan_chunked(*args, T, heads, D, split, ptr(U), ptr(L), 1 if bf else 0,
-                                         stream(r)), "wkv_scan_chunked")
+        # (a single sequence goes here whatever part of the T rows it owns)
+        check(lib().eia_wkv_scan_chunked(*args, T, heads, D, split if nseq > 1 else 1, ptr(U), ptr(L),
+                                         1 if bf else 0, stream(r)), "wkv_scan_chunked")
     return y

@@ -208,3 +208,33 @@ def test_linear_decode_rows(H, D, Dv, rot, mode, dtype):
             assert _rel(v.cpu()[kept], u[kept]) < 2e-6
             if dtype == torch.float32 and u is a.S:
                 assert torch.equal(v.cpu()[4], S0[4])
+
+
+def _wkv_args(g, T, n, H, D, dtype):
+    """Everything that wkv_scan takes before ``slots``; decays from 0.998 a token to about 0.4."""
+    rnd = lambda *s: torch.randn(*s, generator=g)
+    HD = H * D
+    r, k, v, gate = rnd(4, T, HD).mul(0.5).to(dtype)
+    w0, u, nw = torch.linspace(-6.0, -0.1, HD), rnd(HD), 1 + 0.1 * rnd(HD)
+    return [r, k, v, gate, 0.3 * rnd(T, HD), w0.to(dtype), u.to(dtype), nw.to(dtype),
+            rnd(n, H, D, D), rnd(n, 24), rnd(T, 24)]
+
+
+@pytest.mark.parametrize("cu", [[0, 40], [20, 60], [0, 0], [70, 71], [3, 99], [50, 100]])
+def test_wkv_sequence_of_a_wider_step(cu):
+    """One sequence that owns some of the step's rows, on both sides of the length from which
+    sequences are cut into chunks."""
+    from enterprise_inference_amd.ops import wkv
+    H, D, T = 2, 64, 100
+    assert T >= wkv.chunk_rows(1, H) > 40
+    args = _wkv_args(torch.Generator().manual_seed(cu[1]), T, 1, H, D, torch.float32)
+    args += [torch.zeros(1, dtype=torch.int32), torch.tensor(cu, dtype=torch.int32)]
+    pos = (torch.arange(T) + 5 - cu[0]).to(torch.int32)
+    dev = [t.to("cuda") for t in args]
+    y = wkv.wkv_scan(*args, 1, pos, None, 1e-5, H)
+    z = wkv.wkv_scan(*dev, 1, pos.to("cuda"), None, 1e-5, H).cpu()
+    # fp32 sums over at most 64 products and a few exponentials
+    rows = slice(*cu)
+    assert cu[0] == cu[1] or _rel(z[rows], y[rows]) < 1e-5
+    assert _rel(dev[8], args[8]) < 2e-6
+    assert torch.equal(dev[9].cpu(), args[9])

@@ -309,6 +309,15 @@ struct WkvTile {
       }
     }
   }
+  // Whether one of this thread's values is infinite or no number.
+  EIA_DEV bool wild() const {
+    float z = 0.f;
+#pragma unroll
+    for (int x = 0; x < N; ++x)
+#pragma unroll
+      for (int e = 0; e < E; ++e) z += 0.f * (float)v[x][e];
+    return z != 0.f;
+  }
 };
 
 // Base-2 log decays of channel i, tokens t0 .. t0 + 15 (0 past the chunk and past D): a weight then
@@ -450,6 +459,7 @@ __global__ void __launch_bounds__(256, 3)
 wkv_chunk_out_kernel(WkvArgs a, WkvChunkArgs c) {
   __shared__ __align__(16) float sr[WC * WD], sk[WC * WD], sAv[WC * WD];
   __shared__ __align__(16) float se[8][WD], su[WD];    // decays over whole 8-token blocks; u
+  __shared__ int swild;                                // a value of the chunk is not finite
   int s, row0, n;
   if (!wkv_chunk(a, c.nseq, blockIdx.x, s, row0, n)) return;
   const int h = blockIdx.y, lane = threadIdx.x & 63, w = ((threadIdx.x >> 6) + blockIdx.x) & 3;
@@ -475,6 +485,7 @@ wkv_chunk_out_kernel(WkvArgs a, WkvChunkArgs c) {
     se[2 * w + b][lane] = __builtin_amdgcn_exp2f(tot);
   }
   if (w == 0) su[lane] = lane < D ? ld_f32<T>(static_cast<const T*>(a.u), hc + lane) : 0.f;
+  if (threadIdx.x == 0) swild = 0;
   __syncthreads();
   // weights inside the wave's two 8-token blocks: lane = pair s < t, then to the lane that holds
   // them as an operand (query l16, keys 4 g4 + i)
@@ -526,6 +537,7 @@ wkv_chunk_out_kernel(WkvArgs a, WkvChunkArgs c) {
     }
   }
   tv.store(sAv, n, D);
+  if (tv.wild()) swild = 1;
   __syncthreads();
   if (t0 >= n) return;
   f32x4 rt[4], o[4], pq = {0.f, 0.f, 0.f, 0.f};
@@ -539,16 +551,34 @@ wkv_chunk_out_kernel(WkvArgs a, WkvChunkArgs c) {
   }
   // (weights are formed transposed, keys x queries: their registers are the A operand of P v)
   if (l16 >= 8 && g4 < 2) p += pq;                     // second 8 queries, first 8 keys
+  const bool wild = swild;
   for (int b = w;;) {
-    f32x4 vb[4];
+    if (wild && b == w) {
+      // key by key: in the product a later token's value times a weight of zero would be no number
+#pragma unroll 1
+      for (int k4 = 0; k4 < 4; ++k4)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const f32x4 x = wkv_get(sAv, 16 * b + 4 * g4 + e, 4 * l16);
+        for (int e = 0; e < 4; ++e) {
+          const f32x4 x = wkv_get(sAv, t0 + 4 * k4 + e, 4 * l16);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) vb[j][e] = x[j];
+          for (int i = 0; i < 4; ++i) {
+            const float pt = __shfl(p[e], 16 * k4 + 4 * g4 + i, 64);
+            if (4 * k4 + e > 4 * g4 + i) continue;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) o[j][i] += pt * x[j];
+          }
+        }
+    } else {
+      f32x4 vb[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const f32x4 x = wkv_get(sAv, 16 * b + 4 * g4 + e, 4 * l16);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) vb[j][e] = x[j];
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[j] = mfma_f32_k16(p, vb[j], o[j]);
     }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) o[j] = mfma_f32_k16(p, vb[j], o[j]);
     if (--b < 0) break;
     p = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll

@@ -238,3 +238,26 @@ def test_wkv_sequence_of_a_wider_step(cu):
     assert cu[0] == cu[1] or _rel(z[rows], y[rows]) < 1e-5
     assert _rel(dev[8], args[8]) < 2e-6
     assert torch.equal(dev[9].cpu(), args[9])
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+@pytest.mark.parametrize("at", [0, 5, 15, 16, 70, 127, 129])
+def test_wkv_values_that_are_not_finite(at, value):
+    """A value that is no number reaches its own token and later ones, in its own head, only."""
+    from enterprise_inference_amd.ops import wkv
+    H, D, T = 2, 64, 130
+    args = _wkv_args(torch.Generator().manual_seed(at), T, 1, H, D, torch.float32)
+    clean = [t.to("cuda") for t in args]
+    args[2][at, D + 7] = value
+    bad = [t.to("cuda") for t in args]
+    rest = [torch.zeros(1, dtype=torch.int32).cuda(), torch.tensor([0, T], dtype=torch.int32).cuda()]
+    pos = torch.arange(T, dtype=torch.int32).cuda()
+    y = wkv.wkv_scan(*clean, *rest, 1, pos, None, 1e-5, H)
+    z = wkv.wkv_scan(*bad, *rest, 1, pos, None, 1e-5, H)
+    # (the chunk's own sums are taken in another order: 16 fp32 products)
+    assert torch.equal(y[:, :D], z[:, :D]) and (at == 0 or _rel(z[:at], y[:at]) < 1e-6)
+    assert not torch.isfinite(z[at, D + 7]) and torch.isfinite(y).all()
+    S, Z = clean[8][0], bad[8][0]                        # the head's column 7, and nothing else
+    assert not torch.isfinite(Z[1, :, 7]).any()
+    Z[1, :, 7] = S[1, :, 7]
+    assert torch.equal(S, Z)

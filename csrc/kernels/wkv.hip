@@ -234,11 +234,12 @@ EIA_API int eia_wkv_scan(const void* r, const void* k, const void* v, const void
 //   P_ts = sum_channels r_t k_s 2^(sum_(s<x<t) l_x)                    (3) per chunk, in parallel
 //
 // All products are fp32 matrix-core products.  Exponents are formed as sums of the l_x that they
-// cover, never as differences of long running sums, so they are <= 0 and keep their precision; a
-// pair of tokens meets through the edges of the 8-token blocks between them,
+// cover, never as differences, so they are <= 0 and keep their precision behind tokens that forget
+// almost everything; a pair of tokens meets through the edges of the 8-token blocks between them,
 //   P_ts = (r_t 2^(block start .. t)) . (whole blocks between) . (k_s 2^(s .. block end)),
-// and only pairs inside one 8-token block take the difference of a running sum over that block
-// (there a token's l is cut at -40: a weight below 1e-12).
+// inside a block through the edge between its fours, inside a four through the one or two tokens
+// between.  (Differences of a running sum over eight tokens, l cut at -40: 8e-7 instead of 1.2e-7 against
+// 64 bits where every second token forgets, the same time.)
 //
 // Chunks are numbered without a list from the host: sequence s owns the numbers from
 // cu[s] / WC + s on, at least as many as it has chunks; numbers past its last chunk do nothing.
@@ -473,38 +474,66 @@ wkv_chunk_out_kernel(WkvArgs a, WkvChunkArgs c) {
   tv.load(a.v, a.ld, hc, row0, n, D);
   tr.store(sr, n, D);
   tk.store(sk, n, D);
+  // E: l over the rest of a token's four if they are the first of its eight, else from their start on
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
-    float A = 0.f, tot = 0.f;
+    float tot = 0.f;
 #pragma unroll
-    for (int t = 8 * b; t < 8 * b + 8; ++t) {
-      A += fmaxf(l[t], -40.f);
-      tot += l[t];
-      sAv[wkv_at(t0 + t, lane)] = A;
-    }
+    for (int t = 8 * b; t < 8 * b + 8; ++t) tot += l[t];
     se[2 * w + b][lane] = __builtin_amdgcn_exp2f(tot);
+    float suf = 0.f, pre = 0.f;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      sAv[wkv_at(t0 + 8 * b + 3 - t, lane)] = suf;
+      suf += l[8 * b + 3 - t];
+      sAv[wkv_at(t0 + 8 * b + 4 + t, lane)] = pre;
+      pre += l[8 * b + 4 + t];
+    }
   }
   if (w == 0) su[lane] = lane < D ? ld_f32<T>(static_cast<const T*>(a.u), hc + lane) : 0.f;
   if (threadIdx.x == 0) swild = 0;
   __syncthreads();
-  // weights inside the wave's two 8-token blocks: lane = pair s < t, then to the lane that holds
-  // them as an operand (query l16, keys 4 g4 + i)
+  // weights inside the wave's two 8-token blocks: lane = pair s < t and half of the channels, then to
+  // the lane that holds them as an operand (query l16, keys 4 g4 + i)
   f32x4 p = {0.f, 0.f, 0.f, 0.f};
   if (t0 < n) {
-    float v = 0.f;
-    if (lane < 56) {
-      const int x = lane % 28;
-      int t = 1;
-      while (t * (t + 1) / 2 <= x) ++t;
-      const int q = t0 + 8 * (lane / 28), ks = x - t * (t - 1) / 2;
+    const int pr = lane & 31, c0 = lane & 32;
+    float v4 = 0.f, v8 = 0.f;
+    {                                                  // t in the second four of its eight, s in the first
+      const int s8 = t0 + 8 * (pr >> 4) + (pr & 3), t8 = t0 + 8 * (pr >> 4) + 4 + (pr >> 2 & 3);
 #pragma unroll 4
-      for (int i = 0; i < WD; i += 4) {
-        const f32x4 y = wkv_get(sr, q + t, i) * wkv_get(sk, q + ks, i);
-        const f32x4 d = wkv_get(sAv, q + t - 1, i) - wkv_get(sAv, q + ks, i);
+      for (int i = c0; i < c0 + 32; i += 4) {
+        const f32x4 y = wkv_get(sr, t8, i) * wkv_get(sk, s8, i);
+        const f32x4 d = wkv_get(sAv, t8, i) + wkv_get(sAv, s8, i);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v += y[e] * __builtin_amdgcn_exp2f(d[e]);
+        for (int e = 0; e < 4; ++e) v8 += y[e] * __builtin_amdgcn_exp2f(d[e]);
       }
     }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    // E of the wave's fours: l of token 1 in row 0, of token 2 in row 3
+#pragma unroll
+    for (int t = 0; t < 16; t += 4) {
+      sAv[wkv_at(t0 + t, lane)] = l[t + 1];
+      sAv[wkv_at(t0 + t + 3, lane)] = l[t + 2];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (pr < 24) {                                     // s < t in the same four
+      const int x = pr % 6, t = x >= 3 ? 3 : x >= 1 ? 2 : 1, ks = x - t * (t - 1) / 2, q = t0 + 4 * (pr / 6);
+      const bool l1 = ks == 0 && t > 1, l2 = t == 3 && ks < 2;
+#pragma unroll 4
+      for (int i = c0; i < c0 + 32; i += 4) {
+        const f32x4 y = wkv_get(sr, q + t, i) * wkv_get(sk, q + ks, i);
+        const f32x4 d1 = wkv_get(sAv, q, i), d2 = wkv_get(sAv, q + 3, i);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          v4 += y[e] * __builtin_amdgcn_exp2f((l1 ? d1[e] : 0.f) + (l2 ? d2[e] : 0.f));
+      }
+    }
+    v4 += __shfl_xor(v4, 32, 64);
+    v8 += __shfl_xor(v8, 32, 64);
+    const float v = lane < 32 ? v8 : v4;
     float b = 0.f;                                     // r . u . k of token t0 + l16
 #pragma unroll
     for (int i = 0; i < 16; i += 4) {
@@ -515,12 +544,13 @@ wkv_chunk_out_kernel(WkvArgs a, WkvChunkArgs c) {
     }
     b += __shfl_xor(b, 16, 64);
     b += __shfl_xor(b, 32, 64);
-    const int t8 = l16 & 7;
+    const int f4 = l16 >> 2, t4 = l16 & 3;             // the query's four, its place there
+    const int from = g4 == f4 ? 32 + 6 * f4 + (t4 * (t4 - 1) >> 1) : 16 * (f4 >> 1) + 4 * t4;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int ks = 4 * g4 + i;
-      const float x = __shfl(v, 28 * (l16 >> 3) + (t8 * (t8 - 1) >> 1) + (ks & 7), 64);
-      p[i] = ks == l16 ? b : (ks < l16 && ks >> 3 == l16 >> 3) ? x : 0.f;
+      const float x = __shfl(v, from + i, 64);
+      if (g4 == f4) p[i] = i == t4 ? b : i < t4 ? x : 0.f;
+      else p[i] = (f4 & 1) && g4 == f4 - 1 ? x : 0.f;
     }
   }
   __syncthreads();

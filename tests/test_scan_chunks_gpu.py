@@ -261,3 +261,35 @@ def test_wkv_values_that_are_not_finite(at, value):
     assert not torch.isfinite(Z[1, :, 7]).any()
     Z[1, :, 7] = S[1, :, 7]
     assert torch.equal(S, Z)
+
+
+@pytest.mark.parametrize("every", [2, 3, 5])
+def test_wkv_strongly_forgetting_tokens(every):
+    """Channels that some tokens forget almost at once (2^-30 and less) and others keep: weights of
+    the pairs behind such a token stay as exact as fp32 products of the decays."""
+    from enterprise_inference_amd.ops import wkv
+    H, D, T = 2, 64, 128
+    g = torch.Generator().manual_seed(every)
+    args = _wkv_args(g, T, 1, H, D, torch.float32)
+    args[5] = torch.zeros(H * D)
+    dec = torch.full((T, H * D), -6.0) + torch.rand(T, H * D, generator=g)
+    dec[torch.rand(T, H * D, generator=g) < 1 / every] = 3.4
+    args[4] = dec
+    pos = torch.arange(T, dtype=torch.int32)
+    dev = [t.to("cuda") for t in args]
+    z = wkv.wkv_scan(*dev, torch.zeros(1, dtype=torch.int32).cuda(),
+                     torch.tensor([0, T], dtype=torch.int32).cuda(), 1, pos.cuda(), None, 1e-5, H)
+    r, k, v, gate = (t.double().view(T, H, D) for t in args[:4])
+    w = torch.exp(-torch.exp(dec.double())).view(T, H, D)
+    u, nw, S = args[6].double().view(H, D), args[7].double(), torch.zeros(H, D, D, dtype=torch.float64)
+    y = torch.empty(T, H, D, dtype=torch.float64)
+    for t in range(T):
+        kv = k[t][:, :, None] * v[t][:, None]
+        o = ((S + u[:, :, None] * kv) * r[t][:, :, None]).sum(1)
+        S = w[t][:, :, None] * S + kv
+        y[t] = o / torch.sqrt((o * o).mean(-1, keepdim=True) + 1e-5)
+    y = y.flatten(1) * nw * torch.nn.functional.silu(gate.flatten(1))
+    # 2^-23 and less each for the exponent, exp and product of a weight and for the sums: token by token
+    # outputs are 1.4e-7 off; exponents that differ by an ulp of 160, the sum of four such decays, 8e-7
+    assert _rel(z, y) < 3e-7
+    assert _rel(dev[8][0], S) < 3e-7

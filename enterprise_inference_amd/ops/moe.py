@@ -182,14 +182,17 @@ def fused_moe(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, topk_w: torc
     avg = T * k / max(1, El)
     capturable = capturable or torch.cuda.is_current_stream_capturing()
     if act == "silu" and avg <= 96 and _grouped_ok(x, w13, w2) and not (
-            _mfma_pays(avg, El, w13.shape[1] // 2, H) and _mfma_ok(x, w13, w2)):
+            _mfma_pays(avg, El, w13.shape[1] // 2, H) and _mfma_ok(x, w13, w2)
+            and _on16(w13, w2)):
         return _fused_moe_grouped(x, w13, w2, topk_w, topk_ids, e_lo, e_hi,
                                   defer_combine=defer_combine)
     # (small experts stay on the grouped MFMA kernel at any row count: their per-expert library
-    # GEMMs are launch- and read-back-bound, not MFMA-bound)
+    # GEMMs are launch- and read-back-bound, not MFMA-bound; stacks that it would have to copy go
+    # there only where no other form can be captured)
     if act == "silu" and _mfma_ok(x, w13, w2) and (
             avg <= GROUPED_MAX_ROWS or capturable
-            or (w13.shape[1] // 2) * H <= UNGATED_SMALL_EXPERT):
+            or (w13.shape[1] // 2) * H <= UNGATED_SMALL_EXPERT) and (
+            _on16(w13, w2) or (capturable and not _grouped_ok(x, w13, w2))):
         return _fused_moe_grouped(x, w13, w2, topk_w, topk_ids, e_lo, e_hi, mfma=True)
     if capturable:
         if act == "silu" and _grouped_ok(x, w13, w2):
@@ -225,9 +228,13 @@ def _mfma_ok(x, w13, w2) -> bool:
             and x.stride(0) % 8 == 0)
 
 
-def _aligned16(t):
+def _on16(*ts) -> bool:
     """The MFMA grouped GEMM's operands go straight to LDS, 16 bytes at a time."""
-    return t if t.data_ptr() % 16 == 0 else t.clone()
+    return all(t.data_ptr() % 16 == 0 for t in ts)
+
+
+def _aligned16(t):
+    return t if _on16(t) else t.clone()
 
 
 def _fused_moe_grouped(x, w13, w2, topk_w, topk_ids, e_lo, e_hi, mfma: bool = False,
@@ -491,7 +498,8 @@ def ungated_moe(x: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor, topk_
                                     ptr(out), out.stride(0), st), "moe_combine")
         return out
     if bf and H % 128 == 0 and I % 128 == 0 and UNGATED_GROUPED and (
-            avg <= MFMA_MAX_ROWS or capturing or I * H <= UNGATED_SMALL_EXPERT):
+            avg <= MFMA_MAX_ROWS or capturing or I * H <= UNGATED_SMALL_EXPERT) and (
+            _on16(w_up, w_down) or capturing):
         h1 = torch.empty(max(1, n), I, dtype=x.dtype, device=dev)
         h2 = torch.empty(max(1, n), H, dtype=x.dtype, device=dev)
         x, w_up, w_down = _aligned16(x), _aligned16(w_up), _aligned16(w_down)

@@ -190,7 +190,7 @@ def fused_moe(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, topk_w: torc
     # GEMMs are launch- and read-back-bound, not MFMA-bound; stacks that it would have to copy go
     # there only where no other form can be captured)
     if act == "silu" and _mfma_ok(x, w13, w2) and (
-            avg <= GROUPED_MAX_ROWS or capturable
+            avg <= _grouped_max_rows(w13.shape[1] // 2, H) or capturable
             or (w13.shape[1] // 2) * H <= UNGATED_SMALL_EXPERT) and (
             _on16(w13, w2) or (capturable and not _grouped_ok(x, w13, w2))):
         return _fused_moe_grouped(x, w13, w2, topk_w, topk_ids, e_lo, e_hi, mfma=True)
@@ -206,19 +206,45 @@ def fused_moe(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, topk_w: torc
 
 
 # rows per expert above which the per-expert hipBLASLt GEMMs win: ungated experts, and SwiGLU ones
-# (Mixtral-8x7B, grouped against per expert: 256 rows 1149 / 1256 us, 512 rows 1822 / 1839 us)
 MFMA_MAX_ROWS = 128
 GROUPED_MAX_ROWS = 384
 
 
+def _grouped_max_rows(I: int, H: int) -> int:
+    """us, grouped / per expert with its read-back, at 256 and 384 rows per expert: 8 experts of 4096 x
+    14336 1086 / 1226, 1489 / 1478; 16 of 5120 x 8192 1532 / 1832, 2090 / 2271; 16 of 2048 x 4096 345 /
+    946, 442 / 955; only of 6144 x 16384, 1819 / 1967 and 2577 / 2293, the library wins before 384."""
+    return GROUPED_MAX_ROWS if I * H < 1 << 26 else 256
+
+
 def _mfma_pays(avg: float, El: int, I: int, H: int) -> bool:
     """Whether the MFMA grouped GEMM beats the weight-streaming skinny one at ``avg`` rows per expert.
-    The skinny kernel goes over the weights once per 16 to 128 rows, the MFMA kernel once per 128.
-    us, skinny / MFMA: 8 experts of 4096 x 14336, 40 rows 546 / 545, 65 rows 672 / 551; 8 of 1024 x
-    512 (64 workgroups: half the chip idles), 50 rows 28.4 / 29.1, 95 rows 40 / 31.  Experts that
-    fill the chip and whose weights stay in the 256 MB cache gain sooner: 16 of 2048 x 1024, 25 rows
-    56 / 45, 50 rows 73 / 46."""
-    return avg > 48 or (avg > 24 and El * (I // 64) >= 256 and 6 * El * I * H <= 1 << 28)
+    The skinny kernel goes over the weights once per 16 to 128 rows, with more columns in flight from 49
+    and from 73 rows on; the MFMA kernel once per 128, but its down projection has only El * H / 128
+    tiles, each of I / 64 steps in a row: a few long ones leave the chip idle.
+    us, skinny / MFMA (MI355X), tiles of the down projection in brackets:
+      49, 56, 64 rows: 8 of 4096 x 14336 [256] 556 / 541, -, 655 / 555; 8 of 3072 x 8192 [192] 268 / 260,
+      281 / 260, 309 / 262; 8 of 2048 x 3072 [128] 92 / 83, 100 / 84, 109 / 86; but 8 of 2048 x 4096 [128]
+      104 / 124, 111 / 124, 121 / 125; 8 of 1024 x 2048 [64] 39 / 42, 42 / 43, 45 / 44; 8 of 4096 x 4096
+      [256] 187 / 203, 202 / 203, 224 / 206;
+      (49 only with short rows of tiles, 16 of 4096 x 1024 [512] 140 / 92, or long streams of weights, 8
+      of 4096 x 7168 [256] 321 / 276;)
+      with packed weights and the next add + norm, which takes the skinny form's combine along, 8 of 4096 x
+      14336 537 / 538, 577 / 543, 633 / 548;
+      80 rows: 8 of 2048 x 4096 145 / 126, 4 of 2048 x 4096 [64] 76 / 72; but 2 of 4096 x 8192 [64] 126 /
+      153, 8 of 512 x 4096 [32] 62 / 64.
+    Experts that fill the chip and whose weights stay in the 256 MB cache gain sooner, at 25 and 32 rows:
+    16 of 2048 x 1024 [256] 55 / 44, 65 / 44; 32 of 1024 x 1024 [256] 60 / 43, 68 / 45; 16 of 1024 x 2048
+    [128] 55 / 50, 59 / 52; 8 of 2048 x 2048 [128] 52 / 51, 56 / 52; but 8 of 1024 x 4096 [64] 52 / 67, 54 /
+    68; 8 of 1024 x 2048 [64] 33 / 41, 36 / 43."""
+    down = El * H // 128
+    if avg > 72:
+        return I < 128 * down
+    if avg > 52:
+        return down >= 192 or I <= 24 * down
+    if avg > 48 and down >= 192 and (I <= 1024 or 6 * El * I * H > 1 << 30):
+        return True
+    return avg > 24 and down >= 128 and El * (I // 64) >= 256 and 6 * El * I * H <= 1 << 28
 
 
 def _mfma_ok(x, w13, w2) -> bool:

@@ -106,3 +106,18 @@ def test_grouped_moe_cfgs():
     assert moe_cfgs(100, 100) == (1, 0)
     assert moe_cfgs(14336, 4096, 7, 6) == (3, 2)
     assert moe_cfgs(14336, 4096, 1, 0) == (1, 0)
+
+
+@pytest.mark.parametrize("El,H,I,avg,mfma", [
+    # the faster form where the two were measured more than 5 % apart
+    (8, 4096, 14336, 25, False), (8, 4096, 14336, 64, True), (8, 4096, 7168, 49, True),
+    (16, 2048, 1024, 25, True), (8, 1024, 512, 95, True), (16, 4096, 1024, 49, True),
+    (8, 2048, 4096, 49, False), (8, 2048, 4096, 56, False), (8, 2048, 4096, 80, True),
+    (8, 512, 4096, 25, False), (8, 512, 4096, 64, False), (4, 2048, 4096, 32, False),
+    (4, 2048, 4096, 72, False), (8, 1024, 2048, 32, False), (8, 1024, 2048, 80, True),
+    (2, 4096, 8192, 95, False), (8, 2048, 8192, 56, False), (8, 4096, 4096, 49, False),
+    (8, 3072, 8192, 64, True), (64, 1024, 512, 32, True), (16, 1024, 2048, 32, True)])
+def test_grouped_moe_rule(El, H, I, avg, mfma):
+    """Which grouped GEMM a batch of ``avg`` rows per expert takes."""
+    from enterprise_inference_amd.ops.moe import _mfma_pays
+    assert _mfma_pays(avg, El, I, H) == mfma

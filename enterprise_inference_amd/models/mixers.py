@@ -247,7 +247,7 @@ class WKVMixer(nn.Module):
                              self.norm, state.S, state.prev, x, md.seq_slots, md.seq_cu,
                              md.num_seqs, md.positions,
                              md.decode_seq_lens if md.seq_cu is None else None, self.eps,
-                             self.heads)
+                             self.heads, max(md.prefill_q_lens or [0]))
         return gemm.linear(y, self.o)
 
 

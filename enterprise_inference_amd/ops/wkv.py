@@ -31,6 +31,19 @@ def chunk_rows(nseq: int, heads: int) -> int:
     return 48 + min(64, nseq * heads // 32)
 
 
+def takes_chunks(rows: int, nseq: int, split: int, longest: int = 0) -> bool:
+    """Whether the chunk-parallel form is launched beside the token-by-token one, each of which takes
+    its own sequences.  Where the caller does not know the ``longest`` sequence's rows, only the device
+    does: the three launches cost 10 to 13 us when they take nothing (MI355X, 32 heads, without / with
+    them: 8 x 24 rows 18 / 28 us, 64 x 48 82 / 95), a long sequence left to the other form 0.5 us a row
+    (16 sequences, one of 160 rows 93 / 45, of 256 146 / 47).  So they are made where rows enough for a
+    long sequence are there and it is likely -- 24 rows a sequence: 16 sequences of 20 but one of 96 take
+    57 / 51 -- or would cost some fifty us if it were one, 160 rows beside one for every sequence."""
+    if split <= 0 or longest:
+        return 0 < split <= longest
+    return rows - nseq + 1 >= split and (rows >= 24 * nseq or rows - nseq >= 160)
+
+
 def _seq_bounds(cu: Optional[torch.Tensor], nseq: int):
     if cu is None:
         return [(s, s + 1) for s in range(nseq)]
@@ -71,12 +84,14 @@ def wkv_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor,
              dec: torch.Tensor, w0: torch.Tensor, u: torch.Tensor, norm_w: torch.Tensor,
              S: torch.Tensor, prev_state: torch.Tensor, x: torch.Tensor, slots: torch.Tensor,
              cu: Optional[torch.Tensor], nseq: int, positions: torch.Tensor,
-             seq_lens: Optional[torch.Tensor], eps: float, heads: int) -> torch.Tensor:
+             seq_lens: Optional[torch.Tensor], eps: float, heads: int,
+             longest: int = 0) -> torch.Tensor:
     """r, k, v, g [T, H*D] (same row stride), dec fp32 [T, H*D] (decay pre-activation without
     w0) -> y [T, H*D].  Per head and token, in fp32:
         w = exp(-exp(dec + w0));  o = (S + diag(u) k v^T)^T r;  S <- diag(w) S + k v^T
         y = o / rms(o) * norm_w * silu(g)
-    S is read from / written to the sequence's slot; prev_state[slot] <- x[last row]."""
+    S is read from / written to the sequence's slot; prev_state[slot] <- x[last row].
+    ``longest``: rows of the longest sequence, where they are known on the host."""
     T, HD = r.shape
     D = HD // heads
     if not use_hip(r):
@@ -115,11 +130,8 @@ def wkv_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor,
     args = (ptr(r), ptr(k), ptr(v), ptr(g), ld, ptr(dec), dec.stride(0), ptr(w0), ptr(u),
             ptr(norm_w), ptr(S), ptr(prev_state), ptr(x), x.shape[1], ptr(slots), ptr(cu),
             ptr(positions), ptr(seq_lens), ptr(y), y.stride(0), float(eps), nseq)
-    # Only the device knows the sequences' lengths: both forms are launched where a long sequence is
-    # likely, and each takes its own ones.  (The three more launches are 15 us of host time: a step
-    # of 16 x 8 rows that made them for nothing took 30 us instead of 15.)
     split = chunk_rows(nseq, heads) if cu is not None and D <= CHUNK_DIM else 0
-    if T - nseq + 1 < split or not (T >= 24 * nseq or T - nseq >= 160):
+    if not takes_chunks(T, nseq, split, longest):
         split = 0
     if nseq > 1 or not split:
         check(lib().eia_wkv_scan(*args, heads, D, split, 1 if bf else 0, stream(r)), "wkv_scan")

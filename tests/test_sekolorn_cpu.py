@@ -76,3 +76,14 @@ def test_config_reader(tmp_path):
     assert mc.architecture == "Sekolorn" and mc.hidden_size == 48 and mc.vocab_size == 70
     assert mc.extra["layers"][1]["mixer"]["decay_rank"] == 6
     assert mc.num_hidden_layers == 2 and mc.layer_norm_eps == 1e-6
+
+
+@pytest.mark.parametrize("rows,nseq,longest,chunks", [
+    (192, 8, 24, False), (3072, 64, 48, False), (4096, 1, 4096, True), (175, 16, 160, True),
+    (48, 1, 48, False), (49, 1, 49, True),
+    # lengths unknown on the host
+    (64, 8, 0, False), (256, 8, 0, True), (4096, 1, 0, True), (64, 64, 0, False), (224, 64, 0, True)])
+def test_wkv_chunk_launches(rows, nseq, longest, chunks):
+    """Which steps of 32 heads launch the chunk-parallel form: no short prompts whose lengths are known."""
+    from enterprise_inference_amd.ops import wkv
+    assert wkv.takes_chunks(rows, nseq, wkv.chunk_rows(nseq, 32), longest) == chunks

@@ -1008,8 +1008,15 @@ window_decode_kernel(const WinAttnArgs a) {
     for (int t = 0; t < NDV; ++t)
       o.v[t] = *reinterpret_cast<const bf16x8*>(vp + (long)(t < ndv ? t : 0) * 16 * bs);
   };
-  auto block = [&](int b, const Ops& o) {
+  auto block = [&](int b, Ops& o) {
     const int key0 = (b < nsink ? b : wb0 + b - nsink) << 5;
+    if (key0 + 31 > qpos) {                 // (slots behind the last key may hold anything: 0 x inf)
+#pragma unroll
+      for (int t = 0; t < NDV; ++t)
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (key0 + 8 * g + e > qpos) o.v[t][e] = (bf16_t)0.f;
+    }
     bool vis[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {

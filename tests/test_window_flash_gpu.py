@@ -167,3 +167,34 @@ def test_window_flash_heads_without_a_sink(window, new, past, cut, cap, sink):
     a, b = run("cpu").double(), run("cuda").double()
     assert torch.isfinite(b).all()
     assert float((a - b).norm() / a.norm()) < 4e-3           # one bf16 rounding (2^-9) on each side
+
+
+@pytest.mark.parametrize("kind", ["plain", "cap", "sigmoid", "pair"])
+@pytest.mark.parametrize("D,Dv,bs", [(128, 128, 64), (72, 48, 32), (64, 112, 128)])
+@pytest.mark.parametrize("parts", [1, 3])
+def test_window_decode_slots_behind(parts, D, Dv, bs, kind, monkeypatch):
+    """Cache slots behind a row's context hold anything: nothing of them reaches its output."""
+    from enterprise_inference_amd.ops import attention as A
+    from enterprise_inference_amd.ops import window_attention as wa
+    monkeypatch.setenv("EIA_WINDOW_DECODE_P", str(parts))
+    H, G, P, bf = 6, 2, 2 if kind == "pair" else 1, torch.bfloat16
+    D = min(D, 64) if kind == "pair" else D
+    g = torch.Generator().manual_seed(D + bs)
+    lens = [1, 31, 33, 257, 700]
+    bt, n = _pages(g, lens, bs)
+    pos = torch.tensor(lens, dtype=torch.int32) - 1
+    rnd = lambda *s: torch.randn(*s, generator=g).to(bf)
+    q, k, v = rnd(len(lens), H * P * D), rnd(n, bs, G * P * D), rnd(n, G * Dv, bs)
+    for s, m in enumerate(lens):
+        last, used = int(bt[s, -(-m // bs) - 1]), (m - 1) % bs + 1
+        k[last, used:], v[last, :, used:] = float("nan"), float("nan")
+
+    def run(dev):
+        md = A.AttentionMetadata(
+            num_decode=len(lens), num_prefill_tokens=0, slot_mapping=pos.to(dev),
+            positions=pos.to(dev), decode_block_tables=bt.to(dev), decode_seq_lens=(pos + 1).to(dev))
+        return wa.window_attention(q.to(dev), k.to(dev), v.to(dev), md,
+                                   _spec(wa, kind, H, G, D, Dv, 300, dev), None).cpu()
+
+    a, b = run("cpu").double(), run("cuda").double()
+    assert float((a - b).norm() / a.norm()) < 4e-3           # one bf16 rounding (2^-9) on each side

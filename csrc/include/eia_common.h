@@ -83,3 +83,19 @@ EIA_DEV f32x4 mfma_f32_k16(f32x4 a, f32x4 b, f32x4 c) {
   for (int i = 0; i < 4; ++i) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[i], c, 0, 0, 0);
   return c;
 }
+
+// Stands between matrix products and a branch behind which their results are read by other than a
+// matrix product.  Such a read needs up to 12 wait states after the product (32x32x16 bf16; 10 after
+// 16x16x4 fp32, 8 after 16x16x32 bf16), which nothing but the instruction stream provides; the compiler
+// counts them inside a block but has left out half of them where one way round a branch was short.
+// So the wait covers all of it by itself, whatever the code around it becomes.
+// All results are operands of the one statement: products of an accumulator that were not could be moved
+// behind it.
+template <typename V> EIA_DEV void mfma_settle(V& a, V& b) { asm volatile("s_nop 11" : "+v"(a), "+v"(b)); }
+template <typename V> EIA_DEV void mfma_settle(V (&o)[4]) {
+  asm volatile("s_nop 11" : "+v"(o[0]), "+v"(o[1]), "+v"(o[2]), "+v"(o[3]));
+}
+template <typename V> EIA_DEV void mfma_settle(V (&o)[8]) {
+  asm volatile("s_nop 11" : "+v"(o[0]), "+v"(o[1]), "+v"(o[2]), "+v"(o[3]), "+v"(o[4]), "+v"(o[5]),
+               "+v"(o[6]), "+v"(o[7]));
+}

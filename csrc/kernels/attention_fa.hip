@@ -176,8 +176,7 @@ paged_prefill_fa_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __r
     }
     // element i of half sh is key kb + 32 sh + 16 (i >> 3) + 8 h + (i & 7)
     const bool whole = !window && kb + FKB <= L && (!causal || kb + FKB - 1 <= ctx + wq0);
-    // the branch must not carry a reader of the last product past the wait states it needs
-    asm volatile("s_nop 5" : "+v"(sacc[1]));
+    mfma_settle(sacc[0], sacc[1]);
     if (!whole) {
       // key kp is visible iff q_lo <= kp <= kmax: one unsigned compare per score, no branches
       const int kmax = causal ? min(L - 1, qa) : L - 1;

@@ -1780,6 +1780,7 @@ gl_out_kernel(ScanArgs a, KChunkArgs c) {
         for (int j = 0; j < 4; ++j) o[4 * z + j] = mfma_f32_k16(rt[x], sb[j], o[4 * z + j]);
       }
   }
+  mfma_settle(o);
   const T* X = static_cast<const T*>(a.x);
   const T* NW = static_cast<const T*>(a.norm_w);
   T* Y = static_cast<T*>(a.y);

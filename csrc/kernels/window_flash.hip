@@ -230,6 +230,7 @@ window_flash_kernel(FlashArgs a) {
         const bf16x8 kf = *reinterpret_cast<const bf16x8*>(kf0 + 32 * KS * sh + 16 * t);
         sacc[sh] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[t], t == 0 ? f32x16_t{} : sacc[sh], 0, 0, 0);
       }
+    mfma_settle(sacc[0], sacc[1]);
     // element i of half sh is key kb + 32 sh + 16 (i >> 3) + 8 hh + (i & 7)
     if (a.cap > 0.f) {                      // cap tanh(s / cap) = cap - 2 cap / (exp(2 s / cap) + 1)
 #pragma unroll

@@ -636,6 +636,7 @@ wkv_chunk_out_kernel(WkvArgs a, WkvChunkArgs c) {
       for (int j = 0; j < 4; ++j) o[j] = mfma_f32_k16(rt[x], sb[j], o[j]);
     }
   }
+  mfma_settle(o);
   const T* G = static_cast<const T*>(a.g);
   const T* NW = static_cast<const T*>(a.norm_w);
   T* Y = static_cast<T*>(a.y);

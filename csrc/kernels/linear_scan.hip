@@ -27,7 +27,7 @@
 // Batch layout: sequence s owns rows [cu[s], cu[s+1]) (cu == nullptr: row s).
 #include <type_traits>
 
-#include "eia_common.h"
+#include "eia_chunks.h"
 
 struct ScanArgs {
   const void* x; long ld;                   // fused rows [rows, *]
@@ -436,8 +436,7 @@ EIA_API int eia_linear_scan(const void* x, long ld, int q_off, int k_off, int v_
 // run over 16-token blocks and over whole blocks; only inside one block is a sum the difference of
 // two running sums, so every exponent is <= 0 and keeps its precision.  The log gates of mode 1 come
 // from a pre-pass that carries the running maximum, angles of rotated heads from a table.
-// Chunks are numbered without a list from the host: sequence s owns the numbers from
-// cu[s] / LK + s on, at least as many as it has chunks; numbers past its last chunk do nothing.
+// Chunks are found on the device (eia_chunks.h).
 //
 // Products are fp32 matrix-core products, except q . k of unrotated bf16 rows, which is exact in
 // bf16 operands.  128-token chunks: the states between chunks are the larger part of the memory
@@ -450,7 +449,6 @@ EIA_API int eia_linear_scan(const void* x, long ld, int q_off, int k_off, int v_
 // The 64 KB state goes through the LDS that the keys and values take after it: read by every wave for
 // itself (3) took 122 us.
 constexpr int LK = 128;                     // tokens per chunk
-constexpr int LS_AHEAD = 8;                 // chunks whose contributions are in flight in (2)
 constexpr float LS_LOG2E = 1.4426950408889634f;
 
 struct KChunkArgs {
@@ -463,16 +461,7 @@ struct KChunkArgs {
 
 // The chunk of number x; false where there is none or the sequence is skipped.
 EIA_DEV bool ls_chunk(const ScanArgs& a, int nseq, int x, int& s, int& row0, int& n) {
-  int lo = 0, hi = nseq - 1;                // largest s with cu[s] / LK + s <= x
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (a.cu[mid] / LK + mid <= x) lo = mid; else hi = mid - 1;
-  }
-  s = lo;
-  if (x < a.cu[s] / LK + s) return false;   // (rows before the first sequence)
-  row0 = a.cu[s] + (x - a.cu[s] / LK - s) * LK;
-  n = min(LK, a.cu[s + 1] - row0);
-  return n > 0 && a.slots[s] >= 0;
+  return chunk_of<LK>(a.cu, nseq, x, s, row0, n) && a.slots[s] >= 0;
 }
 
 // (A) log gates of mode 1: one workgroup per (sequence, head).  The running maximum m_t =
@@ -603,12 +592,10 @@ EIA_DEV void ls_head8(const ScanArgs& a, const KChunkArgs& c, long row, long off
   }
 }
 
-// Places in LDS tiles [tokens][MX]: the 16-byte units of a row are turned by the token, so that
-// sixteen tokens' units of one channel group, or four tokens' runs of sixteen channels, lie on
-// different banks.  ls_at: fp32 rows; ls_kat: the key rows of (3), units of 16 / sizeof(KT) entries.
-template <int MX> EIA_DEV int ls_at(int t, int i) { return t * MX + (i ^ ((t & 15) << 2)); }
+// Places in LDS tiles [tokens][MX] where four tokens' runs of sixteen channels meet: the key rows of (3),
+// in units of 16 / sizeof(KT) entries; fp32 rows lie as tile_at has them.
 template <int MX, typename KT> EIA_DEV int ls_kat(int t, int i) {
-  if constexpr (sizeof(KT) == 4) return ls_at<MX>(t, i);
+  if constexpr (sizeof(KT) == 4) return tile_at<MX>(t, i);
   else return t * MX + (i ^ (MX == 128 ? (t & 15) << 3 : ((t >> 1) & 7) << 3));
 }
 // value rows: four tokens' runs meet as rows 4 g + e
@@ -706,7 +693,7 @@ ls_chunk_state_kernel(ScanArgs a, KChunkArgs c) {
       const float wt = a.kscale * __builtin_amdgcn_exp2f(e);
 #pragma unroll
       for (int x = 0; x < 8; x += 4)
-        *reinterpret_cast<f32x4*>(sk + ls_at<MX>(t, i + x)) =
+        *reinterpret_cast<f32x4*>(sk + tile_at<MX>(t, i + x)) =
             tk < n ? f32x4{v[x], v[x + 1], v[x + 2], v[x + 3]} * wt : f32x4{0.f, 0.f, 0.f, 0.f};
     }
     __syncthreads();
@@ -718,7 +705,7 @@ ls_chunk_state_kernel(ScanArgs a, KChunkArgs c) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int t = 16 * b + 4 * g4 + e;
-        ka[e] = sk[ls_at<MX>(t, 16 * w + l16)];
+        ka[e] = sk[tile_at<MX>(t, 16 * w + l16)];
 #pragma unroll
         for (int x = 0; x < MX / 64; ++x) {
           const f32x4 v = ls_v4<T>(sv + ls_vat<MX>(t, 64 * x + 4 * l16));
@@ -755,9 +742,7 @@ ls_chunk_state_kernel(ScanArgs a, KChunkArgs c) {
   }
 }
 
-// (2) Four columns of a state row per thread: U of a chunk turns into the state before it; the slot
-// receives the state after the last one.  A group's contributions are requested while the previous
-// group is summed.
+// (2) Four columns of a state row per thread; the slot receives the state after the last chunk.
 __global__ void __launch_bounds__(256)
 ls_chunk_scan_kernel(ScanArgs a, KChunkArgs c) {
   const int s = blockIdx.x, h = blockIdx.y;
@@ -780,34 +765,7 @@ ls_chunk_scan_kernel(ScanArgs a, KChunkArgs c) {
   const long us = (long)a.H * c.DP * c.UW;
   float* U = c.U + (x0 * a.H + h) * c.DP * c.UW + (long)i * c.UW + j;
   const float* G = c.G + x0 * a.H + h;
-  f32x4 u[LS_AHEAD];
-  float d[LS_AHEAD];
-  auto fetch = [&](int b, f32x4 (&u)[LS_AHEAD], float (&d)[LS_AHEAD]) {
-#pragma unroll
-    for (int k = 0; k < LS_AHEAD; ++k) {
-      const int x = min(b + k, nc - 1);
-      u[k] = *reinterpret_cast<const f32x4*>(U + x * us);
-      d[k] = G[(long)x * a.H];
-    }
-  };
-  fetch(0, u, d);
-  for (int b = 0; b < nc; b += LS_AHEAD) {
-    f32x4 un[LS_AHEAD];
-    float dn[LS_AHEAD];
-    fetch(b + LS_AHEAD, un, dn);
-#pragma unroll
-    for (int k = 0; k < LS_AHEAD; ++k) {
-      if (b + k < nc) {
-        *reinterpret_cast<f32x4*>(U + (b + k) * us) = S;
-        S = S * __builtin_amdgcn_exp2f(d[k]) + u[k];
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < LS_AHEAD; ++k) {
-      u[k] = un[k];
-      d[k] = dn[k];
-    }
-  }
+  chunk_walk(U, us, G, a.H, nc, S);
   if (i < a.D) {
 #pragma unroll
     for (int k = 0; k < 4; ++k)
@@ -1399,22 +1357,7 @@ constexpr int GC = 64;                      // tokens per chunk
 constexpr int GD = 64;                      // widest key head
 
 EIA_DEV bool gl_chunk(const ScanArgs& a, int nseq, int x, int& s, int& row0, int& n) {
-  int lo = 0, hi = nseq - 1;                // largest s with cu[s] / GC + s <= x
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (a.cu[mid] / GC + mid <= x) lo = mid; else hi = mid - 1;
-  }
-  s = lo;
-  if (x < a.cu[s] / GC + s) return false;   // (rows before the first sequence)
-  row0 = a.cu[s] + (x - a.cu[s] / GC - s) * GC;
-  n = min(GC, a.cu[s + 1] - row0);
-  return n > 0 && a.slots[s] >= 0;
-}
-
-// Place of (token, channel) in an fp32 tile [GC][W]: units of four channels turned by the token.
-template <int W> EIA_DEV int gl_at(int t, int i) { return t * W + (i ^ ((t & 15) << 2)); }
-template <int W> EIA_DEV f32x4 gl_get(const float* tile, int t, int i) {
-  return *reinterpret_cast<const f32x4*>(tile + gl_at<W>(t, i));
+  return chunk_of<GC>(a.cu, nseq, x, s, row0, n) && a.slots[s] >= 0;
 }
 
 // l of all rows: thread = channel of one head and 16 rows.
@@ -1480,7 +1423,7 @@ struct GlTile {
       const int u = threadIdx.x + 256 * x, t = u >> 3, i = 8 * (u & 7);
 #pragma unroll
       for (int e = 0; e < 8; e += 4)
-        *reinterpret_cast<f32x4*>(tile + gl_at<GD>(t, i + e)) =
+        *reinterpret_cast<f32x4*>(tile + tile_at<GD>(t, i + e)) =
             t < n ? f32x4{v[x][e], v[x][e + 1], v[x][e + 2], v[x][e + 3]} * scale
                   : f32x4{0.f, 0.f, 0.f, 0.f};
     }
@@ -1510,11 +1453,11 @@ struct GlValues {
       if constexpr (VEC) {
 #pragma unroll
         for (int e = 0; e < E; e += 4)
-          *reinterpret_cast<f32x4*>(tile + gl_at<W>(t, i + e)) =
+          *reinterpret_cast<f32x4*>(tile + tile_at<W>(t, i + e)) =
               ok ? f32x4{(float)v[x][e], (float)v[x][e + 1], (float)v[x][e + 2], (float)v[x][e + 3]}
                  : f32x4{0.f, 0.f, 0.f, 0.f};
       } else {
-        tile[gl_at<W>(t, i)] = ok ? (float)v[x][0] : 0.f;
+        tile[tile_at<W>(t, i)] = ok ? (float)v[x][0] : 0.f;
       }
     }
   }
@@ -1549,7 +1492,7 @@ gl_state_kernel(ScanArgs a, KChunkArgs c) {
   for (int b = 3; b > w; --b) after += stot[b][lane];
 #pragma unroll
   for (int t = 15; t >= 0; --t) {
-    sk[gl_at<GD>(16 * w + t, lane)] *= __builtin_amdgcn_exp2f(after);
+    sk[tile_at<GD>(16 * w + t, lane)] *= __builtin_amdgcn_exp2f(after);
     after += l[t];
   }
   const long at = (long)blockIdx.x * a.H + h;
@@ -1565,10 +1508,10 @@ gl_state_kernel(ScanArgs a, KChunkArgs c) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int t = 16 * b + 4 * g4 + e;
-      ka[e] = sk[gl_at<GD>(t, 16 * w + l16)];
+      ka[e] = sk[tile_at<GD>(t, 16 * w + l16)];
 #pragma unroll
       for (int z = 0; z < NV; ++z) {
-        const f32x4 x = gl_get<W>(sv, t, 64 * z + 4 * l16);
+        const f32x4 x = tile_get<W>(sv, t, 64 * z + 4 * l16);
 #pragma unroll
         for (int j = 0; j < 4; ++j) vb[4 * z + j][e] = x[j];
       }
@@ -1585,9 +1528,7 @@ gl_state_kernel(ScanArgs a, KChunkArgs c) {
           f32x4{acc[4 * z][i], acc[4 * z + 1][i], acc[4 * z + 2][i], acc[4 * z + 3][i]};
 }
 
-// (2) Four columns of a state row per thread: U of a chunk turns into the state before it; the slot
-// receives the state after the last one.  A group's contributions are requested while the previous
-// group is summed.
+// (2) Four columns of a state row per thread; the slot receives the state after the last chunk.
 template <int NV>
 __global__ void __launch_bounds__(256)
 gl_scan_kernel(ScanArgs a, KChunkArgs c) {
@@ -1607,35 +1548,7 @@ gl_scan_kernel(ScanArgs a, KChunkArgs c) {
   }
   float* U = c.U + (x0 * a.H + h) * GD * W + e;
   const float* L = c.G + (x0 * a.H + h) * GD + i;
-  const long us = (long)a.H * GD * W, ls = (long)a.H * GD;
-  f32x4 u[LS_AHEAD];
-  float d[LS_AHEAD];
-  auto fetch = [&](int b, f32x4 (&u)[LS_AHEAD], float (&d)[LS_AHEAD]) {
-#pragma unroll
-    for (int k = 0; k < LS_AHEAD; ++k) {
-      const int x = min(b + k, nc - 1);
-      u[k] = *reinterpret_cast<const f32x4*>(U + x * us);
-      d[k] = L[x * ls];
-    }
-  };
-  fetch(0, u, d);
-  for (int b = 0; b < nc; b += LS_AHEAD) {
-    f32x4 un[LS_AHEAD];
-    float dn[LS_AHEAD];
-    fetch(b + LS_AHEAD, un, dn);
-#pragma unroll
-    for (int k = 0; k < LS_AHEAD; ++k) {
-      if (b + k < nc) {
-        *reinterpret_cast<f32x4*>(U + (b + k) * us) = S;
-        S = S * __builtin_amdgcn_exp2f(d[k]) + u[k];
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < LS_AHEAD; ++k) {
-      u[k] = un[k];
-      d[k] = dn[k];
-    }
-  }
+  chunk_walk(U, (long)a.H * GD * W, L, (long)a.H * GD, nc, S);
   if (i < D) {
 #pragma unroll
     for (int k = 0; k < 4; ++k)
@@ -1671,7 +1584,7 @@ gl_out_kernel(ScanArgs a, KChunkArgs c) {
     for (int t = 8 * b; t < 8 * b + 8; ++t) {
       A += fmaxf(l[t], -40.f);
       tot += l[t];
-      sAv[gl_at<GD>(t0 + t, lane)] = A;
+      sAv[tile_at<GD>(t0 + t, lane)] = A;
     }
     se[2 * w + b][lane] = __builtin_amdgcn_exp2f(tot);
   }
@@ -1688,8 +1601,8 @@ gl_out_kernel(ScanArgs a, KChunkArgs c) {
       const int q = t0 + 8 * (lane / 28), ks = x - t * (t - 1) / 2;
 #pragma unroll 4
       for (int i = 0; i < GD; i += 4) {
-        const f32x4 y = gl_get<GD>(sq, q + t, i) * gl_get<GD>(sk, q + ks, i);
-        const f32x4 d = gl_get<GD>(sAv, q + t, i) - gl_get<GD>(sAv, q + ks, i);
+        const f32x4 y = tile_get<GD>(sq, q + t, i) * tile_get<GD>(sk, q + ks, i);
+        const f32x4 d = tile_get<GD>(sAv, q + t, i) - tile_get<GD>(sAv, q + ks, i);
 #pragma unroll
         for (int e = 0; e < 4; ++e) v += y[e] * __builtin_amdgcn_exp2f(d[e]);
       }
@@ -1698,7 +1611,7 @@ gl_out_kernel(ScanArgs a, KChunkArgs c) {
 #pragma unroll
     for (int i = 0; i < 16; i += 4) {
       const int d = 16 * g4 + i;
-      const f32x4 x = gl_get<GD>(sq, t0 + l16, d) * gl_get<GD>(sk, t0 + l16, d);
+      const f32x4 x = tile_get<GD>(sq, t0 + l16, d) * tile_get<GD>(sk, t0 + l16, d);
       b += x[0] + x[1] + x[2] + x[3];
     }
     b += __shfl_xor(b, 16, 64);
@@ -1719,8 +1632,8 @@ gl_out_kernel(ScanArgs a, KChunkArgs c) {
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
       pre += l[8 * b + t];
-      sq[gl_at<GD>(t0 + 8 * b + t, lane)] *= __builtin_amdgcn_exp2f(pre);
-      sk[gl_at<GD>(t0 + 8 * b + 7 - t, lane)] *= __builtin_amdgcn_exp2f(suf);
+      sq[tile_at<GD>(t0 + 8 * b + t, lane)] *= __builtin_amdgcn_exp2f(pre);
+      sk[tile_at<GD>(t0 + 8 * b + 7 - t, lane)] *= __builtin_amdgcn_exp2f(suf);
       suf += l[8 * b + 7 - t];
     }
   }
@@ -1731,8 +1644,8 @@ gl_out_kernel(ScanArgs a, KChunkArgs c) {
 #pragma unroll
   for (int b = 0; b < 4; ++b) {
     const int i = 16 * b + 4 * g4;
-    rt[b] = gl_get<GD>(sq, t0 + l16, i);
-    pq = mfma_f32_k16(gl_get<GD>(sk, t0 + l16, i), rt[b], pq);
+    rt[b] = tile_get<GD>(sq, t0 + l16, i);
+    pq = mfma_f32_k16(tile_get<GD>(sk, t0 + l16, i), rt[b], pq);
     if (l16 >= 8) rt[b] *= *reinterpret_cast<const f32x4*>(&se[2 * w][i]);
   }
 #pragma unroll
@@ -1745,7 +1658,7 @@ gl_out_kernel(ScanArgs a, KChunkArgs c) {
     for (int e = 0; e < 4; ++e)
 #pragma unroll
       for (int z = 0; z < NV; ++z) {
-        const f32x4 x = gl_get<W>(sAv, 16 * b + 4 * g4 + e, 64 * z + 4 * l16);
+        const f32x4 x = tile_get<W>(sAv, 16 * b + 4 * g4 + e, 64 * z + 4 * l16);
 #pragma unroll
         for (int j = 0; j < 4; ++j) vb[4 * z + j][e] = x[j];
       }
@@ -1757,7 +1670,7 @@ gl_out_kernel(ScanArgs a, KChunkArgs c) {
     for (int x = 0; x < 4; ++x) {                      // keys of block b; rt: from its end on
       const int i = 16 * x + 4 * g4;
       const f32x4 e1 = *reinterpret_cast<const f32x4*>(&se[2 * b + 1][i]);
-      f32x4 kk = gl_get<GD>(sk, 16 * b + l16, i);
+      f32x4 kk = tile_get<GD>(sk, 16 * b + l16, i);
       if (l16 < 8) kk *= e1;
       p = mfma_f32_k16(kk, rt[x], p);
       rt[x] *= e1 * *reinterpret_cast<const f32x4*>(&se[2 * b][i]);

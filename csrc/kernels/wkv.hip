@@ -13,7 +13,7 @@
 //
 // Batch layout: sequence s owns rows [cu[s], cu[s+1]) (cu == nullptr: row s).  All recurrence
 // math is fp32; activations are bf16 or fp32 (template T).
-#include "eia_common.h"
+#include "eia_chunks.h"
 
 EIA_DEV int find_seq(const int* cu, int nseq, int row) {
   int lo = 0, hi = nseq - 1;               // largest s with cu[s] <= row
@@ -233,16 +233,12 @@ EIA_API int eia_wkv_scan(const void* r, const void* k, const void* v, const void
 //   o_t = (r_t 2^(sum_(x<t) l_x)) S + sum_(s<t) P_ts v_s + (r_t . u . k_t) v_t
 //   P_ts = sum_channels r_t k_s 2^(sum_(s<x<t) l_x)                    (3) per chunk, in parallel
 //
-// All products are fp32 matrix-core products.  Exponents are formed as sums of the l_x that they
-// cover, never as differences, so they are <= 0 and keep their precision behind tokens that forget
-// almost everything; a pair of tokens meets through the edges of the 8-token blocks between them,
+// All products are fp32 matrix-core products.  Exponents are sums of the l_x that they cover, never
+// differences, so they are <= 0 and keep their precision behind tokens that forget almost everything; a
+// pair of tokens meets through the edges of the 8-token blocks between them,
 //   P_ts = (r_t 2^(block start .. t)) . (whole blocks between) . (k_s 2^(s .. block end)),
-// inside a block through the edge between its fours, inside a four through the one or two tokens
-// between.  (Differences of a running sum over eight tokens, l cut at -40: 8e-7 instead of 1.2e-7 against
-// 64 bits where every second token forgets, the same time.)
-//
-// Chunks are numbered without a list from the host: sequence s owns the numbers from
-// cu[s] / WC + s on, at least as many as it has chunks; numbers past its last chunk do nothing.
+// inside a block see eia_chunks.h.  (With differences of a running sum over eight tokens, l cut at -40: 8e-7
+// instead of 1.2e-7 against 64 bits where every second token forgets, in the same time.)
 //
 // Bound by instruction issue (exponentials, conversions, fp32 products; 31 us of vector and 15 us of
 // matrix issue in (3)), not by memory: one 4096-token prompt, 32 heads of 64, bf16 takes 26 + 14 +
@@ -250,7 +246,6 @@ EIA_API int eia_wkv_scan(const void* r, const void* k, const void* v, const void
 // tile for each of r, k, v and the running sums (two workgroups per CU instead of three).
 constexpr int WC = 64;                      // tokens per chunk
 constexpr int WD = 64;                      // widest head
-constexpr int WKV_AHEAD = 8;                // chunks whose contributions are in flight in (2)
 
 struct WkvChunkArgs {
   float* U;                                 // [numbers, H, WD, WD]: contribution, then state before
@@ -260,23 +255,8 @@ struct WkvChunkArgs {
 
 // The chunk of number x; false where there is none or the sequence is skipped.
 EIA_DEV bool wkv_chunk(const WkvArgs& a, int nseq, int x, int& s, int& row0, int& n) {
-  int lo = 0, hi = nseq - 1;                // largest s with cu[s] / WC + s <= x
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (a.cu[mid] / WC + mid <= x) lo = mid; else hi = mid - 1;
-  }
-  s = lo;
-  if (x < a.cu[s] / WC + s) return false;   // (rows before the first sequence)
-  row0 = a.cu[s] + (x - a.cu[s] / WC - s) * WC;
-  n = min(WC, a.cu[s + 1] - row0);
-  return n > 0 && a.cu[s + 1] - a.cu[s] >= a.split && a.slots[s] >= 0 && (!a.seq_lens || a.seq_lens[s] > 0);
-}
-
-// Place of (token, channel) in an LDS tile [WC][WD]: the 16-byte units of a row are turned by the
-// token, so that sixteen tokens' units of one channel group lie on different banks.
-EIA_DEV int wkv_at(int t, int i) { return t * WD + (i ^ ((t & 15) << 2)); }
-EIA_DEV f32x4 wkv_get(const float* tile, int t, int i) {         // channels i .. i + 3, i % 4 == 0
-  return *reinterpret_cast<const f32x4*>(tile + wkv_at(t, i));
+  return chunk_of<WC>(a.cu, nseq, x, s, row0, n) && a.cu[s + 1] - a.cu[s] >= a.split && a.slots[s] >= 0 &&
+         (!a.seq_lens || a.seq_lens[s] > 0);
 }
 
 // A chunk's [WC][WD] tile of r, k or v on its way to LDS, zero past the chunk and past D: requested
@@ -302,11 +282,11 @@ struct WkvTile {
       if constexpr (VEC) {
 #pragma unroll
         for (int e = 0; e < E; e += 4)
-          *reinterpret_cast<f32x4*>(tile + wkv_at(t, i + e)) =
+          *reinterpret_cast<f32x4*>(tile + tile_at<WD>(t, i + e)) =
               ok ? f32x4{(float)v[x][e], (float)v[x][e + 1], (float)v[x][e + 2], (float)v[x][e + 3]}
                  : f32x4{0.f, 0.f, 0.f, 0.f};
       } else {
-        tile[wkv_at(t, i)] = ok ? (float)v[x][0] : 0.f;
+        tile[tile_at<WD>(t, i)] = ok ? (float)v[x][0] : 0.f;
       }
     }
   }
@@ -362,7 +342,7 @@ wkv_chunk_state_kernel(WkvArgs a, WkvChunkArgs c) {
   for (int b = 3; b > w; --b) after += stot[b][lane];
 #pragma unroll
   for (int t = 15; t >= 0; --t) {
-    sk[wkv_at(16 * w + t, lane)] *= __builtin_amdgcn_exp2f(after);
+    sk[tile_at<WD>(16 * w + t, lane)] *= __builtin_amdgcn_exp2f(after);
     after += l[t];
   }
   const long at = (long)blockIdx.x * a.H + h;
@@ -378,8 +358,8 @@ wkv_chunk_state_kernel(WkvArgs a, WkvChunkArgs c) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int t = 16 * b + 4 * g4 + e;
-      ka[e] = sk[wkv_at(t, 16 * w + l16)];
-      const f32x4 x = wkv_get(sv, t, 4 * l16);
+      ka[e] = sk[tile_at<WD>(t, 16 * w + l16)];
+      const f32x4 x = tile_get<WD>(sv, t, 4 * l16);
 #pragma unroll
       for (int j = 0; j < 4; ++j) vb[j][e] = x[j];
     }
@@ -392,9 +372,7 @@ wkv_chunk_state_kernel(WkvArgs a, WkvChunkArgs c) {
     *reinterpret_cast<f32x4*>(U + i * WD) = f32x4{acc[0][i], acc[1][i], acc[2][i], acc[3][i]};
 }
 
-// (2) Four columns of a state row per thread: U of a chunk turns into the state before it; the slot
-// receives the state after the last one.  A group's contributions are requested while the previous
-// group is summed.
+// (2) Four columns of a state row per thread; the slot receives the state after the last chunk.
 __global__ void __launch_bounds__(256)
 wkv_chunk_scan_kernel(WkvArgs a, WkvChunkArgs c) {
   const int s = blockIdx.x, h = blockIdx.y;
@@ -412,35 +390,7 @@ wkv_chunk_scan_kernel(WkvArgs a, WkvChunkArgs c) {
   }
   float* U = c.U + (x0 * a.H + h) * WD * WD + e;
   const float* L = c.L + (x0 * a.H + h) * WD + i;
-  const long us = (long)a.H * WD * WD, ls = (long)a.H * WD;
-  f32x4 u[WKV_AHEAD];
-  float d[WKV_AHEAD];
-  auto fetch = [&](int b, f32x4 (&u)[WKV_AHEAD], float (&d)[WKV_AHEAD]) {
-#pragma unroll
-    for (int k = 0; k < WKV_AHEAD; ++k) {
-      const int x = min(b + k, nc - 1);
-      u[k] = *reinterpret_cast<const f32x4*>(U + x * us);
-      d[k] = L[x * ls];
-    }
-  };
-  fetch(0, u, d);
-  for (int b = 0; b < nc; b += WKV_AHEAD) {
-    f32x4 un[WKV_AHEAD];
-    float dn[WKV_AHEAD];
-    fetch(b + WKV_AHEAD, un, dn);
-#pragma unroll
-    for (int k = 0; k < WKV_AHEAD; ++k) {
-      if (b + k < nc) {
-        *reinterpret_cast<f32x4*>(U + (b + k) * us) = S;
-        S = S * __builtin_amdgcn_exp2f(d[k]) + u[k];
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < WKV_AHEAD; ++k) {
-      u[k] = un[k];
-      d[k] = dn[k];
-    }
-  }
+  chunk_walk(U, (long)a.H * WD * WD, L, (long)a.H * WD, nc, S);
   if (i < D) {
 #pragma unroll
     for (int k = 0; k < 4; ++k)
@@ -474,84 +424,30 @@ wkv_chunk_out_kernel(WkvArgs a, WkvChunkArgs c) {
   tv.load(a.v, a.ld, hc, row0, n, D);
   tr.store(sr, n, D);
   tk.store(sk, n, D);
-  // E: l over the rest of a token's four if they are the first of its eight, else from their start on
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
     float tot = 0.f;
 #pragma unroll
     for (int t = 8 * b; t < 8 * b + 8; ++t) tot += l[t];
     se[2 * w + b][lane] = __builtin_amdgcn_exp2f(tot);
-    float suf = 0.f, pre = 0.f;
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      sAv[wkv_at(t0 + 8 * b + 3 - t, lane)] = suf;
-      suf += l[8 * b + 3 - t];
-      sAv[wkv_at(t0 + 8 * b + 4 + t, lane)] = pre;
-      pre += l[8 * b + 4 + t];
-    }
   }
+  block_edges<false>(l, sAv, t0, lane);
   if (w == 0) su[lane] = lane < D ? ld_f32<T>(static_cast<const T*>(a.u), hc + lane) : 0.f;
   if (threadIdx.x == 0) swild = 0;
   __syncthreads();
-  // weights inside the wave's two 8-token blocks: lane = pair s < t and half of the channels, then to
-  // the lane that holds them as an operand (query l16, keys 4 g4 + i)
-  f32x4 p = {0.f, 0.f, 0.f, 0.f};
+  f32x4 p = {0.f, 0.f, 0.f, 0.f};                      // weights inside the wave's 8-token blocks
   if (t0 < n) {
-    const int pr = lane & 31, c0 = lane & 32;
-    float v4 = 0.f, v8 = 0.f;
-    {                                                  // t in the second four of its eight, s in the first
-      const int s8 = t0 + 8 * (pr >> 4) + (pr & 3), t8 = t0 + 8 * (pr >> 4) + 4 + (pr >> 2 & 3);
-#pragma unroll 4
-      for (int i = c0; i < c0 + 32; i += 4) {
-        const f32x4 y = wkv_get(sr, t8, i) * wkv_get(sk, s8, i);
-        const f32x4 d = wkv_get(sAv, t8, i) + wkv_get(sAv, s8, i);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v8 += y[e] * __builtin_amdgcn_exp2f(d[e]);
-      }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    // E of the wave's fours: l of token 1 in row 0, of token 2 in row 3
-#pragma unroll
-    for (int t = 0; t < 16; t += 4) {
-      sAv[wkv_at(t0 + t, lane)] = l[t + 1];
-      sAv[wkv_at(t0 + t + 3, lane)] = l[t + 2];
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    if (pr < 24) {                                     // s < t in the same four
-      const int x = pr % 6, t = x >= 3 ? 3 : x >= 1 ? 2 : 1, ks = x - t * (t - 1) / 2, q = t0 + 4 * (pr / 6);
-      const bool l1 = ks == 0 && t > 1, l2 = t == 3 && ks < 2;
-#pragma unroll 4
-      for (int i = c0; i < c0 + 32; i += 4) {
-        const f32x4 y = wkv_get(sr, q + t, i) * wkv_get(sk, q + ks, i);
-        const f32x4 d1 = wkv_get(sAv, q, i), d2 = wkv_get(sAv, q + 3, i);
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          v4 += y[e] * __builtin_amdgcn_exp2f((l1 ? d1[e] : 0.f) + (l2 ? d2[e] : 0.f));
-      }
-    }
-    v4 += __shfl_xor(v4, 32, 64);
-    v8 += __shfl_xor(v8, 32, 64);
-    const float v = lane < 32 ? v8 : v4;
     float b = 0.f;                                     // r . u . k of token t0 + l16
 #pragma unroll
     for (int i = 0; i < 16; i += 4) {
       const int d = 16 * g4 + i;
-      const f32x4 x = wkv_get(sr, t0 + l16, d) * wkv_get(sk, t0 + l16, d) *
+      const f32x4 x = tile_get<WD>(sr, t0 + l16, d) * tile_get<WD>(sk, t0 + l16, d) *
                       *reinterpret_cast<const f32x4*>(&su[d]);
       b += x[0] + x[1] + x[2] + x[3];
     }
     b += __shfl_xor(b, 16, 64);
     b += __shfl_xor(b, 32, 64);
-    const int f4 = l16 >> 2, t4 = l16 & 3;             // the query's four, its place there
-    const int from = g4 == f4 ? 32 + 6 * f4 + (t4 * (t4 - 1) >> 1) : 16 * (f4 >> 1) + 4 * t4;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float x = __shfl(v, from + i, 64);
-      if (g4 == f4) p[i] = i == t4 ? b : i < t4 ? x : 0.f;
-      else p[i] = (f4 & 1) && g4 == f4 - 1 ? x : 0.f;
-    }
+    p = block_weights<false>(sr, sk, sAv, l, b, t0, lane);
   }
   __syncthreads();
   // r_t <- r_t 2^(block start .. t), k_s <- k_s 2^(s .. block end), 8-token blocks; v moves in
@@ -560,9 +456,9 @@ wkv_chunk_out_kernel(WkvArgs a, WkvChunkArgs c) {
     float pre = 0.f, suf = 0.f;
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
-      sr[wkv_at(t0 + 8 * b + t, lane)] *= __builtin_amdgcn_exp2f(pre);
+      sr[tile_at<WD>(t0 + 8 * b + t, lane)] *= __builtin_amdgcn_exp2f(pre);
       pre += l[8 * b + t];
-      sk[wkv_at(t0 + 8 * b + 7 - t, lane)] *= __builtin_amdgcn_exp2f(suf);
+      sk[tile_at<WD>(t0 + 8 * b + 7 - t, lane)] *= __builtin_amdgcn_exp2f(suf);
       suf += l[8 * b + 7 - t];
     }
   }
@@ -574,8 +470,8 @@ wkv_chunk_out_kernel(WkvArgs a, WkvChunkArgs c) {
 #pragma unroll
   for (int b = 0; b < 4; ++b) {
     const int i = 16 * b + 4 * g4;
-    rt[b] = wkv_get(sr, t0 + l16, i);
-    pq = mfma_f32_k16(wkv_get(sk, t0 + l16, i), rt[b], pq);
+    rt[b] = tile_get<WD>(sr, t0 + l16, i);
+    pq = mfma_f32_k16(tile_get<WD>(sk, t0 + l16, i), rt[b], pq);
     if (l16 >= 8) rt[b] *= *reinterpret_cast<const f32x4*>(&se[2 * w][i]);
     o[b] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
@@ -589,7 +485,7 @@ wkv_chunk_out_kernel(WkvArgs a, WkvChunkArgs c) {
       for (int k4 = 0; k4 < 4; ++k4)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const f32x4 x = wkv_get(sAv, t0 + 4 * k4 + e, 4 * l16);
+          const f32x4 x = tile_get<WD>(sAv, t0 + 4 * k4 + e, 4 * l16);
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             const float pt = __shfl(p[e], 16 * k4 + 4 * g4 + i, 64);
@@ -602,7 +498,7 @@ wkv_chunk_out_kernel(WkvArgs a, WkvChunkArgs c) {
       f32x4 vb[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const f32x4 x = wkv_get(sAv, 16 * b + 4 * g4 + e, 4 * l16);
+        const f32x4 x = tile_get<WD>(sAv, 16 * b + 4 * g4 + e, 4 * l16);
 #pragma unroll
         for (int j = 0; j < 4; ++j) vb[j][e] = x[j];
       }
@@ -615,7 +511,7 @@ wkv_chunk_out_kernel(WkvArgs a, WkvChunkArgs c) {
     for (int x = 0; x < 4; ++x) {                      // keys of block b; rt: from its end on
       const int i = 16 * x + 4 * g4;
       const f32x4 e1 = *reinterpret_cast<const f32x4*>(&se[2 * b + 1][i]);
-      f32x4 kk = wkv_get(sk, 16 * b + l16, i);
+      f32x4 kk = tile_get<WD>(sk, 16 * b + l16, i);
       if (l16 < 8) kk *= e1;
       p = mfma_f32_k16(kk, rt[x], p);
       rt[x] *= e1 * *reinterpret_cast<const f32x4*>(&se[2 * b][i]);

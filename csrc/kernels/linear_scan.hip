@@ -1337,8 +1337,8 @@ EIA_API int eia_linear_scan_channels(const void* x, long ld, int q_off, int k_of
 }
 
 // ---------------------------------------------------------------------------------------------
-// Mode 2 for dk <= 64 on matrix cores: the chunks of GC tokens, the block edges and the cut at 2^-40
-// of wkv.hip's chunk-parallel form, with the token itself among its keys,
+// Mode 2 for dk <= 64 on matrix cores: the chunks of GC tokens and the block edges of wkv.hip's
+// chunk-parallel form, with the token itself among its keys,
 //
 //   U   = sum_s 2^(sum_(s<x) l_x) k_s v_s^T                            (1) per chunk, in parallel
 //   S' = 2^(sum_x l_x) S + U                                           (2) a sequence's chunks in order
@@ -1346,10 +1346,10 @@ EIA_API int eia_linear_scan_channels(const void* x, long ld, int q_off, int k_of
 //   P_ts = sum_channels q_t k_s 2^(sum_(s<x<=t) l_x)                   (3) per chunk, in parallel
 //
 // where l_x = log2 a_x per key channel, formed by a pass of its own for all rows and heads (its
-// low-rank product and logarithms are the same for (1) and (3)).  Exponents are sums of the l_x that
-// they cover; pairs of different 8-token blocks meet through the edges of the blocks between them, and
-// only pairs inside a block take the difference of a running sum over that block.  Products are fp32
-// matrix-core products.  Bound by instruction issue (exponentials, operand rows through LDS), as there.
+// low-rank product and logarithms are the same for (1) and (3)).  Exponents are sums of the l_x that they
+// cover; pairs of different 8-token blocks meet through the edges of the blocks between them, for those
+// inside a block see eia_chunks.h.  Products are fp32 matrix-core products.  Bound by instruction issue
+// (exponentials, operand rows through LDS), as there.
 // Four prompts of 490 to 977 tokens, 16 heads of 64 x 128, bf16: 21 + 22 + 11 + 60 us on an MI355X (l, (1),
 // (2), (3)); in the 32-token chunks of vector FMAs above 38 + 71 + 21 + 235 us, which remain for keys
 // wider than 64.
@@ -1579,34 +1579,15 @@ gl_out_kernel(ScanArgs a, KChunkArgs c) {
   tk.store(sk, n, a.kscale);
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
-    float A = 0.f, tot = 0.f;
+    float tot = 0.f;
 #pragma unroll
-    for (int t = 8 * b; t < 8 * b + 8; ++t) {
-      A += fmaxf(l[t], -40.f);
-      tot += l[t];
-      sAv[tile_at<GD>(t0 + t, lane)] = A;
-    }
+    for (int t = 8 * b; t < 8 * b + 8; ++t) tot += l[t];
     se[2 * w + b][lane] = __builtin_amdgcn_exp2f(tot);
   }
+  block_edges<true>(l, sAv, t0, lane);
   __syncthreads();
-  // weights inside the wave's two 8-token blocks: lane = pair s < t, then to the lane that holds
-  // them as an operand (query l16, keys 4 g4 + i)
-  f32x4 p = {0.f, 0.f, 0.f, 0.f};
+  f32x4 p = {0.f, 0.f, 0.f, 0.f};                      // weights inside the wave's 8-token blocks
   if (t0 < n) {
-    float v = 0.f;
-    if (lane < 56) {
-      const int x = lane % 28;
-      int t = 1;
-      while (t * (t + 1) / 2 <= x) ++t;
-      const int q = t0 + 8 * (lane / 28), ks = x - t * (t - 1) / 2;
-#pragma unroll 4
-      for (int i = 0; i < GD; i += 4) {
-        const f32x4 y = tile_get<GD>(sq, q + t, i) * tile_get<GD>(sk, q + ks, i);
-        const f32x4 d = tile_get<GD>(sAv, q + t, i) - tile_get<GD>(sAv, q + ks, i);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v += y[e] * __builtin_amdgcn_exp2f(d[e]);
-      }
-    }
     float b = 0.f;                                     // q . k of token t0 + l16
 #pragma unroll
     for (int i = 0; i < 16; i += 4) {
@@ -1616,13 +1597,7 @@ gl_out_kernel(ScanArgs a, KChunkArgs c) {
     }
     b += __shfl_xor(b, 16, 64);
     b += __shfl_xor(b, 32, 64);
-    const int t8 = l16 & 7;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int ks = 4 * g4 + i;
-      const float x = __shfl(v, 28 * (l16 >> 3) + (t8 * (t8 - 1) >> 1) + (ks & 7), 64);
-      p[i] = ks == l16 ? b : (ks < l16 && ks >> 3 == l16 >> 3) ? x : 0.f;
-    }
+    p = block_weights<true>(sq, sk, sAv, l, b, t0, lane);
   }
   __syncthreads();
   // q_t <- q_t 2^(block start .. t], k_s <- k_s 2^(s .. block end), 8-token blocks; v moves in

@@ -293,3 +293,34 @@ def test_wkv_strongly_forgetting_tokens(every):
     # outputs are 1.4e-7 off; exponents that differ by an ulp of 160, the sum of four such decays, 8e-7
     assert _rel(z, y) < 3e-7
     assert _rel(dev[8][0], S) < 3e-7
+
+
+@pytest.mark.parametrize("spread", [3.0, 8.0, 20.0])
+def test_channel_strongly_forgetting_tokens(spread, monkeypatch):
+    """As above for a decay per key channel, which a token's own entry passes too."""
+    from enterprise_inference_amd.ops import linear_scan as ls
+    H, D, Dv, R, T = 2, 64, 64, 16, 128
+    g = torch.Generator().manual_seed(int(spread))
+    rnd = lambda *s: torch.randn(*s, generator=g)
+    at = [0, H * D, 2 * H * D, 2 * H * D + H * Dv, 2 * H * (D + Dv)]
+    x, a2t, a2b = rnd(T, at[-1] + R), spread * rnd(R, H * D), torch.full((H * D,), 6.0)
+    spec = ls.ScanSpec(H, D, Dv, "channel", kscale=D ** -0.5, eps=1e-5, a2t=a2t.cuda(), a2b=a2b.cuda(), tau=1.0)
+    st = ls.ScanState(torch.zeros(1, H, D, Dv, device="cuda"), None, None)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    monkeypatch.setattr(ls, "FORCE_CHUNKED", True)
+    y = ls.linear_scan(x.cuda(), at[0], at[1], at[2], at[3], spec, st, i32([0]), i32([0, T]), 1,
+                       torch.arange(T, dtype=torch.int32).cuda(), plan=ls.chunk_plan([T], "cuda"),
+                       lo_off=at[4])
+    f = x.double()
+    q, k = f[:, :H * D].view(T, H, D), f[:, H * D:2 * H * D].view(T, H, D) * D ** -0.5
+    v, gate = f[:, at[2]:at[3]].view(T, H, Dv), f[:, at[3]:at[4]]
+    a = torch.sigmoid(f[:, at[4]:] @ a2t.double() + 6.0).view(T, H, D)
+    S, o = torch.zeros(H, D, Dv, dtype=torch.float64), torch.empty(T, H, Dv, dtype=torch.float64)
+    for t in range(T):
+        S = a[t][:, :, None] * S + k[t][:, :, None] * v[t][:, None]
+        w = (S * q[t][:, :, None]).sum(1)
+        o[t] = w / torch.sqrt((w * w).mean(-1, keepdim=True) + 1e-5)
+    r = o.flatten(1) * torch.nn.functional.silu(gate)
+    # differences of a running sum over eight tokens: 3e-7 to 5e-7
+    assert _rel(y, r) < 2.5e-7
+    assert _rel(st.S[0], S) < 2.5e-7

@@ -433,9 +433,10 @@ EIA_API int eia_linear_scan(const void* x, long ld, int q_off, int k_off, int v_
 //         + sum_(s<=t) 2^(m_s + sum_(s<x<=t) l_x) (q_t . k_s) v_s         (3) per chunk, in parallel
 //
 // (the normaliser n is one more state column, n_t . q_t the row sum of the same weights).  Sums of l
-// run over 16-token blocks and over whole blocks; only inside one block is a sum the difference of
-// two running sums, so every exponent is <= 0 and keeps its precision.  The log gates of mode 1 come
-// from a pre-pass that carries the running maximum, angles of rotated heads from a table.
+// run over 16-token blocks and over whole blocks, inside a block over just the tokens between: every
+// exponent is a sum of what it covers, so it is <= 0 and keeps its precision.  (Differences of two running
+// sums inside a block: 9.9e-7 instead of 1.8e-7 against 64 bits, fp32 gates that close hard.)  The log gates
+// of mode 1 come from a pre-pass that carries the running maximum, angles of rotated heads from a table.
 // Chunks are found on the device (eia_chunks.h).
 //
 // Products are fp32 matrix-core products, except q . k of unrotated bf16 rows, which is exact in
@@ -631,9 +632,9 @@ EIA_DEV void ls_stage_v(const ScanArgs& a, int row0, int n, int h, int t0, T* sv
 }
 
 // Sums of l over 16-token blocks: pre up to and with a token, suf behind it, tot of whole blocks;
-// mb: m.  Threads 0 .. LK - 1.
+// mb: m, sl: l.  Threads 0 .. LK - 1.
 EIA_DEV void ls_chunk_logs(const ScanArgs& a, const KChunkArgs& c, int row0, int n, int h, float* pre,
-                           float* suf, float* tot, float* mb) {
+                           float* suf, float* tot, float* mb, float* sl) {
   const int t = threadIdx.x;
   if (t >= LK) return;
   float l = 0.f, b = 0.f;
@@ -645,7 +646,8 @@ EIA_DEV void ls_chunk_logs(const ScanArgs& a, const KChunkArgs& c, int row0, int
       b = c.lb[(long)(row0 + t) * a.H + h] * LS_LOG2E;
     }
   }
-  l = fmaxf(l, -150.f);                                // (2^-150 is zero)
+  l = l < -150.f ? -150.f : l;                         // (2^-150 is zero; what is no number stays so)
+  sl[t] = l;
   float p = l, s = l;
   const int t16 = t & 15;
 #pragma unroll
@@ -661,6 +663,28 @@ EIA_DEV void ls_chunk_logs(const ScanArgs& a, const KChunkArgs& c, int row0, int
   if (t16 == 15) tot[t >> 4] = p;
 }
 
+// Sums of l over the tokens s < x <= t of one 16-token block, for the lane's query t = lane % 16 and keys
+// s = 4 (lane / 16) + i: the rest of the key's four, the fours between, the query's four up to it.
+EIA_DEV f32x4 ls_inside(const float* l, int lane) {
+  const f32x4* four = reinterpret_cast<const f32x4*>(l);
+  const int g4 = lane >> 4, f4 = lane >> 2 & 3, t4 = lane & 3;
+  const f32x4 kf = four[g4], qf = four[f4], f1 = four[1], f2 = four[2];
+  float up = qf[0];
+#pragma unroll
+  for (int j = 1; j < 4; ++j) up += j <= t4 ? qf[j] : 0.f;
+  if (g4 < 1 && f4 > 1) up += f1[0] + f1[1] + f1[2] + f1[3];
+  if (g4 < 2 && f4 > 2) up += f2[0] + f2[1] + f2[2] + f2[3];
+  const int last = g4 == f4 ? t4 : 3;
+  f32x4 e;
+  float rest = g4 < f4 ? up : 0.f;
+#pragma unroll
+  for (int j = 3; j >= 0; --j) {
+    e[j] = rest;
+    rest += j <= last ? kf[j] : 0.f;
+  }
+  return e;
+}
+
 // (1) Eight waves; wave w forms rows 16 w .. of U.  Tokens come in two halves of 64.  A lane of a
 // product over tokens holds columns 64 x + 4 (lane % 16) + j in tile 4 x + j, here and in (3).
 template <typename T, bool VEC, bool ROT, int MX>
@@ -668,12 +692,12 @@ __global__ void __launch_bounds__(512)
 ls_chunk_state_kernel(ScanArgs a, KChunkArgs c) {
   __shared__ __align__(16) float sk[64 * MX];
   __shared__ __align__(16) T sv[64 * MX];
-  __shared__ float pre[LK], suf[LK], mb[LK], tot[LK / 16];
+  __shared__ float pre[LK], suf[LK], mb[LK], tot[LK / 16], sl[LK];
   int s, row0, n;
   if (!ls_chunk(a, c.nseq, blockIdx.x, s, row0, n)) return;
   const int h = blockIdx.y, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int l16 = lane & 15, g4 = lane >> 4;
-  ls_chunk_logs(a, c, row0, n, h, pre, suf, tot, mb);
+  ls_chunk_logs(a, c, row0, n, h, pre, suf, tot, mb, sl);
   f32x4 acc[MX / 16];
   float un = 0.f;                                      // normaliser row 16 w + l16
 #pragma unroll
@@ -787,7 +811,8 @@ ls_chunk_out_kernel(ScanArgs a, KChunkArgs c) {
   float* sS = reinterpret_cast<float*>(tiles);         // [MX][MX] the state, then keys and values
   KT* sk = reinterpret_cast<KT*>(tiles);
   T* sv = reinterpret_cast<T*>(sk + LK * MX);
-  __shared__ float pre[LK], suf[LK], mb[LK], tot[LK / 16], sn[MX];
+  __shared__ __align__(16) float pre[LK], suf[LK], mb[LK], sl[LK];
+  __shared__ float tot[LK / 16], sn[MX];
   int s, row0, n;
   if (!ls_chunk(a, c.nseq, blockIdx.x, s, row0, n)) return;
   const int h = blockIdx.y, lane = threadIdx.x & 63, wv = threadIdx.x >> 6, D = a.D, Dv = a.Dv;
@@ -806,7 +831,7 @@ ls_chunk_out_kernel(ScanArgs a, KChunkArgs c) {
     if (a.mode == 1 && threadIdx.x < MX)
       sn[threadIdx.x] = S[(long)min((int)threadIdx.x, c.DP - 1) * c.UW + c.VP];
   }
-  ls_chunk_logs(a, c, row0, n, h, pre, suf, tot, mb);
+  ls_chunk_logs(a, c, row0, n, h, pre, suf, tot, mb, sl);
   // this lane's query: channels 32 x + 8 g4 + e
   const int tq = t0 + l16;
   typedef KT KT8 __attribute__((ext_vector_type(8)));
@@ -909,11 +934,13 @@ ls_chunk_out_kernel(ScanArgs a, KChunkArgs c) {
                            f32x4{qf[x][e], qf[x][e + 1], qf[x][e + 2], qf[x][e + 3]}, p);
       }
     }
+    f32x4 e;
+    if (b == w) e = ls_inside(sl + t0, lane);
+    else e = *reinterpret_cast<const f32x4*>(suf + 16 * b + 4 * g4) + (pq + back);
+    e += *reinterpret_cast<const f32x4*>(mb + 16 * b + 4 * g4);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int tk = 16 * b + 4 * g4 + i;
-      const float e = b == w ? pq - pre[tk] + mb[tk] : pq + back + suf[tk] + mb[tk];
-      p[i] = tk <= tq ? p[i] * qk * __builtin_amdgcn_exp2f(e) : 0.f;
+      p[i] = 16 * b + 4 * g4 + i <= tq ? p[i] * qk * __builtin_amdgcn_exp2f(e[i]) : 0.f;
       rs += p[i];
     }
 #pragma unroll

@@ -324,3 +324,51 @@ def test_channel_strongly_forgetting_tokens(spread, monkeypatch):
     # differences of a running sum over eight tokens: 3e-7 to 5e-7
     assert _rel(y, r) < 2.5e-7
     assert _rel(st.S[0], S) < 2.5e-7
+
+
+@pytest.mark.parametrize("spread", [8.0, 20.0])
+def test_gates_that_close_hard(spread, monkeypatch):
+    """As above for exponential gates, some of which forget almost everything."""
+    from enterprise_inference_amd.ops import linear_scan as ls
+    monkeypatch.setattr(ls, "FORCE_CHUNKED", True)
+    H, D, T = 4, 64, 256
+    g = torch.Generator().manual_seed(int(spread))
+    x = torch.randn(T, 4 * H * D + 2 * H, generator=g)
+    x[:, -H:] = 4 + spread * torch.randn(T, H, generator=g)
+    at = [0, H * D, 2 * H * D, 3 * H * D, 4 * H * D, 4 * H * D + H]
+    spec = ls.ScanSpec(H, D, D, "exp_gates", kscale=D ** -0.5, eps=1e-5, cap=0.0, gate_act="sigmoid")
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+
+    def run(x):
+        st = ls.ScanState(torch.zeros(1, H, D, D, device="cuda"), torch.zeros(1, H, D, device="cuda"),
+                          torch.zeros(1, H, device="cuda"))
+        y = ls.linear_scan(x.cuda(), at[0], at[1], at[2], at[3], spec, st, i32([0]), i32([0, T]), 1,
+                           torch.arange(T, dtype=torch.int32).cuda(), None, None, at[4], at[5],
+                           plan=ls.chunk_plan([T], "cuda"))
+        return y.cpu(), st.S[0].cpu()
+
+    y, S = run(x)
+    q, k, v, gate = (x[:, a:b].double() for a, b in zip(at, at[1:5]))
+    q, k, v = q.view(T, H, D), k.view(T, H, D) * D ** -0.5, v.view(T, H, D)
+    gi, gf = x[:, at[4]:at[5]].double(), torch.nn.functional.logsigmoid(x[:, at[5]:].double())
+    s, n, m = (torch.zeros(*z, dtype=torch.float64) for z in ((H, D, D), (H, D), (H,)))
+    o = torch.empty(T, H, D, dtype=torch.float64)
+    for t in range(T):
+        top = torch.maximum(gf[t] + m, gi[t])
+        a, b, m = torch.exp(gf[t] + m - top), torch.exp(gi[t] - top), top
+        s = a[:, None, None] * s + b[:, None, None] * k[t][:, :, None] * v[t][:, None]
+        n = a[:, None] * n + b[:, None] * k[t]
+        w = (s * q[t][:, :, None]).sum(1)
+        w = w / (torch.maximum((n * q[t]).sum(-1).abs(), torch.exp(-m)) + 1e-6)[:, None]
+        o[t] = w / torch.sqrt((w * w).mean(-1, keepdim=True) + 1e-5)
+    # token by token 3e-7 and 5e-7; differences of two running sums over a block 3.5e-7 and 1e-6
+    assert _rel(y, o.flatten(1) * torch.sigmoid(gate)) < 3e-7
+    assert _rel(S, s) < 3e-7
+    # a gate that is no number is not taken for one that closes
+    for at_t in (5, 37, 130):
+        bad = x.clone()
+        bad[at_t, at[5] + 1] = float("nan")
+        z, Z = run(bad)
+        rest = [h for h in range(H) if h != 1]
+        assert torch.equal(z[:at_t], y[:at_t]) and torch.isnan(z[at_t:, D:2 * D]).all() and torch.isnan(Z[1]).all()
+        assert torch.equal(z.view(T, H, D)[:, rest], y.view(T, H, D)[:, rest]) and torch.equal(Z[rest], S[rest])

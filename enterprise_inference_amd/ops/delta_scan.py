@@ -270,6 +270,8 @@ def prefill_plan(md, device) -> Optional[ChunkPlan]:
         if md.seq_cu is not None and lens and len(lens) == md.num_seqs - md.num_decode:
             plan = chunk_plan(lens, device, CHUNK, 1 if FORCE_CHUNKED else CHUNK_MIN_ROWS,
                               md.num_decode)
+            if plan is not None:
+                plan.lists()
         md.work_cache["delta_chunks"] = plan
     return md.work_cache["delta_chunks"]
 

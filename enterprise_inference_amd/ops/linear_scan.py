@@ -26,10 +26,12 @@ slot held, so freed slots are reused without clearing.  Batch layout: sequence `
 state slot (< 0: padding row, skipped).
 
 Prompt portions run a chunk-parallel form on the GPU (``chunk_plan``): the step's rows are cut
-into chunks of 128 tokens (32 with a decay per key channel), every chunk's own contribution to the state is formed in parallel, a
-short scan over a sequence's chunks yields the state before each chunk, and the outputs of all
-chunks are formed in parallel from that state and the chunk's own tokens.  The token-by-token
-kernel serves decode steps (also inside captured graphs) and heads wider than 128.
+into chunks of 128 tokens (with a decay per key channel 64, or 32 where keys are wider than 64), every
+chunk's own contribution to the state is formed in parallel, a short scan over a sequence's chunks
+yields the state before each chunk, and the outputs of all chunks are formed in parallel from that
+state and the chunk's own tokens.  Decode steps (also inside captured graphs) run a kernel of their
+own for heads up to 128 wide.  The token-by-token kernel serves wider heads, prompt portions too short
+for chunks or inside a captured graph, and value widths that four does not divide.
 """
 
 from __future__ import annotations
@@ -95,9 +97,9 @@ class ScanState:
         return 4 * per
 
 
-CHUNK = 32                 # tokens per chunk of the chunk-parallel form ("channel", linear_scan.hip LC)
-HEAD_CHUNK = 128           # ... with one decay per head and token (linear_scan.hip LK)
-KEY_CHUNK64, KEY_DIM64 = 64, 64     # ... of the form with a decay per key channel, and its widest dk
+CHUNK = 32                 # tokens per chunk with a decay per key channel (linear_scan.hip LC)
+HEAD_CHUNK = 128           # ... with one decay per head and token (LK)
+KEY_CHUNK64, KEY_DIM64 = 64, 64     # ... with a decay per key channel and narrow keys (GC), its widest dk
 CHUNK_MAX_DIM = 128        # ... and its largest dk / dv
 CHUNK_MIN_ROWS = 48        # a sequence with at least this many rows in the step selects it
 # tests and measurements: take the chunk-parallel form whenever a plan is handed over
@@ -105,15 +107,40 @@ FORCE_CHUNKED = os.environ.get("EIA_SCAN_FORCE_CHUNKED", "0") == "1"
 
 
 class ChunkPlan:
-    """A step's rows cut into chunks for the chunk-parallel form: ``chunks`` int32 [n, 4]
-    (sequence, first row, tokens, 0), ``seq_first`` int32 [nseq + 1] (first chunk of every
-    sequence), both on the device; ``rows`` the step's row count."""
+    """A step's rows cut into chunks for the chunk-parallel forms: ``n`` chunks over sequences of
+    ``lens`` rows from row ``row0`` on; ``rows`` the step's row count, ``longest`` the longest
+    sequence's.  Forms that do not find their chunks themselves read two lists on the device, made
+    when first asked for: ``chunks`` int32 [n, 4] (sequence, first row, tokens, 0) and ``seq_first``
+    int32 [nseq + 1] (first chunk of every sequence)."""
 
-    __slots__ = ("chunks", "seq_first", "n", "rows", "nseq", "longest")
+    __slots__ = ("lens", "device", "chunk", "row0", "n", "rows", "nseq", "longest", "_lists")
 
-    def __init__(self, chunks, seq_first, n, rows, nseq=1, longest=0):
-        self.chunks, self.seq_first, self.n, self.rows = chunks, seq_first, n, rows
-        self.nseq, self.longest = nseq, longest
+    def __init__(self, lens, device, chunk: int, row0: int = 0):
+        self.lens, self.device, self.chunk, self.row0 = list(lens), device, chunk, row0
+        self.n = sum(-(-k // chunk) for k in self.lens)
+        self.rows, self.nseq, self.longest = row0 + sum(self.lens), len(self.lens), max(self.lens)
+        self._lists = None
+
+    def lists(self):
+        """(chunks, seq_first)."""
+        if self._lists is None:
+            chunks, first, row = [], [0], self.row0
+            for s, n in enumerate(self.lens):
+                for lo in range(0, n, self.chunk):
+                    chunks += [s, row + lo, min(self.chunk, n - lo), 0]
+                row += n
+                first.append(len(chunks) // 4)
+            i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=self.device)
+            self._lists = i32(chunks).view(-1, 4), i32(first)
+        return self._lists
+
+    @property
+    def chunks(self) -> torch.Tensor:
+        return self.lists()[0]
+
+    @property
+    def seq_first(self) -> torch.Tensor:
+        return self.lists()[1]
 
     def pays(self, heads: int, dim: int, cus: int = 256, channel: bool = False,
              key_dim: int = 0) -> bool:
@@ -143,19 +170,11 @@ class ChunkPlan:
 
 def chunk_plan(host_lens, device, chunk: int = CHUNK, min_rows: int = CHUNK_MIN_ROWS,
                row0: int = 0) -> Optional["ChunkPlan"]:
-    """The chunk list of a step whose sequences own ``host_lens`` rows each (batch order, from row
+    """The chunk plan of a step whose sequences own ``host_lens`` rows each (batch order, from row
     ``row0`` on), or None when no sequence is long enough for the chunk-parallel form to pay."""
     if not host_lens or max(host_lens) < min_rows:
         return None
-    chunks, first, row = [], [0], row0
-    for s, n in enumerate(host_lens):
-        for lo in range(0, n, chunk):
-            chunks += [s, row + lo, min(chunk, n - lo), 0]
-        row += n
-        first.append(len(chunks) // 4)
-    return ChunkPlan(torch.tensor(chunks, dtype=torch.int32, device=device).view(-1, 4),
-                     torch.tensor(first, dtype=torch.int32, device=device), len(chunks) // 4, row,
-                     len(host_lens), max(host_lens))
+    return ChunkPlan(host_lens, device, chunk, row0)
 
 
 def _seq_bounds(cu: Optional[torch.Tensor], nseq: int):

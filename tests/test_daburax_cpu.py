@@ -82,3 +82,14 @@ def test_every_tensor_has_a_place():
         assert loaded == {n for n, _ in model.named_parameters()}
         with pytest.raises(ValueError):
             model.load_weights([("l0.mix.nothing", torch.zeros(1))])
+
+
+def test_chunk_plan_lists():
+    """Chunks of a step whose sequences begin at row 3: counts on the host, lists when asked for."""
+    from enterprise_inference_amd.ops import linear_scan as ls
+    assert ls.chunk_plan([1, 7], "cpu") is None
+    plan = ls.chunk_plan([70, 0, 1, 64], "cpu", row0=3)
+    assert (plan.n, plan.rows, plan.nseq, plan.longest) == (6, 138, 4, 70) and plan._lists is None
+    assert plan.seq_first.tolist() == [0, 3, 3, 4, 6]
+    assert plan.chunks.tolist() == [[0, 3, 32, 0], [0, 35, 32, 0], [0, 67, 6, 0], [2, 73, 1, 0],
+                                    [3, 74, 32, 0], [3, 106, 32, 0]]

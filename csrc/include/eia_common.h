@@ -99,3 +99,21 @@ template <typename V> EIA_DEV void mfma_settle(V (&o)[8]) {
   asm volatile("s_nop 11" : "+v"(o[0]), "+v"(o[1]), "+v"(o[2]), "+v"(o[3]), "+v"(o[4]), "+v"(o[5]),
                "+v"(o[6]), "+v"(o[7]));
 }
+
+// One access from memory straight to LDS: lane i's 16 bytes at gsrc go to byte lds_addr + 16 i.  Not
+// counted by the compiler: the caller waits for vmcnt, and for its own reads of the place before.
+EIA_DEV void glds16(const void* gsrc, unsigned lds_addr) {
+  unsigned keep;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\t"
+      "s_mov_b32 m0, %2\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, off\n\t"
+      "s_mov_b32 m0, %0"
+      : "=&s"(keep)
+      : "v"(gsrc), "s"(__builtin_amdgcn_readfirstlane(lds_addr))
+      : "memory");
+}
+EIA_DEV unsigned lds_offset(const void* p) {
+  return (unsigned)(uintptr_t)(__attribute__((address_space(3))) const void*)p;
+}

@@ -415,19 +415,6 @@ gemm_skinny_kernel(const bf16_t* __restrict__ X, long ldx, const bf16_t* __restr
 // Phase c: wait until this wave's chunk-c DMAs landed, barrier (every wave's X part of chunk c
 // landed AND every wave finished chunk c-1), DMA chunk c+D-1 into slot (c-1)%D, multiply
 // chunk c.  4 waves; wave w DMAs X step w of every m-tile and its own W tiles.
-EIA_DEV void glds16(const void* gsrc, unsigned lds_addr) {
-  unsigned keep;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\t"
-      "s_mov_b32 m0, %2\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %1, off\n\t"
-      "s_mov_b32 m0, %0"
-      : "=&s"(keep)
-      : "v"(gsrc), "s"(__builtin_amdgcn_readfirstlane(lds_addr))
-      : "memory");
-}
-
 template <int N>
 EIA_DEV void wait_vmcnt() {
   static_assert(N >= 0 && N < 64, "vmcnt range");

@@ -34,6 +34,35 @@ def test_grouped_gemm(counts, K, form):
         assert a == b or ((out[a:b].double() - y).norm() / y.norm()) < 3e-3
 
 
+# (mean rows per expert of 16: 256 takes tiles of up to 320 x 128, 360 of up to 256 x 256)
+@pytest.mark.parametrize("form", [0, 1])
+@pytest.mark.parametrize("K", [64, 128, 192, 448])
+@pytest.mark.parametrize("counts", [
+    [1, 63, 64, 65, 319, 320, 321, 129, 193, 640, 641, 0, 256, 511, 130, 443],
+    [1, 64, 255, 256, 257, 511, 512, 513, 129, 193, 769, 0, 321, 383, 640, 956]])
+def test_grouped_gemm_large_tiles(counts, K, form):
+    from enterprise_inference_amd._native import kernels as lib
+    from enterprise_inference_amd.ops._dispatch import ptr, stream
+    assert sum(counts) in (16 * 256, 16 * 360)
+    g = torch.Generator().manual_seed(K + form)
+    E, n, N = len(counts), sum(counts), 2048
+    X = torch.randn(700, K, generator=g).to("cuda", BF)
+    row_idx = torch.randint(0, 700, (n,), generator=g).to("cuda", torch.int32)
+    offs = torch.tensor([0] + counts).cumsum(0).to("cuda", torch.int32)
+    W = (torch.randn(E, N, K, generator=g) * K ** -0.5).to("cuda", BF)
+    out = torch.full((n + 1, N // 2 if form == 1 else N), float("nan"), device="cuda", dtype=BF)
+    assert lib().eia_moe_grouped_gemm(ptr(X), X.stride(0), ptr(row_idx), ptr(W), N, K, E, ptr(offs),
+                                      n, form, ptr(out), out.stride(0), stream(X)) == 0
+    xs = X.double()[row_idx.long()]
+    for e, (a, b) in enumerate(zip(offs.tolist(), offs.tolist()[1:])):
+        y = xs[a:b] @ W[e].double().t()
+        if form == 1:
+            y = torch.nn.functional.silu(y[:, :N // 2]) * y[:, N // 2:]
+        # fp32 sums of K exact products, one bf16 rounding (2^-9) and a fast exponential
+        assert a == b or ((out[a:b].double() - y).norm() / y.norm()) < 3e-3
+    assert out[n:].isnan().all()
+
+
 @pytest.mark.parametrize("T,E,H,I", [(100, 4, 512, 256), (96, 4, 512, 256), (200, 16, 1024, 1024),
                                      (600, 4, 512, 4352)])
 @pytest.mark.parametrize("shift", [0, 4])

@@ -117,3 +117,42 @@ EIA_DEV void glds16(const void* gsrc, unsigned lds_addr) {
 EIA_DEV unsigned lds_offset(const void* p) {
   return (unsigned)(uintptr_t)(__attribute__((address_space(3))) const void*)p;
 }
+
+// Two fp32 numbers as sums of three bf16 ones each, largest part first: 24 bits in three times eight, exact
+// for finite numbers (down to what bf16 holds).  A matrix product of such parts with bf16 operands, or of the
+// six largest pairs of parts, keeps what an fp32 product keeps at 3/16 or 6/16 of its matrix cycles.  Parts
+// of what is not finite are no numbers, so callers look for sums that are not finite and form those anew.
+EIA_DEV void split3(float a, float b, bf16x2& h, bf16x2& m, bf16x2& l) {
+  typedef __attribute__((ext_vector_type(2))) float f32x2_t;
+  auto up = [](bf16x2 v, int i) {
+    const unsigned u = __builtin_bit_cast(unsigned, v);
+    return __uint_as_float(i ? u & 0xffff0000u : u << 16);
+  };
+  h = __builtin_convertvector(f32x2_t{a, b}, bf16x2);
+  const float ra = a - up(h, 0), rb = b - up(h, 1);
+  m = __builtin_convertvector(f32x2_t{ra, rb}, bf16x2);
+  l = __builtin_convertvector(f32x2_t{ra - up(m, 0), rb - up(m, 1)}, bf16x2);
+}
+EIA_DEV void split3(const float (&v)[8], bf16x8 (&part)[3]) {
+#pragma unroll
+  for (int e = 0; e < 8; e += 2) {
+    bf16x2 x[3];
+    split3(v[e], v[e + 1], x[0], x[1], x[2]);
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+      part[p][e] = x[p][0];
+      part[p][e + 1] = x[p][1];
+    }
+  }
+}
+EIA_DEV f32x4 mfma_bf16_k32(bf16x8 a, bf16x8 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+// Transposing reads of LDS: lane l of sixteen names row l / 4, entries 4 (l % 4) .. + 3 of a tile of 4 rows
+// and 16 columns, and receives its column l.  Two tiles: eight rows of a column, an operand of 16x16x32.
+EIA_DEV bf16x8 lds_columns(const bf16_t* p0, const bf16_t* p1) {
+  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+  const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p0);
+  const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p1);
+  return __builtin_bit_cast(bf16x8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
+}

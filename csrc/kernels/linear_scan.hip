@@ -439,16 +439,19 @@ EIA_API int eia_linear_scan(const void* x, long ld, int q_off, int k_off, int v_
 // of mode 1 come from a pre-pass that carries the running maximum, angles of rotated heads from a table.
 // Chunks are found on the device (eia_chunks.h).
 //
-// Products are fp32 matrix-core products, except q . k of unrotated bf16 rows, which is exact in
-// bf16 operands.  128-token chunks: the states between chunks are the larger part of the memory
+// Rows of bf16: all products take bf16 operands, fp32 factors as the sum of three (split3).  Values, and
+// unrotated keys and queries, are exact as they are, so most products are three of 16x16x32 at 3/16 of the matrix
+// cycles that fp32 products took, and none is less precise: S against 64 bits 0.98e-7 .. 2.4e-7 where fp32
+// products left 1.45e-7 .. 2.6e-7 (fewer roundings of the sums).  Rows of fp32, and chunks in which a sum is not
+// finite, which the parts of a split cannot follow, take fp32 products (ls_state_fp32, ls_out_fp32).
+//
+// 128-token chunks: the states between chunks are the larger part of the memory
 // traffic (4 passes over chunks x H x dk x dv floats), and halving their number costs less than the
 // longer sums inside a chunk add.
-// Four prompts of 1000 .. 2000 tokens (6688 rows), 16 heads of 128, mode 1, bf16 take 13 + 57 + 21 +
-// 103 us on an MI355X (gates, (1), (2), (3)); in 32-token chunks of vector FMAs with a thread per state
-// column it was 63 + 151 + 119 + 581 us.  (3) spends 40 us of it in matrix products and 28 us in
-// vector issue; the rest is waiting for reads, which a round of workgroups makes all at its start.
-// The 64 KB state goes through the LDS that the keys and values take after it: read by every wave for
-// itself (3) took 122 us.
+// Four prompts of 1000 .. 2000 tokens (6688 rows), 16 heads of 128, mode 1, bf16 take 13 + 33 + 21 +
+// 63 us on an MI355X (gates, (1), (2), (3)); in fp32 products (1) and (3) took 57 + 103 us.  Bound by the
+// workspace and the rows, which (1), (2) and (3) move at 3.4, 5.3 and 3.1 TB/s, and by the steps of
+// a workgroup, which reads, splits and multiplies in turn.
 constexpr int LK = 128;                     // tokens per chunk
 constexpr float LS_LOG2E = 1.4426950408889634f;
 
@@ -685,19 +688,31 @@ EIA_DEV f32x4 ls_inside(const float* l, int lane) {
   return e;
 }
 
-// (1) Eight waves; wave w forms rows 16 w .. of U.  Tokens come in two halves of 64.  A lane of a
-// product over tokens holds columns 64 x + 4 (lane % 16) + j in tile 4 x + j, here and in (3).
+// What (1) and (3) share of a chunk: its rows and the sums of l in LDS.
+struct LsChunk {
+  int row0, n, h;
+  const float *pre, *suf, *mb, *tot, *sl;
+};
+
+// The weighted key of token tk, channels i .. i + 7: what it adds to the state after the chunk.
+template <typename T, bool VEC, bool ROT>
+EIA_DEV void ls_weighted_key(const ScanArgs& a, const KChunkArgs& c, const LsChunk& k, int tk, int i, float (&v)[8]) {
+  ls_head8<T, VEC, ROT>(a, c, k.row0 + min(tk, k.n - 1), a.k_off + (long)k.h * a.D, i, v);
+  float e = k.mb[tk] + k.suf[tk];
+  for (int b = (tk >> 4) + 1; b < LK / 16; ++b) e += k.tot[b];
+  const float wt = tk < k.n ? a.kscale * __builtin_amdgcn_exp2f(e) : 0.f;
+#pragma unroll
+  for (int x = 0; x < 8; ++x) v[x] = tk < k.n ? v[x] * wt : 0.f;
+}
+
+// U in fp32 products: wave w forms rows 16 w ..  Tokens come in two halves of 64.  A lane of a product over
+// tokens holds columns 64 x + 4 (lane % 16) + j in tile 4 x + j, here and in (3).
 template <typename T, bool VEC, bool ROT, int MX>
-__global__ void __launch_bounds__(512)
-ls_chunk_state_kernel(ScanArgs a, KChunkArgs c) {
-  __shared__ __align__(16) float sk[64 * MX];
-  __shared__ __align__(16) T sv[64 * MX];
-  __shared__ float pre[LK], suf[LK], mb[LK], tot[LK / 16], sl[LK];
-  int s, row0, n;
-  if (!ls_chunk(a, c.nseq, blockIdx.x, s, row0, n)) return;
-  const int h = blockIdx.y, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+EIA_DEV void ls_state_fp32(const ScanArgs& a, const KChunkArgs& c, const LsChunk& k, long at, unsigned char* lds) {
+  float* sk = reinterpret_cast<float*>(lds);
+  T* sv = reinterpret_cast<T*>(sk + 64 * MX);
+  const int row0 = k.row0, n = k.n, h = k.h, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int l16 = lane & 15, g4 = lane >> 4;
-  ls_chunk_logs(a, c, row0, n, h, pre, suf, tot, mb, sl);
   f32x4 acc[MX / 16];
   float un = 0.f;                                      // normaliser row 16 w + l16
 #pragma unroll
@@ -711,14 +726,10 @@ ls_chunk_state_kernel(ScanArgs a, KChunkArgs c) {
     for (int u = threadIdx.x; u < 64 * MX / 8; u += 512) {
       const int t = u / (MX / 8), i = 8 * (u % (MX / 8)), tk = t0 + t;
       float v[8];
-      ls_head8<T, VEC, ROT>(a, c, row0 + min(tk, n - 1), a.k_off + (long)h * a.D, i, v);
-      float e = mb[tk] + suf[tk];
-      for (int b = (tk >> 4) + 1; b < LK / 16; ++b) e += tot[b];
-      const float wt = a.kscale * __builtin_amdgcn_exp2f(e);
+      ls_weighted_key<T, VEC, ROT>(a, c, k, tk, i, v);
 #pragma unroll
       for (int x = 0; x < 8; x += 4)
-        *reinterpret_cast<f32x4*>(sk + tile_at<MX>(t, i + x)) =
-            tk < n ? f32x4{v[x], v[x + 1], v[x + 2], v[x + 3]} * wt : f32x4{0.f, 0.f, 0.f, 0.f};
+        *reinterpret_cast<f32x4*>(sk + tile_at<MX>(t, i + x)) = f32x4{v[x], v[x + 1], v[x + 2], v[x + 3]};
     }
     __syncthreads();
     if (16 * w >= c.DP) continue;
@@ -742,12 +753,6 @@ ls_chunk_state_kernel(ScanArgs a, KChunkArgs c) {
       un += ka[0] + ka[1] + ka[2] + ka[3];
     }
   }
-  const long at = (long)blockIdx.x * a.H + h;
-  if (threadIdx.x == 0) {
-    float g = 0.f;
-    for (int b = 0; b < LK / 16; ++b) g += tot[b];
-    c.G[at] = g;
-  }
   if (16 * w >= c.DP) return;
   float* U = c.U + (at * c.DP + 16 * w + 4 * g4) * c.UW;
 #pragma unroll
@@ -763,6 +768,133 @@ ls_chunk_state_kernel(ScanArgs a, KChunkArgs c) {
     un += __shfl_xor(un, 32, 64);
     if (g4 == 0)
       *reinterpret_cast<f32x4*>(c.U + (at * c.DP + 16 * w + l16) * c.UW + c.VP) = f32x4{un, 0.f, 0.f, 0.f};
+  }
+}
+
+// U in bf16 products, for bf16 rows: the values are operands as they are, the weighted keys in three parts
+// (split3).  Wave (cw, dw) forms MX / 4 rows and MX / 2 columns, U transposed in its registers; the
+// normaliser is the product with ones.  Rows of an LDS tile are 32 bytes more than a multiple of the banks
+// apart, so that the transposing reads of eight rows meet all of them.  false: something was not finite
+// (uniform over the workgroup; nothing was written).
+template <bool VEC, bool ROT, int MX>
+EIA_DEV bool ls_state_bf16(const ScanArgs& a, const KChunkArgs& c, const LsChunk& k, long at, unsigned char* lds) {
+  constexpr int PITCH = MX + 16, PLANE = 64 * PITCH, NA = MX / 32, NB = MX / 64;
+  bf16_t* sk = reinterpret_cast<bf16_t*>(lds);         // [3][64][PITCH]
+  bf16_t* sv = sk + 3 * PLANE;                         // [64][PITCH]
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l16 = lane & 15, g4 = lane >> 4, c0 = MX / 4 * (w & 3), d0 = MX / 2 * (w >> 2);
+  const bool live = c0 < c.DP, norm = a.mode == 1 && d0 == 0;
+  const bf16_t* X = static_cast<const bf16_t*>(a.x) + a.v_off + (long)k.h * a.Dv;
+  bf16x8 ones;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) ones[e] = (bf16_t)1.f;
+  f32x4 acc[NA][NB], un[NB];
+#pragma unroll
+  for (int j = 0; j < NB; ++j) {
+    un[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < NA; ++i) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  for (int t0 = 0; t0 < k.n; t0 += 64) {
+    __syncthreads();                                   // logs are there; the first half was read
+#pragma unroll
+    for (int u = threadIdx.x; u < 64 * MX / 8; u += 512) {
+      const int t = u / (MX / 8), i = 8 * (u % (MX / 8));
+      const bool ok = t0 + t < k.n && i < a.Dv;
+      const bf16_t* p = X + (long)(k.row0 + (ok ? t0 + t : 0)) * a.ld + (ok ? i : 0);
+      bf16x8 v;
+      if constexpr (VEC) {
+        v = *reinterpret_cast<const bf16x8*>(p);
+        if (!ok) v = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = ok && i + e < a.Dv ? p[e] : (bf16_t)0.f;
+      }
+      *reinterpret_cast<bf16x8*>(sv + t * PITCH + i) = v;
+      float kw[8];
+      ls_weighted_key<bf16_t, VEC, ROT>(a, c, k, t0 + t, i, kw);
+      bf16x8 part[3];
+      split3(kw, part);
+#pragma unroll
+      for (int p3 = 0; p3 < 3; ++p3) *reinterpret_cast<bf16x8*>(sk + p3 * PLANE + t * PITCH + i) = part[p3];
+    }
+    __syncthreads();
+    if (!live) continue;
+#pragma unroll
+    for (int b = 0; b < 64; b += 32) {
+      if (t0 + b >= k.n) break;
+      const int at0 = (b + 4 * g4 + (l16 >> 2)) * PITCH + 4 * (l16 & 3);
+      bf16x8 kf[3][NB];
+#pragma unroll
+      for (int p3 = 0; p3 < 3; ++p3)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+          const bf16_t* q = sk + p3 * PLANE + at0 + c0 + 16 * j;
+          kf[p3][j] = lds_columns(q, q + 16 * PITCH);
+        }
+#pragma unroll
+      for (int i = 0; i < NA; ++i) {
+        const bf16_t* q = sv + at0 + d0 + 16 * i;
+        const bf16x8 vf = lds_columns(q, q + 16 * PITCH);
+#pragma unroll
+        for (int p3 = 2; p3 >= 0; --p3)
+#pragma unroll
+          for (int j = 0; j < NB; ++j) acc[i][j] = mfma_bf16_k32(vf, kf[p3][j], acc[i][j]);
+      }
+      if (norm) {
+#pragma unroll
+        for (int p3 = 2; p3 >= 0; --p3)
+#pragma unroll
+          for (int j = 0; j < NB; ++j) un[j] = mfma_bf16_k32(ones, kf[p3][j], un[j]);
+      }
+    }
+  }
+  bool bad = false;
+#pragma unroll
+  for (int j = 0; j < NB; ++j) {
+    bad |= !(fabsf(un[j][0]) < INFINITY);
+#pragma unroll
+    for (int i = 0; i < NA; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) bad |= !(fabsf(acc[i][j][e]) < INFINITY);
+  }
+  if (__syncthreads_or(bad)) return false;
+  if (!live) return true;
+#pragma unroll
+  for (int j = 0; j < NB; ++j) {
+    if (c0 + 16 * j >= c.DP) break;
+    float* U = c.U + (at * c.DP + c0 + 16 * j + l16) * c.UW;
+#pragma unroll
+    for (int i = 0; i < NA; ++i)
+      if (d0 + 16 * i < c.VP) *reinterpret_cast<f32x4*>(U + d0 + 16 * i + 4 * g4) = acc[i][j];
+    if (norm && g4 == 0) *reinterpret_cast<f32x4*>(U + c.VP) = f32x4{un[j][0], 0.f, 0.f, 0.f};
+  }
+  return true;
+}
+
+// (1) Eight waves.
+template <typename T, bool VEC, bool ROT, int MX>
+__global__ void __launch_bounds__(512, 4)
+ls_chunk_state_kernel(ScanArgs a, KChunkArgs c) {
+  constexpr bool BF = sizeof(T) == 2;
+  constexpr int FP32 = 64 * MX * (4 + (int)sizeof(T)), SPLIT = BF ? 4 * 64 * (MX + 16) * 2 : 0;
+  __shared__ __align__(16) unsigned char tiles[FP32 > SPLIT ? FP32 : SPLIT];
+  __shared__ float pre[LK], suf[LK], mb[LK], tot[LK / 16], sl[LK];
+  int s, row0, n;
+  if (!ls_chunk(a, c.nseq, blockIdx.x, s, row0, n)) return;
+  const int h = blockIdx.y;
+  ls_chunk_logs(a, c, row0, n, h, pre, suf, tot, mb, sl);
+  const long at = (long)blockIdx.x * a.H + h;
+  const LsChunk k{row0, n, h, pre, suf, mb, tot, sl};
+  if constexpr (BF) {
+    if (!ls_state_bf16<VEC, ROT, MX>(a, c, k, at, tiles)) ls_state_fp32<T, VEC, ROT, MX>(a, c, k, at, tiles);
+  } else {
+    ls_state_fp32<T, VEC, ROT, MX>(a, c, k, at, tiles);
+  }
+  if (threadIdx.x == 0) {
+    float g = 0.f;
+    for (int b = 0; b < LK / 16; ++b) g += tot[b];
+    c.G[at] = g;
   }
 }
 
@@ -799,25 +931,23 @@ ls_chunk_scan_kernel(ScanArgs a, KChunkArgs c) {
 
 // (3) Eight waves; a wave forms the outputs of 16 tokens.  A later block meets more keys: waves i
 // and i + 4, which share a SIMD, take blocks that add up to the same work.
+//
+// Sums of a wave's queries in fp32 products (o: query 4 (lane / 16) + i, columns as above; rs: this lane's
+// part of the row sum of query lane % 16).
 template <typename T, bool VEC, bool ROT, int MX>
-__global__ void __launch_bounds__(512, 4)
-ls_chunk_out_kernel(ScanArgs a, KChunkArgs c) {
+EIA_DEV void ls_out_fp32(const ScanArgs& a, const KChunkArgs& c, const LsChunk& k, bool state, unsigned char* tiles,
+                         float* sn, f32x4 (&o)[MX / 16], float& rs) {
   // unrotated bf16 keys and queries meet as they are; else both are fp32
   constexpr bool BF = sizeof(T) == 2 && !ROT;
   using KT = typename std::conditional<BF, T, float>::type;
   constexpr bool PRE = BF && VEC;            // keys fetched while the state is used
-  constexpr int KV = LK * MX * (int)(sizeof(KT) + sizeof(T));
-  __shared__ __align__(16) unsigned char tiles[KV > MX * MX * 4 ? KV : MX * MX * 4];
   float* sS = reinterpret_cast<float*>(tiles);         // [MX][MX] the state, then keys and values
   KT* sk = reinterpret_cast<KT*>(tiles);
   T* sv = reinterpret_cast<T*>(sk + LK * MX);
-  __shared__ __align__(16) float pre[LK], suf[LK], mb[LK], sl[LK];
-  __shared__ float tot[LK / 16], sn[MX];
-  int s, row0, n;
-  if (!ls_chunk(a, c.nseq, blockIdx.x, s, row0, n)) return;
-  const int h = blockIdx.y, lane = threadIdx.x & 63, wv = threadIdx.x >> 6, D = a.D, Dv = a.Dv;
+  const int row0 = k.row0, n = k.n, h = k.h, D = a.D;
+  const float *pre = k.pre, *suf = k.suf, *mb = k.mb, *tot = k.tot, *sl = k.sl;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int w = wv < 4 ? wv : 11 - wv, l16 = lane & 15, g4 = lane >> 4, t0 = 16 * w;
-  const bool state = row0 != a.cu[s] || a.positions[a.cu[s]] != 0;   // (else a fresh sequence: S = 0)
   if (state) {                                         // straight to LDS, 1 KB per access
     const float* S = c.U + ((long)blockIdx.x * a.H + h) * c.DP * c.UW;
 #pragma unroll
@@ -831,7 +961,6 @@ ls_chunk_out_kernel(ScanArgs a, KChunkArgs c) {
     if (a.mode == 1 && threadIdx.x < MX)
       sn[threadIdx.x] = S[(long)min((int)threadIdx.x, c.DP - 1) * c.UW + c.VP];
   }
-  ls_chunk_logs(a, c, row0, n, h, pre, suf, tot, mb, sl);
   // this lane's query: channels 32 x + 8 g4 + e
   const int tq = t0 + l16;
   typedef KT KT8 __attribute__((ext_vector_type(8)));
@@ -856,10 +985,9 @@ ls_chunk_out_kernel(ScanArgs a, KChunkArgs c) {
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  f32x4 o[MX / 16];
 #pragma unroll
   for (int j = 0; j < MX / 16; ++j) o[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float rs = 0.f;                                      // row sum of query l16 (this lane's keys)
+  rs = 0.f;
   const float pq = pre[tq];
   if (state && t0 < n) {
     float front = 0.f;                                 // l of the blocks before the query's
@@ -954,6 +1082,254 @@ ls_chunk_out_kernel(ScanArgs a, KChunkArgs c) {
       }
     if (b < w) back += tot[b];
   }
+}
+
+// The same sums in bf16 products, for bf16 rows: rotated queries and keys, the state and the weights P are
+// three parts (split3), all others operands as they are.  The state goes through LDS in halves of 64 rows,
+// split where it is written.  Tile 4 x + j of the sums takes columns 64 x + 4 l + j, which lie together in
+// LDS, so that the transposing reads find them.  false: something was not finite (uniform).
+template <bool VEC, bool ROT, int MX> struct LsOutTiles {
+  static constexpr int NQ = ROT ? 3 : 1, PITCH = MX + 16, SPLANE = 64 * PITCH, KPLANE = LK * MX;
+  static constexpr int S = 3 * SPLANE * 2, KV = (NQ * KPLANE + LK * PITCH) * 2, BYTES = S > KV ? S : KV;
+};
+// Sixteen columns from 16 u on of row r to the places of their tiles.
+template <int MX> EIA_DEV int ls_col16(int u) { return 64 * (u >> 2) + 4 * (u & 3); }
+
+template <bool VEC, bool ROT, int MX>
+EIA_DEV bool ls_out_bf16(const ScanArgs& a, const KChunkArgs& c, const LsChunk& k, bool state, unsigned char* tiles,
+                         const float* sn, f32x4 (&o)[MX / 16], float& rs, float* logs) {
+  using L = LsOutTiles<VEC, ROT, MX>;
+  constexpr int NQ = L::NQ, PITCH = L::PITCH, NX = MX / 32;
+  bf16_t* sS = reinterpret_cast<bf16_t*>(tiles);       // [3][64][PITCH], then keys and values
+  bf16_t* sk = sS;                                     // [NQ][LK][MX]
+  bf16_t* sv = sk + NQ * L::KPLANE;                    // [LK][PITCH]
+  const int row0 = k.row0, n = k.n, h = k.h, D = a.D;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int w = wv < 4 ? wv : 11 - wv, l16 = lane & 15, g4 = lane >> 4, t0 = 16 * w, tq = t0 + l16;
+  const bf16_t* X0 = static_cast<const bf16_t*>(a.x) + (long)row0 * a.ld;
+  // rows 64 x + r of the state, columns 16 u ..: one unit per thread and half
+  const int su = threadIdx.x % (MX / 16), sr = threadIdx.x / (MX / 16);
+  f32x4 sf[4];
+  auto fetch = [&](int x) {
+    if (!state || sr >= 64) return;
+    const float* S = c.U + (((long)blockIdx.x * a.H + h) * c.DP + min(64 * x + sr, c.DP - 1)) * c.UW +
+                     (16 * su < c.VP ? 16 * su : 0);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sf[e] = *reinterpret_cast<const f32x4*>(S + 4 * e);
+  };
+  fetch(0);
+  ls_chunk_logs(a, c, row0, n, h, logs, logs + LK, logs + 4 * LK, logs + 2 * LK, logs + 3 * LK);
+  __syncthreads();
+  bf16x8 qf[NQ][NX];                                   // this lane's query: channels 32 x + 8 g4 + e
+  float nq = 0.f;
+#pragma unroll
+  for (int x = 0; x < NX; ++x) {
+    float v[8];
+    ls_head8<bf16_t, VEC, ROT>(a, c, row0 + min(tq, n - 1), a.q_off + (long)h * D, 32 * x + 8 * g4, v);
+    if constexpr (ROT) {
+      bf16x8 part[3];
+      split3(v, part);
+#pragma unroll
+      for (int p = 0; p < 3; ++p) qf[p][x] = part[p];
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) qf[0][x][e] = (bf16_t)v[e];
+    }
+    if (a.mode == 1 && state) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) nq += v[e] * sn[32 * x + 8 * g4 + e];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < MX / 16; ++j) o[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  rs = 0.f;
+  auto dot = [&](const bf16x8 (&x)[NQ], const bf16x8 (&y)[3], f32x4 z) {       // y in three parts
+    if constexpr (NQ == 3) {
+      z = mfma_bf16_k32(x[0], y[2], z);
+      z = mfma_bf16_k32(x[2], y[0], z);
+      z = mfma_bf16_k32(x[1], y[1], z);
+      z = mfma_bf16_k32(x[0], y[1], z);
+      z = mfma_bf16_k32(x[1], y[0], z);
+    } else {
+      z = mfma_bf16_k32(x[0], y[2], z);
+      z = mfma_bf16_k32(x[0], y[1], z);
+    }
+    return mfma_bf16_k32(x[0], y[0], z);
+  };
+  const float pq = k.pre[tq];
+  if (state) {
+#pragma unroll
+    for (int x = 0; x < MX / 64; ++x) {
+      if (x) __syncthreads();                          // the half before was read
+      if (sr < 64) {
+        const int at = sr * PITCH + (ls_col16<MX>(su) ^ (MX == 128 ? (sr & 8) << 3 : 0));
+        const bool ok = 64 * x + sr < c.DP;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          bf16x2 lo[3], hi[3];
+          split3(ok ? sf[0][j] : 0.f, ok ? sf[1][j] : 0.f, lo[0], lo[1], lo[2]);
+          split3(ok ? sf[2][j] : 0.f, ok ? sf[3][j] : 0.f, hi[0], hi[1], hi[2]);
+#pragma unroll
+          for (int p = 0; p < 3; ++p)
+            *reinterpret_cast<bf16x4*>(sS + p * L::SPLANE + at + 16 * j) = bf16x4{lo[p][0], lo[p][1], hi[p][0], hi[p][1]};
+        }
+      }
+      if (x + 1 < MX / 64) fetch(x + 1);               // (on its way during these products)
+      __syncthreads();
+      if (t0 >= n) continue;
+#pragma unroll
+      for (int y = 0; y < 2; ++y) {
+        if (64 * x + 32 * y >= c.DP) break;
+        bf16x8 qx[NQ];
+#pragma unroll
+        for (int p = 0; p < NQ; ++p) qx[p] = qf[p][2 * x + y];
+        // (rows 8 apart meet the other half of the banks)
+        const int r = (32 * y + 8 * g4 + (l16 >> 2)) * PITCH, turn = MX == 128 ? (g4 & 1) << 6 : 0;
+#pragma unroll
+        for (int j = 0; j < MX / 16; ++j) {
+          bf16x8 sp[3];
+#pragma unroll
+          for (int p = 0; p < 3; ++p) {
+            const bf16_t* q = sS + p * L::SPLANE + r + ((16 * j + 4 * (l16 & 3)) ^ turn);
+            sp[p] = lds_columns(q, q + 4 * PITCH);
+          }
+          o[j] = dot(qx, sp, o[j]);
+        }
+      }
+    }
+    float front = 0.f;                                 // l of the blocks before the query's
+    for (int b = 0; b < w; ++b) front += k.tot[b];
+    const float eq = a.qscale * __builtin_amdgcn_exp2f(pq + front);
+    rs = nq * eq;
+    f32x4 er;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) er[i] = __shfl(eq, 4 * g4 + i, 64);
+#pragma unroll
+    for (int j = 0; j < MX / 16; ++j) o[j] *= er;
+    __syncthreads();                                   // the state was read
+  }
+#pragma unroll
+  for (int u = threadIdx.x; u < LK * MX / 16; u += 512) {          // values: sixteen columns of a row
+    const int t = u / (MX / 16), cu = u % (MX / 16);
+    bf16x8 v0, v1;
+    const bf16_t* p = X0 + (long)min(t, n - 1) * a.ld + a.v_off + (long)h * a.Dv;
+    if constexpr (VEC) {
+      const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+      v0 = *reinterpret_cast<const bf16x8*>(p + (16 * cu < a.Dv ? 16 * cu : 0));
+      v1 = *reinterpret_cast<const bf16x8*>(p + (16 * cu + 8 < a.Dv ? 16 * cu + 8 : 0));
+      if (t >= n || 16 * cu >= a.Dv) v0 = zero;
+      if (t >= n || 16 * cu + 8 >= a.Dv) v1 = zero;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        v0[e] = t < n && 16 * cu + e < a.Dv ? p[16 * cu + e] : (bf16_t)0.f;
+        v1[e] = t < n && 16 * cu + 8 + e < a.Dv ? p[16 * cu + 8 + e] : (bf16_t)0.f;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      *reinterpret_cast<bf16x4*>(sv + t * PITCH + ls_col16<MX>(cu) + 16 * j) = bf16x4{v0[j], v0[4 + j], v1[j], v1[4 + j]};
+  }
+#pragma unroll
+  for (int u = threadIdx.x; u < LK * MX / 8; u += 512) {
+    const int t = u / (MX / 8), i = 8 * (u % (MX / 8));
+    float v[8];
+    ls_head8<bf16_t, VEC, ROT>(a, c, row0 + min(t, n - 1), a.k_off + (long)h * D, i, v);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = t < n ? v[e] : 0.f;
+    if constexpr (ROT) {
+      bf16x8 part[3];
+      split3(v, part);
+#pragma unroll
+      for (int p = 0; p < 3; ++p) *reinterpret_cast<bf16x8*>(sk + p * L::KPLANE + ls_kat<MX, bf16_t>(t, i)) = part[p];
+    } else {
+      bf16x8 b;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) b[e] = (bf16_t)v[e];
+      *reinterpret_cast<bf16x8*>(sk + ls_kat<MX, bf16_t>(t, i)) = b;
+    }
+  }
+  __syncthreads();
+  bool bad = false;
+  if (t0 < n) {
+    const float qk = a.qscale * a.kscale;
+    float back = 0.f;                                  // l from the end of block b to the query's
+    // weights of block b, transposed (keys x queries): their registers are an operand of P v
+    auto weights = [&](int b) {
+      f32x4 p = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int x = 0; x < NX; ++x) {
+        bf16x8 kb[NQ], qx[NQ];
+#pragma unroll
+        for (int y = 0; y < NQ; ++y) {
+          kb[y] = *reinterpret_cast<const bf16x8*>(sk + y * L::KPLANE + ls_kat<MX, bf16_t>(16 * b + l16, 32 * x + 8 * g4));
+          qx[y] = qf[y][x];
+        }
+        if constexpr (ROT) p = dot(kb, qx, p);
+        else p = mfma_bf16_k32(kb[0], qx[0], p);
+      }
+      f32x4 e;
+      if (b == w) e = ls_inside(k.sl + t0, lane);
+      else e = *reinterpret_cast<const f32x4*>(k.suf + 16 * b + 4 * g4) + (pq + back);
+      e += *reinterpret_cast<const f32x4*>(k.mb + 16 * b + 4 * g4);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        p[i] = 16 * b + 4 * g4 + i <= tq ? p[i] * qk * __builtin_amdgcn_exp2f(e[i]) : 0.f;
+        rs += p[i];
+      }
+      if (b < w) back += k.tot[b];
+      return p;
+    };
+    for (int b = w; b >= 0; b -= 2) {                  // two blocks of keys to a product
+      const f32x4 p0 = weights(b), p1 = b ? weights(b - 1) : f32x4{0.f, 0.f, 0.f, 0.f};
+      const float p8[8] = {p0[0], p0[1], p0[2], p0[3], p1[0], p1[1], p1[2], p1[3]};
+      bf16x8 pp[3];
+      split3(p8, pp);
+      const bf16_t* v0 = sv + (16 * b + 4 * g4 + (l16 >> 2)) * PITCH + 4 * (l16 & 3);
+      const bf16_t* v1 = v0 - (b ? 16 * PITCH : 0);
+#pragma unroll
+      for (int j = 0; j < MX / 16; ++j) {
+        const bf16x8 vf = lds_columns(v0 + 16 * j, v1 + 16 * j);
+#pragma unroll
+        for (int p = 2; p >= 0; --p) o[j] = mfma_bf16_k32(pp[p], vf, o[j]);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < MX / 16; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) bad |= !(fabsf(o[j][i]) < INFINITY);
+  }
+  return !__syncthreads_or(bad);
+}
+
+template <typename T, bool VEC, bool ROT, int MX>
+__global__ void __launch_bounds__(512, 4)
+ls_chunk_out_kernel(ScanArgs a, KChunkArgs c) {
+  constexpr bool BF = sizeof(T) == 2;
+  constexpr int KV = LK * MX * ((BF && !ROT ? 2 : 4) + (int)sizeof(T)), FP32 = KV > MX * MX * 4 ? KV : MX * MX * 4;
+  constexpr int SPLIT = BF ? LsOutTiles<VEC, ROT, MX>::BYTES : 0;
+  __shared__ __align__(16) unsigned char tiles[FP32 > SPLIT ? FP32 : SPLIT];
+  __shared__ __align__(16) float logs[4 * LK + LK / 16], sn[MX];
+  float *pre = logs, *suf = logs + LK, *mb = logs + 2 * LK, *sl = logs + 3 * LK, *tot = logs + 4 * LK;
+  int s, row0, n;
+  if (!ls_chunk(a, c.nseq, blockIdx.x, s, row0, n)) return;
+  const int h = blockIdx.y, lane = threadIdx.x & 63, wv = threadIdx.x >> 6, Dv = a.Dv;
+  const int w = wv < 4 ? wv : 11 - wv, l16 = lane & 15, g4 = lane >> 4, t0 = 16 * w;
+  const bool state = row0 != a.cu[s] || a.positions[a.cu[s]] != 0;   // (else a fresh sequence: S = 0)
+  if (state && a.mode == 1 && threadIdx.x < MX)
+    sn[threadIdx.x] = c.U[(((long)blockIdx.x * a.H + h) * c.DP + min((int)threadIdx.x, c.DP - 1)) * c.UW + c.VP];
+  const LsChunk k{row0, n, h, pre, suf, mb, tot, sl};
+  f32x4 o[MX / 16];
+  float rs;
+  if constexpr (BF) {
+    if (!ls_out_bf16<VEC, ROT, MX>(a, c, k, state, tiles, sn, o, rs, logs))
+      ls_out_fp32<T, VEC, ROT, MX>(a, c, k, state, tiles, sn, o, rs);
+  } else {
+    ls_chunk_logs(a, c, row0, n, h, pre, suf, tot, mb, sl);
+    __syncthreads();
+    ls_out_fp32<T, VEC, ROT, MX>(a, c, k, state, tiles, sn, o, rs);
+  }
+  if (t0 >= n) return;
   rs += __shfl_xor(rs, 16, 64);                        // n_t . q_t of query l16
   rs += __shfl_xor(rs, 32, 64);
   const T* X = static_cast<const T*>(a.x);

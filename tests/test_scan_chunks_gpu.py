@@ -94,6 +94,52 @@ def test_linear_chunks(lens, H, D, Dv, mode, rot, half, dtype, monkeypatch):
         assert u is None or _rel(v, u) < 2e-6
 
 
+@pytest.mark.parametrize("mode,rot", [("exp_gates", 0), ("decay", 64)])
+@pytest.mark.parametrize("H,D,Dv", [(2, 128, 128), (2, 64, 64), (2, 72, 40)])
+@pytest.mark.parametrize("where,value", [("v", float("inf")), ("v", float("nan")), ("k", float("-inf")),
+                                         ("q", float("inf")), ("S", float("inf")), ("", 0.0)])
+def test_linear_rows_that_are_not_finite(where, value, H, D, Dv, mode, rot, monkeypatch):
+    """One entry of head 1 that is not finite stays where the recurrence leaves it."""
+    from enterprise_inference_amd.ops import linear_scan as ls
+    monkeypatch.setattr(ls, "FORCE_CHUNKED", True)
+    g = torch.Generator().manual_seed(D + rot)
+    lens, hit = [200, 150], 70                 # row 70 of the first sequence
+    T = sum(lens)
+    cu, pos, slots = _step(lens, [5, 0], False)
+    at = [0, H * D, 2 * H * D, 2 * H * D + H * Dv, 2 * H * (D + Dv), 2 * H * (D + Dv) + H]
+    x = torch.randn(T, at[-1] + H, generator=g)
+    x[:, at[-1]:] += 3.0
+    S0 = torch.randn(2, H, D, Dv, generator=g)
+    if where == "S":
+        S0[slots[0], 1, 3, 5] = value
+    elif where:
+        x[hit, at["qkv".index(where)] + (Dv if where == "v" else D) + 5] = value
+    x = x.to(torch.bfloat16)
+    inv = 10000.0 ** (-torch.arange(rot // 2) / max(1, rot // 2))
+
+    def run(dev):
+        spec = ls.ScanSpec(H, D, Dv, mode, cap=15.0, kscale=D ** -0.5, eps=1e-5, rot_dims=rot, rot_half=True,
+                           inv_freq=inv.to(dev), decay=torch.linspace(0.999, 0.9, H).to(dev))
+        st = ls.ScanState.allocate(2, spec, dev)
+        st.S.copy_(S0)
+        plan = ls.chunk_plan(lens, dev) if dev == "cuda" else None
+        y = ls.linear_scan(x.to(dev), at[0], at[1], at[2], at[3], spec, st, slots.to(dev), cu.to(dev), 2,
+                           pos.to(dev), None, None, at[4], at[5], plan=plan)
+        return y.cpu().double(), st.S.cpu().double()
+
+    (y, S), (z, R) = run("cpu"), run("cuda")
+    live = torch.isfinite(S)
+    assert bool(live.all()) == (where in ("", "q"))
+    assert torch.equal(torch.isfinite(R), live)
+    assert _rel(R[live], S[live]) < 2e-6
+    # outputs of the other head, of the other sequence, and before the row's block of sixteen
+    same = torch.ones(T, H, Dv, dtype=torch.bool)
+    if where:
+        same[0 if where == "S" else hit // 16 * 16:lens[0], 1] = False
+    same = same.view(T, H * Dv)
+    assert torch.isfinite(z[same]).all() and _rel(z[same], y[same]) < 4e-3
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("H,G,D,Dv", [(4, 2, 128, 128), (2, 2, 64, 64), (3, 1, 72, 40),
                                       (2, 1, 16, 120), (2, 2, 112, 6)])

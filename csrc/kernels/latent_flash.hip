@@ -304,21 +304,22 @@ latent_flash_kernel(LatentFlashArgs a) {
   lf_finish<NDV>(a, rw, hh, c0, oacc, m_run, lsum);
 }
 
-// The parts of a row block put together: the workgroups, lanes and registers of the kernel above.
+// The parts of a row block put together: the rows, lanes and registers of the kernel above, a workgroup
+// for each 32 columns of every wave's part (one for all of them, one wave per SIMD that reads part after part:
+// 16.4 instead of 12.2 us for 256 row blocks of up to 5 parts x 69 KB).
 template <int NDV, int KT, int CS>
-__global__ void __launch_bounds__(256, 1)
+__global__ void __launch_bounds__(256)
 latent_flash_merge_kernel(LatentFlashArgs a) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, dt = blockIdx.z;
   const LfRows rw = lf_rows<KT, CS>(a, w, lane & 31);
   if (rw.ntok <= 0) return;
   const int parts = min(a.nparts, (rw.ntile + a.per - 1) / a.per);
   if (parts <= 1 || !rw.live) return;
   float m = -INFINITY, lsum = 0.f;
-  f32x16_t oacc[NDV];
+  f32x16_t oacc[1];
 #pragma unroll
-  for (int dt = 0; dt < NDV; ++dt)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) oacc[dt][i] = 0.f;
+  for (int i = 0; i < 16; ++i) oacc[0][i] = 0.f;
+#pragma unroll 2
   for (int z = 0; z < parts; ++z) {
     const float* x = lf_part(a, z, w, NDV) + 4 * lane;
     const f32x4 ml = *reinterpret_cast<const f32x4*>(x + 4 * NDV * 256);
@@ -327,15 +328,13 @@ latent_flash_merge_kernel(LatentFlashArgs a) {
     m = mn;
     lsum = lsum * w0 + ml[1] * w1;
 #pragma unroll
-    for (int dt = 0; dt < NDV; ++dt)
+    for (int i = 0; i < 4; ++i) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(x + (4 * dt + i) * 256);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const f32x4 v = *reinterpret_cast<const f32x4*>(x + (4 * dt + i) * 256);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) oacc[dt][4 * i + e] = oacc[dt][4 * i + e] * w0 + v[e] * w1;
-      }
+      for (int e = 0; e < 4; ++e) oacc[0][4 * i + e] = oacc[0][4 * i + e] * w0 + v[e] * w1;
+    }
   }
-  lf_finish<NDV>(a, rw, lane >> 5, 32 * NDV * (w % CS), oacc, m, lsum);
+  lf_finish<1>(a, rw, lane >> 5, 32 * (NDV * (w % CS) + dt), oacc, m, lsum);
 }
 
 template <int NK, int NDV, int KT, int WPS, int CS, bool SPLIT>
@@ -347,7 +346,7 @@ static void lf_launch(const LatentFlashArgs& a, dim3 grid, hipStream_t st) {
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(f), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
   hipLaunchKernelGGL(f, grid, dim3(256), bytes, st, a);
   if (SPLIT)
-    hipLaunchKernelGGL((latent_flash_merge_kernel<NDV, KT, CS>), dim3(grid.x, grid.y), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((latent_flash_merge_kernel<NDV, KT, CS>), dim3(grid.x, grid.y, NDV), dim3(256), 0, st, a);
 }
 
 }  // namespace

@@ -91,6 +91,7 @@ EIA_DEV f32x4 mfma_f32_k16(f32x4 a, f32x4 b, f32x4 c) {
 // So the wait covers all of it by itself, whatever the code around it becomes.
 // All results are operands of the one statement: products of an accumulator that were not could be moved
 // behind it.
+template <typename V> EIA_DEV void mfma_settle(V& a) { asm volatile("s_nop 11" : "+v"(a)); }
 template <typename V> EIA_DEV void mfma_settle(V& a, V& b) { asm volatile("s_nop 11" : "+v"(a), "+v"(b)); }
 template <typename V> EIA_DEV void mfma_settle(V (&o)[4]) {
   asm volatile("s_nop 11" : "+v"(o[0]), "+v"(o[1]), "+v"(o[2]), "+v"(o[3]));

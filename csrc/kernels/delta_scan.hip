@@ -10,12 +10,13 @@
 // divided by its root mean square, multiplied by a weight shared by the heads, by silu of its gate
 // columns and by out_scale.
 //
-// q, k, v, la and b arrive as the fp32 rows that delta_prep.hip leaves.  Everything here is fp32, the
-// matrix products included (v_mfma_f32_16x16x4_f32 in the chunk-parallel form).
+// q, k, v, la and b arrive as the fp32 rows that delta_prep.hip leaves.  Everything here keeps fp32; matrix
+// products are fp32 ones or take fp32 factors as sums of bf16 parts.
 //
 // A sequence whose first row of the step is position 0 starts from zeros whatever its slot held, so
 // slots are reused without clearing.  Batch layout: sequence s owns rows [cu[s], cu[s+1])
 // (cu == nullptr: row s).
+#include <type_traits>
 #include "eia_common.h"
 
 EIA_DEV float dl_silu(float z) { return z / (1.0f + expf(-z)); }
@@ -207,504 +208,847 @@ EIA_API int eia_delta_scan(const float* q, const float* k, const float* v, const
 //
 // whose right side is linear in S:  with T = (I + L)^-1,  u = X - Y S,  X = T diag(b) V,
 // Y = T diag(b exp(A)) K.
-//   (1) T, X, Y of every chunk, in parallel (T by 16-token blocks, diagonal inverses first)
+//   (1) T, X, Y and P_ts = exp(A_t - A_s) (q_t . k_s), s <= t, of every chunk, in parallel (T by 16-token
+//       blocks, diagonal inverses first)
 //   (2) a sequence's chunks in order, in parallel over heads and slices of the state's columns:
-//       u = X - Y S (replaces X), S <- exp(A_end) S + sum_t exp(A_end - A_t) k_t u_t^T
-//   (3) outputs of every chunk, in parallel:
-//       o_t = exp(A_t) S^T q_t + sum_(s<=t) exp(A_t - A_s) (q_t . k_s) u_s
-// Every exponent is <= 0.  All products are fp32 matrix-core products (16x16x4): an accumulator's
-// registers (row 4 (lane / 16) + i, column lane % 16) are, step i, the B operand of a product over
-// its rows; an A operand's lane holds four consecutive k of row lane % 16.
+//       u = X - Y S,  o_t = exp(A_t) S^T q_t + sum_s P_ts u_s,  S <- exp(A_end) S + sum_t exp(A_end - A_t) k_t u_t^T
+//   (3) norm, weight and gate of all outputs, in parallel
+// Every exponent is <= 0.
 //
-// Layout.  With row-major workspaces most operands were 4-byte accesses, and issuing them took longer
-// than the products.  So everything that passes between the kernels lies as the lanes of the next
-// product take it, 16 bytes per lane and 1 KB per access: a fragment [64 lanes][4].  The row and
-// column order inside a head is free as long as all products agree, and is chosen so that rows of q, k and v are
-// read 8 or 16 bytes at a time: tile j of a group of 64 holds entries 64 g + 4 x + j; its column r is
-// x = r, its row r (dk only) x = 4 (r % 4) + r / 4, the order in which an A operand's rows are read.
-//   Y  [chunk, H, 4 token tiles, DP tiles]   A operand, rows tokens
-//   X  [chunk, H, 4 token tiles, VP tiles]   B operand, rows tokens (u after the scan)
-//   Kt [chunk, G, DP tiles, 4 token tiles]   A operand, rows dk
-//   S  [chunk, H, DP tiles, VP tiles]        B operand, rows dk
-// with DP and VP rounded up to 64.  MI355X, 16 heads of 128 x 128, three prompts of 750 to 1500
-// tokens: 48 + 77 + 83 us (row-major: 87 + 138 + 129), of which the products alone are 14 + 46 + 26.
+// Layout.  Everything that passes between the kernels lies as the lanes of the next product take it, 16 bytes
+// per lane and 1 KB per access.  A product over 32 rows (16x16x32) takes two tiles of 16, entry e of a
+// lane from row 4 (lane / 16) + e % 4 of tile e / 4: two accumulators are an operand as they are, and so are rows
+// of q 16 bytes at a time.
+// Factors of the scan's products are three bf16 parts each (split3, six products for one: 6/16 of the
+// matrix cycles of fp32 ones, and no less precise), made once where they are formed:
+//   Y  [chunk, H, 4 token tiles, DP / 32, 3 parts]    A operand, rows tokens
+//   Kt [chunk, G, DP / 16 tiles, 2, 3 parts]          A operand, rows dk
+//   Qt [chunk, G, 4 token tiles, DP / 32, 3 parts]    A operand, rows tokens
+//   P  [chunk, H, 6 blocks, 3 parts]                  A operand, rows queries: blocks of 32 keys that queries
+//                                                     of a 16-token tile see, tiles in order (1, 1, 2, 2)
+//   X  [chunk, H, 4 token tiles, VP / 16 tiles]       fp32, B operand, rows tokens
+//   O  [chunk, 64, H, VP]                             fp32, outputs before their norm
+// with DP rounded up to 64 and VP to 32; tile j of 32 columns holds columns 2 x + j.
+// MI355X, 16 heads of 128 x 128, three prompts of 750 to 1500 tokens: 54 + 68 + 21 us
+// ((1), (2), (3)).  Before, with fp32 products and the states between chunks and u in memory for a kernel that formed
+// the outputs, 48 + 77 + 83 (the op: 197 -> 147).  S against 64 bits: 1.2e-7 .. 1.5e-7 where fp32 products left 1.3e-7 .. 1.6e-7.
+// (1) and (3) are bound by their writes and reads (3.4, 3.3 TB/s), (2) by the chain of its chunks: 6000 cycles
+// each, of which matrix products take 2700 of a SIMD's.
 constexpr int DC = 64;                      // tokens per chunk
 constexpr int DL = DC + 4;                  // LDS row pitch of the triangular blocks
 
 struct DeltaChunkArgs {
   const int* chunks;                        // [nchunk, 4]: sequence, first row, tokens, unused
   const int* seq_first;                     // [nseq + 1]: first chunk of every sequence
-  float* Y; float* X; float* Kt; float* wsS;   // fragments, as above (wsS: the state before each chunk)
-  float* cA;                                // [nchunk, H, DC] running sums of la, constant past the end
-  int ncg;                                  // groups of 64 state columns
+  bf16_t *Y, *Kt, *Qt, *P; float *X, *O;    // as above
+  float* cA;                                // [nchunk, H, 2, DC] exp(A_t), exp(A_end - A_t); A constant past the end
+  int ncu, nseq;                            // units of 32 state columns
   int vec;                                  // out, gate and weight rows can be taken 4 at a time
 };
 
 EIA_DEV f32x4 mm(f32x4 a, f32x4 b, f32x4 c) { return mfma_f32_k16(a, b, c); }
-EIA_DEV int dl_row(int r) { return 4 * (r & 3) + (r >> 2); }
 EIA_DEV f32x4 frag(const float* p, long tile, int lane) {
   return *reinterpret_cast<const f32x4*>(p + tile * 256 + 4 * lane);
 }
 EIA_DEV void put_frag(float* p, long tile, int lane, f32x4 v) {
   *reinterpret_cast<f32x4*>(p + tile * 256 + 4 * lane) = v;
 }
+struct Parts { bf16x8 p[3]; };
+// split3 of eight numbers whose parts' sum is the number whatever it is: one that is not finite is its first
+// part, one that rounds out of bf16 is cut instead.
+EIA_DEV void split_whole(const float (&v)[8], Parts& f) {
+  split3(v, f.p);
+  float z = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) z += (float)f.p[2][e];
+  if (__any(!(fabsf(z) < INFINITY))) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      float h = (float)(bf16_t)v[e];
+      if (fabsf(h) == INFINITY) h = __uint_as_float(__float_as_uint(v[e]) & 0xffff0000u);
+      float r = v[e] - h;
+      if (!(fabsf(r) < INFINITY)) r = 0.f;
+      const bf16_t m = (bf16_t)r;
+      f.p[0][e] = (bf16_t)h;
+      f.p[1][e] = m;
+      f.p[2][e] = (bf16_t)(r - (float)m);
+    }
+  }
+}
+// split3 with a cut first part: any finite number, in parts that are finite.  (Y and P that are not finite reach
+// all columns alike, so that it does not matter which such number they become.)
+EIA_DEV void split_cut(const float (&v)[8], Parts& f) {
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float h = __uint_as_float(__float_as_uint(v[e]) & 0xffff0000u), r = v[e] - h;
+    const bf16_t m = (bf16_t)r;
+    f.p[0][e] = (bf16_t)h;
+    f.p[1][e] = m;
+    f.p[2][e] = (bf16_t)(r - (float)m);
+  }
+}
+EIA_DEV void put_parts(bf16_t* p, long block, int lane, f32x4 lo, f32x4 hi) {
+  const float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+  Parts f;
+  split_cut(v, f);
+#pragma unroll
+  for (int i = 0; i < 3; ++i) *reinterpret_cast<bf16x8*>(p + ((block * 3 + i) * 64 + lane) * 8) = f.p[i];
+}
+EIA_DEV Parts parts(const bf16_t* p, long block, int lane) {
+  Parts f;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) f.p[i] = *reinterpret_cast<const bf16x8*>(p + ((block * 3 + i) * 64 + lane) * 8);
+  return f;
+}
+EIA_DEV f32x4 whole(const Parts& f, int half) {        // of a tile of the two
+  f32x4 v;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    v[e] = ((float)f.p[0][4 * half + e] + (float)f.p[1][4 * half + e]) + (float)f.p[2][4 * half + e];
+  return v;
+}
+// The six largest products of parts; what is left out is below 2^-26 of the product.
+template <int N> EIA_DEV void mm6(const Parts& a, const Parts (&b)[N], f32x4 (&c)[N]) {
+  constexpr int pa[6] = {0, 2, 1, 0, 1, 0}, pb[6] = {2, 0, 1, 1, 0, 0};
+#pragma unroll
+  for (int x = 0; x < 6; ++x)
+#pragma unroll
+    for (int j = 0; j < N; ++j) c[j] = mfma_bf16_k32(a.p[pa[x]], b[j].p[pb[x]], c[j]);
+}
+template <int N> EIA_DEV void mm6(const Parts (&a)[N], const Parts& b, f32x4 (&c)[N]) {
+  constexpr int pa[6] = {0, 2, 1, 0, 1, 0}, pb[6] = {2, 0, 1, 1, 0, 0};
+#pragma unroll
+  for (int x = 0; x < 6; ++x)
+#pragma unroll
+    for (int j = 0; j < N; ++j) c[j] = mfma_bf16_k32(a[j].p[pa[x]], b.p[pb[x]], c[j]);
+}
+// A tile's four numbers per lane to their half of an operand in LDS.
+EIA_DEV void put_half(bf16_t* lds, int half, int lane, f32x4 v) {
+  bf16x2 a[3], b[3];
+  split3(v[0], v[1], a[0], a[1], a[2]);
+  split3(v[2], v[3], b[0], b[1], b[2]);
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+    *reinterpret_cast<bf16x4*>(lds + (i * 64 + lane) * 8 + 4 * half) = bf16x4{a[i][0], a[i][1], b[i][0], b[i][1]};
+}
+EIA_DEV bool all_finite(f32x4 v) {
+  bool ok = true;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) ok &= fabsf(v[e]) < INFINITY;
+  return ok;
+}
 
-// (1) one workgroup per (chunk, head).  K is staged in LDS: the triangle takes it by rows, Y by
-// columns.  Y and X are made in units of 32 columns, 8-byte reads; a wave has at most one unit of
-// each, and the rows of v for its unit are on their way from the start.
+// (1) one workgroup per (chunk, key head), its heads in turn.  K is staged in LDS in parts: the triangle and P
+// take it by rows, Y and Kt by columns (transposing reads).  Waves 0 .. 3 form the triangle, its inverse and Y,
+// a token tile each; waves 4 .. 7 meanwhile P, and then X in units of 32 columns.  k . k and q . k are
+// formed once for all heads.  X takes fp32 products: a value that is not finite stays in its column and out
+// of earlier tiles.  (Products of 32 tokens would carry it over: an operand's half that a tile does not meet is
+// zero.)
+constexpr int DHB = 8;                                 // heads whose sums of la are formed at a time
 template <int NDG>                                     // groups of 64 dk
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(512, 4)
 delta_chunk_solve_kernel(DeltaArgs a, DeltaChunkArgs c) {
-  constexpr int KP = 64 * NDG + 4;
-  __shared__ __align__(16) float ks[DC][KP];
+  constexpr int KP = 64 * NDG + 8, PLANE = DC * KP, NK = 2 * NDG;
+  __shared__ __align__(16) bf16_t ks[3 * PLANE];
   __shared__ __align__(16) float Ls[DC][DL];           // -L, then T
-  __shared__ float sA[DC], sb[DC];
-  const int ch = blockIdx.y, h = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  __shared__ __align__(16) float sAs[DHB][DC], sbs[DHB][DC], sfs[DHB][DC];
+  const int ch = blockIdx.y, kh = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), w = wave & 3;
   const int s = c.chunks[4 * ch], row0 = c.chunks[4 * ch + 1], n = c.chunks[4 * ch + 2];
   if (a.slots[s] < 0) return;
-  const int H = a.H, G = a.G, DP = a.DP, VP = a.VP, kh = h / (H / G);
+  const int H = a.H, G = a.G, DP = a.DP, VP = a.VP, rep = H / G;
   const int g4 = lane >> 4, l16 = lane & 15;
   const long ldk = (long)G * DP, ldv = (long)H * VP;
   const float* K = a.k + (long)row0 * ldk + (long)kh * DP;
-  f32x4 kst[4 * NDG];
+  float kst[NDG][8];
 #pragma unroll
-  for (int i = 0; i < 4 * NDG; ++i) {
-    const int e = tid + 256 * i, r = e / (16 * NDG), d = 4 * (e % (16 * NDG));
-    kst[i] = *reinterpret_cast<const f32x4*>(K + min(r, n - 1) * ldk + min(d, DP - 4));
+  for (int i = 0; i < NDG; ++i) {
+    const int e = tid + 512 * i, r = e / (8 * NDG), d = 8 * (e % (8 * NDG));
+    const float* p = K + min(r, n - 1) * ldk + min(d, DP - 8);
+#pragma unroll
+    for (int x = 0; x < 8; x += 4) *reinterpret_cast<f32x4*>(&kst[i][x]) = *reinterpret_cast<const f32x4*>(p + x);
   }
-  const int xu = wave >= 2 * NDG ? wave - 2 * NDG : wave + 4 - 2 * NDG;     // this wave's unit of X
-  const bool hasx = xu < 2 * c.ncg;
-  float2 vf[4][4];
-  if (hasx) {
-    const int col = min(64 * (xu >> 1) + 4 * l16 + 2 * (xu & 1), VP - 2);   // past VP: unused columns
-    const float* V = a.v + (long)row0 * ldv + (long)h * VP + col;
+  f32x4 q[2 * NK];
+  if (wave >= 4) {                                     // q rows of tile w
+    const float* Q = a.q + (long)row0 * ldk + (long)kh * DP + min(16 * w + l16, n - 1) * ldk;
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
+    for (int b = 0; b < 2 * NK; ++b) q[b] = *reinterpret_cast<const f32x4*>(Q + min(16 * b + 4 * g4, DP - 4));
+  }
+#pragma unroll
+  for (int i = 0; i < NDG; ++i) {
+    const int e = tid + 512 * i, r = e / (8 * NDG), d = 8 * (e % (8 * NDG));
+    if (d >= DP) {
+#pragma unroll
+      for (int x = 0; x < 8; ++x) kst[i][x] = 0.f;
+    }
+    Parts f;
+    split_whole(kst[i], f);
+#pragma unroll
+    for (int p = 0; p < 3; ++p) *reinterpret_cast<bf16x8*>(ks + p * PLANE + r * KP + d) = f.p[p];
+  }
+  __syncthreads();
+  auto k_rows = [&](int t, int b) {                    // 32 dk of a token tile's rows, in order
+    Parts f;
+#pragma unroll
+    for (int p = 0; p < 3; ++p) f.p[p] = *reinterpret_cast<const bf16x8*>(ks + p * PLANE + (16 * t + l16) * KP + 32 * b + 8 * g4);
+    return f;
+  };
+  auto k_columns = [&](int x, int b) {                 // dk tile x, tokens of 32 as two tiles' rows
+    Parts f;
+    const bf16_t* p0 = ks + (32 * b + 4 * g4 + (l16 >> 2)) * KP + 16 * x + 4 * (l16 & 3);
+#pragma unroll
+    for (int p = 0; p < 3; ++p) f.p[p] = lds_columns(p0 + p * PLANE, p0 + p * PLANE + 16 * KP);
+    return f;
+  };
+  // the ten blocks of k . k, two or three per wave: block p is row tile t, column tile u; q . k of a wave's
+  // tile (keys by queries)
+  f32x4 raw[4][1];
+  auto block_of = [](int p, int& t, int& u) {
+    t = p >= 6 ? 3 : p >= 3 ? 2 : p >= 1 ? 1 : 0;
+    u = p - t * (t + 1) / 2;
+  };
+  auto weights = [&](auto tile) {                      // (the tile's number is a constant: no branches)
+    constexpr int W = decltype(tile)::value;
+#pragma unroll
+    for (int b = 0; b < NK; ++b) {
+      // (q comes as rows 4 g4 .. of two dk tiles; the keys' 32 dk are read the same way)
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = 32 * b + 16 * (e >> 2) + 4 * g4 < DP ? q[2 * b + (e >> 2)][e & 3] : 0.f;
+      Parts y[1];
+      split_cut(v, y[0]);
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+        *reinterpret_cast<bf16x8*>(c.Qt + ((((((long)ch * G + kh) * 4 + W) * NK + b) * 3 + p) * 64 + lane) * 8) = y[0].p[p];
+#pragma unroll
+      for (int u = 0; u <= W; ++u) {
+        Parts f;
+        const bf16_t* p0 = ks + (16 * u + l16) * KP + 32 * b + 4 * g4;
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+          const bf16x4 lo = *reinterpret_cast<const bf16x4*>(p0 + p * PLANE);
+          const bf16x4 hi = *reinterpret_cast<const bf16x4*>(p0 + p * PLANE + 16);
+          f.p[p] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        }
+        mm6(f, y, raw[u]);
+      }
+    }
+  };
+#pragma unroll
+  for (int u = 0; u < 4; ++u) raw[u][0] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (wave < 4) {
+#pragma unroll
+    for (int x = 0; x < 3; ++x) {
+      int t, u;
+      block_of(min(wave + 4 * x, 9), t, u);
+#pragma unroll
+      for (int b = 0; b < NK; ++b) {
+        const Parts y[1] = {k_rows(u, b)};
+        mm6(k_rows(t, b), y, raw[x]);
+      }
+    }
+  } else if (w == 0) {
+    weights(std::integral_constant<int, 0>());
+  } else if (w == 1) {
+    weights(std::integral_constant<int, 1>());
+  } else if (w == 2) {
+    weights(std::integral_constant<int, 2>());
+  } else {
+    weights(std::integral_constant<int, 3>());
+  }
+  mfma_settle(raw[0][0], raw[1][0]);
+  mfma_settle(raw[2][0], raw[3][0]);
+  if (wave < 4 * NDG) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const Parts f = k_columns(wave, b);
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+        *reinterpret_cast<bf16x8*>(c.Kt + ((((((long)ch * G + kh) * (4 * NDG) + wave) * 2 + b) * 3 + p) * 64 + lane) * 8) = f.p[p];
+    }
+  }
+  int here = lane;
+  for (int x = 0; x < rep; ++x) {
+    asm volatile("" : "+v"(here));                     // (addresses are formed anew: kept for the next head they spill)
+    const int lane = here, g4 = lane >> 4, l16 = lane & 15, h = kh * rep + x;
+    const long hb = (long)ch * H + h;
+    const float *sA = sAs[x % DHB], *sb = sbs[x % DHB], *sf = sfs[x % DHB];
+    const bool hasx = wave >= 4 && w < c.ncu;
+    float2 vf[4][4];
+    if (hasx) {
+      const int col = min(32 * w + 2 * l16, VP - 2);   // past VP: unused columns
+      const float* V = a.v + (long)row0 * ldv + (long)h * VP + col;
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          vf[k][i] = *reinterpret_cast<const float2*>(V + min(16 * k + 4 * g4 + i, n - 1) * ldv);
+    }
+    __syncthreads();                                   // the head before has been read
+    if (x % DHB == 0) {
+      if (x + wave < rep) {                            // running sums of the log decays
+        const int hx = h + wave;
+        const long hbx = (long)ch * H + hx;
+        float la = lane < n ? a.la[(long)(row0 + lane) * H + hx] : 0.f;
+        const float b = lane < n ? a.beta[(long)(row0 + lane) * H + hx] : 0.f;
+#pragma unroll
+        for (int o = 1; o < DC; o <<= 1) {
+          const float up = __shfl_up(la, o, 64);
+          if (lane >= o) la += up;
+        }
+        const float e = expf(la);
+        sAs[wave][lane] = la;
+        sbs[wave][lane] = b;
+        sfs[wave][lane] = b * e;
+        c.cA[hbx * 2 * DC + lane] = e;
+        c.cA[(hbx * 2 + 1) * DC + lane] = expf(__shfl(la, DC - 1, 64) - la);
+      }
+      __syncthreads();
+    }
+    if (wave < 4) {                                    // -L
+#pragma unroll
+      for (int y = 0; y < 3; ++y)
+        if (wave + 4 * y < 10) {
+          int t, u;
+          block_of(wave + 4 * y, t, u);
+          const int tc = 16 * u + l16, t0 = 16 * t + 4 * g4;
+          const f32x4 at = *reinterpret_cast<const f32x4*>(sA + t0), bt = *reinterpret_cast<const f32x4*>(sb + t0);
+          const float ac = sA[tc];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float z = -bt[i] * expf(at[i] - ac) * raw[y][0][i];
+            Ls[t0 + i][tc] = tc < t0 + i ? z : 0.f;
+          }
+        }
+    }
+    __syncthreads();
+    if (wave < 4) {                                    // column l16 of the wave's diagonal inverse
+      float z[16];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        float v = r == l16 ? 1.f : 0.f;
+#pragma unroll
+        for (int u = 0; u < r; ++u) v += Ls[16 * wave + r][16 * wave + u] * z[u];
+        z[r] = v;
+      }
+      if (lane < 16) {                                 // after every lane's reads: one wave, in order
+#pragma unroll
+        for (int r = 0; r < 16; ++r) Ls[16 * wave + r][16 * wave + l16] = z[r];
+      }
+    } else {                                           // P
+      const int tq = 16 * w + l16;
+      const float aq = sA[tq];
+      f32x4 p[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const f32x4 ak = *reinterpret_cast<const f32x4*>(sA + 16 * u + 4 * g4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int tk = 16 * u + 4 * g4 + i;
+          const float z = raw[u][0][i] * expf(aq - ak[i]);
+          p[u][i] = tk <= tq && tk < n ? z : 0.f;
+        }
+      }
+      const long first = hb * 6 + (w < 2 ? w : 2 * w - 2);
+      put_parts(c.P, first, lane, p[0], p[1]);
+      if (w >= 2) put_parts(c.P, first + 1, lane, p[2], p[3]);
+    }
+    __syncthreads();
+    // block column `wave` of T:  T_ij = T_ii sum_(j<=k<i) (-L_ik) T_kj
+    f32x4 tc[4];
+    if (wave < 4) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) tc[0][e] = Ls[16 * wave + 4 * g4 + e][16 * wave + l16];
+#pragma unroll
+      for (int i = 1; i < 4; ++i)
+        if (wave + i < 4) {
+          f32x4 r = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int k = 0; k < i; ++k)
+            r = mm(*reinterpret_cast<const f32x4*>(&Ls[16 * (wave + i) + l16][16 * (wave + k) + 4 * g4]),
+                   tc[k], r);
+          tc[i] = mm(*reinterpret_cast<const f32x4*>(&Ls[16 * (wave + i) + l16][16 * (wave + i) + 4 * g4]),
+                     r, f32x4{0.f, 0.f, 0.f, 0.f});
+          mfma_settle(tc[i]);
+        }
+    }
+    __syncthreads();
+    if (wave < 4) {
+#pragma unroll
+      for (int i = 1; i < 4; ++i)
+        if (wave + i < 4) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) Ls[16 * (wave + i) + 4 * g4 + e][16 * wave + l16] = tc[i][e];
+        }
+    }
+    __syncthreads();
+    if (wave < 4) {                                      // Y^T = K^T (T diag(b exp A))^T, token tile w
+      Parts tp[2][1];
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        float v[8];
+#pragma unroll
+        for (int y = 0; y < 2; ++y) {
+          const int at = 32 * b + 16 * y + 4 * g4;
+          const f32x4 f = *reinterpret_cast<const f32x4*>(&Ls[16 * w + l16][at]) * *reinterpret_cast<const f32x4*>(&sf[at]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[4 * y + e] = 2 * b + y <= w ? f[e] : 0.f;
+        }
+        split_cut(v, tp[b][0]);
+      }
+#pragma unroll
+      for (int d = 0; d < NK; ++d) {
+        f32x4 o[2][1];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          o[j][0] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int b = 0; b < 2; ++b)
+            if (2 * b <= w) {
+              Parts f = k_columns(2 * d + j, b);
+              if (2 * b == w) {                          // (the tile's own 16 tokens alone)
+#pragma unroll
+                for (int p = 0; p < 3; ++p)
+#pragma unroll
+                  for (int e = 4; e < 8; ++e) f.p[p][e] = (bf16_t)0.f;
+              }
+              mm6(f, tp[b], o[j]);
+            }
+        }
+        mfma_settle(o[0][0], o[1][0]);
+        put_parts(c.Y, (hb * 4 + w) * NK + d, lane, o[0][0], o[1][0]);
+      }
+    } else if (hasx) {                                   // X = T diag(b) V
+      f32x4 o[2][4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        f32x4 vt[2];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float f = sb[16 * k + 4 * g4 + i];
+          vt[0][i] = vf[k][i].x * f;
+          vt[1][i] = vf[k][i].y * f;
+        }
+#pragma unroll
+        for (int i = k; i < 4; ++i) {
+          const f32x4 t = *reinterpret_cast<const f32x4*>(&Ls[16 * i + l16][16 * k + 4 * g4]);
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            o[j][i] = mm(t, vt[j], k ? o[j][i] : f32x4{0.f, 0.f, 0.f, 0.f});
+        }
+      }
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        vf[k][i] = *reinterpret_cast<const float2*>(V + min(16 * k + 4 * g4 + i, n - 1) * ldv);
-  }
-  if (wave == 0) {                                     // running sums of the log decays
-    float la = lane < n ? a.la[(long)(row0 + lane) * H + h] : 0.f;
-    const float b = lane < n ? a.beta[(long)(row0 + lane) * H + h] : 0.f;
-#pragma unroll
-    for (int o = 1; o < DC; o <<= 1) {
-      const float up = __shfl_up(la, o, 64);
-      if (lane >= o) la += up;
-    }
-    sA[lane] = la;
-    sb[lane] = b;
-    c.cA[((long)ch * H + h) * DC + lane] = la;
-  }
-#pragma unroll
-  for (int i = 0; i < 4 * NDG; ++i) {
-    const int e = tid + 256 * i, r = e / (16 * NDG), d = 4 * (e % (16 * NDG));
-    *reinterpret_cast<f32x4*>(&ks[r][d]) = d < DP ? kst[i] : f32x4{0.f, 0.f, 0.f, 0.f};
-  }
-  __syncthreads();
-  // the ten blocks of -L, two or three per wave: block p is row tile t, column tile u
-  for (int p = wave; p < 10; p += 4) {
-    const int t = p >= 6 ? 3 : p >= 3 ? 2 : p >= 1 ? 1 : 0, u = p - t * (t + 1) / 2;
-    f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-    for (int b = 0; b < 4 * NDG; ++b)
-      acc[b & 1] = mm(*reinterpret_cast<const f32x4*>(&ks[16 * t + l16][16 * b + 4 * g4]),
-                      *reinterpret_cast<const f32x4*>(&ks[16 * u + l16][16 * b + 4 * g4]), acc[b & 1]);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int tr = 16 * t + 4 * g4 + i, tc = 16 * u + l16;
-      const float z = acc[0][i] + acc[1][i];
-      Ls[tr][tc] = tc < tr ? -sb[tr] * expf(sA[tr] - sA[tc]) * z : 0.f;
-    }
-  }
-  __syncthreads();
-  {                                                    // column l16 of the wave's diagonal inverse
-    float x[16];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      float v = r == l16 ? 1.f : 0.f;
-#pragma unroll
-      for (int u = 0; u < r; ++u) v += Ls[16 * wave + r][16 * wave + u] * x[u];
-      x[r] = v;
-    }
-    if (lane < 16) {                                   // after every lane's reads: one wave, in order
-#pragma unroll
-      for (int r = 0; r < 16; ++r) Ls[16 * wave + r][16 * wave + l16] = x[r];
-    }
-  }
-  __syncthreads();
-  // block column `wave` of T:  T_ij = T_ii sum_(j<=k<i) (-L_ik) T_kj
-  f32x4 tc[4];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) tc[0][e] = Ls[16 * wave + 4 * g4 + e][16 * wave + l16];
-#pragma unroll
-  for (int i = 1; i < 4; ++i)
-    if (wave + i < 4) {
-      f32x4 r = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int k = 0; k < i; ++k)
-        r = mm(*reinterpret_cast<const f32x4*>(&Ls[16 * (wave + i) + l16][16 * (wave + k) + 4 * g4]),
-               tc[k], r);
-      tc[i] = mm(*reinterpret_cast<const f32x4*>(&Ls[16 * (wave + i) + l16][16 * (wave + i) + 4 * g4]),
-                 r, f32x4{0.f, 0.f, 0.f, 0.f});
-    }
-  __syncthreads();
-#pragma unroll
-  for (int i = 1; i < 4; ++i)
-    if (wave + i < 4) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) Ls[16 * (wave + i) + 4 * g4 + e][16 * wave + l16] = tc[i][e];
-    }
-  __syncthreads();
-  f32x4 tf[4][4];                                      // row l16 of token tile i, tokens 16 k + 4 g4 ..
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int k = 0; k <= i; ++k)
-      tf[i][k] = *reinterpret_cast<const f32x4*>(&Ls[16 * i + l16][16 * k + 4 * g4]);
-  const long blk = ((long)ch * H + h) * 4;
-  if (wave < 2 * NDG) {                                // Y^T = (diag(b exp A) K)^T T^T
-    f32x4 o[2][4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      f32x4 kt[2], fs;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int t = 16 * k + 4 * g4 + i;
-        const float f = sb[t] * expf(sA[t]);
-        const int d = 64 * (wave >> 1) + 4 * dl_row(l16) + 2 * (wave & 1);
-        const float2 z = *reinterpret_cast<const float2*>(&ks[t][d]);
-        kt[0][i] = z.x;
-        kt[1][i] = z.y;
-        fs[i] = f;
-      }
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        if (h == kh * (H / G))
-          put_frag(c.Kt, (((long)ch * G + kh) * (4 * NDG) + 2 * wave + j) * 4 + k, lane, kt[j]);
-        kt[j] *= fs;
-      }
-#pragma unroll
-      for (int i = k; i < 4; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j)
-          o[j][i] = mm(kt[j], tf[i][k], k ? o[j][i] : f32x4{0.f, 0.f, 0.f, 0.f});
+          put_frag(c.X, (hb * 4 + i) * (2 * c.ncu) + 2 * w + j, lane, o[j][i]);
     }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-        put_frag(c.Y, (blk + i) * (4 * NDG) + 2 * wave + j, lane, o[j][i]);
-  }
-  if (hasx) {                                          // X = T diag(b) V
-    f32x4 o[2][4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      f32x4 vt[2];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float f = sb[16 * k + 4 * g4 + i];
-        vt[0][i] = vf[k][i].x * f;
-        vt[1][i] = vf[k][i].y * f;
-      }
-#pragma unroll
-      for (int i = k; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          o[j][i] = mm(tf[i][k], vt[j], k ? o[j][i] : f32x4{0.f, 0.f, 0.f, 0.f});
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-        put_frag(c.X, (blk + i) * (4 * c.ncg) + 2 * xu + j, lane, o[j][i]);
   }
 }
 
-// (2) one workgroup per (sequence, head, tile of 16 state columns).  Wave w owns tokens 16 w .. of u and
-// NDG row tiles of the state; u and S pass between the waves through LDS.  The next chunk's operands
-// are fetched between this one's products: issued in one go they held every wave up for 2800 to 6100
-// cycles of the 9400 that a chunk took, 5800 now.  Two tiles per workgroup halve the reads but leave
-// a quarter of the CUs idle here: 93 us instead of 77.
-template <int NDG>
-__global__ void __launch_bounds__(256)
-delta_chunk_scan_kernel(DeltaArgs a, DeltaChunkArgs c) {
-  constexpr int NB = 4 * NDG;                          // row tiles
-  __shared__ __align__(16) f32x4 Ss[NB][64];
-  __shared__ __align__(16) f32x4 Us[4][64];
-  const int s = blockIdx.x, h = blockIdx.y, ct = blockIdx.z;
-  const int tid = threadIdx.x, lane = tid & 63, g4 = lane >> 4, l16 = lane & 15;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int slot = a.slots[s];
-  if (slot < 0) return;
-  const int c0 = c.seq_first[s], c1 = c.seq_first[s + 1];
-  if (c1 <= c0) return;
-  const int H = a.H, G = a.G, D = a.D, Dv = a.Dv, kh = h / (H / G), nct = 4 * c.ncg;
-  const bool fresh = a.positions[c.chunks[4 * c0 + 1]] == 0;
-  const int tile0 = NDG * wave;                        // tiles tile0 .. + NDG - 1, one group's
-  const int d0 = 64 * (tile0 >> 2) + (tile0 & 3);      // entries d0 + 4 x + o
-  const int col = 64 * (ct >> 2) + 4 * l16 + (ct & 3);
-  float* Sg = a.S + ((long)slot * H + h) * D * Dv;
-  f32x4 S[NDG];
-#pragma unroll
-  for (int o = 0; o < NDG; ++o) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = d0 + 4 * (4 * i + g4) + o;
-      S[o][i] = (!fresh && r < D && col < Dv) ? Sg[(long)r * Dv + col] : 0.f;
-    }
-    Ss[tile0 + o][lane] = S[o];
-  }
-  struct Op { f32x4 y[NB], x, k[NDG][4], ca; float ga; };
-  auto load = [&](int ch, Op& p) {
-    const long hb = (long)ch * H + h, gb = (long)ch * G + kh;
-    p.ca = *reinterpret_cast<const f32x4*>(c.cA + hb * DC + 16 * wave + 4 * g4);
-    p.ga = c.cA[hb * DC + DC - 1];
-#pragma unroll
-    for (int b = 0; b < NB; ++b) p.y[b] = frag(c.Y, (hb * 4 + wave) * NB + b, lane);
-    p.x = frag(c.X, (hb * 4 + wave) * nct + ct, lane);
-#pragma unroll
-    for (int o = 0; o < NDG; ++o)
-#pragma unroll
-      for (int t = 0; t < 4; ++t) p.k[o][t] = frag(c.Kt, (gb * NB + tile0 + o) * 4 + t, lane);
-  };
-  auto step = [&](int ch, const Op& p) {
-    const long hb = (long)ch * H + h;
-#pragma unroll
-    for (int o = 0; o < NDG; ++o)                      // the state before the chunk, for the outputs
-      put_frag(c.wsS, (hb * NB + tile0 + o) * nct + ct, lane, S[o]);
-    f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-    for (int b = 0; b < NB; ++b) acc[b & 1] = mm(p.y[b], Ss[b][lane], acc[b & 1]);
-    f32x4 us = p.x - acc[0] - acc[1];
-    put_frag(c.X, (hb * 4 + wave) * nct + ct, lane, us);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) us[i] *= expf(p.ga - p.ca[i]);
-    Us[wave][lane] = us;
-#pragma unroll
-    for (int i = 0; i < NB + 4 * NDG + 3; ++i) {       // one load per product
-      __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-    }
-    __syncthreads();
-    const float eg = expf(p.ga);
-#pragma unroll
-    for (int o = 0; o < NDG; ++o) {
-      f32x4 v[2] = {S[o] * eg, {0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-      for (int tt = 0; tt < 4; ++tt) v[tt & 1] = mm(p.k[o][tt], Us[tt][lane], v[tt & 1]);
-      S[o] = v[0] + v[1];
-      Ss[tile0 + o][lane] = S[o];
-    }
-    __syncthreads();
-  };
-  Op p0, p1;
-  load(c0, p0);
-  __syncthreads();
-  for (int ch = c0; ch < c1; ch += 2) {
-    load(min(ch + 1, c1 - 1), p1);
-    step(ch, p0);
-    if (ch + 1 >= c1) break;
-    load(min(ch + 2, c1 - 1), p0);
-    step(ch + 1, p1);
-  }
+// (2) one workgroup per (sequence, head, 16 NC state columns).  Waves 0 .. 3 carry the state: wave w owns
+// tokens 16 w .. of u and NDG row tiles of S.  Waves 4 .. 7, a half step behind, form the outputs of
+// their 16 tokens from the same S and u while the first four wait for each other, so that neither goes to memory.
+// u and S pass between the waves through LDS, in parts; a chunk has two steps, u and then S.
+// An operand of the next chunk is requested where this chunk's has been used, a whole chunk ahead.
+// 32 columns halve the reads per product, which a workgroup of 16 columns is bound by; 16 give twice the
+// workgroups: dn_columns.  A sum that is not finite, which parts cannot follow, sends the workgroup through
+// delta_scan_fp32: fp32 products from the start.
+template <int NDG, int NC> struct ScanTiles {
+  static constexpr int OP = 3 * 64 * 8;                // one operand, in bf16 numbers
+  static constexpr int S = 2 * NDG * NC * OP, U = 2 * NC * OP;
+  static constexpr int TOTAL = 2 * S + 2 * U;          // S twice, u weighted and not
+};
+// What the waves of (2) share: a group of tiles' state columns is ct0 .. ct0 + NC - 1.
+struct ScanAt {
+  int h, kh, ct0, c0, c1, last, wave, lane;
+  bool fresh;
+  float* Sg;
+  EIA_DEV int rows(int ch) const { return ch + 1 < c1 ? DC : last; }
+};
+
+template <int NDG, int NC>
+EIA_DEV void scan_state(const DeltaArgs& a, const ScanAt& k, f32x4 (&S)[NDG][NC], bool put) {
+  const int g4 = k.lane >> 4, l16 = k.lane & 15, tile0 = NDG * (k.wave & 3);
 #pragma unroll
   for (int o = 0; o < NDG; ++o)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int r = d0 + 4 * (4 * i + g4) + o;
-      if (r < D && col < Dv) Sg[(long)r * Dv + col] = S[o][i];
+      const int r = 16 * (tile0 + o) + 4 * g4 + i;
+#pragma unroll
+      for (int j = 0; j < NC; ++j) {
+        const int ct = k.ct0 + j, col = 32 * (ct >> 1) + 2 * l16 + (ct & 1);
+        const bool in = r < a.D && col < a.Dv;
+        if (put) {
+          if (in) k.Sg[(long)r * a.Dv + col] = S[o][j][i];
+        } else {
+          S[o][j][i] = in && !k.fresh ? k.Sg[(long)r * a.Dv + col] : 0.f;
+        }
+      }
     }
 }
-
-// (3) one workgroup per (chunk, head).  A wave owns one query tile and 64 columns; the waves of the same
-// queries share the weights P through LDS, key tiles in turn.  The state is read once, straight to LDS,
-// while the weights are formed.  Bound by the reads of a round of workgroups, which all come at its start.
-template <typename T, int NDG, int NCG>
-__global__ void __launch_bounds__(256 * NCG)
-delta_chunk_out_kernel(DeltaArgs a, DeltaChunkArgs c) {
-  constexpr int NB = 4 * NDG, NCT = 4 * NCG;
-  __shared__ __align__(16) f32x4 Ss[NB * NCT][64];
-  __shared__ __align__(16) f32x4 Ps[10][64];
-  __shared__ float red[NCG][DC];
-  const int ch = blockIdx.y, h = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int s = c.chunks[4 * ch], row0 = c.chunks[4 * ch + 1], n = c.chunks[4 * ch + 2];
-  if (a.slots[s] < 0) return;
-  const int H = a.H, G = a.G, Dv = a.Dv, DP = a.DP, kh = h / (H / G);
-  const int g4 = lane >> 4, l16 = lane & 15, cg = wave % NCG, qt = wave / NCG;
-  const long ldk = (long)G * DP, hb = (long)ch * H + h;
-  // entries 64 g + 4 (4 i + g4) + j of a row, i = 0 .. 3: the k of tile j's fragment
-  auto rows = [&](const float* base, int tile, f32x4 (&f)[NDG][4]) {
-    const float* p = base + (long)(row0 + min(16 * tile + l16, n - 1)) * ldk + (long)kh * DP;
+template <int NC>
+EIA_DEV void scan_put_out(const DeltaArgs& a, const DeltaChunkArgs& c, const ScanAt& k, int ch, const f32x4 (&o)[NC]) {
+  const int g4 = k.lane >> 4, l16 = k.lane & 15, n = k.rows(ch), VQ = 32 * c.ncu;
 #pragma unroll
-    for (int g = 0; g < NDG; ++g)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const f32x4 z = *reinterpret_cast<const f32x4*>(p + min(64 * g + 16 * i + 4 * g4, DP - 4));
-#pragma unroll
-        for (int j = 0; j < 4; ++j) f[g][j][i] = z[j];
-      }
-  };
-  f32x4 qf[NDG][4], kf[NDG][4];
-  rows(a.q, qt, qf);
-  rows(a.k, cg, kf);
-  const float* cA = c.cA + hb * DC;
-  const int tq = 16 * qt + l16;
-  const float aq = cA[tq];
-  const f32x4 ar = *reinterpret_cast<const f32x4*>(cA + 16 * qt + 4 * g4);
-  f32x4 ak = *reinterpret_cast<const f32x4*>(cA + 16 * cg + 4 * g4);
-  // the state goes to LDS while the weights are formed; nothing reads LDS until it is there
-#pragma unroll
-  for (int t = 0; t < NB; ++t) {
-    const int tile = wave + 4 * NCG * t;
-    __builtin_amdgcn_global_load_lds(
-        (const __attribute__((address_space(1))) void*)(c.wsS + (hb * NB * NCT + tile) * 256 + 4 * lane),
-        (__attribute__((address_space(3))) void*)&Ss[tile][0], 16, 0, 0);
-  }
-  if (DP & 63) {                                       // entries past DP are not the row's
-#pragma unroll
-    for (int g = 0; g < NDG; ++g)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (64 * g + 16 * i + 4 * g4 >= DP) {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) qf[g][j][i] = 0.f;
-        }
-  }
-  // P^T = K Q^T: its registers are the A operand of P u
-  for (int kt = cg; kt <= qt; kt += NCG) {
-    if (kt != cg) {
-      rows(a.k, kt, kf);
-      ak = *reinterpret_cast<const f32x4*>(cA + 16 * kt + 4 * g4);
+  for (int i = 0; i < 4; ++i) {
+    const int t = 16 * (k.wave & 3) + 4 * g4 + i;
+    float* p = c.O + (((long)ch * DC + t) * a.H + k.h) * VQ + 32 * (k.ct0 >> 1) + 2 * l16 + (k.ct0 & 1);
+    if (t < n) {
+      if constexpr (NC == 2) *reinterpret_cast<float2*>(p) = float2{o[0][i], o[1][i]};
+      else *p = o[0][i];
     }
-    f32x4 p[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-    for (int b = 0; b < NB; ++b) p[b & 1] = mm(kf[b >> 2][b & 3], qf[b >> 2][b & 3], p[b & 1]);
-    f32x4 w;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int tk = 16 * kt + 4 * g4 + i;
-      w[i] = tk <= tq && tk < n ? (p[0][i] + p[1][i]) * expf(aq - ak[i]) : 0.f;
-    }
-    Ps[qt * (qt + 1) / 2 + kt][lane] = w;
   }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+template <int NDG, int NC>
+EIA_DEV void delta_scan_fp32(const DeltaArgs& a, const DeltaChunkArgs& c, const ScanAt& k, bf16_t* lds) {
+  constexpr int NB = 4 * NDG;
+  f32x4* Ss = reinterpret_cast<f32x4*>(lds);           // [NB][NC][64]
+  f32x4* Us = Ss + NB * NC * 64;                       // [2][4][NC][64]: weighted, not
+  const int lane = k.lane, g4 = lane >> 4, w = k.wave & 3, nct = 2 * c.ncu;
+  const bool carry = k.wave < 4;
+  f32x4 S[NDG][NC];
+  if (carry) {
+    scan_state<NDG, NC>(a, k, S, false);
+#pragma unroll
+    for (int o = 0; o < NDG; ++o)
+#pragma unroll
+      for (int j = 0; j < NC; ++j) Ss[((NDG * w + o) * NC + j) * 64 + lane] = S[o][j];
+  }
   __syncthreads();
-  f32x4 z[4], o[4];
+  for (int ch = k.c0; ch < k.c1; ++ch) {
+    const long hb = (long)ch * a.H + k.h, gb = (long)ch * a.G + k.kh;
+    const float* cA = c.cA + hb * 2 * DC;
+    const f32x4 ea = *reinterpret_cast<const f32x4*>(cA + 16 * w + 4 * g4);
+    const f32x4 ew = *reinterpret_cast<const f32x4*>(cA + DC + 16 * w + 4 * g4);
+    const float eg = cA[DC - 1];
+    f32x4 o[NC];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) z[j] = frag(c.X, hb * 4 * NCT + 4 * cg + j, lane);
+    for (int j = 0; j < NC; ++j) o[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int j = 0; j < 4; ++j) o[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int b = 0; b < NB; ++b) {
+      const f32x4 f = carry ? whole(parts(c.Y, (hb * 4 + w) * (2 * NDG) + (b >> 1), lane), b & 1)
+                            : whole(parts(c.Qt, (gb * 4 + w) * (2 * NDG) + (b >> 1), lane), b & 1);
 #pragma unroll
-  for (int b = 0; b < NB; ++b)
+      for (int j = 0; j < NC; ++j) o[j] = mm(f, Ss[(b * NC + j) * 64 + lane], o[j]);
+    }
+    if constexpr (NC == 2) mfma_settle(o[0], o[1]);
+    else mfma_settle(o[0]);
+    if (carry) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      o[j] = mm(qf[b >> 2][b & 3], Ss[b * NCT + 4 * cg + j][lane], o[j]);
+      for (int j = 0; j < NC; ++j) {
+        const f32x4 u = frag(c.X, (hb * 4 + w) * nct + k.ct0 + j, lane) - o[j];
+        Us[((4 + w) * NC + j) * 64 + lane] = u;
+        Us[(w * NC + j) * 64 + lane] = u * ew;
+      }
+    } else {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float e = expf(ar[i]);
+      for (int j = 0; j < NC; ++j) o[j] *= ea;
+    }
+    __syncthreads();
+    if (carry) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) o[j][i] *= e;
+      for (int x = 0; x < NDG; ++x) {
+#pragma unroll
+        for (int j = 0; j < NC; ++j) S[x][j] *= eg;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const f32x4 f = whole(parts(c.Kt, (gb * NB + NDG * w + x) * 2 + (t >> 1), lane), t & 1);
+#pragma unroll
+          for (int j = 0; j < NC; ++j) S[x][j] = mm(f, Us[(t * NC + j) * 64 + lane], S[x][j]);
+        }
+#pragma unroll
+        for (int j = 0; j < NC; ++j) Ss[((NDG * w + x) * NC + j) * 64 + lane] = S[x][j];
+      }
+    } else {
+      for (int t = 0; t <= w; ++t) {
+        const f32x4 f = whole(parts(c.P, hb * 6 + (w < 2 ? w : 2 * w - 2 + (t >> 1)), lane), t & 1);
+#pragma unroll
+        for (int j = 0; j < NC; ++j) o[j] = mm(f, Us[((4 + t) * NC + j) * 64 + lane], o[j]);
+        if constexpr (NC == 2) mfma_settle(o[0], o[1]);
+        else mfma_settle(o[0]);
+      }
+      scan_put_out<NC>(a, c, k, ch, o);
+    }
+    __syncthreads();
   }
-  for (int kt = 0; kt <= qt; ++kt) {
-    f32x4 zn[4];
+  if (carry) scan_state<NDG, NC>(a, k, S, true);
+}
+
+template <int NDG, int NC>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+delta_chunk_scan_kernel(DeltaArgs a, DeltaChunkArgs c) {
+  constexpr int NB = 4 * NDG, NK = 2 * NDG;            // row tiles; pairs of them
+  using L = ScanTiles<NDG, NC>;
+  __shared__ __align__(16) bf16_t lds[L::TOTAL];
+  const int tid = threadIdx.x, lane = tid & 63, g4 = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), w = wave & 3;
+  // the column groups of a head meet the same Y and P, the heads of a key head the same Kt and Qt: on one XCD
+  const int nct = 2 * c.ncu, ncg = nct / NC, rep = a.H / a.G, slot8 = blockIdx.x >> 3;
+  const int kv = slot8 / (ncg * rep) * 8 + (blockIdx.x & 7), in = slot8 % (ncg * rep);
+  if (kv >= c.nseq * a.G) return;
+  const int s = kv / a.G, h = kv % a.G * rep + in / ncg, slot = a.slots[s];
+  if (slot < 0) return;
+  const int c0 = c.seq_first[s], c1 = c.seq_first[s + 1];
+  if (c1 <= c0) return;
+  const ScanAt k{h, kv % a.G, in % ncg * NC, c0, c1, c.chunks[4 * c1 - 2], wave, lane,
+                 a.positions[c.chunks[4 * c0 + 1]] == 0, a.S + ((long)slot * a.H + h) * a.D * a.Dv};
+  auto Ss = [&](int buf, int kb, int j) { return lds + buf * L::S + (kb * NC + j) * L::OP; };
+  auto Us = [&](int raw, int kb, int j) { return lds + 2 * L::S + raw * L::U + (kb * NC + j) * L::OP; };
+  auto operands = [&](const bf16_t* p, Parts (&f)[NC]) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) zn[j] = frag(c.X, (hb * 4 + min(kt + 1, qt)) * NCT + 4 * cg + j, lane);
-    const f32x4 w = Ps[qt * (qt + 1) / 2 + kt][lane];
+    for (int j = 0; j < NC; ++j) f[j] = parts(p + j * L::OP, 0, lane);
+  };
+  // stands between reads of LDS and products that do not need them: left alone, the compiler moves each read
+  // to the product that it is for
+  auto in_order = [] { __builtin_amdgcn_sched_barrier(0); };
+  bool bad = false;
+  f32x4 S[NDG][NC];
+  if (wave < 4) {
+    const int tile0 = NDG * w;
+    auto put_state = [&](int buf) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) o[j] = mm(w, z[j], o[j]);
+      for (int o = 0; o < NDG; ++o)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) z[j] = zn[j];
+        for (int j = 0; j < NC; ++j) put_half(Ss(buf, (tile0 + o) >> 1, j), (tile0 + o) & 1, lane, S[o][j]);
+    };
+    Parts y[NK], kt[NDG][2];
+    f32x4 x[NC], ew;
+    float eg;
+    auto load_y = [&](int ch, int b) { y[b] = parts(c.Y, (((long)ch * a.H + h) * 4 + w) * NK + b, lane); };
+    auto load_k = [&](int ch, int o, int b) {
+      kt[o][b] = parts(c.Kt, (((long)ch * a.G + k.kh) * NB + tile0 + o) * 2 + b, lane);
+    };
+    auto load_x = [&](int ch) {
+      const long hb = (long)ch * a.H + h;
+      ew = *reinterpret_cast<const f32x4*>(c.cA + (hb * 2 + 1) * DC + 16 * w + 4 * g4);
+      eg = c.cA[hb * 2 * DC + DC - 1];
+#pragma unroll
+      for (int j = 0; j < NC; ++j) x[j] = frag(c.X, (hb * 4 + w) * nct + k.ct0 + j, lane);
+    };
+#pragma unroll
+    for (int b = 0; b < NK; ++b) load_y(c0, b);
+    load_x(c0);
+#pragma unroll
+    for (int o = 0; o < NDG; ++o)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) load_k(c0, o, b);
+    scan_state<NDG, NC>(a, k, S, false);
+    put_state(0);
+    __syncthreads();
+    for (int ch = c0; ch < c1; ++ch) {
+      const int buf = (ch - c0) & 1, nx = min(ch + 1, c1 - 1);
+      f32x4 acc[2][NC];
+#pragma unroll
+      for (int j = 0; j < NC; ++j) acc[0][j] = acc[1][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      Parts f[2][NC];
+      operands(Ss(buf, 0, 0), f[0]);
+#pragma unroll
+      for (int b = 0; b < NK; ++b) {
+        if (b + 1 < NK) operands(Ss(buf, b + 1, 0), f[(b + 1) & 1]);
+        in_order();
+        mm6(y[b], f[b & 1], acc[b & 1]);
+        load_y(nx, b);
+        in_order();
+      }
+      f32x4 u[NC];
+      const float decay = eg;
+#pragma unroll
+      for (int j = 0; j < NC; ++j) {
+        u[j] = x[j] - acc[0][j] - acc[1][j];
+        put_half(Us(0, w >> 1, j), w & 1, lane, u[j] * ew);
+      }
+      load_x(nx);
+      __syncthreads();
+      operands(Us(0, 0, 0), f[0]);
+      operands(Us(0, 1, 0), f[1]);
+      in_order();
+#pragma unroll
+      for (int o = 0; o < NDG; ++o)
+#pragma unroll
+        for (int j = 0; j < NC; ++j) S[o][j] *= decay;
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int o = 0; o < NDG; ++o) {
+          mm6(kt[o][b], f[b], S[o]);
+          load_k(nx, o, b);
+        }
+#pragma unroll
+      for (int j = 0; j < NC; ++j) put_half(Us(1, w >> 1, j), w & 1, lane, u[j]);
+      put_state(buf ^ 1);
+      __syncthreads();
+    }
+#pragma unroll
+    for (int o = 0; o < NDG; ++o)
+#pragma unroll
+      for (int j = 0; j < NC; ++j) bad |= !all_finite(S[o][j]);
+  } else {
+    f32x4 ea, o[NC];
+    Parts p[2], q[NK];
+    const int blocks = w < 2 ? 1 : 2, first = w < 2 ? w : 2 * w - 2;
+    auto load_q = [&](int ch) {
+#pragma unroll
+      for (int b = 0; b < NK; ++b) q[b] = parts(c.Qt, (((long)ch * a.G + k.kh) * 4 + w) * NK + b, lane);
+      ea = *reinterpret_cast<const f32x4*>(c.cA + ((long)ch * a.H + h) * 2 * DC + 16 * w + 4 * g4);
+    };
+    auto load_p = [&](int ch) {
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+        if (b < blocks) p[b] = parts(c.P, ((long)ch * a.H + h) * 6 + first + b, lane);
+    };
+    auto finish = [&](int ch) {                        // P u, and out with it
+      Parts f[2][NC];
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+        if (b < blocks) operands(Us(1, b, 0), f[b]);
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+        if (b < blocks) mm6(p[b], f[b], o);
+      if constexpr (NC == 2) mfma_settle(o[0], o[1]);
+      else mfma_settle(o[0]);
+#pragma unroll
+      for (int j = 0; j < NC; ++j) bad |= !all_finite(o[j]);
+      scan_put_out<NC>(a, c, k, ch, o);
+    };
+    load_q(c0);
+    __syncthreads();
+    for (int ch = c0; ch < c1; ++ch) {
+      const int buf = (ch - c0) & 1;
+      if (ch > c0) finish(ch - 1);
+      load_p(ch);
+      __syncthreads();
+      f32x4 acc[2][NC];
+#pragma unroll
+      for (int j = 0; j < NC; ++j) acc[0][j] = acc[1][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      Parts f[2][NC];
+      operands(Ss(buf, 0, 0), f[0]);
+#pragma unroll
+      for (int b = 0; b < NK; ++b) {
+        if (b + 1 < NK) operands(Ss(buf, b + 1, 0), f[(b + 1) & 1]);
+        in_order();
+        mm6(q[b], f[b & 1], acc[b & 1]);
+        in_order();
+      }
+#pragma unroll
+      for (int j = 0; j < NC; ++j) o[j] = (acc[0][j] + acc[1][j]) * ea;
+      load_q(min(ch + 1, c1 - 1));
+      __syncthreads();
+    }
+    finish(c1 - 1);
   }
-  // head RMS norm, weight, gate
-  const int col = 64 * cg + 4 * l16;
-  float ss[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    float z = 0.f;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) z += col + j < Dv ? o[j][i] * o[j][i] : 0.f;
-    z += __shfl_xor(z, 1, 64);
-    z += __shfl_xor(z, 2, 64);
-    z += __shfl_xor(z, 4, 64);
-    z += __shfl_xor(z, 8, 64);
-    ss[i] = z;
-    if (NCG == 2 && l16 == 0) red[cg][16 * qt + 4 * g4 + i] = z;
+  if (__syncthreads_or(bad)) {
+    delta_scan_fp32<NDG, NC>(a, c, k, lds);
+    return;
   }
-  if (NCG == 2) __syncthreads();
-  const T* NW = static_cast<const T*>(a.norm_w);
-  const T* GT = static_cast<const T*>(a.g);
-  T* Yo = static_cast<T*>(a.y);
-  if (col >= Dv) return;
-  float nw[4];
+  if (wave < 4) scan_state<NDG, NC>(a, k, S, true);
+}
+
+// (3) Norm, weight and gate of the outputs: LN lanes per token and head, four heads each.  Bound by memory.
+template <typename T, int LN>
+__global__ void __launch_bounds__(256)
+delta_chunk_norm_kernel(DeltaArgs a, DeltaChunkArgs c) {
+  constexpr int NH = 4;
+  const int ch = blockIdx.x, sub = threadIdx.x % LN, t = blockIdx.y * (256 / LN) + threadIdx.x / LN;
+  const int s = c.chunks[4 * ch], row0 = c.chunks[4 * ch + 1], n = c.chunks[4 * ch + 2];
+  if (a.slots[s] < 0 || t >= n) return;
+  const int col = 4 * sub, Dv = a.Dv, VQ = 32 * c.ncu;
+  const long r = row0 + t;
+  f32x4 o[NH];
+  float gv[NH][4], nw[4];
+  const T* GT = static_cast<const T*>(a.g) + r * a.ldg;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) nw[j] = ld_f32<T>(NW, min(col + j, Dv - 1)) * a.out_scale;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int tr = 16 * qt + 4 * g4 + i;
-    if (tr >= n) continue;
-    const float sq = NCG == 2 ? ss[i] + red[NCG - 1 - cg][tr] : ss[i];
-    const float inv = 1.0f / sqrtf(sq / (float)Dv + a.eps);
-    const long r = row0 + tr;
-    const T* gp = GT + r * a.ldg + (long)h * Dv + col;
-    T* yp = Yo + r * a.ldy + (long)h * Dv + col;
+  for (int x = 0; x < NH; ++x) {
+    const int h = min((int)blockIdx.z * NH + x, a.H - 1);
+    o[x] = *reinterpret_cast<const f32x4*>(c.O + (((long)ch * DC + t) * a.H + h) * VQ + min(col, VQ - 4));
     if (c.vec) {
       typedef T T4 __attribute__((ext_vector_type(4)));
-      const T4 gz = *reinterpret_cast<const T4*>(gp);
-      T4 yz;
+      const T4 z = *reinterpret_cast<const T4*>(GT + (long)h * Dv + min(col, Dv - 4));
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const T gj = gz[j];
-        T v;
-        st_f32<T>(&v, 0, o[j][i] * inv * nw[j] * dl_silu(ld_f32<T>(&gj, 0)));
-        yz[j] = v;
+        const T zj = z[j];
+        gv[x][j] = ld_f32<T>(&zj, 0);
       }
-      *reinterpret_cast<T4*>(yp) = yz;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) gv[x][j] = ld_f32<T>(GT, (long)h * Dv + min(col + j, Dv - 1));
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    nw[j] = ld_f32<T>(static_cast<const T*>(a.norm_w), min(col + j, Dv - 1)) * a.out_scale;
+#pragma unroll
+  for (int x = 0; x < NH; ++x) {
+    const int h = (int)blockIdx.z * NH + x;
+    float sq = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) sq += col + j < Dv ? o[x][j] * o[x][j] : 0.f;
+#pragma unroll
+    for (int b = 1; b < LN; b <<= 1) sq += __shfl_xor(sq, b, 64);
+    const float inv = 1.0f / sqrtf(sq / (float)Dv + a.eps);
+    if (h >= a.H || col >= Dv) continue;
+    T* yp = static_cast<T*>(a.y) + r * a.ldy + (long)h * Dv + col;
+    T v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) st_f32<T>(v, j, o[x][j] * inv * nw[j] * dl_silu(gv[x][j]));
+    if (c.vec) {
+      typedef T T4 __attribute__((ext_vector_type(4)));
+      *reinterpret_cast<T4*>(yp) = T4{v[0], v[1], v[2], v[3]};
     } else {
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        if (col + j < Dv) st_f32<T>(yp, j, o[j][i] * inv * nw[j] * dl_silu(ld_f32<T>(gp, j)));
+        if (col + j < Dv) yp[j] = v[j];
     }
   }
 }
 
+// State columns per workgroup of (2), in tiles of 16, for nunit workgroups of 32 columns: 16 while that leaves
+// no CU (256) with two workgroups, 32 beyond.  Heads of 128, the whole op in us with 16 / 32 columns: 64
+// workgroups of 32 (one prompt of 4096 tokens, 16 heads) 186 / 216, 128 (two of 1500) 105 / 113, 192 (three)
+// 146 / 130, 256 (four of 1024) 123 / 108, 1024 (sixteen of 256) 145 / 119; heads of 64: 128 54 / 57, 192 128 / 118.
+static int dn_columns(int nunit) { return nunit > 128 ? 2 : 1; }
+
 // As eia_delta_scan for sequences whose chunk list is given (chunks int32 [nchunk, 4]: sequence,
-// first row, tokens (1 .. 64), 0; seq_first int32 [nseq + 1], indexed by sequence), with fp32
-// workspaces Y [nchunk, H, 64, DQ], X [nchunk, H, 64, VQ], Kt [nchunk, G, DQ, 64], wsS [nchunk, H, DQ,
-// VQ], cA [nchunk, H, 64], 16-byte aligned; DP and VP multiples of 16, at most 128, DQ and VQ the
-// same rounded up to 64.
+// first row, tokens (64, of a sequence's last chunk 1 .. 64), 0; seq_first int32 [nseq + 1], indexed by sequence), with workspaces,
+// 16-byte aligned: bf16 Y [nchunk, H, 64, DQ, 3], Kt and Qt [nchunk, G, DQ, 64, 3], P [nchunk, H, 6, 3, 512], fp32
+// X [nchunk, H, 64, VQ], O [nchunk, 64, H, VQ], cA [nchunk, H, 2, 64]; DP and VP multiples of 16, at most
+// 128; DQ: DP rounded up to 64, VQ: VP rounded up to 32.
 EIA_API int eia_delta_scan_chunked(const float* q, const float* k, const float* v, const float* la,
                                    const float* beta, int H, int G, int D, int Dv, int DP, int VP,
                                    const void* g, long ldg, const void* norm_w, float out_scale,
                                    float eps, float* S, const int* slots, const int* positions,
                                    void* y, long ldy, int nseq, const int* chunks,
-                                   const int* seq_first, int nchunk, float* Y, float* X, float* Kt,
-                                   float* wsS, float* cA, int is_bf16, hipStream_t st) {
+                                   const int* seq_first, int nchunk, void* Y, void* Kt, void* Qt, void* P,
+                                   float* X, float* O, float* cA, int is_bf16, hipStream_t st) {
   DeltaArgs a{q, k, v, la, beta, H, G, D, Dv, DP, VP, g, ldg, norm_w, out_scale, eps, S, slots,
               nullptr, positions, nullptr, y, ldy};
-  if (!delta_args_ok(a, nseq) || nchunk < 0 || !chunks || !seq_first || !Y || !X || !Kt || !wsS || !cA ||
+  if (!delta_args_ok(a, nseq) || nchunk < 0 || !chunks || !seq_first || !Y || !X || !Kt || !Qt || !P || !O || !cA ||
       DP % 16 || VP % 16)
     return EIA_BAD_SHAPE;
   if (DP > 128 || VP > 128) return EIA_UNSUPPORTED;
   if (nseq == 0 || nchunk == 0) return EIA_OK;
-  const int ndg = (DP + 63) / 64, ncg = (VP + 63) / 64, es = is_bf16 ? 2 : 4;
+  const int ndg = (DP + 63) / 64, ncu = (VP + 31) / 32, es = is_bf16 ? 2 : 4;
   const bool vec = Dv % 4 == 0 && ldy % 4 == 0 && ldg % 4 == 0 &&
                    (reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(g)) % (4 * es) == 0;
-  DeltaChunkArgs c{chunks, seq_first, Y, X, Kt, wsS, cA, ncg, vec};
-  const dim3 gc(H, nchunk), b(256);
-#define DO_GO(TT, A, B) \
-  hipLaunchKernelGGL((delta_chunk_out_kernel<TT, A, B>), gc, dim3(256 * B), 0, st, a, c)
-#define DO_DIMS(A, B)                                                                              \
+  DeltaChunkArgs c{chunks, seq_first, static_cast<bf16_t*>(Y), static_cast<bf16_t*>(Kt), static_cast<bf16_t*>(Qt),
+                   static_cast<bf16_t*>(P), X, O, cA, ncu, nseq, vec};
+  const dim3 gc(G, nchunk), b(256);
+  const int groups = (nseq * G + 7) / 8 * 8 * (H / G);         // of columns
+  const int nc = dn_columns(nseq * H * ncu);
+#define DO_SCAN(A, C) \
+  hipLaunchKernelGGL((delta_chunk_scan_kernel<A, C>), dim3(groups * (2 * ncu / C)), dim3(512), 0, st, a, c)
+#define DO_DIMS(A)                                                                                 \
   do {                                                                                             \
-    hipLaunchKernelGGL(delta_chunk_solve_kernel<A>, gc, b, 0, st, a, c);                           \
-    hipLaunchKernelGGL(delta_chunk_scan_kernel<A>, dim3(nseq, H, 4 * ncg), b, 0, st, a, c);        \
-    if (is_bf16) DO_GO(bf16_t, A, B); else DO_GO(float, A, B);                                     \
+    hipLaunchKernelGGL(delta_chunk_solve_kernel<A>, gc, dim3(512), 0, st, a, c);                           \
+    if (nc == 2) DO_SCAN(A, 2); else DO_SCAN(A, 1);                                                \
   } while (0)
-  if (ndg == 2) { if (ncg == 2) DO_DIMS(2, 2); else DO_DIMS(2, 1); }
-  else { if (ncg == 2) DO_DIMS(1, 2); else DO_DIMS(1, 1); }
+#define DO_NORM(TT, LN)                                                                            \
+  hipLaunchKernelGGL((delta_chunk_norm_kernel<TT, LN>), dim3(nchunk, DC * LN / 256, (H + 3) / 4), b, 0, st, a, c)
+  if (ndg == 2) DO_DIMS(2); else DO_DIMS(1);
+  if (is_bf16) { if (VP > 64) DO_NORM(bf16_t, 32); else DO_NORM(bf16_t, 16); }
+  else { if (VP > 64) DO_NORM(float, 32); else DO_NORM(float, 16); }
+#undef DO_NORM
 #undef DO_DIMS
-#undef DO_GO
+#undef DO_SCAN
   EIA_LAUNCH_CHECK();
 }

@@ -95,7 +95,7 @@ _SIGNATURES = {
     "eia_delta_scan": [P, P, P, P, P, I, I, I, I, I, I, P, L, P, F, F, P, IP, IP, IP, IP, P, L, I, I,
                        S],
     "eia_delta_scan_chunked": [P, P, P, P, P, I, I, I, I, I, I, P, L, P, F, F, P, IP, IP, P, L, I, IP,
-                               IP, I, P, P, P, P, P, I, S],
+                               IP, I, P, P, P, P, P, P, P, I, S],
     "eia_moe_combine_postnorm": [P, L, P, P, I, P, L, P, F, P, P, L, I, I, I, S],
     "eia_gnorm": [P, L, P, I, P, P, P, P, P, P, L, F, I, I, I, I, S],
     "eia_splitk_act_and_mul": [P, I, I, I, P, L, I, S],

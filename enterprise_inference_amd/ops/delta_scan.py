@@ -345,11 +345,13 @@ def delta_scan(rows: DeltaRows, spec: DeltaSpec, state: DeltaState, md, norm_w: 
     step(0, nd)
     dev = out.device
     f32 = lambda *s: torch.empty(*s, dtype=torch.float32, device=dev)
-    DQ, VQ, n = -(-DP // 64) * 64, -(-VP // 64) * 64, plan.n
-    Y, X = f32(n, H, CHUNK, DQ), f32(n, H, CHUNK, VQ)
-    Kt, wsS, cA = f32(n, G, DQ, CHUNK), f32(n, H, DQ, VQ), f32(n, H, CHUNK)
+    b16 = lambda *s: torch.empty(*s, dtype=torch.bfloat16, device=dev)
+    DQ, VQ, n = -(-DP // 64) * 64, -(-VP // 32) * 32, plan.n
+    Y, P = b16(n, H, CHUNK, DQ, 3), b16(n, H, 6, 3, 512)
+    Kt, Qt = b16(n, G, DQ, CHUNK, 3), b16(n, G, CHUNK, DQ, 3)
+    X, O, cA = f32(n, H, CHUNK, VQ), f32(n, CHUNK, H, VQ), f32(n, H, 2, CHUNK)
     check(lib().eia_delta_scan_chunked(
         *common, ptr(md.seq_slots[nd:]), ptr(md.positions), ptr(out), out.stride(0), plan.nseq,
-        ptr(plan.chunks), ptr(plan.seq_first), n, ptr(Y), ptr(X), ptr(Kt), ptr(wsS),
-        ptr(cA), 1 if bf else 0, stream(out)), "delta_scan_chunked")
+        ptr(plan.chunks), ptr(plan.seq_first), n, ptr(Y), ptr(Kt), ptr(Qt), ptr(P), ptr(X), ptr(O), ptr(cA),
+        1 if bf else 0, stream(out)), "delta_scan_chunked")
     return out

@@ -145,6 +145,24 @@ def test_linear_rows_that_are_not_finite(where, value, H, D, Dv, mode, rot, monk
                                       (2, 1, 16, 120), (2, 2, 112, 6)])
 @pytest.mark.parametrize("lens", [[1, 64, 63, 65, 130], [200], [15, 16, 17, 129, 3]])
 def test_delta_chunks(lens, H, G, D, Dv, dtype, monkeypatch):
+    y, S, z, Z, live = _delta_chunks(lens, H, G, D, Dv, dtype, monkeypatch)
+    # fp32 sums over at most 128 products and a 64-row triangular solve; bf16 adds one rounding and
+    # at times one step more
+    assert _rel(z[live], y[live]) < (1e-5 if dtype == torch.float32 else 4e-3)
+    assert _rel(Z, S) < 4e-6
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("lens,H,G,D,Dv", [([1, 64, 63, 65, 130], 16, 4, 128, 128), ([70] * 9, 8, 8, 64, 120),
+                                           ([129, 150, 1, 16], 18, 2, 40, 64), ([65] * 8, 9, 9, 128, 33)])
+def test_delta_chunks_many_heads(lens, H, G, D, Dv, dtype, monkeypatch):
+    """More columns than CUs: 32 a workgroup; and more than eight heads to a key head."""
+    y, S, z, Z, live = _delta_chunks(lens, H, G, D, Dv, dtype, monkeypatch)
+    assert _rel(z[live], y[live]) < (1e-5 if dtype == torch.float32 else 4e-3)      # as above
+    assert _rel(Z, S) < 4e-6
+
+
+def _delta_chunks(lens, H, G, D, Dv, dtype, monkeypatch, plant=lambda rows, S: None):
     from types import SimpleNamespace
     from enterprise_inference_amd.ops import delta_scan as ds
     monkeypatch.setattr(ds, "FORCE_CHUNKED", True)
@@ -158,6 +176,7 @@ def test_delta_chunks(lens, H, G, D, Dv, dtype, monkeypatch):
             -torch.rand(T, H, generator=g) ** 4, torch.sigmoid(2.0 * rnd(T, H)),
             rnd(T, H * Dv).to(dtype)]
     S0, nw = rnd(n, H, D, Dv), (1 + 0.1 * rnd(Dv)).to(dtype)
+    plant(rows, S0)
 
     def run(dev):
         md = SimpleNamespace(seq_cu=cu.to(dev), seq_slots=slots.to(dev), positions=pos.to(dev),
@@ -173,10 +192,33 @@ def test_delta_chunks(lens, H, G, D, Dv, dtype, monkeypatch):
 
     (y, S), (z, Z) = run("cpu"), run("cuda")
     live = torch.cat([torch.full((m,), int(s) >= 0) for m, s in zip(lens, slots)])
-    # fp32 sums over at most 128 products and a 64-row triangular solve; bf16 adds one rounding and
-    # at times one step more
-    assert _rel(z[live], y[live]) < (1e-5 if dtype == torch.float32 else 4e-3)
-    assert _rel(Z, S) < 4e-6
+    return y, S, z, Z, live
+
+
+@pytest.mark.parametrize("H,G,D,Dv", [(4, 2, 128, 128), (3, 3, 64, 72), (32, 8, 128, 128)])
+@pytest.mark.parametrize("where,value", [("v", float("inf")), ("v", float("nan")), ("k", float("nan")),
+                                         ("q", float("inf")), ("q", float("nan")), ("S", float("-inf")),
+                                         ("v", 3.4e38), ("", 0.0)])
+def test_delta_rows_that_are_not_finite(where, value, H, G, D, Dv, monkeypatch):
+    """One entry of the last (key) head that is not finite stays where the recurrence leaves it."""
+    lens, hit = [150, 200], 70                 # row 70 of the second sequence, past that which is its state's
+
+    def plant(rows, S):
+        if where == "S":
+            S[0, H - 1, 3, 5] = value          # (slots run backwards)
+        elif where:
+            rows["qkv".index(where)][lens[0] + hit, -1, 5] = value
+
+    y, S, z, Z, _ = _delta_chunks(lens, H, G, D, Dv, torch.bfloat16, monkeypatch, plant)
+    fine, ok = torch.isfinite(S), torch.isfinite(y) & torch.isfinite(z)
+    assert torch.equal(torch.isfinite(Z), fine)
+    assert _rel(z[ok], y[ok]) < 4e-3 and _rel(Z[fine], S[fine]) < 4e-6              # as above
+    first = H - (1 if where in ("v", "S") else H // G)                  # heads that meet it
+    same = torch.ones(sum(lens), H, Dv, dtype=torch.bool)
+    if where:                                                           # (products take 16 tokens at a time)
+        lo = lens[0] + (0 if where == "S" else hit if where == "q" else hit // 16 * 16)
+        same[lo:lo + 1 if where == "q" else None, first:] = False
+    assert torch.isfinite(z)[same.view(sum(lens), H * Dv)].all()
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])

@@ -50,12 +50,12 @@ struct GroupedArgs {
 };
 
 // One tile: MU x 64 rows from row m0 of the slice [rb, rb + rows) of expert weights We, N tile n_tile.
-template <bool SWIGLU, int MU, int NU, int MAXMU>
+template <bool SWIGLU, int MU, int NU, int MAXMU, bool FRONT>
 EIA_DEV void grouped_tile(const GroupedArgs& a, bf16_t* lds, const bf16_t* We, int rb, int rows, int m0,
                           int n_tile) {
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r32 = lane & 31, h = lane >> 5;
-  // Access i of a step stands behind product i * RATE.  Small tiles wait for memory rather than for the
+  // Access i of a step stands behind product i * RATE, with FRONT before all products.  Small tiles wait for memory rather than for the
   // access path: 8 experts of 4096 x 14336, 64 rows, gate_up 346 us (RATE 2: 366, 8 of 1024 x 512, 512 rows
   // 19.6 against 17.7); a step of large ones with all accesses in front stalls its first products.
   constexpr int RATE = MU == 1 || MU * NU <= 4 ? 1 : 2;
@@ -173,11 +173,15 @@ EIA_DEV void grouped_tile(const GroupedArgs& a, bf16_t* lds, const bf16_t* We, i
   auto advance = [&](int kt, auto fx, auto fw) {
     const int xs = kt & 1, wn1 = ws + 1 < WS ? ws + 1 : 0;
     arrive(fx);
+    if constexpr (FRONT) {
+      if (fx) all_x(kt + 2, xs);
+      if (fw) all_w(kt + 3, ws);
+    }
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       frags(q, xs ^ 1, wn1);
       __builtin_amdgcn_sched_barrier(0);                   // the next fragments before these products
-      products((q + 3) & 3, q * NU * MU, fx, kt + 2, xs, fw, kt + 3, ws);
+      products((q + 3) & 3, q * NU * MU, fx && !FRONT, kt + 2, xs, fw && !FRONT, kt + 3, ws);
     }
     ws = wn1;
   };
@@ -215,10 +219,10 @@ EIA_DEV void grouped_tile(const GroupedArgs& a, bf16_t* lds, const bf16_t* We, i
   }
 }
 
-template <bool SWIGLU, int NU, int MAXMU, int OCC>
+template <bool SWIGLU, int NU, int MAXMU, int OCC, bool FRONT>
 __global__ void __launch_bounds__(256, OCC)
 moe_grouped_mfma_kernel(GroupedArgs a) {
-  extern __shared__ __align__(16) bf16_t lds[];
+  __shared__ __align__(16) bf16_t lds[(XS * MAXMU + WS * NU) * UNIT];
   const int lane = threadIdx.x & 63, E = a.E, NT = a.NT;
   auto tiles = [&](int e) {                                // M tiles of expert e
     return e < E ? (a.offs[e + 1] - a.offs[e] + 64 * MAXMU - 1) / (64 * MAXMU) : 0;
@@ -266,9 +270,11 @@ moe_grouped_mfma_kernel(GroupedArgs a) {
   const int units = (rows + 63) / 64, lo = units * m_tile / m_tiles, mu = units * (m_tile + 1) / m_tiles - lo;
 #define GG_TILE(M)                                                                            \
   case M:                                                                                     \
-    if constexpr (M <= MAXMU) grouped_tile<SWIGLU, M, NU, MAXMU>(a, lds, We, rb, rows, 64 * lo, n_tile); \
+    if constexpr (M <= MAXMU) grouped_tile<SWIGLU, M, NU, MAXMU, FRONT>(a, lds, We, rb, rows, 64 * lo, n_tile); \
     break
-  switch (mu) { GG_TILE(1); GG_TILE(2); GG_TILE(3); GG_TILE(4); GG_TILE(5); }
+  // long K loops of 64 rows fall behind those of 128 (8 experts of 4096 x 14336, 55 rows: the op 533 us, and
+  // 528), short ones do not (16 of 2048 x 1024, 50 rows: 60.8, and 63.8)
+  switch (FRONT && a.K > 2048 ? max(mu, 2) : mu) { GG_TILE(1); GG_TILE(2); GG_TILE(3); GG_TILE(4); GG_TILE(5); }
 #undef GG_TILE
 }
 
@@ -320,19 +326,25 @@ EIA_API int eia_moe_grouped_gemm(const void* X, long ldx, const int* row_idx, co
   if (swiglu ? (N % 2 != 0 || (N / 2) % 64 != 0) : (N % 128 != 0)) return EIA_BAD_SHAPE;
   if (max_rows <= 0) return EIA_OK;
   const int form = grouped_form((float)max_rows / E, E, N, K);
-#define GG_GO(SW, NU, MM, OCC)                                                                      \
+  // Up to 128 rows an expert, its weights take longer from memory than its products: the sooner a step asks, the
+  // better, while beyond it holds the products up.  The op, spread / in front, us, cold weights: 8 experts of 4096 x
+  // 14336, 64 rows 558 / 545; 16 of 2048 x 1024, 112 rows 70.6 / 69.8; 8 of 1024 x 512, 512 rows (form 0) 44.5 / 47.7.
+  const bool front = max_rows <= 128L * E;
+#define GG_GO(SW, NU, MM, OCC, FRONT)                                                               \
   do {                                                                                              \
-    constexpr int BYTES = (XS * MM + WS * NU) * UNIT * 2;                                           \
     const int nt = N / (64 * NU);                                                                   \
     GroupedArgs a{(const bf16_t*)X, ldx, row_idx, (const bf16_t*)W, (long)N * K, offs, E, N / 2, K, \
                   nt, (bf16_t*)out, ldo, relu2};                                                    \
     const dim3 grid((unsigned)((((max_rows + 64 * MM - 1) / (64 * MM) + E) * (long)nt + 7) / 8 * 8)); \
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(moe_grouped_mfma_kernel<SW, NU, MM, OCC>), \
-                              hipFuncAttributeMaxDynamicSharedMemorySize, BYTES);                   \
-    hipLaunchKernelGGL((moe_grouped_mfma_kernel<SW, NU, MM, OCC>), grid, dim3(256), BYTES, st, a);  \
+    hipLaunchKernelGGL((moe_grouped_mfma_kernel<SW, NU, MM, OCC, FRONT>), grid, dim3(256), 0, st, a);      \
   } while (0)
 #define GG_FORM(SW) \
-  do { if (form == 0) GG_GO(SW, 2, 2, 2); else if (form == 1) GG_GO(SW, 2, 5, 1); else GG_GO(SW, 4, 4, 1); } while (0)
+  do {                                                                                              \
+    if (form == 0 && front) GG_GO(SW, 2, 2, 2, true);                                               \
+    else if (form == 0) GG_GO(SW, 2, 2, 2, false);                                                  \
+    else if (form == 1) GG_GO(SW, 2, 5, 1, false);                                                  \
+    else GG_GO(SW, 4, 4, 1, false);                                                                 \
+  } while (0)
   if (swiglu) GG_FORM(true); else GG_FORM(false);
 #undef GG_FORM
 #undef GG_GO

@@ -11,8 +11,9 @@
 // bf16 high part plus a remainder, normaliser over the fp32 values, deferred rescale.  Rows of an LDS
 // tile are an odd number of 16-byte units apart, so that sixteen rows lie on different banks.
 //
-// MI355X, one 4096-token causal prompt: 8 heads, R 128 + 32: 103 us in parts (141 uncut, 290 before);
-// 8 heads, R 256 + 64: 298 (579); 16 heads, R 512 + 64: 1102 (2117), with a window of 1024 573 (1039).
+// MI355X, one 4096-token causal prompt: 8 heads, R 128 + 32: 79 + 12 us in parts; 8 heads, R 256 + 64: 248 us; 16
+// heads, R 512 + 64: 915, with a window of 1024 488.  With the page of a tile looked up by its fetch, every read of LDS in
+// front of its product and no priorities 86 + 12, 299, 1100 and 573 us.
 // A wave's registers hold the sums of 32 rows over 256 columns beside its queries only alone on its
 // SIMD; at R 512 two waves share the rows and form the same scores (one wave alone spilled 1.3 KB a
 // lane and took 1847 us at the window of 1024).
@@ -105,7 +106,8 @@ __global__ void __launch_bounds__(256, WPS)
 latent_flash_kernel(LatentFlashArgs a) {
   constexpr int KS = 16 * NK + 8, BUF = KT * KS;        // (2 NK + 1 units of 16 bytes per row)
   constexpr int NU = KT * 2 * NK / 256;                 // 16-byte units of a tile per thread
-  constexpr int SH = KT / 32;
+  constexpr int SH = KT / 32, VB = 4;
+  static_assert(NDV % VB == 0, "whole groups");
   static_assert(KT * 2 * NK % 256 == 0, "whole units");
   extern __shared__ __align__(16) bf16_t lf_lds[];      // 2 * BUF + 64
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r32 = lane & 31, hh = lane >> 5;
@@ -172,8 +174,21 @@ latent_flash_kernel(LatentFlashArgs a) {
   const bool paged = bs % KT == 0;                      // a tile lies in one page
   bf16x8 kst[NU];
   // (nothing may look at the values before stash: the loads are in flight during a whole tile)
+  // the page of a tile is looked up a tile ahead of its fetch: the fetch would wait for it
+  int off = 0, at = 0, page = 0;                        // the next fetch: token in its page, page's place, page
+  auto look = [&](int it) {
+    if (!paged) return;
+    if (it == it0) {
+      at = (rw.lo + it * KT) / bs;
+      off = rw.lo + it * KT - at * bs;
+    } else {
+      off += KT;
+      if (off == bs) off = 0, ++at;
+    }
+    page = bt[at];
+  };
   auto fetch = [&](int kb) {
-    const long base = paged ? (long)bt[kb / bs] * bs + kb % bs : 0;
+    const long base = paged ? (long)__builtin_amdgcn_readfirstlane(page) * bs + off : 0;
 #pragma unroll
     for (int i = 0; i < NU; ++i) {
       const int u = tid + 256 * i, j = u / (2 * NK), d = 8 * (u % (2 * NK));
@@ -208,14 +223,35 @@ latent_flash_kernel(LatentFlashArgs a) {
 
   auto compute = [&](int buf, int kb) {
     const bf16_t* kf0 = lf_lds + buf * BUF + krow0 * KS + 8 * hh;
+    // reads of LDS go AH fragments ahead of the products, kept there by the barriers to the scheduler: left alone,
+    // each is moved to its product, which then waits for it
+    // (R 512, whose registers are short: 16 heads, 4096 tokens 915 us with one ahead, 980 with two, 1100 with four)
+    constexpr int AH = NK >= 36 && NDV == 8 ? 1 : 4, NF = SH * NK;
+    static_assert(NF % AH == 0, "whole groups");
     f32x16_t sacc[SH];
+    bf16x8 kf[2][AH];
+    auto keys = [&](int b) {
 #pragma unroll
-    for (int sh = 0; sh < SH; ++sh)
-#pragma unroll
-      for (int t = 0; t < NK; ++t) {
-        const bf16x8 kf = *reinterpret_cast<const bf16x8*>(kf0 + 32 * KS * sh + 16 * t);
-        sacc[sh] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[t], t == 0 ? f32x16_t{} : sacc[sh], 0, 0, 0);
+      for (int x = 0; x < AH; ++x) {
+        const int f = AH * b + x;
+        kf[b & 1][x] = *reinterpret_cast<const bf16x8*>(kf0 + 32 * KS * (f % SH) + 16 * (f / SH));
       }
+    };
+    // matrix products go first, the second ones before all: else the two waves of a SIMD wait for the same unit in turn
+    __builtin_amdgcn_s_setprio(1);
+    keys(0);
+#pragma unroll
+    for (int b = 0; b < NF / AH; ++b) {
+      if (b + 1 < NF / AH) keys(b + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int x = 0; x < AH; ++x) {
+        const int f = AH * b + x, sh = f % SH, t = f / SH;
+        sacc[sh] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[b & 1][x], qf[t], t == 0 ? f32x16_t{} : sacc[sh], 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __builtin_amdgcn_s_setprio(0);
     // element i of half sh is key kb + 32 sh + 16 (i >> 3) + 8 hh + (i & 7); scores of the wave's
     // first products are read here, in line with them
 #pragma unroll
@@ -251,6 +287,7 @@ latent_flash_kernel(LatentFlashArgs a) {
 #pragma unroll
       for (int dt = 0; dt < NDV; ++dt) oacc[dt] *= alpha;
     }
+    __builtin_amdgcn_s_setprio(2);
 #pragma unroll
     for (int ks = 0; ks < 2 * SH; ++ks) {
       bf16x8 ph, pl;
@@ -264,25 +301,34 @@ latent_flash_kernel(LatentFlashArgs a) {
       }
       l_run += ps;
       const bf16_t* v0 = lf_lds + buf * BUF + (16 * ks + vrow) * KS + vcol;
+      bf16x8 vf[VB];
 #pragma unroll
-      for (int dt = 0; dt < NDV; ++dt) {
-        typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-        const s16x4 a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(v0 + 32 * dt));
-        const s16x4 a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(v0 + 32 * dt + 4 * KS));
-        const bf16x8 vf = __builtin_bit_cast(bf16x8, __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7));
-        oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, ph, oacc[dt], 0, 0, 0);
-        oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pl, oacc[dt], 0, 0, 0);
+      for (int d0 = 0; d0 < NDV; d0 += VB) {
+#pragma unroll
+        for (int x = 0; x < VB; ++x) {
+          vf[x] = lds_columns(v0 + 32 * (d0 + x), v0 + 32 * (d0 + x) + 4 * KS);
+          oacc[d0 + x] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[x], ph, oacc[d0 + x], 0, 0, 0);
+        }
+#pragma unroll
+        for (int x = 0; x < VB; ++x)
+          oacc[d0 + x] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[x], pl, oacc[d0 + x], 0, 0, 0);
       }
     }
+    __builtin_amdgcn_s_setprio(0);
   };
 
+  look(it0);
   fetch(rw.lo + it0 * KT);
+  if (it0 + 1 < it1) look(it0 + 1);
   stash(0, rw.lo + it0 * KT);
   __syncthreads();
   for (int it = it0; it < it1; ++it) {
     const int kb = rw.lo + it * KT;
     const bool more = it + 1 < it1;
-    if (more) fetch(kb + KT);
+    if (more) {
+      fetch(kb + KT);
+      if (it + 2 < it1) look(it + 2);
+    }
     // does any row of the wave see a key of the tile?
     if (rw.live && kb <= rw.w_last && (a.window <= 0 || rw.w_first - (kb + KT - 1) < a.window))
       compute((it - it0) & 1, kb);

@@ -15,12 +15,16 @@
 // bf16 remainder, and the normaliser sums the fp32 values.  The running maximum moves only when a
 // tile exceeds it by 2^8.  Tile i + 1 is fetched into registers before tile i is multiplied and
 // written to the other LDS buffer behind it; one barrier per tile.  Rows are padded by 16 bytes, so
-// that the sixteen rows of an operand read lie on different banks.
+// that the sixteen rows of an operand read lie on different banks.  The page of a tile is looked up a tile
+// before its fetch, and keys are read four fragments ahead of their products.
 //
-// Four ragged prompts of up to 2048 tokens, 16 heads of 128 on 4, window 1024, soft-capped: 74 us on an
-// MI355X (249 us in the 16-query form); one 4096-token causal prompt, 8 heads on 2: 79 + 16 us in
-// parts (459 us), 126 us uncut -- a tile takes a lone workgroup 2.0 us, of which its matrix products
-// are 0.64 us; where two workgroups share a CU their products and exponentials overlap.
+// Four ragged prompts of up to 2048 tokens, 16 heads of 128 on 4, window 1024, soft-capped: 65 us on an
+// MI355X (249 us in the 16-query form); one 4096-token causal prompt, 8 heads on 2: 70 + 12 us in
+// parts (459 us).  With the page looked up by the fetch, each read in front of its product and no priorities 72 and 75 +
+// 12 us: of a tile's 5600 cycles (two workgroups on a CU) the fetch took 1100.  What bounds it now is issue: 1540 cycles of
+// matrix products and 1800 (soft-capped 3300) of vector instructions a tile and wave, two waves on a SIMD.
+// Tiles straight to LDS (128 registers' worth of staging less, but one more wait at a time) were no faster, nor were equal
+// shares of all tiles over the workgroups, where beginning a row block costs more than the evenness gives.
 #include "eia_flash.h"
 
 namespace {
@@ -129,7 +133,8 @@ window_flash_kernel(FlashArgs a) {
   constexpr int KW = P * 16 * ND, KS = KW + 8, VS = WF_KEYS + 8;
   constexpr int KBUF = WF_KEYS * KS, BUF = KBUF + 32 * NDV * VS;
   constexpr int NKU = WF_KEYS * KW / 8 / NT, NVU = 32 * NDV * WF_KEYS / 8 / NT;   // 16-byte units per thread
-  extern __shared__ __align__(16) bf16_t wf_lds[];      // 2 * BUF
+  __shared__ __align__(16) bf16_t wf_lds[2 * BUF];
+  static_assert(P == 1 || sizeof(wf_lds) >= 4 * 4 * 64 * 16 * NDV, "room to hand rows over");
   const int tid = threadIdx.x, lane = tid & 63, grp = tid >> 8, w = (tid >> 6) & 3;
   const int r32 = lane & 31, hh = lane >> 5, map = P == 2 ? grp : 0;
   const WfRows rw = wf_rows(a, w, r32);
@@ -155,7 +160,7 @@ window_flash_kernel(FlashArgs a) {
     qf[t] = d < D ? v : zero8;
   }
   // base-2 scores are raw * ml (a negative multiplier changes the sign of the query instead, so that
-  // the largest raw score is the largest score); soft-capped scores are formed in base 2 at once
+  // the largest raw score is the largest score); soft-capped, cap + 2 cap x with x = -1 / (exp(2 raw / cap) + 1)
   float ml = a.mult[h * P + map] * FLASH_LOG2E;
   if (ml < 0.f) {
     ml = -ml;
@@ -163,34 +168,60 @@ window_flash_kernel(FlashArgs a) {
     for (int t = 0; t < ND; ++t) qf[t] = -qf[t];
   }
   const float capl = a.cap * FLASH_LOG2E, icap = a.cap > 0.f ? 2.f * ml / a.cap : 0.f;
-  const float sc = a.cap > 0.f ? 1.f : fmaxf(ml, 1e-30f);
+  const float sc = a.cap > 0.f ? 2.f * capl : fmaxf(ml, 1e-30f), shift = a.cap > 0.f ? capl : 0.f;
 
   const int* bt = a.bt + (long)rw.s * a.ldbt;
-  const long krow = (long)a.G * P * D, vpage = (long)a.G * Dv * bs;
+  const long vpage = (long)a.G * Dv * bs;
+  const int krow = a.G * P * D;
+  const bool whole = D == 16 * ND && Dv == 32 * NDV;    // no channel and no column to be zeroed
+  unsigned koff[NKU], voff[NVU];
+#pragma unroll
+  for (int i = 0; i < NKU; ++i) {
+    const int u = tid + NT * i, m = u % (KW / 8) / (2 * ND), d = 8 * (u % (KW / 8) % (2 * ND));
+    koff[i] = u / (KW / 8) * krow + m * D + (d < D ? d : 0);
+  }
+#pragma unroll
+  for (int i = 0; i < NVU; ++i) {
+    const int u = tid + NT * i, c = u >> 3;
+    voff[i] = (c < Dv ? c : 0) * bs + 8 * (u & 7);
+  }
+  // the page of a tile is looked up a tile ahead of its fetch: the fetch would wait for it
+  int off = 0, at = 0, page = 0;                        // the next fetch: token in its page, page's place, page
+  auto look = [&](int it) {
+    if (it == it0 || it == nkeep) {
+      at = tile_key(it) / bs;
+      off = tile_key(it) - at * bs;
+    } else {
+      off += WF_KEYS;
+      if (off == bs) off = 0, ++at;
+    }
+    page = bt[at];
+  };
   bf16x8 kst[NKU], vst[NVU];
   // (nothing may look at the values before stash: the loads are in flight during a whole tile)
-  auto fetch = [&](int kb) {
-    const long page = bt[kb / bs];
-    const bf16_t* kp = a.kc + (page * bs + kb % bs) * krow + (long)kvh * P * D;
-    const bf16_t* vp = a.vc + page * vpage + (long)kvh * Dv * bs + kb % bs;
+  auto fetch = [&] {
+    const long pg = __builtin_amdgcn_readfirstlane(page);
+    const bf16_t* kp = a.kc + (pg * bs + off) * krow + (long)kvh * P * D;
+    const bf16_t* vp = a.vc + pg * vpage + (long)kvh * Dv * bs + off;
 #pragma unroll
-    for (int i = 0; i < NKU; ++i) {
-      const int u = tid + NT * i, m = u % (KW / 8) / (2 * ND), d = 8 * (u % (KW / 8) % (2 * ND));
-      kst[i] = *reinterpret_cast<const bf16x8*>(kp + u / (KW / 8) * krow + m * D + (d < D ? d : 0));
-    }
+    for (int i = 0; i < NKU; ++i) kst[i] = *reinterpret_cast<const bf16x8*>(kp + koff[i]);
 #pragma unroll
-    for (int i = 0; i < NVU; ++i) {
-      const int u = tid + NT * i, c = u >> 3;
-      vst[i] = *reinterpret_cast<const bf16x8*>(vp + (long)(c < Dv ? c : 0) * bs + 8 * (u & 7));
-    }
+    for (int i = 0; i < NVU; ++i) vst[i] = *reinterpret_cast<const bf16x8*>(vp + voff[i]);
   };
   auto stash = [&](int buf, int kb) {
     bf16_t* kl = wf_lds + buf * BUF;
+    if (!whole) {
+#pragma unroll
+      for (int i = 0; i < NKU; ++i)
+        if (8 * ((tid + NT * i) % (KW / 8) % (2 * ND)) >= D) kst[i] = zero8;
+#pragma unroll
+      for (int i = 0; i < NVU; ++i)
+        if ((tid + NT * i) >> 3 >= Dv) vst[i] = zero8;
+    }
 #pragma unroll
     for (int i = 0; i < NKU; ++i) {
       const int u = tid + NT * i;
-      *reinterpret_cast<bf16x8*>(kl + u / (KW / 8) * KS + 8 * (u % (KW / 8))) =
-          8 * (u % (KW / 8) % (2 * ND)) < D ? kst[i] : zero8;
+      *reinterpret_cast<bf16x8*>(kl + u / (KW / 8) * KS + 8 * (u % (KW / 8))) = kst[i];
     }
     if (kb + WF_KEYS > p_last + 1) {        // (slots behind the last key may hold anything: 0 x inf)
 #pragma unroll
@@ -202,7 +233,7 @@ window_flash_kernel(FlashArgs a) {
 #pragma unroll
     for (int i = 0; i < NVU; ++i) {
       const int u = tid + NT * i;
-      *reinterpret_cast<bf16x8*>(kl + KBUF + (u >> 3) * VS + 8 * (u & 7)) = u >> 3 < Dv ? vst[i] : zero8;
+      *reinterpret_cast<bf16x8*>(kl + KBUF + (u >> 3) * VS + 8 * (u & 7)) = vst[i];
     }
   };
 
@@ -217,28 +248,47 @@ window_flash_kernel(FlashArgs a) {
   const float sinkl = snk ? a.sink[h * P + map] * FLASH_LOG2E : 0.f;
   float m_run = snk ? fmaxf(sinkl, -1e30f) : -1e30f;
   float l_run = snk && hh == 0 ? __builtin_amdgcn_exp2f(sinkl - m_run) : 0.f;
-  const float bl = SIG && a.bias ? a.bias[h] * FLASH_LOG2E : 0.f;
+  const float bl = (SIG && a.bias ? a.bias[h] * FLASH_LOG2E : 0.f) + shift;
   const int krow0 = (r32 & ~12) | ((r32 & 4) << 1) | ((r32 & 8) >> 1);
 
   auto compute = [&](int buf, int kb) {
     const bf16_t* kf0 = wf_lds + buf * BUF + krow0 * KS + map * 16 * ND + 8 * hh;
     const bf16_t* vf0 = wf_lds + buf * BUF + KBUF + r32 * VS + 8 * hh;
+    // reads of LDS go four fragments ahead of the products, kept there by the barriers to the scheduler:
+    // left alone, each is moved to its product, which then waits for it
+    constexpr int NF = 2 * ND;
     f32x16_t sacc[2];
+    bf16x8 kf[2][4];
+    auto keys = [&](int b) {
 #pragma unroll
-    for (int sh = 0; sh < 2; ++sh)
+      for (int x = 0; x < 4; ++x)
+        kf[b & 1][x] = *reinterpret_cast<const bf16x8*>(kf0 + 32 * KS * (x & 1) + 16 * (2 * b + (x >> 1)));
+    };
+    // matrix products go first, the second ones before all: else the two waves of a SIMD wait for the same unit in
+    // turn.  (Heads of 64, whose exponentials take longer than their products, lose 5 % by it.)
+    constexpr bool PRIO = NDV > 2;
+    if (PRIO) __builtin_amdgcn_s_setprio(1);
+    keys(0);
 #pragma unroll
-      for (int t = 0; t < ND; ++t) {
-        const bf16x8 kf = *reinterpret_cast<const bf16x8*>(kf0 + 32 * KS * sh + 16 * t);
-        sacc[sh] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[t], t == 0 ? f32x16_t{} : sacc[sh], 0, 0, 0);
+    for (int b = 0; b < NF / 4; ++b) {
+      if (b + 1 < NF / 4) keys(b + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const int sh = x & 1, t = 2 * b + (x >> 1);
+        sacc[sh] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[b & 1][x], qf[t], t == 0 ? f32x16_t{} : sacc[sh], 0, 0, 0);
       }
+      __builtin_amdgcn_sched_barrier(0);
+    }
     mfma_settle(sacc[0], sacc[1]);
+    if (PRIO) __builtin_amdgcn_s_setprio(0);
     // element i of half sh is key kb + 32 sh + 16 (i >> 3) + 8 hh + (i & 7)
-    if (a.cap > 0.f) {                      // cap tanh(s / cap) = cap - 2 cap / (exp(2 s / cap) + 1)
+    if (a.cap > 0.f) {
 #pragma unroll
       for (int sh = 0; sh < 2; ++sh)
 #pragma unroll
         for (int i = 0; i < 16; ++i)
-          sacc[sh][i] = fmaf(-2.f * capl, __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(sacc[sh][i] * icap) + 1.f), capl);
+          sacc[sh][i] = __builtin_amdgcn_rcpf(-1.f - __builtin_amdgcn_exp2f(sacc[sh][i] * icap));
     }
     // every query of the wave sees every key of the tile?
     if (kb + WF_KEYS - 1 > w_first ||
@@ -262,7 +312,7 @@ window_flash_kernel(FlashArgs a) {
 #pragma unroll
         for (int j = 1; j < 8; ++j) mx4[c] = fmaxf(mx4[c], sacc[c >> 1][8 * (c & 1) + j]);
       }
-      const float mt = flash_pair_max(fmaxf(fmaxf(mx4[0], mx4[1]), fmaxf(mx4[2], mx4[3]))) * sc;
+      const float mt = flash_pair_max(fmaxf(fmaxf(mx4[0], mx4[1]), fmaxf(mx4[2], mx4[3]))) * sc + shift;
       const bool grow = mt > m_run + FLASH_DEFER;
       if (__any(grow)) {
         const float m_new = grow ? mt : m_run;
@@ -272,8 +322,9 @@ window_flash_kernel(FlashArgs a) {
 #pragma unroll
         for (int dt = 0; dt < NDV; ++dt) oacc[dt] *= alpha;
       }
-      muse = m_run;
+      muse = m_run - shift;
     }
+    if (PRIO) __builtin_amdgcn_s_setprio(2);
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
       bf16x8 ph, pl;
@@ -291,22 +342,31 @@ window_flash_kernel(FlashArgs a) {
         flash_split(p[0], p[1], j, ph, pl);
       }
       l_run += ps;
+      bf16x8 vf[NDV];
 #pragma unroll
       for (int dt = 0; dt < NDV; ++dt) {
-        const bf16x8 vf = *reinterpret_cast<const bf16x8*>(vf0 + 32 * VS * dt + 16 * ks);
-        oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, ph, oacc[dt], 0, 0, 0);
-        oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pl, oacc[dt], 0, 0, 0);
+        vf[dt] = *reinterpret_cast<const bf16x8*>(vf0 + 32 * VS * dt + 16 * ks);
+        oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[dt], ph, oacc[dt], 0, 0, 0);
       }
+#pragma unroll
+      for (int dt = 0; dt < NDV; ++dt)
+        oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[dt], pl, oacc[dt], 0, 0, 0);
     }
+    if (PRIO) __builtin_amdgcn_s_setprio(0);
   };
 
-  fetch(tile_key(it0));
+  look(it0);
+  fetch();
+  if (it0 + 1 < it1) look(it0 + 1);
   stash(0, tile_key(it0));
   __syncthreads();
   for (int it = it0; it < it1; ++it) {
     const int kb = tile_key(it);
     const bool more = it + 1 < it1;
-    if (more) fetch(tile_key(it + 1));
+    if (more) {
+      fetch();
+      if (it + 2 < it1) look(it + 2);
+    }
     // does any query of the wave see a key of the tile?
     if (live && kb <= w_last && (a.window <= 0 || w_first - (kb + WF_KEYS - 1) < a.window || kb < a.keep))
       compute((it - it0) & 1, kb);
@@ -385,12 +445,8 @@ window_flash_merge_kernel(FlashArgs a) {
 
 template <int P, int ND, int NDV, bool SIG, bool SPLIT>
 static void wf_launch(const FlashArgs& a, int n_items, int parts, hipStream_t st) {
-  constexpr int BYTES = 4 * (WF_KEYS * (P * 16 * ND + 8) + 32 * NDV * (WF_KEYS + 8));
-  static_assert(P == 1 || BYTES >= 4 * 4 * 64 * 16 * NDV, "room to hand rows over");
-  auto* f = &window_flash_kernel<P, ND, NDV, SIG, SPLIT>;
-  if (BYTES > 64 * 1024)
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(f), hipFuncAttributeMaxDynamicSharedMemorySize, BYTES);
-  hipLaunchKernelGGL(f, dim3(a.H / a.hpw, n_items, parts), dim3(256 * P), BYTES, st, a);
+  hipLaunchKernelGGL((window_flash_kernel<P, ND, NDV, SIG, SPLIT>), dim3(a.H / a.hpw, n_items, parts), dim3(256 * P),
+                     0, st, a);
   if (SPLIT)
     hipLaunchKernelGGL((window_flash_merge_kernel<NDV, SIG>), dim3(a.H / a.hpw, n_items, NDV), dim3(256), 0, st, a);
 }

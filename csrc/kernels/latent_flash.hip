@@ -11,9 +11,9 @@
 // bf16 high part plus a remainder, normaliser over the fp32 values, deferred rescale.  Rows of an LDS
 // tile are an odd number of 16-byte units apart, so that sixteen rows lie on different banks.
 //
-// MI355X, one 4096-token causal prompt: 8 heads, R 128 + 32: 79 + 12 us in parts; 8 heads, R 256 + 64: 248 us; 16
+// MI355X, one 4096-token causal prompt: 8 heads, R 128 + 32: 72 + 12 us in parts; 8 heads, R 256 + 64: 202 us; 16
 // heads, R 512 + 64: 915, with a window of 1024 488.  With the page of a tile looked up by its fetch, every read of LDS in
-// front of its product and no priorities 86 + 12, 299, 1100 and 573 us.
+// front of its product, no priorities and parts in more than one round 82 + 12, 299, 1100 and 573 us.
 // A wave's registers hold the sums of 32 rows over 256 columns beside its queries only alone on its
 // SIMD; at R 512 two waves share the rows and form the same scores (one wave alone spilled 1.3 KB a
 // lane and took 1847 us at the window of 1024).

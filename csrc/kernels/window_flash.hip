@@ -19,9 +19,9 @@
 // before its fetch, and keys are read four fragments ahead of their products.
 //
 // Four ragged prompts of up to 2048 tokens, 16 heads of 128 on 4, window 1024, soft-capped: 65 us on an
-// MI355X (249 us in the 16-query form); one 4096-token causal prompt, 8 heads on 2: 70 + 12 us in
+// MI355X (249 us in the 16-query form); one 4096-token causal prompt, 8 heads on 2: 64 + 12 us in
 // parts (459 us).  With the page looked up by the fetch, each read in front of its product and no priorities 72 and 75 +
-// 12 us: of a tile's 5600 cycles (two workgroups on a CU) the fetch took 1100.  What bounds it now is issue: 1540 cycles of
+// 12 us (parts of 13 tiles; 70 + 12 with both): of a tile's 5600 cycles (two workgroups on a CU) the fetch took 1100.  What bounds it now is issue: 1540 cycles of
 // matrix products and 1800 (soft-capped 3300) of vector instructions a tile and wave, two waves on a SIMD.
 // Tiles straight to LDS (128 registers' worth of staging less, but one more wait at a time) were no faster, nor were equal
 // shares of all tiles over the workgroups, where beginning a row block costs more than the evenness gives.

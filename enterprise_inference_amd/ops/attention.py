@@ -100,17 +100,27 @@ def build_prefill_work(q_lens: Sequence[int], qblock: int) -> List[int]:
 
 def split_keys(wgs: int, tiles: int, mean: int, slots: int, least: int = 12):
     """(parts, tiles per part) of a prefill launch of ``wgs`` workgroups that walk up to ``tiles`` and
-    on average ``mean`` key tiles, ``slots`` of which run at a time.  Where there is not one for each
-    of half the slots, row blocks are cut along the keys: where they are about equally long into as
-    many parts as there is room for, from three on; else so that a part is about 0.8 of a slot's
-    share.  Fewer than ``least`` tiles are not worth the second launch."""
+    on average ``mean`` key tiles, ``slots`` of which run at a time.  Row blocks are cut along the keys
+    into as many parts as run in one round.  Where row blocks are about equally long these have to be three or more of
+    each; else there are about ``wgs (mean / per + 1/2)`` parts of ``per`` tiles, for which 15/16 of the slots
+    are counted (they do not spread evenly over the XCDs), and two rounds where one would leave row blocks
+    nearly whole.  Fewer than ``least`` tiles are not worth the second launch.  MI355X, window_flash.hip, heads of
+    128, causal, tiles per part: us.  256 row blocks of up to 64 tiles, 13: 82, 22 (504 parts): 79, 24:
+    76, 32: 87, uncut 112; 220 of 56, 10: 69, 18: 60, 28: 70; 314 of 80, 16: 107, 28: 117, 40: 107, uncut
+    141; 438 of 110, 20: 185, 34: 184, 48: 191, uncut 215; 512 of 64, 16: 141, 24: 133, uncut 140."""
     wgs, mean = max(1, wgs), max(1, mean)
-    if 2 * wgs > slots or tiles < least:
+    if wgs > slots or tiles < least:
         return 1, tiles
-    if 4 * mean >= 3 * tiles:
-        per = -(-tiles // (slots // wgs)) if 3 * wgs <= slots else tiles
+    if 8 * mean >= 7 * tiles:
+        parts = slots // wgs
+        per = -(-tiles // parts) if parts >= 3 else tiles
     else:
-        per = -(-wgs * mean * 4 // (slots * 5))
+        per = tiles
+        for rounds, most in ((1, 0.85), (2, 0.4)):
+            share = rounds * 0.9375 * slots / wgs - 0.5
+            if share > 0 and math.ceil(mean / share) <= most * tiles:
+                per = math.ceil(mean / share)
+                break
     per = max(least // 2, per)
     return -(-tiles // per), per
 

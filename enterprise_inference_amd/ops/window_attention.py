@@ -150,18 +150,18 @@ def flash_queries(spec: WindowSpec, block_size: int) -> int:
 def flash_parts(n_items: int, spec: WindowSpec, queries: int, longest: int, context: int,
                 cus: int = 256):
     """(parts, 64-key tiles per part) of a flash prefill launch whose longest portion has
-    ``longest`` queries and whose block tables reach ``context`` tokens; two workgroups fit a CU.
-    MI355X, 8 heads of 128 on 2, one portion, uncut / cut: 4096 tokens causal 126 / 99 us, 2048 62 /
-    43, 1000 34 / 29, 500 23 / 28, 96 behind 2000 64 / 32; 16 heads on 4: 4096 causal (512
-    workgroups) 147 / 158, 1000 behind 1900 88 / 58, 500 behind 1000 with a window of 1024 47 / 30,
-    2000 with it (252) 51 / 56."""
+    ``longest`` queries and whose block tables reach ``context`` tokens; two workgroups fit a CU, three
+    of heads up to 64.  MI355X, 8 heads of 128 on 2, one portion, uncut / cut: 4096 tokens causal 112 /
+    76 us, 2048 59 / 33, 1000 32 / 24, 96 behind 2000 64 / 25; 16 heads on 4: 2048 causal 61 / 47, 4096 140 /
+    133, 1000 behind 1900 81 / 49, with a window of 1024 46 / 35, 2048 with it 43 / 43 in halves."""
     tiles = -(-context // 64)
     if spec.window > 0:
         tiles = min(tiles, (spec.window + queries + 62) // 64 + 1 + (spec.keep + 63) // 64)
     if spec.maps == 2:
         return 1, tiles
     return split_keys(n_items * (spec.heads * queries // 128), tiles,
-                      tiles if spec.window > 0 else tiles - longest // 128, 2 * cus)
+                      tiles if spec.window > 0 else tiles - longest // 128,
+                      (3 if max(spec.dim, spec.vdim) <= 64 else 2) * cus)
 
 
 def query_block(spec: WindowSpec, dtype: torch.dtype, block_size: int) -> int:

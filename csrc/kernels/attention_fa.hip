@@ -22,7 +22,7 @@
 // PHYSICAL key 16s + 8h + j, so the V^T operand of the same k-step is 8 consecutive keys --
 // one 16-B LDS read per lane.
 //
-// LDS (70 KiB, dynamic): two buffers of [K 64 x (128+8) | V^T 128 x (64+8)] bf16.  One 16-B
+// LDS (70 KiB): two buffers of [K 64 x (128+8) | V^T 128 x (64+8)] bf16.  One 16-B
 // pad per row makes every ds_read_b128 group conflict-free (K slot = (row + chunk) mod 16,
 // V^T slot = (9 d + chunk) mod 16; a 16-lane read group touches rows distinct mod 16 under pi)
 // AND keeps a lane's fragment addresses one base register plus immediate offsets (an XOR
@@ -34,13 +34,17 @@
 // MFMA / exp orders: all within 3 %; a software pipeline holding two tiles' S (QK(i+1) beside
 // the exp work of tile i) and two 32-query sub-blocks per wave (one wave per SIMD) both exceed
 // the register file and spill.  Round 4 (profiles/prefill_attn_fa_r4.md): raw v_exp_f32, a
-// branch-free mask, tree max / sum chains, static young-half priority and dwordx4 output stores
+// branch-free mask, tree max / sum chains and dwordx4 output stores
 // (65x128: 135 -> 174 TFLOP/s); fetching K/V two tiles ahead (+24 VGPRs) was slower at 1x8192
 // (800 vs 757 us) -- the one-tile-ahead fetch is not the bound there -- and a software
 // pipeline computing S of tile i+1 beside the exponentials of tile i (three LDS buffers, two S
 // register sets, 256 VGPRs) ran at 0.81x, and running the two wave halves half a tile apart
 // (two raw barriers per tile, the younger half one slot behind, so one wave of each SIMD is in
 // its softmax while the other is in P.V) at 0.92-0.94x (profiles/prefill_attn_fa_r4.md).
+// Pages looked up a tile ahead, LDS fragments read ahead of their products and matrix products first (a priority
+// per phase instead of one for the younger half of the waves): 32 heads on 8, 1 x 8192 582 -> 543 us, 1 x 2048 72 -> 65,
+// 40 heads 1 x 4096 232 -> 219, the same bits.  A tile and wave takes 1020 cycles of matrix products and about 1500
+// of vector instructions, two waves on a SIMD.
 #include "eia_common.h"
 
 namespace {
@@ -54,7 +58,6 @@ constexpr int FTHREADS = 512;  // 8 waves
 constexpr int KS = FD + 8;           // K row stride (elements)
 constexpr int VS = FKB + 8;          // V^T row stride (elements)
 constexpr int KBUF = FKB * KS, BUF = KBUF + FD * VS;
-constexpr int FA_LDS_BYTES = 2 * BUF * 2;
 constexpr float DEFER_LOG2 = 8.f;
     // rescale only when the max grows by > 2^8
 
@@ -77,7 +80,7 @@ paged_prefill_fa_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __r
                         const int* __restrict__ cu_q, const int* __restrict__ work,
                         float scale_log2, int Hq, int Hkv, int bs, int causal, int sliding_window,
                         int chunk_size) {
-  extern __shared__ __align__(16) bf16_t lds[];         // FA_LDS_BYTES
+  __shared__ __align__(16) bf16_t lds[2 * BUF];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int r32 = lane & 31, h = lane >> 5;
   // grid (head groups, work items): the heads of one query block are dispatched together and
@@ -127,10 +130,15 @@ paged_prefill_fa_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __r
   const int w_lo = wave_live ? lo_of(ctx + wq0) : 0;      // no query of the wave sees below
 
   const int* bt = block_tables + (long)s * bt_stride;
-  auto fetch = [&](int kb, bf16x8 (&st)[4]) {
-    const int blk = bt[kb / bs];
-    const long base = ((long)blk * Hkv + kvh) * (long)bs * FD;
-    const int o = kb % bs;
+  // the page of a tile is looked up a tile ahead of its fetch: the fetch would wait for it
+  int o = lo % bs, at = lo / bs, page = ntile > 0 ? bt[at] : 0;          // the next fetch: token in its page, page
+  auto look = [&] {
+    o += FKB;
+    if (o == bs) o = 0, ++at;
+    page = bt[at];
+  };
+  auto fetch = [&](bf16x8 (&st)[4]) {
+    const long base = ((long)__builtin_amdgcn_readfirstlane(page) * Hkv + kvh) * (long)bs * FD;
     const bf16_t* kp = kc + base + (long)o * FD;          // 64 rows x 128, contiguous
     const bf16_t* vp = vc + base + o;                     // 128 rows x 64 keys, row stride bs
 #pragma unroll
@@ -165,15 +173,29 @@ paged_prefill_fa_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __r
     const bf16_t* kf0 = lds + buf * BUF + krow0 * KS + 8 * h;
     const bf16_t* vf0 = lds + buf * BUF + KBUF + r32 * VS + 8 * h;
     f32x16_t sacc[2];
+    // reads of LDS go four fragments ahead of the products, kept there by the barriers to the scheduler:
+    // left alone, each is moved to its product, which then waits for it
+    bf16x8 kf[2][4];
+    auto keys = [&](int b) {
 #pragma unroll
-    for (int sh = 0; sh < 2; ++sh) {
+      for (int x = 0; x < 4; ++x)
+        kf[b & 1][x] = *reinterpret_cast<const bf16x8*>(kf0 + 32 * KS * (x & 1) + 16 * (2 * b + (x >> 1)));
+    };
+    // matrix products go first, the second ones before all: else the two waves of a SIMD wait for the same unit in turn
+    __builtin_amdgcn_s_setprio(1);
+    keys(0);
 #pragma unroll
-      for (int t = 0; t < FD / 16; ++t) {
-        const bf16x8 kf = *reinterpret_cast<const bf16x8*>(kf0 + 32 * KS * sh + 16 * t);
-        sacc[sh] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[t], t == 0 ? f32x16_t{} : sacc[sh],
-                                                           0, 0, 0);
+    for (int b = 0; b < FD / 32; ++b) {
+      if (b + 1 < FD / 32) keys(b + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const int sh = x & 1, t = 2 * b + (x >> 1);
+        sacc[sh] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[b & 1][x], qf[t], t == 0 ? f32x16_t{} : sacc[sh], 0, 0, 0);
       }
+      __builtin_amdgcn_sched_barrier(0);
     }
+    __builtin_amdgcn_s_setprio(0);
     // element i of half sh is key kb + 32 sh + 16 (i >> 3) + 8 h + (i & 7)
     const bool whole = !window && kb + FKB <= L && (!causal || kb + FKB - 1 <= ctx + wq0);
     mfma_settle(sacc[0], sacc[1]);
@@ -210,10 +232,8 @@ paged_prefill_fa_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __r
       for (int dt = 0; dt < FD / 32; ++dt) oacc[dt] *= alpha;
     }
     const float muse = m_run == (-INFINITY) ? 0.f : m_run;
-    // row sums as four independent chains.  P^T of key half a (k-steps 0, 1) first, its P.V
-    // MFMAs next to the exponentials of half b, then half b's P.V: +1-2 % over all exponentials
-    // first (profiles/prefill_attn_fa_r4.md); pinning that interleave with sched_group_barrier
-    // (one V^T read, one MFMA, five VALU per gap) exposed the LDS read latency: -2 %.
+    // row sums as four independent chains.  V^T fragments and exponentials of a k-step stand beside the
+    // products of the one before.
     bf16x8 pb[4];
     float ps4[4] = {0.f, 0.f, 0.f, 0.f};
     auto expk = [&](int ks) {
@@ -224,38 +244,46 @@ paged_prefill_fa_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __r
         ps4[ks] += HPW == 4 ? p : bf2f(pb[ks][j]);
       }
     };
-    auto pv = [&](int ks0) {
+    bf16x8 vf[2][4];
+    auto values = [&](int ks) {
 #pragma unroll
-      for (int dt = 0; dt < FD / 32; ++dt)
-#pragma unroll
-        for (int ks = ks0; ks < ks0 + 2; ++ks) {
-          const bf16x8 vf = *reinterpret_cast<const bf16x8*>(vf0 + 32 * VS * dt + 16 * ks);
-          oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pb[ks], oacc[dt], 0, 0, 0);
-        }
+      for (int dt = 0; dt < FD / 32; ++dt) vf[ks & 1][dt] = *reinterpret_cast<const bf16x8*>(vf0 + 32 * VS * dt + 16 * ks);
     };
+    auto pv = [&](int ks) {
+#pragma unroll
+      for (int dt = 0; dt < FD / 32; ++dt) oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[ks & 1][dt], pb[ks], oacc[dt], 0, 0, 0);
+    };
+    __builtin_amdgcn_s_setprio(2);
+    values(0);
+    __builtin_amdgcn_sched_barrier(0);
     expk(0);
-    expk(1);
-    pv(0);
-    expk(2);
-    expk(3);
-    pv(2);
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      if (ks < 3) {
+        values(ks + 1);
+        expk(ks + 1);
+      }
+      pv(ks);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     l_run += (ps4[0] + ps4[1]) + (ps4[2] + ps4[3]);
+    __builtin_amdgcn_s_setprio(0);
   };
 
-  // static priority for the younger half (waves 4-7): it otherwise loses VALU arbitration to
-  // the older half at the start of every segment (guide T5, static form); readfirstlane makes
-  // the condition provably wave-uniform so only those waves execute the s_setprio
-  if (__builtin_amdgcn_readfirstlane(tid) >= FTHREADS / 2) __builtin_amdgcn_s_setprio(1);
   bf16x8 st[4];
   if (ntile > 0) {
-    fetch(lo, st);
+    fetch(st);
+    if (ntile > 1) look();
     stash(0, st);
   }
   __syncthreads();
   for (int it = 0; it < ntile; ++it) {
     const int kb = lo + FKB * it;
     const bool more = it + 1 < ntile;
-    if (more) fetch(kb + FKB, st);
+    if (more) {
+      fetch(st);
+      if (it + 2 < ntile) look();
+    }
     // wave-uniform: does any of this wave's queries see a key of the tile?
     if (kb < w_hi && kb + FKB > w_lo) compute(it & 1, kb);
     if (more) stash((it + 1) & 1, st);
@@ -305,10 +333,8 @@ EIA_API int eia_paged_prefill_fa(const void* q, long q_stride, void* out, long o
   const int G = Hq / Hkv, hpw = G % 4 == 0 ? 4 : G % 2 == 0 ? 2 : 1;
 #define FA_GO(HPW)                                                                                  \
   do {                                                                                              \
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(paged_prefill_fa_kernel<HPW>),          \
-                              hipFuncAttributeMaxDynamicSharedMemorySize, FA_LDS_BYTES);            \
     hipLaunchKernelGGL(paged_prefill_fa_kernel<HPW>, dim3(Hq / HPW, n_work), dim3(FTHREADS),        \
-                       FA_LDS_BYTES, st, (const bf16_t*)q, q_stride, (bf16_t*)out, out_stride,      \
+                       0, st, (const bf16_t*)q, q_stride, (bf16_t*)out, out_stride,      \
                        (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, bt_stride,     \
                        seq_lens, cu_q, work, scale * 1.4426950408889634f, Hq, Hkv, bs, causal,      \
                        sliding_window, chunk_size);                                                 \

@@ -348,8 +348,12 @@ EIA_API int eia_latent_attn(const void* qa, long qa_st, long qa_sh, const void* 
 //
 // Bound by latency: a row's 64-key tiles are a chain of cache loads and two barriers, and the launch
 // lasts as long as the longest partition.  MI355X, 48 rows at up to 4096 tokens, window 1024, 16
-// heads, R 512 + 64: 25 + 5 us in five partitions.  (32-key units that went through LDS twice, the
-// second time as transposed 2-byte stores, with the scores formed by every wave and sixteen
+// heads, R 512 + 64: 23.8 + 4.8 us in five partitions; 200 rows at up to 2500 tokens, no window, with
+// 16 heads 153 -> 134 us and with 64 heads 499 -> 437 us since a tile's page is known before its fetch and
+// its LDS reads are asked for before the first product; R 128 + 32 with 64 heads 120 -> 115 us, R 256 + 64
+// 292 -> 292 us.  (Two tiles of cache loads in flight, in registers: 27 us instead of 24; the reads held in
+// front by barriers to the scheduler and two chains of products: 25 us.  32-key units that went through LDS
+// twice, the second time as transposed 2-byte stores, with the scores formed by every wave and sixteen
 // partitions: 91 + 21 us.)
 constexpr int lat_bufs(int NK) { return NK <= 18 ? 2 : 1; }       // tiles that fit 160 KB of LDS
 
@@ -359,10 +363,10 @@ latent_decode_kernel(LatentAttnArgs a) {
   constexpr int NB = lat_bufs(NK), KT = LAT_UNIT;
   constexpr int KS = 32 * NK + 8;                       // 4 NK + 1 units of 16 bytes per row
   constexpr int SP = KT + 4;                            // pitch of the exchanged scores
-  extern __shared__ __align__(16) unsigned char smem[];
-  bf16_t* tiles = reinterpret_cast<bf16_t*>(smem);      // [NB][KT][KS]
-  float* sS = reinterpret_cast<float*>(tiles + NB * KT * KS);      // [16][SP]
-  float2* rot = reinterpret_cast<float2*>(sS + 16 * SP);          // [rot_dims / 2]
+  // (static: more than 64 KB of dynamic LDS takes a call to the runtime for each launch)
+  __shared__ __align__(16) bf16_t tiles[NB * KT * KS];
+  __shared__ __align__(16) float sS[16 * SP];           // the exchanged scores
+  __shared__ float2 rot[16 * NK];                       // [rot_dims / 2], rot_dims <= 32 NK
   const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int l16 = lane & 15, g4 = lane >> 4;
   if (a.seq_lens && a.seq_lens[row] <= 0) return;
@@ -379,9 +383,22 @@ latent_decode_kernel(LatentAttnArgs a) {
   const bool paged = bs % KT == 0;                      // a tile lies in one page
   const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
   bf16x8 kst[NK];
+  // the page of a tile is looked up a tile ahead of its fetch: the fetch would wait for it
+  int off = 0, at = 0, page = 0;                        // the next fetch: token in its page, page's place, page
+  auto look = [&](int k0) {
+    if (!paged || k0 >= k_end) return;
+    if (k0 == k_begin) {
+      at = k0 / bs;
+      off = k0 - at * bs;
+    } else {
+      off += KT;
+      if (off == bs) off = 0, ++at;
+    }
+    page = bt[at];
+  };
   // (nothing may look at the values before stash)
   auto fetch = [&](int k0) {
-    const long base = paged ? (long)bt[k0 / bs] * bs + k0 % bs : 0;
+    const long base = paged ? (long)__builtin_amdgcn_readfirstlane(page) * bs + off : 0;
 #pragma unroll
     for (int i = 0; i < NK; ++i) {
       const int u = tid + 256 * i, j = u / (4 * NK), d = 8 * (u % (4 * NK));
@@ -397,7 +414,9 @@ latent_decode_kernel(LatentAttnArgs a) {
       *reinterpret_cast<bf16x8*>(tiles + (buf * KT + j) * KS + d) = d < Dk && k0 + j < k_end ? kst[i] : zero8;
     }
   };
+  look(k_begin);
   fetch(k_begin);
+  look(k_begin + KT);
 
   // the rotary query parts, rotated once into LDS: the heads of a row turn by the same angles
   const int hp = a.rot_dims >> 1, npass = a.rd - a.rot_dims;
@@ -459,12 +478,16 @@ latent_decode_kernel(LatentAttnArgs a) {
   for (int k0 = k_begin, buf = 0; k0 < k_end; k0 += KT, buf ^= NB - 1) {
     const bf16_t* t = tiles + buf * KT * KS;
     __syncthreads();
-    if (k0 + KT < k_end) fetch(k0 + KT);
+    if (k0 + KT < k_end) {
+      fetch(k0 + KT);
+      look(k0 + 2 * KT);
+    }
     f32x4 sc = {0.f, 0.f, 0.f, 0.f};
+    bf16x8 kf[NK];                                      // (all asked for before the first product)
 #pragma unroll
-    for (int s = 0; s < NK; ++s)
-      sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-          *reinterpret_cast<const bf16x8*>(t + (16 * w + l16) * KS + 32 * s + 8 * g4), qf[s], sc, 0, 0, 0);
+    for (int s = 0; s < NK; ++s) kf[s] = *reinterpret_cast<const bf16x8*>(t + (16 * w + l16) * KS + 32 * s + 8 * g4);
+#pragma unroll
+    for (int s = 0; s < NK; ++s) sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[s], qf[s], sc, 0, 0, 0);
     *reinterpret_cast<f32x4*>(sS + l16 * SP + 16 * w + 4 * g4) = sc * scale_log2;
     __syncthreads();
     // head l16, keys 32 x + 8 g4 + e
@@ -506,11 +529,8 @@ latent_decode_kernel(LatentAttnArgs a) {
     for (int x = 0; x < 2; ++x)
 #pragma unroll
       for (int i = 0; i < NCW; ++i) {
-        typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
         const bf16_t* p = t + (32 * x + vrow) * KS + vcol + 16 * i;
-        const s16x4 a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p);
-        const s16x4 a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p + 4 * KS));
-        const bf16x8 vf = __builtin_bit_cast(bf16x8, __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7));
+        const bf16x8 vf = lds_columns(p, p + 4 * KS);
         acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, ph[x], acc[i], 0, 0, 0);
         acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pl[x], acc[i], 0, 0, 0);
       }
@@ -615,15 +635,7 @@ EIA_API int eia_latent_attn_mfma(const void* qa, long qa_st, long qa_sh, const v
                    gate_st, out, out_st, out_sh, scale, H, R, rd, bs, 1, HB, 0, 0, window, sink,
                    rot_half, rot_amp, nparts, part_acc, part_ml};
   const dim3 grid(n_items, (H + HB - 1) / HB, nparts);
-#define LAT_DECODE(NK, NCW)                                                                        \
-  do {                                                                                             \
-    const int lds = 2 * lat_bufs(NK) * LAT_UNIT * (32 * NK + 8) +                                  \
-                    4 * 16 * (LAT_UNIT + 4) + 4 * rot_dims;                                        \
-    if (lds > 64 * 1024)                                                                           \
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&latent_decode_kernel<NK, NCW>),     \
-                                hipFuncAttributeMaxDynamicSharedMemorySize, lds);                  \
-    hipLaunchKernelGGL((latent_decode_kernel<NK, NCW>), grid, dim3(256), lds, st, a);              \
-  } while (0)
+#define LAT_DECODE(NK, NCW) hipLaunchKernelGGL((latent_decode_kernel<NK, NCW>), grid, dim3(256), 0, st, a)
   if (Dk <= 160 && R <= 128) LAT_DECODE(5, 2);
   else if (Dk <= 288 && R <= 256) LAT_DECODE(9, 4);
   else if (Dk <= 320 && R <= 256) LAT_DECODE(10, 4);

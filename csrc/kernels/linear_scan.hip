@@ -448,7 +448,7 @@ EIA_API int eia_linear_scan(const void* x, long ld, int q_off, int k_off, int v_
 // 128-token chunks: the states between chunks are the larger part of the memory
 // traffic (4 passes over chunks x H x dk x dv floats), and halving their number costs less than the
 // longer sums inside a chunk add.
-// Four prompts of 1000 .. 2000 tokens (6688 rows), 16 heads of 128, mode 1, bf16 take 13 + 33 + 21 +
+// Four prompts of 1000 .. 2000 tokens (6688 rows), 16 heads of 128, mode 1, bf16 take 11 + 33 + 21 +
 // 63 us on an MI355X (gates, (1), (2), (3)); in fp32 products (1) and (3) took 57 + 103 us.  Bound by the
 // workspace and the rows, which (1), (2) and (3) move at 3.4, 5.3 and 3.1 TB/s, and by the steps of
 // a workgroup, which reads, splits and multiplies in turn.
@@ -472,10 +472,12 @@ EIA_DEV bool ls_chunk(const ScanArgs& a, int nseq, int x, int& s, int& row0, int
 // max(f_t + m_(t-1), i_t) is a scan over pairs (f, i); a thread walks four tokens, the pairs of the
 // threads before it come from a scan over lanes and waves.  Serially in one thread the longest of
 // four 2000-token prompts took 63 us.
-template <typename T>
-__global__ void __launch_bounds__(256)
+// Bound by the latency of a pass, whose rows lie a whole projected row apart: the next pass's are asked for
+// before this one's scan.  Four 2000-token prompts of 16 heads: 13.0 -> 10.9 us.
+template <typename T, int LS_GT>            // LS_GT threads
+__global__ void __launch_bounds__(LS_GT)
 ls_gates_kernel(ScanArgs a, KChunkArgs c) {
-  __shared__ float2 wsum[4];
+  __shared__ float2 wsum[LS_GT / 64];
   __shared__ float carry;
   const int s = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int slot = a.slots[s];
@@ -484,18 +486,26 @@ ls_gates_kernel(ScanArgs a, KChunkArgs c) {
   if (hi <= lo) return;
   float m0 = a.positions[lo] == 0 ? 0.f : a.M[(long)slot * a.H + h];
   const T* X = static_cast<const T*>(a.x);
-  for (int base = lo; base < hi; base += 1024) {
+  float xi[4], xf[4];
+  auto load = [&](int base) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const T* xr = X + (long)min(base + 4 * tid + k, hi - 1) * a.ld;
+      xi[k] = ld_f32<T>(xr, a.i_off + h);
+      xf[k] = ld_f32<T>(xr, a.f_off + h);
+    }
+  };
+  load(lo);
+  for (int base = lo; base < hi; base += 4 * LS_GT) {
     float gi[4], gf[4];
     float2 p = {0.f, -INFINITY};                       // the thread's pair: sum of f, max with decays
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const int row = base + 4 * tid + k;
-      const T* xr = X + (long)min(row, hi - 1) * a.ld;
-      const float xi = ld_f32<T>(xr, a.i_off + h), xf = ld_f32<T>(xr, a.f_off + h);
-      gi[k] = a.cap > 0.f ? a.cap * tanhf(xi / a.cap) : xi;
-      gf[k] = ls_logsigmoid(a.cap > 0.f ? a.cap * tanhf(xf / a.cap) : xf);
-      if (row < hi) p = {p.x + gf[k], fmaxf(p.y + gf[k], gi[k])};
+      gi[k] = a.cap > 0.f ? a.cap * tanhf(xi[k] / a.cap) : xi[k];
+      gf[k] = ls_logsigmoid(a.cap > 0.f ? a.cap * tanhf(xf[k] / a.cap) : xf[k]);
+      if (base + 4 * tid + k < hi) p = {p.x + gf[k], fmaxf(p.y + gf[k], gi[k])};
     }
+    if (base + 4 * LS_GT < hi) load(base + 4 * LS_GT);
     float2 q = p;                                      // inclusive over the lanes
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -520,11 +530,11 @@ ls_gates_kernel(ScanArgs a, KChunkArgs c) {
         m = mn;
       }
     }
-    if (tid == 255) carry = m;
+    if (tid == LS_GT - 1) carry = m;
     __syncthreads();
     m0 = carry;
     // (the thread that holds the last token knows the final maximum)
-    if (base + 1024 >= hi && (hi - 1 - base) >> 2 == tid) a.M[(long)slot * a.H + h] = m;
+    if (base + 4 * LS_GT >= hi && (hi - 1 - base) >> 2 == tid) a.M[(long)slot * a.H + h] = m;
   }
 }
 
@@ -1390,7 +1400,13 @@ template <typename T, bool VEC, bool ROT, int MX>
 static void ls_chunked(const ScanArgs& a, const KChunkArgs& c, hipStream_t st) {
   const dim3 gc(c.rows / LK + c.nseq, a.H), gs(c.nseq, a.H);
   const dim3 gz(c.nseq, a.H, (c.DP * c.UW / 4 + 255) / 256);
-  if (a.mode == 1) hipLaunchKernelGGL((ls_gates_kernel<T>), gs, dim3(256), 0, st, a, c);
+  // 512 threads take 2048 tokens at once, 256 take 1024.  Some sequence needs a second pass of 256 where the rows
+  // are more than 1024 per sequence: the whole op at 4 x 2000 tokens 142 -> 139 us, 1 x 4096 79 -> 73 us with 512;
+  // 1 x 500 39.6 -> 40.3 us.
+  if (a.mode == 1 && c.rows > 1024L * c.nseq)
+    hipLaunchKernelGGL((ls_gates_kernel<T, 512>), gs, dim3(512), 0, st, a, c);
+  else if (a.mode == 1)
+    hipLaunchKernelGGL((ls_gates_kernel<T, 256>), gs, dim3(256), 0, st, a, c);
   if (ROT) {
     const long u = (long)c.rows * (a.rot_dims >> 1);
     hipLaunchKernelGGL(ls_angles_kernel, dim3((unsigned)((u + 255) / 256)), dim3(256), 0, st, a, c);

@@ -94,6 +94,13 @@ def test_linear_chunks(lens, H, D, Dv, mode, rot, half, dtype, monkeypatch):
         assert u is None or _rel(v, u) < 2e-6
 
 
+@pytest.mark.parametrize("lens", [[1024], [1025], [2048], [2049], [4100, 1]])
+def test_gates_over_several_passes(lens, monkeypatch):
+    """Edges of the passes in which the running maximum of the gates is formed.  The states forget within some
+    hundred tokens (decays of about 0.95), so the bounds of short prompts hold."""
+    test_linear_chunks(lens, 2, 16, 16, "exp_gates", 0, True, torch.float32, monkeypatch)
+
+
 @pytest.mark.parametrize("mode,rot", [("exp_gates", 0), ("decay", 64)])
 @pytest.mark.parametrize("H,D,Dv", [(2, 128, 128), (2, 64, 64), (2, 72, 40)])
 @pytest.mark.parametrize("where,value", [("v", float("inf")), ("v", float("nan")), ("k", float("-inf")),

@@ -32,6 +32,7 @@
 //   8 of 1024 x 512, 340 rows: 14.8 + 10.9 / 12.0 + 9.5; 1024: 34 + 24 / 25 + 18.5
 //   8 of 4096 x 14336, 122 rows: 442 + 305 / 376 + 234 (2.8 GB of weights: 550); 256: 717 + 416 / 568 + 297
 #include "eia_common.h"
+#include "eia_moe_tiles.h"
 #include <math.h>
 
 namespace {
@@ -225,7 +226,7 @@ moe_grouped_mfma_kernel(GroupedArgs a) {
   __shared__ __align__(16) bf16_t lds[(XS * MAXMU + WS * NU) * UNIT];
   const int lane = threadIdx.x & 63, E = a.E, NT = a.NT;
   auto tiles = [&](int e) {                                // M tiles of expert e
-    return e < E ? (a.offs[e + 1] - a.offs[e] + 64 * MAXMU - 1) / (64 * MAXMU) : 0;
+    return e < E ? moe_slice_tiles(a.offs[e + 1] - a.offs[e], MAXMU) : 0;
   };
   // blockIdx.x -> tile -> (expert, N tile, M tile); every wave for itself
   int total = 0;
@@ -266,15 +267,15 @@ moe_grouped_mfma_kernel(GroupedArgs a) {
   m_tiles = __builtin_amdgcn_readfirstlane(m_tiles);
   const int rb = a.offs[ex], rows = a.offs[ex + 1] - rb;
   const bf16_t* We = a.W + (long)ex * a.w_estride;
-  // the slice's 64-row units, evenly over its tiles
-  const int units = (rows + 63) / 64, lo = units * m_tile / m_tiles, mu = units * (m_tile + 1) / m_tiles - lo;
+  // Where weights come first (FRONT), tiles of 64 rows fall behind ones of 128 in long K loops: the op with 8 experts
+  // of 4096 x 14336, 50 and 55 rows an expert: shares 578 and 573 us, whole tiles 555 and 557; not in short ones: 16
+  // of 2048 x 1024, 50 rows 60.8 and 63.8.
+  const MoeTile m = moe_slice_tile(rows, m_tiles, m_tile, FRONT && a.K > 2048, MAXMU);
 #define GG_TILE(M)                                                                            \
   case M:                                                                                     \
-    if constexpr (M <= MAXMU) grouped_tile<SWIGLU, M, NU, MAXMU, FRONT>(a, lds, We, rb, rows, 64 * lo, n_tile); \
+    if constexpr (M <= MAXMU) grouped_tile<SWIGLU, M, NU, MAXMU, FRONT>(a, lds, We, rb, rows, 64 * m.lo, n_tile); \
     break
-  // long K loops of 64 rows fall behind those of 128 (8 experts of 4096 x 14336, 55 rows: the op 533 us, and
-  // 528), short ones do not (16 of 2048 x 1024, 50 rows: 60.8, and 63.8)
-  switch (FRONT && a.K > 2048 ? max(mu, 2) : mu) { GG_TILE(1); GG_TILE(2); GG_TILE(3); GG_TILE(4); GG_TILE(5); }
+  switch (m.mu) { GG_TILE(1); GG_TILE(2); GG_TILE(3); GG_TILE(4); GG_TILE(5); }
 #undef GG_TILE
 }
 

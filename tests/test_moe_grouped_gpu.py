@@ -63,6 +63,35 @@ def test_grouped_gemm_large_tiles(counts, K, form):
     assert out[n:].isnan().all()
 
 
+@pytest.mark.parametrize("form", [0, 1, 2])
+@pytest.mark.parametrize("K", [2048, 2112, 4096])
+@pytest.mark.parametrize("counts", [[1, 64, 65, 128, 129, 192, 193, 0], [130, 191, 127, 63, 66, 256, 1, 190]])
+def test_grouped_gemm_few_rows_of_long_experts(counts, K, form):
+    """Up to 128 rows an expert (a step's accesses in front of its products), slices of one to five units."""
+    from enterprise_inference_amd._native import kernels as lib
+    from enterprise_inference_amd.ops._dispatch import ptr, stream
+    g = torch.Generator().manual_seed(K + form)
+    E, n, N = len(counts), sum(counts), 256
+    assert n <= 128 * E
+    X = torch.randn(300, K, generator=g).to("cuda", BF)
+    row_idx = torch.randint(0, 300, (n,), generator=g).to("cuda", torch.int32)
+    offs = torch.tensor([0] + counts).cumsum(0).to("cuda", torch.int32)
+    W = (torch.randn(E, N, K, generator=g) * K ** -0.5).to("cuda", BF)
+    out = torch.full((n + 1, N // 2 if form == 1 else N), float("nan"), device="cuda", dtype=BF)
+    assert lib().eia_moe_grouped_gemm(ptr(X), X.stride(0), ptr(row_idx), ptr(W), N, K, E, ptr(offs),
+                                      n, form, ptr(out), out.stride(0), stream(X)) == 0
+    xs = X.double()[row_idx.long()]
+    for e, (a, b) in enumerate(zip(offs.tolist(), offs.tolist()[1:])):
+        y = xs[a:b] @ W[e].double().t()
+        if form == 1:
+            y = torch.nn.functional.silu(y[:, :N // 2]) * y[:, N // 2:]
+        elif form == 2:
+            y = torch.relu(y) ** 2
+        # fp32 sums of K exact products, one bf16 rounding (2^-9) and a fast exponential
+        assert a == b or ((out[a:b].double() - y).norm() / y.norm()) < 3e-3
+    assert out[n:].isnan().all()
+
+
 @pytest.mark.parametrize("T,E,H,I", [(100, 4, 512, 256), (96, 4, 512, 256), (200, 16, 1024, 1024),
                                      (600, 4, 512, 4352)])
 @pytest.mark.parametrize("shift", [0, 4])

@@ -18,6 +18,7 @@
 // (cu == nullptr: row s).
 #include <type_traits>
 #include "eia_common.h"
+#include "eia_delta_plan.h"
 
 EIA_DEV float dl_silu(float z) { return z / (1.0f + expf(-z)); }
 
@@ -243,6 +244,7 @@ struct DeltaChunkArgs {
   bf16_t *Y, *Kt, *Qt, *P; float *X, *O;    // as above
   float* cA;                                // [nchunk, H, 2, DC] exp(A_t), exp(A_end - A_t); A constant past the end
   int ncu, nseq;                            // units of 32 state columns
+  int parts;                                // workgroups of (1) that share a key head's heads
   int vec;                                  // out, gate and weight rows can be taken 4 at a time
 };
 
@@ -338,7 +340,7 @@ EIA_DEV bool all_finite(f32x4 v) {
   return ok;
 }
 
-// (1) one workgroup per (chunk, key head), its heads in turn.  K is staged in LDS in parts: the triangle and P
+// (1) one workgroup per (chunk, key head, part of its heads: dn_parts), those heads in turn.  K is staged in LDS in parts: the triangle and P
 // take it by rows, Y and Kt by columns (transposing reads).  Waves 0 .. 3 form the triangle, its inverse and Y,
 // a token tile each; waves 4 .. 7 meanwhile P, and then X in units of 32 columns.  k . k and q . k are
 // formed once for all heads.  X takes fp32 products: a value that is not finite stays in its column and out
@@ -352,11 +354,12 @@ delta_chunk_solve_kernel(DeltaArgs a, DeltaChunkArgs c) {
   __shared__ __align__(16) bf16_t ks[3 * PLANE];
   __shared__ __align__(16) float Ls[DC][DL];           // -L, then T
   __shared__ __align__(16) float sAs[DHB][DC], sbs[DHB][DC], sfs[DHB][DC];
-  const int ch = blockIdx.y, kh = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+  const int ch = blockIdx.y, kh = blockIdx.x / c.parts, part = blockIdx.x % c.parts, tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), w = wave & 3;
   const int s = c.chunks[4 * ch], row0 = c.chunks[4 * ch + 1], n = c.chunks[4 * ch + 2];
   if (a.slots[s] < 0) return;
   const int H = a.H, G = a.G, DP = a.DP, VP = a.VP, rep = H / G;
+  const int x0 = dn_first_head(rep, c.parts, part), nh = dn_first_head(rep, c.parts, part + 1) - x0, h0 = kh * rep + x0;
   const int g4 = lane >> 4, l16 = lane & 15;
   const long ldk = (long)G * DP, ldv = (long)H * VP;
   const float* K = a.k + (long)row0 * ldk + (long)kh * DP;
@@ -417,9 +420,11 @@ delta_chunk_solve_kernel(DeltaArgs a, DeltaChunkArgs c) {
       for (int e = 0; e < 8; ++e) v[e] = 32 * b + 16 * (e >> 2) + 4 * g4 < DP ? q[2 * b + (e >> 2)][e & 3] : 0.f;
       Parts y[1];
       split_cut(v, y[0]);
+      if (part == 0) {
 #pragma unroll
-      for (int p = 0; p < 3; ++p)
-        *reinterpret_cast<bf16x8*>(c.Qt + ((((((long)ch * G + kh) * 4 + W) * NK + b) * 3 + p) * 64 + lane) * 8) = y[0].p[p];
+        for (int p = 0; p < 3; ++p)
+          *reinterpret_cast<bf16x8*>(c.Qt + ((((((long)ch * G + kh) * 4 + W) * NK + b) * 3 + p) * 64 + lane) * 8) = y[0].p[p];
+      }
 #pragma unroll
       for (int u = 0; u <= W; ++u) {
         Parts f;
@@ -458,7 +463,7 @@ delta_chunk_solve_kernel(DeltaArgs a, DeltaChunkArgs c) {
   }
   mfma_settle(raw[0][0], raw[1][0]);
   mfma_settle(raw[2][0], raw[3][0]);
-  if (wave < 4 * NDG) {
+  if (part == 0 && wave < 4 * NDG) {
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
       const Parts f = k_columns(wave, b);
@@ -468,9 +473,9 @@ delta_chunk_solve_kernel(DeltaArgs a, DeltaChunkArgs c) {
     }
   }
   int here = lane;
-  for (int x = 0; x < rep; ++x) {
+  for (int x = 0; x < nh; ++x) {
     asm volatile("" : "+v"(here));                     // (addresses are formed anew: kept for the next head they spill)
-    const int lane = here, g4 = lane >> 4, l16 = lane & 15, h = kh * rep + x;
+    const int lane = here, g4 = lane >> 4, l16 = lane & 15, h = h0 + x;
     const long hb = (long)ch * H + h;
     const float *sA = sAs[x % DHB], *sb = sbs[x % DHB], *sf = sfs[x % DHB];
     const bool hasx = wave >= 4 && w < c.ncu;
@@ -486,7 +491,7 @@ delta_chunk_solve_kernel(DeltaArgs a, DeltaChunkArgs c) {
     }
     __syncthreads();                                   // the head before has been read
     if (x % DHB == 0) {
-      if (x + wave < rep) {                            // running sums of the log decays
+      if (x + wave < nh) {                             // running sums of the log decays
         const int hx = h + wave;
         const long hbx = (long)ch * H + hx;
         float la = lane < n ? a.la[(long)(row0 + lane) * H + hx] : 0.f;
@@ -1031,8 +1036,8 @@ EIA_API int eia_delta_scan_chunked(const float* q, const float* k, const float* 
   const bool vec = Dv % 4 == 0 && ldy % 4 == 0 && ldg % 4 == 0 &&
                    (reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(g)) % (4 * es) == 0;
   DeltaChunkArgs c{chunks, seq_first, static_cast<bf16_t*>(Y), static_cast<bf16_t*>(Kt), static_cast<bf16_t*>(Qt),
-                   static_cast<bf16_t*>(P), X, O, cA, ncu, nseq, vec};
-  const dim3 gc(G, nchunk), b(256);
+                   static_cast<bf16_t*>(P), X, O, cA, ncu, nseq, dn_parts(G * (long)nchunk, H / G), vec};
+  const dim3 gc(G * c.parts, nchunk), b(256);
   const int groups = (nseq * G + 7) / 8 * 8 * (H / G);         // of columns
   const int nc = dn_columns(nseq * H * ncu);
 #define DO_SCAN(A, C) \

@@ -169,6 +169,15 @@ def test_delta_chunks_many_heads(lens, H, G, D, Dv, dtype, monkeypatch):
     assert _rel(Z, S) < 4e-6
 
 
+@pytest.mark.parametrize("lens,H,G,D,Dv", [([129, 64], 8, 1, 128, 128), ([129, 64], 10, 2, 64, 64), ([100], 48, 3, 16, 16),
+                                           ([1] * 520, 9, 1, 16, 16), ([1] * 150 + [70] * 25, 18, 1, 16, 32),
+                                           ([66] * 45, 20, 4, 40, 24)])
+def test_delta_chunks_few_key_heads(lens, H, G, D, Dv, monkeypatch):
+    """A key head's heads one to a workgroup, in parts (of two and more than eight heads), or all in one."""
+    y, S, z, Z, live = _delta_chunks(lens, H, G, D, Dv, torch.float32, monkeypatch)
+    assert _rel(z[live], y[live]) < 1e-5 and _rel(Z, S) < 4e-6                      # as above
+
+
 def _delta_chunks(lens, H, G, D, Dv, dtype, monkeypatch, plant=lambda rows, S: None):
     from types import SimpleNamespace
     from enterprise_inference_amd.ops import delta_scan as ds

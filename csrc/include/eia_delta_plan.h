@@ -24,3 +24,23 @@ inline int dn_parts(long nwg, int rep) {
 }
 // First head of part `part` of a key head's rep heads (part == parts: the end).
 EIA_DELTA_HD int dn_first_head(int rep, int parts, int part) { return rep * part / parts; }
+
+// Workgroups of the scan: the per_kv ones of a (sequence, key head) meet the same keys and queries, and lie on as few
+// XCDs (workgroup b runs on XCD b % 8) as leave all eight of them the same share: 8 / G where G key heads divide
+// eight, then the XCD that solved a head also scans it; one where eight divides G; two for others.  MI355X, the
+// whole op in us on 1 / 2 / 4 / 8, heads of 128: 8 on 1, one prompt of 3000 tokens 217 / 125 / 120 / 120; 16 on 2, 200
+// tokens 47 / 38 / 35 / 33, 1500 130 / 83 / 81 / 81, five of 700 103 / 103 / 91 / 92; 32 on 4, three of 1500 246 / 210 /
+// 214 / 217; 8 on 4, 500 tokens 46 / 40 / 44 / 45; 16 on 8, 1000 60 / 60 / 61 / 63; 12 on 3, 1000 61 / 59 / 59 / 59; 10 on
+// 5, 1000 58 / 57 / 58 / 60.
+inline int dn_xcds(int G) { return G % 8 == 0 ? 1 : 8 % G == 0 ? 8 / G : 2; }
+EIA_DELTA_HD int dn_each(int per_kv, int xcds) { return (per_kv + xcds - 1) / xcds; }
+inline int dn_grid(int kvs, int per_kv, int xcds) {
+  return (int)(((long)kvs * xcds + 7) / 8 * 8 * dn_each(per_kv, xcds));
+}
+struct DeltaWg {
+  int kv, in;                                          // in >= per_kv or kv >= kvs: surplus
+};
+EIA_DELTA_HD DeltaWg dn_place(int block, int per_kv, int xcds) {
+  const int slot = block >> 3, each = dn_each(per_kv, xcds), unit = slot / each * 8 + (block & 7);
+  return {unit / xcds, unit % xcds * each + slot % each};
+}

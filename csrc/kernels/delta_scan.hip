@@ -245,6 +245,7 @@ struct DeltaChunkArgs {
   float* cA;                                // [nchunk, H, 2, DC] exp(A_t), exp(A_end - A_t); A constant past the end
   int ncu, nseq;                            // units of 32 state columns
   int parts;                                // workgroups of (1) that share a key head's heads
+  int xcds;                                 // XCDs that share a key head's workgroups of (2)
   int vec;                                  // out, gate and weight rows can be taken 4 at a time
 };
 
@@ -788,10 +789,11 @@ delta_chunk_scan_kernel(DeltaArgs a, DeltaChunkArgs c) {
   __shared__ __align__(16) bf16_t lds[L::TOTAL];
   const int tid = threadIdx.x, lane = tid & 63, g4 = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), w = wave & 3;
-  // the column groups of a head meet the same Y and P, the heads of a key head the same Kt and Qt: on one XCD
-  const int nct = 2 * c.ncu, ncg = nct / NC, rep = a.H / a.G, slot8 = blockIdx.x >> 3;
-  const int kv = slot8 / (ncg * rep) * 8 + (blockIdx.x & 7), in = slot8 % (ncg * rep);
-  if (kv >= c.nseq * a.G) return;
+  // the column groups of a head meet the same Y and P, the heads of a key head the same Kt and Qt (dn_xcds)
+  const int nct = 2 * c.ncu, ncg = nct / NC, rep = a.H / a.G;
+  const DeltaWg wg = dn_place(blockIdx.x, ncg * rep, c.xcds);
+  const int kv = wg.kv, in = wg.in;
+  if (kv >= c.nseq * a.G || in >= ncg * rep) return;
   const int s = kv / a.G, h = kv % a.G * rep + in / ncg, slot = a.slots[s];
   if (slot < 0) return;
   const int c0 = c.seq_first[s], c1 = c.seq_first[s + 1];
@@ -1036,12 +1038,12 @@ EIA_API int eia_delta_scan_chunked(const float* q, const float* k, const float* 
   const bool vec = Dv % 4 == 0 && ldy % 4 == 0 && ldg % 4 == 0 &&
                    (reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(g)) % (4 * es) == 0;
   DeltaChunkArgs c{chunks, seq_first, static_cast<bf16_t*>(Y), static_cast<bf16_t*>(Kt), static_cast<bf16_t*>(Qt),
-                   static_cast<bf16_t*>(P), X, O, cA, ncu, nseq, dn_parts(G * (long)nchunk, H / G), vec};
+                   static_cast<bf16_t*>(P), X, O, cA, ncu, nseq, dn_parts(G * (long)nchunk, H / G), dn_xcds(G), vec};
   const dim3 gc(G * c.parts, nchunk), b(256);
-  const int groups = (nseq * G + 7) / 8 * 8 * (H / G);         // of columns
-  const int nc = dn_columns(nseq * H * ncu);
+  const int nc = dn_columns(nseq * H * ncu), per_kv = 2 * ncu / nc * (H / G);
+  const int grid = dn_grid(nseq * G, per_kv, c.xcds);
 #define DO_SCAN(A, C) \
-  hipLaunchKernelGGL((delta_chunk_scan_kernel<A, C>), dim3(groups * (2 * ncu / C)), dim3(512), 0, st, a, c)
+  hipLaunchKernelGGL((delta_chunk_scan_kernel<A, C>), dim3(grid), dim3(512), 0, st, a, c)
 #define DO_DIMS(A)                                                                                 \
   do {                                                                                             \
     hipLaunchKernelGGL(delta_chunk_solve_kernel<A>, gc, dim3(512), 0, st, a, c);                           \

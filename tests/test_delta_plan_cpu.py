@@ -14,6 +14,13 @@ SOURCE = """
 extern "C" {
 int parts(long nwg, int rep) { return dn_parts(nwg, rep); }
 int first_head(int rep, int parts, int part) { return dn_first_head(rep, parts, part); }
+int xcds(int G) { return dn_xcds(G); }
+int grid(int kvs, int per_kv, int xcds) { return dn_grid(kvs, per_kv, xcds); }
+int place(int block, int per_kv, int xcds, int* kv) {
+  const DeltaWg wg = dn_place(block, per_kv, xcds);
+  *kv = wg.kv;
+  return wg.in;
+}
 }
 """
 
@@ -41,3 +48,22 @@ def test_heads_of_a_key_head(plan, rep):
         assert n == 1 or nwg * n <= 512
         if nwg * rep <= 512:
             assert n == rep
+
+
+@pytest.mark.parametrize("per_kv", [1, 2, 3, 8, 15, 16, 32, 64, 128])
+@pytest.mark.parametrize("G", [1, 2, 3, 4, 5, 6, 7, 8, 9, 12, 16, 24])
+@pytest.mark.parametrize("nseq", [1, 2, 3, 7])
+def test_workgroups_of_the_scan(plan, nseq, G, per_kv):
+    """Every (sequence, key head) and column group once; and all XCDs take the same share of every sequence."""
+    x, kvs = plan.xcds(G), nseq * G
+    kv, seen, full = ctypes.c_int(), set(), [0] * 8
+    for b in range(plan.grid(kvs, per_kv, x)):
+        at = plan.place(b, per_kv, x, ctypes.byref(kv))
+        if kv.value < kvs and at < per_kv:
+            assert at >= 0 and (kv.value, at) not in seen
+            seen.add((kv.value, at))
+            full[b % 8] += 1
+    assert len(seen) == kvs * per_kv
+    if (G % 8 == 0 or 8 % G == 0) and per_kv % x == 0:
+        assert max(full) == min(full) == kvs * per_kv // 8
+    assert max(full) <= -(-kvs * x // 8) * -(-per_kv // x)

@@ -343,15 +343,16 @@ def delta_scan(rows: DeltaRows, spec: DeltaSpec, state: DeltaState, md, norm_w: 
         return out
     nd = nseq - plan.nseq                       # decode rows stay token by token
     step(0, nd)
-    dev = out.device
-    f32 = lambda *s: torch.empty(*s, dtype=torch.float32, device=dev)
-    b16 = lambda *s: torch.empty(*s, dtype=torch.bfloat16, device=dev)
+    # one allocation for the workspaces (each costs the host 1 us, and a short prompt is bound by it); all of them are
+    # multiples of 512 bytes
     DQ, VQ, n = -(-DP // 64) * 64, -(-VP // 32) * 32, plan.n
-    Y, P = b16(n, H, CHUNK, DQ, 3), b16(n, H, 6, 3, 512)
-    Kt, Qt = b16(n, G, DQ, CHUNK, 3), b16(n, G, CHUNK, DQ, 3)
-    X, O, cA = f32(n, H, CHUNK, VQ), f32(n, CHUNK, H, VQ), f32(n, H, 2, CHUNK)
+    Y, K = n * H * CHUNK * DQ * 3 * 2, n * G * CHUNK * DQ * 3 * 2            # bytes of Y, and of Kt or Qt
+    P, X, cA = n * H * 6 * 3 * 512 * 2, n * H * CHUNK * VQ * 4, n * H * 2 * CHUNK * 4   # X or O
+    ws = torch.empty(Y + 2 * K + P + 2 * X + cA, dtype=torch.uint8, device=out.device)
+    at = [ws.data_ptr()]
+    for size in (Y, K, K, P, X, X):
+        at.append(at[-1] + size)
     check(lib().eia_delta_scan_chunked(
         *common, ptr(md.seq_slots[nd:]), ptr(md.positions), ptr(out), out.stride(0), plan.nseq,
-        ptr(plan.chunks), ptr(plan.seq_first), n, ptr(Y), ptr(Kt), ptr(Qt), ptr(P), ptr(X), ptr(O), ptr(cA),
-        1 if bf else 0, stream(out)), "delta_scan_chunked")
+        ptr(plan.chunks), ptr(plan.seq_first), n, *at, 1 if bf else 0, stream(out)), "delta_scan_chunked")
     return out

@@ -178,6 +178,20 @@ def test_delta_chunks_few_key_heads(lens, H, G, D, Dv, monkeypatch):
     assert _rel(z[live], y[live]) < 1e-5 and _rel(Z, S) < 4e-6                      # as above
 
 
+def test_delta_chunks_allocate_once(monkeypatch):
+    """The workspaces of a step are one allocation beside its outputs: more of them show in short prompts."""
+    from enterprise_inference_amd.ops import delta_scan as ds
+    seen, empty = [], torch.empty
+
+    def counted(*a, **k):
+        seen.extend([a] if str(k.get("device")).startswith("cuda") else [])
+        return empty(*a, **k)
+
+    monkeypatch.setattr(ds.torch, "empty", counted)
+    _, _, z, _, _ = _delta_chunks([100], 4, 2, 64, 64, torch.bfloat16, monkeypatch)
+    assert torch.isfinite(z).all() and len(seen) == 2 + 1          # (one in the helper)
+
+
 def _delta_chunks(lens, H, G, D, Dv, dtype, monkeypatch, plant=lambda rows, S: None):
     from types import SimpleNamespace
     from enterprise_inference_amd.ops import delta_scan as ds

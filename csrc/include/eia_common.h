@@ -93,6 +93,8 @@ EIA_DEV f32x4 mfma_f32_k16(f32x4 a, f32x4 b, f32x4 c) {
 // behind it.
 template <typename V> EIA_DEV void mfma_settle(V& a) { asm volatile("s_nop 11" : "+v"(a)); }
 template <typename V> EIA_DEV void mfma_settle(V& a, V& b) { asm volatile("s_nop 11" : "+v"(a), "+v"(b)); }
+template <typename V> EIA_DEV void mfma_settle(V (&o)[1]) { mfma_settle(o[0]); }
+template <typename V> EIA_DEV void mfma_settle(V (&o)[2]) { mfma_settle(o[0], o[1]); }
 template <typename V> EIA_DEV void mfma_settle(V (&o)[4]) {
   asm volatile("s_nop 11" : "+v"(o[0]), "+v"(o[1]), "+v"(o[2]), "+v"(o[3]));
 }

@@ -859,6 +859,9 @@ EIA_DEV bool ls_state_bf16(const ScanArgs& a, const KChunkArgs& c, const LsChunk
       }
     }
   }
+  mfma_settle(un);
+#pragma unroll
+  for (int i = 0; i < NA; ++i) mfma_settle(acc[i]);
   bool bad = false;
 #pragma unroll
   for (int j = 0; j < NB; ++j) {
@@ -1214,6 +1217,7 @@ EIA_DEV bool ls_out_bf16(const ScanArgs& a, const KChunkArgs& c, const LsChunk& 
     f32x4 er;
 #pragma unroll
     for (int i = 0; i < 4; ++i) er[i] = __shfl(eq, 4 * g4 + i, 64);
+    mfma_settle(o);
 #pragma unroll
     for (int j = 0; j < MX / 16; ++j) o[j] *= er;
     __syncthreads();                                   // the state was read
@@ -1304,6 +1308,7 @@ EIA_DEV bool ls_out_bf16(const ScanArgs& a, const KChunkArgs& c, const LsChunk& 
         for (int p = 2; p >= 0; --p) o[j] = mfma_bf16_k32(pp[p], vf, o[j]);
       }
     }
+    mfma_settle(o);
 #pragma unroll
     for (int j = 0; j < MX / 16; ++j)
 #pragma unroll

@@ -885,9 +885,12 @@ EIA_DEV bool ls_state_bf16(const ScanArgs& a, const KChunkArgs& c, const LsChunk
   return true;
 }
 
-// (1) Eight waves.
+// (1) Eight waves, two workgroups on a CU: 128 registers a lane.  Rotated bf16 rows of any alignment need 204 and
+// spilled 122 of them; they take a CU to themselves: four prompts of up to 2000 tokens, 16 heads of 128, 371 -> 355
+// us.  (fp32 rows, rotated: aligned 274 us with 128 registers, 289 with the 130 they would like; unaligned, where
+// 128 spill 9, 492 and 516.)
 template <typename T, bool VEC, bool ROT, int MX>
-__global__ void __launch_bounds__(512, 4)
+__global__ void __launch_bounds__(512, sizeof(T) == 2 && ROT && !VEC && MX == 128 ? 2 : 4)
 ls_chunk_state_kernel(ScanArgs a, KChunkArgs c) {
   constexpr bool BF = sizeof(T) == 2;
   constexpr int FP32 = 64 * MX * (4 + (int)sizeof(T)), SPLIT = BF ? 4 * 64 * (MX + 16) * 2 : 0;

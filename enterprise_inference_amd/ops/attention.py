@@ -98,16 +98,22 @@ def build_prefill_work(q_lens: Sequence[int], qblock: int) -> List[int]:
     return work
 
 
-def split_keys(wgs: int, tiles: int, mean: int, slots: int, least: int = 12):
+def split_keys(wgs: int, tiles: int, mean: int, slots: int, least: int = 12, crowded: bool = False):
     """(parts, tiles per part) of a prefill launch of ``wgs`` workgroups that walk up to ``tiles`` and
     on average ``mean`` key tiles, ``slots`` of which run at a time.  Row blocks are cut along the keys
     into as many parts as run in one round.  Where row blocks are about equally long these have to be three or more of
     each; else there are about ``wgs (mean / per + 1/2)`` parts of ``per`` tiles, for which 15/16 of the slots
-    are counted (they do not spread evenly over the XCDs), and two rounds where one would leave row blocks
-    nearly whole.  Fewer than ``least`` tiles are not worth the second launch.  MI355X, window_flash.hip, heads of
-    128, causal, tiles per part: us.  256 row blocks of up to 64 tiles, 13: 82, 22 (504 parts): 79, 24:
-    76, 32: 87, uncut 112; 220 of 56, 10: 69, 18: 60, 28: 70; 314 of 80, 16: 107, 28: 117, 40: 107, uncut
-    141; 438 of 110, 20: 185, 34: 184, 48: 191, uncut 215; 512 of 64, 16: 141, 24: 133, uncut 140."""
+    are counted (they do not spread evenly over the XCDs); where that makes parts longer than half of the longest row
+    block, which leave its rest to few slots, halves; and two rounds where one would leave row blocks nearly whole.
+    Fewer than ``least`` tiles are not worth the second launch.  MI355X, window_flash.hip, heads of 128, causal, row
+    blocks of up to so many tiles, tiles per part: us.  256 of 64, 13: 82, 22 (504 parts): 79, 24: 76, 32: 87, uncut
+    112; 220 of 56, 10: 69, 18: 60, 28: 70; 314 of 80, 16: 107, 28: 117, 40: 107, uncut 141; 376 of 94, 23: 135, 32:
+    143, 47: 128, 61: 148, uncut 174; 400 of 100, 27: 148, 50: 145, 72: 157; 420 of 106, 30: 161, 53: 158, 80: 170;
+    438 of 110, 24: 186, 34: 175, 55: 175, 80: 188, 93: 194, uncut 213; 482 of 122, 40: 205, 60: 217; 512 of 64, 16:
+    133, 24: 128, 32: 123, uncut 135.
+    ``crowded``: three workgroups share a CU (heads of 64), whose units they keep busy without being even, so neither
+    halves nor a second round pay for their merge: 564 of 72, 36: 98, 54: 94, uncut 100; 688 of 86, 28: 134, 43: 132,
+    uncut 126; 752 of 94, 34: 153, 47: 152, uncut 145."""
     wgs, mean = max(1, wgs), max(1, mean)
     if wgs > slots or tiles < least:
         return 1, tiles
@@ -116,10 +122,12 @@ def split_keys(wgs: int, tiles: int, mean: int, slots: int, least: int = 12):
         per = -(-tiles // parts) if parts >= 3 else tiles
     else:
         per = tiles
-        for rounds, most in ((1, 0.85), (2, 0.4)):
+        for rounds, most in ((1, 0.85),) if crowded else ((1, 0.85), (2, 0.4)):
             share = rounds * 0.9375 * slots / wgs - 0.5
             if share > 0 and math.ceil(mean / share) <= most * tiles:
                 per = math.ceil(mean / share)
+                if not crowded:
+                    per = min(per, -(-tiles // 2))
                 break
     per = max(least // 2, per)
     return -(-tiles // per), per

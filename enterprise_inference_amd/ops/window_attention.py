@@ -159,9 +159,10 @@ def flash_parts(n_items: int, spec: WindowSpec, queries: int, longest: int, cont
         tiles = min(tiles, (spec.window + queries + 62) // 64 + 1 + (spec.keep + 63) // 64)
     if spec.maps == 2:
         return 1, tiles
+    narrow = max(spec.dim, spec.vdim) <= 64
     return split_keys(n_items * (spec.heads * queries // 128), tiles,
-                      tiles if spec.window > 0 else tiles - longest // 128,
-                      (3 if max(spec.dim, spec.vdim) <= 64 else 2) * cus)
+                      tiles if spec.window > 0 else tiles - longest // 128, (3 if narrow else 2) * cus,
+                      crowded=narrow)
 
 
 def query_block(spec: WindowSpec, dtype: torch.dtype, block_size: int) -> int:

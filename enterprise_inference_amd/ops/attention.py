@@ -98,37 +98,44 @@ def build_prefill_work(q_lens: Sequence[int], qblock: int) -> List[int]:
     return work
 
 
-def split_keys(wgs: int, tiles: int, mean: int, slots: int, least: int = 12, crowded: bool = False):
+def split_keys(wgs: int, tiles: int, mean: int, slots: int, least: int = 12, merge: int = 6):
     """(parts, tiles per part) of a prefill launch of ``wgs`` workgroups that walk up to ``tiles`` and
     on average ``mean`` key tiles, ``slots`` of which run at a time.  Row blocks are cut along the keys
     into as many parts as run in one round.  Where row blocks are about equally long these have to be three or more of
     each; else there are about ``wgs (mean / per + 1/2)`` parts of ``per`` tiles, for which 15/16 of the slots
-    are counted (they do not spread evenly over the XCDs); where that makes parts longer than half of the longest row
-    block, which leave its rest to few slots, halves; and two rounds where one would leave row blocks nearly whole.
-    Fewer than ``least`` tiles are not worth the second launch.  MI355X, window_flash.hip, heads of 128, causal, row
-    blocks of up to so many tiles, tiles per part: us.  256 of 64, 13: 82, 22 (504 parts): 79, 24: 76, 32: 87, uncut
-    112; 220 of 56, 10: 69, 18: 60, 28: 70; 314 of 80, 16: 107, 28: 117, 40: 107, uncut 141; 376 of 94, 23: 135, 32:
-    143, 47: 128, 61: 148, uncut 174; 400 of 100, 27: 148, 50: 145, 72: 157; 420 of 106, 30: 161, 53: 158, 80: 170;
-    438 of 110, 24: 186, 34: 175, 55: 175, 80: 188, 93: 194, uncut 213; 482 of 122, 40: 205, 60: 217; 512 of 64, 16:
-    133, 24: 128, 32: 123, uncut 135.
-    ``crowded``: three workgroups share a CU (heads of 64), whose units they keep busy without being even, so neither
-    halves nor a second round pay for their merge: 564 of 72, 36: 98, 54: 94, uncut 100; 688 of 86, 28: 134, 43: 132,
-    uncut 126; 752 of 94, 34: 153, 47: 152, uncut 145."""
+    are counted (they do not spread evenly over the XCDs), or halves, where such parts were nearly as long or longer
+    (not much longer where most row blocks are long: halves of all of them take two rounds).
+    Fewer than ``least`` tiles are not worth the second launch, and launches that use more than half of the slots
+    only if the longest row block stands out from the mean slot's share by half of it and by the ``merge``'s time in
+    tiles.
+
+    MI355X, window_flash.hip, heads of 128, causal, row blocks of up to so many tiles, tiles per part: us.  256 of 64,
+    13: 82, 22 (504 parts): 79, 24: 76, 32: 87, uncut 112; 220 of 56, 10: 69, 18: 60, 28: 70; 314 of 80, 16: 107, 28:
+    117, 40: 107, uncut 141; 376 of 94, 23: 135, 47: 128, 61: 148, uncut 174; 420 of 106, 30: 161, 53: 158, 80: 170; 438
+    of 110, 34: 175, 55: 175, 93: 194, uncut 213; 482 of 122, 40: 205, 60: 217; 504 of 38, 15: 79, 19: 74, uncut 79; 512
+    of 64, 24: 128, 32: 123, uncut 135.  Several prompts, halves / uncut: 324 of up to 14, mean 8: 31 / 33; 408 of 12,
+    7: 33 / 29; 410 of 16, 11: 43 / 33; 456 of 30, 18: 68 / 65; 348 of 26, 16: 47 / 48.  latent_flash.hip, R 256, 256
+    slots, 166 of 16, 12: 13: 66, 8: 73, uncut 68; 160 of 36, 30: 30: 135, 18: 140, uncut 149; 185 of 48, 36: 18: 159,
+    24: 160, 36: 175; R 128, 410 of 30, 16: 15: 68, uncut 66.
+    More than 512 slots are three workgroups on a CU (heads of 64), which share its units rather than add to them:
+    512 are counted for the mean slot's share, and halves do not pay.  564 of 72, 36: 98, 54: 94, uncut 100; 688 of 86,
+    43: 132, 81: 126, uncut 126; 752 of 94, 34: 153, uncut 145; 512 of 34, 20: 51, uncut 47; 326 of 14, 6: 25, uncut 22."""
     wgs, mean = max(1, wgs), max(1, mean)
     if wgs > slots or tiles < least:
+        return 1, tiles
+    crowded, slots_even = slots > 512, min(slots, 512)
+    if 2 * wgs > slots_even and tiles <= 1.5 * wgs * mean / slots_even + merge:
         return 1, tiles
     if 8 * mean >= 7 * tiles:
         parts = slots // wgs
         per = -(-tiles // parts) if parts >= 3 else tiles
     else:
-        per = tiles
-        for rounds, most in ((1, 0.85),) if crowded else ((1, 0.85), (2, 0.4)):
-            share = rounds * 0.9375 * slots / wgs - 0.5
-            if share > 0 and math.ceil(mean / share) <= most * tiles:
-                per = math.ceil(mean / share)
-                if not crowded:
-                    per = min(per, -(-tiles // 2))
-                break
+        share = 0.9375 * slots / wgs - 0.5
+        per = math.ceil(mean / share) if share > 0 else tiles
+        if crowded:
+            per = per if per <= 0.85 * tiles else tiles
+        elif per > 0.85 * tiles or (per > 0.45 * tiles and mean <= 0.7 * tiles):
+            per = -(-tiles // 2)
     per = max(least // 2, per)
     return -(-tiles // per), per
 

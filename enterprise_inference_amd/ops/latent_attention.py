@@ -226,8 +226,10 @@ def latent_attention(q_abs: torch.Tensor, q_rot: torch.Tensor, inv_freq: torch.T
             longest = max(md.prefill_q_lens or [T])
             if window > 0:
                 tiles = min(tiles, (window + qb + KT - 2) // KT + 1)
+            # the merge's time in tiles: those of a workgroup that has a CU to itself are long
+            two = R <= 128 and R + rd <= 160
             P, per = split_keys(n_items * hg, tiles, tiles if window else tiles - longest // (2 * KT),
-                                512 if R <= 128 and R + rd <= 160 else 256, 12 * 64 // KT)
+                                512 if two else 256, 12 * 64 // KT, 11 if two else 3 * 64 // KT)
             pa = None
             if P > 1:
                 pa = torch.empty(n_items * hg * P * 4 * (4 * lib().eia_latent_flash_columns(R, rd) + 1) * 256,

@@ -162,7 +162,7 @@ def flash_parts(n_items: int, spec: WindowSpec, queries: int, longest: int, cont
     narrow = max(spec.dim, spec.vdim) <= 64
     return split_keys(n_items * (spec.heads * queries // 128), tiles,
                       tiles if spec.window > 0 else tiles - longest // 128, (3 if narrow else 2) * cus,
-                      crowded=narrow)
+                      merge=7 if narrow else 6)
 
 
 def query_block(spec: WindowSpec, dtype: torch.dtype, block_size: int) -> int:

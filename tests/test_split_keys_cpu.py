@@ -28,28 +28,38 @@ def test_one_round_where_it_fits():
     assert split_keys(513, 64, 32, 512) == (1, 64)
 
 
-@pytest.mark.parametrize("wgs,tiles,mean,best", [(220, 56, 28, 18), (314, 80, 40, 40), (344, 86, 44, 43), (376, 94, 48, 47),
-                                                 (400, 100, 50, 50), (420, 106, 54, 53), (422, 40, 21, 20),
-                                                 (436, 109, 55, 55), (438, 110, 55, 55), (438, 110, 56, 34), (482, 122, 62, 42)])
-def test_parts_near_the_best_measured(wgs, tiles, mean, best):
-    """Tiles per part of causal row blocks on 512 slots: the setting that measured best of the docstring's lists (438
-    row blocks take halves or two rounds, which measured the same), within two tiles."""
-    parts, per = split_keys(wgs, tiles, mean, 512)
-    assert abs(per - best) <= 2
+# (row blocks, longest and mean tiles, slots, the merge's time in tiles): tiles per part that measured best, of the
+# docstring's lists; within two tiles, or within one of the whole row block
+@pytest.mark.parametrize("wgs,tiles,mean,slots,merge,best", [
+    (220, 56, 28, 512, 6, 18), (314, 80, 40, 512, 6, 40), (344, 86, 44, 512, 6, 43), (376, 94, 48, 512, 6, 47),
+    (400, 100, 50, 512, 6, 50), (420, 106, 54, 512, 6, 53), (422, 40, 21, 512, 6, 20), (436, 109, 55, 512, 6, 55),
+    (438, 110, 55, 512, 6, 55), (438, 110, 56, 512, 6, 55), (500, 126, 64, 512, 6, 63), (504, 38, 20, 512, 6, 19),
+    (512, 64, 32, 512, 6, 32), (454, 66, 34, 512, 6, 33),
+    (324, 14, 8, 512, 6, 7), (408, 12, 7, 512, 6, 12), (410, 16, 11, 512, 6, 16), (456, 30, 18, 512, 6, 30),
+    (348, 26, 16, 512, 6, 13), (412, 52, 27, 512, 6, 26),
+    (688, 86, 44, 768, 7, 86), (752, 94, 48, 768, 7, 94), (512, 34, 18, 768, 7, 34), (326, 14, 8, 768, 7, 14),
+    (488, 14, 8, 768, 7, 14), (540, 18, 10, 768, 7, 18), (410, 78, 47, 768, 7, 39), (338, 56, 29, 768, 7, 18),
+    (166, 16, 12, 256, 3, 13), (160, 36, 30, 256, 3, 30), (152, 38, 19, 256, 3, 19), (186, 24, 13, 256, 3, 12),
+    (233, 36, 19, 256, 3, 18), (185, 48, 36, 256, 3, 24), (410, 30, 16, 512, 11, 30), (462, 68, 39, 512, 11, 34)])
+def test_parts_near_the_best_measured(wgs, tiles, mean, slots, merge, best):
+    parts, per = split_keys(wgs, tiles, mean, slots, 12, merge)
+    assert abs(per - best) <= (2 if best < tiles else 1)
 
 
 @pytest.mark.parametrize("slots", [256, 512])
-def test_no_part_is_longer_than_half_a_row_block(slots):
+def test_no_part_is_longer_than_half_a_causal_row_block(slots):
     for wgs in range(1, slots + 1):
-        for tiles in (24, 50, 64, 110, 300):
+        for tiles in (50, 64, 110, 300):
             parts, per = split_keys(wgs, tiles, tiles // 2, slots)
             assert parts >= 2 and 2 * per <= tiles + 1
 
 
-def test_three_workgroups_on_a_cu():
-    """... take no second round: 688 and 752 row blocks of heads of 64 measured best uncut."""
-    assert split_keys(688, 86, 44, 768, crowded=True) == (1, 86)
-    assert split_keys(752, 94, 48, 768, crowded=True) == (1, 94)
-    for wgs in range(1, 769):
-        parts, per = split_keys(wgs, 94, 47, 768, crowded=True)
-        assert parts * per >= 94 > (parts - 1) * per and (parts == 1 or wgs * (47 / per + 0.5) <= 768)
+@pytest.mark.parametrize("merge", [3, 7, 11])
+@pytest.mark.parametrize("slots", [256, 512, 768])
+def test_parts_cover_every_tile_whatever_the_merge_takes(slots, merge):
+    for wgs in (1, 127, 128, 129, 256, 257, 376, 512, 700, 768, 769):
+        for tiles in (12, 13, 24, 65, 300):
+            for mean in (tiles // 2, 3 * tiles // 4, tiles):
+                parts, per = split_keys(wgs, tiles, mean, slots, 12, merge)
+                assert per >= 1 and parts * per >= tiles > (parts - 1) * per
+                assert parts == 1 or (wgs <= slots and per >= 6)

@@ -237,8 +237,11 @@ latent_flash_kernel(LatentFlashArgs a) {
         kf[b & 1][x] = *reinterpret_cast<const bf16x8*>(kf0 + 32 * KS * (f % SH) + 16 * (f / SH));
       }
     };
-    // matrix products go first, the second ones before all: else the two waves of a SIMD wait for the same unit in turn
-    __builtin_amdgcn_s_setprio(1);
+    // matrix products go first, the second ones before all: else the two waves of a SIMD wait for the same unit in turn.
+    // (Not in whole row blocks of R 128, whose waves are rarely at the same place: two prompts of up to 3743 tokens,
+    // 8 heads 130 us with priorities, 122 without, in halves 109 and 113.)
+    constexpr bool PRIO = SPLIT || NK > 10;
+    if (PRIO) __builtin_amdgcn_s_setprio(1);
     keys(0);
 #pragma unroll
     for (int b = 0; b < NF / AH; ++b) {
@@ -251,7 +254,7 @@ latent_flash_kernel(LatentFlashArgs a) {
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    __builtin_amdgcn_s_setprio(0);
+    if (PRIO) __builtin_amdgcn_s_setprio(0);
     // element i of half sh is key kb + 32 sh + 16 (i >> 3) + 8 hh + (i & 7); scores of the wave's
     // first products are read here, in line with them
 #pragma unroll
@@ -287,7 +290,7 @@ latent_flash_kernel(LatentFlashArgs a) {
 #pragma unroll
       for (int dt = 0; dt < NDV; ++dt) oacc[dt] *= alpha;
     }
-    __builtin_amdgcn_s_setprio(2);
+    if (PRIO) __builtin_amdgcn_s_setprio(2);
 #pragma unroll
     for (int ks = 0; ks < 2 * SH; ++ks) {
       bf16x8 ph, pl;
@@ -314,7 +317,7 @@ latent_flash_kernel(LatentFlashArgs a) {
           oacc[d0 + x] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[x], pl, oacc[d0 + x], 0, 0, 0);
       }
     }
-    __builtin_amdgcn_s_setprio(0);
+    if (PRIO) __builtin_amdgcn_s_setprio(0);
   };
 
   look(it0);

@@ -657,9 +657,12 @@ delta_chunk_solve_kernel(DeltaArgs a, DeltaChunkArgs c) {
 // their 16 tokens from the same S and u while the first four wait for each other, so that neither goes to memory.
 // u and S pass between the waves through LDS, in parts; a chunk has two steps, u and then S.
 // An operand of the next chunk is requested where this chunk's has been used, a whole chunk ahead.
+// S, u and the outputs are carried times 2^24, so that the third part of a number as small as 2^-126 is still one (parts
+// of those of 2^-105, unscaled, left an error of 1.1e-6 in S, fp32 products 2.5e-7).
 // 32 columns halve the reads per product, which a workgroup of 16 columns is bound by; 16 give twice the
 // workgroups: dn_columns.  A sum that is not finite, which parts cannot follow, sends the workgroup through
 // delta_scan_fp32: fp32 products from the start.
+constexpr float DN_UP = 0x1p24f;
 template <int NDG, int NC> struct ScanTiles {
   static constexpr int OP = 3 * 64 * 8;                // one operand, in bf16 numbers
   static constexpr int S = 2 * NDG * NC * OP, U = 2 * NC * OP;
@@ -673,8 +676,9 @@ struct ScanAt {
   EIA_DEV int rows(int ch) const { return ch + 1 < c1 ? DC : last; }
 };
 
+// (f: a power of two that S is multiplied by on its way)
 template <int NDG, int NC>
-EIA_DEV void scan_state(const DeltaArgs& a, const ScanAt& k, f32x4 (&S)[NDG][NC], bool put) {
+EIA_DEV void scan_state(const DeltaArgs& a, const ScanAt& k, f32x4 (&S)[NDG][NC], bool put, float f) {
   const int g4 = k.lane >> 4, l16 = k.lane & 15, tile0 = NDG * (k.wave & 3);
 #pragma unroll
   for (int o = 0; o < NDG; ++o)
@@ -686,23 +690,23 @@ EIA_DEV void scan_state(const DeltaArgs& a, const ScanAt& k, f32x4 (&S)[NDG][NC]
         const int ct = k.ct0 + j, col = 32 * (ct >> 1) + 2 * l16 + (ct & 1);
         const bool in = r < a.D && col < a.Dv;
         if (put) {
-          if (in) k.Sg[(long)r * a.Dv + col] = S[o][j][i];
+          if (in) k.Sg[(long)r * a.Dv + col] = S[o][j][i] * f;
         } else {
-          S[o][j][i] = in && !k.fresh ? k.Sg[(long)r * a.Dv + col] : 0.f;
+          S[o][j][i] = in && !k.fresh ? k.Sg[(long)r * a.Dv + col] * f : 0.f;
         }
       }
     }
 }
 template <int NC>
-EIA_DEV void scan_put_out(const DeltaArgs& a, const DeltaChunkArgs& c, const ScanAt& k, int ch, const f32x4 (&o)[NC]) {
+EIA_DEV void scan_put_out(const DeltaArgs& a, const DeltaChunkArgs& c, const ScanAt& k, int ch, const f32x4 (&o)[NC], float f) {
   const int g4 = k.lane >> 4, l16 = k.lane & 15, n = k.rows(ch), VQ = 32 * c.ncu;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int t = 16 * (k.wave & 3) + 4 * g4 + i;
     float* p = c.O + (((long)ch * DC + t) * a.H + k.h) * VQ + 32 * (k.ct0 >> 1) + 2 * l16 + (k.ct0 & 1);
     if (t < n) {
-      if constexpr (NC == 2) *reinterpret_cast<float2*>(p) = float2{o[0][i], o[1][i]};
-      else *p = o[0][i];
+      if constexpr (NC == 2) *reinterpret_cast<float2*>(p) = float2{o[0][i] * f, o[1][i] * f};
+      else *p = o[0][i] * f;
     }
   }
 }
@@ -715,7 +719,7 @@ EIA_DEV void delta_scan_fp32(const DeltaArgs& a, const DeltaChunkArgs& c, const 
   const bool carry = k.wave < 4;
   f32x4 S[NDG][NC];
   if (carry) {
-    scan_state<NDG, NC>(a, k, S, false);
+    scan_state<NDG, NC>(a, k, S, false, 1.f);
 #pragma unroll
     for (int o = 0; o < NDG; ++o)
 #pragma unroll
@@ -774,11 +778,11 @@ EIA_DEV void delta_scan_fp32(const DeltaArgs& a, const DeltaChunkArgs& c, const 
         if constexpr (NC == 2) mfma_settle(o[0], o[1]);
         else mfma_settle(o[0]);
       }
-      scan_put_out<NC>(a, c, k, ch, o);
+      scan_put_out<NC>(a, c, k, ch, o, 1.f);
     }
     __syncthreads();
   }
-  if (carry) scan_state<NDG, NC>(a, k, S, true);
+  if (carry) scan_state<NDG, NC>(a, k, S, true, 1.f);
 }
 
 template <int NDG, int NC>
@@ -840,7 +844,7 @@ delta_chunk_scan_kernel(DeltaArgs a, DeltaChunkArgs c) {
     for (int o = 0; o < NDG; ++o)
 #pragma unroll
       for (int b = 0; b < 2; ++b) load_k(c0, o, b);
-    scan_state<NDG, NC>(a, k, S, false);
+    scan_state<NDG, NC>(a, k, S, false, DN_UP);
     put_state(0);
     __syncthreads();
     for (int ch = c0; ch < c1; ++ch) {
@@ -862,7 +866,7 @@ delta_chunk_scan_kernel(DeltaArgs a, DeltaChunkArgs c) {
       const float decay = eg;
 #pragma unroll
       for (int j = 0; j < NC; ++j) {
-        u[j] = x[j] - acc[0][j] - acc[1][j];
+        u[j] = x[j] * DN_UP - acc[0][j] - acc[1][j];
         put_half(Us(0, w >> 1, j), w & 1, lane, u[j] * ew);
       }
       load_x(nx);
@@ -916,7 +920,7 @@ delta_chunk_scan_kernel(DeltaArgs a, DeltaChunkArgs c) {
       else mfma_settle(o[0]);
 #pragma unroll
       for (int j = 0; j < NC; ++j) bad |= !all_finite(o[j]);
-      scan_put_out<NC>(a, c, k, ch, o);
+      scan_put_out<NC>(a, c, k, ch, o, 1.f / DN_UP);
     };
     load_q(c0);
     __syncthreads();
@@ -948,7 +952,7 @@ delta_chunk_scan_kernel(DeltaArgs a, DeltaChunkArgs c) {
     delta_scan_fp32<NDG, NC>(a, c, k, lds);
     return;
   }
-  if (wave < 4) scan_state<NDG, NC>(a, k, S, true);
+  if (wave < 4) scan_state<NDG, NC>(a, k, S, true, 1.f / DN_UP);
 }
 
 // (3) Norm, weight and gate of the outputs: LN lanes per token and head, four heads each.  Bound by memory.

@@ -178,6 +178,21 @@ def test_delta_chunks_few_key_heads(lens, H, G, D, Dv, monkeypatch):
     assert _rel(z[live], y[live]) < 1e-5 and _rel(Z, S) < 4e-6                      # as above
 
 
+@pytest.mark.parametrize("H,G,D,Dv", [(4, 2, 128, 128), (8, 4, 64, 72), (32, 8, 128, 128)])
+@pytest.mark.parametrize("e,most", [(60, 0.0), (100, 2.0 ** -25), (-110, 2.0 ** -25)])
+def test_delta_of_small_and_large_magnitudes(e, most, H, G, D, Dv, monkeypatch):
+    """Values and state times 2^-e: so is the state after them.  At 2^-100 what falls below the smallest normal
+    number is 2^-26 of the rest; times 2^110 overflows the parts, which fp32 products take over."""
+    def run(scale):
+        def plant(rows, S):
+            rows[2].mul_(scale)
+            S.mul_(scale)
+        return _delta_chunks([150, 200], H, G, D, Dv, torch.float32, monkeypatch, plant)[3].double() / scale
+
+    S, Z = run(1.0), run(2.0 ** -e)
+    assert float((Z - S).norm() / S.norm()) <= (most if e > 0 else 4e-6)            # (other products: as above)
+
+
 def test_delta_chunks_allocate_once(monkeypatch):
     """The workspaces of a step are one allocation beside its outputs: more of them show in short prompts."""
     from enterprise_inference_amd.ops import delta_scan as ds

@@ -32,15 +32,18 @@ EIA_DELTA_HD int dn_first_head(int rep, int parts, int part) { return rep * part
 // tokens 47 / 38 / 35 / 33, 1500 130 / 83 / 81 / 81, five of 700 103 / 103 / 91 / 92; 32 on 4, three of 1500 246 / 210 /
 // 214 / 217; 8 on 4, 500 tokens 46 / 40 / 44 / 45; 16 on 8, 1000 60 / 60 / 61 / 63; 12 on 3, 1000 61 / 59 / 59 / 59; 10 on
 // 5, 1000 58 / 57 / 58 / 60.
-inline int dn_xcds(int G) { return G % 8 == 0 ? 1 : 8 % G == 0 ? 8 / G : 2; }
-EIA_DELTA_HD int dn_each(int per_kv, int xcds) { return (per_kv + xcds - 1) / xcds; }
-inline int dn_grid(int kvs, int per_kv, int xcds) {
-  return (int)(((long)kvs * xcds + 7) / 8 * 8 * dn_each(per_kv, xcds));
+struct DeltaSpread {
+  int per_kv, shift, each;                             // 2^shift XCDs, `each` workgroups on one
+};
+inline DeltaSpread dn_spread(int G, int per_kv) {
+  const int shift = G % 8 == 0 ? 0 : G == 1 ? 3 : G == 2 ? 2 : 1;
+  return {per_kv, shift, (per_kv + (1 << shift) - 1) >> shift};
 }
+inline int dn_grid(int kvs, const DeltaSpread& x) { return (int)((((long)kvs << x.shift) + 7) / 8 * 8 * x.each); }
 struct DeltaWg {
   int kv, in;                                          // in >= per_kv or kv >= kvs: surplus
 };
-EIA_DELTA_HD DeltaWg dn_place(int block, int per_kv, int xcds) {
-  const int slot = block >> 3, each = dn_each(per_kv, xcds), unit = slot / each * 8 + (block & 7);
-  return {unit / xcds, unit % xcds * each + slot % each};
+EIA_DELTA_HD DeltaWg dn_place(int block, const DeltaSpread& x) {
+  const int slot = block >> 3, row = slot / x.each, unit = 8 * row + (block & 7);
+  return {unit >> x.shift, (unit & ((1 << x.shift) - 1)) * x.each + slot - row * x.each};
 }

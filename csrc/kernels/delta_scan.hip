@@ -230,7 +230,7 @@ EIA_API int eia_delta_scan(const float* q, const float* k, const float* v, const
 //   X  [chunk, H, 4 token tiles, VP / 16 tiles]       fp32, B operand, rows tokens
 //   O  [chunk, 64, H, VP]                             fp32, outputs before their norm
 // with DP rounded up to 64 and VP to 32; tile j of 32 columns holds columns 2 x + j.
-// MI355X, 16 heads of 128 x 128, three prompts of 750 to 1500 tokens: 54 + 68 + 21 us
+// MI355X, 16 heads of 128 x 128 on 8, three prompts of 750 to 1500 tokens: 57 + 69 + 21 us
 // ((1), (2), (3)).  Before, with fp32 products and the states between chunks and u in memory for a kernel that formed
 // the outputs, 48 + 77 + 83 (the op: 197 -> 147).  S against 64 bits: 1.2e-7 .. 1.5e-7 where fp32 products left 1.3e-7 .. 1.6e-7.
 // (1) and (3) are bound by their writes and reads (3.4, 3.3 TB/s), (2) by the chain of its chunks: 6000 cycles
@@ -245,7 +245,7 @@ struct DeltaChunkArgs {
   float* cA;                                // [nchunk, H, 2, DC] exp(A_t), exp(A_end - A_t); A constant past the end
   int ncu, nseq;                            // units of 32 state columns
   int parts;                                // workgroups of (1) that share a key head's heads
-  int xcds;                                 // XCDs that share a key head's workgroups of (2)
+  DeltaSpread spread;                       // the workgroups of (2) over the XCDs
   int vec;                                  // out, gate and weight rows can be taken 4 at a time
 };
 
@@ -310,7 +310,9 @@ EIA_DEV f32x4 whole(const Parts& f, int half) {        // of a tile of the two
     v[e] = ((float)f.p[0][4 * half + e] + (float)f.p[1][4 * half + e]) + (float)f.p[2][4 * half + e];
   return v;
 }
-// The six largest products of parts; what is left out is below 2^-26 of the product.
+// The six largest products of parts.  What is left out (m l, l m, l l) is below 2^-24 of the product where both numbers
+// were split by rounding (m up to 2^-8 of the number, l up to 2^-17), below 2^-23 where one was cut (split_cut:
+// 2^-7, 2^-16): about the one rounding of an fp32 product.
 template <int N> EIA_DEV void mm6(const Parts& a, const Parts (&b)[N], f32x4 (&c)[N]) {
   constexpr int pa[6] = {0, 2, 1, 0, 1, 0}, pb[6] = {2, 0, 1, 1, 0, 0};
 #pragma unroll
@@ -793,11 +795,11 @@ delta_chunk_scan_kernel(DeltaArgs a, DeltaChunkArgs c) {
   __shared__ __align__(16) bf16_t lds[L::TOTAL];
   const int tid = threadIdx.x, lane = tid & 63, g4 = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), w = wave & 3;
-  // the column groups of a head meet the same Y and P, the heads of a key head the same Kt and Qt (dn_xcds)
+  // the column groups of a head meet the same Y and P, the heads of a key head the same Kt and Qt (dn_spread)
   const int nct = 2 * c.ncu, ncg = nct / NC, rep = a.H / a.G;
-  const DeltaWg wg = dn_place(blockIdx.x, ncg * rep, c.xcds);
+  const DeltaWg wg = dn_place(blockIdx.x, c.spread);
   const int kv = wg.kv, in = wg.in;
-  if (kv >= c.nseq * a.G || in >= ncg * rep) return;
+  if (kv >= c.nseq * a.G || in >= c.spread.per_kv) return;
   const int s = kv / a.G, h = kv % a.G * rep + in / ncg, slot = a.slots[s];
   if (slot < 0) return;
   const int c0 = c.seq_first[s], c1 = c.seq_first[s + 1];
@@ -1042,10 +1044,11 @@ EIA_API int eia_delta_scan_chunked(const float* q, const float* k, const float* 
   const bool vec = Dv % 4 == 0 && ldy % 4 == 0 && ldg % 4 == 0 &&
                    (reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(g)) % (4 * es) == 0;
   DeltaChunkArgs c{chunks, seq_first, static_cast<bf16_t*>(Y), static_cast<bf16_t*>(Kt), static_cast<bf16_t*>(Qt),
-                   static_cast<bf16_t*>(P), X, O, cA, ncu, nseq, dn_parts(G * (long)nchunk, H / G), dn_xcds(G), vec};
+                   static_cast<bf16_t*>(P), X, O, cA, ncu, nseq, dn_parts(G * (long)nchunk, H / G), {}, vec};
   const dim3 gc(G * c.parts, nchunk), b(256);
-  const int nc = dn_columns(nseq * H * ncu), per_kv = 2 * ncu / nc * (H / G);
-  const int grid = dn_grid(nseq * G, per_kv, c.xcds);
+  const int nc = dn_columns(nseq * H * ncu);
+  c.spread = dn_spread(G, 2 * ncu / nc * (H / G));
+  const int grid = dn_grid(nseq * G, c.spread);
 #define DO_SCAN(A, C) \
   hipLaunchKernelGGL((delta_chunk_scan_kernel<A, C>), dim3(grid), dim3(512), 0, st, a, c)
 #define DO_DIMS(A)                                                                                 \

@@ -343,15 +343,16 @@ def delta_scan(rows: DeltaRows, spec: DeltaSpec, state: DeltaState, md, norm_w: 
         return out
     nd = nseq - plan.nseq                       # decode rows stay token by token
     step(0, nd)
-    # one allocation for the workspaces (each costs the host 1 us, and a short prompt is bound by it); all of them are
-    # multiples of 512 bytes
+    # one allocation for the workspaces (each costs the host 1 us, and a short prompt is bound by it): multiples of 512
+    # bytes, and of 2 MiB from there on (three prompts of up to 1500 tokens, 16 heads 151.6 -> 150.2 us)
     DQ, VQ, n = -(-DP // 64) * 64, -(-VP // 32) * 32, plan.n
     Y, K = n * H * CHUNK * DQ * 3 * 2, n * G * CHUNK * DQ * 3 * 2            # bytes of Y, and of Kt or Qt
     P, X, cA = n * H * 6 * 3 * 512 * 2, n * H * CHUNK * VQ * 4, n * H * 2 * CHUNK * 4   # X or O
-    ws = torch.empty(Y + 2 * K + P + 2 * X + cA, dtype=torch.uint8, device=out.device)
-    at = [ws.data_ptr()]
-    for size in (Y, K, K, P, X, X):
-        at.append(at[-1] + size)
+    at = [0]
+    for size in (Y, K, K, P, X, X, cA):
+        at.append(at[-1] + (size if size < 1 << 21 else -(-size >> 21) << 21))
+    ws = torch.empty(at.pop(), dtype=torch.uint8, device=out.device)
+    at = [ws.data_ptr() + a for a in at]
     check(lib().eia_delta_scan_chunked(
         *common, ptr(md.seq_slots[nd:]), ptr(md.positions), ptr(out), out.stride(0), plan.nseq,
         ptr(plan.chunks), ptr(plan.seq_first), n, *at, 1 if bf else 0, stream(out)), "delta_scan_chunked")

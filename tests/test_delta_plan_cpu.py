@@ -14,10 +14,10 @@ SOURCE = """
 extern "C" {
 int parts(long nwg, int rep) { return dn_parts(nwg, rep); }
 int first_head(int rep, int parts, int part) { return dn_first_head(rep, parts, part); }
-int xcds(int G) { return dn_xcds(G); }
-int grid(int kvs, int per_kv, int xcds) { return dn_grid(kvs, per_kv, xcds); }
-int place(int block, int per_kv, int xcds, int* kv) {
-  const DeltaWg wg = dn_place(block, per_kv, xcds);
+int xcds(int G, int per_kv) { return 1 << dn_spread(G, per_kv).shift; }
+int grid(int G, int per_kv, int nseq) { return dn_grid(nseq * G, dn_spread(G, per_kv)); }
+int place(int block, int G, int per_kv, int* kv) {
+  const DeltaWg wg = dn_place(block, dn_spread(G, per_kv));
   *kv = wg.kv;
   return wg.in;
 }
@@ -55,15 +55,15 @@ def test_heads_of_a_key_head(plan, rep):
 @pytest.mark.parametrize("nseq", [1, 2, 3, 7])
 def test_workgroups_of_the_scan(plan, nseq, G, per_kv):
     """Every (sequence, key head) and column group once; and all XCDs take the same share of every sequence."""
-    x, kvs = plan.xcds(G), nseq * G
+    x, kvs = plan.xcds(G, per_kv), nseq * G
     kv, seen, full = ctypes.c_int(), set(), [0] * 8
-    for b in range(plan.grid(kvs, per_kv, x)):
-        at = plan.place(b, per_kv, x, ctypes.byref(kv))
+    for b in range(plan.grid(G, per_kv, nseq)):
+        at = plan.place(b, G, per_kv, ctypes.byref(kv))
         if kv.value < kvs and at < per_kv:
             assert at >= 0 and (kv.value, at) not in seen
             seen.add((kv.value, at))
             full[b % 8] += 1
-    assert len(seen) == kvs * per_kv
+    assert len(seen) == kvs * per_kv and x == (1 if G % 8 == 0 else 8 // G if 8 % G == 0 else 2)
     if (G % 8 == 0 or 8 % G == 0) and per_kv % x == 0:
         assert max(full) == min(full) == kvs * per_kv // 8
     assert max(full) <= -(-kvs * x // 8) * -(-per_kv // x)

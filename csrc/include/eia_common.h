@@ -121,10 +121,11 @@ EIA_DEV unsigned lds_offset(const void* p) {
   return (unsigned)(uintptr_t)(__attribute__((address_space(3))) const void*)p;
 }
 
-// Two fp32 numbers as sums of three bf16 ones each, largest part first: 24 bits in three times eight, exact
-// for finite numbers (down to what bf16 holds).  A matrix product of such parts with bf16 operands, or of the
-// six largest pairs of parts, keeps what an fp32 product keeps at 3/16 or 6/16 of its matrix cycles.  Parts
-// of what is not finite are no numbers, so callers look for sums that are not finite and form those anew.
+// Two fp32 numbers as sums of three bf16 ones each, largest part first: 24 bits in three times eight, exact from
+// 2^-103 (what is left of smaller numbers for the third part may be flushed) up to bf16's largest, 2^127 (2 - 2^-7).  A
+// matrix product of such parts with bf16 operands, or of the six largest pairs of parts, keeps what an fp32
+// product keeps at 3/16 or 6/16 of its matrix cycles.  The first part of what rounds past bf16's largest is infinite,
+// and parts of what is not finite are no numbers, so callers look for sums that are not finite and form those anew.
 EIA_DEV void split3(float a, float b, bf16x2& h, bf16x2& m, bf16x2& l) {
   typedef __attribute__((ext_vector_type(2))) float f32x2_t;
   auto up = [](bf16x2 v, int i) {

@@ -101,6 +101,23 @@ def test_gates_over_several_passes(lens, monkeypatch):
     test_linear_chunks(lens, 2, 16, 16, "exp_gates", 0, True, torch.float32, monkeypatch)
 
 
+def _stays_not_finite(y, z, H, col, hit):
+    """What the recurrence (y) leaves not finite does not come out as a number (z), and where both are numbers they are
+    the same.  col: an infinite value is one number of its column, (q . k) v, in sums over tokens, and a sum of infinities of
+    both signs, none, in ones over the state's rows; the other columns are divided by its norm, to 0 or to no
+    number.  So only that column is compared."""
+    rows = lambda t: t.double().view(t.shape[0], H, -1)
+    a, b = rows(y), rows(z)
+    bad = ~torch.isfinite(a)
+    assert bool(bad.any()) == hit
+    if col is not None:
+        a, b, bad = a[:, :, col], b[:, :, col], bad[:, :, col]
+        assert bad.any()
+    assert not torch.isfinite(b[bad]).any()
+    ok = ~bad & torch.isfinite(b)
+    assert ok.any() and _rel(b[ok], a[ok]) < 4e-3
+
+
 @pytest.mark.parametrize("mode,rot", [("exp_gates", 0), ("decay", 64)])
 @pytest.mark.parametrize("H,D,Dv", [(2, 128, 128), (2, 64, 64), (2, 72, 40)])
 @pytest.mark.parametrize("where,value", [("v", float("inf")), ("v", float("nan")), ("k", float("-inf")),
@@ -139,12 +156,15 @@ def test_linear_rows_that_are_not_finite(where, value, H, D, Dv, mode, rot, monk
     assert bool(live.all()) == (where in ("", "q"))
     assert torch.equal(torch.isfinite(R), live)
     assert _rel(R[live], S[live]) < 2e-6
-    # outputs of the other head, of the other sequence, and before the row's block of sixteen
+    # outputs of the other head, of the other sequence, and before the row's block of sixteen; a query is its row's own
     same = torch.ones(T, H, Dv, dtype=torch.bool)
-    if where:
+    if where == "q":
+        same[hit, 1] = False
+    elif where:
         same[0 if where == "S" else hit // 16 * 16:lens[0], 1] = False
     same = same.view(T, H * Dv)
     assert torch.isfinite(z[same]).all() and _rel(z[same], y[same]) < 4e-3
+    _stays_not_finite(y, z, H, 5 if value == float("inf") and where == "v" else None, where != "")
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
@@ -256,6 +276,8 @@ def test_delta_rows_that_are_not_finite(where, value, H, G, D, Dv, monkeypatch):
 
     y, S, z, Z, _ = _delta_chunks(lens, H, G, D, Dv, torch.bfloat16, monkeypatch, plant)
     fine, ok = torch.isfinite(S), torch.isfinite(y) & torch.isfinite(z)
+    if value != 3.4e38:                        # (at the edge of fp32's range the order of sums decides)
+        _stays_not_finite(y, z, H, 5 if value == float("inf") and where == "v" else None, where != "")
     assert torch.equal(torch.isfinite(Z), fine)
     assert _rel(z[ok], y[ok]) < 4e-3 and _rel(Z[fine], S[fine]) < 4e-6              # as above
     first = H - (1 if where in ("v", "S") else H // G)                  # heads that meet it

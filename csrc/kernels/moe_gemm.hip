@@ -285,13 +285,20 @@ moe_grouped_mfma_kernel(GroupedArgs a) {
 // a random routing shorter and longer than the mean.  A K step of a tile costs its products (0.06 per 64
 // x 64), its reads (0.03 per 64 rows) and a constant; fitted to 76 measured shapes (2 to 64 experts, 32 to
 // 1024 rows), where its choice is within 1 % of the best form in the mean and 12 % at worst (always form 0:
-// 9 % in the mean, always form 1: 7 %).  Wide tiles of up to a unit and a half of rows never won.
+// 9 % in the mean, always form 1: 7 %).  Wide tiles of up to a unit and a half of rows never won.  Up to 104 rows, where
+// hardly a slice needs more than form 0's two units, they are left out too where form 0 just fills the chip, two
+// workgroups on every CU, whose overlap the estimate does not see.  The op with 100 rows an expert without / with wide tiles,
+// us: 512 tiles of form 0, 64 experts of 1024 x 512 70 / 75, 32 of 1024 x 1024 66 / 68, 16 of 1024 x 2048 65 / 67, 8 of
+// 4096 x 4096 197 / 206; 384, 32 of 2048 x 768 94 / 90, 8 of 2048 x 3072 (97 rows) 100 / 91; 1024, 8 of 3072 x 8192
+// 286 / 278; 1792, 8 of 4096 x 14336 604 / 588.  With 120 rows 64 of 1024 x 512 95 / 81, 32 of 1024 x 1024 84 / 79.
 static int grouped_form(float avg, int E, int N, int K) {
   constexpr int MM[3] = {2, 5, 4}, NU[3] = {2, 2, 4};
+  const int tiles0 = E * (N / 128);
+  const bool fills = avg <= 104.f && tiles0 > 384 && tiles0 <= 512;
   int best = 0;
   float least = 0.f;
   for (int f = 0; f < 3; ++f) {
-    if (f == 2 && (N % 256 != 0 || avg <= 96.f)) continue;
+    if (f == 2 && (N % 256 != 0 || avg <= 96.f || fills)) continue;
     float tiles = 0.f, work = 0.f, longest = 0.f;
     for (int z = -1; z <= 1; ++z) {
       const float units = ceilf(fmaxf(1.f, floorf(avg + 1.8f * z * sqrtf(avg))) / 64.f);

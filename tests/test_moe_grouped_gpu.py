@@ -64,14 +64,16 @@ def test_grouped_gemm_large_tiles(counts, K, form):
 
 
 @pytest.mark.parametrize("form", [0, 1, 2])
-@pytest.mark.parametrize("K", [2048, 2112, 4096])
-@pytest.mark.parametrize("counts", [[1, 64, 65, 128, 129, 192, 193, 0], [130, 191, 127, 63, 66, 256, 1, 190]])
-def test_grouped_gemm_few_rows_of_long_experts(counts, K, form):
-    """Up to 128 rows an expert (a step's accesses in front of its products), slices of one to five units."""
+@pytest.mark.parametrize("K,N", [(2048, 256), (2112, 256), (4096, 256), (128, 8192), (64, 7936), (64, 8448)])
+@pytest.mark.parametrize("counts", [[1, 64, 65, 128, 129, 192, 193, 0], [130, 191, 127, 63, 66, 256, 1, 190],
+                                    [100, 101, 99, 98, 97, 129, 102, 104]])
+def test_grouped_gemm_few_rows_of_long_experts(counts, K, N, form):
+    """Up to 128 rows an expert (a step's accesses in front of its products), slices of one to five units; and
+    launches of 496, 512 and 528 tiles of 128 x 128, of which the first two leave wide tiles out at 104 rows."""
     from enterprise_inference_amd._native import kernels as lib
     from enterprise_inference_amd.ops._dispatch import ptr, stream
     g = torch.Generator().manual_seed(K + form)
-    E, n, N = len(counts), sum(counts), 256
+    E, n = len(counts), sum(counts)
     assert n <= 128 * E
     X = torch.randn(300, K, generator=g).to("cuda", BF)
     row_idx = torch.randint(0, 300, (n,), generator=g).to("cuda", torch.int32)

@@ -694,10 +694,17 @@ EIA_DEV void scan_state(const DeltaArgs& a, const ScanAt& k, f32x4 (&S)[NDG][NC]
         if (put) {
           if (in) k.Sg[(long)r * a.Dv + col] = S[o][j][i] * f;
         } else {
-          S[o][j][i] = in && !k.fresh ? k.Sg[(long)r * a.Dv + col] * f : 0.f;
+          S[o][j][i] = in && !k.fresh ? k.Sg[(long)r * a.Dv + col] : 0.f;
         }
       }
     }
+  if (!put) {                                          // (beside its load each product would wait for it)
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int o = 0; o < NDG; ++o)
+#pragma unroll
+      for (int j = 0; j < NC; ++j) S[o][j] *= f;
+  }
 }
 template <int NC>
 EIA_DEV void scan_put_out(const DeltaArgs& a, const DeltaChunkArgs& c, const ScanAt& k, int ch, const f32x4 (&o)[NC], float f) {

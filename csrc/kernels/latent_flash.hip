@@ -11,7 +11,7 @@
 // bf16 high part plus a remainder, normaliser over the fp32 values, deferred rescale.  Rows of an LDS
 // tile are an odd number of 16-byte units apart, so that sixteen rows lie on different banks.
 //
-// MI355X, one 4096-token causal prompt: 8 heads, R 128 + 32: 72 + 12 us in parts; 8 heads, R 256 + 64: 202 us; 16
+// MI355X, one 4096-token causal prompt: 8 heads, R 128 + 32: 71 + 9 us in parts; 8 heads, R 256 + 64: 202 us; 16
 // heads, R 512 + 64: 915, with a window of 1024 488.  With the page of a tile looked up by its fetch, every read of LDS in
 // front of its product, no priorities and parts in more than one round 82 + 12, 299, 1100 and 573 us.
 // A wave's registers hold the sums of 32 rows over 256 columns beside its queries only alone on its
@@ -355,7 +355,7 @@ latent_flash_kernel(LatentFlashArgs a) {
 
 // The parts of a row block put together: the rows, lanes and registers of the kernel above, a workgroup
 // for each 32 columns of every wave's part (one for all of them, one wave per SIMD that reads part after part:
-// 16.4 instead of 12.2 us for 256 row blocks of up to 5 parts x 69 KB).
+// 16.4 instead of 12.2 us for 256 row blocks of up to 5 parts x 69 KB; of up to 3 parts 8.2).
 template <int NDV, int KT, int CS>
 __global__ void __launch_bounds__(256)
 latent_flash_merge_kernel(LatentFlashArgs a) {

@@ -1320,6 +1320,8 @@ EIA_DEV bool ls_out_bf16(const ScanArgs& a, const KChunkArgs& c, const LsChunk& 
   return !__syncthreads_or(bad);
 }
 
+// Two workgroups on a CU where the LDS holds two: 128 registers a lane, of which aligned, unrotated heads of 128 spill 14.
+// One with all registers: four gated prompts of up to 2000 tokens, 16 heads, the op 123 -> 150 us.
 template <typename T, bool VEC, bool ROT, int MX>
 __global__ void __launch_bounds__(512, 4)
 ls_chunk_out_kernel(ScanArgs a, KChunkArgs c) {

@@ -19,7 +19,7 @@
 // before its fetch, and keys are read four fragments ahead of their products.
 //
 // Four ragged prompts of up to 2048 tokens, 16 heads of 128 on 4, window 1024, soft-capped: 65 us on an
-// MI355X (249 us in the 16-query form); one 4096-token causal prompt, 8 heads on 2: 64 + 12 us in
+// MI355X (249 us in the 16-query form); one 4096-token causal prompt, 8 heads on 2: 65 + 9 us in
 // parts (459 us).  With the page looked up by the fetch, each read in front of its product and no priorities 72 and 75 +
 // 12 us (parts of 13 tiles; 70 + 12 with both): of a tile's 5600 cycles (two workgroups on a CU) the fetch took 1100.  What bounds it now is issue: 1540 cycles of
 // matrix products and 1800 (soft-capped 3300) of vector instructions a tile and wave, two waves on a SIMD.
@@ -408,7 +408,7 @@ window_flash_kernel(FlashArgs a) {
 
 // The parts of a row block put together: the rows, lanes and registers of the kernel above, a workgroup
 // for each 32 columns.  Bound by the parts' traffic and by the dependent reads in front of it: 256 row blocks of
-// up to 5 parts x 69 KB, 44 MB in all, take 12.4 us; with one workgroup for all columns of a row block (one
+// up to 5 parts x 69 KB, 44 MB in all, take 12.4 us (of up to 3 parts 8.4); with one workgroup for all columns of a row block (one
 // wave per SIMD, part after part) 16.4 us.
 template <int NDV, bool SIG>
 __global__ void __launch_bounds__(256)

@@ -17,7 +17,7 @@ launch also rotates an attention mixer's queries and keys from the same projecti
 its cache.  ``delta_scan`` runs the recurrence: token by token (decode rows, short portions, heads
 up to 256 wide), or -- prompt portions on the GPU, heads up to 128 wide -- chunk by chunk of 64
 tokens: every chunk's triangular system is solved in parallel, a scan over a sequence's chunks
-carries the state, and all outputs are formed in parallel.
+carries the state and forms the outputs beside it, and these are normalised in parallel.
 
 A sequence whose first row of the step is position 0 starts from zeros whatever its slot held.
 Batch layout: [decode rows (one per sequence) | prefill portions]; ``md.seq_slots`` names the slots
@@ -38,7 +38,9 @@ from .window_attention import PREP_MAX_TAPS, PREP_ROWS, PrepSpec, _prep_ref, bui
 
 CHUNK = 64                 # tokens per chunk of the chunk-parallel form (delta_scan.hip DC)
 CHUNK_MAX_DIM = 128        # ... and its largest dk / dv
-CHUNK_MIN_ROWS = 48        # a portion with at least this many rows selects it
+# a portion with at least this many rows selects it.  us, token by token / chunks, 16 heads of 128 on 8: 1 x 32 rows 52 / 30,
+# 1 x 48 75 / 30, 16 x 48 84 / 60; 32 of 64 on 16: 1 x 48 53 / 27, 16 x 48 65 / 54 (drawn where the form of then was level)
+CHUNK_MIN_ROWS = 48
 # tests and measurements: take the chunk-parallel form for every step that has prompt portions (1),
 # or never (0)
 FORCE_CHUNKED = {"0": False, "1": True}.get(os.environ.get("EIA_DELTA_FORCE_CHUNKED", ""))

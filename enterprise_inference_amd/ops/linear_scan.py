@@ -150,11 +150,13 @@ class ChunkPlan:
         former costs 30 us for its launches and 0.7 ns (2 ns) per row and head, a short sequence
         counting as 96 rows; with a decay per key channel 0.8 ns (1.7 ns, 64 rows), and 5 ns (7 ns)
         for keys above KEY_DIM64, against 0.6 us (1.0 us) a token.  MI355X, 16 heads of 128,
-        exponential gates, token by token / chunks: 1 x 48 rows 62 / 29 us, 1 x 4096 4793 / 145,
-        16 x 64 84 / 63, 16 x 512 599 / 196; 32 heads of 64, fixed decays: 1 x 48 24 / 27, 16 x 64
-        34 / 47, 16 x 128 75 / 68, 1 x 4096 2035 / 104; 16 heads of 64 x 128, a decay per channel: 1 x
-        48 52 / 36, 16 x 64 70 / 60, 16 x 512 536 / 185, 1 x 4096 4307 / 122; 32 of 32 x 64: 1 x 48
-        33 / 31, 16 x 64 48 / 56, 16 x 128 93 / 87, 64 x 64 128 / 142."""
+        exponential gates, token by token / chunks: 1 x 48 rows 64 / 31 us, 1 x 4096 4815 / 91,
+        16 x 64 89 / 59, 16 x 512 604 / 144; 32 heads of 64, fixed decays: 1 x 48 27 / 28, 16 x 64
+        40 / 50, 16 x 128 81 / 74, 1 x 4096 2041 / 82; 16 heads of 64 x 128, a decay per channel: 1 x
+        48 54 / 38, 16 x 64 75 / 67, 16 x 512 538 / 215, 1 x 4096 4316 / 125; 32 of 32 x 64: 1 x 48
+        35 / 33, 16 x 64 52 / 74, 16 x 128 96 / 91, 64 x 64 135 / 199.  The costs were fitted to chunks in fp32
+        products (16 x 64 rows of 16 heads 63 us, 1 x 4096 145): some steps near the line, 16 x 64 rows of 16 heads and
+        16 x 128 of 32 among them, take the token form although chunks are faster now."""
         wide = dim > 64
         if channel and key_dim <= KEY_DIM64:
             busy = self.nseq * heads / (cus if wide else 2.7 * cus)

@@ -211,32 +211,34 @@ GROUPED_MAX_ROWS = 384
 
 
 def _grouped_max_rows(I: int, H: int) -> int:
-    """us, grouped / per expert with its read-back, at 256 and 384 rows per expert: 8 experts of 4096 x
-    14336 1086 / 1226, 1489 / 1478; 16 of 5120 x 8192 1532 / 1832, 2090 / 2271; 16 of 2048 x 4096 345 /
-    946, 442 / 955; only of 6144 x 16384, 1819 / 1967 and 2577 / 2293, the library wins before 384."""
+    """The limits were drawn with a GEMM of 128 x 128 tiles, to which the library was equal at 384 rows (8 experts of
+    4096 x 14336 1489 / 1478 us) or better before (6144 x 16384).  us, the GEMM of now / per expert with its
+    read-back, at 256 and 384 rows per expert: 8 experts of 4096 x 14336 944 / 1294, 1180 / 1484 (at 512 1548 /
+    1890); 16 of 5120 x 8192 1301 / 1912, 1734 / 2301; 16 of 2048 x 4096 290 / 902, 398 / 903; 8 of 6144 x 16384 1886 /
+    1871, 2151 / 2318.  So they lie where the grouped form still wins, and could lie higher."""
     return GROUPED_MAX_ROWS if I * H < 1 << 26 else 256
 
 
 def _mfma_pays(avg: float, El: int, I: int, H: int) -> bool:
     """Whether the MFMA grouped GEMM beats the weight-streaming skinny one at ``avg`` rows per expert.
     The skinny kernel goes over the weights once per 16 to 128 rows, with more columns in flight from 49
-    and from 73 rows on; the MFMA kernel once per 128, but its down projection has only El * H / 128
+    and from 73 rows on; the MFMA kernel once per 128 to 320, but its down projection has only El * H / 128
     tiles, each of I / 64 steps in a row: a few long ones leave the chip idle.
-    us, skinny / MFMA (MI355X), tiles of the down projection in brackets:
-      49, 56, 64 rows: 8 of 4096 x 14336 [256] 556 / 541, -, 655 / 555; 8 of 3072 x 8192 [192] 268 / 260,
-      281 / 260, 309 / 262; 8 of 2048 x 3072 [128] 92 / 83, 100 / 84, 109 / 86; but 8 of 2048 x 4096 [128]
-      104 / 124, 111 / 124, 121 / 125; 8 of 1024 x 2048 [64] 39 / 42, 42 / 43, 45 / 44; 8 of 4096 x 4096
-      [256] 187 / 203, 202 / 203, 224 / 206;
-      (49 only with short rows of tiles, 16 of 4096 x 1024 [512] 140 / 92, or long streams of weights, 8
-      of 4096 x 7168 [256] 321 / 276;)
-      with packed weights and the next add + norm, which takes the skinny form's combine along, 8 of 4096 x
-      14336 537 / 538, 577 / 543, 633 / 548;
-      80 rows: 8 of 2048 x 4096 145 / 126, 4 of 2048 x 4096 [64] 76 / 72; but 2 of 4096 x 8192 [64] 126 /
-      153, 8 of 512 x 4096 [32] 62 / 64.
-    Experts that fill the chip and whose weights stay in the 256 MB cache gain sooner, at 25 and 32 rows:
-    16 of 2048 x 1024 [256] 55 / 44, 65 / 44; 32 of 1024 x 1024 [256] 60 / 43, 68 / 45; 16 of 1024 x 2048
-    [128] 55 / 50, 59 / 52; 8 of 2048 x 2048 [128] 52 / 51, 56 / 52; but 8 of 1024 x 4096 [64] 52 / 67, 54 /
-    68; 8 of 1024 x 2048 [64] 33 / 41, 36 / 43."""
+    us, skinny / MFMA (MI355X, weights from memory), tiles of the down projection in brackets:
+      49, 56, 64 rows: 8 of 4096 x 14336 [256] 604 / 552, 629 / 551, 674 / 566; 8 of 3072 x 8192 [192] 280 / 269,
+      292 / 272, 316 / 276; 8 of 2048 x 3072 [128] 99 / 97, 105 / 98, 114 / 100; but 8 of 2048 x 4096 [128]
+      110 / 116, 117 / 117, 125 / 118; 8 of 1024 x 2048 [64] 42 / 41, 45 / 43, 48 / 45; 8 of 4096 x 4096
+      [256] 196 / 190, 211 / 188, 235 / 189;
+      (49 only with short rows of tiles, 16 of 4096 x 1024 [512] 143 / 103, or long streams of weights, 8
+      of 4096 x 7168 [256] 328 / 301;)
+      80 rows: 8 of 2048 x 4096 152 / 120, 4 of 2048 x 4096 [64] 84 / 85; but 2 of 4096 x 8192 [64] 135 /
+      151, 8 of 512 x 4096 [32] 67 / 62.
+    Experts that fill the chip and fit the 256 MB cache gain sooner, at 25 and 32 rows: 16 of 2048 x 1024 [256] 63 / 58,
+    72 / 59; 32 of 1024 x 1024 [256] 66 / 52, 76 / 53; 16 of 1024 x 2048 [128] 61 / 59, 67 / 60; 8 of 2048 x 2048
+    [128] 59 / 65, 64 / 65 (52 / 51, 56 / 52 with weights in the cache); but 8 of 1024 x 4096 [64] 58 / 71, 61 /
+    72; 8 of 1024 x 2048 [64] 36 / 40, 39 / 40.
+    The lines were drawn with 128 x 128 tiles in one form, before accesses stood in front of the products: several
+    shapes of 49 to 64 rows that they leave to the skinny kernel are level or better on the other one now."""
     down = El * H // 128
     if avg > 72:
         return I < 128 * down

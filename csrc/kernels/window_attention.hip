@@ -929,7 +929,7 @@ EIA_DEV void wa_finish_head(const WinAttnArgs& a, long row, int h, int lane, con
 // times the blocks and most batches need none.  Products, masks and weights as above.
 //
 // Bound by latency: a wave's blocks are a chain of loads, two products and a softmax, 1 us each.
-// MI355X, window 1024, 8 heads on 2, 3 rows: 15.5 us in four partitions (7 of them the merge's launch),
+// MI355X, window 1024, 8 heads on 2, 3 rows: 11 + 4.5 us in four partitions (the merge is a launch of its own),
 // 64 rows: 22, 128 rows: 28 us; a wave per head took 21, 45 and 72 us.
 template <int P, int ND, int NDV, bool SIG>
 __global__ void __launch_bounds__(256, 2)

@@ -151,9 +151,9 @@ def flash_parts(n_items: int, spec: WindowSpec, queries: int, longest: int, cont
                 cus: int = 256):
     """(parts, 64-key tiles per part) of a flash prefill launch whose longest portion has
     ``longest`` queries and whose block tables reach ``context`` tokens; two workgroups fit a CU, three
-    of heads up to 64.  MI355X, 8 heads of 128 on 2, one portion, uncut / cut: 4096 tokens causal 112 /
-    76 us, 2048 59 / 33, 1000 32 / 24, 96 behind 2000 64 / 25; 16 heads on 4: 2048 causal 61 / 47, 4096 140 /
-    133, 1000 behind 1900 81 / 49, with a window of 1024 46 / 35, 2048 with it 43 / 43 in halves."""
+    of heads up to 64.  MI355X, 8 heads of 128 on 2, one portion, uncut / cut: 4096 tokens causal 110 /
+    75 us, 2048 58 / 31, 1000 32 / 23, 96 behind 2000 60 / 23; 16 heads on 4: 2048 causal 59 / 47, 4096 135 /
+    123, 1000 behind 1900 82 / 48, with a window of 1024 39 / 31."""
     tiles = -(-context // 64)
     if spec.window > 0:
         tiles = min(tiles, (spec.window + queries + 62) // 64 + 1 + (spec.keep + 63) // 64)

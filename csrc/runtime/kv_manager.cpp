@@ -292,6 +292,7 @@ class KVCacheManager {
 
 void register_shm(py::module_& m);       // shm_ring.cpp
 void register_grammar(py::module_& m);   // grammar.cpp
+void register_kernel_call(py::module_& m);   // kernel_call.cpp
 
 PYBIND11_MODULE(_eia_runtime, m) {
   m.doc() = "MI355X inference runtime: native KV block manager, batch builder, shm broadcast";
@@ -320,4 +321,5 @@ PYBIND11_MODULE(_eia_runtime, m) {
       .def("stats", &KVCacheManager::stats);
   register_shm(m);
   register_grammar(m);
+  register_kernel_call(m);
 }

@@ -20,6 +20,14 @@ EIA_DEV bool chunk_of(const int* cu, int nseq, int x, int& s, int& row0, int& n)
   return n > 0;
 }
 
+// Grids of a workgroup per (head, chunk): all heads of a chunk run side by side, so that the rows they share a
+// part of each come in whole.  chunk_number: the workgroup's chunk (past the last one: none).
+constexpr int CHUNKS_Y = 32768;
+inline dim3 chunk_grid(int chunks, int H) {
+  return dim3(H, chunks < CHUNKS_Y ? chunks : CHUNKS_Y, (chunks + CHUNKS_Y - 1) / CHUNKS_Y);
+}
+EIA_DEV int chunk_number() { return blockIdx.z * CHUNKS_Y + blockIdx.y; }
+
 // Four columns of a state row over a sequence's nc chunks, us and ls apart: U of a chunk, its own
 // contribution, turns into the state before it; S, the state before the first one, into the state after
 // the last.  L: log2 of a chunk's decay.  A group's contributions are requested while the previous group

@@ -448,10 +448,12 @@ EIA_API int eia_linear_scan(const void* x, long ld, int q_off, int k_off, int v_
 // 128-token chunks: the states between chunks are the larger part of the memory
 // traffic (4 passes over chunks x H x dk x dv floats), and halving their number costs less than the
 // longer sums inside a chunk add.
-// Four prompts of 1000 .. 2000 tokens (6688 rows), 16 heads of 128, mode 1, bf16 take 11 + 33 + 21 +
-// 63 us on an MI355X (gates, (1), (2), (3)); in fp32 products (1) and (3) took 57 + 103 us.  Bound by the
-// workspace and the rows, which (1), (2) and (3) move at 3.4, 5.3 and 3.1 TB/s, and by the steps of
-// a workgroup, which reads, splits and multiplies in turn.
+// Four prompts of 1000 .. 2000 tokens (6688 rows), 16 heads of 128, mode 1, bf16 take 11 + 31 + 21 +
+// 60 us on an MI355X (gates, (1), (2), (3)); in fp32 products (1) and (3) took 57 + 103 us.  Bound by the
+// workspace and the rows, which (1), (2) and (3) move at 3.8, 5.4 and 3.3 TB/s, and by the steps of
+// a workgroup, which reads, splits and multiplies in turn.  All heads of a chunk run side by side in (1) and (3), so
+// that whole rows are read together, and (3) asks for its queries before it waits for the gates: 123 -> 118 us for the
+// op; three rotated prompts of up to 2700 tokens 188 -> 178, five of up to 1100 of 32 heads of 64 78 -> 77.
 constexpr int LK = 128;                     // tokens per chunk
 constexpr float LS_LOG2E = 1.4426950408889634f;
 
@@ -644,21 +646,27 @@ EIA_DEV void ls_stage_v(const ScanArgs& a, int row0, int n, int h, int t0, T* sv
   }
 }
 
+// Log decay and log weight of the chunk's token threadIdx.x, in base 2 (threads 0 .. LK - 1).
+EIA_DEV void ls_log_load(const ScanArgs& a, const KChunkArgs& c, int row0, int n, int h, float& l, float& b) {
+  const int t = threadIdx.x;
+  l = b = 0.f;
+  if (t >= min(n, LK)) return;
+  if (a.mode == 0) {
+    l = a.decay[h];
+  } else {
+    l = c.la[(long)(row0 + t) * a.H + h];
+    b = c.lb[(long)(row0 + t) * a.H + h];
+  }
+}
 // Sums of l over 16-token blocks: pre up to and with a token, suf behind it, tot of whole blocks;
-// mb: m, sl: l.  Threads 0 .. LK - 1.
-EIA_DEV void ls_chunk_logs(const ScanArgs& a, const KChunkArgs& c, int row0, int n, int h, float* pre,
-                           float* suf, float* tot, float* mb, float* sl) {
+// mb: m, sl: l.  Threads 0 .. LK - 1, l and b as ls_log_load leaves them.
+EIA_DEV void ls_chunk_logs(const ScanArgs& a, int n, float l, float b, float* pre, float* suf, float* tot, float* mb,
+                           float* sl) {
   const int t = threadIdx.x;
   if (t >= LK) return;
-  float l = 0.f, b = 0.f;
-  if (t < n) {
-    if (a.mode == 0) {
-      l = logf(a.decay[h]) * LS_LOG2E;
-    } else {
-      l = c.la[(long)(row0 + t) * a.H + h] * LS_LOG2E;
-      b = c.lb[(long)(row0 + t) * a.H + h] * LS_LOG2E;
-    }
-  }
+  if (a.mode == 0) l = t < n ? logf(l) : 0.f;
+  l *= LS_LOG2E;
+  b *= LS_LOG2E;
   l = l < -150.f ? -150.f : l;                         // (2^-150 is zero; what is no number stays so)
   sl[t] = l;
   float p = l, s = l;
@@ -897,10 +905,12 @@ ls_chunk_state_kernel(ScanArgs a, KChunkArgs c) {
   __shared__ __align__(16) unsigned char tiles[FP32 > SPLIT ? FP32 : SPLIT];
   __shared__ float pre[LK], suf[LK], mb[LK], tot[LK / 16], sl[LK];
   int s, row0, n;
-  if (!ls_chunk(a, c.nseq, blockIdx.x, s, row0, n)) return;
-  const int h = blockIdx.y;
-  ls_chunk_logs(a, c, row0, n, h, pre, suf, tot, mb, sl);
-  const long at = (long)blockIdx.x * a.H + h;
+  if (!ls_chunk(a, c.nseq, chunk_number(), s, row0, n)) return;
+  const int h = blockIdx.x;
+  float l, b;
+  ls_log_load(a, c, row0, n, h, l, b);
+  ls_chunk_logs(a, n, l, b, pre, suf, tot, mb, sl);
+  const long at = (long)chunk_number() * a.H + h;
   const LsChunk k{row0, n, h, pre, suf, mb, tot, sl};
   if constexpr (BF) {
     if (!ls_state_bf16<VEC, ROT, MX>(a, c, k, at, tiles)) ls_state_fp32<T, VEC, ROT, MX>(a, c, k, at, tiles);
@@ -965,7 +975,7 @@ EIA_DEV void ls_out_fp32(const ScanArgs& a, const KChunkArgs& c, const LsChunk& 
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int w = wv < 4 ? wv : 11 - wv, l16 = lane & 15, g4 = lane >> 4, t0 = 16 * w;
   if (state) {                                         // straight to LDS, 1 KB per access
-    const float* S = c.U + ((long)blockIdx.x * a.H + h) * c.DP * c.UW;
+    const float* S = c.U + ((long)chunk_number() * a.H + h) * c.DP * c.UW;
 #pragma unroll
     for (int u = 0; u < MX * MX / 256 / 8; ++u) {
       const int at = 256 * (8 * u + wv), r = (at + 4 * lane) / MX, d = (at + 4 * lane) % MX;
@@ -1128,33 +1138,49 @@ EIA_DEV bool ls_out_bf16(const ScanArgs& a, const KChunkArgs& c, const LsChunk& 
   f32x4 sf[4];
   auto fetch = [&](int x) {
     if (!state || sr >= 64) return;
-    const float* S = c.U + (((long)blockIdx.x * a.H + h) * c.DP + min(64 * x + sr, c.DP - 1)) * c.UW +
+    const float* S = c.U + (((long)chunk_number() * a.H + h) * c.DP + min(64 * x + sr, c.DP - 1)) * c.UW +
                      (16 * su < c.VP ? 16 * su : 0);
 #pragma unroll
     for (int e = 0; e < 4; ++e) sf[e] = *reinterpret_cast<const f32x4*>(S + 4 * e);
   };
-  fetch(0);
-  ls_chunk_logs(a, c, row0, n, h, logs, logs + LK, logs + 4 * LK, logs + 2 * LK, logs + 3 * LK);
-  __syncthreads();
+  float l, b;
+  ls_log_load(a, c, row0, n, h, l, b);
   bf16x8 qf[NQ][NX];                                   // this lane's query: channels 32 x + 8 g4 + e
+  auto queries = [&](bool use) {                       // use: q . n, else nothing but qf
+    float z = 0.f;
+#pragma unroll
+    for (int x = 0; x < NX; ++x) {
+      float v[8];
+      ls_head8<bf16_t, VEC, ROT>(a, c, row0 + min(tq, n - 1), a.q_off + (long)h * D, 32 * x + 8 * g4, v);
+      if constexpr (ROT) {
+        bf16x8 part[3];
+        split3(v, part);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) qf[p][x] = part[p];
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) qf[0][x][e] = (bf16_t)v[e];
+      }
+      if (use) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) z += v[e] * sn[32 * x + 8 * g4 + e];
+      }
+    }
+    return z;
+  };
+  const bool norm = a.mode == 1 && state;
+  if constexpr (!ROT) queries(false);                  // (asked for before the state and the logs are waited for)
+  fetch(0);
+  ls_chunk_logs(a, n, l, b, logs, logs + LK, logs + 4 * LK, logs + 2 * LK, logs + 3 * LK);
+  __syncthreads();
   float nq = 0.f;
+  if constexpr (ROT) {
+    nq = queries(norm);
+  } else if (norm) {
 #pragma unroll
-  for (int x = 0; x < NX; ++x) {
-    float v[8];
-    ls_head8<bf16_t, VEC, ROT>(a, c, row0 + min(tq, n - 1), a.q_off + (long)h * D, 32 * x + 8 * g4, v);
-    if constexpr (ROT) {
-      bf16x8 part[3];
-      split3(v, part);
+    for (int x = 0; x < NX; ++x)
 #pragma unroll
-      for (int p = 0; p < 3; ++p) qf[p][x] = part[p];
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) qf[0][x][e] = (bf16_t)v[e];
-    }
-    if (a.mode == 1 && state) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) nq += v[e] * sn[32 * x + 8 * g4 + e];
-    }
+      for (int e = 0; e < 8; ++e) nq += (float)qf[0][x][e] * sn[32 * x + 8 * g4 + e];
   }
 #pragma unroll
   for (int j = 0; j < MX / 16; ++j) o[j] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -1332,12 +1358,12 @@ ls_chunk_out_kernel(ScanArgs a, KChunkArgs c) {
   __shared__ __align__(16) float logs[4 * LK + LK / 16], sn[MX];
   float *pre = logs, *suf = logs + LK, *mb = logs + 2 * LK, *sl = logs + 3 * LK, *tot = logs + 4 * LK;
   int s, row0, n;
-  if (!ls_chunk(a, c.nseq, blockIdx.x, s, row0, n)) return;
-  const int h = blockIdx.y, lane = threadIdx.x & 63, wv = threadIdx.x >> 6, Dv = a.Dv;
+  if (!ls_chunk(a, c.nseq, chunk_number(), s, row0, n)) return;
+  const int h = blockIdx.x, lane = threadIdx.x & 63, wv = threadIdx.x >> 6, Dv = a.Dv;
   const int w = wv < 4 ? wv : 11 - wv, l16 = lane & 15, g4 = lane >> 4, t0 = 16 * w;
   const bool state = row0 != a.cu[s] || a.positions[a.cu[s]] != 0;   // (else a fresh sequence: S = 0)
   if (state && a.mode == 1 && threadIdx.x < MX)
-    sn[threadIdx.x] = c.U[(((long)blockIdx.x * a.H + h) * c.DP + min((int)threadIdx.x, c.DP - 1)) * c.UW + c.VP];
+    sn[threadIdx.x] = c.U[(((long)chunk_number() * a.H + h) * c.DP + min((int)threadIdx.x, c.DP - 1)) * c.UW + c.VP];
   const LsChunk k{row0, n, h, pre, suf, mb, tot, sl};
   f32x4 o[MX / 16];
   float rs;
@@ -1345,7 +1371,9 @@ ls_chunk_out_kernel(ScanArgs a, KChunkArgs c) {
     if (!ls_out_bf16<VEC, ROT, MX>(a, c, k, state, tiles, sn, o, rs, logs))
       ls_out_fp32<T, VEC, ROT, MX>(a, c, k, state, tiles, sn, o, rs);
   } else {
-    ls_chunk_logs(a, c, row0, n, h, pre, suf, tot, mb, sl);
+    float l, b;
+    ls_log_load(a, c, row0, n, h, l, b);
+    ls_chunk_logs(a, n, l, b, pre, suf, tot, mb, sl);
     __syncthreads();
     ls_out_fp32<T, VEC, ROT, MX>(a, c, k, state, tiles, sn, o, rs);
   }
@@ -1408,7 +1436,7 @@ ls_chunk_out_kernel(ScanArgs a, KChunkArgs c) {
 
 template <typename T, bool VEC, bool ROT, int MX>
 static void ls_chunked(const ScanArgs& a, const KChunkArgs& c, hipStream_t st) {
-  const dim3 gc(c.rows / LK + c.nseq, a.H), gs(c.nseq, a.H);
+  const dim3 gc = chunk_grid(c.rows / LK + c.nseq, a.H), gs(c.nseq, a.H);
   const dim3 gz(c.nseq, a.H, (c.DP * c.UW / 4 + 255) / 256);
   // 512 threads take 2048 tokens at once, 256 take 1024.  Some sequence needs a second pass of 256 where the rows
   // are more than 1024 per sequence: the whole op at 4 x 2000 tokens 142 -> 139 us, 1 x 4096 79 -> 73 us with 512;

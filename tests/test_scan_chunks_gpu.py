@@ -527,3 +527,32 @@ def test_gates_that_close_hard(spread, monkeypatch):
         rest = [h for h in range(H) if h != 1]
         assert torch.equal(z[:at_t], y[:at_t]) and torch.isnan(z[at_t:, D:2 * D]).all() and torch.isnan(Z[1]).all()
         assert torch.equal(z.view(T, H, D)[:, rest], y.view(T, H, D)[:, rest]) and torch.equal(Z[rest], S[rest])
+
+
+def test_linear_chunks_past_a_grid_column(monkeypatch):
+    """More chunks than one dimension of the grid takes (chunk_grid: 32768): sequences of one token, whose output is
+    (q . k) v / rms, and a longer one behind them, which comes out as it does alone."""
+    from enterprise_inference_amd.ops import linear_scan as ls
+    monkeypatch.setattr(ls, "FORCE_CHUNKED", True)
+    lens, D = [1] * 32900 + [130], 16
+    n, T = len(lens), sum(lens)
+    g = torch.Generator().manual_seed(5)
+    x = torch.randn(T, 64, generator=g).to(torch.bfloat16).cuda()
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32).cuda()
+    pos = torch.cat([torch.zeros(n - 1), torch.arange(130)]).to(torch.int32).cuda()
+    spec = ls.ScanSpec(1, D, D, "decay", decay=torch.tensor([0.9]).cuda(), eps=1e-5)
+
+    def run(x, cu, n, pos, lens):
+        st = ls.ScanState.allocate(n, spec, "cuda")
+        y = ls.linear_scan(x, 0, D, 2 * D, 3 * D, spec, st, torch.arange(n, dtype=torch.int32).cuda(), cu, n, pos,
+                           plan=ls.chunk_plan(lens, "cuda"))
+        return y, st.S
+
+    y, S = run(x, cu, n, pos, lens)
+    q, k, v, gate = x[:n - 1].float().split(D, 1)
+    o = (q * k).sum(1, keepdim=True) * v
+    want = o / torch.sqrt((o * o).mean(1, keepdim=True) + 1e-5) * torch.nn.functional.silu(gate)
+    assert _rel(y[:n - 1], want) < 4e-3          # (one rounding to bf16 and at times one step more)
+    assert _rel(S[:n - 1, 0], k[:, :, None] * v[:, None, :]) < 2e-6
+    alone, Sa = run(x[n - 1:], torch.tensor([0, 130], dtype=torch.int32).cuda(), 1, pos[n - 1:], [130])
+    assert torch.equal(y[n - 1:], alone) and torch.equal(S[n - 1:], Sa)

@@ -31,6 +31,22 @@ EIA_DEV float wave_max(float v) {
   return v;
 }
 
+// Over the sixteen lanes of a row, in all of them (row_ror by 8, 4, 2, 1: no LDS).
+#define EIA_ROW_ROR(v, n) \
+  __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + (n), 0xf, 0xf, true))
+EIA_DEV float row16_sum(float v) {
+  v += EIA_ROW_ROR(v, 8);
+  v += EIA_ROW_ROR(v, 4);
+  v += EIA_ROW_ROR(v, 2);
+  return v + EIA_ROW_ROR(v, 1);
+}
+EIA_DEV float row16_max(float v) {
+  v = fmaxf(v, EIA_ROW_ROR(v, 8));
+  v = fmaxf(v, EIA_ROW_ROR(v, 4));
+  v = fmaxf(v, EIA_ROW_ROR(v, 2));
+  return fmaxf(v, EIA_ROW_ROR(v, 1));
+}
+
 // Block-wide sum through LDS; `scratch` must hold blockDim.x/64 floats.
 EIA_DEV float block_sum(float v, float* scratch) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;

@@ -265,6 +265,7 @@ struct WinAttnArgs {
   float cap;                        // > 0: scores soft-capped, cap * tanh(s / cap)
   int talk_post;                    // talk mixes the softmax weights, not the scores (scalar form)
   int gate_heads;                   // gate [rows, H]: one value per head
+  int rows;                         // window_decode_kernel and its merge: rows of the launch
 };
 
 // The visible keys of a 16-query tile as absolute 32-key blocks: the blocks of the kept first
@@ -285,8 +286,8 @@ EIA_DEV float wa_softcap(float s, float cap, float icap2) {
 // so short contexts use few partitions whatever the launch's grid.z (the same on both sides of
 // the merge).
 EIA_DEV int wa_parts(int nparts, int nblocks) { return min(nparts, max(1, nblocks >> 1)); }
-// (of window_decode_kernel: two blocks for each of its four waves)
-EIA_DEV int wd_parts(int nparts, int nblocks) { return min(nparts, max(1, nblocks >> 3)); }
+// (of window_decode_kernel: a block for each of its four waves; below 16 blocks the merge costs what it gains)
+EIA_DEV int wd_parts(int nparts, int nblocks) { return nblocks < 16 ? 1 : min(nparts, nblocks >> 2); }
 
 constexpr int WA_KT = 64;           // keys per tile = lanes of a wave
 constexpr int WA_PAGES = 256;       // MFMA form: block -> page entries kept in LDS
@@ -928,20 +929,24 @@ EIA_DEV void wa_finish_head(const WinAttnArgs& a, long row, int h, int lane, con
 // take every fourth 32-key block of the partition and meet in LDS, so that a partition holds four
 // times the blocks and most batches need none.  Products, masks and weights as above.
 //
-// Bound by latency: a wave's blocks are a chain of loads, two products and a softmax, 1 us each.
-// MI355X, window 1024, 8 heads on 2, 3 rows: 11 + 4.5 us in four partitions (the merge is a launch of its own),
-// 64 rows: 22, 128 rows: 28 us; a wave per head took 21, 45 and 72 us.
+// A CU has about 16 KB of reads in flight, one block of 128 + 128, and moves 30 bytes a ns whatever waves and
+// prefetches ask for (eight or sixteen waves, or the next block in flight, were no faster): so small batches are cut
+// into as many partitions as there are CUs.  The workgroups of a row, and of its merge, share an XCD, row % 8 (the
+// grid is padded to it): the partials then meet in that L2.  (Merged by the last workgroup of a row to arrive,
+// through atomics that pass the L2s, the three rows below took 16.9 us.)  MI355X, window 1024, 8 heads of 128 on 2, both
+// launches: 3 rows 15.7 -> 10.4 us, 17 rows 17.0 -> 12.5, 64 rows 22.4 -> 20.7; 8 rows at 4000 tokens without a window
+// 22.2 -> 12.7.
 template <int P, int ND, int NDV, bool SIG>
 __global__ void __launch_bounds__(256, 2)
 window_decode_kernel(const WinAttnArgs a) {
   constexpr float LOG2E = 1.4426950408889634f;
-  constexpr bool PIPE = P == 1;                         // the next block's operands are in flight
   extern __shared__ float so[];                         // [4][P][rep][Dv]
   __shared__ float sm[4][P][16], sl[4][P][16];
   __shared__ int page_s[WA_PAGES];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, c = lane & 15, g = lane >> 4;
   const int H = a.H, D = a.D, Dv = a.Dv, M = H * P, rep = H / a.G, bs = a.bs, kvh = blockIdx.y;
   const long row = blockIdx.x;
+  if (row >= a.rows) return;
   const int h0 = kvh * rep;
   bf16_t* out = (bf16_t*)a.out + row * a.ldo + (long)h0 * Dv;
   if (a.lens && a.lens[row] <= 0) {                     // padding row: zeros
@@ -1079,22 +1084,10 @@ window_decode_kernel(const WinAttnArgs a) {
       }
     }
   };
-  if constexpr (PIPE) {
-    Ops o0, o1;
-    if (b_lo + w < b_hi) load(b_lo + w, o0);
-    for (int b = b_lo + w; b < b_hi; b += 8) {
-      if (b + 4 < b_hi) load(b + 4, o1);
-      block(b, o0);
-      if (b + 4 >= b_hi) break;
-      if (b + 8 < b_hi) load(b + 8, o0);
-      block(b + 4, o1);
-    }
-  } else {
-    Ops o;
-    for (int b = b_lo + w; b < b_hi; b += 4) {
-      load(b, o);
-      block(b, o);
-    }
+  Ops o;
+  for (int b = b_lo + w; b < b_hi; b += 4) {
+    load(b, o);
+    block(b, o);
   }
   // the waves' sums meet: this lane holds, per map and tile t, value columns 16 t + 4 g + i of head c
   if (c < rep) {
@@ -1144,33 +1137,61 @@ window_decode_kernel(const WinAttnArgs a) {
 }
 
 // Merge of key partitions and the row's epilogue: one wave per (row, head).  Lane z first turns
-// partition z's (max, sum) into its weight; the value columns are then summed over the partitions
-// with independent loads (nparts <= 64).
+// partition z's (max, sum) into its weight; the value columns are then summed over the partitions.
+// Bound by latency: the partials of up to 16 partitions are asked for together with the weights' inputs, and these
+// meet within rows of 16 lanes (three rows of 8 heads, 8 partitions: 4.8 -> 2.9 us).
+constexpr int WM_Z = 16;
 template <bool PACKED>
 __global__ void __launch_bounds__(64)
 window_attn_merge_kernel(const WinAttnArgs a) {
   const int H = a.H, P = a.P, Dv = a.Dv, M = H * P, NP = a.nparts;
   const long row = blockIdx.x;
   const int h = blockIdx.y, lane = threadIdx.x;
-  if (a.lens && a.lens[row] <= 0) return;           // padding row: the partition kernel wrote zeros
-  const int pos = a.positions[row];
+  if (row >= a.rows) return;
+  const int pos = a.positions[row], len = (a.lens ? a.lens : a.positions)[row];
+  if (a.lens && len <= 0) return;                   // padding row: the partition kernel wrote zeros
   const int nblocks = wa_blocks(pos, pos, a.window, a.keep).nblocks;
   const int np = PACKED ? wd_parts(NP, nblocks) : wa_parts(NP, nblocks);
   if (np == 1) return;                              // a whole row: already finished and written
+  const int d0 = min(lane, Dv - 1), d1 = min(lane + 64, Dv - 1);
   float o[2][2];                                    // [map][column lane, lane + 64]
   for (int pm = 0; pm < P; ++pm) {
     const long pr = (row * M + h * P + pm) * NP;
-    const float mz = lane < np ? a.part_ml[(pr + lane) * 2] : -1e30f;
-    const float lz = lane < np ? a.part_ml[(pr + lane) * 2 + 1] : 0.f;
-    // sigmoid weights: the partitions' sums simply add up
-    const float wz = a.wmode == 1 ? (lane < np ? 1.f : 0.f) : __expf(mz - wave_max(mz));
-    const float inv = a.wmode == 1 ? 1.f : 1.0f / wave_sum(wz * lz);
-    float v0 = 0.f, v1 = 0.f;
-#pragma unroll 4
-    for (int z = 0; z < np; ++z) {
-      const float w = __shfl(wz, z, 64);
-      if (lane < Dv) v0 += w * a.part_acc[(pr + z) * Dv + lane];
-      if (lane + 64 < Dv) v1 += w * a.part_acc[(pr + z) * Dv + lane + 64];
+    float v0 = 0.f, v1 = 0.f, inv;
+    if (np <= WM_Z) {
+      float x0[WM_Z], x1[WM_Z];
+      const int z = lane & 15;
+      const float mz = z < np ? a.part_ml[(pr + z) * 2] : -1e30f;
+      const float lz = z < np ? a.part_ml[(pr + z) * 2 + 1] : 0.f;
+#pragma unroll
+      for (int y = 0; y < WM_Z; ++y) {              // (past the last one: the last one, with no weight)
+        const float* p = a.part_acc + (pr + min(y, np - 1)) * Dv;
+        x0[y] = p[d0];
+        x1[y] = p[d1];
+      }
+      // sigmoid weights: the partitions' sums simply add up
+      const float top = row16_max(mz);              // (of all lanes: none may have branched off)
+      const float wz = z >= np ? 0.f : a.wmode == 1 ? 1.f : __expf(mz - top);
+      inv = a.wmode == 1 ? 1.f : 1.0f / row16_sum(wz * lz);
+#pragma unroll
+      for (int y = 0; y < WM_Z; ++y) {
+        const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wz), y));
+        if (y < np) {                               // (a sum that is not finite stays in its partition)
+          v0 += w * x0[y];
+          v1 += w * x1[y];
+        }
+      }
+    } else {                                        // nparts <= 64
+      const float mz = lane < np ? a.part_ml[(pr + lane) * 2] : -1e30f;
+      const float lz = lane < np ? a.part_ml[(pr + lane) * 2 + 1] : 0.f;
+      const float top = wave_max(mz);
+      const float wz = lane >= np ? 0.f : a.wmode == 1 ? 1.f : __expf(mz - top);
+      inv = a.wmode == 1 ? 1.f : 1.0f / wave_sum(wz * lz);
+      for (int z = 0; z < np; ++z) {
+        const float w = __shfl(wz, z, 64);
+        v0 += w * a.part_acc[(pr + z) * Dv + d0];
+        v1 += w * a.part_acc[(pr + z) * Dv + d1];
+      }
     }
     o[pm][0] = v0 * inv;
     o[pm][1] = v1 * inv;
@@ -1222,7 +1243,7 @@ EIA_API int eia_window_attn_mfma(const void* q, long ldq, const void* kc, const 
   if (n_items == 0) return EIA_OK;
   WinAttnArgs a{q, ldq, kc, vc, bt, ldbt, positions, cu, work, lens, mult, slope, talk, gate, ldg,
                 out, ldo, H, G, P, D, Dv, bs, window, keep, 16, epilogue, lam, eps, post, nparts,
-                2, part_acc, part_ml, wmode, bias, sink, cap, 0, gate_heads};
+                2, part_acc, part_ml, wmode, bias, sink, cap, 0, gate_heads, n_items};
   const bool packed = !cu && !talk && eia_window_decode_packed(H, G);
   // raw-score buffers of the head-mixing form: two (one barrier per block) while they fit 48 KiB
   if (talk) a.raw_bufs = (size_t)2 * H * P * 128 * sizeof(f32x4) > 48 * 1024 ? 1 : 2;
@@ -1262,7 +1283,8 @@ EIA_API int eia_window_attn_mfma(const void* q, long ldq, const void* kc, const 
                          block, lds, st, a);                                                    \
   } while (0)
   if (packed) {
-    const dim3 dg(n_items, G, nparts), db(256);
+    const int rows8 = nparts > 1 ? (n_items + 7) / 8 * 8 : n_items;      // (a row's workgroups on one XCD)
+    const dim3 dg(rows8, G, nparts), db(256);
     const size_t dl = sizeof(float) * 4 * P * (H / G) * Dv;
 #define WD_GO(PV, NDX, NDVX, SG)                                                                \
   do {                                                                                          \
@@ -1280,7 +1302,7 @@ EIA_API int eia_window_attn_mfma(const void* q, long ldq, const void* kc, const 
 #undef WD_DIMS
 #undef WD_GO
     if (nparts > 1)
-      hipLaunchKernelGGL(window_attn_merge_kernel<true>, dim3(n_items, H), dim3(64), 0, st, a);
+      hipLaunchKernelGGL(window_attn_merge_kernel<true>, dim3(rows8, H), dim3(64), 0, st, a);
     EIA_LAUNCH_CHECK();
   }
   // without head mixing the key width may be half the value width (a differential pair)

@@ -1,0 +1,84 @@
+"""Decode rows in key partitions, against the ops' own plain CPU path: rows that the grid is padded for, a padding
+row, lengths where a row has one partition more or less, and more partitions than the merge takes at once."""
+
+import pytest
+import torch
+
+from enterprise_inference_amd.ops import attention as A
+from enterprise_inference_amd.ops import window_attention as WA
+
+PAGE = 64
+
+
+def _rel(a, b):
+    a, b = a.double().cpu(), b.double().cpu()
+    return float((a - b).norm() / b.norm())
+
+
+def _step(lens, g):
+    """Metadata of a decode step; a length of 0 is a padding row."""
+    pages = [-(-max(n, 1) // PAGE) for n in lens]
+    order = torch.randperm(sum(pages), generator=g).to(torch.int32)
+    table = torch.zeros(len(lens), max(pages), dtype=torch.int32)
+    at = 0
+    for s, k in enumerate(pages):
+        table[s, :k] = order[at:at + k]
+        at += k
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32)
+    return dict(slot_mapping=i32([0] * len(lens)), positions=i32([max(n - 1, 0) for n in lens]), num_seqs=len(lens),
+                num_decode=len(lens), num_prefill_tokens=0, decode_block_tables=table, decode_seq_lens=i32(lens)), sum(pages)
+
+
+def _both(call, tensors, md, lens):
+    """On the CPU and on the GPU, live rows."""
+    live = torch.tensor([n > 0 for n in lens])
+    out = []
+    for dev in ("cpu", "cuda"):
+        m = A.AttentionMetadata(**{k: v.to(dev) if isinstance(v, torch.Tensor) else v for k, v in md.items()})
+        out.append(call(dev, [None if t is None else t.to(dev) for t in tensors], m).cpu()[live])
+    return out
+
+
+LENS = {"edges": [1, 449, 480, 481, 512, 513, 544, 0, 2100], "one": [900], "few": [1500, 33, 1024]}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("parts", [0, 5, 23])
+@pytest.mark.parametrize("lens", LENS.values(), ids=LENS.keys())
+@pytest.mark.parametrize("kind,D,Dv,window", [("sink", 128, 128, 0), ("sigmoid", 96, 96, 500), ("pair", 64, 128, 1024),
+                                              ("plain", 64, 64, 0)])
+def test_window(kind, D, Dv, window, lens, parts, monkeypatch):
+    monkeypatch.setenv("EIA_WINDOW_DECODE_P", str(parts))
+    g = torch.Generator().manual_seed(len(lens) + D)
+    H, G, P = 4, 2, 2 if kind == "pair" else 1
+    md, pages = _step(lens, g)
+    rnd = lambda *s: torch.randn(*s, generator=g)
+    bf = lambda *s: rnd(*s).to(torch.bfloat16)
+    q, k, v = bf(len(lens), H * P * D), bf(pages, PAGE, G * P * D), bf(pages, G * Dv, PAGE)
+    sink, bias = rnd(H), torch.full((H,), -4.0)
+
+    def call(dev, t, m):
+        spec = WA.WindowSpec(H, G, P, D, Dv, window, 0, torch.full((H * P,), D ** -0.5, device=dev))
+        if kind == "sink":
+            spec.sink = t[3]
+        elif kind == "sigmoid":
+            spec.weights, spec.bias = 1, t[4]
+        elif kind == "pair":
+            spec.keep, spec.epilogue, spec.eps, spec.post, spec.lam = 4, 1, 1e-5, 0.7, torch.tensor([0.4], device=dev)
+        return WA.window_attention(t[0], t[1], t[2], m, spec)
+
+    want, got = _both(call, [q, k, v, sink, bias], md, lens)
+    # one rounding to bf16 on either side, 2^-9 / sqrt(3) each, and the products' order
+    assert _rel(got, want) < 4e-3
+
+
+def test_partitions():
+    """No more workgroups of an XCD's rows than its 32 CUs hold, none for what one workgroup does as fast."""
+    spec = lambda w, G=2: WA.WindowSpec(8, G, 1, 128, 128, w, 0, torch.ones(8))
+    assert [WA.decode_partitions(n, spec(1024)) for n in (1, 8, 9, 16, 17, 31, 64, 128)] == [8, 8, 8, 8, 5, 4, 2, 1]
+    assert [WA.decode_partitions(n, spec(0)) for n in (1, 8, 9, 17, 128)] == [16, 16, 8, 5, 1]
+    assert [WA.decode_partitions(3, spec(w)) for w in (300, 448, 449, 512)] == [1, 1, 4, 4]
+    for n in range(1, 300, 7):
+        rows = -(-n // 8)
+        for G in (1, 2, 4, 8):
+            assert WA.decode_partitions(n, spec(0, G)) == 1 or rows * G * WA.decode_partitions(n, spec(0, G)) <= 32

@@ -348,7 +348,7 @@ EIA_API int eia_latent_attn(const void* qa, long qa_st, long qa_sh, const void* 
 //
 // Bound by latency: a row's 64-key tiles are a chain of cache loads and two barriers, and the launch
 // lasts as long as the longest partition.  MI355X, 48 rows at up to 4096 tokens, window 1024, 16
-// heads, R 512 + 64: 23.8 + 4.8 us in five partitions; 200 rows at up to 2500 tokens, no window, with
+// heads, R 512 + 64: 23.2 + 4.1 us in five partitions; 200 rows at up to 2500 tokens, no window, with
 // 16 heads 153 -> 134 us and with 64 heads 499 -> 437 us since a tile's page is known before its fetch and
 // its LDS reads are asked for before the first product; R 128 + 32 with 64 heads 120 -> 115 us, R 256 + 64
 // 292 -> 292 us.  (Two tiles of cache loads in flight, in registers: 27 us instead of 24; the reads held in
@@ -369,7 +369,7 @@ latent_decode_kernel(LatentAttnArgs a) {
   __shared__ float2 rot[16 * NK];                       // [rot_dims / 2], rot_dims <= 32 NK
   const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int l16 = lane & 15, g4 = lane >> 4;
-  if (a.seq_lens && a.seq_lens[row] <= 0) return;
+  if (row >= a.n_work || (a.seq_lens && a.seq_lens[row] <= 0)) return;
   const int qpos = a.positions[row], kmax = qpos + 1;
   const int wlo = a.window > 0 ? max(0, kmax - a.window) : 0, kmin = wlo & ~(KT - 1);
   const int np = lat_parts(a.nparts, kmin, kmax);
@@ -571,45 +571,56 @@ latent_decode_kernel(LatentAttnArgs a) {
 
 // Merge of the decode partitions: out = sum_p acc_p 2^(m_p - M) / sum_p l_p 2^(m_p - M), times
 // the head gate.  One workgroup per (row, head); lane p first turns partition p's (max, sum) into
-// its weight, then the threads sum four latent columns each over the partitions with independent
-// loads (nparts <= 64).  Rows whose context is too short for two partitions were finished by the
-// attention kernel itself.
+// its weight, then the threads sum four latent columns each over the partitions (nparts <= 64).
+// Rows whose context is too short for two partitions were finished by the
+// attention kernel itself.  Bound by latency: the partials of up to eight partitions are asked for together with the
+// weights' inputs (48 rows of 16 heads, R 512, five partitions: 4.8 -> 4.1 us).
+constexpr int LM_P = 8;
 __global__ void __launch_bounds__(128)
 latent_merge_kernel(const float* __restrict__ part_acc, const float* __restrict__ part_ml,
                     int nparts, const int* __restrict__ seq_lens, const int* __restrict__ positions,
                     int window, const bf16_t* __restrict__ gate, long gate_st,
                     const float* __restrict__ sink, bf16_t* __restrict__ out, long out_st,
-                    long out_sh, int H, int R) {
+                    long out_sh, int n_items, int H, int R) {
   const int row = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63;
-  if (seq_lens && seq_lens[row] <= 0) return;
-  const int kmax = positions[row] + 1;
+  if (row >= n_items) return;
+  const int kmax = positions[row] + 1, len = (seq_lens ? seq_lens : positions)[row];
+  if (seq_lens && len <= 0) return;
   const int kmin = window > 0 ? max(0, kmax - window) & ~(LAT_UNIT - 1) : 0;
   const int np = lat_parts(nparts, kmin, kmax);
   if (np == 1) return;
   const long pr = ((long)row * H + h) * nparts;
   const float mp = lane < np ? part_ml[2 * (pr + lane)] : -INFINITY;
   const float lp = lane < np ? part_ml[2 * (pr + lane) + 1] : 0.f;
+  const float gv = gate ? bf2f(gate[row * gate_st + h]) : 0.f, sk = sink ? sink[h] : 0.f;
+  // (R % 8 == 0, R <= 512: one unit of four columns per thread; past R: the last one, unused)
+  const int c = min(4 * (int)threadIdx.x, R - 4);
+  f32x4 x[LM_P];
+#pragma unroll
+  for (int p = 0; p < LM_P; ++p)                        // (past the last one: the last one, unused)
+    x[p] = *reinterpret_cast<const f32x4*>(part_acc + (pr + min(p, np - 1)) * R + c);
   const float M = wave_max(mp);
   const float wp = (mp == -INFINITY) ? 0.f : exp2f(mp - M);
   float L = wave_sum(lp * wp);
-  if (sink && M != -INFINITY) L += exp2f(sink[h] * 1.4426950408889634f - M);
+  if (sink && M != -INFINITY) L += exp2f(sk * 1.4426950408889634f - M);
   float f = L > 0.f ? 1.0f / L : 0.f;
-  if (gate) f *= 1.0f / (1.0f + expf(-bf2f(gate[row * gate_st + h])));
-  for (int c0 = 0; c0 < R; c0 += 4 * blockDim.x) {      // (R % 8 == 0; every lane takes part)
-    const int c = c0 + 4 * threadIdx.x;
-    f32x4 v = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-    for (int p = 0; p < np; ++p) {
-      const float w = __shfl(wp, p, 64);
-      if (c < R) v += *reinterpret_cast<const f32x4*>(part_acc + (pr + p) * R + c) * w;
-    }
-    if (c < R) {
-      bf16x4 o;
+  if (gate) f *= 1.0f / (1.0f + expf(-gv));
+  f32x4 v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int e = 0; e < 4; ++e) o[e] = f2bf(v[e] * f);
-      *reinterpret_cast<bf16x4*>(out + row * out_st + h * out_sh + c) = o;
-    }
+  for (int p = 0; p < LM_P; ++p) {
+    const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wp), p));
+    if (p < np) v += x[p] * w;
   }
+#pragma unroll 4
+  for (int p = LM_P; p < np; ++p) {
+    const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wp), p));
+    v += *reinterpret_cast<const f32x4*>(part_acc + (pr + p) * R + c) * w;
+  }
+  if (4 * (int)threadIdx.x >= R) return;
+  bf16x4 o;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) o[e] = f2bf(v[e] * f);
+  *reinterpret_cast<bf16x4*>(out + row * out_st + h * out_sh + c) = o;
 }
 
 // Decode rows (one query each); prompt portions: latent_flash.hip.
@@ -634,7 +645,9 @@ EIA_API int eia_latent_attn_mfma(const void* qa, long qa_st, long qa_sh, const v
                    block_table, bt_stride, seq_lens, nullptr, nullptr, n_items, positions, gate,
                    gate_st, out, out_st, out_sh, scale, H, R, rd, bs, 1, HB, 0, 0, window, sink,
                    rot_half, rot_amp, nparts, part_acc, part_ml};
-  const dim3 grid(n_items, (H + HB - 1) / HB, nparts);
+  // (a row's workgroups, and its merge's, on one XCD: the partials meet in that L2)
+  const int rows = nparts > 1 ? (n_items + 7) / 8 * 8 : n_items;
+  const dim3 grid(rows, (H + HB - 1) / HB, nparts);
 #define LAT_DECODE(NK, NCW) hipLaunchKernelGGL((latent_decode_kernel<NK, NCW>), grid, dim3(256), 0, st, a)
   if (Dk <= 160 && R <= 128) LAT_DECODE(5, 2);
   else if (Dk <= 288 && R <= 256) LAT_DECODE(9, 4);
@@ -643,8 +656,8 @@ EIA_API int eia_latent_attn_mfma(const void* qa, long qa_st, long qa_sh, const v
   else LAT_DECODE(20, 8);
 #undef LAT_DECODE
   if (nparts > 1)
-    hipLaunchKernelGGL(latent_merge_kernel, dim3(n_items, H), dim3(128), 0, st, part_acc, part_ml,
+    hipLaunchKernelGGL(latent_merge_kernel, dim3(rows, H), dim3(128), 0, st, part_acc, part_ml,
                        nparts, seq_lens, positions, window, static_cast<const bf16_t*>(gate),
-                       gate_st, sink, static_cast<bf16_t*>(out), out_st, out_sh, H, R);
+                       gate_st, sink, static_cast<bf16_t*>(out), out_st, out_sh, n_items, H, R);
   EIA_LAUNCH_CHECK();
 }

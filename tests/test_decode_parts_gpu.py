@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from enterprise_inference_amd.ops import attention as A
+from enterprise_inference_amd.ops import latent_attention as LA
 from enterprise_inference_amd.ops import window_attention as WA
 
 PAGE = 64
@@ -72,13 +73,38 @@ def test_window(kind, D, Dv, window, lens, parts, monkeypatch):
     assert _rel(got, want) < 4e-3
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("parts", [0, 5, 23])
+@pytest.mark.parametrize("lens", [[1, 63, 64, 65, 128, 129, 0, 700, 2100], [900], [1500, 33, 1024]],
+                         ids=["edges", "one", "few"])
+@pytest.mark.parametrize("H,R,rd,window", [(8, 128, 32, 0), (20, 256, 32, 500), (16, 512, 64, 1024)])
+def test_latent(H, R, rd, window, lens, parts, monkeypatch):
+    monkeypatch.setenv("EIA_LATENT_DECODE_P", str(parts))
+    g = torch.Generator().manual_seed(len(lens) + R)
+    md, pages = _step(lens, g)
+    bf = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16)
+    t = [bf(len(lens), H, R), bf(len(lens), H, rd), bf(pages, PAGE, R + rd), bf(len(lens), H),
+         torch.randn(H, generator=g) if window else None]
+
+    def call(dev, t, m):
+        return LA.latent_attention(t[0], t[1], LA.inv_frequencies(rd, 10000.0, dev), rd, t[2], m, t[3], (R + rd) ** -0.5,
+                                   window, t[4])
+
+    want, got = _both(call, t, md, lens)
+    # as above, and the rotated queries' rounding to bf16 (2^-9 of a score of about one)
+    assert _rel(got, want) < 8e-3
+
+
 def test_partitions():
     """No more workgroups of an XCD's rows than its 32 CUs hold, none for what one workgroup does as fast."""
     spec = lambda w, G=2: WA.WindowSpec(8, G, 1, 128, 128, w, 0, torch.ones(8))
     assert [WA.decode_partitions(n, spec(1024)) for n in (1, 8, 9, 16, 17, 31, 64, 128)] == [8, 8, 8, 8, 5, 4, 2, 1]
     assert [WA.decode_partitions(n, spec(0)) for n in (1, 8, 9, 17, 128)] == [16, 16, 8, 5, 1]
     assert [WA.decode_partitions(3, spec(w)) for w in (300, 448, 449, 512)] == [1, 1, 4, 4]
+    assert [LA.decode_partitions(n, 16, window=1024) for n in (1, 8, 13, 24, 48, 100, 400)] == [17, 17, 16, 10, 5, 2, 1]
+    assert [LA.decode_partitions(n, 8, wide=False) for n in (1, 13, 48, 100)] == [32, 32, 10, 4]
     for n in range(1, 300, 7):
         rows = -(-n // 8)
         for G in (1, 2, 4, 8):
             assert WA.decode_partitions(n, spec(0, G)) == 1 or rows * G * WA.decode_partitions(n, spec(0, G)) <= 32
+        assert LA.decode_partitions(n, 64) == 1 or rows * 4 * LA.decode_partitions(n, 64) <= 32

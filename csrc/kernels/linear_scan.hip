@@ -1929,8 +1929,8 @@ gl_state_kernel(ScanArgs a, KChunkArgs c) {
   __shared__ __align__(16) float sk[GC * GD], sv[GC * W];
   __shared__ float stot[4][GD];
   int s, row0, n;
-  if (!gl_chunk(a, c.nseq, blockIdx.x, s, row0, n)) return;
-  const int h = blockIdx.y, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  if (!gl_chunk(a, c.nseq, chunk_number(), s, row0, n)) return;
+  const int h = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int l16 = lane & 15, g4 = lane >> 4;
   GlTile<T, VEC, ROT> tk;
   GlValues<T, VEC, NV> tv;
@@ -1952,7 +1952,7 @@ gl_state_kernel(ScanArgs a, KChunkArgs c) {
     sk[tile_at<GD>(16 * w + t, lane)] *= __builtin_amdgcn_exp2f(after);
     after += l[t];
   }
-  const long at = (long)blockIdx.x * a.H + h;
+  const long at = (long)chunk_number() * a.H + h;
   if (w == 0) c.G[at * GD + lane] = after;
   __syncthreads();
   f32x4 acc[4 * NV];
@@ -1990,10 +1990,11 @@ template <int NV>
 __global__ void __launch_bounds__(256)
 gl_scan_kernel(ScanArgs a, KChunkArgs c) {
   constexpr int W = 64 * NV;
-  const int s = blockIdx.x, h = blockIdx.y;
+  const int s = chunk_number(), h = blockIdx.x % a.H;
+  if (s >= c.nseq) return;
   const int slot = a.slots[s], lo = a.cu[s], hi = a.cu[s + 1];
   if (slot < 0 || hi <= lo) return;
-  const int e = 4 * (blockIdx.z * 256 + threadIdx.x), i = e / W, j = e % W, D = a.D, Dv = a.Dv;
+  const int e = 4 * (blockIdx.x / a.H * 256 + threadIdx.x), i = e / W, j = e % W, D = a.D, Dv = a.Dv;
   const long x0 = lo / GC + s;
   const int nc = (hi - lo + GC - 1) / GC;
   float* Sg = a.S + ((long)slot * a.H + h) * D * Dv + (long)i * Dv + j;
@@ -2022,8 +2023,8 @@ gl_out_kernel(ScanArgs a, KChunkArgs c) {
   __shared__ __align__(16) float sq[GC * GD], sk[GC * GD], sAv[GC * W];
   __shared__ __align__(16) float se[8][GD];            // decays over whole 8-token blocks
   int s, row0, n;
-  if (!gl_chunk(a, c.nseq, blockIdx.x, s, row0, n)) return;
-  const int h = blockIdx.y, lane = threadIdx.x & 63, w = ((threadIdx.x >> 6) + blockIdx.x) & 3;
+  if (!gl_chunk(a, c.nseq, chunk_number(), s, row0, n)) return;
+  const int h = blockIdx.x, lane = threadIdx.x & 63, w = ((threadIdx.x >> 6) + blockIdx.y) & 3;
   const int Dv = a.Dv, l16 = lane & 15, g4 = lane >> 4, t0 = 16 * w;
   GlTile<T, VEC, ROT> tq, tk;
   GlValues<T, VEC, NV> tv;
@@ -2109,7 +2110,7 @@ gl_out_kernel(ScanArgs a, KChunkArgs c) {
     }
   }
   if (row0 != a.cu[s] || a.positions[a.cu[s]] != 0) {  // (a fresh sequence's first chunk: S = 0)
-    const float* S = c.U + ((long)blockIdx.x * a.H + h) * GD * W + (long)4 * g4 * W + 4 * l16;
+    const float* S = c.U + ((long)chunk_number() * a.H + h) * GD * W + (long)4 * g4 * W + 4 * l16;
 #pragma unroll
     for (int x = 0; x < 4; ++x)
 #pragma unroll
@@ -2161,7 +2162,7 @@ gl_out_kernel(ScanArgs a, KChunkArgs c) {
 
 template <typename T, bool VEC, bool ROT, int NV>
 static void gl_launch(const ScanArgs& a, const KChunkArgs& c, hipStream_t st) {
-  const dim3 gc(c.rows / GC + c.nseq, a.H), gs(c.nseq, a.H, GD * 64 * NV / 1024);
+  const dim3 gc = chunk_grid(c.rows / GC + c.nseq, a.H), gs = chunk_grid(c.nseq, a.H * (GD * 64 * NV / 1024));
   hipLaunchKernelGGL((gl_logs_kernel<T>), dim3((c.rows + 63) / 64, a.H), dim3(256), 0, st, a, c);
   if (ROT) {
     const long u = (long)c.rows * (a.rot_dims >> 1);

@@ -322,8 +322,8 @@ wkv_chunk_state_kernel(WkvArgs a, WkvChunkArgs c) {
   __shared__ __align__(16) float sk[WC * WD], sv[WC * WD];
   __shared__ float stot[4][WD];
   int s, row0, n;
-  if (!wkv_chunk(a, c.nseq, blockIdx.x, s, row0, n)) return;
-  const int h = blockIdx.y, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  if (!wkv_chunk(a, c.nseq, chunk_number(), s, row0, n)) return;
+  const int h = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int l16 = lane & 15, g4 = lane >> 4;
   const long hc = (long)h * a.D;
   WkvTile<T, VEC> tk, tv;
@@ -345,7 +345,7 @@ wkv_chunk_state_kernel(WkvArgs a, WkvChunkArgs c) {
     sk[tile_at<WD>(16 * w + t, lane)] *= __builtin_amdgcn_exp2f(after);
     after += l[t];
   }
-  const long at = (long)blockIdx.x * a.H + h;
+  const long at = (long)chunk_number() * a.H + h;
   if (w == 0) c.L[at * WD + lane] = after;
   __syncthreads();
   f32x4 acc[4];
@@ -375,10 +375,11 @@ wkv_chunk_state_kernel(WkvArgs a, WkvChunkArgs c) {
 // (2) Four columns of a state row per thread; the slot receives the state after the last chunk.
 __global__ void __launch_bounds__(256)
 wkv_chunk_scan_kernel(WkvArgs a, WkvChunkArgs c) {
-  const int s = blockIdx.x, h = blockIdx.y;
+  const int s = chunk_number(), h = blockIdx.x % a.H;
+  if (s >= c.nseq) return;
   const int slot = a.slots[s], lo = a.cu[s], hi = a.cu[s + 1];
   if (slot < 0 || hi - lo < a.split || (a.seq_lens && a.seq_lens[s] <= 0)) return;
-  const int e = 4 * (blockIdx.z * 256 + threadIdx.x), i = e / WD, j = e % WD, D = a.D;
+  const int e = 4 * (blockIdx.x / a.H * 256 + threadIdx.x), i = e / WD, j = e % WD, D = a.D;
   const long x0 = lo / WC + s;
   const int nc = (hi - lo + WC - 1) / WC;
   float* Sg = a.S + ((long)slot * a.H + h) * D * D + (long)i * D + j;
@@ -412,8 +413,8 @@ wkv_chunk_out_kernel(WkvArgs a, WkvChunkArgs c) {
   __shared__ __align__(16) float se[8][WD], su[WD];    // decays over whole 8-token blocks; u
   __shared__ int swild;                                // a value of the chunk is not finite
   int s, row0, n;
-  if (!wkv_chunk(a, c.nseq, blockIdx.x, s, row0, n)) return;
-  const int h = blockIdx.y, lane = threadIdx.x & 63, w = ((threadIdx.x >> 6) + blockIdx.x) & 3;
+  if (!wkv_chunk(a, c.nseq, chunk_number(), s, row0, n)) return;
+  const int h = blockIdx.x, lane = threadIdx.x & 63, w = ((threadIdx.x >> 6) + blockIdx.y) & 3;
   const int D = a.D, l16 = lane & 15, g4 = lane >> 4, t0 = 16 * w;
   const long hc = (long)h * D;
   WkvTile<T, VEC> tr, tk, tv;
@@ -518,7 +519,7 @@ wkv_chunk_out_kernel(WkvArgs a, WkvChunkArgs c) {
     }
   }
   if (row0 != a.cu[s] || a.positions[a.cu[s]] != 0) {  // (a fresh sequence's first chunk: S = 0)
-    const float* S = c.U + ((long)blockIdx.x * a.H + h) * WD * WD + (long)4 * g4 * WD + 4 * l16;
+    const float* S = c.U + ((long)chunk_number() * a.H + h) * WD * WD + (long)4 * g4 * WD + 4 * l16;
 #pragma unroll
     for (int x = 0; x < 4; ++x) {
       f32x4 sb[4];
@@ -565,7 +566,7 @@ wkv_chunk_out_kernel(WkvArgs a, WkvChunkArgs c) {
 
 template <typename T, bool VEC>
 static void wkv_chunked(const WkvArgs& a, const WkvChunkArgs& c, int rows, hipStream_t st) {
-  const dim3 gc(rows / WC + c.nseq, a.H), gs(c.nseq, a.H, WD * WD / 1024);
+  const dim3 gc = chunk_grid(rows / WC + c.nseq, a.H), gs = chunk_grid(c.nseq, a.H * (WD * WD / 1024));
   hipLaunchKernelGGL((wkv_chunk_state_kernel<T, VEC>), gc, dim3(256), 0, st, a, c);
   hipLaunchKernelGGL(wkv_chunk_scan_kernel, gs, dim3(256), 0, st, a, c);
   hipLaunchKernelGGL((wkv_chunk_out_kernel<T, VEC>), gc, dim3(256), 0, st, a, c);

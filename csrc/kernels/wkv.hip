@@ -251,6 +251,7 @@ struct WkvChunkArgs {
   float* U;                                 // [numbers, H, WD, WD]: contribution, then state before
   float* L;                                 // [numbers, H, WD]: sums of l
   int nseq;
+  int wide;                                 // gate, weight and output rows can be taken 4 at a time
 };
 
 // The chunk of number x; false where there is none or the sequence is skipped.
@@ -518,6 +519,27 @@ wkv_chunk_out_kernel(WkvArgs a, WkvChunkArgs c) {
       rt[x] *= e1 * *reinterpret_cast<const f32x4*>(&se[2 * b][i]);
     }
   }
+  // the gates and the norm's weight are on their way during the last products
+  typedef T T4 __attribute__((ext_vector_type(4)));
+  T4 gv[4], nw;
+  {
+    const T* G = static_cast<const T*>(a.g) + hc;
+    const T* NW = static_cast<const T*>(a.norm_w) + hc;
+    if (c.wide) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        gv[i] = *reinterpret_cast<const T4*>(G + (long)(row0 + min(t0 + 4 * g4 + i, n - 1)) * a.ld + 4 * l16);
+      nw = *reinterpret_cast<const T4*>(NW + 4 * l16);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int d = min(4 * l16 + j, D - 1);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) gv[i][j] = G[(long)(row0 + min(t0 + 4 * g4 + i, n - 1)) * a.ld + d];
+        nw[j] = NW[d];
+      }
+    }
+  }
   if (row0 != a.cu[s] || a.positions[a.cu[s]] != 0) {  // (a fresh sequence's first chunk: S = 0)
     const float* S = c.U + ((long)chunk_number() * a.H + h) * WD * WD + (long)4 * g4 * WD + 4 * l16;
 #pragma unroll
@@ -534,32 +556,30 @@ wkv_chunk_out_kernel(WkvArgs a, WkvChunkArgs c) {
     }
   }
   mfma_settle(o);
-  const T* G = static_cast<const T*>(a.g);
-  const T* NW = static_cast<const T*>(a.norm_w);
   T* Y = static_cast<T*>(a.y);
 #pragma unroll
   for (int i = 0; i < 4; ++i) {                        // head RMS norm (zeros past D), weight, gate
     float ss = 0.f;
 #pragma unroll
     for (int j = 0; j < 4; ++j) ss += o[j][i] * o[j][i];
-    ss += __shfl_xor(ss, 1, 64);
-    ss += __shfl_xor(ss, 2, 64);
-    ss += __shfl_xor(ss, 4, 64);
-    ss += __shfl_xor(ss, 8, 64);
+    ss = row16_sum(ss);
     const int tok = t0 + 4 * g4 + i;
     if (tok >= n) continue;
     const float inv = 1.0f / sqrtf(ss / (float)D + a.eps);
-    const long row = row0 + tok;
+    T* y = Y + (long)(row0 + tok) * a.ldy + hc + 4 * l16;
+    T4 yv;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int d = 4 * l16 + j;
-      if (d < D) {
-        const float g = ld_f32<T>(G, row * a.ld + hc + d);
-        st_f32<T>(Y, row * a.ldy + hc + d,
-                  o[j][i] * inv * ld_f32<T>(NW, hc + d) *
-                      (sizeof(T) == 2 ? g * __builtin_amdgcn_rcpf(1.0f + __expf(-g))
-                                      : g / (1.0f + expf(-g))));
-      }
+      const float g = (float)gv[i][j];
+      yv[j] = (T)(o[j][i] * inv * (float)nw[j] *
+                  (sizeof(T) == 2 ? g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)) : g / (1.0f + expf(-g))));
+    }
+    if (c.wide) {
+      *reinterpret_cast<T4*>(y) = yv;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (4 * l16 + j < D) y[j] = yv[j];
     }
   }
 }
@@ -587,7 +607,9 @@ EIA_API int eia_wkv_scan_chunked(const void* r, const void* k, const void* v, co
   if (nseq == 0 || rows == 0) return EIA_OK;
   WkvArgs a{r, k, v, g, ld, dec, ld_dec, w0, u, norm_w, S, prev, x, W, slots, cu, positions,
             seq_lens, y, ldy, eps, H, D, split};
-  WkvChunkArgs c{U, L, nseq};
+  const int es = is_bf16 ? 2 : 4;
+  const uintptr_t io = (uintptr_t)g | (uintptr_t)y | (uintptr_t)norm_w | (uintptr_t)(ld * es) | (uintptr_t)(ldy * es);
+  WkvChunkArgs c{U, L, nseq, D == WD && io % (4 * es) == 0};
   const uintptr_t any = (uintptr_t)r | (uintptr_t)k | (uintptr_t)v | (uintptr_t)(ld * (is_bf16 ? 2 : 4));
   const bool vec = D == WD && any % 16 == 0;
   if (is_bf16 && vec) wkv_chunked<bf16_t, true>(a, c, rows, st);

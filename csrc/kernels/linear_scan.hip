@@ -463,6 +463,7 @@ struct KChunkArgs {
   float* la; float* lb; float* nm;          // [rows, H] log a, log b, -m  (mode 1)
   float2* rot;                              // [rows, rot_dims / 2]: cos, sin
   int nseq, rows, DP, VP, UW;               // UW: VP, and in mode 1 four more (the normaliser, 0, 0, 0)
+  bool wide = false;                        // per channel: gate, weight and output rows can be taken 4 at a time
 };
 
 // The chunk of number x; false where there is none or the sequence is skipped.
@@ -2109,6 +2110,32 @@ gl_out_kernel(ScanArgs a, KChunkArgs c) {
       rt[x] *= e1 * *reinterpret_cast<const f32x4*>(&se[2 * b][i]);
     }
   }
+  // the gates and the norm's weight are on their way during the last products
+  typedef T T4 __attribute__((ext_vector_type(4)));
+  T4 gv[4][NV], nw[NV];
+  {
+    const T* G = static_cast<const T*>(a.x) + a.g_off + (long)h * Dv;
+    const T* NW = static_cast<const T*>(a.norm_w) + (a.norm_w ? (long)h * a.norm_h : 0);
+#pragma unroll
+    for (int z = 0; z < NV; ++z) {
+      const int d = 64 * z + 4 * l16;
+      if (c.wide) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          gv[i][z] = *reinterpret_cast<const T4*>(G + (row0 + min(t0 + 4 * g4 + i, n - 1)) * a.ld + min(d, Dv - 4));
+        if (a.norm_w) nw[z] = *reinterpret_cast<const T4*>(NW + min(d, Dv - 4));
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int dj = min(d + j, Dv - 1);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) gv[i][z][j] = G[(row0 + min(t0 + 4 * g4 + i, n - 1)) * a.ld + dj];
+          if (a.norm_w) nw[z][j] = NW[dj];
+        }
+      }
+      if (!a.norm_w) nw[z] = T4{(T)1.f, (T)1.f, (T)1.f, (T)1.f};
+    }
+  }
   if (row0 != a.cu[s] || a.positions[a.cu[s]] != 0) {  // (a fresh sequence's first chunk: S = 0)
     const float* S = c.U + ((long)chunk_number() * a.H + h) * GD * W + (long)4 * g4 * W + 4 * l16;
 #pragma unroll
@@ -2127,8 +2154,6 @@ gl_out_kernel(ScanArgs a, KChunkArgs c) {
       }
   }
   mfma_settle(o);
-  const T* X = static_cast<const T*>(a.x);
-  const T* NW = static_cast<const T*>(a.norm_w);
   T* Y = static_cast<T*>(a.y);
 #pragma unroll
   for (int i = 0; i < 4; ++i) {                        // head RMS norm (zeros past Dv), weight, gate
@@ -2136,27 +2161,28 @@ gl_out_kernel(ScanArgs a, KChunkArgs c) {
     float ss = 0.f;
 #pragma unroll
     for (int j = 0; j < 4 * NV; ++j) ss += o[j][i] * o[j][i];
-    ss += __shfl_xor(ss, 1, 64);
-    ss += __shfl_xor(ss, 2, 64);
-    ss += __shfl_xor(ss, 4, 64);
-    ss += __shfl_xor(ss, 8, 64);
+    ss = row16_sum(ss);
     if (t >= n) continue;
     const float inv = a.out_scale / sqrtf(ss / (float)Dv + a.eps);
-    const long row = row0 + t;
 #pragma unroll
-    for (int z = 0; z < NV; ++z)
+    for (int z = 0; z < NV; ++z) {
+      const int d = 64 * z + 4 * l16;
+      T* y = Y + (long)(row0 + t) * a.ldy + (long)h * Dv + d;
+      T4 yv;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const int d = 64 * z + 4 * l16 + j;
-        if (d < Dv) {
-          const float g = ld_f32<T>(X + row * a.ld, a.g_off + (long)h * Dv + d);
-          const float sig = sizeof(T) == 2 ? __builtin_amdgcn_rcpf(1.0f + __expf(-g))
-                                           : 1.0f / (1.0f + expf(-g));
-          const float nw = NW ? ld_f32<T>(NW, (long)h * a.norm_h + d) : 1.f;
-          st_f32<T>(Y + row * a.ldy, (long)h * Dv + d,
-                    o[4 * z + j][i] * inv * nw * (a.gate_act == 0 ? g * sig : sig));
-        }
+        const float g = (float)gv[i][z][j];
+        const float sig = sizeof(T) == 2 ? __builtin_amdgcn_rcpf(1.0f + __expf(-g)) : 1.0f / (1.0f + expf(-g));
+        yv[j] = (T)(o[4 * z + j][i] * inv * (float)nw[z][j] * (a.gate_act == 0 ? g * sig : sig));
       }
+      if (c.wide) {
+        if (d < Dv) *reinterpret_cast<T4*>(y) = yv;
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (d + j < Dv) y[j] = yv[j];
+      }
+    }
   }
 }
 
@@ -2174,8 +2200,10 @@ static void gl_launch(const ScanArgs& a, const KChunkArgs& c, hipStream_t st) {
 }
 
 template <typename T>
-static void gl_forms(const ScanArgs& a, const KChunkArgs& c, hipStream_t st) {
+static void gl_forms(const ScanArgs& a, KChunkArgs c, hipStream_t st) {
   constexpr int A = 16 / (int)sizeof(T);               // elements in 16 bytes
+  const uintptr_t io = reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.y) | reinterpret_cast<uintptr_t>(a.norm_w);
+  c.wide = io % (4 * sizeof(T)) == 0 && (a.ld | a.ldy | a.g_off | a.Dv | a.norm_h) % 4 == 0;
   const int rot8 = a.rot_dims ? (a.rot_half ? a.rot_dims / 2 : a.rot_dims) : 0;
   const bool vec = reinterpret_cast<uintptr_t>(a.x) % 16 == 0 &&
                    (a.ld | a.q_off | a.k_off | a.v_off) % A == 0 && a.D % 8 == 0 && a.Dv % 8 == 0 &&

@@ -556,3 +556,61 @@ def test_linear_chunks_past_a_grid_column(monkeypatch):
     assert _rel(S[:n - 1, 0], k[:, :, None] * v[:, None, :]) < 2e-6
     alone, Sa = run(x[n - 1:], torch.tensor([0, 130], dtype=torch.int32).cuda(), 1, pos[n - 1:], [130])
     assert torch.equal(y[n - 1:], alone) and torch.equal(S[n - 1:], Sa)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("mode,H,D,Dv", [("channel", 2, 64, 128), ("channel", 3, 32, 64), ("exp_gates", 2, 128, 128),
+                                         ("decay", 2, 64, 64)])
+def test_outputs_into_a_view(mode, H, D, Dv, dtype, monkeypatch):
+    """Rows of an output that vector accesses cannot take hold the same numbers as rows that they can."""
+    from enterprise_inference_amd.ops import linear_scan as ls
+    monkeypatch.setattr(ls, "FORCE_CHUNKED", True)
+    g = torch.Generator(device="cuda").manual_seed(D)
+    lens = [130, 64, 1]
+    T, n, W = sum(lens), len(lens), H * Dv
+    at = [0, H * D, 2 * H * D, 2 * H * D + W, 2 * H * D + 2 * W, 2 * H * D + 2 * W + H]
+    x = torch.randn(T, at[-1] + H + 8, generator=g, device="cuda").to(dtype)
+    nw = (1 + 0.1 * torch.randn(W, generator=g, device="cuda")).to(dtype)
+    spec = ls.ScanSpec(H, D, Dv, mode, kscale=D ** -0.5, eps=1e-5, decay=torch.linspace(0.9, 0.5, H).cuda(),
+                       a2t=torch.randn(8, H * D, generator=g, device="cuda"), tau=8.0)
+    cu, pos, slots = (t.cuda() for t in _step(lens, [0, 5, 0], False))
+
+    def run(out, w):
+        st = ls.ScanState.allocate(n, spec, "cuda")
+        st.S.fill_(0.3)
+        y = ls.linear_scan(x, at[0], at[1], at[2], at[3], spec, st, slots, cu, n, pos, None, w, at[4], at[5], out=out,
+                           plan=ls.chunk_plan(lens, "cuda"), lo_off=at[-1] + H)
+        return y.clone(), st.S
+
+    y, S = run(None, nw)
+    for left, width in ((3, W + 5), (4, W + 8)):
+        z, R = run(torch.full((T, width), 7.0, device="cuda", dtype=dtype)[:, left:left + W], nw)
+        assert torch.equal(z, y) and torch.equal(R, S)
+    odd = torch.empty(W + 1, device="cuda", dtype=dtype)[1:].copy_(nw)
+    assert torch.equal(run(None, odd)[0], y)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_wkv_rows_of_any_alignment(dtype):
+    """Rows, weights and gates that vector accesses cannot take give what rows give that they can."""
+    from enterprise_inference_amd.ops import wkv
+    g = torch.Generator(device="cuda").manual_seed(3)
+    lens, H, D = [130, 64, 300], 2, 64
+    T, HD = sum(lens), H * D
+    cu, pos, slots = (t.cuda() for t in _step(lens, [0, 5, 0], False))
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    rows, dec, w0, u, nw = rnd(4, T, HD).to(dtype), rnd(T, HD), rnd(HD).to(dtype), rnd(HD).to(dtype), rnd(HD).to(dtype)
+    x = rnd(T, 24)
+    out = []
+    for odd in (False, True):
+        r, k, v, gate = rows
+        w = nw
+        if odd:
+            r, k, v, gate = (torch.empty(T, HD + 3, device="cuda", dtype=dtype)[:, 1:1 + HD].copy_(t) for t in rows)
+            w = torch.empty(HD + 1, device="cuda", dtype=dtype)[1:].copy_(nw)
+        S = torch.full((3, H, D, D), 0.2, device="cuda")
+        y = wkv.wkv_scan(r, k, v, gate, dec, w0, u, w, S, torch.zeros(3, 24, device="cuda"), x, slots, cu, 3, pos, None,
+                         1e-5, H)
+        out.append((y, S))
+    # the same fp32 sums, whichever way their factors came
+    assert _rel(out[1][0], out[0][0]) < (1e-6 if dtype == torch.float32 else 1e-3) and _rel(out[1][1], out[0][1]) < 1e-6

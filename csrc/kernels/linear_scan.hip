@@ -449,11 +449,12 @@ EIA_API int eia_linear_scan(const void* x, long ld, int q_off, int k_off, int v_
 // traffic (4 passes over chunks x H x dk x dv floats), and halving their number costs less than the
 // longer sums inside a chunk add.
 // Four prompts of 1000 .. 2000 tokens (6688 rows), 16 heads of 128, mode 1, bf16 take 11 + 31 + 21 +
-// 60 us on an MI355X (gates, (1), (2), (3)); in fp32 products (1) and (3) took 57 + 103 us.  Bound by the
+// 58 us on an MI355X (gates, (1), (2), (3)); in fp32 products (1) and (3) took 57 + 103 us.  Bound by the
 // workspace and the rows, which (1), (2) and (3) move at 3.8, 5.4 and 3.3 TB/s, and by the steps of
 // a workgroup, which reads, splits and multiplies in turn.  All heads of a chunk run side by side in (1) and (3), so
 // that whole rows are read together, and (3) asks for its queries before it waits for the gates: 123 -> 118 us for the
-// op; three rotated prompts of up to 2700 tokens 188 -> 178, five of up to 1100 of 32 heads of 64 78 -> 77.
+// op; three rotated prompts of up to 2700 tokens 188 -> 178, five of up to 1100 of 32 heads of 64 78 -> 77.  What the
+// normaliser, the norm and the gate read is asked for at once (four rounds behind each other: 118 -> 116 us).
 constexpr int LK = 128;                     // tokens per chunk
 constexpr float LS_LOG2E = 1.4426950408889634f;
 
@@ -1347,10 +1348,11 @@ EIA_DEV bool ls_out_bf16(const ScanArgs& a, const KChunkArgs& c, const LsChunk& 
   return !__syncthreads_or(bad);
 }
 
-// Two workgroups on a CU where the LDS holds two: 128 registers a lane, of which aligned, unrotated heads of 128 spill 14.
-// One with all registers: four gated prompts of up to 2000 tokens, 16 heads, the op 123 -> 150 us.
+// Two workgroups on a CU where the LDS holds two: 128 registers a lane, of which aligned, unrotated heads of 128 spill 11.
+// One with all registers: four gated prompts of up to 2000 tokens, 16 heads, the op 123 -> 150 us.  Heads of 64, unrotated:
+// three, 80 registers (82, and two, without the bound: five prompts of up to 1100 tokens, 32 heads, 76 -> 82 us).
 template <typename T, bool VEC, bool ROT, int MX>
-__global__ void __launch_bounds__(512, 4)
+__global__ void __launch_bounds__(512, sizeof(T) == 2 && VEC && !ROT && MX == 64 ? 6 : 4)
 ls_chunk_out_kernel(ScanArgs a, KChunkArgs c) {
   constexpr bool BF = sizeof(T) == 2;
   constexpr int KV = LK * MX * ((BF && !ROT ? 2 : 4) + (int)sizeof(T)), FP32 = KV > MX * MX * 4 ? KV : MX * MX * 4;
@@ -1384,13 +1386,36 @@ ls_chunk_out_kernel(ScanArgs a, KChunkArgs c) {
   const T* X = static_cast<const T*>(a.x);
   const T* NW = static_cast<const T*>(a.norm_w);
   T* Y = static_cast<T*>(a.y);
+  typedef T T4 __attribute__((ext_vector_type(4)));
+  // what a lane's four tokens need besides, asked for together
+  float nm[4];
+  T4 gt[4][MX / 64], nw[MX / 64];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const long row = row0 + min(t0 + 4 * g4 + i, n - 1);
+    nm[i] = a.mode == 1 ? c.nm[row * a.H + h] : 0.f;
+#pragma unroll
+    for (int x = 0; x < MX / 64; ++x) {
+      const int d = 64 * x + 4 * l16;
+      const T* gp = X + row * a.ld + a.g_off + (long)h * Dv;
+      if constexpr (VEC) gt[i][x] = *reinterpret_cast<const T4*>(gp + (d < Dv ? d : 0));
+      else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) gt[i][x][j] = gp[min(d + j, Dv - 1)];
+      }
+    }
+  }
+#pragma unroll
+  for (int x = 0; x < MX / 64; ++x)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      nw[x][j] = NW ? NW[(long)h * a.norm_h + min(64 * x + 4 * l16 + j, Dv - 1)] : (T)1.f;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {                        // normaliser, head RMS norm, weight, gate
     const int t = t0 + 4 * g4 + i;
     const float nqi = __shfl(rs, 4 * g4 + i, 64);
-    const long row = row0 + min(t, n - 1);
     float den = 1.f;
-    if (a.mode == 1) den = 1.0f / (fmaxf(fabsf(nqi), expf(c.nm[row * a.H + h])) + 1e-6f);
+    if (a.mode == 1) den = 1.0f / (fmaxf(fabsf(nqi), expf(nm[i])) + 1e-6f);
     float ss = 0.f;
 #pragma unroll
     for (int j = 0; j < MX / 16; ++j) {
@@ -1398,34 +1423,22 @@ ls_chunk_out_kernel(ScanArgs a, KChunkArgs c) {
       o[j][i] = col ? o[j][i] * den : 0.f;             // (padded columns read column 0 of S)
       ss += o[j][i] * o[j][i];
     }
-    ss += __shfl_xor(ss, 1, 64);
-    ss += __shfl_xor(ss, 2, 64);
-    ss += __shfl_xor(ss, 4, 64);
-    ss += __shfl_xor(ss, 8, 64);
+    ss = row16_sum(ss);
     if (t >= n) continue;
     const float inv = a.out_scale / sqrtf(ss / (float)Dv + a.eps);
 #pragma unroll
     for (int x = 0; x < MX / 64; ++x) {
       const int d = 64 * x + 4 * l16;
       if (d >= Dv) continue;
-      const T* gp = X + row * a.ld + a.g_off + (long)h * Dv + d;
-      T* yp = Y + row * a.ldy + (long)h * Dv + d;
-      alignas(16) T g4v[4], y4[4];
-      if constexpr (VEC && sizeof(T) == 2) *reinterpret_cast<float2*>(g4v) = *reinterpret_cast<const float2*>(gp);
-      else if constexpr (VEC) *reinterpret_cast<f32x4*>(g4v) = *reinterpret_cast<const f32x4*>(gp);
-      else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) g4v[j] = gp[d + j < Dv ? j : 0];
-      }
+      T* yp = Y + (row0 + t) * a.ldy + (long)h * Dv + d;
+      T4 y4;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const float g = (float)g4v[j];
+        const float g = (float)gt[i][x][j];
         const float sig = sizeof(T) == 2 ? __builtin_amdgcn_rcpf(1.0f + __expf(-g)) : 1.0f / (1.0f + expf(-g));
-        const float nw = (NW && d + j < Dv) ? ld_f32<T>(NW, (long)h * a.norm_h + d + j) : 1.f;
-        y4[j] = (T)(o[4 * x + j][i] * inv * nw * (a.gate_act == 0 ? g * sig : sig));
+        y4[j] = (T)(o[4 * x + j][i] * inv * (float)nw[x][j] * (a.gate_act == 0 ? g * sig : sig));
       }
-      if constexpr (VEC && sizeof(T) == 2) *reinterpret_cast<float2*>(yp) = *reinterpret_cast<const float2*>(y4);
-      else if constexpr (VEC) *reinterpret_cast<f32x4*>(yp) = *reinterpret_cast<const f32x4*>(y4);
+      if constexpr (VEC) *reinterpret_cast<T4*>(yp) = y4;
       else {
 #pragma unroll
         for (int j = 0; j < 4; ++j)

@@ -964,12 +964,15 @@ delta_chunk_scan_kernel(DeltaArgs a, DeltaChunkArgs c) {
   if (wave < 4) scan_state<NDG, NC>(a, k, S, true, 1.f / DN_UP);
 }
 
-// (3) Norm, weight and gate of the outputs: LN lanes per token and head, four heads each.  Bound by memory.
+// (3) Norm, weight and gate of the outputs: LN lanes per token and head, two heads each; the heads come first in the
+// grid, so that those of a key head run on the XCD that formed them where G is eight.  Bound by memory.  (Four heads, chunks
+// first: three prompts of 155 tokens, 8 heads 32.9 -> 30.8 us, three of up to 1500, 16 heads 146.0 -> 145.2.)
+constexpr int DN_HEADS = 2;
 template <typename T, int LN>
 __global__ void __launch_bounds__(256)
 delta_chunk_norm_kernel(DeltaArgs a, DeltaChunkArgs c) {
-  constexpr int NH = 4;
-  const int ch = blockIdx.x, sub = threadIdx.x % LN, t = blockIdx.y * (256 / LN) + threadIdx.x / LN;
+  constexpr int NH = DN_HEADS;
+  const int ch = blockIdx.y, sub = threadIdx.x % LN, t = blockIdx.z * (256 / LN) + threadIdx.x / LN;
   const int s = c.chunks[4 * ch], row0 = c.chunks[4 * ch + 1], n = c.chunks[4 * ch + 2];
   if (a.slots[s] < 0 || t >= n) return;
   const int col = 4 * sub, Dv = a.Dv, VQ = 32 * c.ncu;
@@ -979,7 +982,7 @@ delta_chunk_norm_kernel(DeltaArgs a, DeltaChunkArgs c) {
   const T* GT = static_cast<const T*>(a.g) + r * a.ldg;
 #pragma unroll
   for (int x = 0; x < NH; ++x) {
-    const int h = min((int)blockIdx.z * NH + x, a.H - 1);
+    const int h = min((int)blockIdx.x * NH + x, a.H - 1);
     o[x] = *reinterpret_cast<const f32x4*>(c.O + (((long)ch * DC + t) * a.H + h) * VQ + min(col, VQ - 4));
     if (c.vec) {
       typedef T T4 __attribute__((ext_vector_type(4)));
@@ -999,7 +1002,7 @@ delta_chunk_norm_kernel(DeltaArgs a, DeltaChunkArgs c) {
     nw[j] = ld_f32<T>(static_cast<const T*>(a.norm_w), min(col + j, Dv - 1)) * a.out_scale;
 #pragma unroll
   for (int x = 0; x < NH; ++x) {
-    const int h = (int)blockIdx.z * NH + x;
+    const int h = (int)blockIdx.x * NH + x;
     float sq = 0.f;
 #pragma unroll
     for (int j = 0; j < 4; ++j) sq += col + j < Dv ? o[x][j] * o[x][j] : 0.f;
@@ -1064,7 +1067,7 @@ EIA_API int eia_delta_scan_chunked(const float* q, const float* k, const float* 
     if (nc == 2) DO_SCAN(A, 2); else DO_SCAN(A, 1);                                                \
   } while (0)
 #define DO_NORM(TT, LN)                                                                            \
-  hipLaunchKernelGGL((delta_chunk_norm_kernel<TT, LN>), dim3(nchunk, DC * LN / 256, (H + 3) / 4), b, 0, st, a, c)
+  hipLaunchKernelGGL((delta_chunk_norm_kernel<TT, LN>), dim3((H + DN_HEADS - 1) / DN_HEADS, nchunk, DC * LN / 256), b, 0, st, a, c)
   if (ndg == 2) DO_DIMS(2); else DO_DIMS(1);
   if (is_bf16) { if (VP > 64) DO_NORM(bf16_t, 32); else DO_NORM(bf16_t, 16); }
   else { if (VP > 64) DO_NORM(float, 32); else DO_NORM(float, 16); }

@@ -141,3 +141,61 @@ def test_moved_weights_are_not_copied(act, T):
         x, w13, w2, w, ids).double()
     # hidden rows, expert outputs and sums are rounded to bf16 on both sides: 3 x 1.7e-3 each
     assert (out.double().cpu() - r).norm() / r.norm() < 1.1e-2
+
+
+@pytest.mark.parametrize("n,E,lo,hi,k", [(1, 1, 0, 1, 1), (1023, 8, 0, 8, 3), (1025, 5, 2, 3, 2),
+                                         (4096, 256, 0, 256, 2), (4097, 255, 3, 250, 1),
+                                         (8192, 16, 0, 16, 4), (8195, 256, 250, 256, 5)])
+def test_align_sorts_entries_by_expert(n, E, lo, hi, k):
+    from enterprise_inference_amd._native import kernels as lib
+    from enterprise_inference_amd.ops._dispatch import ptr, stream
+    g = torch.Generator().manual_seed(n + E)
+    ids = torch.randint(0, E + 1, (n,), generator=g).to("cuda", torch.int32)   # E: no expert
+    offs = torch.full((hi - lo + 1,), -7, device="cuda", dtype=torch.int32)
+    row_idx, inv = (torch.full((n,), -7, device="cuda", dtype=torch.int32) for _ in range(2))
+    assert lib().eia_moe_align(ptr(ids), n, E, lo, hi, ptr(offs), ptr(row_idx), ptr(inv), k,
+                               stream(ids)) == 0
+    ids, offs, row_idx, inv = (t.tolist() for t in (ids, offs, row_idx, inv))
+    here = [i for i in range(n) if lo <= ids[i] < hi]
+    want = [0]
+    for e in range(lo, hi):
+        want.append(want[-1] + ids.count(e))
+    assert offs == want and sorted(inv[i] for i in here) == list(range(len(here)))
+    for i in range(n):
+        if lo <= ids[i] < hi:
+            assert offs[ids[i] - lo] <= inv[i] < offs[ids[i] - lo + 1] and row_idx[inv[i]] == i // k
+        else:
+            assert inv[i] == -1
+    assert row_idx[len(here):] == [0] * (n - len(here))
+
+
+@pytest.mark.parametrize("sk", [0, 1, 2, 3, 4])             # 0: the bf16 rows of an unsplit product
+@pytest.mark.parametrize("T,k,H", [(1, 1, 8), (3, 2, 1032), (5, 3, 2056), (2, 5, 4096), (70, 8, 1024)])
+def test_combine(T, k, H, sk):
+    from enterprise_inference_amd._native import kernels as lib
+    from enterprise_inference_amd.ops._dispatch import ptr, stream
+    g = torch.Generator().manual_seed(T + H + sk)
+    n = T * k
+    w = torch.rand(T, k, generator=g).to("cuda")
+    inv = torch.randperm(n, generator=g).to("cuda", torch.int32)
+    inv[torch.rand(n, generator=g).to("cuda") < 0.2] = -1          # another rank's expert
+    out = torch.full((T, H + 8), float("nan"), device="cuda", dtype=BF)
+    if sk:
+        part = torch.randn(sk, n, H, generator=g).to("cuda")
+        rows = part[0].clone()
+        for j in range(1, sk):
+            rows += part[j]
+        rows = rows.to(BF)
+        rc = lib().eia_moe_combine_sk(ptr(part), sk, n, ptr(w), ptr(inv), T, k, H, ptr(out),
+                                      out.stride(0), stream(out))
+    else:
+        rows = torch.randn(n, H, generator=g).to("cuda", BF)
+        rc = lib().eia_moe_combine(ptr(rows), rows.stride(0), ptr(w), ptr(inv), T, k, H, ptr(out),
+                                   out.stride(0), stream(out))
+    assert rc == 0
+    terms = rows.double()[inv.long().clamp(min=0)].view(T, k, H) * w.double()[:, :, None]
+    terms[(inv < 0).view(T, k)] = 0
+    # k fp32 products and sums, then one rounding to bf16
+    bound = terms.abs().sum(1) * (k * 2.0 ** -23) + terms.sum(1).abs() * 2.0 ** -8
+    assert ((out[:, :H].double() - terms.sum(1)).abs() <= bound).all()
+    assert out[:, H:].isnan().all()

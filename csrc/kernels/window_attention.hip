@@ -256,7 +256,7 @@ struct WinAttnArgs {
   int H, G, P, D, Dv, bs, window, keep, qb, epilogue;
   const float* lam;                 // [1], epilogue 1
   float eps, post;
-  int nparts;                       // MFMA form: key partitions over grid.z (1: none)
+  int nparts;                       // MFMA form: key partitions over grid.z (1: none; prefill: talk only)
   int raw_bufs;                     // MFMA form with head mixing: raw-score buffers in LDS (1, 2)
   float* part_acc; float* part_ml;  // [rows, M, nparts, Dv] and [rows, M, nparts, 2] partials
   int wmode;                        // 0: softmax; 1: sigmoid(score + bias), un-normalised
@@ -265,7 +265,7 @@ struct WinAttnArgs {
   float cap;                        // > 0: scores soft-capped, cap * tanh(s / cap)
   int talk_post;                    // talk mixes the softmax weights, not the scores (scalar form)
   int gate_heads;                   // gate [rows, H]: one value per head
-  int rows;                         // window_decode_kernel and its merge: rows of the launch
+  int rows;                         // rows of the launch
 };
 
 // The visible keys of a 16-query tile as absolute 32-key blocks: the blocks of the kept first
@@ -572,7 +572,7 @@ window_attn_mfma_kernel(const WinAttnArgs a) {
   const int pos_first = a.positions[row0], pos_last = a.positions[row0 + nq - 1];
   const WaBlocks kbs = wa_blocks(pos_first, pos_last, a.window, a.keep);
   const int wb0 = kbs.wb0, nsink = kbs.nsink, nblocks = kbs.nblocks;
-  const int np = wa_parts(a.nparts, nblocks);
+  const int np = a.cu ? a.nparts : wa_parts(a.nparts, nblocks);
   if ((int)blockIdx.z >= np) return;                                // (whole workgroup)
 
   // Q^T operands of this wave's maps: column = query c, rows = d 32 s + 8 g .. + 8
@@ -609,7 +609,8 @@ window_attn_mfma_kernel(const WinAttnArgs a) {
   const int r0 = 8 * (c >> 2) + (c & 3);                            // key of row c in tile 0
   const int dq = 8 * g;
 
-  // with key partitions (decode rows of small batches) this workgroup takes a slice of the blocks
+  // with key partitions (small batches) this workgroup takes a slice of the blocks; a prefill tile always has
+  // nparts of them, the last ones possibly empty, as its rows' merge does not know the tile
   const int per = (nblocks + np - 1) / np;
   const int b_lo = blockIdx.z * per, b_hi = min(nblocks, b_lo + per);
   // the pages of this workgroup's blocks, looked up once (the block loop then has no dependent
@@ -1139,7 +1140,8 @@ window_decode_kernel(const WinAttnArgs a) {
 // Merge of key partitions and the row's epilogue: one wave per (row, head).  Lane z first turns
 // partition z's (max, sum) into its weight; the value columns are then summed over the partitions.
 // Bound by latency: the partials of up to 16 partitions are asked for together with the weights' inputs, and these
-// meet within rows of 16 lanes (three rows of 8 heads, 8 partitions: 4.8 -> 2.9 us).
+// meet within rows of 16 lanes (three rows of 8 heads, 8 partitions: 4.8 -> 2.9 us), four at a time as far as there
+// are any (725 rows of 8 heads, 4 partitions: 7.7 us with all sixteen, 6.2).
 constexpr int WM_Z = 16;
 template <bool PACKED>
 __global__ void __launch_bounds__(64)
@@ -1151,7 +1153,7 @@ window_attn_merge_kernel(const WinAttnArgs a) {
   const int pos = a.positions[row], len = (a.lens ? a.lens : a.positions)[row];
   if (a.lens && len <= 0) return;                   // padding row: the partition kernel wrote zeros
   const int nblocks = wa_blocks(pos, pos, a.window, a.keep).nblocks;
-  const int np = PACKED ? wd_parts(NP, nblocks) : wa_parts(NP, nblocks);
+  const int np = a.cu ? NP : PACKED ? wd_parts(NP, nblocks) : wa_parts(NP, nblocks);
   if (np == 1) return;                              // a whole row: already finished and written
   const int d0 = min(lane, Dv - 1), d1 = min(lane + 64, Dv - 1);
   float o[2][2];                                    // [map][column lane, lane + 64]
@@ -1164,10 +1166,15 @@ window_attn_merge_kernel(const WinAttnArgs a) {
       const float mz = z < np ? a.part_ml[(pr + z) * 2] : -1e30f;
       const float lz = z < np ? a.part_ml[(pr + z) * 2 + 1] : 0.f;
 #pragma unroll
-      for (int y = 0; y < WM_Z; ++y) {              // (past the last one: the last one, with no weight)
-        const float* p = a.part_acc + (pr + min(y, np - 1)) * Dv;
-        x0[y] = p[d0];
-        x1[y] = p[d1];
+      for (int y0 = 0; y0 < WM_Z; y0 += 4) {        // (past the last one: the last one, with no weight)
+        if (y0 < np) {
+#pragma unroll
+          for (int y = y0; y < y0 + 4; ++y) {
+            const float* p = a.part_acc + (pr + min(y, np - 1)) * Dv;
+            x0[y] = p[d0];
+            x1[y] = p[d1];
+          }
+        }
       }
       // sigmoid weights: the partitions' sums simply add up
       const float top = row16_max(mz);              // (of all lanes: none may have branched off)
@@ -1227,7 +1234,7 @@ EIA_API int eia_window_attn_mfma(const void* q, long ldq, const void* kc, const 
                                  int window, int keep, int epilogue, const float* lam, float eps,
                                  float post, int wmode, const float* bias, int nparts,
                                  float* part_acc, float* part_ml, const float* sink, float cap,
-                                 int gate_heads, hipStream_t st) {
+                                 int gate_heads, int rows, hipStream_t st) {
   if (n_items < 0 || H < 1 || G < 1 || H % G || (P != 1 && P != 2) || bs < 1 || keep < 0 || !q ||
       !kc || !vc || !bt || !positions || !mult || !out)
     return EIA_BAD_SHAPE;
@@ -1237,13 +1244,14 @@ EIA_API int eia_window_attn_mfma(const void* q, long ldq, const void* kc, const 
   if (!eia_window_attn_mfma_ok(H, G, P, D, Dv, bs, talk != nullptr)) return EIA_UNSUPPORTED;
   if (cap < 0.f) return EIA_BAD_SHAPE;
   if (ldq % 8 || ldo % 4) return EIA_BAD_SHAPE;
-  // key partitions: decode rows only (a row is its own work item), partials in the workspace
-  if (nparts < 1 || nparts > 64 || (nparts > 1 && (cu || !part_acc || !part_ml)))
+  // key partitions: decode rows (a row is its own work item) and head mixing, partials in the workspace
+  if (nparts < 1 || nparts > 64 || (nparts > 1 && ((cu && !talk) || !part_acc || !part_ml)) ||
+      (!cu && rows < n_items))
     return EIA_BAD_SHAPE;
   if (n_items == 0) return EIA_OK;
   WinAttnArgs a{q, ldq, kc, vc, bt, ldbt, positions, cu, work, lens, mult, slope, talk, gate, ldg,
                 out, ldo, H, G, P, D, Dv, bs, window, keep, 16, epilogue, lam, eps, post, nparts,
-                2, part_acc, part_ml, wmode, bias, sink, cap, 0, gate_heads, n_items};
+                2, part_acc, part_ml, wmode, bias, sink, cap, 0, gate_heads, rows};
   const bool packed = !cu && !talk && eia_window_decode_packed(H, G);
   // raw-score buffers of the head-mixing form: two (one barrier per block) while they fit 48 KiB
   if (talk) a.raw_bufs = (size_t)2 * H * P * 128 * sizeof(f32x4) > 48 * 1024 ? 1 : 2;
@@ -1326,6 +1334,6 @@ EIA_API int eia_window_attn_mfma(const void* q, long ldq, const void* kc, const 
 #undef WA_LAUNCH
 #undef WA_LAUNCH1
   if (nparts > 1)
-    hipLaunchKernelGGL(window_attn_merge_kernel<false>, dim3(n_items, H), dim3(64), 0, st, a);
+    hipLaunchKernelGGL(window_attn_merge_kernel<false>, dim3(rows, H), dim3(64), 0, st, a);
   EIA_LAUNCH_CHECK();
 }

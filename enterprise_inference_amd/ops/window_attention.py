@@ -165,6 +165,26 @@ def flash_parts(n_items: int, spec: WindowSpec, queries: int, longest: int, cont
                       merge=7 if narrow else 6)
 
 
+def mix_parts(n_items: int, spec: WindowSpec, context: int, cus: int = 256) -> int:
+    """Key partitions of a prefill launch of the 16-query MFMA form with head mixing, whose block tables reach
+    ``context`` tokens.  A workgroup holds every head of its queries and waits for its keys and values (about 4 us per
+    32-key block of 8 heads of 128, 6 of 16), so launches that leave CUs idle cut the keys until each CU has one
+    workgroup of more than 8 heads or two smaller ones, down to two blocks each.  Above half a workgroup per CU only
+    long windows are cut: there the partials cost more than the few blocks that a cut saves.  MI355X, us in 1 / 2 / 4 / 8 / 16
+    partitions, 8 heads on 2, window 1024: 725 tokens behind 1362 (46 row blocks) 129 / 73 / 48 / 41 / 42, 4 portions of
+    500 behind 500 (128) 126 / 77 / 56 / 61 / 72, 2 of 2000 (250, heads of 96) 125 / 97 / 99 / 105, 2 of 4000 (500, heads
+    of 64) 112 / - / 116; 16 heads on 4: 200 behind 600 (13) 154 / 84 / 53 / 40 / 31, 6 of 500 (192) 111 / 87 / 93 / 104,
+    4096 within 300 (256) 87 / 132, 16 of 96 (96 of three blocks) 24 / 35."""
+    if spec.talk is None:
+        return 1
+    blocks = -(-context // 32)
+    if spec.window > 0:
+        blocks = min(blocks, (spec.window + MFMA_QB + 29) // 32 + 1 + (spec.keep + 31) // 32)
+    if 2 * n_items > cus and blocks < 16:
+        return 1
+    return max(1, min(16, blocks // 2, (2 if spec.heads <= 8 else 1) * cus // max(1, n_items)))
+
+
 def query_block(spec: WindowSpec, dtype: torch.dtype, block_size: int) -> int:
     if not mfma_ok(spec, dtype, block_size):
         return SCALAR_QB
@@ -601,10 +621,12 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
                 "window_flash")
             return
         if mfma:
-            NP = decode_partitions(n_items, spec) if cu is None else 1
+            rows = n_items if cu is None else T - lo
+            NP = (decode_partitions(n_items, spec) if cu is None else
+                  mix_parts(n_items, spec, bt.shape[1] * bs))
             pa = pm = None
             if NP > 1:
-                n = n_items * H * P * NP
+                n = rows * H * P * NP
                 ws = torch.empty(n * (Dv + 2), dtype=torch.float32, device=q.device)
                 pa = ws.data_ptr()
                 pm = pa + 4 * n * Dv
@@ -615,7 +637,7 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
                 ptr(o), o.stride(0), H, spec.kv_heads, P, D, Dv, bs, spec.window, spec.keep,
                 spec.epilogue, ptr(spec.lam), float(spec.eps), float(spec.post), spec.weights,
                 ptr(spec.bias), NP, pa, pm, ptr(spec.sink), float(spec.cap),
-                1 if spec.gate_heads else 0, stream(q)), "window_attn_mfma")
+                1 if spec.gate_heads else 0, rows, stream(q)), "window_attn_mfma")
             return
         check(lib().eia_window_attn(
             ptr(qa), qa.stride(0), ptr(k_cache), ptr(v_cache), ptr(bt), bt.stride(0),

@@ -1,4 +1,4 @@
-"""Decode rows in key partitions, against the ops' own plain CPU path: rows that the grid is padded for, a padding
+"""Rows in key partitions, against the ops' own plain CPU path: rows that the grid is padded for, a padding
 row, lengths where a row has one partition more or less, and more partitions than the merge takes at once."""
 
 import pytest
@@ -108,3 +108,36 @@ def test_partitions():
         for G in (1, 2, 4, 8):
             assert WA.decode_partitions(n, spec(0, G)) == 1 or rows * G * WA.decode_partitions(n, spec(0, G)) <= 32
         assert LA.decode_partitions(n, 64) == 1 or rows * 4 * LA.decode_partitions(n, 64) <= 32
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("parts", [0, 2, 5, 16])                # 0: the layer's own rule
+@pytest.mark.parametrize("H,G,D,window,keep", [(8, 2, 128, 100, 0), (16, 4, 64, 0, 0), (3, 1, 96, 300, 5), (6, 3, 32, 40, 0)])
+@pytest.mark.parametrize("new,past", [([1, 40, 17], [0, 250, 31]), ([33], [300])], ids=["ragged", "one"])
+def test_mixed_prefill(new, past, H, G, D, window, keep, parts, monkeypatch):
+    if parts:
+        monkeypatch.setattr(WA, "mix_parts", lambda *a: parts)
+    g = torch.Generator().manual_seed(H + D)
+    md, pages = _step([n + p for n, p in zip(new, past)], g)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32)
+    T, cu = sum(new), [0]
+    for n in new:
+        cu.append(cu[-1] + n)
+    md = dict(md, num_decode=0, num_prefill_tokens=T, decode_block_tables=None, decode_seq_lens=None,
+              positions=i32([p + i for n, p in zip(new, past) for i in range(n)]), prefill_cu_q=i32(cu),
+              prefill_block_tables=md["decode_block_tables"], prefill_q_lens=new)
+    rnd = lambda *s: torch.randn(*s, generator=g)
+    bf = lambda *s: rnd(*s).to(torch.bfloat16)
+    tensors = [bf(T, H * D), bf(pages, PAGE, G * D), bf(pages, G * D, PAGE), bf(T, H * D), rnd(H).abs() * 0.02,
+               torch.eye(H) + 0.05 * rnd(H, H), rnd(H) if keep else None]
+
+    def call(dev, t, m):
+        spec = WA.WindowSpec(H, G, 1, D, D, window, keep, torch.full((H,), D ** -0.5, device=dev))
+        spec.slope, spec.talk, spec.sink = t[4:]
+        return WA.window_attention(t[0], t[1], t[2], m, spec, t[3])
+
+    ref, out = [], []
+    for dev, to in (("cpu", ref), ("cuda", out)):
+        m = A.AttentionMetadata(**{k: v.to(dev) if isinstance(v, torch.Tensor) else v for k, v in md.items()})
+        to.append(call(dev, [None if t is None else t.to(dev) for t in tensors], m))
+    assert torch.isfinite(out[0]).all() and _rel(out[0], ref[0]) < 2.0 ** -8 * 2      # two roundings to bf16

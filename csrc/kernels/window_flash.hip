@@ -78,10 +78,31 @@ EIA_DEV WfRows wf_rows(const FlashArgs& a, int w, int r32) {
   return r;
 }
 
-// Wave w's place for part z of the workgroup's rows: 4 NDV + 1 units of 64 lanes x 4 floats.
-EIA_DEV float* wf_part(const FlashArgs& a, int z, int w, int ndv) {
+// The place of wave w of P maps for part z of the workgroup's rows: 4 NDV + 1 units of 64 lanes x 4 floats.
+template <int P, int NDV>
+EIA_DEV float* wf_part(const FlashArgs& a, int z, int w) {
   const long wg = (long)blockIdx.y * gridDim.x + blockIdx.x;
-  return a.part + ((wg * a.nparts + z) * 4 + w) * (4 * ndv + 1) * 256;
+  return a.part + ((wg * a.nparts + z) * 4 * P + w) * (4 * NDV + 1) * 256;
+}
+
+// Column tile dt of the part at x joins the lane's sums.
+template <bool SIG, int NDV>
+EIA_DEV void wf_join(const float* x, int dt, float& m, float& lsum, f32x16_t (&o)[1]) {
+  const f32x4 ml = *reinterpret_cast<const f32x4*>(x + 4 * NDV * 256);
+  float w0 = 1.f, w1 = 1.f;
+  if constexpr (!SIG) {
+    const float mn = fmaxf(m, ml[0]);
+    w0 = __builtin_amdgcn_exp2f(m - mn);
+    w1 = __builtin_amdgcn_exp2f(ml[0] - mn);
+    m = mn;
+  }
+  lsum = SIG ? 1.f : lsum * w0 + ml[1] * w1;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const f32x4 v = *reinterpret_cast<const f32x4*>(x + (4 * dt + i) * 256);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[0][4 * i + e] = o[0][4 * i + e] * w0 + v[e] * w1;
+  }
 }
 
 // From a lane's sums to its outputs: columns c0 + 32 dt + 8 j + 4 hh + i of its query.
@@ -375,7 +396,7 @@ window_flash_kernel(FlashArgs a) {
   }
   float lsum = SIG ? 1.f : flash_pair_sum(l_run);
   if (SPLIT && parts > 1) {
-    float* x = wf_part(a, blockIdx.z, w, NDV) + 4 * lane;
+    float* x = wf_part<P, NDV>(a, blockIdx.z, 4 * map + w) + 4 * lane;
 #pragma unroll
     for (int dt = 0; dt < NDV; ++dt)
 #pragma unroll
@@ -422,44 +443,67 @@ window_flash_merge_kernel(FlashArgs a) {
 #pragma unroll
   for (int i = 0; i < 16; ++i) oacc[0][i] = 0.f;
 #pragma unroll 2
-  for (int z = 0; z < parts; ++z) {
-    const float* x = wf_part(a, z, w, NDV) + 4 * lane;
-    const f32x4 ml = *reinterpret_cast<const f32x4*>(x + 4 * NDV * 256);
-    float w0 = 1.f, w1 = 1.f;
-    if constexpr (!SIG) {
-      const float mn = fmaxf(m, ml[0]);
-      w0 = __builtin_amdgcn_exp2f(m - mn);
-      w1 = __builtin_amdgcn_exp2f(ml[0] - mn);
-      m = mn;
-    }
-    lsum = SIG ? 1.f : lsum * w0 + ml[1] * w1;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const f32x4 v = *reinterpret_cast<const f32x4*>(x + (4 * dt + i) * 256);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) oacc[0][4 * i + e] = oacc[0][4 * i + e] * w0 + v[e] * w1;
-    }
-  }
+  for (int z = 0; z < parts; ++z) wf_join<SIG, NDV>(wf_part<1, NDV>(a, z, w) + 4 * lane, dt, m, lsum, oacc);
   wf_finish<1, 1>(a, rw, lane >> 5, oacc, lsum, 32 * dt);
+}
+
+// The parts of a differential pair, 32 rows a workgroup: a wave for each map and 32 columns, as above; the second
+// map's waves hand theirs over, and the root mean square of the difference meets in LDS.  (One wave a map with all
+// columns: 2 parts of 46 row blocks of 128 columns 44 us with the products, this way 36; uncut 49.)
+template <int NDV>
+__global__ void __launch_bounds__(128 * NDV)
+window_flash_merge_pair_kernel(FlashArgs a) {
+  __shared__ float other[NDV][16][64], sq[NDV][64];
+  const int lane = threadIdx.x & 63, dt = (threadIdx.x >> 6) % NDV, map = threadIdx.x / (64 * NDV), w = blockIdx.z;
+  const WfRows rw = wf_rows(a, w, lane & 31);
+  const int parts = min(a.nparts, (rw.ntile + a.per - 1) / a.per);
+  if (rw.qn <= 0 || parts <= 1 || !rw.live) return;     // (whole workgroup)
+  float m = -INFINITY, lsum = 0.f, ss = 0.f;
+  f32x16_t o[1];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) o[0][i] = 0.f;
+#pragma unroll 2
+  for (int z = 0; z < parts; ++z)
+    wf_join<false, NDV>(wf_part<2, NDV>(a, z, 4 * map + w) + 4 * lane, dt, m, lsum, o);
+  const float f = map ? -a.lam[0] / lsum : 1.f / lsum;
+  if (map) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) other[dt][i][lane] = o[0][i] * f;
+  }
+  __syncthreads();
+  if (!map) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      o[0][i] = o[0][i] * f + other[dt][i][lane];
+      ss += o[0][i] * o[0][i];
+    }
+    sq[dt][lane] = flash_pair_sum(ss);
+  }
+  __syncthreads();
+  if (map) return;
+  ss = 0.f;
+#pragma unroll
+  for (int t = 0; t < NDV; ++t) ss += sq[t][lane];
+  wf_finish<1, 1>(a, rw, lane >> 5, o, sqrtf(ss / (float)a.Dv + a.eps), 32 * dt);
 }
 
 template <int P, int ND, int NDV, bool SIG, bool SPLIT>
 static void wf_launch(const FlashArgs& a, int n_items, int parts, hipStream_t st) {
   hipLaunchKernelGGL((window_flash_kernel<P, ND, NDV, SIG, SPLIT>), dim3(a.H / a.hpw, n_items, parts), dim3(256 * P),
                      0, st, a);
-  if (SPLIT)
+  if constexpr (SPLIT && P == 2)
+    hipLaunchKernelGGL((window_flash_merge_pair_kernel<NDV>), dim3(a.H / a.hpw, n_items, 4), dim3(128 * NDV), 0,
+                       st, a);
+  else if constexpr (SPLIT)
     hipLaunchKernelGGL((window_flash_merge_kernel<NDV, SIG>), dim3(a.H / a.hpw, n_items, NDV), dim3(256), 0, st, a);
 }
 
 template <int P, int ND, int NDV, bool SIG>
 static void wf_go(const FlashArgs& a, int n_items, int parts, hipStream_t st) {
-  if constexpr (P == 1) {
-    if (parts > 1) {
-      wf_launch<P, ND, NDV, SIG, true>(a, n_items, parts, st);
-      return;
-    }
-  }
-  wf_launch<P, ND, NDV, SIG, false>(a, n_items, 1, st);
+  if (parts > 1)
+    wf_launch<P, ND, NDV, SIG, true>(a, n_items, parts, st);
+  else
+    wf_launch<P, ND, NDV, SIG, false>(a, n_items, 1, st);
 }
 
 }  // namespace
@@ -474,9 +518,9 @@ EIA_API int eia_window_flash_queries(int H, int G, int P, int D, int Dv, int bs)
 }
 
 // Prompt portions of window attention without head mixing or slopes; the arguments are those of
-// eia_window_attn_mfma, work holds blocks of eia_window_flash_queries queries.  nparts > 1 (P == 1):
+// eia_window_attn_mfma, work holds blocks of eia_window_flash_queries queries.  nparts > 1:
 // row blocks of more than per 64-key tiles are cut into parts of at most that many (nparts * per
-// tiles cover the longest), which meet in part [n_items * H / hpw, nparts, 4, 4 ceil(Dv / 32) + 1,
+// tiles cover the longest), which meet in part [n_items * H / hpw, nparts, 4 P, 4 ceil(Dv / 32) + 1,
 // 256] fp32, hpw = 128 / queries (Dv counted as 128 where D > 96 or Dv > 96 or D <= 64 < Dv).
 EIA_API int eia_window_flash(const void* q, long ldq, const void* kc, const void* vc, const int* bt,
                              int ldbt, const int* positions, const int* cu, const int* work,
@@ -488,7 +532,7 @@ EIA_API int eia_window_flash(const void* q, long ldq, const void* kc, const void
   if (n_items < 0 || keep < 0 || cap < 0.f || !q || !kc || !vc || !bt || !positions || !cu || !work ||
       !mult || !out || (P == 2) != (lam != nullptr) || (P == 2 && gate) ||
       (wmode != 0 && wmode != 1) || (wmode == 1 && (P != 1 || sink)) || ldq % 8 || ldo % 4 ||
-      nparts < 1 || (nparts > 1 && (P != 1 || per < 1 || !part)))
+      nparts < 1 || (nparts > 1 && (per < 1 || !part)))
     return EIA_BAD_SHAPE;
   const int qb = eia_window_flash_queries(H, G, P, D, Dv, bs);
   if (!qb) return EIA_UNSUPPORTED;

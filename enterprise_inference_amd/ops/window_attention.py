@@ -157,12 +157,28 @@ def flash_parts(n_items: int, spec: WindowSpec, queries: int, longest: int, cont
     tiles = -(-context // 64)
     if spec.window > 0:
         tiles = min(tiles, (spec.window + queries + 62) // 64 + 1 + (spec.keep + 63) // 64)
-    if spec.maps == 2:
+    if spec.maps == 2:                                   # (cut by pair_parts)
         return 1, tiles
     narrow = max(spec.dim, spec.vdim) <= 64
     return split_keys(n_items * (spec.heads * queries // 128), tiles,
                       tiles if spec.window > 0 else tiles - longest // 128, (3 if narrow else 2) * cus,
                       merge=7 if narrow else 6)
+
+
+def pair_parts(n_items: int, spec: WindowSpec, queries: int, context: int, cus: int = 256):
+    """(parts, 64-key tiles per part) of a flash prefill launch of a differential pair: one workgroup (eight waves) a
+    CU, so launches that leave CUs idle are cut until each has one, down to three tiles a part; fewer than 12 tiles
+    are not worth the second launch.  MI355X, heads of 64 + 64 and 128, window 1024 (18 tiles), us in 1 / 2 / 3 / 4 / 6
+    parts: 8 workgroups 45 / 29 / 24 / 22 / 20, 46: 49 / 36 / 33 / 32 / 31, 126: 47 / 42 / 51 / 49, 128: 42 / 38 / 45 / 47,
+    250: 53 / 73; window 300 (7 tiles), 128: 26 / 30."""
+    tiles = -(-context // 64)
+    if spec.window > 0:
+        tiles = min(tiles, (spec.window + queries + 62) // 64 + 1 + (spec.keep + 63) // 64)
+    parts = min(cus // max(1, n_items * (spec.heads * queries // 128)), tiles // 3)
+    if tiles < 12 or parts < 2:
+        return 1, tiles
+    per = -(-tiles // parts)
+    return -(-tiles // per), per
 
 
 def mix_parts(n_items: int, spec: WindowSpec, context: int, cus: int = 256) -> int:
@@ -605,11 +621,14 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
                 "head_mix_attn")
             return
         if mfma and cu is not None and flash_queries(spec, bs):
-            NP, per = flash_parts(n_items, spec, qb, max(md.prefill_q_lens or [T]), bt.shape[1] * bs)
+            if P == 2:
+                NP, per = pair_parts(n_items, spec, qb, bt.shape[1] * bs)
+            else:
+                NP, per = flash_parts(n_items, spec, qb, max(md.prefill_q_lens or [T]), bt.shape[1] * bs)
             pa = None
             if NP > 1:
                 vt = 4 if max(D, Dv) > 96 or D <= 64 < Dv else -(-max(D, Dv) // 32)
-                pa = torch.empty(n_items * (H * qb // 128) * NP * 4 * (4 * vt + 1) * 256,
+                pa = torch.empty(n_items * (H * qb // 128) * NP * 4 * P * (4 * vt + 1) * 256,
                                  dtype=torch.float32, device=q.device)
             check(lib().eia_window_flash(
                 ptr(qa), qa.stride(0), ptr(k_cache), ptr(v_cache), ptr(bt), bt.stride(0),

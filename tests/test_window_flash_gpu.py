@@ -198,3 +198,35 @@ def test_window_decode_slots_behind(parts, D, Dv, bs, kind, monkeypatch):
 
     a, b = run("cpu").double(), run("cuda").double()
     assert float((a - b).norm() / a.norm()) < 4e-3           # one bf16 rounding (2^-9) on each side
+
+
+@pytest.mark.parametrize("H,G,D,Dv,bs", [(8, 2, 64, 128, 64), (3, 1, 40, 48, 64), (2, 2, 64, 80, 128)])
+@pytest.mark.parametrize("window,keep,new,past", [(900, 5, [130, 1, 31], [1500, 0, 800]), (0, 0, [40, 700], [1000, 0])])
+@pytest.mark.parametrize("parts", [0, 2, 7])                 # 0: the layer's own rule
+def test_window_flash_pairs_in_parts(parts, window, keep, new, past, H, G, D, Dv, bs, monkeypatch):
+    """Differential pairs whose keys are cut: both maps' parts, row blocks with fewer parts than others or one."""
+    from enterprise_inference_amd.ops import attention as A
+    from enterprise_inference_amd.ops import window_attention as wa
+    if parts:
+        monkeypatch.setattr(wa, "pair_parts", lambda n, sp, q, c: (parts, -(-(-(-c // 64)) // parts)))
+    g, bf = torch.Generator().manual_seed(H + Dv), torch.bfloat16
+    bt, n = _pages(g, [a + b for a, b in zip(new, past)], bs)
+    cu = torch.tensor([0] + new).cumsum(0).to(torch.int32)
+    pos = torch.cat([torch.arange(k) + f for k, f in zip(new, past)]).to(torch.int32)
+    T = int(cu[-1])
+    rnd = lambda *s: torch.randn(*s, generator=g).to(bf)
+    q, k, v = rnd(T, H * 2 * D), rnd(n, bs, G * 2 * D), rnd(n, G * Dv, bs)
+
+    def run(dev):
+        md = A.AttentionMetadata(
+            num_decode=0, num_prefill_tokens=T, slot_mapping=pos.to(dev), positions=pos.to(dev),
+            prefill_block_tables=bt.to(dev), prefill_cu_q=cu.to(dev), prefill_q_lens=new)
+        spec = wa.WindowSpec(H, G, 2, D, Dv, window, keep, mult=torch.full((2 * H,), D ** -0.5).to(dev))
+        spec.epilogue, spec.eps, spec.post, spec.lam = 1, 1e-5, 0.7, torch.tensor([0.4]).to(dev)
+        if dev == "cuda" and not parts:
+            qb = wa.query_block(spec, bf, bs)
+            assert wa.pair_parts(sum(-(-a // qb) for a in new), spec, qb, bt.shape[1] * bs)[0] > 1
+        return wa.window_attention(q.to(dev), k.to(dev), v.to(dev), md, spec, None).cpu()
+
+    a, b = run("cpu").double(), run("cuda").double()
+    assert float((a - b).norm() / a.norm()) < 4e-3           # one bf16 rounding (2^-9) on each side

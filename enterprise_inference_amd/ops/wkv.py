@@ -31,6 +31,15 @@ def chunk_rows(nseq: int, heads: int) -> int:
     return 48 + min(64, nseq * heads // 32)
 
 
+def chunk_rows_beside(nseq: int, heads: int) -> int:
+    """Rows from which the shorter sequences of a step go along where the chunk-parallel form is launched for a long
+    one: they then cost a chunk each, but no more tokens after one another.  MI355X, a sequence of 500 rows and so many
+    shorter ones, token by token / along: 40 heads, 3 of 8 43 / 36 us, 3 of 48 64 / 43, 15 of 8 49 / 63, 15 of 24 59 / 64,
+    15 of 48 74 / 67, 63 of 48 147 / 160; 16 heads, 15 of 8 33 / 32, 15 of 24 41 / 34, 63 of 24 55 / 72, 63 of 48 75 / 82;
+    51 to 102 rows, 11 sequences of 40 heads 84 / 54."""
+    return max(1, nseq * heads // 20)
+
+
 def takes_chunks(rows: int, nseq: int, split: int, longest: int = 0) -> bool:
     """Whether the chunk-parallel form is launched beside the token-by-token one, each of which takes
     its own sequences.  Where the caller does not know the ``longest`` sequence's rows, only the device
@@ -133,13 +142,14 @@ def wkv_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor,
     split = chunk_rows(nseq, heads) if cu is not None and D <= CHUNK_DIM else 0
     if not takes_chunks(T, nseq, split, longest):
         split = 0
+    least = min(split, chunk_rows_beside(nseq, heads))
     if nseq > 1 or not split:
-        check(lib().eia_wkv_scan(*args, heads, D, split, 1 if bf else 0, stream(r)), "wkv_scan")
+        check(lib().eia_wkv_scan(*args, heads, D, least, 1 if bf else 0, stream(r)), "wkv_scan")
     if split:
         n = T // CHUNK + nseq
         U = torch.empty(n, heads, CHUNK_DIM, CHUNK_DIM, dtype=torch.float32, device=r.device)
         L = torch.empty(n, heads, CHUNK_DIM, dtype=torch.float32, device=r.device)
         # (a single sequence goes here whatever part of the T rows it owns)
-        check(lib().eia_wkv_scan_chunked(*args, T, heads, D, split if nseq > 1 else 1, ptr(U), ptr(L),
+        check(lib().eia_wkv_scan_chunked(*args, T, heads, D, least if nseq > 1 else 1, ptr(U), ptr(L),
                                          1 if bf else 0, stream(r)), "wkv_scan_chunked")
     return y

@@ -52,6 +52,23 @@ def test_wkv_chunks(lens, H, D, dtype):
     assert torch.equal(dev[9].cpu(), prev)
 
 
+@pytest.mark.parametrize("least", [1, 8, 10, 64])
+@pytest.mark.parametrize("lens", [[9, 150, 8, 7, 63, 64, 65], [70, 9]])
+def test_wkv_short_sequences_beside_a_long_one(lens, least, monkeypatch):
+    """The same whichever of the two forms the shorter sequences take."""
+    from enterprise_inference_amd.ops import wkv
+    monkeypatch.setattr(wkv, "chunk_rows_beside", lambda n, h: least)
+    n, T, H, D = len(lens), sum(lens), 2, 64
+    cu, pos, slots = _step(lens, [3] * n, False)
+    args = _wkv_args(torch.Generator().manual_seed(n), T, n, H, D, torch.float32) + [slots, cu]
+    dev = [t.to("cuda") for t in args]
+    y = wkv.wkv_scan(*args, n, pos, None, 1e-5, H)
+    z = wkv.wkv_scan(*dev, n, pos.to("cuda"), None, 1e-5, H).cpu()
+    # fp32 sums over at most 64 products and a few exponentials
+    assert _rel(z, y) < 1e-5 and _rel(dev[8], args[8]) < 2e-6
+    assert torch.equal(dev[9].cpu(), args[9])
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("mode,rot,half", [("exp_gates", 0, True), ("decay", 64, True),
                                            ("decay", 12, False), ("exp_gates", 20, True)])

@@ -106,6 +106,19 @@ CHUNK_MIN_ROWS = 48        # a sequence with at least this many rows in the step
 FORCE_CHUNKED = os.environ.get("EIA_SCAN_FORCE_CHUNKED", "0") == "1"
 
 
+# (decays 0 / exponential gates 1 / a decay per channel 2, wider than 64): us per token of the token-by-token form; us for
+# the launches, per row and head, per sequence and head of the chunk-parallel one (fitted to the figures behind).
+# Sequences x rows, token by token / chunks, us:
+RATES = {
+    (0, False): (0.52, 24, 0.00034, 0.015),   # 32 x 64: 1x64 33 / 27, 16x64 36 / 43, 16x128 78 / 55, 64x64 107 / 126
+    (0, True): (0.90, 36, 0.0012, 0.10),      # 16 x 128, rotated: 1x48 44 / 36, 16x64 67 / 82, 16x128 120 / 101, 64x64 241 / 209
+    (1, False): (0.85, 25, 0.0003, 0.025),    # 32 x 64: 1x48 38 / 32, 16x48 43 / 47, 16x64 53 / 48, 64x64 166 / 115
+    (1, True): (1.30, 31, 0.0010, 0.065),     # 16 x 128: 1x48 65 / 32, 16x48 70 / 61, 16x128 166 / 74, 64x64 339 / 159
+    (2, False): (0.70, 30, 0.00059, 0.019),   # 32 x 32 x 64: 1x48 34 / 32, 16x64 50 / 59, 16x128 97 / 78, 64x64 130 / 146
+    (2, True): (1.00, 32, 0.0017, 0.0),       # 16 x 64 x 128: 1x48 54 / 36, 16x64 72 / 60, 16x128 142 / 71, 64x64 281 / 141
+}
+
+
 class ChunkPlan:
     """A step's rows cut into chunks for the chunk-parallel forms: ``n`` chunks over sequences of
     ``lens`` rows from row ``row0`` on; ``rows`` the step's row count, ``longest`` the longest
@@ -143,31 +156,19 @@ class ChunkPlan:
         return self.lists()[1]
 
     def pays(self, heads: int, dim: int, cus: int = 256, channel: bool = False,
-             key_dim: int = 0) -> bool:
+             key_dim: int = 0, exp_gates: bool = False) -> bool:
         """Whether the chunk-parallel form beats the token-by-token one for a layer of ``heads``
-        heads up to ``dim`` wide.  The latter walks the longest sequence at about 0.5 us a token
-        (0.85 us above 64) while its workgroups, one per (sequence, head), do not share CUs.  The
-        former costs 30 us for its launches and 0.7 ns (2 ns) per row and head, a short sequence
-        counting as 96 rows; with a decay per key channel 0.8 ns (1.7 ns, 64 rows), and 5 ns (7 ns)
-        for keys above KEY_DIM64, against 0.6 us (1.0 us) a token.  MI355X, 16 heads of 128,
-        exponential gates, token by token / chunks: 1 x 48 rows 64 / 31 us, 1 x 4096 4815 / 91,
-        16 x 64 89 / 59, 16 x 512 604 / 144; 32 heads of 64, fixed decays: 1 x 48 27 / 28, 16 x 64
-        40 / 50, 16 x 128 81 / 74, 1 x 4096 2041 / 82; 16 heads of 64 x 128, a decay per channel: 1 x
-        48 54 / 38, 16 x 64 75 / 67, 16 x 512 538 / 215, 1 x 4096 4316 / 125; 32 of 32 x 64: 1 x 48
-        35 / 33, 16 x 64 52 / 74, 16 x 128 96 / 91, 64 x 64 135 / 199.  The costs were fitted to chunks in fp32
-        products (16 x 64 rows of 16 heads 63 us, 1 x 4096 145): some steps near the line, 16 x 64 rows of 16 heads and
-        16 x 128 of 32 among them, take the token form although chunks are faster now."""
+        heads up to ``dim`` wide.  The latter walks the longest sequence, so many us a token, while its
+        workgroups, one per (sequence, head), do not share CUs.  The former costs so many us for its
+        launches and for a head so many per row and per sequence."""
         wide = dim > 64
-        if channel and key_dim <= KEY_DIM64:
-            busy = self.nseq * heads / (cus if wide else 2.7 * cus)
-            serial = self.longest * (1.0 if wide else 0.6) * max(1.0, busy)
-            return 32 + max(self.rows, 64 * self.nseq) * heads * (0.0017 if wide else 0.0008) < serial
-        if channel:
+        if channel and key_dim > KEY_DIM64:
             serial = self.longest * (0.85 if wide else 0.5) * -(-self.nseq * heads // cus)
             return self.rows * heads * (0.0072 if wide else 0.0052) < serial
+        token, launches, row, seq = RATES[(2 if channel else 1 if exp_gates else 0, wide)]
         busy = self.nseq * heads / (cus if wide else 2.7 * cus)
-        serial = self.longest * (0.85 if wide else 0.5) * max(1.0, busy)
-        return 30 + max(self.rows, 96 * self.nseq) * heads * (0.002 if wide else 0.0007) < serial
+        return (launches + heads * (row * self.rows + seq * self.nseq) <
+                token * self.longest * max(1.0, busy))
 
 
 def chunk_plan(host_lens, device, chunk: int = CHUNK, min_rows: int = CHUNK_MIN_ROWS,
@@ -310,7 +311,7 @@ def linear_scan(fused: torch.Tensor, q_off: int, k_off: int, v_off: int, g_off: 
             0 if spec.norm_shared else Dv)
     if (plan is not None and plan.n and max(D, Dv) <= CHUNK_MAX_DIM and cu is not None
             and plan.rows == T and
-            (FORCE_CHUNKED or plan.pays(H, max(D, Dv), channel=channel, key_dim=D))
+            (FORCE_CHUNKED or plan.pays(H, max(D, Dv), channel=channel, key_dim=D, exp_gates=exp_gates))
             and not torch.cuda.is_current_stream_capturing()):
         dev = fused.device
         f32 = lambda *shape: torch.empty(*shape, dtype=torch.float32, device=dev)

@@ -1821,7 +1821,7 @@ EIA_API int eia_linear_scan_channels(const void* x, long ld, int q_off, int k_of
 // cover; pairs of different 8-token blocks meet through the edges of the blocks between them, for those
 // inside a block see eia_chunks.h.  Products are fp32 matrix-core products.  Bound by instruction issue
 // (exponentials, operand rows through LDS), as there.
-// Four prompts of 490 to 977 tokens, 16 heads of 64 x 128, bf16: 21 + 22 + 11 + 60 us on an MI355X (l, (1),
+// Four prompts of 490 to 977 tokens, 16 heads of 64 x 128, bf16: 21 + 22 + 11 + 48 us on an MI355X (l, (1),
 // (2), (3)); in the 32-token chunks of vector FMAs above 38 + 71 + 21 + 235 us, which remain for keys
 // wider than 64.
 constexpr int GC = 64;                      // tokens per chunk

@@ -513,6 +513,11 @@ static void wf_go(const FlashArgs& a, int n_items, int parts, hipStream_t st) {
 
 }  // namespace
 
+// 32-column tiles of a wave's part in the workspace: those of the kernel that takes the shape, whatever Dv needs.
+EIA_API int eia_window_flash_columns(int P, int D, int Dv) {
+  return P == 2 ? 4 : D <= 64 && Dv <= 64 ? 2 : D <= 64 ? 4 : D <= 96 && Dv <= 96 ? 3 : 4;
+}
+
 // Queries per work item of eia_window_flash, 0 where it does not take the shape.
 EIA_API int eia_window_flash_queries(int H, int G, int P, int D, int Dv, int bs) {
   if (G < 1 || H < 1 || H % G || (P != 1 && P != 2) || D < 8 || D % 8 || Dv < 16 || Dv % 16 ||
@@ -525,8 +530,8 @@ EIA_API int eia_window_flash_queries(int H, int G, int P, int D, int Dv, int bs)
 // Prompt portions of window attention without head mixing or slopes; the arguments are those of
 // eia_window_attn_mfma, work holds blocks of eia_window_flash_queries queries.  nparts > 1:
 // row blocks of more than per 64-key tiles are cut into parts of at most that many (nparts * per
-// tiles cover the longest), which meet in part [n_items * H / hpw, nparts, 4 P, 4 ceil(Dv / 32) + 1,
-// 256] fp32, hpw = 128 / queries (Dv counted as 128 where D > 96 or Dv > 96 or D <= 64 < Dv).
+// tiles cover the longest), which meet in part [n_items * H / hpw, nparts, 4 P, 4 eia_window_flash_columns + 1,
+// 256] fp32, hpw = 128 / queries.
 EIA_API int eia_window_flash(const void* q, long ldq, const void* kc, const void* vc, const int* bt,
                              int ldbt, const int* positions, const int* cu, const int* work,
                              int n_items, const float* mult, const void* gate, long ldg, void* out,
@@ -545,12 +550,13 @@ EIA_API int eia_window_flash(const void* q, long ldq, const void* kc, const void
   FlashArgs a{(const bf16_t*)q, ldq, (const bf16_t*)kc, (const bf16_t*)vc, bt, ldbt, positions, cu,
               work, mult, bias, sink, lam, (const bf16_t*)gate, ldg, (bf16_t*)out, ldo, H, G, D, Dv,
               bs, window, keep, gate_heads, WF_ROWS / qb, cap, eps, post, per, nparts, n_items, part};
+  const int cols = eia_window_flash_columns(P, D, Dv);
 #define WF_SIZES(SG)                                                    \
   do {                                                                  \
-    if (D <= 64 && Dv <= 64) wf_go<1, 4, 2, SG>(a, n_items, nparts, st);  \
-    else if (D <= 64) wf_go<1, 4, 4, SG>(a, n_items, nparts, st);         \
-    else if (D <= 96 && Dv <= 96) wf_go<1, 6, 3, SG>(a, n_items, nparts, st); \
-    else wf_go<1, 8, 4, SG>(a, n_items, nparts, st);                      \
+    if (cols == 2) wf_go<1, 4, 2, SG>(a, n_items, nparts, st);          \
+    else if (cols == 3) wf_go<1, 6, 3, SG>(a, n_items, nparts, st);     \
+    else if (D <= 64) wf_go<1, 4, 4, SG>(a, n_items, nparts, st);       \
+    else wf_go<1, 8, 4, SG>(a, n_items, nparts, st);                    \
   } while (0)
   if (P == 2) wf_go<2, 4, 4, false>(a, n_items, nparts, st);
   else if (wmode == 1) WF_SIZES(true);

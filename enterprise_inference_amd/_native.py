@@ -111,6 +111,7 @@ _SIGNATURES = {
     "eia_latent_flash_queries": [I, I, I],
     "eia_latent_flash_keys": [I, I],
     "eia_latent_flash_columns": [I, I],
+    "eia_window_flash_columns": [I, I, I],
     "eia_window_flash": [P, L, P, P, IP, I, IP, IP, IP, I, P, P, L, P, L, I, I, I, I, I, I, I, I, P,
                          F, F, I, P, P, F, I, I, I, P, S],
     "eia_window_flash_queries": [I, I, I, I, I, I],

@@ -165,6 +165,12 @@ def flash_parts(n_items: int, spec: WindowSpec, queries: int, longest: int, cont
                       merge=7 if narrow else 6)
 
 
+def flash_workspace(n_items: int, spec: WindowSpec, queries: int, parts: int) -> int:
+    """Floats of the workspace of a flash prefill launch in ``parts`` parts."""
+    cols = lib().eia_window_flash_columns(spec.maps, spec.dim, spec.vdim)
+    return n_items * (spec.heads * queries // 128) * parts * 4 * spec.maps * (4 * cols + 1) * 256
+
+
 def pair_parts(n_items: int, spec: WindowSpec, queries: int, context: int, cus: int = 256):
     """(parts, 64-key tiles per part) of a flash prefill launch of a differential pair: one workgroup (eight waves) a
     CU, so launches that leave CUs idle are cut until each has one, down to three tiles a part; fewer than 12 tiles
@@ -627,9 +633,7 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
                 NP, per = flash_parts(n_items, spec, qb, max(md.prefill_q_lens or [T]), bt.shape[1] * bs)
             pa = None
             if NP > 1:
-                vt = 4 if max(D, Dv) > 96 or D <= 64 < Dv else -(-max(D, Dv) // 32)
-                pa = torch.empty(n_items * (H * qb // 128) * NP * 4 * P * (4 * vt + 1) * 256,
-                                 dtype=torch.float32, device=q.device)
+                pa = torch.empty(flash_workspace(n_items, spec, qb, NP), dtype=torch.float32, device=q.device)
             check(lib().eia_window_flash(
                 ptr(qa), qa.stride(0), ptr(k_cache), ptr(v_cache), ptr(bt), bt.stride(0),
                 ptr(pos), ptr(cu), ptr(work), n_items, ptr(spec.mult), ptr(g),

@@ -265,7 +265,7 @@ struct WinAttnArgs {
   float cap;                        // > 0: scores soft-capped, cap * tanh(s / cap)
   int talk_post;                    // talk mixes the softmax weights, not the scores (scalar form)
   int gate_heads;                   // gate [rows, H]: one value per head
-  int rows;                         // rows of the launch
+  int rows;                         // rows of a decode launch, those the partials have room for otherwise
 };
 
 // The visible keys of a 16-query tile as absolute 32-key blocks: the blocks of the kept first
@@ -1147,9 +1147,15 @@ template <bool PACKED>
 __global__ void __launch_bounds__(64)
 window_attn_merge_kernel(const WinAttnArgs a) {
   const int H = a.H, P = a.P, Dv = a.Dv, M = H * P, NP = a.nparts;
-  const long row = blockIdx.x;
+  long row = blockIdx.x;
   const int h = blockIdx.y, lane = threadIdx.x;
-  if (row >= a.rows) return;
+  if (a.cu) {                                       // the rows of the tiles, 16 each: no others have partials
+    const int* wk = a.work + 2 * (blockIdx.x >> 4);
+    row = a.cu[wk[0]] + wk[1] + (blockIdx.x & 15);
+    if (row >= a.cu[wk[0] + 1]) return;
+  } else if (row >= a.rows) {
+    return;
+  }
   const int pos = a.positions[row], len = (a.lens ? a.lens : a.positions)[row];
   if (a.lens && len <= 0) return;                   // padding row: the partition kernel wrote zeros
   const int nblocks = wa_blocks(pos, pos, a.window, a.keep).nblocks;
@@ -1334,6 +1340,6 @@ EIA_API int eia_window_attn_mfma(const void* q, long ldq, const void* kc, const 
 #undef WA_LAUNCH
 #undef WA_LAUNCH1
   if (nparts > 1)
-    hipLaunchKernelGGL(window_attn_merge_kernel<false>, dim3(rows, H), dim3(64), 0, st, a);
+    hipLaunchKernelGGL(window_attn_merge_kernel<false>, dim3(cu ? 16 * n_items : rows, H), dim3(64), 0, st, a);
   EIA_LAUNCH_CHECK();
 }

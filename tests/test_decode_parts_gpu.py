@@ -134,7 +134,12 @@ def test_mixed_prefill(new, past, H, G, D, window, keep, parts, monkeypatch):
     def call(dev, t, m):
         spec = WA.WindowSpec(H, G, 1, D, D, window, keep, torch.full((H,), D ** -0.5, device=dev))
         spec.slope, spec.talk, spec.sink = t[4:]
-        return WA.window_attention(t[0], t[1], t[2], m, spec, t[3])
+        y = torch.full((T + 2, H * D), 7.0, dtype=torch.bfloat16, device=dev)      # two rows of no sequence
+        rows = torch.cat([t[0], t[0][:2]])
+        m.positions = torch.cat([m.positions, m.positions[:2]])
+        WA.window_attention(rows, t[1], t[2], m, spec, torch.cat([t[3], t[3][:2]]), out=y)
+        assert dev == "cpu" or bool((y[T:] == 7).all())
+        return y[:T]
 
     ref, out = [], []
     for dev, to in (("cpu", ref), ("cuda", out)):

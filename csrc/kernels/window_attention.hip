@@ -266,7 +266,15 @@ struct WinAttnArgs {
   int talk_post;                    // talk mixes the softmax weights, not the scores (scalar form)
   int gate_heads;                   // gate [rows, H]: one value per head
   int rows;                         // rows of a decode launch, those the partials have room for otherwise
+  unsigned inv_g;                   // decode, grid.x of (row, kv head) pairs in order: 2^32 / G, rounded up; of rows: 0
 };
+
+// Row and kv head of a decode workgroup (x / G is exact: x G < 2^32).
+EIA_DEV void wd_unit(const WinAttnArgs& a, long& row, int& kvh) {
+  const int r = __umulhi(blockIdx.x, a.inv_g);
+  row = a.inv_g ? r : blockIdx.x;
+  kvh = a.inv_g ? blockIdx.x - r * a.G : blockIdx.y;
+}
 
 // The visible keys of a 16-query tile as absolute 32-key blocks: the blocks of the kept first
 // tokens that lie before the window (nsink of them, from block 0), then blocks wb0 .. wb1.
@@ -933,10 +941,12 @@ EIA_DEV void wa_finish_head(const WinAttnArgs& a, long row, int h, int lane, con
 // A CU has about 16 KB of reads in flight, one block of 128 + 128, and moves 30 bytes a ns whatever waves and
 // prefetches ask for (eight or sixteen waves, or the next block in flight, were no faster): so small batches are cut
 // into as many partitions as there are CUs.  The workgroups of a row, and of its merge, share an XCD, row % 8 (the
-// grid is padded to it): the partials then meet in that L2.  (Merged by the last workgroup of a row to arrive,
-// through atomics that pass the L2s, the three rows below took 16.9 us.)  MI355X, window 1024, 8 heads of 128 on 2, both
-// launches: 3 rows 15.7 -> 10.4 us, 17 rows 17.0 -> 12.5, 64 rows 22.4 -> 20.7; 8 rows at 4000 tokens without a window
-// 22.2 -> 12.7.
+// grid is padded to it): the partials then meet in that L2.  Where the CUs of an XCD do not hold its rows' partitions, the
+// (row, kv head) pairs are dealt over the XCDs instead, each with its merge.  (Merged by the last workgroup of a row to arrive,
+// through atomics that pass the L2s, three rows took 16.9 us.)  MI355X, window 1024, 8 heads of 128 on 2, both
+// launches, us, unpadded in powers of two / rows / as it is: 3 rows 14.9 / 9.8 / 9.9, 17 rows 15.5 / 12.2 / 10.8, 64 rows 21.6 /
+// 19.5 / 19.5; without a window, 32 heads on 8, one row at 4000 tokens 22 / 23 / 11, at 32768 48 / 122 / 38, three there
+// 94 / 145 / 75.
 template <int P, int ND, int NDV, bool SIG>
 __global__ void __launch_bounds__(256, 2)
 window_decode_kernel(const WinAttnArgs a) {
@@ -945,8 +955,11 @@ window_decode_kernel(const WinAttnArgs a) {
   __shared__ float sm[4][P][16], sl[4][P][16];
   __shared__ int page_s[WA_PAGES];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, c = lane & 15, g = lane >> 4;
-  const int H = a.H, D = a.D, Dv = a.Dv, M = H * P, rep = H / a.G, bs = a.bs, kvh = blockIdx.y;
-  const long row = blockIdx.x;
+  const int H = a.H, D = a.D, Dv = a.Dv, M = H * P, rep = H / a.G, bs = a.bs;
+  const int z = blockIdx.z;
+  long row;
+  int kvh;
+  wd_unit(a, row, kvh);
   if (row >= a.rows) return;
   const int h0 = kvh * rep;
   bf16_t* out = (bf16_t*)a.out + row * a.ldo + (long)h0 * Dv;
@@ -958,9 +971,9 @@ window_decode_kernel(const WinAttnArgs a) {
   const WaBlocks kbs = wa_blocks(qpos, qpos, a.window, a.keep);
   const int wb0 = kbs.wb0, nsink = kbs.nsink, nblocks = kbs.nblocks;
   const int np = wd_parts(a.nparts, nblocks);
-  if ((int)blockIdx.z >= np) return;                    // (whole workgroup)
+  if (z >= np) return;                                  // (whole workgroup)
   const int per = (nblocks + np - 1) / np;
-  const int b_lo = blockIdx.z * per, b_hi = min(nblocks, b_lo + per);
+  const int b_lo = z * per, b_hi = min(nblocks, b_lo + per);
   const int* bt = a.bt + row * a.ldbt;
   for (int i = tid; i < min(b_hi - b_lo, WA_PAGES); i += 256) {
     const int bb = b_lo + i;
@@ -987,7 +1000,7 @@ window_decode_kernel(const WinAttnArgs a) {
     mult[m] = a.mult[hd * P + m];
     slope[m] = a.slope ? a.slope[hd * P + m] : 0.f;
     bias[m] = (SIG && a.bias) ? a.bias[hd * P + m] : 0.f;
-    const bool snk = !SIG && a.sink && blockIdx.z == 0 && w == 0;
+    const bool snk = !SIG && a.sink && z == 0 && w == 0;
     mrun[m] = snk ? a.sink[hd * P + m] : -1e30f;
     lrun[m] = snk ? 1.f : 0.f;
 #pragma unroll
@@ -1111,17 +1124,17 @@ window_decode_kernel(const WinAttnArgs a) {
     for (int m = 0; m < P; ++m) {
       float mx = sm[0][m][x], ls = 0.f, v0 = 0.f, v1 = 0.f;
 #pragma unroll
-      for (int z = 1; z < 4; ++z) mx = fmaxf(mx, sm[z][m][x]);
+      for (int y = 1; y < 4; ++y) mx = fmaxf(mx, sm[y][m][x]);
 #pragma unroll
-      for (int z = 0; z < 4; ++z) {
-        const float wz = SIG ? 1.f : exp2f((sm[z][m][x] - mx) * LOG2E);
-        const float* p = so + ((z * P + m) * rep + x) * Dv;
-        ls += wz * sl[z][m][x];
-        if (lane < Dv) v0 += wz * p[lane];
-        if (lane + 64 < Dv) v1 += wz * p[lane + 64];
+      for (int y = 0; y < 4; ++y) {
+        const float wy = SIG ? 1.f : exp2f((sm[y][m][x] - mx) * LOG2E);
+        const float* p = so + ((y * P + m) * rep + x) * Dv;
+        ls += wy * sl[y][m][x];
+        if (lane < Dv) v0 += wy * p[lane];
+        if (lane + 64 < Dv) v1 += wy * p[lane + 64];
       }
       if (np > 1) {                                     // window_attn_merge_kernel finishes the row
-        const long pr = (row * M + (h0 + x) * P + m) * a.nparts + blockIdx.z;
+        const long pr = (row * M + (h0 + x) * P + m) * a.nparts + z;
         if (lane == 0) {
           a.part_ml[pr * 2] = mx;
           a.part_ml[pr * 2 + 1] = ls;
@@ -1147,8 +1160,13 @@ template <bool PACKED>
 __global__ void __launch_bounds__(64)
 window_attn_merge_kernel(const WinAttnArgs a) {
   const int H = a.H, P = a.P, Dv = a.Dv, M = H * P, NP = a.nparts;
+  const int lane = threadIdx.x;
   long row = blockIdx.x;
-  const int h = blockIdx.y, lane = threadIdx.x;
+  int h = blockIdx.y;
+  if constexpr (PACKED) {                           // (row, kv head, head of it)
+    wd_unit(a, row, h);
+    h = h * gridDim.z + blockIdx.z;
+  }
   if (a.cu) {                                       // the rows of the tiles, 16 each: no others have partials
     const int* wk = a.work + 2 * (blockIdx.x >> 4);
     row = a.cu[wk[0]] + wk[1] + (blockIdx.x & 15);
@@ -1297,8 +1315,10 @@ EIA_API int eia_window_attn_mfma(const void* q, long ldq, const void* kc, const 
                          block, lds, st, a);                                                    \
   } while (0)
   if (packed) {
-    const int rows8 = nparts > 1 ? (n_items + 7) / 8 * 8 : n_items;      // (a row's workgroups on one XCD)
-    const dim3 dg(rows8, G, nparts), db(256);
+    const int rows8 = (n_items + 7) / 8 * 8, units8 = (n_items * G + 7) / 8 * 8;
+    const bool unit = nparts > 1 && G > 1 && rows8 / 8 * G * nparts > 32;
+    if (unit) a.inv_g = (unsigned)(((1ll << 32) + G - 1) / G);
+    const dim3 db(256), dg = unit ? dim3(units8, 1, nparts) : dim3(nparts > 1 ? rows8 : n_items, G, nparts);
     const size_t dl = sizeof(float) * 4 * P * (H / G) * Dv;
 #define WD_GO(PV, NDX, NDVX, SG)                                                                \
   do {                                                                                          \
@@ -1316,7 +1336,7 @@ EIA_API int eia_window_attn_mfma(const void* q, long ldq, const void* kc, const 
 #undef WD_DIMS
 #undef WD_GO
     if (nparts > 1)
-      hipLaunchKernelGGL(window_attn_merge_kernel<true>, dim3(rows8, H), dim3(64), 0, st, a);
+      hipLaunchKernelGGL(window_attn_merge_kernel<true>, dim3(dg.x, dg.y, H / G), dim3(64), 0, st, a);
     EIA_LAUNCH_CHECK();
   }
   // without head mixing the key width may be half the value width (a differential pair)

@@ -99,10 +99,11 @@ def decode_partitions(batch: int, spec: WindowSpec, cus: int = 256) -> int:
     batch and the layer's constants only, so a captured decode graph keeps its grid.
 
     Without head mixing and up to 16 heads per kv head a workgroup takes one kv head's heads and its
-    four waves share the blocks.  The workgroups of a row share one of the eight XCDs (row % 8), 32 CUs:
-    as many partitions as give each CU one, down to a block per wave, and none for windows below 16 blocks (window
-    1024, 8 heads on 2, 17 rows: 21.3 / 18.4 / 15.8 / 15.2 / 15.7 / 17.9 us in 1 / 2 / 4 / 5 / 6 / 9 partitions, 64 rows
-    23.2 / 21.8 / 23.5 in 1 / 2 / 3; 300 tokens, 17 rows: 10.6 / 12.4 in 1 / 3)."""
+    four waves share the blocks.  The workgroups of a row and kv head share one of the eight XCDs, 32 CUs:
+    as many partitions as give each CU one, four blocks at least, and none for windows below 16 blocks (window
+    1024, 8 heads on 2, 17 rows: 21.3 / 18.4 / 15.8 / 15.2 / 15.7 / 17.9 us in 1 / 2 / 4 / 5 / 6 / 9 partitions with
+    a row's kv heads on one XCD, 10.8 in 6 with each on its own, 64 rows 23.2 / 21.8 / 23.5 in 1 / 2 / 3; 300 tokens,
+    17 rows: 10.6 / 12.4 in 1 / 3)."""
     forced = int(os.environ.get("EIA_WINDOW_DECODE_P", "0"))
     if forced > 0:
         return min(forced, 64)
@@ -112,7 +113,7 @@ def decode_partitions(batch: int, spec: WindowSpec, cus: int = 256) -> int:
             blocks = (spec.window + 31) // 32 + 1 + (spec.keep + 31) // 32
         if blocks < 16:
             return 1
-        return max(1, min(16, blocks // 4, cus // 8 // (spec.kv_heads * -(-max(1, batch) // 8))))
+        return max(1, min(16, blocks // 4, cus // 8 // -(-max(1, batch) * spec.kv_heads // 8)))
     # (sigmoid weights: a wave takes two heads where they share a kv head)
     per_wave = 2 if (spec.weights == 1 and (spec.heads // spec.kv_heads) % 2 == 0) else 1
     wgs = max(1, batch) * (1 if spec.talk is not None else -(-(spec.heads // per_wave) // 4))

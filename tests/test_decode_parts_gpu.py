@@ -95,19 +95,50 @@ def test_latent(H, R, rd, window, lens, parts, monkeypatch):
     assert _rel(got, want) < 8e-3
 
 
+# heads on kv heads, rows: (row, kv head) pairs that do not fill eight XCDs, rows one XCD each does not hold
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,G,rows", [(32, 8, 1), (8, 8, 3), (16, 4, 2), (6, 3, 9), (5, 5, 7), (12, 6, 20), (64, 32, 1), (8, 1, 1)])
+def test_window_units(H, G, rows):
+    g = torch.Generator().manual_seed(H + rows)
+    lens = [1300 - 151 * (i % 8) for i in range(rows)]
+    lens[rows // 2] = 0 if rows > 2 else 700
+    md, pages = _step(lens, g)
+    bf = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16)
+    t = [bf(rows, H * 64), bf(pages, PAGE, G * 64), bf(pages, G * 64, PAGE), torch.randn(H, generator=g)]
+
+    def call(dev, t, m):
+        spec = WA.WindowSpec(H, G, 1, 64, 64, 0, 0, torch.full((H,), 0.125, device=dev))
+        spec.sink = t[3]
+        assert WA.decode_partitions(rows, spec) > 1
+        return WA.window_attention(t[0], t[1], t[2], m, spec)
+
+    want, got = _both(call, t, md, lens)
+    assert _rel(got, want) < 4e-3                       # as in test_window
+
+
+def test_window_partitions():
+    """No more workgroups of an XCD's (row, kv head) pairs than its 32 CUs hold, none for what one workgroup does as fast,
+    and no fewer than powers of two over the whole chip: few rows use every XCD."""
+    spec = lambda w, G=2: WA.WindowSpec(4 * G, G, 1, 128, 128, w, 0, torch.ones(4 * G))
+    assert [WA.decode_partitions(n, spec(1024)) for n in (1, 8, 9, 16, 17, 31, 64, 128)] == [8, 8, 8, 8, 6, 4, 2, 1]
+    assert [WA.decode_partitions(n, spec(0)) for n in (1, 8, 9, 17, 128)] == [16, 16, 10, 6, 1]
+    assert [WA.decode_partitions(3, spec(w)) for w in (300, 448, 449, 512)] == [1, 1, 4, 4]
+    assert [WA.decode_partitions(n, spec(0, 8)) for n in (1, 2, 3, 4, 8)] == [16, 16, 10, 8, 4]
+    for n in range(1, 300):
+        for G in (1, 2, 3, 4, 6, 8, 16, 32):
+            p, q = WA.decode_partitions(n, spec(0, G)), 1
+            assert p == 1 or -(-n * G // 8) * p <= 32
+            while 2 * q <= 16 and n * G * 2 * q <= 256:
+                q *= 2
+            assert p >= q
+
+
 def test_partitions():
     """No more workgroups of an XCD's rows than its 32 CUs hold, none for what one workgroup does as fast."""
-    spec = lambda w, G=2: WA.WindowSpec(8, G, 1, 128, 128, w, 0, torch.ones(8))
-    assert [WA.decode_partitions(n, spec(1024)) for n in (1, 8, 9, 16, 17, 31, 64, 128)] == [8, 8, 8, 8, 5, 4, 2, 1]
-    assert [WA.decode_partitions(n, spec(0)) for n in (1, 8, 9, 17, 128)] == [16, 16, 8, 5, 1]
-    assert [WA.decode_partitions(3, spec(w)) for w in (300, 448, 449, 512)] == [1, 1, 4, 4]
     assert [LA.decode_partitions(n, 16, window=1024) for n in (1, 8, 13, 24, 48, 100, 400)] == [17, 17, 16, 10, 5, 2, 1]
     assert [LA.decode_partitions(n, 8, wide=False) for n in (1, 13, 48, 100)] == [32, 32, 10, 4]
     for n in range(1, 300, 7):
-        rows = -(-n // 8)
-        for G in (1, 2, 4, 8):
-            assert WA.decode_partitions(n, spec(0, G)) == 1 or rows * G * WA.decode_partitions(n, spec(0, G)) <= 32
-        assert LA.decode_partitions(n, 64) == 1 or rows * 4 * LA.decode_partitions(n, 64) <= 32
+        assert LA.decode_partitions(n, 64) == 1 or -(-n // 8) * 4 * LA.decode_partitions(n, 64) <= 32
 
 
 @pytest.mark.gpu

@@ -102,9 +102,15 @@ EIA_API int eia_latent_prep(const void* fused, long ld, int q_off, int q_rank, c
 // ------------------------------------------------------------------------------------- attention
 constexpr int LAT_UNIT = 64;       // keys per tile of the decode form, cut at multiples of it
 
-// Key partitions a decode row uses out of the launch's grid.z: at least one tile each.
-EIA_DEV int lat_parts(int nparts, int kmin, int kmax) {
-  return min(nparts, (kmax - kmin + LAT_UNIT - 1) / LAT_UNIT);
+
+// Tiles of a decode row, and of each of the key partitions that it uses out of the launch's: the fewest that leave the
+// longest one as short; where a tile takes less than its partition's place in the merge (R up to 256), two tiles each beyond
+// 32 partitions (eight rows at 4000 tokens, 256 + 32: 15.7 us in 63, 14.8 in 32).
+struct LatTiles { int n, per; };
+EIA_DEV LatTiles lat_tiles(int nparts, int kmin, int kmax, int R) {
+  const int n = (kmax - kmin + LAT_UNIT - 1) / LAT_UNIT;
+  const int most = R <= 256 && n < 2 * nparts ? min(nparts, 32) : nparts;
+  return {n, (n + most - 1) / most};
 }
 
 #define LAT_ACC_MAX 32     // fp32 accumulators per thread: QB * HB * R <= 256 * LAT_ACC_MAX
@@ -348,7 +354,7 @@ EIA_API int eia_latent_attn(const void* qa, long qa_st, long qa_sh, const void* 
 //
 // Bound by latency: a row's 64-key tiles are a chain of cache loads and two barriers, and the launch
 // lasts as long as the longest partition.  MI355X, 48 rows at up to 4096 tokens, window 1024, 16
-// heads, R 512 + 64: 23.2 + 4.1 us in five partitions; 200 rows at up to 2500 tokens, no window, with
+// heads, R 512 + 64: 23.7 + 4.1 us in five partitions; 200 rows at up to 2500 tokens, no window, with
 // 16 heads 153 -> 134 us and with 64 heads 499 -> 437 us since a tile's page is known before its fetch and
 // its LDS reads are asked for before the first product; R 128 + 32 with 64 heads 120 -> 115 us, R 256 + 64
 // 292 -> 292 us.  (Two tiles of cache loads in flight, in registers: 27 us instead of 24; the reads held in
@@ -367,16 +373,21 @@ latent_decode_kernel(LatentAttnArgs a) {
   __shared__ __align__(16) bf16_t tiles[NB * KT * KS];
   __shared__ __align__(16) float sS[16 * SP];           // the exchanged scores
   __shared__ float2 rot[16 * NK];                       // [rot_dims / 2], rot_dims <= 32 NK
-  const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  int row = blockIdx.x, z = blockIdx.z;
+  if (row >= a.n_work) {                                // beside the rows: the partitions that their own places do not hold
+    const int others = a.nparts - gridDim.z, at = row - a.n_work + (gridDim.x - a.n_work) * z;
+    if (others <= 0) return;
+    row = at / others;
+    z = gridDim.z + at - row * others;
+  }
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int l16 = lane & 15, g4 = lane >> 4;
   if (row >= a.n_work || (a.seq_lens && a.seq_lens[row] <= 0)) return;
   const int qpos = a.positions[row], kmax = qpos + 1;
   const int wlo = a.window > 0 ? max(0, kmax - a.window) : 0, kmin = wlo & ~(KT - 1);
-  const int np = lat_parts(a.nparts, kmin, kmax);
-  if ((int)blockIdx.z >= np) return;                    // (whole workgroup)
-  const int units = (kmax - kmin + KT - 1) / KT;        // (equal parts)
-  const int k_begin = kmin + units * (int)blockIdx.z / np * KT;
-  const int k_end = min(kmax, kmin + units * ((int)blockIdx.z + 1) / np * KT);
+  const LatTiles tl = lat_tiles(a.nparts, kmin, kmax, a.R);
+  if (z * tl.per >= tl.n) return;                       // (whole workgroup)
+  const int k_begin = kmin + z * tl.per * KT, k_end = min(kmax, k_begin + tl.per * KT);
   const int R = a.R, Dk = R + a.rd, bs = a.bs, h0 = blockIdx.y * a.HB, nh = min(a.HB, a.H - h0);
   const bf16_t* cache = static_cast<const bf16_t*>(a.cache);
   const int* bt = a.block_table + (long)row * a.bt_stride;
@@ -541,8 +552,8 @@ latent_decode_kernel(LatentAttnArgs a) {
   }
   if (!ok) return;
   // the lane holds columns c0 + 16 i + 4 g4 .. + 3 of its head (R % 8 == 0)
-  if (np > 1) {
-    const long pr = ((long)row * a.H + h) * a.nparts + blockIdx.z;
+  if (tl.per < tl.n) {
+    const long pr = ((long)row * a.H + h) * a.nparts + z;
 #pragma unroll
     for (int i = 0; i < NCW; ++i) {
       const int c = c0 + 16 * i + 4 * g4;
@@ -574,7 +585,8 @@ latent_decode_kernel(LatentAttnArgs a) {
 // its weight, then the threads sum four latent columns each over the partitions (nparts <= 64).
 // Rows whose context is too short for two partitions were finished by the
 // attention kernel itself.  Bound by latency: the partials of up to eight partitions are asked for together with the
-// weights' inputs (48 rows of 16 heads, R 512, five partitions: 4.8 -> 4.1 us).
+// weights' inputs (48 rows of 16 heads, R 512, five partitions: 4.8 -> 4.1 us), sixteen at a time where there are many more
+// (four at a time: 4000 tokens, 16 heads, one row in 63 partitions, both launches: 28.7 us instead of 19.3).
 constexpr int LM_P = 8;
 __global__ void __launch_bounds__(128)
 latent_merge_kernel(const float* __restrict__ part_acc, const float* __restrict__ part_ml,
@@ -587,8 +599,9 @@ latent_merge_kernel(const float* __restrict__ part_acc, const float* __restrict_
   const int kmax = positions[row] + 1, len = (seq_lens ? seq_lens : positions)[row];
   if (seq_lens && len <= 0) return;
   const int kmin = window > 0 ? max(0, kmax - window) & ~(LAT_UNIT - 1) : 0;
-  const int np = lat_parts(nparts, kmin, kmax);
-  if (np == 1) return;
+  const LatTiles tl = lat_tiles(nparts, kmin, kmax, R);
+  if (tl.per >= tl.n) return;
+  const int np = (tl.n + tl.per - 1) / tl.per;
   const long pr = ((long)row * H + h) * nparts;
   const float mp = lane < np ? part_ml[2 * (pr + lane)] : -INFINITY;
   const float lp = lane < np ? part_ml[2 * (pr + lane) + 1] : 0.f;
@@ -606,16 +619,25 @@ latent_merge_kernel(const float* __restrict__ part_acc, const float* __restrict_
   float f = L > 0.f ? 1.0f / L : 0.f;
   if (gate) f *= 1.0f / (1.0f + expf(-gv));
   f32x4 v = {0.f, 0.f, 0.f, 0.f};
+  int p = 0;
+  auto join = [&](const f32x4& part) {
+    v += part * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wp), p));
+    ++p;
+  };
 #pragma unroll
-  for (int p = 0; p < LM_P; ++p) {
-    const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wp), p));
-    if (p < np) v += x[p] * w;
+  for (int i = 0; i < LM_P; ++i)
+    if (i < np) join(x[i]);
+  while (np - p > LM_P) {
+    f32x4 y[2 * LM_P];
+#pragma unroll
+    for (int i = 0; i < 2 * LM_P; ++i) y[i] = *reinterpret_cast<const f32x4*>(part_acc + (pr + min(p + i, np - 1)) * R + c);
+    const int n = min(2 * LM_P, np - p);
+#pragma unroll
+    for (int i = 0; i < 2 * LM_P; ++i)
+      if (i < n) join(y[i]);
   }
 #pragma unroll 4
-  for (int p = LM_P; p < np; ++p) {
-    const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wp), p));
-    v += *reinterpret_cast<const f32x4*>(part_acc + (pr + p) * R + c) * w;
-  }
+  while (p < np) join(*reinterpret_cast<const f32x4*>(part_acc + (pr + p) * R + c));
   if (4 * (int)threadIdx.x >= R) return;
   bf16x4 o;
 #pragma unroll
@@ -645,9 +667,17 @@ EIA_API int eia_latent_attn_mfma(const void* qa, long qa_st, long qa_sh, const v
                    block_table, bt_stride, seq_lens, nullptr, nullptr, n_items, positions, gate,
                    gate_st, out, out_st, out_sh, scale, H, R, rd, bs, 1, HB, 0, 0, window, sink,
                    rot_half, rot_amp, nparts, part_acc, part_ml};
-  // (a row's workgroups, and its merge's, on one XCD: the partials meet in that L2)
-  const int rows = nparts > 1 ? (n_items + 7) / 8 * 8 : n_items;
-  const dim3 grid(rows, (H + HB - 1) / HB, nparts);
+  // Workgroup b runs on XCD b % 8, and partials that meet on the XCD that wrote them come from its L2: so with partitions
+  // the grid is padded to whole rounds of the XCDs, a row and its merge on one.  Where a row has more partitions than its
+  // share of that XCD's CUs (one workgroup of wide rows each, two of others), the last ones, which only long contexts
+  // use, go to the XCDs with fewer rows, as the workgroups beside the rows there; where these are too few, no row is padded.
+  // us, unpadded / a row on one XCD only / so, R 512 + 64, no window: one row of 16 heads at 1500 tokens 18.8 / 14.6 / 13.8, at
+  // 32768 51 / 64 / 42, of 64 heads at 4000 33 / 34 / 25, at 32768 55 / 193 / 45; 20 rows of 64 heads at 4000 71 / 101 / 73.
+  const int y = (H + HB - 1) / HB, per = (n_items + 7) / 8;
+  const int home = min(nparts, max(1, (Dk <= 288 ? 64 : 32) / y / per));
+  const bool pad = nparts > 1 && (nparts - home) * n_items <= (8 * per - n_items) * home;
+  const int rows = pad ? 8 * per : n_items;
+  const dim3 grid(rows, y, pad ? home : nparts);
 #define LAT_DECODE(NK, NCW) hipLaunchKernelGGL((latent_decode_kernel<NK, NCW>), grid, dim3(256), 0, st, a)
   if (Dk <= 160 && R <= 128) LAT_DECODE(5, 2);
   else if (Dk <= 288 && R <= 256) LAT_DECODE(9, 4);

@@ -54,19 +54,23 @@ def query_block(num_heads: int, kv_rank: int, rot_dim: int = 0,
 def decode_partitions(batch: int, num_heads: int, cus: int = 256, window: int = 0,
                       wide: bool = True) -> int:
     """Key partitions (grid.z) of a decode launch of the MFMA form: a decode row is one workgroup
-    per 16-head slice.  A row's workgroups share one of the eight XCDs (row % 8): its 64-key tiles are
-    split until the CUs of an XCD are taken -- one workgroup per CU with ``wide`` rows (LDS), two
-    otherwise -- at most 32 and no more than the tiles a sliding window can hold; the partials are merged
-    by a second kernel.  Depends on the batch and the layer's constants only, so a captured decode graph
-    keeps its grid.  16 heads, R 512 + 64, window 1024, 13 rows: 36 / 25.4 / 20.2 / 20.2 / 25.0 us in 2 / 4 / 8 /
-    16 / 20 partitions, 48 rows 28.3 / 36.4 in 5 / 6; 8 heads, 256 + 64, 13 rows at 3000 tokens 21.1 / 17.5 / 26.0 in 8 /
-    16 / 20; 16 heads, 256 + 32, 100 rows 29.2 / 26.4 / 32.4 in 2 / 4 / 5."""
+    per 16-head slice: its 64-key tiles are split until the chip's CUs are taken -- one workgroup per CU
+    with ``wide`` rows (LDS), two otherwise -- at most 64 and no more than the tiles a sliding window can hold;
+    the partials are merged by a second kernel.  A row's workgroups share one of the eight XCDs (row % 8) where its CUs
+    hold them; up to a tenth fewer are taken where the launch can then deal the rest to the XCDs with fewer rows.  A row
+    uses as many as its tiles need (decided in the kernel).  Depends on the batch and the layer's constants
+    only, so a captured decode graph keeps its grid.  16 heads, R 512 + 64, window 1024, a row's on one XCD, 13 rows:
+    36 / 25.4 / 20.2 / 20.2 / 25.0 us in 2 / 4 / 8 / 16 / 20 partitions, with the rest dealt out 15.8 in 17; 48 rows 28.3 / 36.4
+    in 5 / 6; no window, one row at 32768 tokens 64 / 42 in 32 / 64."""
     forced = int(os.environ.get("EIA_LATENT_DECODE_P", "0"))
     if forced > 0:
         return min(forced, 64)
-    wgs = -(-max(1, batch) // 8) * ((num_heads + 15) // 16)
-    limit = 32 if window <= 0 else max(1, min(32, (window + 63) // 64 + 1))
-    return max(1, min(limit, (cus if wide else 2 * cus) // 8 // wgs))
+    n = max(1, batch)
+    limit = 64 if window <= 0 else min(64, (window + 63) // 64 + 1)
+    places = (cus if wide else 2 * cus) // 8 // ((num_heads + 15) // 16)     # of an XCD
+    rounds = -(-n // 8)
+    every, placed = 8 * places // n, 8 * rounds * (places // rounds) // n
+    return max(1, min(limit, placed if 10 * placed >= 9 * every else every))
 
 
 def build_work(q_lens: List[int], qblock: int) -> List[int]:

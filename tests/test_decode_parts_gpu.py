@@ -133,12 +133,39 @@ def test_window_partitions():
             assert p >= q
 
 
-def test_partitions():
-    """No more workgroups of an XCD's rows than its 32 CUs hold, none for what one workgroup does as fast."""
-    assert [LA.decode_partitions(n, 16, window=1024) for n in (1, 8, 13, 24, 48, 100, 400)] == [17, 17, 16, 10, 5, 2, 1]
-    assert [LA.decode_partitions(n, 8, wide=False) for n in (1, 13, 48, 100)] == [32, 32, 10, 4]
-    for n in range(1, 300, 7):
-        assert LA.decode_partitions(n, 64) == 1 or -(-n // 8) * 4 * LA.decode_partitions(n, 64) <= 32
+# rows whose partitions an XCD holds, whose last ones go beside the rows of others (1 to 7, 9, 13), or that are not padded
+# (20 of four slices); and contexts that use more partitions than the merge takes at once
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,R,rd,rows,ctx", [(16, 512, 64, 1, 4300), (8, 256, 64, 2, 4300), (16, 256, 64, 5, 3300),
+                                             (64, 512, 64, 3, 1500), (8, 128, 32, 9, 4300), (20, 512, 64, 13, 900),
+                                             (16, 320, 64, 13, 1400), (64, 320, 32, 20, 400), (128, 320, 0, 9, 300)])
+def test_latent_places(H, R, rd, rows, ctx):
+    g = torch.Generator().manual_seed(H + rows)
+    lens = [max(1, ctx - 190 * (i % 8)) for i in range(rows)]
+    if rows > 2:
+        lens[rows // 2] = 0
+    md, pages = _step(lens, g)
+    bf = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16)
+    t = [bf(rows, H, R), bf(rows, H, rd), bf(pages, PAGE, R + rd), bf(rows, H), torch.randn(H, generator=g)]
+
+    def call(dev, t, m):
+        return LA.latent_attention(t[0], t[1], LA.inv_frequencies(rd, 10000.0, dev), rd, t[2], m, t[3], (R + rd) ** -0.5,
+                                   0, t[4])
+
+    want, got = _both(call, t, md, lens)
+    assert _rel(got, want) < 8e-3                       # as in test_latent
+
+
+def test_latent_partitions():
+    """At least nine tenths of the workgroups that the chip's CUs take at once (one each, two of narrow rows), never more."""
+    assert [LA.decode_partitions(n, 16, window=1024) for n in (1, 8, 13, 24, 48, 100, 400)] == [17, 17, 17, 10, 5, 2, 1]
+    assert [LA.decode_partitions(n, 8, wide=False) for n in (1, 13, 48, 100)] == [64, 39, 10, 5]
+    assert [LA.decode_partitions(n, 64) for n in (1, 3, 9, 20, 65)] == [64, 21, 7, 3, 1]
+    for n in range(1, 300):
+        for H in (8, 16, 32, 64, 128):
+            p, wgs = LA.decode_partitions(n, H), n * -(-H // 16)
+            assert p == 1 or wgs * p <= 256
+            assert p == 64 or 10 * p >= 9 * (256 // wgs)
 
 
 @pytest.mark.gpu

@@ -32,11 +32,14 @@ def chunk_rows(nseq: int, heads: int) -> int:
 
 
 def chunk_rows_beside(nseq: int, heads: int) -> int:
-    """Rows from which the shorter sequences of a step go along where the chunk-parallel form is launched for a long
-    one: they then cost a chunk each, but no more tokens after one another.  MI355X, a sequence of 500 rows and so many
+    """Rows from which the shorter sequences of a step go along where a long one takes the chunk-parallel form (the
+    device looks for it where neither ``longest`` nor the average tells): they then cost a chunk each, but no more tokens
+    after one another.  MI355X, a sequence of 500 rows and so many
     shorter ones, token by token / along: 40 heads, 3 of 8 43 / 36 us, 3 of 48 64 / 43, 15 of 8 49 / 63, 15 of 24 59 / 64,
     15 of 48 74 / 67, 63 of 48 147 / 160; 16 heads, 15 of 8 33 / 32, 15 of 24 41 / 34, 63 of 24 55 / 72, 63 of 48 75 / 82;
-    51 to 102 rows, 11 sequences of 40 heads 84 / 54."""
+    51 to 102 rows, 11 sequences of 40 heads 84 / 54.  Where none turns out to be long and the launches were made for
+    nothing, sequences of some 20 rows more use them all the same, token by token / in chunks: 32 heads, 8 of 24 23 / 27, 16
+    of 32 29 / 33, 8 of 50 36 / 32; 16 heads, 16 of 20 21 / 27, 4 of 40 29 / 22, 8 of 50 35 / 24."""
     return max(1, nseq * heads // 20)
 
 
@@ -143,13 +146,18 @@ def wkv_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor,
     if not takes_chunks(T, nseq, split, longest):
         split = 0
     least = min(split, chunk_rows_beside(nseq, heads))
-    if nseq > 1 or not split:
-        check(lib().eia_wkv_scan(*args, heads, D, least, 1 if bf else 0, stream(r)), "wkv_scan")
+    if nseq == 1 and split:
+        split = least = 1                  # (whatever part of the T rows it owns)
+    elif split and max(longest, T // nseq) >= split:
+        split = least                      # a long one is there
+    elif split:
+        split = min(split, least + 20)
+    if split != 1:
+        check(lib().eia_wkv_scan(*args, heads, D, split, least, 1 if bf else 0, stream(r)), "wkv_scan")
     if split:
         n = T // CHUNK + nseq
         U = torch.empty(n, heads, CHUNK_DIM, CHUNK_DIM, dtype=torch.float32, device=r.device)
         L = torch.empty(n, heads, CHUNK_DIM, dtype=torch.float32, device=r.device)
-        # (a single sequence goes here whatever part of the T rows it owns)
-        check(lib().eia_wkv_scan_chunked(*args, T, heads, D, least if nseq > 1 else 1, ptr(U), ptr(L),
+        check(lib().eia_wkv_scan_chunked(*args, T, heads, D, split, least, ptr(U), ptr(L),
                                          1 if bf else 0, stream(r)), "wkv_scan_chunked")
     return y

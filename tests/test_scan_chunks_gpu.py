@@ -69,6 +69,21 @@ def test_wkv_short_sequences_beside_a_long_one(lens, least, monkeypatch):
     assert torch.equal(dev[9].cpu(), args[9])
 
 
+# none of those that might be long is; one of many (more than a wave looks at once) is; the average tells
+@pytest.mark.parametrize("lens", [[20] * 12, [1] * 70 + [120] + [20] * 40, [47, 100, 60], [30, 90]])
+def test_wkv_lengths_not_told(lens):
+    """The same route, and bits, as where the longest sequence's rows are given."""
+    from enterprise_inference_amd.ops import wkv
+    n, T, H, D = len(lens), sum(lens), 2, 64
+    assert wkv.takes_chunks(T, n, wkv.chunk_rows(n, H))
+    cu, pos, slots = _step(lens, [3] * n, False)
+    out = []
+    for longest in (0, max(lens)):
+        dev = [t.to("cuda") for t in _wkv_args(torch.Generator().manual_seed(n), T, n, H, D, torch.float32) + [slots, cu]]
+        out.append((wkv.wkv_scan(*dev, n, pos.to("cuda"), None, 1e-5, H, longest), dev[8], dev[9]))
+    assert all(torch.equal(a, b) for a, b in zip(*out))
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("mode,rot,half", [("exp_gates", 0, True), ("decay", 64, True),
                                            ("decay", 12, False), ("exp_gates", 20, True)])

@@ -258,14 +258,14 @@ struct WinAttnArgs {
   float eps, post;
   int nparts;                       // MFMA form: key partitions over grid.z (1: none; prefill: talk only)
   int raw_bufs;                     // MFMA form with head mixing: raw-score buffers in LDS (1, 2)
-  float* part_acc; float* part_ml;  // [rows, M, nparts, Dv] and [rows, M, nparts, 2] partials
+  float* part_acc; float* part_ml;  // [rows, M, nparts, Dv] and [rows, M, nparts, 2] partials, all rows that cu spans
   int wmode;                        // 0: softmax; 1: sigmoid(score + bias), un-normalised
   const float* bias;                // [M] or null (wmode 1)
   const float* sink;                // [M] or null (wmode 0)
   float cap;                        // > 0: scores soft-capped, cap * tanh(s / cap)
   int talk_post;                    // talk mixes the softmax weights, not the scores (scalar form)
   int gate_heads;                   // gate [rows, H]: one value per head
-  int rows;                         // rows of a decode launch, those the partials have room for otherwise
+  int rows;                         // decode rows
   unsigned inv_g;                   // decode, grid.x of (row, kv head) pairs in order: 2^32 / G, rounded up; of rows: 0
 };
 
@@ -1258,7 +1258,7 @@ EIA_API int eia_window_attn_mfma(const void* q, long ldq, const void* kc, const 
                                  int window, int keep, int epilogue, const float* lam, float eps,
                                  float post, int wmode, const float* bias, int nparts,
                                  float* part_acc, float* part_ml, const float* sink, float cap,
-                                 int gate_heads, int rows, hipStream_t st) {
+                                 int gate_heads, hipStream_t st) {
   if (n_items < 0 || H < 1 || G < 1 || H % G || (P != 1 && P != 2) || bs < 1 || keep < 0 || !q ||
       !kc || !vc || !bt || !positions || !mult || !out)
     return EIA_BAD_SHAPE;
@@ -1269,13 +1269,12 @@ EIA_API int eia_window_attn_mfma(const void* q, long ldq, const void* kc, const 
   if (cap < 0.f) return EIA_BAD_SHAPE;
   if (ldq % 8 || ldo % 4) return EIA_BAD_SHAPE;
   // key partitions: decode rows (a row is its own work item) and head mixing, partials in the workspace
-  if (nparts < 1 || nparts > 64 || (nparts > 1 && ((cu && !talk) || !part_acc || !part_ml)) ||
-      (!cu && rows < n_items))
+  if (nparts < 1 || nparts > 64 || (nparts > 1 && ((cu && !talk) || !part_acc || !part_ml)))
     return EIA_BAD_SHAPE;
   if (n_items == 0) return EIA_OK;
   WinAttnArgs a{q, ldq, kc, vc, bt, ldbt, positions, cu, work, lens, mult, slope, talk, gate, ldg,
                 out, ldo, H, G, P, D, Dv, bs, window, keep, 16, epilogue, lam, eps, post, nparts,
-                2, part_acc, part_ml, wmode, bias, sink, cap, 0, gate_heads, rows};
+                2, part_acc, part_ml, wmode, bias, sink, cap, 0, gate_heads, n_items};
   const bool packed = !cu && !talk && eia_window_decode_packed(H, G);
   // raw-score buffers of the head-mixing form: two (one barrier per block) while they fit 48 KiB
   if (talk) a.raw_bufs = (size_t)2 * H * P * 128 * sizeof(f32x4) > 48 * 1024 ? 1 : 2;
@@ -1360,6 +1359,6 @@ EIA_API int eia_window_attn_mfma(const void* q, long ldq, const void* kc, const 
 #undef WA_LAUNCH
 #undef WA_LAUNCH1
   if (nparts > 1)
-    hipLaunchKernelGGL(window_attn_merge_kernel<false>, dim3(cu ? 16 * n_items : rows, H), dim3(64), 0, st, a);
+    hipLaunchKernelGGL(window_attn_merge_kernel<false>, dim3(cu ? 16 * n_items : n_items, H), dim3(64), 0, st, a);
   EIA_LAUNCH_CHECK();
 }

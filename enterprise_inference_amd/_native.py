@@ -105,7 +105,7 @@ _SIGNATURES = {
     "eia_window_attn": [P, L, P, P, IP, I, IP, IP, IP, IP, I, P, P, P, P, L, P, L, I, I, I, I, I,
                         I, I, I, I, I, P, F, F, I, P, P, F, I, I, I, S],
     "eia_window_attn_mfma": [P, L, P, P, IP, I, IP, IP, IP, IP, I, P, P, P, P, L, P, L, I, I, I, I,
-                             I, I, I, I, I, P, F, F, I, P, I, P, P, P, F, I, I, S],
+                             I, I, I, I, I, P, F, F, I, P, I, P, P, P, F, I, S],
     "eia_latent_flash": [P, L, L, P, L, L, P, I, P, L, IP, I, IP, IP, I, IP, P, L, P, L, L, F, I, I, I,
                          I, I, P, I, F, I, I, P, S],
     "eia_latent_flash_queries": [I, I, I],

@@ -645,12 +645,11 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
                 "window_flash")
             return
         if mfma:
-            rows = n_items if cu is None else T - lo
             NP = (decode_partitions(n_items, spec) if cu is None else
                   mix_parts(n_items, spec, bt.shape[1] * bs))
             pa = pm = None
             if NP > 1:
-                n = rows * H * P * NP
+                n = (n_items if cu is None else T - lo) * H * P * NP
                 ws = torch.empty(n * (Dv + 2), dtype=torch.float32, device=q.device)
                 pa = ws.data_ptr()
                 pm = pa + 4 * n * Dv
@@ -661,7 +660,7 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
                 ptr(o), o.stride(0), H, spec.kv_heads, P, D, Dv, bs, spec.window, spec.keep,
                 spec.epilogue, ptr(spec.lam), float(spec.eps), float(spec.post), spec.weights,
                 ptr(spec.bias), NP, pa, pm, ptr(spec.sink), float(spec.cap),
-                1 if spec.gate_heads else 0, rows, stream(q)), "window_attn_mfma")
+                1 if spec.gate_heads else 0, stream(q)), "window_attn_mfma")
             return
         check(lib().eia_window_attn(
             ptr(qa), qa.stride(0), ptr(k_cache), ptr(v_cache), ptr(bt), bt.stride(0),

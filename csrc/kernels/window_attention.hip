@@ -294,7 +294,8 @@ EIA_DEV float wa_softcap(float s, float cap, float icap2) {
 // so short contexts use few partitions whatever the launch's grid.z (the same on both sides of
 // the merge).
 EIA_DEV int wa_parts(int nparts, int nblocks) { return min(nparts, max(1, nblocks >> 1)); }
-// (of window_decode_kernel: a block for each of its four waves; below 16 blocks the merge costs what it gains)
+// (of window_decode_kernel: four blocks at least, one for each of its waves -- five where the blocks are not a multiple of
+// the partitions, as the 33 of a window of 1024 in 8; below 16 blocks the merge costs what it gains)
 EIA_DEV int wd_parts(int nparts, int nblocks) { return nblocks < 16 ? 1 : min(nparts, nblocks >> 2); }
 
 constexpr int WA_KT = 64;           // keys per tile = lanes of a wave

@@ -158,8 +158,6 @@ def flash_parts(n_items: int, spec: WindowSpec, queries: int, longest: int, cont
     tiles = -(-context // 64)
     if spec.window > 0:
         tiles = min(tiles, (spec.window + queries + 62) // 64 + 1 + (spec.keep + 63) // 64)
-    if spec.maps == 2:                                   # (cut by pair_parts)
-        return 1, tiles
     narrow = max(spec.dim, spec.vdim) <= 64
     return split_keys(n_items * (spec.heads * queries // 128), tiles,
                       tiles if spec.window > 0 else tiles - longest // 128, (3 if narrow else 2) * cus,

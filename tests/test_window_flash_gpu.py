@@ -81,8 +81,9 @@ def test_window_flash(window, new, past, H, G, D, Dv, bs, kind):
             qb = wa.query_block(spec, bf, bs)
             assert qb == 128 // {1: 1, 2: 2, 3: 1, 4: 4}[H // G]
             n = sum(-(-a // qb) for a in new)           # (the long context is cut into parts)
-            assert (wa.flash_parts(n, spec, qb, max(new), bt.shape[1] * bs)[0] > 1) == (
-                max(past) > 900 and P == 1)
+            parts = (wa.pair_parts(n, spec, qb, bt.shape[1] * bs) if P == 2 else
+                     wa.flash_parts(n, spec, qb, max(new), bt.shape[1] * bs))
+            assert (parts[0] > 1) == (max(past) > 900)
         return wa.window_attention(q.to(dev), k.to(dev), v.to(dev), md, spec,
                                    None if gate is None else gate.to(dev)).cpu()
 

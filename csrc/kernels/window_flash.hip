@@ -56,12 +56,12 @@ struct WfRows {
   // from key lo on
   int lo, nkeep, ntile;
 };
-EIA_DEV WfRows wf_rows(const FlashArgs& a, int w, int r32) {
+template <bool SPLIT> EIA_DEV WfRows wf_rows(const FlashArgs& a, int w, int r32) {
   WfRows r;
-  const int item = min((int)blockIdx.y, a.items - 1);
+  const int item = SPLIT ? min((int)blockIdx.y, a.items - 1) : blockIdx.y;         // (with parts the grid is padded)
   r.s = a.work[2 * item];
   const int q0 = a.work[2 * item + 1], qbeg = a.cu[r.s], qlen = a.cu[r.s + 1] - qbeg;
-  r.qn = item == (int)blockIdx.y ? min(WF_ROWS / a.hpw, qlen - q0) : 0;      // (the grid is padded)
+  r.qn = !SPLIT || item == (int)blockIdx.y ? min(WF_ROWS / a.hpw, qlen - q0) : 0;
   r.h = blockIdx.x * a.hpw + w % a.hpw;
   if (r.qn <= 0) return r;
   const int wq0 = q0 + 32 * (w / a.hpw);
@@ -159,7 +159,7 @@ window_flash_kernel(FlashArgs a) {
   static_assert(P == 1 || sizeof(wf_lds) >= 4 * 4 * 64 * 16 * NDV, "room to hand rows over");
   const int tid = threadIdx.x, lane = tid & 63, grp = tid >> 8, w = (tid >> 6) & 3;
   const int r32 = lane & 31, hh = lane >> 5, map = P == 2 ? grp : 0;
-  const WfRows rw = wf_rows(a, w, r32);
+  const WfRows rw = wf_rows<SPLIT>(a, w, r32);
   if (rw.qn <= 0) return;                               // (whole workgroup)
   const int D = a.D, Dv = a.Dv, bs = a.bs, kvh = blockIdx.x * a.hpw / (a.H / a.G), h = rw.h;
   const long row = rw.row;
@@ -436,7 +436,7 @@ template <int NDV, bool SIG>
 __global__ void __launch_bounds__(256)
 window_flash_merge_kernel(FlashArgs a) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, dt = blockIdx.z;
-  const WfRows rw = wf_rows(a, w, lane & 31);
+  const WfRows rw = wf_rows<true>(a, w, lane & 31);
   const int parts = min(a.nparts, (rw.ntile + a.per - 1) / a.per);
   if (rw.qn <= 0 || parts <= 1 || !rw.live) return;
   float m = -INFINITY, lsum = 0.f;
@@ -456,7 +456,7 @@ __global__ void __launch_bounds__(128 * NDV)
 window_flash_merge_pair_kernel(FlashArgs a) {
   __shared__ float other[NDV][16][64], sq[NDV][64];
   const int lane = threadIdx.x & 63, dt = (threadIdx.x >> 6) % NDV, map = threadIdx.x / (64 * NDV), w = blockIdx.z;
-  const WfRows rw = wf_rows(a, w, lane & 31);
+  const WfRows rw = wf_rows<true>(a, w, lane & 31);
   const int parts = min(a.nparts, (rw.ntile + a.per - 1) / a.per);
   if (rw.qn <= 0 || parts <= 1 || !rw.live) return;     // (whole workgroup)
   float m = -INFINITY, lsum = 0.f, ss = 0.f;

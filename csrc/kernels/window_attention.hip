@@ -581,7 +581,7 @@ window_attn_mfma_kernel(const WinAttnArgs a) {
   const int pos_first = a.positions[row0], pos_last = a.positions[row0 + nq - 1];
   const WaBlocks kbs = wa_blocks(pos_first, pos_last, a.window, a.keep);
   const int wb0 = kbs.wb0, nsink = kbs.nsink, nblocks = kbs.nblocks;
-  const int np = a.cu ? a.nparts : wa_parts(a.nparts, nblocks);
+  const int np = a.nparts == 1 ? 1 : a.cu ? a.nparts : wa_parts(a.nparts, nblocks);
   if ((int)blockIdx.z >= np) return;                                // (whole workgroup)
 
   // Q^T operands of this wave's maps: column = query c, rows = d 32 s + 8 g .. + 8
@@ -620,7 +620,7 @@ window_attn_mfma_kernel(const WinAttnArgs a) {
 
   // with key partitions (small batches) this workgroup takes a slice of the blocks; a prefill tile always has
   // nparts of them, the last ones possibly empty, as its rows' merge does not know the tile
-  const int per = (nblocks + np - 1) / np;
+  const int per = a.nparts == 1 ? nblocks : (nblocks + np - 1) / np;
   const int b_lo = blockIdx.z * per, b_hi = min(nblocks, b_lo + per);
   // the pages of this workgroup's blocks, looked up once (the block loop then has no dependent
   // global load in front of its operand addresses); blocks past the table's size look up directly

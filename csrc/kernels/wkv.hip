@@ -72,17 +72,8 @@ struct WkvArgs {
   const int* slots; const int* cu; const int* positions; const int* seq_lens;
   void* y; long ldy;                        // [rows, H*D]
   float eps; int H, D;
-  // Rows from which a sequence takes the chunk-parallel form (0: never), and from which it goes along where another one does.
-  int split, least, nseq;
+  int split;                                // rows from which a sequence takes the chunk-parallel form (0: never)
 };
-
-// Whether a sequence of so many rows takes the chunk-parallel form.
-EIA_DEV bool wkv_in_chunks(const WkvArgs& a, int rows) {
-  if (rows >= a.split || rows < a.least) return rows >= a.split;
-  bool any = false;
-  for (int s = threadIdx.x & 63; s < a.nseq; s += 64) any |= a.cu[s + 1] - a.cu[s] >= a.split;
-  return __any(any);
-}
 
 // One workgroup per (sequence, head), 4 x max(64, DMAX) threads: thread (q, j) owns rows
 // [q DMAX/4, (q+1) DMAX/4) of column j of S in registers and walks the sequence's tokens in
@@ -106,7 +97,7 @@ wkv_scan_kernel(WkvArgs a) {
   const int slot = a.slots[s];
   if (slot < 0 || (a.seq_lens && a.seq_lens[s] <= 0)) return;
   const int lo = a.cu ? a.cu[s] : s, hi = a.cu ? a.cu[s + 1] : s + 1;
-  if (hi <= lo || (SPLIT && wkv_in_chunks(a, hi - lo))) return;
+  if (hi <= lo || (SPLIT && hi - lo >= a.split)) return;
   const bool fresh = a.positions[lo] == 0;
   const bool live = j < D, mine = j < DMAX;
   float* Sg = a.S + ((long)slot * a.H + h) * D * D;
@@ -197,20 +188,18 @@ wkv_scan_kernel(WkvArgs a) {
   }
 }
 
-// split > 0: sequences of that many rows or more are left out (eia_wkv_scan_chunked takes them), and with one of them those
-// of least rows or more.
+// split > 0: sequences of that many rows or more are left out (eia_wkv_scan_chunked takes them).
 EIA_API int eia_wkv_scan(const void* r, const void* k, const void* v, const void* g, long ld,
                          const float* dec, long ld_dec, const void* w0, const void* u,
                          const void* norm_w, float* S, float* prev, const float* x, int W,
                          const int* slots, const int* cu, const int* positions,
                          const int* seq_lens, void* y, long ldy, float eps, int nseq, int H, int D,
-                         int split, int least, int is_bf16, hipStream_t st) {
-  if (nseq < 0 || H < 1 || D < 1 || W < 1 || split < 0 || (split && (!cu || least < 1 || least > split)))
-    return EIA_BAD_SHAPE;
+                         int split, int is_bf16, hipStream_t st) {
+  if (nseq < 0 || H < 1 || D < 1 || W < 1 || split < 0) return EIA_BAD_SHAPE;
   if (D > 256) return EIA_UNSUPPORTED;
   if (nseq == 0) return EIA_OK;
   WkvArgs a{r, k, v, g, ld, dec, ld_dec, w0, u, norm_w, S, prev, x, W, slots, cu, positions,
-            seq_lens, y, ldy, eps, H, D, split, least, nseq};
+            seq_lens, y, ldy, eps, H, D, split};
   dim3 grid(nseq, H);
 #define WKV_LAUNCH(TT, DM)                                                                 \
   do {                                                                                     \
@@ -267,8 +256,8 @@ struct WkvChunkArgs {
 
 // The chunk of number x; false where there is none or the sequence is skipped.
 EIA_DEV bool wkv_chunk(const WkvArgs& a, int nseq, int x, int& s, int& row0, int& n) {
-  return chunk_of<WC>(a.cu, nseq, x, s, row0, n) && wkv_in_chunks(a, a.cu[s + 1] - a.cu[s]) &&
-         a.slots[s] >= 0 && (!a.seq_lens || a.seq_lens[s] > 0);
+  return chunk_of<WC>(a.cu, nseq, x, s, row0, n) && a.cu[s + 1] - a.cu[s] >= a.split && a.slots[s] >= 0 &&
+         (!a.seq_lens || a.seq_lens[s] > 0);
 }
 
 // A chunk's [WC][WD] tile of r, k or v on its way to LDS, zero past the chunk and past D: requested
@@ -390,7 +379,7 @@ wkv_chunk_scan_kernel(WkvArgs a, WkvChunkArgs c) {
   const int s = chunk_number(), h = blockIdx.x % a.H;
   if (s >= c.nseq) return;
   const int slot = a.slots[s], lo = a.cu[s], hi = a.cu[s + 1];
-  if (slot < 0 || !wkv_in_chunks(a, hi - lo) || (a.seq_lens && a.seq_lens[s] <= 0)) return;
+  if (slot < 0 || hi - lo < a.split || (a.seq_lens && a.seq_lens[s] <= 0)) return;
   const int e = 4 * (blockIdx.x / a.H * 256 + threadIdx.x), i = e / WD, j = e % WD, D = a.D;
   const long x0 = lo / WC + s;
   const int nc = (hi - lo + WC - 1) / WC;
@@ -603,21 +592,21 @@ static void wkv_chunked(const WkvArgs& a, const WkvChunkArgs& c, int rows, hipSt
   hipLaunchKernelGGL((wkv_chunk_out_kernel<T, VEC>), gc, dim3(256), 0, st, a, c);
 }
 
-// As eia_wkv_scan for D <= 64 with cu given, for the sequences that it leaves out; rows: cu[nseq] at most; workspaces U
+// As eia_wkv_scan for D <= 64 with cu given, for the sequences of split rows or more; rows: cu[nseq] at most; workspaces U
 // [rows / 64 + nseq, H, 64, 64] and L [rows / 64 + nseq, H, 64] fp32.
 EIA_API int eia_wkv_scan_chunked(const void* r, const void* k, const void* v, const void* g,
                                  long ld, const float* dec, long ld_dec, const void* w0,
                                  const void* u, const void* norm_w, float* S, float* prev,
                                  const float* x, int W, const int* slots, const int* cu,
                                  const int* positions, const int* seq_lens, void* y, long ldy,
-                                 float eps, int nseq, int rows, int H, int D, int split,
-                                 int least, float* U, float* L, int is_bf16, hipStream_t st) {
-  if (nseq < 0 || rows < 0 || H < 1 || D < 1 || W < 1 || least < 1 || least > split || !cu || !U || !L)
+                                 float eps, int nseq, int rows, int H, int D, int split, float* U,
+                                 float* L, int is_bf16, hipStream_t st) {
+  if (nseq < 0 || rows < 0 || H < 1 || D < 1 || W < 1 || split < 1 || !cu || !U || !L)
     return EIA_BAD_SHAPE;
   if (D > WD || H > 65535) return EIA_UNSUPPORTED;
   if (nseq == 0 || rows == 0) return EIA_OK;
   WkvArgs a{r, k, v, g, ld, dec, ld_dec, w0, u, norm_w, S, prev, x, W, slots, cu, positions,
-            seq_lens, y, ldy, eps, H, D, split, least, nseq};
+            seq_lens, y, ldy, eps, H, D, split};
   const int es = is_bf16 ? 2 : 4;
   const uintptr_t io = (uintptr_t)g | (uintptr_t)y | (uintptr_t)norm_w | (uintptr_t)(ld * es) | (uintptr_t)(ldy * es);
   WkvChunkArgs c{U, L, nseq, D == WD && io % (4 * es) == 0};

@@ -74,9 +74,9 @@ _SIGNATURES = {
                              I, I, I, P, I, F, I, P, P, S],
     "eia_token_shift_mix": [P, P, I, P, IP, IP, I, IP, P, L, I, I, I, S],
     "eia_wkv_scan": [P, P, P, P, L, P, L, P, P, P, P, P, P, I, IP, IP, IP, IP, P, L, F, I, I, I,
-                     I, I, I, S],
+                     I, I, S],
     "eia_wkv_scan_chunked": [P, P, P, P, L, P, L, P, P, P, P, P, P, I, IP, IP, IP, IP, P, L, F, I,
-                             I, I, I, I, I, P, P, I, S],
+                             I, I, I, I, P, P, I, S],
     "eia_moe_route_grouped": [P, L, P, I, I, I, I, I, I, F, P, P, IP, I, I, I, I, P, I, P, P, P, S],
     "eia_linear_scan": [P, L, I, I, I, I, I, I, P, P, I, I, F, F, F, F, P, P, P, P, IP, IP, IP, IP,
                         P, L, F, I, I, I, I, I, I, I, I, P, P, F, I, I, S],

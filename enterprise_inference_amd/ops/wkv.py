@@ -26,20 +26,17 @@ def chunk_rows(nseq: int, heads: int) -> int:
     """Rows from which a sequence takes the chunk-parallel form.  The token-by-token kernel costs
     0.5 us a token whatever the batch, until its workgroups share CUs; the other form about 23 us
     for its launches and then work per chunk: 1.7 us per sequence at 32 heads, so that a step of
-    many sequences needs longer ones.  MI355X, 32 heads, token by token / chunks: 1 x 32 rows 20 /
-    24 us, 1 x 64 35 / 24, 16 x 32 25 / 51, 64 x 8 29 / 141, 1 x 4096 2091 / 112."""
+    many sequences needs longer ones.  MI355X, 32 heads, token by token / chunks: 1 x 32 rows 21 /
+    20 us, 1 x 64 35 / 22, 16 x 32 25 / 36, 64 x 8 29 / 95, 1 x 4096 2091 / 100."""
     return 48 + min(64, nseq * heads // 32)
 
 
 def chunk_rows_beside(nseq: int, heads: int) -> int:
-    """Rows from which the shorter sequences of a step go along where a long one takes the chunk-parallel form (the
-    device looks for it where neither ``longest`` nor the average tells): they then cost a chunk each, but no more tokens
-    after one another.  MI355X, a sequence of 500 rows and so many
+    """Rows from which the shorter sequences of a step go along where the chunk-parallel form is launched for a long
+    one: they then cost a chunk each, but no more tokens after one another.  MI355X, a sequence of 500 rows and so many
     shorter ones, token by token / along: 40 heads, 3 of 8 43 / 36 us, 3 of 48 64 / 43, 15 of 8 49 / 63, 15 of 24 59 / 64,
     15 of 48 74 / 67, 63 of 48 147 / 160; 16 heads, 15 of 8 33 / 32, 15 of 24 41 / 34, 63 of 24 55 / 72, 63 of 48 75 / 82;
-    51 to 102 rows, 11 sequences of 40 heads 84 / 54.  Where none turns out to be long and the launches were made for
-    nothing, sequences of some 20 rows more use them all the same, token by token / in chunks: 32 heads, 8 of 24 23 / 27, 16
-    of 32 29 / 33, 8 of 50 36 / 32; 16 heads, 16 of 20 21 / 27, 4 of 40 29 / 22, 8 of 50 35 / 24."""
+    51 to 102 rows, 11 sequences of 40 heads 84 / 54."""
     return max(1, nseq * heads // 20)
 
 
@@ -54,6 +51,21 @@ def takes_chunks(rows: int, nseq: int, split: int, longest: int = 0) -> bool:
     if split <= 0 or longest:
         return 0 < split <= longest
     return rows - nseq + 1 >= split and (rows >= 24 * nseq or rows - nseq >= 160)
+
+
+def chunk_split(rows: int, nseq: int, heads: int, longest: int = 0) -> int:
+    """Rows from which the sequences of a step take the chunk-parallel form, 0: it is not launched.  Shorter ones go
+    along beside a long one.  Where the ``longest`` sequence's rows are not given there may be none, and the launches were
+    made for nothing: then they do if the average is some 20 rows above what goes along.  MI355X, token by token (with
+    those launches 5 to 6 us more) / in chunks: 32 heads, 8 of 24 18 / 28 us, 16 of 32 25 / 36, 8 of 50 31 / 32; 16 heads, 16 of
+    20 16 / 28, 16 of 20 to 40 27 / 33, 8 of 50 30 / 24.  (The device could look for a long one: 1 us in each such step.)"""
+    split = chunk_rows(nseq, heads)
+    if not takes_chunks(rows, nseq, split, longest):
+        return 0
+    if nseq == 1:
+        return 1                           # (whatever part of the rows it owns)
+    least = min(split, chunk_rows_beside(nseq, heads))
+    return least if longest or rows // nseq >= min(split, least + 20) else split
 
 
 def _seq_bounds(cu: Optional[torch.Tensor], nseq: int):
@@ -142,22 +154,13 @@ def wkv_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor,
     args = (ptr(r), ptr(k), ptr(v), ptr(g), ld, ptr(dec), dec.stride(0), ptr(w0), ptr(u),
             ptr(norm_w), ptr(S), ptr(prev_state), ptr(x), x.shape[1], ptr(slots), ptr(cu),
             ptr(positions), ptr(seq_lens), ptr(y), y.stride(0), float(eps), nseq)
-    split = chunk_rows(nseq, heads) if cu is not None and D <= CHUNK_DIM else 0
-    if not takes_chunks(T, nseq, split, longest):
-        split = 0
-    least = min(split, chunk_rows_beside(nseq, heads))
-    if nseq == 1 and split:
-        split = least = 1                  # (whatever part of the T rows it owns)
-    elif split and max(longest, T // nseq) >= split:
-        split = least                      # a long one is there
-    elif split:
-        split = min(split, least + 20)
+    split = chunk_split(T, nseq, heads, longest) if cu is not None and D <= CHUNK_DIM else 0
     if split != 1:
-        check(lib().eia_wkv_scan(*args, heads, D, split, least, 1 if bf else 0, stream(r)), "wkv_scan")
+        check(lib().eia_wkv_scan(*args, heads, D, split, 1 if bf else 0, stream(r)), "wkv_scan")
     if split:
         n = T // CHUNK + nseq
         U = torch.empty(n, heads, CHUNK_DIM, CHUNK_DIM, dtype=torch.float32, device=r.device)
         L = torch.empty(n, heads, CHUNK_DIM, dtype=torch.float32, device=r.device)
-        check(lib().eia_wkv_scan_chunked(*args, T, heads, D, split, least, ptr(U), ptr(L),
+        check(lib().eia_wkv_scan_chunked(*args, T, heads, D, split, ptr(U), ptr(L),
                                          1 if bf else 0, stream(r)), "wkv_scan_chunked")
     return y

@@ -69,19 +69,22 @@ def test_wkv_short_sequences_beside_a_long_one(lens, least, monkeypatch):
     assert torch.equal(dev[9].cpu(), args[9])
 
 
-# none of those that might be long is; one of many (more than a wave looks at once) is; the average tells
-@pytest.mark.parametrize("lens", [[20] * 12, [1] * 70 + [120] + [20] * 40, [47, 100, 60], [30, 90]])
+# none of those that might be long is; one of many is; the average tells
+@pytest.mark.parametrize("lens", [[20] * 12, [1] * 70 + [120] + [20] * 40, [28, 31, 52, 54, 19], [47, 100, 60], [30, 90]])
 def test_wkv_lengths_not_told(lens):
-    """The same route, and bits, as where the longest sequence's rows are given."""
+    """The same where the longest sequence's rows are not given."""
     from enterprise_inference_amd.ops import wkv
     n, T, H, D = len(lens), sum(lens), 2, 64
-    assert wkv.takes_chunks(T, n, wkv.chunk_rows(n, H))
+    assert wkv.chunk_split(T, n, H) > 0
     cu, pos, slots = _step(lens, [3] * n, False)
+    args = _wkv_args(torch.Generator().manual_seed(n), T, n, H, D, torch.float32) + [slots, cu]
     out = []
     for longest in (0, max(lens)):
-        dev = [t.to("cuda") for t in _wkv_args(torch.Generator().manual_seed(n), T, n, H, D, torch.float32) + [slots, cu]]
+        dev = [t.to("cuda") for t in args]
         out.append((wkv.wkv_scan(*dev, n, pos.to("cuda"), None, 1e-5, H, longest), dev[8], dev[9]))
-    assert all(torch.equal(a, b) for a, b in zip(*out))
+    (y, S, prev), (y1, S1, prev1) = out
+    # fp32 sums over at most 64 products and a few exponentials
+    assert _rel(y, y1) < 1e-5 and _rel(S, S1) < 2e-6 and torch.equal(prev, prev1)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])

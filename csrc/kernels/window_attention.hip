@@ -269,11 +269,11 @@ struct WinAttnArgs {
   unsigned inv_g;                   // decode, grid.x of (row, kv head) pairs in order: 2^32 / G, rounded up; of rows: 0
 };
 
-// Row and kv head of a decode workgroup (x / G is exact: x G < 2^32).
-EIA_DEV void wd_unit(const WinAttnArgs& a, long& row, int& kvh) {
+// Row and kv head of a decode workgroup; pairs: blockIdx.x counts (row, kv head) (x / G is exact: x G < 2^32).
+EIA_DEV void wd_unit(const WinAttnArgs& a, bool pairs, long& row, int& kvh) {
   const int r = __umulhi(blockIdx.x, a.inv_g);
-  row = a.inv_g ? r : blockIdx.x;
-  kvh = a.inv_g ? blockIdx.x - r * a.G : blockIdx.y;
+  row = pairs ? r : blockIdx.x;
+  kvh = pairs ? blockIdx.x - r * a.G : blockIdx.y;
 }
 
 // The visible keys of a 16-query tile as absolute 32-key blocks: the blocks of the kept first
@@ -942,13 +942,15 @@ EIA_DEV void wa_finish_head(const WinAttnArgs& a, long row, int h, int lane, con
 // A CU has about 16 KB of reads in flight, one block of 128 + 128, and moves 30 bytes a ns whatever waves and
 // prefetches ask for (eight or sixteen waves, or the next block in flight, were no faster): so small batches are cut
 // into as many partitions as there are CUs.  The workgroups of a row, and of its merge, share an XCD, row % 8 (the
-// grid is padded to it): the partials then meet in that L2.  Where the CUs of an XCD do not hold its rows' partitions, the
-// (row, kv head) pairs are dealt over the XCDs instead, each with its merge.  (Merged by the last workgroup of a row to arrive,
+// grid is padded to it): the partials then meet in that L2.  Where the CUs of an XCD do not hold its rows' partitions, or
+// without a window the rows leave XCDs unevenly loaded, the (row, kv head) pairs are dealt over the XCDs instead, each with its
+// merge (rows / pairs, us: 32 heads on 8, 13 rows at 4096 tokens 42.5 / 37.8, at 600 15.3 / 14.5; 16 on 4, 25 rows at 600
+// 14.5 / 15.1; 8 on 2, window 1024, 3 rows 9.7 / 10.0).  (Merged by the last workgroup of a row to arrive,
 // through atomics that pass the L2s, three rows took 16.9 us.)  MI355X, window 1024, 8 heads of 128 on 2, both
 // launches, us, unpadded in powers of two / rows / as it is: 3 rows 14.9 / 9.8 / 9.9, 17 rows 15.5 / 12.2 / 10.8, 64 rows 21.6 /
 // 19.5 / 19.5; without a window, 32 heads on 8, one row at 4000 tokens 22 / 23 / 11, at 32768 48 / 122 / 38, three there
 // 94 / 145 / 75.
-template <int P, int ND, int NDV, bool SIG>
+template <int P, int ND, int NDV, bool SIG, bool PAIRS>
 __global__ void __launch_bounds__(256, 2)
 window_decode_kernel(const WinAttnArgs a) {
   constexpr float LOG2E = 1.4426950408889634f;
@@ -960,7 +962,7 @@ window_decode_kernel(const WinAttnArgs a) {
   const int z = blockIdx.z;
   long row;
   int kvh;
-  wd_unit(a, row, kvh);
+  wd_unit(a, PAIRS, row, kvh);
   if (row >= a.rows) return;
   const int h0 = kvh * rep;
   bf16_t* out = (bf16_t*)a.out + row * a.ldo + (long)h0 * Dv;
@@ -1165,7 +1167,7 @@ window_attn_merge_kernel(const WinAttnArgs a) {
   long row = blockIdx.x;
   int h = blockIdx.y;
   if constexpr (PACKED) {                           // (row, kv head, head of it)
-    wd_unit(a, row, h);
+    wd_unit(a, a.inv_g != 0, row, h);
     h = h * gridDim.z + blockIdx.z;
   }
   if (a.cu) {                                       // the rows of the tiles, 16 each: no others have partials
@@ -1316,17 +1318,21 @@ EIA_API int eia_window_attn_mfma(const void* q, long ldq, const void* kc, const 
   } while (0)
   if (packed) {
     const int rows8 = (n_items + 7) / 8 * 8, units8 = (n_items * G + 7) / 8 * 8;
-    const bool unit = nparts > 1 && G > 1 && rows8 / 8 * G * nparts > 32;
+    const bool unit = nparts > 1 && G > 1 && rows8 * G > units8 && (window <= 0 || rows8 / 8 * G * nparts > 32);
     if (unit) a.inv_g = (unsigned)(((1ll << 32) + G - 1) / G);
     const dim3 db(256), dg = unit ? dim3(units8, 1, nparts) : dim3(nparts > 1 ? rows8 : n_items, G, nparts);
     const size_t dl = sizeof(float) * 4 * P * (H / G) * Dv;
-#define WD_GO(PV, NDX, NDVX, SG)                                                                \
+#define WD_GO1(PV, NDX, NDVX, SG, PR)                                                           \
   do {                                                                                          \
     if (dl > 48 * 1024)                                                                         \
       (void)hipFuncSetAttribute(                                                                \
-          reinterpret_cast<const void*>(&window_decode_kernel<PV, NDX, NDVX, SG>),              \
+          reinterpret_cast<const void*>(&window_decode_kernel<PV, NDX, NDVX, SG, PR>),          \
           hipFuncAttributeMaxDynamicSharedMemorySize, (int)dl);                                 \
-    hipLaunchKernelGGL((window_decode_kernel<PV, NDX, NDVX, SG>), dg, db, dl, st, a);           \
+    hipLaunchKernelGGL((window_decode_kernel<PV, NDX, NDVX, SG, PR>), dg, db, dl, st, a);       \
+  } while (0)
+#define WD_GO(PV, NDX, NDVX, SG)                                                                \
+  do {                                                                                          \
+    if (unit) WD_GO1(PV, NDX, NDVX, SG, true); else WD_GO1(PV, NDX, NDVX, SG, false);           \
   } while (0)
 #define WD_DIMS(PV, SG)                                                                         \
   do {                                                                                          \
@@ -1335,6 +1341,7 @@ EIA_API int eia_window_attn_mfma(const void* q, long ldq, const void* kc, const 
     if (P == 2) WD_DIMS(2, false); else if (wmode == 1) WD_DIMS(1, true); else WD_DIMS(1, false);
 #undef WD_DIMS
 #undef WD_GO
+#undef WD_GO1
     if (nparts > 1)
       hipLaunchKernelGGL(window_attn_merge_kernel<true>, dim3(dg.x, dg.y, H / G), dim3(64), 0, st, a);
     EIA_LAUNCH_CHECK();

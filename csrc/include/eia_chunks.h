@@ -24,7 +24,8 @@ EIA_DEV bool chunk_of(const int* cu, int nseq, int x, int& s, int& row0, int& n)
 // part of each come in whole; and where eight divides the heads, a head's state stays in the L2 of one XCD between
 // the passes (workgroup b runs on XCD b % 8; a grid of a workgroup per sequence takes parts x heads as its heads).
 // wkv, two prompts of 571 tokens, 32 heads: 47 -> 39 us, eleven of 196, 16 heads: 44 -> 41, sixteen of 433, 40 heads:
-// 178 -> 173, one of 4096: 107.4 -> 107.9; a decay per channel, four of 977, 16 heads: 109.9 -> 108.0.
+// 178 -> 173; with (1) alone chunk by chunk, one of 4096, 32 heads 105.8, of 1000, 16 heads 27.8, heads first 104.2 and
+// 25.8; a decay per channel, four of 977, 16 heads: 109.9 -> 108.0.
 // chunk_number: the workgroup's chunk or sequence (past the last one: none).
 constexpr int CHUNKS_Y = 32768;
 inline dim3 chunk_grid(int chunks, int H) {

@@ -102,7 +102,6 @@ EIA_API int eia_latent_prep(const void* fused, long ld, int q_off, int q_rank, c
 // ------------------------------------------------------------------------------------- attention
 constexpr int LAT_UNIT = 64;       // keys per tile of the decode form, cut at multiples of it
 
-
 // Tiles of a decode row, and of each of the key partitions that it uses out of the launch's: the fewest that leave the
 // longest one as short; where a tile takes less than its partition's place in the merge (R up to 256), two tiles each beyond
 // 32 partitions (eight rows at 4000 tokens, 256 + 32: 15.7 us in 63, 14.8 in 32).
@@ -354,7 +353,7 @@ EIA_API int eia_latent_attn(const void* qa, long qa_st, long qa_sh, const void* 
 //
 // Bound by latency: a row's 64-key tiles are a chain of cache loads and two barriers, and the launch
 // lasts as long as the longest partition.  MI355X, 48 rows at up to 4096 tokens, window 1024, 16
-// heads, R 512 + 64: 23.7 + 4.1 us in five partitions; 200 rows at up to 2500 tokens, no window, with
+// heads, R 512 + 64: 22.0 + 4.0 us in five partitions; 200 rows at up to 2500 tokens, no window, with
 // 16 heads 153 -> 134 us and with 64 heads 499 -> 437 us since a tile's page is known before its fetch and
 // its LDS reads are asked for before the first product; R 128 + 32 with 64 heads 120 -> 115 us, R 256 + 64
 // 292 -> 292 us.  (Two tiles of cache loads in flight, in registers: 27 us instead of 24; the reads held in
@@ -585,7 +584,7 @@ latent_decode_kernel(LatentAttnArgs a) {
 // its weight, then the threads sum four latent columns each over the partitions (nparts <= 64).
 // Rows whose context is too short for two partitions were finished by the
 // attention kernel itself.  Bound by latency: the partials of up to eight partitions are asked for together with the
-// weights' inputs (48 rows of 16 heads, R 512, five partitions: 4.8 -> 4.1 us), sixteen at a time where there are many more
+// weights' inputs (48 rows of 16 heads, R 512, five partitions: 4.8 -> 4.0 us), sixteen at a time where there are many more
 // (four at a time: 4000 tokens, 16 heads, one row in 63 partitions, both launches: 28.7 us instead of 19.3).
 constexpr int LM_P = 8;
 __global__ void __launch_bounds__(128)

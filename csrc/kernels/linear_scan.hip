@@ -449,12 +449,13 @@ EIA_API int eia_linear_scan(const void* x, long ld, int q_off, int k_off, int v_
 // traffic (4 passes over chunks x H x dk x dv floats), and halving their number costs less than the
 // longer sums inside a chunk add.
 // Four prompts of 1000 .. 2000 tokens (6688 rows), 16 heads of 128, mode 1, bf16 take 11 + 31 + 21 +
-// 58 us on an MI355X (gates, (1), (2), (3)); in fp32 products (1) and (3) took 57 + 103 us.  Bound by the
+// 59 us on an MI355X (gates, (1), (2), (3)); in fp32 products (1) and (3) took 57 + 103 us.  Bound by the
 // workspace and the rows, which (1), (2) and (3) move at 3.8, 5.4 and 3.3 TB/s, and by the steps of
 // a workgroup, which reads, splits and multiplies in turn.  All heads of a chunk run side by side in (1) and (3), so
-// that whole rows are read together, and (3) asks for its queries before it waits for the gates: 123 -> 118 us for the
+// that whole rows are read together, and (3) asks for its queries before it waits for the gates: 135 -> 129 us for the
 // op; three rotated prompts of up to 2700 tokens 188 -> 178, five of up to 1100 of 32 heads of 64 78 -> 77.  What the
-// normaliser, the norm and the gate read is asked for at once (four rounds behind each other: 118 -> 116 us).
+// normaliser, the norm and the gate read is asked for at once (four rounds behind each other: 129 -> 124 us, 178 -> 177,
+// 77 -> 76).
 constexpr int LK = 128;                     // tokens per chunk
 constexpr float LS_LOG2E = 1.4426950408889634f;
 

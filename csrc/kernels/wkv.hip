@@ -241,7 +241,7 @@ EIA_API int eia_wkv_scan(const void* r, const void* k, const void* v, const void
 // instead of 1.2e-7 against 64 bits where every second token forgets, in the same time.)
 //
 // Bound by instruction issue (exponentials, conversions, fp32 products; 31 us of vector and 15 us of
-// matrix issue in (3)), not by memory: one 4096-token prompt, 32 heads of 64, bf16 takes 28 + 15 +
+// matrix issue in (3)), not by memory: one 4096-token prompt, 32 heads of 64, bf16 takes 27 + 15 +
 // 64 us on an MI355X, 2091 us token by token.  (3) took 125 us with 2-byte loads and a padded LDS
 // tile for each of r, k, v and the running sums (two workgroups per CU instead of three).
 constexpr int WC = 64;                      // tokens per chunk

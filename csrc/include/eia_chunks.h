@@ -33,32 +33,32 @@ inline dim3 chunk_grid(int chunks, int H) {
 }
 EIA_DEV int chunk_number() { return blockIdx.z * CHUNKS_Y + blockIdx.y; }
 
-// Four columns of a state row over a sequence's nc chunks, us and ls apart: U of a chunk, its own
-// contribution, turns into the state before it; S, the state before the first one, into the state after
-// the last.  L: log2 of a chunk's decay.  A group's contributions are requested while the previous group
-// is summed.
+// Four columns of a state row over a sequence's nc chunks, us apart: U of a chunk, its own contribution, turns into
+// the state S before it; step(x, l, u) then takes S past chunk x, with u what U held and l what load(x) gave.  A
+// group's contributions are requested while the previous group is summed.
 constexpr int CHUNKS_AHEAD = 8;             // chunks whose contributions are in flight
-EIA_DEV void chunk_walk(float* U, long us, const float* L, long ls, int nc, f32x4& S) {
+template <typename L, typename Load, typename Step>
+EIA_DEV void chunk_walk_with(float* U, long us, int nc, const f32x4& S, Load&& load, Step&& step) {
   f32x4 u[CHUNKS_AHEAD];
-  float d[CHUNKS_AHEAD];
-  auto fetch = [&](int b, f32x4 (&u)[CHUNKS_AHEAD], float (&d)[CHUNKS_AHEAD]) {
+  L d[CHUNKS_AHEAD];
+  auto fetch = [&](int b, f32x4 (&u)[CHUNKS_AHEAD], L (&d)[CHUNKS_AHEAD]) {
 #pragma unroll
     for (int k = 0; k < CHUNKS_AHEAD; ++k) {
       const int x = min(b + k, nc - 1);
       u[k] = *reinterpret_cast<const f32x4*>(U + x * us);
-      d[k] = L[x * ls];
+      d[k] = load(x);
     }
   };
   fetch(0, u, d);
   for (int b = 0; b < nc; b += CHUNKS_AHEAD) {
     f32x4 un[CHUNKS_AHEAD];
-    float dn[CHUNKS_AHEAD];
+    L dn[CHUNKS_AHEAD];
     fetch(b + CHUNKS_AHEAD, un, dn);
 #pragma unroll
     for (int k = 0; k < CHUNKS_AHEAD; ++k) {
       if (b + k < nc) {
         *reinterpret_cast<f32x4*>(U + (b + k) * us) = S;
-        S = S * __builtin_amdgcn_exp2f(d[k]) + u[k];
+        step(b + k, d[k], u[k]);
       }
     }
 #pragma unroll
@@ -67,6 +67,11 @@ EIA_DEV void chunk_walk(float* U, long us, const float* L, long ls, int nc, f32x
       d[k] = dn[k];
     }
   }
+}
+// The same where the step is a decay; l: its log2, ls apart.
+EIA_DEV void chunk_walk(float* U, long us, const float* l, long ls, int nc, f32x4& S) {
+  chunk_walk_with<float>(U, us, nc, S, [&](int x) { return l[x * ls]; },
+                         [&](int, float d, f32x4 u) { S = S * __builtin_amdgcn_exp2f(d) + u; });
 }
 
 // Place of (token, channel) in an fp32 LDS tile [tokens][W]: the 16-byte units of a row are turned by the

@@ -435,9 +435,15 @@ EIA_API int eia_linear_scan(const void* x, long ld, int q_off, int k_off, int v_
 // (the normaliser n is one more state column, n_t . q_t the row sum of the same weights).  Sums of l
 // run over 16-token blocks and over whole blocks, inside a block over just the tokens between: every
 // exponent is a sum of what it covers, so it is <= 0 and keeps its precision.  (Differences of two running
-// sums inside a block: 9.9e-7 instead of 1.8e-7 against 64 bits, fp32 gates that close hard.)  The log gates
-// of mode 1 come from a pre-pass that carries the running maximum, angles of rotated heads from a table.
-// Chunks are found on the device (eia_chunks.h).
+// sums inside a block: 9.9e-7 instead of 1.8e-7 against 64 bits, fp32 gates that close hard.)  Angles of rotated heads
+// come from a table.  Chunks are found on the device (eia_chunks.h).
+//
+// The running maximum of mode 1 is a scan over pairs (sum of f, maximum behind it).  (1) forms U relative to the maximum
+// of the chunk's own gates and leaves the chunk's pair, (2) walks the pairs beside the states and brings both to the
+// carried maximum, (3) forms its gates again from the maximum before its chunk.  (A pass of its own for the gates of all
+// rows, one workgroup per sequence and head, was bound by the latency of reads a projected row apart: 11 us and a launch,
+// where the gates now cost (1) 5 us and (3) nothing.  The op below 124.5 -> 111.9 us; S against 64 bits, four shapes,
+// 1.53e-7 .. 1.75e-7 -> 1.29e-7 .. 1.58e-7.)
 //
 // Rows of bf16: all products take bf16 operands, fp32 factors as the sum of three (split3).  Values, and
 // unrotated keys and queries, are exact as they are, so most products are three of 16x16x32 at 3/16 of the matrix
@@ -448,21 +454,23 @@ EIA_API int eia_linear_scan(const void* x, long ld, int q_off, int k_off, int v_
 // 128-token chunks: the states between chunks are the larger part of the memory
 // traffic (4 passes over chunks x H x dk x dv floats), and halving their number costs less than the
 // longer sums inside a chunk add.
-// Four prompts of 1000 .. 2000 tokens (6688 rows), 16 heads of 128, mode 1, bf16 take 11 + 31 + 21 +
-// 59 us on an MI355X (gates, (1), (2), (3)); in fp32 products (1) and (3) took 57 + 103 us.  Bound by the
-// workspace and the rows, which (1), (2) and (3) move at 3.8, 5.4 and 3.3 TB/s, and by the steps of
+// Four prompts of 1000 .. 2000 tokens (6688 rows), 16 heads of 128, mode 1, bf16 take 35 + 21 +
+// 59 us on an MI355X ((1), (2), (3)); in fp32 products (1) and (3) took 57 + 103 us.  Bound by the
+// workspace and the rows, which (1), (2) and (3) move at 3.3, 5.4 and 3.3 TB/s, and by the steps of
 // a workgroup, which reads, splits and multiplies in turn.  All heads of a chunk run side by side in (1) and (3), so
 // that whole rows are read together, and (3) asks for its queries before it waits for the gates: 135 -> 129 us for the
 // op; three rotated prompts of up to 2700 tokens 188 -> 178, five of up to 1100 of 32 heads of 64 78 -> 77.  What the
 // normaliser, the norm and the gate read is asked for at once (four rounds behind each other: 129 -> 124 us, 178 -> 177,
-// 77 -> 76).
+// 77 -> 76).  (1) asks for unrotated rows a half ahead, the first before it waits for the gates (33.2 -> 30.0 us, before it
+// formed the gates itself).
 constexpr int LK = 128;                     // tokens per chunk
 constexpr float LS_LOG2E = 1.4426950408889634f;
 
 struct KChunkArgs {
   float* U;                                 // [numbers, H, DP, UW]: contribution, then state before
-  float* G;                                 // [numbers, H]: sums of l
-  float* la; float* lb; float* nm;          // [rows, H] log a, log b, -m  (mode 1)
+  float* G;                                 // [numbers, H]: sums of l; mode 1: [.., 2] a chunk's pair (f, m)
+  float* m0;                                // [numbers, H]: the running maximum before the chunk (mode 1)
+  float* la;                                // [rows, H * D]: log2 a (mode 2)
   float2* rot;                              // [rows, rot_dims / 2]: cos, sin
   int nseq, rows, DP, VP, UW;               // UW: VP, and in mode 1 four more (the normaliser, 0, 0, 0)
   bool wide = false;                        // per channel: gate, weight and output rows can be taken 4 at a time
@@ -471,76 +479,6 @@ struct KChunkArgs {
 // The chunk of number x; false where there is none or the sequence is skipped.
 EIA_DEV bool ls_chunk(const ScanArgs& a, int nseq, int x, int& s, int& row0, int& n) {
   return chunk_of<LK>(a.cu, nseq, x, s, row0, n) && a.slots[s] >= 0;
-}
-
-// (A) log gates of mode 1: one workgroup per (sequence, head).  The running maximum m_t =
-// max(f_t + m_(t-1), i_t) is a scan over pairs (f, i); a thread walks four tokens, the pairs of the
-// threads before it come from a scan over lanes and waves.  Serially in one thread the longest of
-// four 2000-token prompts took 63 us.
-// Bound by the latency of a pass, whose rows lie a whole projected row apart: the next pass's are asked for
-// before this one's scan.  Four 2000-token prompts of 16 heads: 13.0 -> 10.9 us.
-template <typename T, int LS_GT>            // LS_GT threads
-__global__ void __launch_bounds__(LS_GT)
-ls_gates_kernel(ScanArgs a, KChunkArgs c) {
-  __shared__ float2 wsum[LS_GT / 64];
-  __shared__ float carry;
-  const int s = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int slot = a.slots[s];
-  if (slot < 0) return;
-  const int lo = a.cu[s], hi = a.cu[s + 1];
-  if (hi <= lo) return;
-  float m0 = a.positions[lo] == 0 ? 0.f : a.M[(long)slot * a.H + h];
-  const T* X = static_cast<const T*>(a.x);
-  float xi[4], xf[4];
-  auto load = [&](int base) {
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const T* xr = X + (long)min(base + 4 * tid + k, hi - 1) * a.ld;
-      xi[k] = ld_f32<T>(xr, a.i_off + h);
-      xf[k] = ld_f32<T>(xr, a.f_off + h);
-    }
-  };
-  load(lo);
-  for (int base = lo; base < hi; base += 4 * LS_GT) {
-    float gi[4], gf[4];
-    float2 p = {0.f, -INFINITY};                       // the thread's pair: sum of f, max with decays
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      gi[k] = a.cap > 0.f ? a.cap * tanhf(xi[k] / a.cap) : xi[k];
-      gf[k] = ls_logsigmoid(a.cap > 0.f ? a.cap * tanhf(xf[k] / a.cap) : xf[k]);
-      if (base + 4 * tid + k < hi) p = {p.x + gf[k], fmaxf(p.y + gf[k], gi[k])};
-    }
-    if (base + 4 * LS_GT < hi) load(base + 4 * LS_GT);
-    float2 q = p;                                      // inclusive over the lanes
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const float ux = __shfl_up(q.x, o, 64), uy = __shfl_up(q.y, o, 64);
-      if (lane >= o) q = {ux + q.x, fmaxf(uy + q.x, q.y)};
-    }
-    if (lane == 63) wsum[w] = q;
-    __syncthreads();
-    float m = m0;                                      // m before the thread's first token
-    for (int k = 0; k < w; ++k) m = fmaxf(m + wsum[k].x, wsum[k].y);
-    const float ex = __shfl_up(q.x, 1, 64), ey = __shfl_up(q.y, 1, 64);
-    if (lane > 0) m = fmaxf(m + ex, ey);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int row = base + 4 * tid + k;
-      const float fm = gf[k] + m, mn = fmaxf(fm, gi[k]);
-      if (row < hi) {
-        const long o = (long)row * a.H + h;
-        c.la[o] = fm - mn;
-        c.lb[o] = gi[k] - mn;
-        c.nm[o] = -mn;
-        m = mn;
-      }
-    }
-    if (tid == LS_GT - 1) carry = m;
-    __syncthreads();
-    m0 = carry;
-    // (the thread that holds the last token knows the final maximum)
-    if (base + 4 * LS_GT >= hi && (hi - 1 - base) >> 2 == tid) a.M[(long)slot * a.H + h] = m;
-  }
 }
 
 // Angles of the rotated channels, shared by all heads and by the q and k of (1) and (3).
@@ -649,25 +587,72 @@ EIA_DEV void ls_stage_v(const ScanArgs& a, int row0, int n, int h, int t0, T* sv
   }
 }
 
-// Log decay and log weight of the chunk's token threadIdx.x, in base 2 (threads 0 .. LK - 1).
-EIA_DEV void ls_log_load(const ScanArgs& a, const KChunkArgs& c, int row0, int n, int h, float& l, float& b) {
+// What the logs of the chunk's token threadIdx.x are formed from (threads 0 .. LK - 1): the decay or the two gate
+// pre-activations of the token and, for the second wave, of the token 64 before it.
+struct LsGates {
+  float xi[2], xf[2];
+};
+template <typename T> EIA_DEV LsGates ls_log_load(const ScanArgs& a, int row0, int n, int h) {
+  LsGates g = {};
   const int t = threadIdx.x;
-  l = b = 0.f;
-  if (t >= min(n, LK)) return;
+  if (t >= LK) return g;
   if (a.mode == 0) {
-    l = a.decay[h];
-  } else {
-    l = c.la[(long)(row0 + t) * a.H + h];
-    b = c.lb[(long)(row0 + t) * a.H + h];
+    g.xi[0] = a.decay[h];
+    return g;
   }
+#pragma unroll
+  for (int y = 0; y < 2; ++y) {
+    const T* x = static_cast<const T*>(a.x) + (long)(row0 + min(y ? t & 63 : t, n - 1)) * a.ld + h;
+    g.xi[y] = ld_f32<T>(x, a.i_off);
+    g.xf[y] = ld_f32<T>(x, a.f_off);
+  }
+  return g;
+}
+// Mode 1: log decay l and log weight b of the token, m the running maximum with it, from the maximum m0 before the
+// chunk (-inf: none, what lies before the chunk weighs nothing).  m_t = max(f_t + m_(t-1), i_t) is a scan over pairs
+// (sum of f, maximum behind it).  -> the pair up to and with the token.
+EIA_DEV float2 ls_log_gates(const ScanArgs& a, int n, const LsGates& g, float m0, float& l, float& b, float& m) {
+  const int t = threadIdx.x, lane = t & 63;
+  auto soft = [&](float x) { return a.cap > 0.f ? a.cap * tanhf(x / a.cap) : x; };
+  auto join = [](float2 p, float2 q) { return make_float2(p.x + q.x, fmaxf(p.y + q.x, q.y)); };
+  auto scan = [&](float2 q) {               // inclusive over the lanes
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const float2 up = make_float2(__shfl_up(q.x, o, 64), __shfl_up(q.y, o, 64));
+      if (lane >= o) q = join(up, q);
+    }
+    return q;
+  };
+  const float2 none = make_float2(0.f, -INFINITY);
+  const float gi = soft(g.xi[0]), gf = ls_logsigmoid(soft(g.xf[0]));
+  float2 first = none;                      // of the 64 tokens before the second wave's
+  if (t >= 64) {
+    first = scan(lane < n ? make_float2(ls_logsigmoid(soft(g.xf[1])), soft(g.xi[1])) : none);
+    first = make_float2(__shfl(first.x, 63, 64), __shfl(first.y, 63, 64));
+  }
+  const float2 p = join(first, scan(t < n ? make_float2(gf, gi) : none));
+  m = fmaxf(m0 + p.x, p.y);
+  const float up = __shfl_up(m, 1, 64), before = lane ? up : fmaxf(m0 + first.x, first.y);
+  // (not gf + before - m: where nothing new is met the maximum moves with the decays, and the roundings of its
+  // steps would add up.  S against 64 bits 2.5e-7 instead of 1.6e-7)
+  const float fm = gf + before;
+  l = t >= n || before == -INFINITY || fm >= gi ? 0.f : fm - gi;
+  b = t >= n ? 0.f : m > -INFINITY ? gi - m : -INFINITY;
+  return p;
 }
 // Sums of l over 16-token blocks: pre up to and with a token, suf behind it, tot of whole blocks;
-// mb: m, sl: l.  Threads 0 .. LK - 1, l and b as ls_log_load leaves them.
-EIA_DEV void ls_chunk_logs(const ScanArgs& a, int n, float l, float b, float* pre, float* suf, float* tot, float* mb,
-                           float* sl) {
+// mb: log2 b, sl: l, mx: m (mode 1).  Threads 0 .. LK - 1.  pair: where mode 1's pair of the chunk goes, or null.
+EIA_DEV void ls_chunk_logs(const ScanArgs& a, int n, const LsGates& g, float m0, float* pre, float* suf, float* tot,
+                           float* mb, float* sl, float* mx, float2* pair) {
   const int t = threadIdx.x;
   if (t >= LK) return;
-  if (a.mode == 0) l = t < n ? logf(l) : 0.f;
+  float l, b = 0.f;
+  if (a.mode == 0) {
+    l = t < n ? logf(g.xi[0]) : 0.f;
+  } else {
+    const float2 p = ls_log_gates(a, n, g, m0, l, b, mx[t]);
+    if (pair && t == LK - 1) *pair = p;
+  }
   l *= LS_LOG2E;
   b *= LS_LOG2E;
   l = l < -150.f ? -150.f : l;                         // (2^-150 is zero; what is no number stays so)
@@ -715,13 +700,17 @@ struct LsChunk {
   const float *pre, *suf, *mb, *tot, *sl;
 };
 
+// The weight of token tk's key in what the chunk adds to the state, 0 past the chunk.
+EIA_DEV float ls_key_weight(const ScanArgs& a, const LsChunk& k, int tk) {
+  float e = k.mb[tk] + k.suf[tk];
+  for (int b = (tk >> 4) + 1; b < LK / 16; ++b) e += k.tot[b];
+  return tk < k.n ? a.kscale * __builtin_amdgcn_exp2f(e) : 0.f;
+}
 // The weighted key of token tk, channels i .. i + 7: what it adds to the state after the chunk.
 template <typename T, bool VEC, bool ROT>
 EIA_DEV void ls_weighted_key(const ScanArgs& a, const KChunkArgs& c, const LsChunk& k, int tk, int i, float (&v)[8]) {
   ls_head8<T, VEC, ROT>(a, c, k.row0 + min(tk, k.n - 1), a.k_off + (long)k.h * a.D, i, v);
-  float e = k.mb[tk] + k.suf[tk];
-  for (int b = (tk >> 4) + 1; b < LK / 16; ++b) e += k.tot[b];
-  const float wt = tk < k.n ? a.kscale * __builtin_amdgcn_exp2f(e) : 0.f;
+  const float wt = ls_key_weight(a, k, tk);
 #pragma unroll
   for (int x = 0; x < 8; ++x) v[x] = tk < k.n ? v[x] * wt : 0.f;
 }
@@ -797,15 +786,32 @@ EIA_DEV void ls_state_fp32(const ScanArgs& a, const KChunkArgs& c, const LsChunk
 // normaliser is the product with ones.  Rows of an LDS tile are 32 bytes more than a multiple of the banks
 // apart, so that the transposing reads of eight rows meet all of them.  false: something was not finite
 // (uniform over the workgroup; nothing was written).
-template <bool VEC, bool ROT, int MX>
-EIA_DEV bool ls_state_bf16(const ScanArgs& a, const KChunkArgs& c, const LsChunk& k, long at, unsigned char* lds) {
-  constexpr int PITCH = MX + 16, PLANE = 64 * PITCH, NA = MX / 32, NB = MX / 64;
+template <bool VEC, bool ROT, int MX, typename Logs>
+EIA_DEV bool ls_state_bf16(const ScanArgs& a, const KChunkArgs& c, const LsChunk& k, long at, unsigned char* lds,
+                           Logs&& logs) {
+  constexpr int PITCH = MX + 16, PLANE = 64 * PITCH, NA = MX / 32, NB = MX / 64, NU = 64 * MX / 8 / 512;
+  constexpr bool AHEAD = VEC && !ROT;                  // a half's rows are on their way during what stands before it
   bf16_t* sk = reinterpret_cast<bf16_t*>(lds);         // [3][64][PITCH]
   bf16_t* sv = sk + 3 * PLANE;                         // [64][PITCH]
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, g4 = lane >> 4, c0 = MX / 4 * (w & 3), d0 = MX / 2 * (w >> 2);
   const bool live = c0 < c.DP, norm = a.mode == 1 && d0 == 0;
   const bf16_t* X = static_cast<const bf16_t*>(a.x) + a.v_off + (long)k.h * a.Dv;
+  const int ut = threadIdx.x / (MX / 8), ui = 8 * (threadIdx.x % (MX / 8));        // a thread's first token, its channels
+  constexpr int UT = 512 / (MX / 8);
+  bf16x8 kr[NU], vr[NU];
+  auto fetch = [&](int t0) {
+    const bf16_t* xk = static_cast<const bf16_t*>(a.x) + a.k_off + (long)k.h * a.D + (ui < a.D ? ui : 0);
+    const bf16_t* xv = X + (ui < a.Dv ? ui : 0);
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      const long r = (long)(k.row0 + min(t0 + ut + UT * u, k.n - 1)) * a.ld;
+      kr[u] = *reinterpret_cast<const bf16x8*>(xk + r);
+      vr[u] = *reinterpret_cast<const bf16x8*>(xv + r);
+    }
+  };
+  if constexpr (AHEAD) fetch(0);
+  logs();
   bf16x8 ones;
 #pragma unroll
   for (int e = 0; e < 8; ++e) ones[e] = (bf16_t)1.f;
@@ -819,25 +825,37 @@ EIA_DEV bool ls_state_bf16(const ScanArgs& a, const KChunkArgs& c, const LsChunk
   for (int t0 = 0; t0 < k.n; t0 += 64) {
     __syncthreads();                                   // logs are there; the first half was read
 #pragma unroll
-    for (int u = threadIdx.x; u < 64 * MX / 8; u += 512) {
-      const int t = u / (MX / 8), i = 8 * (u % (MX / 8));
-      const bool ok = t0 + t < k.n && i < a.Dv;
-      const bf16_t* p = X + (long)(k.row0 + (ok ? t0 + t : 0)) * a.ld + (ok ? i : 0);
+    for (int u = 0; u < NU; ++u) {
+      const int t = ut + UT * u;
+      const bool ok = t0 + t < k.n && ui < a.Dv;
       bf16x8 v;
-      if constexpr (VEC) {
-        v = *reinterpret_cast<const bf16x8*>(p);
+      float kw[8];
+      if constexpr (AHEAD) {
+        const bool in = t0 + t < k.n && ui < a.D;
+        const float wt = ls_key_weight(a, k, t0 + t);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) kw[e] = in ? (float)kr[u][e] * wt : 0.f;
+        v = vr[u];
         if (!ok) v = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
       } else {
+        const bf16_t* p = X + (long)(k.row0 + (ok ? t0 + t : 0)) * a.ld + (ok ? ui : 0);
+        if constexpr (VEC) {
+          v = *reinterpret_cast<const bf16x8*>(p);
+          if (!ok) v = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+        } else {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = ok && i + e < a.Dv ? p[e] : (bf16_t)0.f;
+          for (int e = 0; e < 8; ++e) v[e] = ok && ui + e < a.Dv ? p[e] : (bf16_t)0.f;
+        }
+        ls_weighted_key<bf16_t, VEC, ROT>(a, c, k, t0 + t, ui, kw);
       }
-      *reinterpret_cast<bf16x8*>(sv + t * PITCH + i) = v;
-      float kw[8];
-      ls_weighted_key<bf16_t, VEC, ROT>(a, c, k, t0 + t, i, kw);
+      *reinterpret_cast<bf16x8*>(sv + t * PITCH + ui) = v;
       bf16x8 part[3];
       split3(kw, part);
 #pragma unroll
-      for (int p3 = 0; p3 < 3; ++p3) *reinterpret_cast<bf16x8*>(sk + p3 * PLANE + t * PITCH + i) = part[p3];
+      for (int p3 = 0; p3 < 3; ++p3) *reinterpret_cast<bf16x8*>(sk + p3 * PLANE + t * PITCH + ui) = part[p3];
+    }
+    if constexpr (AHEAD) {
+      if (t0 + 64 < k.n) fetch(t0 + 64);
     }
     __syncthreads();
     if (!live) continue;
@@ -906,24 +924,26 @@ ls_chunk_state_kernel(ScanArgs a, KChunkArgs c) {
   constexpr bool BF = sizeof(T) == 2;
   constexpr int FP32 = 64 * MX * (4 + (int)sizeof(T)), SPLIT = BF ? 4 * 64 * (MX + 16) * 2 : 0;
   __shared__ __align__(16) unsigned char tiles[FP32 > SPLIT ? FP32 : SPLIT];
-  __shared__ float pre[LK], suf[LK], mb[LK], tot[LK / 16], sl[LK];
+  __shared__ float pre[LK], suf[LK], mb[LK], tot[LK / 16], sl[LK], mx[LK];
   int s, row0, n;
   if (!ls_chunk(a, c.nseq, chunk_number(), s, row0, n)) return;
   const int h = blockIdx.x;
-  float l, b;
-  ls_log_load(a, c, row0, n, h, l, b);
-  ls_chunk_logs(a, n, l, b, pre, suf, tot, mb, sl);
+  const LsGates g = ls_log_load<T>(a, row0, n, h);
   const long at = (long)chunk_number() * a.H + h;
   const LsChunk k{row0, n, h, pre, suf, mb, tot, sl};
+  auto logs = [&] {
+    ls_chunk_logs(a, n, g, -INFINITY, pre, suf, tot, mb, sl, mx, reinterpret_cast<float2*>(c.G) + at);
+  };
   if constexpr (BF) {
-    if (!ls_state_bf16<VEC, ROT, MX>(a, c, k, at, tiles)) ls_state_fp32<T, VEC, ROT, MX>(a, c, k, at, tiles);
+    if (!ls_state_bf16<VEC, ROT, MX>(a, c, k, at, tiles, logs)) ls_state_fp32<T, VEC, ROT, MX>(a, c, k, at, tiles);
   } else {
+    logs();
     ls_state_fp32<T, VEC, ROT, MX>(a, c, k, at, tiles);
   }
-  if (threadIdx.x == 0) {
-    float g = 0.f;
-    for (int b = 0; b < LK / 16; ++b) g += tot[b];
-    c.G[at] = g;
+  if (a.mode == 0 && threadIdx.x == 0) {
+    float sum = 0.f;
+    for (int b = 0; b < LK / 16; ++b) sum += tot[b];
+    c.G[at] = sum;
   }
 }
 
@@ -949,8 +969,19 @@ ls_chunk_scan_kernel(ScanArgs a, KChunkArgs c) {
   }
   const long us = (long)a.H * c.DP * c.UW;
   float* U = c.U + (x0 * a.H + h) * c.DP * c.UW + (long)i * c.UW + j;
-  const float* G = c.G + x0 * a.H + h;
-  chunk_walk(U, us, G, a.H, nc, S);
+  if (a.mode == 0) {
+    chunk_walk(U, us, c.G + x0 * a.H + h, a.H, nc, S);
+  } else {                                             // U stands relative to the chunk's own maximum
+    const float2* G = reinterpret_cast<const float2*>(c.G) + x0 * a.H + h;
+    float* m0 = c.m0 + x0 * a.H + h;                   // ((3) leaves the slot's new maximum: others here still read it)
+    float m = a.positions[lo] == 0 ? 0.f : a.M[(long)slot * a.H + h];
+    chunk_walk_with<float2>(U, us, nc, S, [&](int x) { return G[(long)x * a.H]; }, [&](int x, float2 p, f32x4 u) {
+      if (u4 == 0) m0[(long)x * a.H] = m;
+      const float mn = fmaxf(m + p.x, p.y);
+      S = S * __builtin_amdgcn_exp2f((m + p.x - mn) * LS_LOG2E) + u * __builtin_amdgcn_exp2f((p.y - mn) * LS_LOG2E);
+      m = mn;
+    });
+  }
   if (i < a.D) {
 #pragma unroll
     for (int k = 0; k < 4; ++k)
@@ -1124,9 +1155,9 @@ template <bool VEC, bool ROT, int MX> struct LsOutTiles {
 // Sixteen columns from 16 u on of row r to the places of their tiles.
 template <int MX> EIA_DEV int ls_col16(int u) { return 64 * (u >> 2) + 4 * (u & 3); }
 
-template <bool VEC, bool ROT, int MX>
+template <bool VEC, bool ROT, int MX, typename Logs>
 EIA_DEV bool ls_out_bf16(const ScanArgs& a, const KChunkArgs& c, const LsChunk& k, bool state, unsigned char* tiles,
-                         const float* sn, f32x4 (&o)[MX / 16], float& rs, float* logs) {
+                         const float* sn, f32x4 (&o)[MX / 16], float& rs, Logs&& logs) {
   using L = LsOutTiles<VEC, ROT, MX>;
   constexpr int NQ = L::NQ, PITCH = L::PITCH, NX = MX / 32;
   bf16_t* sS = reinterpret_cast<bf16_t*>(tiles);       // [3][64][PITCH], then keys and values
@@ -1146,8 +1177,6 @@ EIA_DEV bool ls_out_bf16(const ScanArgs& a, const KChunkArgs& c, const LsChunk& 
 #pragma unroll
     for (int e = 0; e < 4; ++e) sf[e] = *reinterpret_cast<const f32x4*>(S + 4 * e);
   };
-  float l, b;
-  ls_log_load(a, c, row0, n, h, l, b);
   bf16x8 qf[NQ][NX];                                   // this lane's query: channels 32 x + 8 g4 + e
   auto queries = [&](bool use) {                       // use: q . n, else nothing but qf
     float z = 0.f;
@@ -1174,7 +1203,7 @@ EIA_DEV bool ls_out_bf16(const ScanArgs& a, const KChunkArgs& c, const LsChunk& 
   const bool norm = a.mode == 1 && state;
   if constexpr (!ROT) queries(false);                  // (asked for before the state and the logs are waited for)
   fetch(0);
-  ls_chunk_logs(a, n, l, b, logs, logs + LK, logs + 4 * LK, logs + 2 * LK, logs + 3 * LK);
+  logs();
   __syncthreads();
   float nq = 0.f;
   if constexpr (ROT) {
@@ -1359,28 +1388,30 @@ ls_chunk_out_kernel(ScanArgs a, KChunkArgs c) {
   constexpr int KV = LK * MX * ((BF && !ROT ? 2 : 4) + (int)sizeof(T)), FP32 = KV > MX * MX * 4 ? KV : MX * MX * 4;
   constexpr int SPLIT = BF ? LsOutTiles<VEC, ROT, MX>::BYTES : 0;
   __shared__ __align__(16) unsigned char tiles[FP32 > SPLIT ? FP32 : SPLIT];
-  __shared__ __align__(16) float logs[4 * LK + LK / 16], sn[MX];
-  float *pre = logs, *suf = logs + LK, *mb = logs + 2 * LK, *sl = logs + 3 * LK, *tot = logs + 4 * LK;
+  __shared__ __align__(16) float pre[LK], suf[LK], mb[LK], sl[LK], tot[LK / 16], mx[LK], sn[MX];
   int s, row0, n;
   if (!ls_chunk(a, c.nseq, chunk_number(), s, row0, n)) return;
   const int h = blockIdx.x, lane = threadIdx.x & 63, wv = threadIdx.x >> 6, Dv = a.Dv;
   const int w = wv < 4 ? wv : 11 - wv, l16 = lane & 15, g4 = lane >> 4, t0 = 16 * w;
+  const long at = (long)chunk_number() * a.H + h;
+  const LsGates g = ls_log_load<T>(a, row0, n, h);
+  const float m0 = a.mode == 1 ? c.m0[at] : 0.f;
   const bool state = row0 != a.cu[s] || a.positions[a.cu[s]] != 0;   // (else a fresh sequence: S = 0)
   if (state && a.mode == 1 && threadIdx.x < MX)
-    sn[threadIdx.x] = c.U[(((long)chunk_number() * a.H + h) * c.DP + min((int)threadIdx.x, c.DP - 1)) * c.UW + c.VP];
+    sn[threadIdx.x] = c.U[(at * c.DP + min((int)threadIdx.x, c.DP - 1)) * c.UW + c.VP];
   const LsChunk k{row0, n, h, pre, suf, mb, tot, sl};
+  auto logs = [&] { ls_chunk_logs(a, n, g, m0, pre, suf, tot, mb, sl, mx, nullptr); };
   f32x4 o[MX / 16];
   float rs;
   if constexpr (BF) {
     if (!ls_out_bf16<VEC, ROT, MX>(a, c, k, state, tiles, sn, o, rs, logs))
       ls_out_fp32<T, VEC, ROT, MX>(a, c, k, state, tiles, sn, o, rs);
   } else {
-    float l, b;
-    ls_log_load(a, c, row0, n, h, l, b);
-    ls_chunk_logs(a, n, l, b, pre, suf, tot, mb, sl);
+    logs();
     __syncthreads();
     ls_out_fp32<T, VEC, ROT, MX>(a, c, k, state, tiles, sn, o, rs);
   }
+  if (a.mode == 1 && threadIdx.x == n - 1 && row0 + n == a.cu[s + 1]) a.M[(long)a.slots[s] * a.H + h] = mx[n - 1];
   if (t0 >= n) return;
   rs += __shfl_xor(rs, 16, 64);                        // n_t . q_t of query l16
   rs += __shfl_xor(rs, 32, 64);
@@ -1389,12 +1420,10 @@ ls_chunk_out_kernel(ScanArgs a, KChunkArgs c) {
   T* Y = static_cast<T*>(a.y);
   typedef T T4 __attribute__((ext_vector_type(4)));
   // what a lane's four tokens need besides, asked for together
-  float nm[4];
   T4 gt[4][MX / 64], nw[MX / 64];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const long row = row0 + min(t0 + 4 * g4 + i, n - 1);
-    nm[i] = a.mode == 1 ? c.nm[row * a.H + h] : 0.f;
 #pragma unroll
     for (int x = 0; x < MX / 64; ++x) {
       const int d = 64 * x + 4 * l16;
@@ -1416,7 +1445,7 @@ ls_chunk_out_kernel(ScanArgs a, KChunkArgs c) {
     const int t = t0 + 4 * g4 + i;
     const float nqi = __shfl(rs, 4 * g4 + i, 64);
     float den = 1.f;
-    if (a.mode == 1) den = 1.0f / (fmaxf(fabsf(nqi), expf(nm[i])) + 1e-6f);
+    if (a.mode == 1) den = 1.0f / (fmaxf(fabsf(nqi), expf(-mx[min(t, n - 1)])) + 1e-6f);
     float ss = 0.f;
 #pragma unroll
     for (int j = 0; j < MX / 16; ++j) {
@@ -1453,13 +1482,6 @@ template <typename T, bool VEC, bool ROT, int MX>
 static void ls_chunked(const ScanArgs& a, const KChunkArgs& c, hipStream_t st) {
   const dim3 gc = chunk_grid(c.rows / LK + c.nseq, a.H), gs(c.nseq, a.H);
   const dim3 gz(c.nseq, a.H, (c.DP * c.UW / 4 + 255) / 256);
-  // 512 threads take 2048 tokens at once, 256 take 1024.  Some sequence needs a second pass of 256 where the rows
-  // are more than 1024 per sequence: the whole op at 4 x 2000 tokens 142 -> 139 us, 1 x 4096 79 -> 73 us with 512;
-  // 1 x 500 39.6 -> 40.3 us.
-  if (a.mode == 1 && c.rows > 1024L * c.nseq)
-    hipLaunchKernelGGL((ls_gates_kernel<T, 512>), gs, dim3(512), 0, st, a, c);
-  else if (a.mode == 1)
-    hipLaunchKernelGGL((ls_gates_kernel<T, 256>), gs, dim3(256), 0, st, a, c);
   if (ROT) {
     const long u = (long)c.rows * (a.rot_dims >> 1);
     hipLaunchKernelGGL(ls_angles_kernel, dim3((unsigned)((u + 255) / 256)), dim3(256), 0, st, a, c);
@@ -1485,19 +1507,19 @@ static void ls_chunked_forms(const ScanArgs& a, const KChunkArgs& c, hipStream_t
 }
 
 // Modes 0 and 1 for steps with prompt portions (cu given; rows: at least cu[nseq]): fp32 workspaces
-// U [rows / 128 + nseq, H, DP, UW] and G [rows / 128 + nseq, H] with DP and VP = dk and dv rounded up
-// to 16, UW = VP + 4 mode; la, lb, nm [rows, H] (mode 1); rot [rows, rot_dims] (rotated heads).
+// U [rows / 128 + nseq, H, DP, UW] and G [rows / 128 + nseq, H, 1 + mode] with DP and VP = dk and dv rounded up
+// to 16, UW = VP + 4 mode; m0 [rows / 128 + nseq, H] (mode 1); rot [rows, rot_dims] (rotated heads).
 EIA_API int eia_linear_scan_chunked(const void* x, long ld, int q_off, int k_off, int v_off, int g_off,
                                     int i_off, int f_off, const float* decay, const float* inv_freq,
                                     int rot_dims, int rot_half, float qscale, float kscale, float cap,
                                     float out_scale, const void* norm_w, float* S, float* N, float* M,
                                     const int* slots, const int* cu, const int* positions, void* y,
                                     long ldy, float eps, int nseq, int rows, int H, int D, int Dv,
-                                    int mode, int gate_act, int norm_h, float* U, float* G, float* la,
-                                    float* lb, float* nm, float* rot, int is_bf16, hipStream_t st) {
+                                    int mode, int gate_act, int norm_h, float* U, float* G, float* m0,
+                                    float* rot, int is_bf16, hipStream_t st) {
   if (nseq < 0 || rows < 0 || H < 1 || D < 1 || Dv < 1 || !x || !y || !S || !slots || !cu ||
       !positions || !U || !G || (mode != 0 && mode != 1) || (mode == 0 && !decay) ||
-      (mode == 1 && (!N || !M || cap < 0.f || !la || !lb || !nm)) || rot_dims < 0 || rot_dims > D ||
+      (mode == 1 && (!N || !M || cap < 0.f || !m0)) || rot_dims < 0 || rot_dims > D ||
       (rot_dims & 1) || (rot_dims && (!inv_freq || !rot)) || (gate_act != 0 && gate_act != 1))
     return EIA_BAD_SHAPE;
   if (D > 128 || Dv > 128 || H > 65535) return EIA_UNSUPPORTED;
@@ -1506,7 +1528,7 @@ EIA_API int eia_linear_scan_chunked(const void* x, long ld, int q_off, int k_off
              qscale, kscale, cap, out_scale, norm_w, S, N, M, slots, cu, positions, nullptr, y,
              ldy, eps, H, D, Dv, mode, gate_act, 0, 0, nullptr, nullptr, 1.f, norm_h};
   const int DP = (D + 15) / 16 * 16, VP = (Dv + 15) / 16 * 16;
-  KChunkArgs c{U, G, la, lb, nm, reinterpret_cast<float2*>(rot), nseq, rows, DP, VP, VP + 4 * mode};
+  KChunkArgs c{U, G, m0, nullptr, reinterpret_cast<float2*>(rot), nseq, rows, DP, VP, VP + 4 * mode};
   if (is_bf16) ls_chunked_forms<bf16_t>(a, c, st); else ls_chunked_forms<float>(a, c, st);
   EIA_LAUNCH_CHECK();
 }
@@ -2250,7 +2272,7 @@ EIA_API int eia_linear_scan_channels64(const void* x, long ld, int q_off, int k_
   ScanArgs a{x, ld, q_off, k_off, v_off, g_off, 0, 0, nullptr, inv_freq, rot_dims, rot_half,
              qscale, kscale, 0.f, out_scale, norm_w, S, nullptr, nullptr, slots, cu, positions,
              nullptr, y, ldy, eps, H, D, Dv, 2, gate_act, lo_off, R, a2t, a2b, inv_tau, norm_h};
-  KChunkArgs c{U, L, l, nullptr, nullptr, reinterpret_cast<float2*>(rot), nseq, rows, GD, Dv, Dv};
+  KChunkArgs c{U, L, nullptr, l, reinterpret_cast<float2*>(rot), nseq, rows, GD, Dv, Dv};
   if (is_bf16) gl_forms<bf16_t>(a, c, st); else gl_forms<float>(a, c, st);
   EIA_LAUNCH_CHECK();
 }

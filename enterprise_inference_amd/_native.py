@@ -82,7 +82,7 @@ _SIGNATURES = {
                         P, L, F, I, I, I, I, I, I, I, I, P, P, F, I, I, S],
     "eia_moe_finish": [P, L, P, L, P, P, L, P, I, P, P, L, I, I, I, S],
     "eia_linear_scan_chunked": [P, L, I, I, I, I, I, I, P, P, I, I, F, F, F, F, P, P, P, P, IP, IP,
-                                IP, P, L, F, I, I, I, I, I, I, I, I, P, P, P, P, P, P, I, S],
+                                IP, P, L, F, I, I, I, I, I, I, I, I, P, P, P, P, I, S],
     "eia_linear_scan_channels": [P, L, I, I, I, I, P, I, I, F, F, F, P, P, IP, IP, IP, P, L, F, I,
                                  I, I, I, I, I, IP, IP, I, P, P, I, I, P, P, F, P, I, S],
     "eia_linear_scan_channels64": [P, L, I, I, I, I, P, I, I, F, F, F, P, P, IP, IP, IP, P, L, F, I,

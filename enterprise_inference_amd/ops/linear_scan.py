@@ -341,8 +341,7 @@ def linear_scan(fused: torch.Tensor, q_off: int, k_off: int, v_off: int, g_off: 
         # (these chunks are longer than the plan's and found on the device)
         n, up16 = T // HEAD_CHUNK + nseq, lambda v: -(-v // 16) * 16
         U = f32(n, H, up16(D), up16(Dv) + (4 if exp_gates else 0))
-        G = f32(n, H)
-        la, lb, nm = (f32(T, H), f32(T, H), f32(T, H)) if exp_gates else (None, None, None)
+        G, m0 = (f32(n, H, 2), f32(n, H)) if exp_gates else (f32(n, H), None)
         rot = f32(T, spec.rot_dims) if spec.rot_dims else None
         check(lib().eia_linear_scan_chunked(
             ptr(fused), fused.stride(0), q_off, k_off, v_off, g_off, i_off, f_off,
@@ -350,7 +349,7 @@ def linear_scan(fused: torch.Tensor, q_off: int, k_off: int, v_off: int, g_off: 
             float(spec.qscale), float(spec.kscale), float(spec.cap), float(spec.out_scale),
             ptr(norm_w), ptr(state.S), ptr(state.n), ptr(state.m), ptr(slots), ptr(cu),
             ptr(positions), ptr(out), out.stride(0), float(spec.eps), nseq, T, H, D, Dv, mode, act,
-            chan[-1], ptr(U), ptr(G), ptr(la), ptr(lb), ptr(nm), ptr(rot), 1 if bf else 0,
+            chan[-1], ptr(U), ptr(G), ptr(m0), ptr(rot), 1 if bf else 0,
             stream(fused)), "linear_scan_chunked")
         return out
     check(lib().eia_linear_scan(

@@ -136,6 +136,44 @@ def test_gates_over_several_passes(lens, monkeypatch):
     test_linear_chunks(lens, 2, 16, 16, "exp_gates", 0, True, torch.float32, monkeypatch)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("lens", [[300, 128, 63, 65], [64, 129, 1, 400]])
+def test_gates_that_shut(lens, dtype, monkeypatch):
+    """Tokens, and whole chunks, that add nothing (an input gate of -inf), before and behind others, and tokens that
+    forget almost everything: the maximum of a chunk's own gates is then none, or lies far below the one carried in."""
+    from enterprise_inference_amd.ops import linear_scan as ls
+    monkeypatch.setattr(ls, "FORCE_CHUNKED", True)
+    H, D, Dv, n, T = 3, 32, 64, len(lens), sum(lens)
+    g = torch.Generator().manual_seed(T)
+    cu, pos, slots = _step(lens, [0, 5, 0, 7], False)
+    at = [0, H * D, 2 * H * D, 2 * H * D + H * Dv, 2 * H * (D + Dv), 2 * H * (D + Dv) + H]
+    x = torch.randn(T, at[-1] + H, generator=g)
+    x[:, at[5]:] += 3.0
+    x[::7, at[5]] = -30.0                                  # forgets
+    x[3::5, at[4] + 1] = float("-inf")                     # adds nothing
+    for lo in cu[:-1].tolist():
+        x[lo:lo + 2, at[4]:at[5]] = float("-inf")          # nor do the first two
+    x[cu[0] + 128:cu[0] + 256, at[4] + 2] = float("-inf")  # nor does a chunk of the first sequence, head 2
+    x = x.to(dtype)
+
+    def run(dev):
+        spec = ls.ScanSpec(H, D, Dv, "exp_gates", kscale=D ** -0.5, eps=1e-5)
+        st = ls.ScanState.allocate(n, spec, "cpu")
+        gs = torch.Generator().manual_seed(1)
+        for t in (st.S, st.n, st.m):
+            t.copy_(torch.randn(t.shape, generator=gs))
+        st = ls.ScanState(*(t.to(dev) for t in (st.S, st.n, st.m)))
+        plan = ls.chunk_plan(lens, dev) if dev == "cuda" else None
+        y = ls.linear_scan(x.to(dev), at[0], at[1], at[2], at[3], spec, st, slots.to(dev), cu.to(dev), n, pos.to(dev),
+                           None, None, at[4], at[5], plan=plan)
+        return y.cpu(), st
+
+    (y, a), (z, b) = run("cpu"), run("cuda")
+    assert torch.isfinite(y).all() and _rel(z, y) < (1e-5 if dtype == torch.float32 else 4e-3)      # as above
+    for u, v in ((a.S, b.S), (a.n, b.n), (a.m, b.m)):
+        assert _rel(v, u) < 2e-6
+
+
 def _stays_not_finite(y, z, H, col, hit):
     """What the recurrence (y) leaves not finite does not come out as a number (z), and where both are numbers they are
     the same.  col: an infinite value is one number of its column, (q . k) v, in sums over tokens, and a sum of infinities of

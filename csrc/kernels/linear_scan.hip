@@ -455,13 +455,16 @@ EIA_API int eia_linear_scan(const void* x, long ld, int q_off, int k_off, int v_
 // traffic (4 passes over chunks x H x dk x dv floats), and halving their number costs less than the
 // longer sums inside a chunk add.
 // Four prompts of 1000 .. 2000 tokens (6688 rows), 16 heads of 128, mode 1, bf16 take 35 + 21 +
-// 59 us on an MI355X ((1), (2), (3)); in fp32 products (1) and (3) took 57 + 103 us.  Bound by the
-// workspace and the rows, which (1), (2) and (3) move at 3.3, 5.4 and 3.3 TB/s, and by the steps of
-// a workgroup, which reads, splits and multiplies in turn.  All heads of a chunk run side by side in (1) and (3), so
+// 57 us on an MI355X ((1), (2), (3)); in fp32 products (1) and (3) took 57 + 103 us.  Bound by the
+// workspace and the rows, which (1), (2) and (3) move at 3.3, 5.4 and 3.4 TB/s, and by the steps of
+// a workgroup, which reads, splits and multiplies in turn: half of (3)'s wave cycles wait, and vector instructions
+// fill 0.4 of the others.  All heads of a chunk run side by side in (1) and (3), so
 // that whole rows are read together, and (3) asks for its queries before it waits for the gates: 135 -> 129 us for the
 // op; three rotated prompts of up to 2700 tokens 188 -> 178, five of up to 1100 of 32 heads of 64 78 -> 77.  What the
 // normaliser, the norm and the gate read is asked for at once (four rounds behind each other: 129 -> 124 us, 178 -> 177,
-// 77 -> 76).  (1) asks for unrotated rows a half ahead, the first before it waits for the gates (33.2 -> 30.0 us, before it
+// 77 -> 76).  (3) asks for unrotated keys and values before the last products of the state, and forms what is one number
+// a token in one lane of the sixteen that hold it (61.4 -> 57.0 us; the op, eight heads, 4000 tokens 47.0 -> 45.3, four
+// rotated prompts of up to 2000 173 -> 168).  Asking for the gates before the last products spills: 64 us.  (1) asks for unrotated rows a half ahead, the first before it waits for the gates (33.2 -> 30.0 us, before it
 // formed the gates itself).
 constexpr int LK = 128;                     // tokens per chunk
 constexpr float LS_LOG2E = 1.4426950408889634f;
@@ -1231,6 +1234,27 @@ EIA_DEV bool ls_out_bf16(const ScanArgs& a, const KChunkArgs& c, const LsChunk& 
     return mfma_bf16_k32(x[0], y[0], z);
   };
   const float pq = k.pre[tq];
+  // keys and values of unrotated rows are on their way during the last products of the state
+  constexpr bool AHEAD = VEC && !ROT;
+  constexpr int NV = LK * MX / 16 / 512, NK = 2 * NV, UT = 512 / (MX / 8);
+  const int vt = threadIdx.x / (MX / 16), vu = threadIdx.x % (MX / 16);          // a thread's first value row, its columns
+  const int kt = threadIdx.x / (MX / 8), ki = 8 * (threadIdx.x % (MX / 8));
+  bf16x8 vr[AHEAD ? NV : 1][2], kr[AHEAD ? NK : 1];
+  auto ahead = [&] {
+    if constexpr (AHEAD) {
+      const bf16_t* xv = X0 + a.v_off + (long)h * a.Dv;
+      const bf16_t* xk = X0 + a.k_off + (long)h * D + (ki < D ? ki : 0);
+#pragma unroll
+      for (int u = 0; u < NV; ++u) {
+        const bf16_t* p = xv + (long)min(vt + 2 * UT * u, n - 1) * a.ld;
+        vr[u][0] = *reinterpret_cast<const bf16x8*>(p + (16 * vu < a.Dv ? 16 * vu : 0));
+        vr[u][1] = *reinterpret_cast<const bf16x8*>(p + (16 * vu + 8 < a.Dv ? 16 * vu + 8 : 0));
+      }
+#pragma unroll
+      for (int u = 0; u < NK; ++u) kr[u] = *reinterpret_cast<const bf16x8*>(xk + (long)min(kt + UT * u, n - 1) * a.ld);
+    }
+  };
+  if (!state) ahead();
   if (state) {
 #pragma unroll
     for (int x = 0; x < MX / 64; ++x) {
@@ -1249,6 +1273,7 @@ EIA_DEV bool ls_out_bf16(const ScanArgs& a, const KChunkArgs& c, const LsChunk& 
         }
       }
       if (x + 1 < MX / 64) fetch(x + 1);               // (on its way during these products)
+      else ahead();
       __syncthreads();
       if (t0 >= n) continue;
 #pragma unroll
@@ -1284,44 +1309,55 @@ EIA_DEV bool ls_out_bf16(const ScanArgs& a, const KChunkArgs& c, const LsChunk& 
     __syncthreads();                                   // the state was read
   }
 #pragma unroll
-  for (int u = threadIdx.x; u < LK * MX / 16; u += 512) {          // values: sixteen columns of a row
-    const int t = u / (MX / 16), cu = u % (MX / 16);
+  for (int u = 0; u < NV; ++u) {                       // values: sixteen columns of a row
+    const int t = vt + 2 * UT * u;
     bf16x8 v0, v1;
-    const bf16_t* p = X0 + (long)min(t, n - 1) * a.ld + a.v_off + (long)h * a.Dv;
     if constexpr (VEC) {
       const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
-      v0 = *reinterpret_cast<const bf16x8*>(p + (16 * cu < a.Dv ? 16 * cu : 0));
-      v1 = *reinterpret_cast<const bf16x8*>(p + (16 * cu + 8 < a.Dv ? 16 * cu + 8 : 0));
-      if (t >= n || 16 * cu >= a.Dv) v0 = zero;
-      if (t >= n || 16 * cu + 8 >= a.Dv) v1 = zero;
+      if constexpr (AHEAD) {
+        v0 = vr[u][0];
+        v1 = vr[u][1];
+      } else {
+        const bf16_t* p = X0 + (long)min(t, n - 1) * a.ld + a.v_off + (long)h * a.Dv;
+        v0 = *reinterpret_cast<const bf16x8*>(p + (16 * vu < a.Dv ? 16 * vu : 0));
+        v1 = *reinterpret_cast<const bf16x8*>(p + (16 * vu + 8 < a.Dv ? 16 * vu + 8 : 0));
+      }
+      if (t >= n || 16 * vu >= a.Dv) v0 = zero;
+      if (t >= n || 16 * vu + 8 >= a.Dv) v1 = zero;
     } else {
+      const bf16_t* p = X0 + (long)min(t, n - 1) * a.ld + a.v_off + (long)h * a.Dv;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        v0[e] = t < n && 16 * cu + e < a.Dv ? p[16 * cu + e] : (bf16_t)0.f;
-        v1[e] = t < n && 16 * cu + 8 + e < a.Dv ? p[16 * cu + 8 + e] : (bf16_t)0.f;
+        v0[e] = t < n && 16 * vu + e < a.Dv ? p[16 * vu + e] : (bf16_t)0.f;
+        v1[e] = t < n && 16 * vu + 8 + e < a.Dv ? p[16 * vu + 8 + e] : (bf16_t)0.f;
       }
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      *reinterpret_cast<bf16x4*>(sv + t * PITCH + ls_col16<MX>(cu) + 16 * j) = bf16x4{v0[j], v0[4 + j], v1[j], v1[4 + j]};
+      *reinterpret_cast<bf16x4*>(sv + t * PITCH + ls_col16<MX>(vu) + 16 * j) = bf16x4{v0[j], v0[4 + j], v1[j], v1[4 + j]};
   }
 #pragma unroll
-  for (int u = threadIdx.x; u < LK * MX / 8; u += 512) {
-    const int t = u / (MX / 8), i = 8 * (u % (MX / 8));
-    float v[8];
-    ls_head8<bf16_t, VEC, ROT>(a, c, row0 + min(t, n - 1), a.k_off + (long)h * D, i, v);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = t < n ? v[e] : 0.f;
-    if constexpr (ROT) {
-      bf16x8 part[3];
-      split3(v, part);
-#pragma unroll
-      for (int p = 0; p < 3; ++p) *reinterpret_cast<bf16x8*>(sk + p * L::KPLANE + ls_kat<MX, bf16_t>(t, i)) = part[p];
+  for (int u = 0; u < NK; ++u) {
+    const int t = kt + UT * u;
+    if constexpr (AHEAD) {
+      if (t >= n || ki >= D) kr[u] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+      *reinterpret_cast<bf16x8*>(sk + ls_kat<MX, bf16_t>(t, ki)) = kr[u];
     } else {
-      bf16x8 b;
+      float v[8];
+      ls_head8<bf16_t, VEC, ROT>(a, c, row0 + min(t, n - 1), a.k_off + (long)h * D, ki, v);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) b[e] = (bf16_t)v[e];
-      *reinterpret_cast<bf16x8*>(sk + ls_kat<MX, bf16_t>(t, i)) = b;
+      for (int e = 0; e < 8; ++e) v[e] = t < n ? v[e] : 0.f;
+      if constexpr (ROT) {
+        bf16x8 part[3];
+        split3(v, part);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) *reinterpret_cast<bf16x8*>(sk + p * L::KPLANE + ls_kat<MX, bf16_t>(t, ki)) = part[p];
+      } else {
+        bf16x8 b;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) b[e] = (bf16_t)v[e];
+        *reinterpret_cast<bf16x8*>(sk + ls_kat<MX, bf16_t>(t, ki)) = b;
+      }
     }
   }
   __syncthreads();
@@ -1413,8 +1449,6 @@ ls_chunk_out_kernel(ScanArgs a, KChunkArgs c) {
   }
   if (a.mode == 1 && threadIdx.x == n - 1 && row0 + n == a.cu[s + 1]) a.M[(long)a.slots[s] * a.H + h] = mx[n - 1];
   if (t0 >= n) return;
-  rs += __shfl_xor(rs, 16, 64);                        // n_t . q_t of query l16
-  rs += __shfl_xor(rs, 32, 64);
   const T* X = static_cast<const T*>(a.x);
   const T* NW = static_cast<const T*>(a.norm_w);
   T* Y = static_cast<T*>(a.y);
@@ -1423,11 +1457,10 @@ ls_chunk_out_kernel(ScanArgs a, KChunkArgs c) {
   T4 gt[4][MX / 64], nw[MX / 64];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const long row = row0 + min(t0 + 4 * g4 + i, n - 1);
+    const T* gp = X + (row0 + min(t0 + 4 * g4 + i, n - 1)) * a.ld + a.g_off + (long)h * Dv;
 #pragma unroll
     for (int x = 0; x < MX / 64; ++x) {
       const int d = 64 * x + 4 * l16;
-      const T* gp = X + row * a.ld + a.g_off + (long)h * Dv;
       if constexpr (VEC) gt[i][x] = *reinterpret_cast<const T4*>(gp + (d < Dv ? d : 0));
       else {
 #pragma unroll
@@ -1440,22 +1473,33 @@ ls_chunk_out_kernel(ScanArgs a, KChunkArgs c) {
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       nw[x][j] = NW ? NW[(long)h * a.norm_h + min(64 * x + 4 * l16 + j, Dv - 1)] : (T)1.f;
+  // normaliser, head RMS norm, weight, gate.  What is one number a token is formed by one lane of the sixteen that
+  // hold it.
+  float ss[4], den = 1.f;
+  if (a.mode == 1) {
+    rs += __shfl_xor(rs, 16, 64);                      // n_t . q_t of query l16
+    rs += __shfl_xor(rs, 32, 64);
+    den = 1.0f / (fmaxf(fabsf(rs), expf(-mx[min(t0 + l16, n - 1)])) + 1e-6f);
+  }
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {                        // normaliser, head RMS norm, weight, gate
-    const int t = t0 + 4 * g4 + i;
-    const float nqi = __shfl(rs, 4 * g4 + i, 64);
-    float den = 1.f;
-    if (a.mode == 1) den = 1.0f / (fmaxf(fabsf(nqi), expf(-mx[min(t, n - 1)])) + 1e-6f);
-    float ss = 0.f;
+  for (int i = 0; i < 4; ++i) {
+    const float di = a.mode == 1 ? __shfl(den, 4 * g4 + i, 64) : 1.f;
+    ss[i] = 0.f;
 #pragma unroll
     for (int j = 0; j < MX / 16; ++j) {
       const bool col = 64 * (j >> 2) + 4 * l16 + (j & 3) < Dv;
-      o[j][i] = col ? o[j][i] * den : 0.f;             // (padded columns read column 0 of S)
-      ss += o[j][i] * o[j][i];
+      o[j][i] = col ? o[j][i] * di : 0.f;              // (padded columns read column 0 of S)
+      ss[i] += o[j][i] * o[j][i];
     }
-    ss = row16_sum(ss);
+    ss[i] = row16_sum(ss[i]);
+  }
+  const float lo = l16 & 1 ? ss[1] : ss[0], hi = l16 & 1 ? ss[3] : ss[2];
+  const float mine = a.out_scale / sqrtf((l16 & 2 ? hi : lo) / (float)Dv + a.eps);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int t = t0 + 4 * g4 + i;
+    const float inv = __shfl(mine, 16 * g4 + i, 64);
     if (t >= n) continue;
-    const float inv = a.out_scale / sqrtf(ss / (float)Dv + a.eps);
 #pragma unroll
     for (int x = 0; x < MX / 64; ++x) {
       const int d = 64 * x + 4 * l16;

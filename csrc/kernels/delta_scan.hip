@@ -230,10 +230,10 @@ EIA_API int eia_delta_scan(const float* q, const float* k, const float* v, const
 //   X  [chunk, H, 4 token tiles, VP / 16 tiles]       fp32, B operand, rows tokens
 //   O  [chunk, 64, H, VP]                             fp32, outputs before their norm
 // with DP rounded up to 64 and VP to 32; tile j of 32 columns holds columns 2 x + j.
-// MI355X, 16 heads of 128 x 128 on 8, three prompts of 750 to 1500 tokens: 59 + 69 + 19 us
+// MI355X, 16 heads of 128 x 128 on 8, three prompts of 750 to 1500 tokens: 51 + 69 + 17 us
 // ((1), (2), (3)).  Before, with fp32 products and the states between chunks and u in memory for a kernel that formed
 // the outputs, 48 + 77 + 83 (the op: 197 -> 147).  S against 64 bits: 1.2e-7 .. 1.5e-7 where fp32 products left 1.3e-7 .. 1.6e-7.
-// (1) and (3) are bound by their writes and reads (3.4, 3.7 TB/s), (2) by the chain of its chunks: 6000 cycles
+// (1) and (3) are bound by their writes and reads (3.0, 3.4 TB/s), (2) by the chain of its chunks: 6000 cycles
 // each, of which matrix products take 2700 of a SIMD's.
 constexpr int DC = 64;                      // tokens per chunk
 constexpr int DL = DC + 4;                  // LDS row pitch of the triangular blocks
@@ -244,7 +244,7 @@ struct DeltaChunkArgs {
   bf16_t *Y, *Kt, *Qt, *P; float *X, *O;    // as above
   float* cA;                                // [nchunk, H, 2, DC] exp(A_t), exp(A_end - A_t); A constant past the end
   int ncu, nseq;                            // units of 32 state columns
-  int parts;                                // workgroups of (1) that share a key head's heads
+  int whole, parts;                         // the workgroups of (1): dn_solve
   DeltaSpread spread;                       // the workgroups of (2) over the XCDs
   int vec;                                  // out, gate and weight rows can be taken 4 at a time
 };
@@ -343,7 +343,7 @@ EIA_DEV bool all_finite(f32x4 v) {
   return ok;
 }
 
-// (1) one workgroup per (chunk, key head, part of its heads: dn_parts), those heads in turn.  K is staged in LDS in parts: the triangle and P
+// (1) one workgroup per (chunk, key head, part of its heads: dn_solve), those heads in turn.  K is staged in LDS in parts: the triangle and P
 // take it by rows, Y and Kt by columns (transposing reads).  Waves 0 .. 3 form the triangle, its inverse and Y,
 // a token tile each; waves 4 .. 7 meanwhile P, and then X in units of 32 columns.  k . k and q . k are
 // formed once for all heads.  X takes fp32 products: a value that is not finite stays in its column and out
@@ -357,12 +357,12 @@ delta_chunk_solve_kernel(DeltaArgs a, DeltaChunkArgs c) {
   __shared__ __align__(16) bf16_t ks[3 * PLANE];
   __shared__ __align__(16) float Ls[DC][DL];           // -L, then T
   __shared__ __align__(16) float sAs[DHB][DC], sbs[DHB][DC], sfs[DHB][DC];
-  const int ch = blockIdx.y, kh = blockIdx.x / c.parts, part = blockIdx.x % c.parts, tid = threadIdx.x, lane = tid & 63;
+  const DeltaSolveWg wg = dn_solve_place(blockIdx.x, a.G, c.whole, c.parts);
+  const int ch = wg.chunk, kh = wg.kh, part = wg.part, tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), w = wave & 3;
-  const int s = c.chunks[4 * ch], row0 = c.chunks[4 * ch + 1], n = c.chunks[4 * ch + 2];
-  if (a.slots[s] < 0) return;
+  const int row0 = c.chunks[4 * ch + 1], n = c.chunks[4 * ch + 2], slot = a.slots[c.chunks[4 * ch]];
   const int H = a.H, G = a.G, DP = a.DP, VP = a.VP, rep = H / G;
-  const int x0 = dn_first_head(rep, c.parts, part), nh = dn_first_head(rep, c.parts, part + 1) - x0, h0 = kh * rep + x0;
+  const int x0 = dn_first_head(rep, wg.parts, part), nh = dn_first_head(rep, wg.parts, part + 1) - x0, h0 = kh * rep + x0;
   const int g4 = lane >> 4, l16 = lane & 15;
   const long ldk = (long)G * DP, ldv = (long)H * VP;
   const float* K = a.k + (long)row0 * ldk + (long)kh * DP;
@@ -392,6 +392,7 @@ delta_chunk_solve_kernel(DeltaArgs a, DeltaChunkArgs c) {
 #pragma unroll
     for (int p = 0; p < 3; ++p) *reinterpret_cast<bf16x8*>(ks + p * PLANE + r * KP + d) = f.p[p];
   }
+  if (slot < 0) return;                                // (whole workgroup; the rows did not wait for it)
   __syncthreads();
   auto k_rows = [&](int t, int b) {                    // 32 dk of a token tile's rows, in order
     Parts f;
@@ -966,17 +967,20 @@ delta_chunk_scan_kernel(DeltaArgs a, DeltaChunkArgs c) {
 
 // (3) Norm, weight and gate of the outputs: LN lanes per token and head, two heads each; the heads come first in the
 // grid, so that those of a key head run on the XCD that formed them where G is eight.  Bound by memory.  (Four heads, chunks
-// first: three prompts of 155 tokens, 8 heads 32.9 -> 30.8 us, three of up to 1500, 16 heads 146.0 -> 145.2.)
+// first: three prompts of 155 tokens, 8 heads 32.9 -> 30.8 us, three of up to 1500, 16 heads 146.0 -> 145.2.)  Of bf16
+// outputs, whose rounding is 2^-9, the root and silu take the instructions' own reciprocal and exponential (1 ulp, some
+// 2^-21): with divisions and expf vector instructions filled 13 of 19.2 us, now the kernel takes 16.6; error of the
+// outputs against 64 bits 1.7e-3 as before.
 constexpr int DN_HEADS = 2;
 template <typename T, int LN>
 __global__ void __launch_bounds__(256)
 delta_chunk_norm_kernel(DeltaArgs a, DeltaChunkArgs c) {
   constexpr int NH = DN_HEADS;
   const int ch = blockIdx.y, sub = threadIdx.x % LN, t = blockIdx.z * (256 / LN) + threadIdx.x / LN;
-  const int s = c.chunks[4 * ch], row0 = c.chunks[4 * ch + 1], n = c.chunks[4 * ch + 2];
-  if (a.slots[s] < 0 || t >= n) return;
+  // no branch before the store: the outputs are asked for beside the chunk, the gates beside its slot
+  const int row0 = c.chunks[4 * ch + 1], n = c.chunks[4 * ch + 2], slot = a.slots[c.chunks[4 * ch]];
   const int col = 4 * sub, Dv = a.Dv, VQ = 32 * c.ncu;
-  const long r = row0 + t;
+  const long r = row0 + min(t, n - 1);
   f32x4 o[NH];
   float gv[NH][4], nw[4];
   const T* GT = static_cast<const T*>(a.g) + r * a.ldg;
@@ -1008,12 +1012,15 @@ delta_chunk_norm_kernel(DeltaArgs a, DeltaChunkArgs c) {
     for (int j = 0; j < 4; ++j) sq += col + j < Dv ? o[x][j] * o[x][j] : 0.f;
 #pragma unroll
     for (int b = 1; b < LN; b <<= 1) sq += __shfl_xor(sq, b, 64);
-    const float inv = 1.0f / sqrtf(sq / (float)Dv + a.eps);
-    if (h >= a.H || col >= Dv) continue;
+    const float ms = sq / (float)Dv + a.eps, inv = sizeof(T) == 2 ? __builtin_amdgcn_rsqf(ms) : 1.0f / sqrtf(ms);
+    if (slot < 0 || t >= n || h >= a.H || col >= Dv) continue;
     T* yp = static_cast<T*>(a.y) + r * a.ldy + (long)h * Dv + col;
     T v[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) st_f32<T>(v, j, o[x][j] * inv * nw[j] * dl_silu(gv[x][j]));
+    for (int j = 0; j < 4; ++j) {
+      const float z = gv[x][j], silu = sizeof(T) == 2 ? z * __builtin_amdgcn_rcpf(1.0f + __expf(-z)) : dl_silu(z);
+      st_f32<T>(v, j, o[x][j] * inv * nw[j] * silu);
+    }
     if (c.vec) {
       typedef T T4 __attribute__((ext_vector_type(4)));
       *reinterpret_cast<T4*>(yp) = T4{v[0], v[1], v[2], v[3]};
@@ -1053,9 +1060,10 @@ EIA_API int eia_delta_scan_chunked(const float* q, const float* k, const float* 
   const int ndg = (DP + 63) / 64, ncu = (VP + 31) / 32, es = is_bf16 ? 2 : 4;
   const bool vec = Dv % 4 == 0 && ldy % 4 == 0 && ldg % 4 == 0 &&
                    (reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(g)) % (4 * es) == 0;
+  const DeltaSolve solve = dn_solve(G, nchunk, H / G);
   DeltaChunkArgs c{chunks, seq_first, static_cast<bf16_t*>(Y), static_cast<bf16_t*>(Kt), static_cast<bf16_t*>(Qt),
-                   static_cast<bf16_t*>(P), X, O, cA, ncu, nseq, dn_parts(G * (long)nchunk, H / G), {}, vec};
-  const dim3 gc(G * c.parts, nchunk), b(256);
+                   static_cast<bf16_t*>(P), X, O, cA, ncu, nseq, solve.whole, solve.parts, {}, vec};
+  const dim3 gc((unsigned)solve.blocks), b(256);
   const int nc = dn_columns(nseq * H * ncu);
   c.spread = dn_spread(G, 2 * ncu / nc * (H / G));
   const int grid = dn_grid(nseq * G, c.spread);

@@ -14,6 +14,14 @@ SOURCE = """
 extern "C" {
 int parts(long nwg, int rep) { return dn_parts(nwg, rep); }
 int first_head(int rep, int parts, int part) { return dn_first_head(rep, parts, part); }
+void solve(int G, int nchunk, int rep, long* out) {
+  const DeltaSolve s = dn_solve(G, nchunk, rep);
+  out[0] = s.whole; out[1] = s.parts; out[2] = s.blocks;
+}
+void solve_place(long block, int G, int whole, int parts, int* out) {
+  const DeltaSolveWg w = dn_solve_place(block, G, whole, parts);
+  out[0] = w.chunk; out[1] = w.kh; out[2] = w.parts; out[3] = w.part;
+}
 int xcds(int G, int per_kv) { return 1 << dn_spread(G, per_kv).shift; }
 int grid(int G, int per_kv, int nseq) { return dn_grid(nseq * G, dn_spread(G, per_kv)); }
 int place(int block, int G, int per_kv, int* kv) {
@@ -48,6 +56,28 @@ def test_heads_of_a_key_head(plan, rep):
         assert n == 1 or nwg * n <= 512
         if nwg * rep <= 512:
             assert n == rep
+
+
+@pytest.mark.parametrize("rep", [1, 2, 3, 8])
+@pytest.mark.parametrize("G", [1, 3, 7, 8, 16, 513])
+@pytest.mark.parametrize("nchunk", [1, 2, 63, 64, 65, 66, 170, 171, 172, 300])
+def test_workgroups_of_the_solve(plan, nchunk, G, rep):
+    """Every head of every chunk once; heads are spread in the last round of 512 workgroups only."""
+    out, wg = (ctypes.c_long * 3)(), (ctypes.c_int * 4)()
+    plan.solve(G, nchunk, rep, out)
+    whole, parts, blocks = out
+    assert 0 <= whole <= nchunk and whole * G <= G * nchunk // 512 * 512
+    assert G * (nchunk - whole) * parts <= 512 or parts == 1
+    plan.solve_place.argtypes = [ctypes.c_long, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p]
+    heads = set()
+    for b in range(blocks):
+        plan.solve_place(b, G, whole, parts, wg)
+        chunk, kh, n, part = wg
+        assert 0 <= chunk < nchunk and 0 <= kh < G and 0 <= part < n
+        mine = {(chunk, kh, h) for h in range(plan.first_head(rep, n, part), plan.first_head(rep, n, part + 1))}
+        assert mine and not mine & heads
+        heads |= mine
+    assert len(heads) == nchunk * G * rep
 
 
 @pytest.mark.parametrize("per_kv", [1, 2, 3, 8, 15, 16, 32, 64, 128])

@@ -21,12 +21,29 @@ def use_hip(*tensors: torch.Tensor) -> bool:
     """True when the HIP kernels must be used for these tensors."""
     if FORCE_TORCH:
         return False
-    return all(t is None or t.is_cuda for t in tensors) and any(
-        t is not None and t.is_cuda for t in tensors)
+    hip = False
+    for t in tensors:
+        if t is not None:
+            if not t.is_cuda:
+                return False
+            hip = True
+    return hip
 
 
 def ptr(t):
     return None if t is None else t.data_ptr()
+
+
+def workspace(device, *sizes: int):
+    """One allocation of so many bytes each, at multiples of 512 bytes -> (the tensor that owns it, addresses).  An
+    allocation costs the host 1.3 us, and small steps are bound by their launches."""
+    at, total = [], 0
+    for n in sizes:
+        at.append(total)
+        total += -(-n // 512) * 512
+    ws = torch.empty(total, dtype=torch.uint8, device=device)
+    base = ws.data_ptr()
+    return ws, [base + a for a in at]
 
 
 def stream(t: torch.Tensor) -> int:

@@ -406,8 +406,8 @@ def attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
     """Dispatch the step's decode and prefill parts. q [T, Hq, D]."""
     nd = md.num_decode
     if md.num_prefill_tokens == 0:
-        return paged_decode(q[:nd], k_cache, v_cache, md.decode_block_tables, md.decode_seq_lens,
-                            scale, md.decode_partitions, md.decode_part_o, md.decode_part_ml,
+        return paged_decode(q if nd == q.shape[0] else q[:nd], k_cache, v_cache, md.decode_block_tables,
+                            md.decode_seq_lens, scale, md.decode_partitions, md.decode_part_o, md.decode_part_ml,
                             sliding_window=sliding_window, chunk_size=chunk_size,
                             part_cnt=md.decode_part_cnt, p_dyn=md.decode_p_dyn)
     out = torch.empty_like(q)

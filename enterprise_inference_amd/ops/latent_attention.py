@@ -17,7 +17,7 @@ from typing import List, Optional
 
 import torch
 
-from ._dispatch import check, lib, ptr, require, stream, use_hip
+from ._dispatch import check, lib, ptr, require, stream, use_hip, workspace
 from .attention import split_keys
 
 ACC_ROWS = 256 * 32        # csrc/kernels/latent_attention.hip: QB * HB * R <= 256 * LAT_ACC_MAX
@@ -223,8 +223,10 @@ def latent_attention(q_abs: torch.Tensor, q_rot: torch.Tensor, inv_freq: torch.T
     mfma = mfma_ok(R, rd, q_abs.dtype)
 
     def launch(lo, n_items, bt, lens, cu, work, qb):
-        qa, qr, o = q_abs[lo:], q_rot[lo:], out[lo:]
-        g = None if gate is None else gate[lo:]
+        qa, qr, o, g, pos = q_abs, q_rot, out, gate, md.positions
+        if lo:
+            qa, qr, o, pos = q_abs[lo:], q_rot[lo:], out[lo:], pos[lo:]
+            g = None if gate is None else gate[lo:]
         require(bt.dtype == torch.int32 and bt.stride(1) == 1, "block tables int32")
         if mfma and cu is not None:
             KT = lib().eia_latent_flash_keys(R, rd)
@@ -244,7 +246,7 @@ def latent_attention(q_abs: torch.Tensor, q_rot: torch.Tensor, inv_freq: torch.T
             check(lib().eia_latent_flash(
                 ptr(qa), qa.stride(0), qa.stride(1), ptr(qr), qr.stride(0), qr.stride(1),
                 ptr(inv_freq), rot_dims, ptr(cache), cache.shape[-1], ptr(bt), bt.stride(0), ptr(cu),
-                ptr(work), n_items, ptr(md.positions[lo:]), ptr(g),
+                ptr(work), n_items, ptr(pos), ptr(g),
                 g.stride(0) if g is not None else 0, ptr(o), o.stride(0), o.stride(1), float(scale),
                 H, R, rd, bs, window, ptr(sink), rh, amp, P, per, ptr(pa), stream(q_abs)),
                 "latent_flash")
@@ -253,20 +255,19 @@ def latent_attention(q_abs: torch.Tensor, q_rot: torch.Tensor, inv_freq: torch.T
             P = decode_partitions(n_items, H, window=window, wide=R + rd > 288)
             pa = pm = None
             if P > 1:
-                pa = torch.empty(n_items * H * P * R, dtype=torch.float32, device=q_abs.device)
-                pm = torch.empty(n_items * H * P * 2, dtype=torch.float32, device=q_abs.device)
+                ws, (pa, pm) = workspace(q_abs.device, 4 * n_items * H * P * R, 4 * n_items * H * P * 2)
             check(lib().eia_latent_attn_mfma(
                 ptr(qa), qa.stride(0), qa.stride(1), ptr(qr), qr.stride(0), qr.stride(1),
                 ptr(inv_freq), rot_dims, ptr(cache), cache.shape[-1], ptr(bt), bt.stride(0),
-                ptr(lens), n_items, ptr(md.positions[lo:]), ptr(g),
+                ptr(lens), n_items, ptr(pos), ptr(g),
                 g.stride(0) if g is not None else 0, ptr(o), o.stride(0), o.stride(1),
-                float(scale), H, R, rd, bs, window, ptr(sink), rh, amp, P, ptr(pa), ptr(pm),
-                stream(q_abs)), "latent_attn_mfma")
+                float(scale), H, R, rd, bs, window, ptr(sink), rh, amp, P, pa, pm, stream(q_abs)),
+                "latent_attn_mfma")
             return
         check(lib().eia_latent_attn(
             ptr(qa), qa.stride(0), qa.stride(1), ptr(qr), qr.stride(0), qr.stride(1),
             ptr(inv_freq), rot_dims, ptr(cache), cache.shape[-1], ptr(bt), bt.stride(0), ptr(lens),
-            ptr(cu), ptr(work), n_items, ptr(md.positions[lo:]), ptr(g),
+            ptr(cu), ptr(work), n_items, ptr(pos), ptr(g),
             g.stride(0) if g is not None else 0, ptr(o), o.stride(0), o.stride(1), float(scale),
             H, R, rd, bs, qb, window, ptr(sink), rh, amp, 1 if bf else 0, stream(q_abs)),
             "latent_attn")

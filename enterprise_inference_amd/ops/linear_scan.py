@@ -43,7 +43,7 @@ from typing import Optional
 
 import torch
 
-from ._dispatch import check, lib, ptr, require, stream, use_hip
+from ._dispatch import check, lib, ptr, require, stream, use_hip, workspace
 
 
 @dataclasses.dataclass
@@ -314,42 +314,40 @@ def linear_scan(fused: torch.Tensor, q_off: int, k_off: int, v_off: int, g_off: 
             (FORCE_CHUNKED or plan.pays(H, max(D, Dv), channel=channel, key_dim=D, exp_gates=exp_gates))
             and not torch.cuda.is_current_stream_capturing()):
         dev = fused.device
-        f32 = lambda *shape: torch.empty(*shape, dtype=torch.float32, device=dev)
         act = 0 if spec.gate_act == "silu" else 1
         if channel and D <= KEY_DIM64:
             n, W = T // KEY_CHUNK64 + nseq, -(-Dv // 64) * 64
-            U, L, l = f32(n, H, KEY_DIM64, W), f32(n, H, KEY_DIM64), f32(T, H, D)
-            rot = f32(T, spec.rot_dims) if spec.rot_dims else None
+            ws, (U, L, l, rot) = workspace(dev, 4 * n * H * KEY_DIM64 * W, 4 * n * H * KEY_DIM64, 4 * T * H * D,
+                                           4 * T * spec.rot_dims)
             check(lib().eia_linear_scan_channels64(
                 ptr(fused), fused.stride(0), q_off, k_off, v_off, g_off, ptr(spec.inv_freq),
                 spec.rot_dims, 1 if spec.rot_half else 0, float(spec.qscale), float(spec.kscale),
                 float(spec.out_scale), ptr(norm_w), ptr(state.S), ptr(slots), ptr(cu),
                 ptr(positions), ptr(out), out.stride(0), float(spec.eps), nseq, T, H, D, Dv, act,
-                chan[-1], *chan[:-1], ptr(U), ptr(L), ptr(l), ptr(rot), 1 if bf else 0,
+                chan[-1], *chan[:-1], U, L, l, rot if spec.rot_dims else None, 1 if bf else 0,
                 stream(fused)), "linear_scan_channels64")
             return out
         if channel:
-            wsS, wsG, cA = f32(plan.n, H, D, Dv), f32(plan.n, H, D), f32(T, H, D)
+            ws, (wsS, wsG, cA) = workspace(dev, 4 * plan.n * H * D * Dv, 4 * plan.n * H * D, 4 * T * H * D)
             check(lib().eia_linear_scan_channels(
                 ptr(fused), fused.stride(0), q_off, k_off, v_off, g_off, ptr(spec.inv_freq),
                 spec.rot_dims, 1 if spec.rot_half else 0, float(spec.qscale), float(spec.kscale),
                 float(spec.out_scale), ptr(norm_w), ptr(state.S), ptr(slots), ptr(cu),
                 ptr(positions), ptr(out), out.stride(0), float(spec.eps), nseq, H, D, Dv, act,
-                chan[-1], ptr(plan.chunks), ptr(plan.seq_first), plan.n, ptr(wsS), ptr(wsG),
-                *chan[:-1], ptr(cA), 1 if bf else 0, stream(fused)), "linear_scan_channels")
+                chan[-1], ptr(plan.chunks), ptr(plan.seq_first), plan.n, wsS, wsG,
+                *chan[:-1], cA, 1 if bf else 0, stream(fused)), "linear_scan_channels")
             return out
         # (these chunks are longer than the plan's and found on the device)
         n, up16 = T // HEAD_CHUNK + nseq, lambda v: -(-v // 16) * 16
-        U = f32(n, H, up16(D), up16(Dv) + (4 if exp_gates else 0))
-        G, m0 = (f32(n, H, 2), f32(n, H)) if exp_gates else (f32(n, H), None)
-        rot = f32(T, spec.rot_dims) if spec.rot_dims else None
+        ws, (U, G, m0, rot) = workspace(dev, 4 * n * H * up16(D) * (up16(Dv) + (4 if exp_gates else 0)),
+                                        8 * n * H, 4 * n * H, 4 * T * spec.rot_dims)
         check(lib().eia_linear_scan_chunked(
             ptr(fused), fused.stride(0), q_off, k_off, v_off, g_off, i_off, f_off,
             ptr(spec.decay), ptr(spec.inv_freq), spec.rot_dims, 1 if spec.rot_half else 0,
             float(spec.qscale), float(spec.kscale), float(spec.cap), float(spec.out_scale),
             ptr(norm_w), ptr(state.S), ptr(state.n), ptr(state.m), ptr(slots), ptr(cu),
             ptr(positions), ptr(out), out.stride(0), float(spec.eps), nseq, T, H, D, Dv, mode, act,
-            chan[-1], ptr(U), ptr(G), ptr(m0), ptr(rot), 1 if bf else 0,
+            chan[-1], U, G, m0 if exp_gates else None, rot if spec.rot_dims else None, 1 if bf else 0,
             stream(fused)), "linear_scan_chunked")
         return out
     check(lib().eia_linear_scan(

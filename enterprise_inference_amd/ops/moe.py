@@ -26,7 +26,7 @@ import torch
 import torch.nn.functional as F
 
 from . import reference as ref
-from ._dispatch import check, lib, ptr, require, stream, use_hip
+from ._dispatch import check, lib, ptr, require, stream, use_hip, workspace
 
 SCORING = {"softmax": 0, "sigmoid": 1}
 
@@ -274,16 +274,25 @@ def _fused_moe_grouped(x, w13, w2, topk_w, topk_ids, e_lo, e_hi, mfma: bool = Fa
     n = T * k
     dev = x.device
     st = stream(x)
-    offs, row_idx, inv = _align(topk_ids, El, e_lo, e_hi, n, dev, st)
-    h1 = torch.empty(max(1, n), I, dtype=x.dtype, device=dev)
-    h2 = torch.empty(max(1, n), H, dtype=x.dtype, device=dev)
+    m, es = max(1, n), x.element_size()
+    slabs = not mfma and DOWN_SK > 1 and I % (DOWN_SK * 256) == 0
+    inv = part = None
+    if slabs and defer_combine:                      # (these two may go to the caller)
+        inv = torch.empty(m, dtype=torch.int32, device=dev)
+        part = torch.empty(DOWN_SK, m, H, dtype=torch.float32, device=dev)
+    ws, (offs, row_idx, p_inv, h1, h2) = workspace(
+        dev, 4 * (El + 1), 4 * m, 0 if inv is not None else 4 * m, es * m * I,
+        0 if part is not None else 4 * DOWN_SK * m * H if slabs else es * m * H)
+    p_inv = p_inv if inv is None else ptr(inv)
+    p_part = h2 if part is None else ptr(part)
+    _align_into(topk_ids, El, e_lo, e_hi, n, offs, row_idx, p_inv, st)
     if mfma:
         x, w13, w2 = _aligned16(x), _aligned16(w13), _aligned16(w2)
-        check(lib().eia_moe_grouped_gemm(ptr(x), x.stride(0), ptr(row_idx), ptr(w13), I2, H, El,
-                                         ptr(offs), n, 1, ptr(h1), h1.stride(0), st),
+        check(lib().eia_moe_grouped_gemm(ptr(x), x.stride(0), row_idx, ptr(w13), I2, H, El,
+                                         offs, n, 1, h1, I, st),
               "moe_grouped_gemm_gate_up")
-        check(lib().eia_moe_grouped_gemm(ptr(h1), h1.stride(0), None, ptr(w2), H, I, El,
-                                         ptr(offs), n, 0, ptr(h2), h2.stride(0), st),
+        check(lib().eia_moe_grouped_gemm(h1, I, None, ptr(w2), H, I, El,
+                                         offs, n, 0, h2, H, st),
               "moe_grouped_gemm_down")
     else:
         mt = max(1, min(8, -(-int(1.5 * n / El + 1) // 16)))
@@ -295,8 +304,8 @@ def _fused_moe_grouped(x, w13, w2, topk_w, topk_ids, e_lo, e_hi, mfma: bool = Fa
             # weight stream per workgroup
             w_up = packed[(2 if up_cfg == 1 else 4, True)]
             up_cfg |= 1024
-        check(lib().eia_moe_gemm(ptr(x), x.stride(0), ptr(w_up), w13.stride(1), None, ptr(h1),
-                                 h1.stride(0), I2, H, El, ptr(offs), ptr(row_idx), mt, 2,
+        check(lib().eia_moe_gemm(ptr(x), x.stride(0), ptr(w_up), w13.stride(1), None, h1,
+                                 I, I2, H, El, offs, row_idx, mt, 2,
                                  up_cfg, st), "moe_gemm_gate_up")
         w_down = w2
         if packed_down := getattr(w2, "_eia_wg", None):
@@ -305,36 +314,38 @@ def _fused_moe_grouped(x, w13, w2, topk_w, topk_ids, e_lo, e_hi, mfma: bool = Fa
             if wp is not None:       # workgroup-packed expert down (one tile per wave)
                 w_down = wp
                 down_cfg |= 1024
-        if DOWN_SK > 1 and I % (DOWN_SK * 256) == 0:
-            part = torch.empty(DOWN_SK, max(1, n), H, dtype=torch.float32, device=dev)
-            check(lib().eia_moe_gemm_sk(ptr(h1), h1.stride(0), ptr(w_down), w2.stride(1),
-                                        ptr(part), max(1, n), H, I, El, ptr(offs), None, mt,
+        if slabs:
+            check(lib().eia_moe_gemm_sk(h1, I, ptr(w_down), w2.stride(1),
+                                        p_part, m, H, I, El, offs, None, mt,
                                         DOWN_SK, down_cfg, st), "moe_gemm_down_sk")
             if (defer_combine and FUSED_NORMS and k <= 2 and H % 4 == 0 and H <= 8192
                     and DOWN_SK in (1, 2, 4) and x.dtype == torch.bfloat16):
-                return MoECombine(part, DOWN_SK, max(1, n), topk_w, inv, T, k, H)
+                return MoECombine(part, DOWN_SK, m, topk_w, inv, T, k, H)
             out = torch.empty(T, H, dtype=x.dtype, device=dev)
-            check(lib().eia_moe_combine_sk(ptr(part), DOWN_SK, max(1, n), ptr(topk_w), ptr(inv),
+            check(lib().eia_moe_combine_sk(p_part, DOWN_SK, m, ptr(topk_w), p_inv,
                                            T, k, H, ptr(out), out.stride(0), st), "moe_combine_sk")
             return out
-        check(lib().eia_moe_gemm(ptr(h1), h1.stride(0), ptr(w_down), w2.stride(1), None, ptr(h2),
-                                 h2.stride(0), H, I, El, ptr(offs), None, mt, 0,
+        check(lib().eia_moe_gemm(h1, I, ptr(w_down), w2.stride(1), None, h2,
+                                 H, H, I, El, offs, None, mt, 0,
                                  down_cfg, st), "moe_gemm_down")
     out = torch.empty(T, H, dtype=x.dtype, device=dev)
-    check(lib().eia_moe_combine(ptr(h2), h2.stride(0), ptr(topk_w), ptr(inv), T, k, H, ptr(out),
+    check(lib().eia_moe_combine(h2, H, ptr(topk_w), p_inv, T, k, H, ptr(out),
                                 out.stride(0), st), "moe_combine")
     return out
 
 
 def _align(topk_ids, El, e_lo, e_hi, n, dev, st):
-    E_total = max(e_hi, int(El + e_lo))
     offs = torch.empty(El + 1, dtype=torch.int32, device=dev)
-    # with expert parallelism the align kernel scatters only the local rows and zeroes the rest
     row_idx = torch.empty(max(1, n), dtype=torch.int32, device=dev)
     inv = torch.empty(max(1, n), dtype=torch.int32, device=dev)
-    check(lib().eia_moe_align(ptr(topk_ids), n, E_total, e_lo, e_hi, ptr(offs), ptr(row_idx),
-                              ptr(inv), topk_ids.shape[1], st), "moe_align")
+    _align_into(topk_ids, El, e_lo, e_hi, n, ptr(offs), ptr(row_idx), ptr(inv), st)
     return offs, row_idx, inv
+
+
+def _align_into(topk_ids, El, e_lo, e_hi, n, offs, row_idx, inv, st):
+    # with expert parallelism the align kernel scatters only the local rows and zeroes the rest
+    check(lib().eia_moe_align(ptr(topk_ids), n, max(e_hi, int(El + e_lo)), e_lo, e_hi, offs, row_idx, inv,
+                              topk_ids.shape[1], st), "moe_align")
 
 
 def _fused_moe_sorted_blas(x, w13, w2, topk_w, topk_ids, e_lo, e_hi, act):

@@ -79,7 +79,12 @@ def mfma_ok(spec: WindowSpec, dtype: torch.dtype, block_size: int) -> bool:
     multiple of 32 tokens and, with head mixing, at most 16 heads (one workgroup of up to eight
     waves holds them all, one or two heads per wave); everything else (fp32 models too) runs
     the scalar-FMA kernel."""
-    if dtype != torch.bfloat16 or not _MFMA_ENV or not torch.cuda.is_available():
+    return dtype == torch.bfloat16 and torch.cuda.is_available() and _mfma_takes(spec, block_size)
+
+
+def _mfma_takes(spec: WindowSpec, block_size: int) -> bool:
+    """``mfma_ok`` for bf16 rows that are on the GPU."""
+    if not _MFMA_ENV:
         return False
     if spec.talk_post:
         return (spec.maps == 1 and spec.keep == 0 and spec.slope is None and
@@ -566,8 +571,9 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     nd = md.num_decode
     if out is None:
         out = torch.empty(T, H * Dv, dtype=q.dtype, device=q.device)
-    require(out.shape == (T, H * Dv) and out.dtype == q.dtype and out.stride(1) == 1,
-            "window_attention: out layout")
+    else:
+        require(out.shape == (T, H * Dv) and out.dtype == q.dtype and out.stride(1) == 1,
+                "window_attention: out layout")
     if not use_hip(q, k_cache):
         if nd:
             out[:nd] = _ref_rows(q[:nd], k_cache, v_cache, md.decode_block_tables,
@@ -598,11 +604,12 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
                                    spec.sink is None and gate is None and spec.epilogue == 0),
             "window_attention: mixed weights come with a plain softmax, one map per head, no gate")
     for t in (spec.mult, spec.slope, spec.talk, spec.lam, spec.bias, spec.sink):
-        require(t is None or (t.dtype == torch.float32 and t.is_cuda and t.is_contiguous()),
-                "window_attention: fp32 device constants")
+        if t is not None:
+            require(t.dtype == torch.float32 and t.is_cuda and t.is_contiguous(),
+                    "window_attention: fp32 device constants")
     bs = k_cache.shape[1]
 
-    mfma = mfma_ok(spec, q.dtype, bs)
+    mfma = bf and _mfma_takes(spec, bs)
     if mfma:
         require(q.stride(0) % 8 == 0 and q.data_ptr() % 16 == 0, "window_attention: q alignment")
 

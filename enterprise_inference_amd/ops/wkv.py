@@ -15,7 +15,7 @@ from typing import Optional
 
 import torch
 
-from ._dispatch import check, lib, ptr, require, stream, use_hip
+from ._dispatch import check, lib, ptr, require, stream, use_hip, workspace
 
 
 CHUNK = 64                 # tokens per chunk of the chunk-parallel form (wkv.hip WC)
@@ -159,8 +159,7 @@ def wkv_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor,
         check(lib().eia_wkv_scan(*args, heads, D, split, 1 if bf else 0, stream(r)), "wkv_scan")
     if split:
         n = T // CHUNK + nseq
-        U = torch.empty(n, heads, CHUNK_DIM, CHUNK_DIM, dtype=torch.float32, device=r.device)
-        L = torch.empty(n, heads, CHUNK_DIM, dtype=torch.float32, device=r.device)
-        check(lib().eia_wkv_scan_chunked(*args, T, heads, D, split, ptr(U), ptr(L),
+        ws, (U, L) = workspace(r.device, 4 * n * heads * CHUNK_DIM * CHUNK_DIM, 4 * n * heads * CHUNK_DIM)
+        check(lib().eia_wkv_scan_chunked(*args, T, heads, D, split, U, L,
                                          1 if bf else 0, stream(r)), "wkv_scan_chunked")
     return y

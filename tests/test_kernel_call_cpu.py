@@ -75,3 +75,14 @@ def test_what_is_not_plain(echo):
     for bad in ((0, "i", plain), (1, "z", plain), (1, "f" * 9, plain), (1, "i" * 65, plain), (1, "i", 5)):
         with pytest.raises(ValueError):
             _native.runtime().KernelCall(*bad)
+
+
+@pytest.mark.parametrize("sizes", [(1,), (0, 4, 0, 513), (512, 511, 1), (4096, 0)])
+def test_workspace_places(sizes):
+    """The places of one allocation lie apart, on 512-byte steps of it, inside it."""
+    from enterprise_inference_amd.ops._dispatch import workspace
+    ws, at = workspace("cpu", *sizes)
+    base = ws.data_ptr()
+    for a, n, b in zip(at, sizes, at[1:] + [base + ws.numel()]):
+        assert (a - base) % 512 == 0 and a + n <= b
+    assert ws.numel() >= sum(sizes)

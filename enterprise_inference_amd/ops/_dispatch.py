@@ -35,12 +35,15 @@ def ptr(t):
 
 
 def workspace(device, *sizes: int):
-    """One allocation of so many bytes each, at multiples of 512 bytes -> (the tensor that owns it, addresses).  An
+    """One allocation of so many bytes each, at multiples of 512 bytes, large ones of 2 MiB as allocations of their own
+    would lie (expert layers of 2000 to 4000 rows without: 2 % slower) -> (the tensor that owns it, addresses).  An
     allocation costs the host 1.3 us, and small steps are bound by their launches."""
     at, total = [], 0
     for n in sizes:
+        step = 512 if n < 1 << 21 else 1 << 21
+        total = -(-total // step) * step
         at.append(total)
-        total += -(-n // 512) * 512
+        total += n
     ws = torch.empty(total, dtype=torch.uint8, device=device)
     base = ws.data_ptr()
     return ws, [base + a for a in at]

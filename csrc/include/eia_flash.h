@@ -16,6 +16,16 @@ EIA_DEV float flash_pair_sum(float v) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
+// Over the four lanes of a column of a 16 x 16 tile (those with the same lane % 16), in all of them: quarters and
+// halves of the wave change places in registers, where shuffles over 16 and 32 lanes wait for LDS.
+EIA_DEV float column_max(float v) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return flash_pair_max(fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])));
+}
+EIA_DEV float column_sum(float v) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return flash_pair_sum(__uint_as_float(r[0]) + __uint_as_float(r[1]));
+}
 EIA_DEV bf16x2 flash_pack(float a, float b) {          // one v_cvt_pk_bf16_f32
   typedef __attribute__((ext_vector_type(2))) float f32x2_t;
   return __builtin_convertvector(f32x2_t{a, b}, bf16x2);

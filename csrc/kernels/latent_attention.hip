@@ -343,17 +343,20 @@ EIA_API int eia_latent_attn(const void* qa, long qa_st, long qa_sh, const void* 
 }
 
 // ------------------------------------------------------------------------- decode rows, MFMA (bf16)
-// One workgroup of four waves per (decode row, 16 heads, key partition), v_mfma_f32_16x16x32_bf16.
-// 64 cache rows at a time are staged in LDS as they are; wave w forms the scores of keys 16 w .. + 15
-// (S^T: keys x heads), the waves exchange them through LDS, every wave forms the softmax weights of
-// all 64 keys and takes a quarter of the latent columns in O^T += C^T P^T, whose operand comes from the
-// same rows through the transposing LDS read.  Weights stay fp32: a bf16 high part plus a bf16
+// One workgroup of NW waves per (decode row, 16 heads, key partition), v_mfma_f32_16x16x32_bf16.
+// 64 cache rows at a time are staged in LDS as they are; wave w forms the scores of keys 16 (w % 4) .. + 15
+// (S^T: keys x heads), with eight waves over half of the entries each, the waves exchange them through LDS, every wave
+// forms the softmax weights of all 64 keys and takes its share of the latent columns in O^T += C^T P^T, whose operand
+// comes from the same rows through the transposing LDS read.  Rows that leave a CU to one workgroup (R + rd > 288) take
+// eight waves: half of a tile's chain for each (48 rows of 16 heads, 512 + 64, below: 27.6 -> 25.9 us with the merge, 13 rows
+// 19.0 -> 16.3, 100 rows at 2500 tokens, no window 79.3 -> 75.6, 30 rows of 64 heads at 4000 109 -> 103).  Weights stay fp32: a bf16 high part plus a bf16
 // remainder (two products), and the normaliser sums the fp32 weights.  The next rows are in flight
 // during the products, the first ones during the rotation of the queries.
 //
 // Bound by latency: a row's 64-key tiles are a chain of cache loads and two barriers, and the launch
 // lasts as long as the longest partition.  MI355X, 48 rows at up to 4096 tokens, window 1024, 16
-// heads, R 512 + 64: 22.0 + 4.0 us in five partitions; 200 rows at up to 2500 tokens, no window, with
+// heads, R 512 + 64: 20.4 + 4.0 us in five partitions, 7 of them before the first tile is there and 2.6 a tile; (pages read beside
+// the position, not behind it: 25.9 -> 25.8); 200 rows at up to 2500 tokens, no window, with
 // 16 heads 153 -> 134 us and with 64 heads 499 -> 437 us since a tile's page is known before its fetch and
 // its LDS reads are asked for before the first product; R 128 + 32 with 64 heads 120 -> 115 us, R 256 + 64
 // 292 -> 292 us.  (Two tiles of cache loads in flight, in registers: 27 us instead of 24; the reads held in
@@ -362,15 +365,18 @@ EIA_API int eia_latent_attn(const void* qa, long qa_st, long qa_sh, const void* 
 // partitions: 91 + 21 us.)
 constexpr int lat_bufs(int NK) { return NK <= 18 ? 2 : 1; }       // tiles that fit 160 KB of LDS
 
-template <int NK, int NCW>                  // 32-entry steps of a cache row; column tiles of a wave
-__global__ void __launch_bounds__(256)
+// NK: 32-entry steps of a cache row; NCW: column tiles of a wave; NW: waves, four or eight.
+template <int NK, int NCW, int NW>
+__global__ void __launch_bounds__(64 * NW)
 latent_decode_kernel(LatentAttnArgs a) {
   constexpr int NB = lat_bufs(NK), KT = LAT_UNIT;
   constexpr int KS = 32 * NK + 8;                       // 4 NK + 1 units of 16 bytes per row
   constexpr int SP = KT + 4;                            // pitch of the exchanged scores
+  constexpr int NT = 64 * NW, NH = NW / 4, NS = NK / NH, NU = KT * 4 * NK / NT;    // steps of a wave; 16-byte units of a thread
+  static_assert(NK % NH == 0 && KT * 4 * NK % NT == 0, "whole shares");
   // (static: more than 64 KB of dynamic LDS takes a call to the runtime for each launch)
   __shared__ __align__(16) bf16_t tiles[NB * KT * KS];
-  __shared__ __align__(16) float sS[16 * SP];           // the exchanged scores
+  __shared__ __align__(16) float sS[NH * 16 * SP];      // the exchanged scores
   __shared__ float2 rot[16 * NK];                       // [rot_dims / 2], rot_dims <= 32 NK
   int row = blockIdx.x, z = blockIdx.z;
   if (row >= a.n_work) {                                // beside the rows: the partitions that their own places do not hold
@@ -392,7 +398,7 @@ latent_decode_kernel(LatentAttnArgs a) {
   const int* bt = a.block_table + (long)row * a.bt_stride;
   const bool paged = bs % KT == 0;                      // a tile lies in one page
   const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
-  bf16x8 kst[NK];
+  bf16x8 kst[NU];
   // the page of a tile is looked up a tile ahead of its fetch: the fetch would wait for it
   int off = 0, at = 0, page = 0;                        // the next fetch: token in its page, page's place, page
   auto look = [&](int k0) {
@@ -410,8 +416,8 @@ latent_decode_kernel(LatentAttnArgs a) {
   auto fetch = [&](int k0) {
     const long base = paged ? (long)__builtin_amdgcn_readfirstlane(page) * bs + off : 0;
 #pragma unroll
-    for (int i = 0; i < NK; ++i) {
-      const int u = tid + 256 * i, j = u / (4 * NK), d = 8 * (u % (4 * NK));
+    for (int i = 0; i < NU; ++i) {
+      const int u = tid + NT * i, j = u / (4 * NK), d = 8 * (u % (4 * NK));
       const int kp = min(k0 + j, kmax - 1);
       const long slot = paged ? base + j : (long)bt[kp / bs] * bs + kp % bs;
       kst[i] = *reinterpret_cast<const bf16x8*>(cache + slot * a.cache_row + (d < Dk ? d : 0));
@@ -419,8 +425,8 @@ latent_decode_kernel(LatentAttnArgs a) {
   };
   auto stash = [&](int buf, int k0) {       // (slots behind the last key may hold anything: 0 x inf)
 #pragma unroll
-    for (int i = 0; i < NK; ++i) {
-      const int u = tid + 256 * i, j = u / (4 * NK), d = 8 * (u % (4 * NK));
+    for (int i = 0; i < NU; ++i) {
+      const int u = tid + NT * i, j = u / (4 * NK), d = 8 * (u % (4 * NK));
       *reinterpret_cast<bf16x8*>(tiles + (buf * KT + j) * KS + d) = d < Dk && k0 + j < k_end ? kst[i] : zero8;
     }
   };
@@ -430,7 +436,7 @@ latent_decode_kernel(LatentAttnArgs a) {
 
   // the rotary query parts, rotated once into LDS: the heads of a row turn by the same angles
   const int hp = a.rot_dims >> 1, npass = a.rd - a.rot_dims;
-  for (int i = tid; i < hp; i += 256) {
+  for (int i = tid; i < hp; i += NT) {
     float sn, cs;
     sincosf((float)qpos * a.inv_freq[i], &sn, &cs);
     rot[i] = make_float2(cs * a.rot_amp, sn * a.rot_amp);
@@ -438,7 +444,7 @@ latent_decode_kernel(LatentAttnArgs a) {
   __syncthreads();
   bf16_t* qrs = tiles;                                  // [16][rd]
   const bf16_t* qrb = static_cast<const bf16_t*>(a.qr) + (long)row * a.qr_st;
-  for (int e = tid; e < nh * hp; e += 256) {
+  for (int e = tid; e < nh * hp; e += NT) {
     const int m = e / hp, i = e - m * hp;
     const bf16_t* src = qrb + (long)(h0 + m) * a.qr_sh;
     const int ia = a.rot_half ? i : 2 * i, ib = a.rot_half ? i + hp : 2 * i + 1;
@@ -447,21 +453,22 @@ latent_decode_kernel(LatentAttnArgs a) {
     qrs[m * a.rd + ia] = f2bf(u * cs.x - v * cs.y);
     qrs[m * a.rd + ib] = f2bf(v * cs.x + u * cs.y);
   }
-  for (int e = tid; e < nh * npass; e += 256) {         // entries past rot_dims pass unchanged
+  for (int e = tid; e < nh * npass; e += NT) {         // entries past rot_dims pass unchanged
     const int m = e / npass, d = a.rot_dims + e - m * npass;
     qrs[m * a.rd + d] = qrb[(long)(h0 + m) * a.qr_sh + d];
   }
   __syncthreads();
   const bool ok = l16 < nh;                             // this lane's head
   const int h = h0 + (ok ? l16 : 0);
-  bf16x8 qf[NK];
+  const int kg = w & 3, s0 = NS * (w >> 2);             // the wave's keys of a tile, and steps of their rows
+  bf16x8 qf[NS];
   {
     // R % 8 == 0 and rd % 8 == 0: a lane's eight entries lie wholly in one of the two parts
     const bf16_t* qa = static_cast<const bf16_t*>(a.qa) + (long)row * a.qa_st + (long)h * a.qa_sh;
     const bool vec = ((reinterpret_cast<uintptr_t>(a.qa) | (uintptr_t)(a.qa_st * 2) | (uintptr_t)(a.qa_sh * 2)) & 15) == 0;
 #pragma unroll
-    for (int s = 0; s < NK; ++s) {
-      const int d = 32 * s + 8 * g4;
+    for (int s = 0; s < NS; ++s) {
+      const int d = 32 * (s0 + s) + 8 * g4;
       bf16x8 v = zero8;
       if (ok && d < Dk) {
         if (d >= R) {
@@ -493,12 +500,12 @@ latent_decode_kernel(LatentAttnArgs a) {
       look(k0 + 2 * KT);
     }
     f32x4 sc = {0.f, 0.f, 0.f, 0.f};
-    bf16x8 kf[NK];                                      // (all asked for before the first product)
+    bf16x8 kf[NS];                                      // (all asked for before the first product)
 #pragma unroll
-    for (int s = 0; s < NK; ++s) kf[s] = *reinterpret_cast<const bf16x8*>(t + (16 * w + l16) * KS + 32 * s + 8 * g4);
+    for (int s = 0; s < NS; ++s) kf[s] = *reinterpret_cast<const bf16x8*>(t + (16 * kg + l16) * KS + 32 * (s0 + s) + 8 * g4);
 #pragma unroll
-    for (int s = 0; s < NK; ++s) sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[s], qf[s], sc, 0, 0, 0);
-    *reinterpret_cast<f32x4*>(sS + l16 * SP + 16 * w + 4 * g4) = sc * scale_log2;
+    for (int s = 0; s < NS; ++s) sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[s], qf[s], sc, 0, 0, 0);
+    *reinterpret_cast<f32x4*>(sS + (16 * (w >> 2) + l16) * SP + 16 * kg + 4 * g4) = sc * scale_log2;
     __syncthreads();
     // head l16, keys 32 x + 8 g4 + e
     float v[2][8];
@@ -507,7 +514,8 @@ latent_decode_kernel(LatentAttnArgs a) {
     for (int x = 0; x < 2; ++x)
 #pragma unroll
       for (int e = 0; e < 8; e += 4) {
-        const f32x4 q = *reinterpret_cast<const f32x4*>(sS + l16 * SP + 32 * x + 8 * g4 + e);
+        f32x4 q = *reinterpret_cast<const f32x4*>(sS + l16 * SP + 32 * x + 8 * g4 + e);
+        if constexpr (NH == 2) q += *reinterpret_cast<const f32x4*>(sS + (16 + l16) * SP + 32 * x + 8 * g4 + e);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int key = k0 + 32 * x + 8 * g4 + e + i;
@@ -515,8 +523,7 @@ latent_decode_kernel(LatentAttnArgs a) {
           mloc = fmaxf(mloc, v[x][e + i]);
         }
       }
-    mloc = fmaxf(mloc, __shfl_xor(mloc, 16, 64));
-    mloc = fmaxf(mloc, __shfl_xor(mloc, 32, 64));
+    mloc = column_max(mloc);
     const float mnew = fmaxf(mrun, mloc), muse = mnew == -INFINITY ? 0.f : mnew;
     const float alpha = exp2f(mrun - muse);             // mrun = -inf: 0 (nothing summed yet)
     bf16x8 ph[2], pl[2];
@@ -529,8 +536,7 @@ latent_decode_kernel(LatentAttnArgs a) {
         psum += p0 + p1;
         flash_split(p0, p1, e, ph[x], pl[x]);
       }
-    psum += __shfl_xor(psum, 16, 64);
-    psum += __shfl_xor(psum, 32, 64);
+    psum = column_sum(psum);
     lrun = lrun * alpha + psum;
     mrun = mnew;
 #pragma unroll
@@ -677,12 +683,12 @@ EIA_API int eia_latent_attn_mfma(const void* qa, long qa_st, long qa_sh, const v
   const bool pad = nparts > 1 && (nparts - home) * n_items <= (8 * per - n_items) * home;
   const int rows = pad ? 8 * per : n_items;
   const dim3 grid(rows, y, pad ? home : nparts);
-#define LAT_DECODE(NK, NCW) hipLaunchKernelGGL((latent_decode_kernel<NK, NCW>), grid, dim3(256), 0, st, a)
-  if (Dk <= 160 && R <= 128) LAT_DECODE(5, 2);
-  else if (Dk <= 288 && R <= 256) LAT_DECODE(9, 4);
-  else if (Dk <= 320 && R <= 256) LAT_DECODE(10, 4);
-  else if (Dk <= 576) LAT_DECODE(18, 8);
-  else LAT_DECODE(20, 8);
+#define LAT_DECODE(NK, NCW, NW) hipLaunchKernelGGL((latent_decode_kernel<NK, NCW, NW>), grid, dim3(64 * NW), 0, st, a)
+  if (Dk <= 160 && R <= 128) LAT_DECODE(5, 2, 4);
+  else if (Dk <= 288 && R <= 256) LAT_DECODE(9, 4, 4);
+  else if (Dk <= 320 && R <= 256) LAT_DECODE(10, 2, 8);
+  else if (Dk <= 576) LAT_DECODE(18, 4, 8);
+  else LAT_DECODE(20, 4, 8);
 #undef LAT_DECODE
   if (nparts > 1)
     hipLaunchKernelGGL(latent_merge_kernel, dim3(rows, H), dim3(128), 0, st, part_acc, part_ml,

@@ -45,6 +45,12 @@
 // per phase instead of one for the younger half of the waves): 32 heads on 8, 1 x 8192 582 -> 543 us, 1 x 2048 72 -> 65,
 // 40 heads 1 x 4096 232 -> 219, the same bits.  A tile and wave takes 1020 cycles of matrix products and about 1500
 // of vector instructions, two waves on a SIMD.
+//
+// Launches of fewer workgroups than CUs wait for their longest one (a tile of 64 keys takes 1.65 us): there blocks
+// are cut along the keys (CUT; attention.py fa_parts says where), parts hand over fp32 sums as their lanes hold
+// them, and a second kernel puts them together.  32 heads on 8, 100 tokens behind 2000: 59.5 -> 21 us, 1000 behind
+// 2000 85 -> 61, 1 x 1000 34 -> 28; 16 on 4, 500 behind 1000 45.5 -> 22.6, 1 x 4000 110 -> 97.5; error against 64
+// bits 2.35e-3 -> 2.29e-3.  Uncut launches run as before (1 x 8192 537, 4 x 300 15.7).
 #include "eia_common.h"
 
 namespace {
@@ -71,7 +77,55 @@ EIA_DEV float pair_sum(float v) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-template <int HPW>
+// The key tiles of a query block: from key lo on (64-aligned), n of them.
+struct KeyTiles { int lo, n; };
+
+EIA_DEV int first_key(int qa, int sliding_window, int chunk_size) {
+  int lo = 0;
+  if (sliding_window > 0) lo = max(lo, qa - sliding_window + 1);
+  if (chunk_size > 0) lo = max(lo, (qa / chunk_size) * chunk_size);
+  return lo;
+}
+
+EIA_DEV KeyTiles key_tiles(int q0, int queries, int qlen, int L, int causal, int sliding_window, int chunk_size) {
+  const int ctx = L - qlen, qlast = min(q0 + queries, qlen) - 1;
+  const int hi = causal ? min(L, ctx + qlast + 1) : L;
+  const int lo = first_key(ctx + q0, sliding_window, chunk_size) & ~(FKB - 1);
+  return {lo, (hi - lo + FKB - 1) / FKB};
+}
+
+// Where the keys of query blocks are cut: at most `per` tiles a part, `most` parts a block.  A wave's part of
+// O^T lies in o as its lanes hold it ([part][16 registers of four][64 lanes]), maxima and sums of its 32
+// queries in ml.
+struct KeyParts {
+  float* o; float2* ml;
+  int per, most;
+};
+
+EIA_DEV int parts_of(int tiles, const KeyParts& cut) { return max(1, min((tiles + cut.per - 1) / cut.per, cut.most)); }
+
+// Output rows of a wave, one 32-dim tile: lane (q, h) holds d = 8 j + 4 h + [0, 4) of it, the two lane halves of
+// a query own alternating 8-B pieces.  One permlane32_swap per dword pairs pieces j / j+1 so each lane
+// stores 16 contiguous bytes: dwordx4 stores instead of dwordx2.
+// Both lanes of a swap pair hold the same query, so they are valid (or exited) together.
+EIA_DEV void put_rows(bf16_t* op, const f32x16_t& o, float inv) {
+  uint2 pk[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    bf16x4 o4;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o4[r] = f2bf(o[4 * j + r] * inv);
+    pk[j] = __builtin_bit_cast(uint2, o4);
+  }
+#pragma unroll
+  for (int j = 0; j < 4; j += 2) {
+    const auto rx = __builtin_amdgcn_permlane32_swap(pk[j].x, pk[j + 1].x, false, false);
+    const auto ry = __builtin_amdgcn_permlane32_swap(pk[j].y, pk[j + 1].y, false, false);
+    *reinterpret_cast<uint4*>(op + 8 * j) = make_uint4(rx[0], ry[0], rx[1], ry[1]);
+  }
+}
+
+template <int HPW, bool CUT>
 __global__ void __launch_bounds__(FTHREADS, 1)
 paged_prefill_fa_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __restrict__ out,
                         long out_stride, const bf16_t* __restrict__ kc,
@@ -79,14 +133,15 @@ paged_prefill_fa_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __r
                         int bt_stride, const int* __restrict__ seq_lens,
                         const int* __restrict__ cu_q, const int* __restrict__ work,
                         float scale_log2, int Hq, int Hkv, int bs, int causal, int sliding_window,
-                        int chunk_size) {
+                        int chunk_size, KeyParts cut) {
   __shared__ __align__(16) bf16_t lds[2 * BUF];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int r32 = lane & 31, h = lane >> 5;
   // grid (head groups, work items): the heads of one query block are dispatched together and
   // the work list is latest-block-first, so the dispatch order is longest-first over the
-  // whole grid (causal blocks grow with their position), not per head
-  const int s = work[2 * blockIdx.y], q0 = work[2 * blockIdx.y + 1];
+  // whole grid (causal blocks grow with their position), not per head; parts of a block stay together
+  const int item = CUT ? blockIdx.z : blockIdx.y;
+  const int s = work[2 * item], q0 = work[2 * item + 1];
   constexpr int FQB = FROWS / HPW;
   const int G = Hq / Hkv, NHG = G / HPW;
   const int kvh = blockIdx.x / NHG, hg = blockIdx.x % NHG;
@@ -96,20 +151,13 @@ paged_prefill_fa_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __r
   if (q0 >= qlen) return;                                  // workgroup-uniform
   const int L = seq_lens[s], ctx = L - qlen;
   const bool window = sliding_window > 0 || chunk_size > 0;
-  auto lo_of = [&](int qa) {
-    int lo = 0;
-    if (sliding_window > 0) lo = max(lo, qa - sliding_window + 1);
-    if (chunk_size > 0) lo = max(lo, (qa / chunk_size) * chunk_size);
-    return lo;
-  };
-
   // this lane's query column
   const int qi = q0 + 32 * qsub + r32;
   const bool qvalid = qi < qlen;
   const int qe = min(qi, qlen - 1);
   const long tok = qbeg + qe;
   const int qa = ctx + qe;
-  const int q_lo = lo_of(qa);
+  const int q_lo = first_key(qa, sliding_window, chunk_size);
   // Q^T fragments (B operand): k-step t = dims [16t, 16t+16), lane half h holds 16t+8h..+8
   bf16x8 qf[FD / 16];
   {
@@ -118,16 +166,22 @@ paged_prefill_fa_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __r
     for (int t = 0; t < FD / 16; ++t) qf[t] = *reinterpret_cast<const bf16x8*>(qp + 16 * t);
   }
 
-  // workgroup key range [lo, hi) (tiles of 64 from a 64-aligned lo) and this wave's range
-  const int qlast = min(q0 + FQB, qlen) - 1;
-  const int hi = causal ? min(L, ctx + qlast + 1) : L;
-  const int lo = lo_of(ctx + q0) & ~(FKB - 1);
-  const int ntile = (hi - lo + FKB - 1) / FKB;
+  // workgroup key range (tiles of 64 from a 64-aligned lo)
+  KeyTiles kt = key_tiles(q0, FQB, qlen, L, causal, sliding_window, chunk_size);
+  const int parts = CUT ? parts_of(kt.n, cut) : 1;
+  if (CUT) {
+    const int part = blockIdx.y, each = (kt.n + parts - 1) / parts;
+    if (part >= parts) return;
+    kt.lo += FKB * each * part;
+    kt.n = min(each, kt.n - each * part);
+  }
+  const int lo = kt.lo, ntile = kt.n;
+  // this wave's key range
   const int wq0 = q0 + 32 * qsub;                          // wave's first query
   const bool wave_live = wq0 < qlen;
   const int wq1 = min(wq0 + 32, qlen) - 1;                 // wave's last valid query
   const int w_hi = !wave_live ? 0 : (causal ? min(L, ctx + wq1 + 1) : L);
-  const int w_lo = wave_live ? lo_of(ctx + wq0) : 0;      // no query of the wave sees below
+  const int w_lo = wave_live ? first_key(ctx + wq0, sliding_window, chunk_size) : 0;      // no query of the wave sees below
 
   const int* bt = block_tables + (long)s * bt_stride;
   // the page of a tile is looked up a tile ahead of its fetch: the fetch would wait for it
@@ -291,53 +345,119 @@ paged_prefill_fa_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __r
   }
 
   const float lt = pair_sum(l_run);
+  if (CUT && parts > 1) {
+    if (!wave_live) return;
+    const long at = (((long)item * cut.most + blockIdx.y) * gridDim.x + blockIdx.x) * (FTHREADS / 64) + w;
+    f32x4* po = reinterpret_cast<f32x4*>(cut.o) + at * (FD / 8 * 64) + lane;
+#pragma unroll
+    for (int dt = 0; dt < FD / 32; ++dt)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        po[(4 * dt + j) * 64] = f32x4{oacc[dt][4 * j], oacc[dt][4 * j + 1], oacc[dt][4 * j + 2], oacc[dt][4 * j + 3]};
+    if (h == 0) cut.ml[at * 32 + r32] = make_float2(m_run, lt);
+    return;
+  }
   if (!qvalid) return;
   const float inv = lt > 0.f ? 1.f / lt : 0.f;
-  // Lane (q, h) holds d = 32 dt + 8 j + 4 h + [0, 4): the two lane halves of a query own
-  // alternating 8-B pieces.  One permlane32_swap per dword pairs pieces j / j+1 so each lane
-  // stores 16 contiguous bytes (guide T21): 8 dwordx4 stores per lane instead of 16 dwordx2.
-  // Both lanes of a swap pair hold the same query, so they are valid (or exited) together.
   bf16_t* op = out + tok * out_stride + (long)hq * FD + 8 * h;
 #pragma unroll
-  for (int dt = 0; dt < FD / 32; ++dt) {
-    uint2 pk[4];
+  for (int dt = 0; dt < FD / 32; ++dt) put_rows(op + 32 * dt, oacc[dt], inv);
+}
+
+// A workgroup puts the parts of one wave's 32 queries together, wave dt 32 dims of them; the head group comes
+// first in both grids, so where there are a multiple of eight the parts are read on the XCD that wrote them.
+template <int HPW>
+__global__ void __launch_bounds__(256)
+paged_prefill_fa_merge_kernel(bf16_t* __restrict__ out, long out_stride, const int* __restrict__ seq_lens,
+                              const int* __restrict__ cu_q, const int* __restrict__ work, int Hq, int Hkv,
+                              int causal, int sliding_window, int chunk_size, KeyParts cut) {
+  constexpr int FQB = FROWS / HPW, NP = 4;
+  const int item = blockIdx.z, w = blockIdx.y, lane = threadIdx.x & 63, dt = threadIdx.x >> 6;
+  const int r32 = lane & 31, h = lane >> 5;
+  const int s = work[2 * item], q0 = work[2 * item + 1];
+  const int qbeg = cu_q[s], qlen = cu_q[s + 1] - qbeg;
+  if (q0 + 32 * (w / HPW) >= qlen) return;
+  const KeyTiles kt = key_tiles(q0, FQB, qlen, seq_lens[s], causal, sliding_window, chunk_size);
+  const int parts = parts_of(kt.n, cut);
+  if (parts == 1) return;
+  const long step = (long)gridDim.x * (FTHREADS / 64);
+  const long at = ((long)item * cut.most * gridDim.x + blockIdx.x) * (FTHREADS / 64) + w;
+  const f32x4* po = reinterpret_cast<const f32x4*>(cut.o) + at * (FD / 8 * 64) + dt * 4 * 64 + lane;
+  const float2* ml = cut.ml + at * 32 + r32;
+  f32x16_t o;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      bf16x4 o4;
+  for (int i = 0; i < 16; ++i) o[i] = 0.f;
+  float m = (-INFINITY), l = 0.f;
+  for (int p0 = 0; p0 < parts; p0 += NP) {
+    float2 x[NP];
+    f32x4 v[NP][4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) o4[r] = f2bf(oacc[dt][4 * j + r] * inv);
-      pk[j] = __builtin_bit_cast(uint2, o4);
+    for (int k = 0; k < NP; ++k) {                         // (a part past the last: the last one again, weight 0)
+      const long p = min(p0 + k, parts - 1) * step;
+      x[k] = ml[p * 32];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[k][j] = po[p * (FD / 8 * 64) + j * 64];
     }
+    float mx = m;
 #pragma unroll
-    for (int j = 0; j < 4; j += 2) {
-      const auto rx = __builtin_amdgcn_permlane32_swap(pk[j].x, pk[j + 1].x, false, false);
-      const auto ry = __builtin_amdgcn_permlane32_swap(pk[j].y, pk[j + 1].y, false, false);
-      *reinterpret_cast<uint4*>(op + 32 * dt + 8 * j) = make_uint4(rx[0], ry[0], rx[1], ry[1]);
+    for (int k = 0; k < NP; ++k) mx = fmaxf(mx, x[k].x);
+    const float ref = mx == (-INFINITY) ? 0.f : mx, old = __builtin_amdgcn_exp2f(m - ref);
+    m = mx;
+    l *= old;
+    o *= old;
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+      if (p0 + k >= parts) break;
+      const float c = __builtin_amdgcn_exp2f(x[k].x - ref);
+      l += c * x[k].y;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[4 * j + i] += c * v[k][j][i];
     }
   }
+  const int qi = q0 + 32 * (w / HPW) + r32;
+  if (qi >= qlen) return;
+  const int G = Hq / Hkv, NHG = G / HPW;
+  const int hq = blockIdx.x / NHG * G + blockIdx.x % NHG * HPW + w % HPW;
+  put_rows(out + (long)(qbeg + qi) * out_stride + (long)hq * FD + 8 * h + 32 * dt, o, l > 0.f ? 1.f / l : 0.f);
 }
 
 }  // namespace
 
 // work = [seq, first query] pairs with blocks of 256 / HPW queries (attention.prefill_query_block);
 // grid (Hkv * G / HPW, n_work).  Requires D = 128, block size % 64 == 0.
+// parts > 1: blocks of more than `per` key tiles are cut into up to `parts` parts; ws holds
+// n_work * parts * (Hq / HPW) * 256 * (128 + 2) floats.  (Longer ones than parts * per get longer parts.)
 EIA_API int eia_paged_prefill_fa(const void* q, long q_stride, void* out, long out_stride,
                                  const void* k_cache, const void* v_cache,
                                  const int* block_tables, int bt_stride, const int* seq_lens,
                                  const int* cu_q, const int* work, int n_work, float scale, int Hq,
                                  int Hkv, int D, int bs, int causal, int sliding_window,
-                                 int chunk_size, hipStream_t st) {
+                                 int chunk_size, int parts, int per, float* ws, hipStream_t st) {
   if (Hkv <= 0 || Hq % Hkv != 0) return EIA_BAD_SHAPE;
   if (D != FD || bs % FKB != 0 || out_stride % 8 != 0) return EIA_UNSUPPORTED;   // (16-B output stores)
   if (n_work == 0) return EIA_OK;
   const int G = Hq / Hkv, hpw = G % 4 == 0 ? 4 : G % 2 == 0 ? 2 : 1;
+  if (parts > 1 && (per < 1 || !ws || n_work > 65535)) return EIA_BAD_SHAPE;
+  KeyParts cut{nullptr, nullptr, per, parts};
+  if (parts > 1) {
+    cut.o = ws;
+    cut.ml = reinterpret_cast<float2*>(ws + (long)n_work * parts * (Hq / hpw) * FROWS * FD);
+  }
 #define FA_GO(HPW)                                                                                  \
   do {                                                                                              \
-    hipLaunchKernelGGL(paged_prefill_fa_kernel<HPW>, dim3(Hq / HPW, n_work), dim3(FTHREADS),        \
-                       0, st, (const bf16_t*)q, q_stride, (bf16_t*)out, out_stride,      \
-                       (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, bt_stride,     \
-                       seq_lens, cu_q, work, scale * 1.4426950408889634f, Hq, Hkv, bs, causal,      \
-                       sliding_window, chunk_size);                                                 \
+    const float sl = scale * 1.4426950408889634f;                                                   \
+    const dim3 grid = parts > 1 ? dim3(Hq / HPW, parts, n_work) : dim3(Hq / HPW, n_work);           \
+    auto* f = parts > 1 ? paged_prefill_fa_kernel<HPW, true> : paged_prefill_fa_kernel<HPW, false>; \
+    hipLaunchKernelGGL(f, grid, dim3(FTHREADS), 0, st, (const bf16_t*)q, q_stride, (bf16_t*)out,    \
+                       out_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables,    \
+                       bt_stride, seq_lens, cu_q, work, sl, Hq, Hkv, bs, causal, sliding_window,    \
+                       chunk_size, cut);                                                            \
+    if (parts > 1)                                                                                  \
+      hipLaunchKernelGGL(paged_prefill_fa_merge_kernel<HPW>, dim3(Hq / HPW, FTHREADS / 64, n_work), \
+                         dim3(256), 0, st, (bf16_t*)out, out_stride, seq_lens, cu_q, work, Hq, Hkv, \
+                         causal, sliding_window, chunk_size, cut);                                  \
   } while (0)
   if (hpw == 4) FA_GO(4); else if (hpw == 2) FA_GO(2); else FA_GO(1);
 #undef FA_GO

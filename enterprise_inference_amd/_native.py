@@ -44,7 +44,7 @@ _SIGNATURES = {
     "eia_paged_decode_rope": [P, L, P, I, P, P, P, F, IP, P, IP, I, P, P, IP, I, IP, P, L, P, P, P,
                               F, I, I, I, I, I, I, I, I, IP, S],
     "eia_paged_prefill": [P, L, P, L, P, P, IP, I, IP, IP, IP, I, F, I, I, I, I, I, I, I, I, I, S],
-    "eia_paged_prefill_fa": [P, L, P, L, P, P, IP, I, IP, IP, IP, I, F, I, I, I, I, I, I, I, S],
+    "eia_paged_prefill_fa": [P, L, P, L, P, P, IP, I, IP, IP, IP, I, F, I, I, I, I, I, I, I, I, I, P, S],
     "eia_act_and_mul": [P, P, I, I, L, L, I, S],
     "eia_act": [P, P, L, I, S],
     "eia_sample": [P, L, I, I, P, P, P, P, P, P, S],

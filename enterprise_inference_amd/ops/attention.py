@@ -140,6 +140,51 @@ def split_keys(wgs: int, tiles: int, mean: int, slots: int, least: int = 12, mer
     return -(-tiles // per), per
 
 
+FA_SLOTS = 256        # workgroups of the flash form that run at a time: one a CU
+
+
+def fa_parts(wgs: int, tiles: int, mean: float, tile_us: float = 1.65):
+    """(parts, tiles per part) of a launch of the flash form: ``wgs`` workgroups that walk up to ``tiles``
+    and on average ``mean`` key tiles, of lengths spread evenly about the mean.  A tile takes ``tile_us`` (with fewer
+    than four heads a workgroup 1.95), the merge's launch 4 us and a part's rows, written and read, 1/28 us (of the
+    whole chip).  Parts run in one round (232 of them: not every XCD gets the same number), or in two where short
+    ones fill the gaps.  1024 are at most 136 MB.  More workgroups than run at a time even themselves out.
+
+    MI355X, workgroups of up to so many tiles, mean: tiles per part: us.  Heads 32 on 8: 16 of 12, 11: uncut 24.8, 6:
+    19.7, 3: 15.6, 2: 15.4, 1: 17.8; 16 of 34, 33: 58.6, 9: 25.4, 4: 20.9, 3: 21.3; 64 of 8, 4: 19.4, 3: 17.8, 1: 26.3;
+    64 of 258, 254: 425, 129: 224, 65: 138, 52: 197; 104 of 28, 27: 51.4, 14: 38.9, 12: 47.3, 5: 56.8; 128 of 6, 4: 15.6, 3:
+    17.7; 128 of 16, 8: 34.4, 9: 29.2, 7: 27.3, 5: 37.2, 2: 45; 128 of 48, 40: 85.4, 36: 75.4, 24: 59.1, 16: 67.8; 192 of
+    24, 12: 47.4, 12: 44.6, 6: 56.5; 256 of 32, 16: 61.1, 16: 63.5, 11: 61.1, 8: 82.5; 504 of 64, 33: 155, 32: 179.
+    16 on 4: 32 of 24, 20: 45.2, 5: 23.2, 2: 31.1; 52 of 26, 25: 48.1, 7: 27.8, 6: 34; 128 of 32, 16: 58.2, 13: 38.6, 8: 47.7;
+    236 of 24, 14: 47, 16: 50; 252 of 64, 33: 116, 34: 108, 22: 97, 16: 124.  28 on 4: 112 of 22, 16: 46.2, 11: 36.3, 8: 41;
+    168 of 48, 36: 98, 24: 90, 16: 92, 15: 107; 224 of 30, 27: 66.2, 15: 81.7."""
+    if wgs > FA_SLOTS or tiles < 6:
+        return 1, tiles
+    work = wgs * max(1.0, mean)
+    least = max(1, math.ceil(tiles * wgs / 1024))
+    even = 4 * mean >= 3 * tiles
+    # one round: as many parts of each where workgroups are about equally long, else wgs (mean / per + 1/2) parts
+    if even:
+        per = -(-tiles // (FA_SLOTS // wgs))
+    else:
+        share = 232 / wgs - 0.5
+        per = math.ceil(mean / share) if share > 0 else tiles
+    per = min(tiles, max(per, least, math.ceil(math.sqrt(work / 36))))
+    shortest = max(0.0, 2 * mean - tiles)
+
+    def rows_us(per):                                        # (workgroups of up to ``per`` tiles stay whole)
+        whole = max(0.0, (per - shortest) / (tiles - shortest)) if per > shortest else 0.0
+        return 4 + (work / per + wgs * (0.5 - whole)) / 28
+
+    took = tile_us * per + rows_us(per)
+    if not even:                                             # two rounds; 0.15: they do not meet everywhere
+        half = min(tiles, max(least, math.ceil(mean / (500 / wgs - 0.5))))
+        two = 2.3 * tile_us * half + rows_us(half)
+        if two < took:
+            per, took = half, two
+    return (-(-tiles // per), per) if took < tile_us * tiles else (1, tiles)
+
+
 def decode_partitions(batch: int, num_kv_heads: int, num_heads: int, max_len: int,
                       cus: int = 256, max_parts: int = 8) -> int:
     """Context partitions (flash-decoding split) for a decode batch.
@@ -304,11 +349,23 @@ def paged_prefill(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
     hpw = heads_per_workgroup(Hq, Hkv)
     code = qt or prefill_variant(Hq, Hkv, D, bs)
     if code & PREFILL_FA:
+        wgs, ws = n_work * (Hq // hpw), None
+        parts = per = 1
+        if wgs <= FA_SLOTS and block_tables.shape[1] * bs >= 6 * 64:
+            rows = PREFILL_FA_QB * (4 // hpw)
+            tiles = block_tables.shape[1] * bs / 64          # (of the longest sequence)
+            mean = tiles - T / (128 * (cu_q.numel() - 1)) if causal else tiles
+            span = sliding_window or chunk_size
+            if span:
+                tiles = min(tiles, (span + rows) / 64 + 1)
+            parts, per = fa_parts(wgs, math.ceil(tiles), min(mean, tiles), 1.65 if hpw == 4 else 1.95)
+            if parts > 1:
+                ws = torch.empty(wgs * parts * 256 * (D + 2), dtype=torch.float32, device=q.device)
         rc = lib().eia_paged_prefill_fa(
             ptr(q), q.stride(0), ptr(o), o.stride(0), ptr(k_cache), ptr(v_cache),
             ptr(block_tables), block_tables.stride(0), ptr(seq_lens), ptr(cu_q), ptr(work), n_work,
             float(scale), Hq, Hkv, D, bs, 1 if causal else 0, sliding_window or 0, chunk_size or 0,
-            stream(q))
+            parts, per, ptr(ws), stream(q))
         if rc != EIA_UNSUPPORTED:
             check(rc, "paged_prefill_fa")
             return o

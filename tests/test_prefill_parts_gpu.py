@@ -1,0 +1,53 @@
+"""Flash prefill whose query blocks are cut along the keys: parts of one tile, parts that do not divide a block's
+tiles, more tiles than the parts were counted for, waves without queries and parts without keys."""
+
+import pytest
+import torch
+
+BF = torch.bfloat16
+
+
+def test_parts_cover_and_fit():
+    from enterprise_inference_amd.ops.attention import FA_SLOTS, fa_parts
+    for wgs in (1, 2, 7, 16, 40, 64, 127, 128, 129, 192, 232, 255, 256, 257, 4000):
+        for tiles in (1, 2, 5, 6, 16, 33, 64, 500, 2049, 40000):
+            for share in (0.5, 0.6, 0.75, 0.9, 1.0):
+                parts, per = fa_parts(wgs, tiles, max(1.0, tiles * share))
+                assert parts >= 1 and 1 <= per <= tiles and (parts - 1) * per < tiles <= parts * per
+                assert parts == 1 or (wgs <= FA_SLOTS and wgs * parts <= 1024)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Hq,Hkv", [(8, 2), (6, 3), (3, 1)])
+@pytest.mark.parametrize("qlens,ctxs", [([1, 33, 64, 127], [700, 5, 70, 0]), ([255, 40], [63, 600]), ([300], [0])])
+@pytest.mark.parametrize("causal,window,chunk", [(True, None, None), (False, None, None),
+                                                 (True, 200, None), (True, None, 192)])
+@pytest.mark.parametrize("parts,per", [(12, 1), (5, 3), (3, 2)])
+def test_flash_prefill_parts(Hq, Hkv, qlens, ctxs, causal, window, chunk, parts, per, monkeypatch):
+    from enterprise_inference_amd.ops import attention
+    from enterprise_inference_amd.ops import reference as ref
+    g = torch.Generator().manual_seed(sum(qlens) + Hq)
+    D, bs = 128, 128
+    lens = [a + b for a, b in zip(qlens, ctxs)]
+    need = [-(-n // bs) for n in lens]
+    bt = torch.zeros(len(lens), max(need), dtype=torch.int32)
+    perm, at = torch.randperm(sum(need), generator=g).to(torch.int32), 0
+    for s, n in enumerate(need):
+        bt[s, :n] = perm[at:at + n]
+        at += n
+    k = torch.randn(sum(need), Hkv, bs, D, generator=g).to(BF)
+    v = torch.randn(sum(need), Hkv, D, bs, generator=g).to(BF)
+    q = torch.randn(sum(qlens), Hq, D, generator=g).to(BF)
+    q[0] = 0                                               # (equal scores)
+    sl = torch.tensor(lens, dtype=torch.int32)
+    cu = torch.tensor([0] + qlens).cumsum(0).to(torch.int32)
+    r = ref.paged_attention_prefill(q.float(), k.float(), v.float(), bt, cu, sl, D ** -0.5, causal,
+                                    window, chunk)
+    work = torch.tensor(attention.build_prefill_work(
+        qlens, attention.prefill_query_block(Hq, Hkv, D, block_size=bs)), dtype=torch.int32)
+    monkeypatch.setattr(attention, "fa_parts", lambda *a: (parts, per))
+    d = [t.cuda() for t in (q, k, v, bt, sl, cu, work)]
+    o = attention.paged_prefill(*d[:6], d[6], work.numel() // 2, D ** -0.5, causal, window, chunk)
+    # weights and outputs rounded to bf16 (2^-9 each, relative), fp32 sums
+    err = (o.double().cpu() - r.double()).norm() / r.double().norm()
+    assert err < 4e-3

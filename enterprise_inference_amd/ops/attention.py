@@ -9,6 +9,7 @@ caching need no special path.
 from __future__ import annotations
 
 import dataclasses
+import functools
 import math
 import os
 from typing import List, Optional, Sequence
@@ -143,11 +144,13 @@ def split_keys(wgs: int, tiles: int, mean: int, slots: int, least: int = 12, mer
 FA_SLOTS = 256        # workgroups of the flash form that run at a time: one a CU
 
 
-def fa_parts(wgs: int, tiles: int, mean: float, tile_us: float = 1.65):
+@functools.lru_cache(maxsize=1024)            # (numbers to numbers; a step's layers ask the same)
+def fa_parts(wgs: int, tiles: int, mean: float, tile_us: float = 1.65, merge_us: float = 4.0,
+             rows_us: float = 1 / 28, rounds: int = 2):
     """(parts, tiles per part) of a launch of the flash form: ``wgs`` workgroups that walk up to ``tiles``
     and on average ``mean`` key tiles, of lengths spread evenly about the mean.  A tile takes ``tile_us`` (with fewer
-    than four heads a workgroup 1.95), the merge's launch 4 us and a part's rows, written and read, 1/28 us (of the
-    whole chip).  Parts run in one round (232 of them: not every XCD gets the same number), or in two where short
+    than four heads a workgroup 1.95), the merge's launch ``merge_us`` and a part's rows, written and read, ``rows_us``
+    (of the whole chip).  Parts run in one round (232 of them: not every XCD gets the same number), or in two where short
     ones fill the gaps.  1024 are at most 136 MB.  More workgroups than run at a time even themselves out.
 
     MI355X, workgroups of up to so many tiles, mean: tiles per part: us.  Heads 32 on 8: 16 of 12, 11: uncut 24.8, 6:
@@ -158,7 +161,7 @@ def fa_parts(wgs: int, tiles: int, mean: float, tile_us: float = 1.65):
     16 on 4: 32 of 24, 20: 45.2, 5: 23.2, 2: 31.1; 52 of 26, 25: 48.1, 7: 27.8, 6: 34; 128 of 32, 16: 58.2, 13: 38.6, 8: 47.7;
     236 of 24, 14: 47, 16: 50; 252 of 64, 33: 116, 34: 108, 22: 97, 16: 124.  28 on 4: 112 of 22, 16: 46.2, 11: 36.3, 8: 41;
     168 of 48, 36: 98, 24: 90, 16: 92, 15: 107; 224 of 30, 27: 66.2, 15: 81.7."""
-    if wgs > FA_SLOTS or tiles < 6:
+    if wgs > FA_SLOTS or tile_us * tiles < 9:
         return 1, tiles
     work = wgs * max(1.0, mean)
     least = max(1, math.ceil(tiles * wgs / 1024))
@@ -169,17 +172,17 @@ def fa_parts(wgs: int, tiles: int, mean: float, tile_us: float = 1.65):
     else:
         share = 232 / wgs - 0.5
         per = math.ceil(mean / share) if share > 0 else tiles
-    per = min(tiles, max(per, least, math.ceil(math.sqrt(work / 36))))
+    per = min(tiles, max(per, least, math.ceil(math.sqrt(1.28 * work * rows_us / tile_us))))
     shortest = max(0.0, 2 * mean - tiles)
 
-    def rows_us(per):                                        # (workgroups of up to ``per`` tiles stay whole)
+    def cost(per, factor=1.0):                               # (workgroups of up to ``per`` tiles stay whole)
         whole = max(0.0, (per - shortest) / (tiles - shortest)) if per > shortest else 0.0
-        return 4 + (work / per + wgs * (0.5 - whole)) / 28
+        return factor * tile_us * per + merge_us + (work / per + wgs * (0.5 - whole)) * rows_us
 
-    took = tile_us * per + rows_us(per)
-    if not even:                                             # two rounds; 0.15: they do not meet everywhere
+    took = cost(per)
+    if rounds == 2 and not even:                                             # two rounds; 0.15: they do not meet everywhere
         half = min(tiles, max(least, math.ceil(mean / (500 / wgs - 0.5))))
-        two = 2.3 * tile_us * half + rows_us(half)
+        two = cost(half, 2.3)
         if two < took:
             per, took = half, two
     return (-(-tiles // per), per) if took < tile_us * tiles else (1, tiles)

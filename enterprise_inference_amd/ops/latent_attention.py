@@ -18,7 +18,7 @@ from typing import List, Optional
 import torch
 
 from ._dispatch import check, lib, ptr, require, stream, use_hip, workspace
-from .attention import split_keys
+from .attention import fa_parts, split_keys
 
 ACC_ROWS = 256 * 32        # csrc/kernels/latent_attention.hip: QB * HB * R <= 256 * LAT_ACC_MAX
 
@@ -176,6 +176,25 @@ def _ref_rows(q_abs, q_rot, inv_freq, rot_dims, cache, block_table, positions, g
     return out
 
 
+def flash_parts(wgs: int, lens, context: int, tiles: int, KT: int, window: int, two: bool):
+    """(parts, tiles per part) of a prefill launch of ``wgs`` workgroups for portions of ``lens`` tokens whose
+    block tables reach ``context`` tokens; ``two``: two workgroups fit a CU.
+
+    Up to 64 workgroups, and where ``split_keys`` leaves launches of wide rows uncut, parts go by what a tile and a part
+    cost (``fa_parts``; a tile of 64 keys 3.6 us, 32 keys of R 512 the same, 64 of R 128 1.85).  MI355X, workgroups of up
+    to so many tiles, tiles per part: us.  R 256: 13 of 4: uncut 27.5, 2: 26.9; 37 of 10: 49.2, 5: 38.9, 2: 31.0, 1: 35.1;
+    39 of 6: 34.3, 2: 28.6; 40 of 14: 55.4, 6: 34.5, 3: 29.9; 133 of 18: 73.5, 9: 91.8.  R 512: 38 of 8: 32.0, 4: 32.9, 2:
+    28.0; 157 of 16: 60.8, 8: 51.3, 4: 64.2.  R 128: 32 of 10: 26.6, 2: 17.5; 37 of 10: 25.3, 2: 18.0; 63 of 18: 43.3, 6:
+    26.9, 5: 25.9, 2: 37.9; 108 of 32: 65.9, 6: 34.0, 5: 35.7, 4: 45.3 (split_keys: 6)."""
+    # the merge's time in tiles: those of a workgroup that has a CU to itself are long
+    P, per = split_keys(wgs, tiles, tiles if window > 0 else tiles - max(lens) // (2 * KT),
+                        512 if two else 256, 12 * 64 // KT, 11 if two else 3 * 64 // KT)
+    if wgs <= 64 or (P == 1 and not two):
+        mean = (context - max(lens) + sum(n * n for n in lens) / (2 * sum(lens))) / KT
+        P, per = fa_parts(wgs, tiles, min(mean, tiles), 1.85 if two else 3.6, 6.5, 0.02, 1)
+    return P, per
+
+
 def latent_attention(q_abs: torch.Tensor, q_rot: torch.Tensor, inv_freq: torch.Tensor,
                      rot_dims: int, cache: torch.Tensor, md, gate: Optional[torch.Tensor],
                      scale: float, window: int = 0, sink: Optional[torch.Tensor] = None,
@@ -232,13 +251,11 @@ def latent_attention(q_abs: torch.Tensor, q_rot: torch.Tensor, inv_freq: torch.T
             KT = lib().eia_latent_flash_keys(R, rd)
             hg = -(-H // 16)
             tiles = -(-bt.shape[1] * bs // KT)
-            longest = max(md.prefill_q_lens or [T])
+            lens = md.prefill_q_lens or [T]
             if window > 0:
                 tiles = min(tiles, (window + qb + KT - 2) // KT + 1)
-            # the merge's time in tiles: those of a workgroup that has a CU to itself are long
-            two = R <= 128 and R + rd <= 160
-            P, per = split_keys(n_items * hg, tiles, tiles if window else tiles - longest // (2 * KT),
-                                512 if two else 256, 12 * 64 // KT, 11 if two else 3 * 64 // KT)
+            P, per = flash_parts(n_items * hg, lens, bt.shape[1] * bs, tiles, KT, window,
+                                 R <= 128 and R + rd <= 160)
             pa = None
             if P > 1:
                 pa = torch.empty(n_items * hg * P * 4 * (4 * lib().eia_latent_flash_columns(R, rd) + 1) * 256,

@@ -30,7 +30,7 @@ from typing import List, Optional
 import torch
 
 from ._dispatch import check, lib, ptr, require, stream, use_hip
-from .attention import build_prefill_work, split_keys
+from .attention import build_prefill_work, fa_parts, split_keys
 
 SCALAR_QB = 4            # queries per prefill work item of the scalar-FMA kernel
 MFMA_QB = 16             # ... and of the MFMA kernel (one 16-row tile)
@@ -159,12 +159,20 @@ def flash_parts(n_items: int, spec: WindowSpec, queries: int, longest: int, cont
     ``longest`` queries and whose block tables reach ``context`` tokens; two workgroups fit a CU, three
     of heads up to 64.  MI355X, 8 heads of 128 on 2, one portion, uncut / cut: 4096 tokens causal 110 /
     75 us, 2048 58 / 31, 1000 32 / 23, 96 behind 2000 60 / 23; 16 heads on 4: 2048 causal 59 / 47, 4096 135 /
-    123, 1000 behind 1900 82 / 48, with a window of 1024 39 / 31."""
+    123, 1000 behind 1900 82 / 48, with a window of 1024 39 / 31.
+    Up to 64 workgroups go by what a tile and a part cost (``fa_parts``), in about one part a CU; tiles per part: us.
+    20 of 18: uncut 44.1, 6: 23.0, 3: 18.3, 2: 17.9; 32 of 8: 19.8, 4: 17.0, 2: 15.9; 32 of 16 (96 wide): 29.8, 6: 19.5, 3:
+    16.4; 32 of 32: 59.5, 6: 23.0, 4: 22.7, 2: 25.2; 38 of 18: 43.3, 6: 23.5, 3: 19.0, 2: 20.9; 64 of 16: 32.9, 6: 21.6,
+    4: 19.0, 3: 19.5."""
     tiles = -(-context // 64)
     if spec.window > 0:
         tiles = min(tiles, (spec.window + queries + 62) // 64 + 1 + (spec.keep + 63) // 64)
     narrow = max(spec.dim, spec.vdim) <= 64
-    return split_keys(n_items * (spec.heads * queries // 128), tiles,
+    wgs = n_items * (spec.heads * queries // 128)
+    if wgs <= 64:
+        mean = tiles if spec.window > 0 else tiles - longest / 128
+        return fa_parts(wgs, tiles, mean, 1.1 if narrow else 1.6, 4.5, 0.015, 1)
+    return split_keys(wgs, tiles,
                       tiles if spec.window > 0 else tiles - longest // 128, (3 if narrow else 2) * cus,
                       merge=7 if narrow else 6)
 
@@ -175,20 +183,17 @@ def flash_workspace(n_items: int, spec: WindowSpec, queries: int, parts: int) ->
     return n_items * (spec.heads * queries // 128) * parts * 4 * spec.maps * (4 * cols + 1) * 256
 
 
-def pair_parts(n_items: int, spec: WindowSpec, queries: int, context: int, cus: int = 256):
+def pair_parts(n_items: int, spec: WindowSpec, queries: int, context: int):
     """(parts, 64-key tiles per part) of a flash prefill launch of a differential pair: one workgroup (eight waves) a
-    CU, so launches that leave CUs idle are cut until each has one, down to three tiles a part; fewer than 12 tiles
-    are not worth the second launch.  MI355X, heads of 64 + 64 and 128, window 1024 (18 tiles), us in 1 / 2 / 3 / 4 / 6
+    CU, so launches that leave CUs idle are cut until each has one, as far as the cost of a part allows
+    (``fa_parts``, 2.2 us a tile).  MI355X, heads of 64 + 64 and 128, window 1024 (18 tiles), us in 1 / 2 / 3 / 4 / 6
     parts: 8 workgroups 45 / 29 / 24 / 22 / 20, 46: 49 / 36 / 33 / 32 / 31, 126: 47 / 42 / 51 / 49, 128: 42 / 38 / 45 / 47,
-    250: 53 / 73; window 300 (7 tiles), 128: 26 / 30."""
+    250: 53 / 73; window 300 (7 tiles), 128: 26 / 30.  Short ones, tiles per part: 20 of 6: uncut 18.1, 3: 19.2, 2: 17.4;
+    44 of 14: 34.8, 4: 24.0, 3: 23.6, 1: 32.1; 64 of 8: 25.0, 4: 22.5, 3: 21.5, 1: 27.7; 140 of 4: 19.0, 2: 24.0."""
     tiles = -(-context // 64)
     if spec.window > 0:
         tiles = min(tiles, (spec.window + queries + 62) // 64 + 1 + (spec.keep + 63) // 64)
-    parts = min(cus // max(1, n_items * (spec.heads * queries // 128)), tiles // 3)
-    if tiles < 12 or parts < 2:
-        return 1, tiles
-    per = -(-tiles // parts)
-    return -(-tiles // per), per
+    return fa_parts(n_items * (spec.heads * queries // 128), tiles, tiles, 2.2, 4.0, 0.025, 1)
 
 
 def mix_parts(n_items: int, spec: WindowSpec, context: int, cus: int = 256) -> int:

@@ -17,6 +17,19 @@ def test_parts_cover_and_fit():
                 assert parts == 1 or (wgs <= FA_SLOTS and wgs * parts <= 1024)
 
 
+@pytest.mark.parametrize("KT,two", [(64, True), (64, False), (32, False)])
+@pytest.mark.parametrize("lens,past", [([1], 0), ([9], 1000), ([200, 31], 0), ([500, 3, 90], 5000)])
+@pytest.mark.parametrize("window", [0, 300])
+def test_latent_parts_cover(lens, past, window, KT, two):
+    from enterprise_inference_amd.ops.latent_attention import flash_parts
+    context = -(-(past + max(lens)) // 128) * 128
+    tiles = -(-context // KT) if window == 0 else min(-(-context // KT), window // KT + 2)
+    for wgs in (1, 13, 64, 65, 128, 157, 256, 257, 600):
+        parts, per = flash_parts(wgs, lens, context, tiles, KT, window, two)
+        assert per >= 1 and parts * per >= tiles > (parts - 1) * per
+        assert parts == 1 or wgs * parts <= max(1024, 3 * 512)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("Hq,Hkv", [(8, 2), (6, 3), (3, 1)])
 @pytest.mark.parametrize("qlens,ctxs", [([1, 33, 64, 127], [700, 5, 70, 0]), ([255, 40], [63, 600]), ([300], [0])])

@@ -241,9 +241,10 @@ EIA_API int eia_wkv_scan(const void* r, const void* k, const void* v, const void
 // instead of 1.2e-7 against 64 bits where every second token forgets, in the same time.)
 //
 // Bound by instruction issue (exponentials, conversions, fp32 products; 31 us of vector and 15 us of
-// matrix issue in (3)), not by memory: one 4096-token prompt, 32 heads of 64, bf16 takes 27 + 15 +
-// 64 us on an MI355X, 2091 us token by token.  (3) took 125 us with 2-byte loads and a padded LDS
-// tile for each of r, k, v and the running sums (two workgroups per CU instead of three).
+// matrix issue in (3)), not by memory: one 4096-token prompt, 32 heads of 64, bf16 takes 97 us on an
+// MI355X (25 + 16 + 60 in a trace), 2091 us token by token.  All that a workgroup reads is asked for before
+// it waits for any: with a row of r, u and half the decays behind branches and conversions, the state at
+// its products and a wait for each stored row 105 us (27 + 15 + 64).
 constexpr int WC = 64;                      // tokens per chunk
 constexpr int WD = 64;                      // widest head
 
@@ -251,7 +252,6 @@ struct WkvChunkArgs {
   float* U;                                 // [numbers, H, WD, WD]: contribution, then state before
   float* L;                                 // [numbers, H, WD]: sums of l
   int nseq;
-  int wide;                                 // gate, weight and output rows can be taken 4 at a time
 };
 
 // The chunk of number x; false where there is none or the sequence is skipped.
@@ -261,11 +261,12 @@ EIA_DEV bool wkv_chunk(const WkvArgs& a, int nseq, int x, int& s, int& row0, int
 }
 
 // A chunk's [WC][WD] tile of r, k or v on its way to LDS, zero past the chunk and past D: requested
-// by load, stored as fp32 by store.  VEC: 16-byte loads (D == WD, rows on 16-byte addresses).
+// by load, stored as fp32 by store.  VEC: 16-byte loads (D == WD, rows on 16-byte addresses; then the others' rows too).
 template <typename T, bool VEC>
 struct WkvTile {
+  typedef __attribute__((ext_vector_type(4))) int i32x4;
   static constexpr int E = VEC ? 16 / sizeof(T) : 1, N = WC * WD / (256 * E);
-  T v[N][E];
+  alignas(16) T v[N][E];
   EIA_DEV void load(const void* src, long ld, long hc, int row0, int n, int D) {
 #pragma unroll
     for (int x = 0; x < N; ++x) {
@@ -275,19 +276,22 @@ struct WkvTile {
       else v[x][0] = *p;
     }
   }
+  // (what lies past the chunk is masked away: behind a branch the compiler would ask for some of it only there, and wait)
   EIA_DEV void store(float* tile, int n, int D) const {
 #pragma unroll
     for (int x = 0; x < N; ++x) {
       const int u = threadIdx.x + 256 * x, t = u / (WD / E), i = E * (u % (WD / E));
-      const bool ok = t < n && (VEC || i < D);
-      if constexpr (VEC) {
+      const int keep = t < n && (VEC || i < D) ? -1 : 0;
+      if constexpr (VEC && sizeof(T) == 2) {
+        const i32x4 q = *reinterpret_cast<const i32x4*>(v[x]) & keep;
 #pragma unroll
-        for (int e = 0; e < E; e += 4)
-          *reinterpret_cast<f32x4*>(tile + tile_at<WD>(t, i + e)) =
-              ok ? f32x4{(float)v[x][e], (float)v[x][e + 1], (float)v[x][e + 2], (float)v[x][e + 3]}
-                 : f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int e = 0; e < 4; e += 2)
+          *reinterpret_cast<i32x4*>(tile + tile_at<WD>(t, i + 2 * e)) =
+              i32x4{q[e] << 16, q[e] & (int)0xffff0000, q[e + 1] << 16, q[e + 1] & (int)0xffff0000};
+      } else if constexpr (VEC) {
+        *reinterpret_cast<i32x4*>(tile + tile_at<WD>(t, i)) = *reinterpret_cast<const i32x4*>(v[x]) & keep;
       } else {
-        tile[tile_at<WD>(t, i)] = ok ? (float)v[x][0] : 0.f;
+        tile[tile_at<WD>(t, i)] = __int_as_float(__float_as_int((float)v[x][0]) & keep);
       }
     }
   }
@@ -304,12 +308,15 @@ struct WkvTile {
 
 // Base-2 log decays of channel i, tokens t0 .. t0 + 15 (0 past the chunk and past D): a weight then
 // costs one v_exp_f32.
-template <typename T>
-EIA_DEV void wkv_decays(const WkvArgs& a, long hc, int row0, int n, int t0, int i, float (&l)[16]) {
+// ask: requests of the caller that go out behind the decays' own.
+template <typename T, typename Ask>
+EIA_DEV void wkv_decays(const WkvArgs& a, long hc, int row0, int n, int t0, int i, float (&l)[16], Ask&& ask) {
   const int ic = min(i, a.D - 1);
   const float w0 = ld_f32<T>(static_cast<const T*>(a.w0), hc + ic);
 #pragma unroll
   for (int t = 0; t < 16; ++t) l[t] = a.dec[(long)(row0 + min(t0 + t, n - 1)) * a.ld_dec + hc + ic];
+  ask();
+  __builtin_amdgcn_sched_barrier(0);                   // (else the second half of them behind the first's exponentials)
 #pragma unroll
   for (int t = 0; t < 16; ++t)
     l[t] = (i < a.D && t0 + t < n) ? -1.4426950408889634f * expf(l[t] + w0) : 0.f;
@@ -328,10 +335,11 @@ wkv_chunk_state_kernel(WkvArgs a, WkvChunkArgs c) {
   const int l16 = lane & 15, g4 = lane >> 4;
   const long hc = (long)h * a.D;
   WkvTile<T, VEC> tk, tv;
-  tk.load(a.k, a.ld, hc, row0, n, a.D);
-  tv.load(a.v, a.ld, hc, row0, n, a.D);
   float l[16];
-  wkv_decays<T>(a, hc, row0, n, 16 * w, lane, l);
+  wkv_decays<T>(a, hc, row0, n, 16 * w, lane, l, [&] {
+    tk.load(a.k, a.ld, hc, row0, n, a.D);
+    tv.load(a.v, a.ld, hc, row0, n, a.D);
+  });
   float tot = 0.f;
 #pragma unroll
   for (int t = 0; t < 16; ++t) tot += l[t];
@@ -419,11 +427,14 @@ wkv_chunk_out_kernel(WkvArgs a, WkvChunkArgs c) {
   const int D = a.D, l16 = lane & 15, g4 = lane >> 4, t0 = 16 * w;
   const long hc = (long)h * D;
   WkvTile<T, VEC> tr, tk, tv;
-  tr.load(a.r, a.ld, hc, row0, n, D);
-  tk.load(a.k, a.ld, hc, row0, n, D);
+  const T u = static_cast<const T*>(a.u)[hc + min(lane, D - 1)];
+  __builtin_amdgcn_sched_barrier(0);
   float l[16];
-  wkv_decays<T>(a, hc, row0, n, t0, lane, l);
-  tv.load(a.v, a.ld, hc, row0, n, D);
+  wkv_decays<T>(a, hc, row0, n, t0, lane, l, [&] {
+    tr.load(a.r, a.ld, hc, row0, n, D);
+    tk.load(a.k, a.ld, hc, row0, n, D);
+    tv.load(a.v, a.ld, hc, row0, n, D);
+  });
   tr.store(sr, n, D);
   tk.store(sk, n, D);
 #pragma unroll
@@ -434,7 +445,7 @@ wkv_chunk_out_kernel(WkvArgs a, WkvChunkArgs c) {
     se[2 * w + b][lane] = __builtin_amdgcn_exp2f(tot);
   }
   block_edges<false>(l, sAv, t0, lane);
-  if (w == 0) su[lane] = lane < D ? ld_f32<T>(static_cast<const T*>(a.u), hc + lane) : 0.f;
+  su[lane] = lane < D ? (float)u : 0.f;                // (from every wave: no load behind a branch)
   if (threadIdx.x == 0) swild = 0;
   __syncthreads();
   f32x4 p = {0.f, 0.f, 0.f, 0.f};                      // weights inside the wave's 8-token blocks
@@ -480,6 +491,16 @@ wkv_chunk_out_kernel(WkvArgs a, WkvChunkArgs c) {
   // (weights are formed transposed, keys x queries: their registers are the A operand of P v)
   if (l16 >= 8 && g4 < 2) p += pq;                     // second 8 queries, first 8 keys
   const bool wild = swild;
+  // the first half of the state is on its way during the weights' products, the rest during its own
+  const float* S = c.U + ((long)chunk_number() * a.H + h) * WD * WD + (long)4 * g4 * WD + 4 * l16;
+  f32x4 sq[2][2][4];
+  auto ask = [&](int half) {
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sq[half][x][e] = *reinterpret_cast<const f32x4*>(S + (16 * (2 * half + x) + e) * WD);
+  };
+  ask(0);
   for (int b = w;;) {
     if (wild && b == w) {
       // key by key: in the product a later token's value times a weight of zero would be no number
@@ -519,67 +540,70 @@ wkv_chunk_out_kernel(WkvArgs a, WkvChunkArgs c) {
       rt[x] *= e1 * *reinterpret_cast<const f32x4*>(&se[2 * b][i]);
     }
   }
+  ask(1);
   // the gates and the norm's weight are on their way during the last products
   typedef T T4 __attribute__((ext_vector_type(4)));
   T4 gv[4], nw;
   {
     const T* G = static_cast<const T*>(a.g) + hc;
     const T* NW = static_cast<const T*>(a.norm_w) + hc;
-    if (c.wide) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        gv[i] = *reinterpret_cast<const T4*>(G + (long)(row0 + min(t0 + 4 * g4 + i, n - 1)) * a.ld + 4 * l16);
+    for (int i = 0; i < 4; ++i) {
+      const T* q = G + (long)(row0 + min(t0 + 4 * g4 + i, n - 1)) * a.ld;
+      if constexpr (VEC) {
+        gv[i] = *reinterpret_cast<const T4*>(q + 4 * l16);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) gv[i][j] = q[min(4 * l16 + j, D - 1)];
+      }
+    }
+    if constexpr (VEC) {
       nw = *reinterpret_cast<const T4*>(NW + 4 * l16);
     } else {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int d = min(4 * l16 + j, D - 1);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) gv[i][j] = G[(long)(row0 + min(t0 + 4 * g4 + i, n - 1)) * a.ld + d];
-        nw[j] = NW[d];
-      }
+      for (int j = 0; j < 4; ++j) nw[j] = NW[min(4 * l16 + j, D - 1)];
     }
   }
   if (row0 != a.cu[s] || a.positions[a.cu[s]] != 0) {  // (a fresh sequence's first chunk: S = 0)
-    const float* S = c.U + ((long)chunk_number() * a.H + h) * WD * WD + (long)4 * g4 * WD + 4 * l16;
 #pragma unroll
     for (int x = 0; x < 4; ++x) {
       f32x4 sb[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const f32x4 q = *reinterpret_cast<const f32x4*>(S + (16 * x + e) * WD);
+      for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) sb[j][e] = q[j];
-      }
+        for (int j = 0; j < 4; ++j) sb[j][e] = sq[x >> 1][x & 1][e][j];
 #pragma unroll
       for (int j = 0; j < 4; ++j) o[j] = mfma_f32_k16(rt[x], sb[j], o[j]);
     }
   }
   mfma_settle(o);
-  T* Y = static_cast<T*>(a.y);
+  T4 yv[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {                        // head RMS norm (zeros past D), weight, gate
     float ss = 0.f;
 #pragma unroll
     for (int j = 0; j < 4; ++j) ss += o[j][i] * o[j][i];
-    ss = row16_sum(ss);
-    const int tok = t0 + 4 * g4 + i;
-    if (tok >= n) continue;
-    const float inv = 1.0f / sqrtf(ss / (float)D + a.eps);
-    T* y = Y + (long)(row0 + tok) * a.ldy + hc + 4 * l16;
-    T4 yv;
+    const float ms = row16_sum(ss) / (float)D + a.eps;
+    const float inv = sizeof(T) == 2 ? __builtin_amdgcn_rsqf(ms) : 1.0f / sqrtf(ms);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const float g = (float)gv[i][j];
-      yv[j] = (T)(o[j][i] * inv * (float)nw[j] *
-                  (sizeof(T) == 2 ? g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)) : g / (1.0f + expf(-g))));
+      yv[i][j] = (T)(o[j][i] * inv * (float)nw[j] *
+                     (sizeof(T) == 2 ? g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)) : g / (1.0f + expf(-g))));
     }
-    if (c.wide) {
-      *reinterpret_cast<T4*>(y) = yv;
+    // formed here: behind the branches below, each row's gate would be waited for, and the store before it with it
+    asm volatile("" : "+v"(yv[i]));
+  }
+  T* Y = static_cast<T*>(a.y) + (long)(row0 + t0 + 4 * g4) * a.ldy + hc + 4 * l16;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (t0 + 4 * g4 + i >= n) break;
+    if constexpr (VEC) {
+      *reinterpret_cast<T4*>(Y + i * a.ldy) = yv[i];
     } else {
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        if (4 * l16 + j < D) y[j] = yv[j];
+        if (4 * l16 + j < D) Y[i * a.ldy + j] = yv[i][j];
     }
   }
 }
@@ -607,11 +631,12 @@ EIA_API int eia_wkv_scan_chunked(const void* r, const void* k, const void* v, co
   if (nseq == 0 || rows == 0) return EIA_OK;
   WkvArgs a{r, k, v, g, ld, dec, ld_dec, w0, u, norm_w, S, prev, x, W, slots, cu, positions,
             seq_lens, y, ldy, eps, H, D, split};
+  const WkvChunkArgs c{U, L, nseq};
+  // 16-byte rows of r, k and v, gates, weights and outputs four at a time
   const int es = is_bf16 ? 2 : 4;
-  const uintptr_t io = (uintptr_t)g | (uintptr_t)y | (uintptr_t)norm_w | (uintptr_t)(ld * es) | (uintptr_t)(ldy * es);
-  WkvChunkArgs c{U, L, nseq, D == WD && io % (4 * es) == 0};
-  const uintptr_t any = (uintptr_t)r | (uintptr_t)k | (uintptr_t)v | (uintptr_t)(ld * (is_bf16 ? 2 : 4));
-  const bool vec = D == WD && any % 16 == 0;
+  const uintptr_t any = (uintptr_t)r | (uintptr_t)k | (uintptr_t)v | (uintptr_t)(ld * es);
+  const uintptr_t io = (uintptr_t)g | (uintptr_t)y | (uintptr_t)norm_w | (uintptr_t)(ldy * es);
+  const bool vec = D == WD && any % 16 == 0 && io % (4 * es) == 0;
   if (is_bf16 && vec) wkv_chunked<bf16_t, true>(a, c, rows, st);
   else if (is_bf16) wkv_chunked<bf16_t, false>(a, c, rows, st);
   else if (vec) wkv_chunked<float, true>(a, c, rows, st);

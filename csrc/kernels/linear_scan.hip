@@ -593,29 +593,33 @@ EIA_DEV void ls_stage_v(const ScanArgs& a, int row0, int n, int h, int t0, T* sv
 // What the logs of the chunk's token threadIdx.x are formed from (threads 0 .. LK - 1): the decay or the two gate
 // pre-activations of the token and, for the second wave, of the token 64 before it.
 struct LsGates {
-  float xi[2], xf[2];
+  unsigned xi[2], xf[2];                    // as they lie in memory: a conversion here would wait for them
+  float decay;
 };
 template <typename T> EIA_DEV LsGates ls_log_load(const ScanArgs& a, int row0, int n, int h) {
+  using Bits = typename std::conditional<sizeof(T) == 2, unsigned short, unsigned>::type;
   LsGates g = {};
   const int t = threadIdx.x;
-  if (t >= LK) return g;
   if (a.mode == 0) {
-    g.xi[0] = a.decay[h];
-    return g;
-  }
+    g.decay = a.decay[h];
+  } else if (__builtin_amdgcn_readfirstlane(t) < LK) {
 #pragma unroll
-  for (int y = 0; y < 2; ++y) {
-    const T* x = static_cast<const T*>(a.x) + (long)(row0 + min(y ? t & 63 : t, n - 1)) * a.ld + h;
-    g.xi[y] = ld_f32<T>(x, a.i_off);
-    g.xf[y] = ld_f32<T>(x, a.f_off);
+    for (int y = 0; y < 2; ++y) {
+      const Bits* x = static_cast<const Bits*>(a.x) + (long)(row0 + min(y ? t & 63 : t, n - 1)) * a.ld + h;
+      g.xi[y] = x[a.i_off];
+      g.xf[y] = x[a.f_off];
+    }
   }
   return g;
 }
 // Mode 1: log decay l and log weight b of the token, m the running maximum with it, from the maximum m0 before the
 // chunk (-inf: none, what lies before the chunk weighs nothing).  m_t = max(f_t + m_(t-1), i_t) is a scan over pairs
 // (sum of f, maximum behind it).  -> the pair up to and with the token.
-EIA_DEV float2 ls_log_gates(const ScanArgs& a, int n, const LsGates& g, float m0, float& l, float& b, float& m) {
+template <typename T>
+EIA_DEV float2 ls_log_gates(const ScanArgs& a, int n, LsGates g, float m0, float& l, float& b, float& m) {
   const int t = threadIdx.x, lane = t & 63;
+  asm volatile("" : "+v"(g.xi[0]), "+v"(g.xi[1]), "+v"(g.xf[0]), "+v"(g.xf[1]));     // (keeps the conversions here)
+  auto value = [](unsigned u) { return __uint_as_float(sizeof(T) == 2 ? u << 16 : u); };
   auto soft = [&](float x) { return a.cap > 0.f ? a.cap * tanhf(x / a.cap) : x; };
   auto join = [](float2 p, float2 q) { return make_float2(p.x + q.x, fmaxf(p.y + q.x, q.y)); };
   auto scan = [&](float2 q) {               // inclusive over the lanes
@@ -627,10 +631,10 @@ EIA_DEV float2 ls_log_gates(const ScanArgs& a, int n, const LsGates& g, float m0
     return q;
   };
   const float2 none = make_float2(0.f, -INFINITY);
-  const float gi = soft(g.xi[0]), gf = ls_logsigmoid(soft(g.xf[0]));
+  const float gi = soft(value(g.xi[0])), gf = ls_logsigmoid(soft(value(g.xf[0])));
   float2 first = none;                      // of the 64 tokens before the second wave's
   if (t >= 64) {
-    first = scan(lane < n ? make_float2(ls_logsigmoid(soft(g.xf[1])), soft(g.xi[1])) : none);
+    first = scan(lane < n ? make_float2(ls_logsigmoid(soft(value(g.xf[1]))), soft(value(g.xi[1]))) : none);
     first = make_float2(__shfl(first.x, 63, 64), __shfl(first.y, 63, 64));
   }
   const float2 p = join(first, scan(t < n ? make_float2(gf, gi) : none));
@@ -645,15 +649,16 @@ EIA_DEV float2 ls_log_gates(const ScanArgs& a, int n, const LsGates& g, float m0
 }
 // Sums of l over 16-token blocks: pre up to and with a token, suf behind it, tot of whole blocks;
 // mb: log2 b, sl: l, mx: m (mode 1).  Threads 0 .. LK - 1.  pair: where mode 1's pair of the chunk goes, or null.
+template <typename T>
 EIA_DEV void ls_chunk_logs(const ScanArgs& a, int n, const LsGates& g, float m0, float* pre, float* suf, float* tot,
                            float* mb, float* sl, float* mx, float2* pair) {
   const int t = threadIdx.x;
   if (t >= LK) return;
   float l, b = 0.f;
   if (a.mode == 0) {
-    l = t < n ? logf(g.xi[0]) : 0.f;
+    l = t < n ? logf(g.decay) : 0.f;
   } else {
-    const float2 p = ls_log_gates(a, n, g, m0, l, b, mx[t]);
+    const float2 p = ls_log_gates<T>(a, n, g, m0, l, b, mx[t]);
     if (pair && t == LK - 1) *pair = p;
   }
   l *= LS_LOG2E;
@@ -935,7 +940,7 @@ ls_chunk_state_kernel(ScanArgs a, KChunkArgs c) {
   const long at = (long)chunk_number() * a.H + h;
   const LsChunk k{row0, n, h, pre, suf, mb, tot, sl};
   auto logs = [&] {
-    ls_chunk_logs(a, n, g, -INFINITY, pre, suf, tot, mb, sl, mx, reinterpret_cast<float2*>(c.G) + at);
+    ls_chunk_logs<T>(a, n, g, -INFINITY, pre, suf, tot, mb, sl, mx, reinterpret_cast<float2*>(c.G) + at);
   };
   if constexpr (BF) {
     if (!ls_state_bf16<VEC, ROT, MX>(a, c, k, at, tiles, logs)) ls_state_fp32<T, VEC, ROT, MX>(a, c, k, at, tiles);
@@ -1414,7 +1419,7 @@ EIA_DEV bool ls_out_bf16(const ScanArgs& a, const KChunkArgs& c, const LsChunk& 
   return !__syncthreads_or(bad);
 }
 
-// Two workgroups on a CU where the LDS holds two: 128 registers a lane, of which aligned, unrotated heads of 128 spill 11.
+// Two workgroups on a CU where the LDS holds two: 128 registers a lane, of which aligned, unrotated heads of 128 spill 7.
 // One with all registers: four gated prompts of up to 2000 tokens, 16 heads, the op 123 -> 150 us.  Heads of 64, unrotated:
 // three, 80 registers (82, and two, without the bound: five prompts of up to 1100 tokens, 32 heads, 76 -> 82 us).
 template <typename T, bool VEC, bool ROT, int MX>
@@ -1433,10 +1438,14 @@ ls_chunk_out_kernel(ScanArgs a, KChunkArgs c) {
   const LsGates g = ls_log_load<T>(a, row0, n, h);
   const float m0 = a.mode == 1 ? c.m0[at] : 0.f;
   const bool state = row0 != a.cu[s] || a.positions[a.cu[s]] != 0;   // (else a fresh sequence: S = 0)
-  if (state && a.mode == 1 && threadIdx.x < MX)
-    sn[threadIdx.x] = c.U[(at * c.DP + min((int)threadIdx.x, c.DP - 1)) * c.UW + c.VP];
+  float sv = 0.f;                                      // (stored with the logs: a store here would wait for it)
+  if (a.mode == 1 && __builtin_amdgcn_readfirstlane(threadIdx.x) < MX)
+    sv = c.U[(at * c.DP + min((int)threadIdx.x, c.DP - 1)) * c.UW + c.VP];
   const LsChunk k{row0, n, h, pre, suf, mb, tot, sl};
-  auto logs = [&] { ls_chunk_logs(a, n, g, m0, pre, suf, tot, mb, sl, mx, nullptr); };
+  auto logs = [&] {
+    ls_chunk_logs<T>(a, n, g, m0, pre, suf, tot, mb, sl, mx, nullptr);
+    if (threadIdx.x < MX) sn[threadIdx.x] = sv;
+  };
   f32x4 o[MX / 16];
   float rs;
   if constexpr (BF) {
@@ -1468,11 +1477,15 @@ ls_chunk_out_kernel(ScanArgs a, KChunkArgs c) {
       }
     }
   }
+  if (NW) {
 #pragma unroll
-  for (int x = 0; x < MX / 64; ++x)
+    for (int x = 0; x < MX / 64; ++x)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      nw[x][j] = NW ? NW[(long)h * a.norm_h + min(64 * x + 4 * l16 + j, Dv - 1)] : (T)1.f;
+      for (int j = 0; j < 4; ++j) nw[x][j] = NW[(long)h * a.norm_h + min(64 * x + 4 * l16 + j, Dv - 1)];
+  } else {
+#pragma unroll
+    for (int x = 0; x < MX / 64; ++x) nw[x] = T4{(T)1.f, (T)1.f, (T)1.f, (T)1.f};
+  }
   // normaliser, head RMS norm, weight, gate.  What is one number a token is formed by one lane of the sixteen that
   // hold it.
   float ss[4], den = 1.f;

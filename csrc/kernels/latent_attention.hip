@@ -355,8 +355,9 @@ EIA_API int eia_latent_attn(const void* qa, long qa_st, long qa_sh, const void* 
 //
 // Bound by latency: a row's 64-key tiles are a chain of cache loads and two barriers, and the launch
 // lasts as long as the longest partition.  MI355X, 48 rows at up to 4096 tokens, window 1024, 16
-// heads, R 512 + 64: 20.4 + 4.0 us in five partitions, 7 of them before the first tile is there and 2.6 a tile; (pages read beside
-// the position, not behind it: 25.9 -> 25.8); 200 rows at up to 2500 tokens, no window, with
+// heads, R 512 + 64: 19.8 + 4.0 us in five partitions, 6 of them before the first tile is there and 2.6 a tile (pages read beside
+// the position, not behind it: 25.9 -> 25.8; queries and angles asked for before the first rows, not behind them and two
+// barriers: 24.5 -> 23.9); 200 rows at up to 2500 tokens, no window, with
 // 16 heads 153 -> 134 us and with 64 heads 499 -> 437 us since a tile's page is known before its fetch and
 // its LDS reads are asked for before the first product; R 128 + 32 with 64 heads 120 -> 115 us, R 256 + 64
 // 292 -> 292 us.  (Two tiles of cache loads in flight, in registers: 27 us instead of 24; the reads held in
@@ -431,33 +432,25 @@ latent_decode_kernel(LatentAttnArgs a) {
     }
   };
   look(k_begin);
-  fetch(k_begin);
-  look(k_begin + KT);
-
-  // the rotary query parts, rotated once into LDS: the heads of a row turn by the same angles
+  // what the queries are formed from is asked for before the first rows, of whose arrival nothing then waits
   const int hp = a.rot_dims >> 1, npass = a.rd - a.rot_dims;
-  for (int i = tid; i < hp; i += NT) {
-    float sn, cs;
-    sincosf((float)qpos * a.inv_freq[i], &sn, &cs);
-    rot[i] = make_float2(cs * a.rot_amp, sn * a.rot_amp);
+  const bf16_t* qrb = static_cast<const bf16_t*>(a.qr) + (long)row * a.qr_st + (long)h0 * a.qr_sh;
+  auto pair = [&](int e, int& m, int& ia, int& ib) {    // pair e of the rotary parts: head, places
+    m = e / hp;
+    const int i = e - m * hp;
+    ia = a.rot_half ? i : 2 * i;
+    ib = a.rot_half ? i + hp : 2 * i + 1;
+    return i;
+  };
+  const float turn = tid < hp ? a.inv_freq[tid] : 0.f;
+  unsigned pu = 0, pv = 0;                              // (as they lie in memory: a conversion here would wait for them)
+  if (tid < nh * hp) {
+    int m, ia, ib;
+    pair(tid, m, ia, ib);
+    const unsigned short* src = reinterpret_cast<const unsigned short*>(qrb) + (long)m * a.qr_sh;
+    pu = src[ia];
+    pv = src[ib];
   }
-  __syncthreads();
-  bf16_t* qrs = tiles;                                  // [16][rd]
-  const bf16_t* qrb = static_cast<const bf16_t*>(a.qr) + (long)row * a.qr_st;
-  for (int e = tid; e < nh * hp; e += NT) {
-    const int m = e / hp, i = e - m * hp;
-    const bf16_t* src = qrb + (long)(h0 + m) * a.qr_sh;
-    const int ia = a.rot_half ? i : 2 * i, ib = a.rot_half ? i + hp : 2 * i + 1;
-    const float u = bf2f(src[ia]), v = bf2f(src[ib]);
-    const float2 cs = rot[i];
-    qrs[m * a.rd + ia] = f2bf(u * cs.x - v * cs.y);
-    qrs[m * a.rd + ib] = f2bf(v * cs.x + u * cs.y);
-  }
-  for (int e = tid; e < nh * npass; e += NT) {         // entries past rot_dims pass unchanged
-    const int m = e / npass, d = a.rot_dims + e - m * npass;
-    qrs[m * a.rd + d] = qrb[(long)(h0 + m) * a.qr_sh + d];
-  }
-  __syncthreads();
   const bool ok = l16 < nh;                             // this lane's head
   const int h = h0 + (ok ? l16 : 0);
   const int kg = w & 3, s0 = NS * (w >> 2);             // the wave's keys of a tile, and steps of their rows
@@ -465,23 +458,54 @@ latent_decode_kernel(LatentAttnArgs a) {
   {
     // R % 8 == 0 and rd % 8 == 0: a lane's eight entries lie wholly in one of the two parts
     const bf16_t* qa = static_cast<const bf16_t*>(a.qa) + (long)row * a.qa_st + (long)h * a.qa_sh;
-    const bool vec = ((reinterpret_cast<uintptr_t>(a.qa) | (uintptr_t)(a.qa_st * 2) | (uintptr_t)(a.qa_sh * 2)) & 15) == 0;
+    if (((reinterpret_cast<uintptr_t>(a.qa) | (uintptr_t)(a.qa_st * 2) | (uintptr_t)(a.qa_sh * 2)) & 15) == 0) {
 #pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      const int d = 32 * (s0 + s) + 8 * g4;
-      bf16x8 v = zero8;
-      if (ok && d < Dk) {
-        if (d >= R) {
-          v = *reinterpret_cast<const bf16x8*>(qrs + l16 * a.rd + (d - R));
-        } else if (vec) {
-          v = *reinterpret_cast<const bf16x8*>(qa + d);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) v[e] = qa[d + e];
-        }
+      for (int s = 0; s < NS; ++s) {
+        const int d = 32 * (s0 + s) + 8 * g4;
+        qf[s] = *reinterpret_cast<const bf16x8*>(qa + (d < R ? d : 0));
       }
-      qf[s] = v;
+    } else {
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        const int d = 32 * (s0 + s) + 8 * g4;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) qf[s][e] = qa[(d < R ? d : 0) + e];
+      }
     }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  fetch(k_begin);
+  look(k_begin + KT);
+
+  // the rotary query parts, rotated once into LDS: the heads of a row turn by the same angles
+  for (int i = tid; i < hp; i += NT) {
+    float sn, cs;
+    sincosf((float)qpos * (i == tid ? turn : a.inv_freq[i]), &sn, &cs);
+    rot[i] = make_float2(cs * a.rot_amp, sn * a.rot_amp);
+  }
+  __syncthreads();
+  bf16_t* qrs = tiles;                                  // [16][rd]
+  asm volatile("" : "+v"(pu), "+v"(pv));
+  for (int e = tid; e < nh * hp; e += NT) {
+    int m, ia, ib;
+    const int i = pair(e, m, ia, ib);
+    const bf16_t* src = qrb + (long)m * a.qr_sh;
+    const float u = e == tid ? __uint_as_float(pu << 16) : bf2f(src[ia]);
+    const float v = e == tid ? __uint_as_float(pv << 16) : bf2f(src[ib]);
+    const float2 cs = rot[i];
+    qrs[m * a.rd + ia] = f2bf(u * cs.x - v * cs.y);
+    qrs[m * a.rd + ib] = f2bf(v * cs.x + u * cs.y);
+  }
+  for (int e = tid; e < nh * npass; e += NT) {         // entries past rot_dims pass unchanged
+    const int m = e / npass, d = a.rot_dims + e - m * npass;
+    qrs[m * a.rd + d] = qrb[(long)m * a.qr_sh + d];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    const int d = 32 * (s0 + s) + 8 * g4;
+    if (!ok || d >= Dk) qf[s] = zero8;
+    else if (d >= R) qf[s] = *reinterpret_cast<const bf16x8*>(qrs + l16 * a.rd + (d - R));
   }
   __syncthreads();                                      // the rotary parts make room for tiles
   stash(0, k_begin);

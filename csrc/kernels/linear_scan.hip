@@ -476,7 +476,6 @@ struct KChunkArgs {
   float* la;                                // [rows, H * D]: log2 a (mode 2)
   float2* rot;                              // [rows, rot_dims / 2]: cos, sin
   int nseq, rows, DP, VP, UW;               // UW: VP, and in mode 1 four more (the normaliser, 0, 0, 0)
-  bool wide = false;                        // per channel: gate, weight and output rows can be taken 4 at a time
 };
 
 // The chunk of number x; false where there is none or the sequence is skipped.
@@ -1953,6 +1952,7 @@ EIA_DEV void gl_decays(const ScanArgs& a, const KChunkArgs& c, int h, int row0, 
   const float* p = c.la + (long)h * a.D + min(i, a.D - 1);
 #pragma unroll
   for (int t = 0; t < 16; ++t) l[t] = p[(long)(row0 + min(t0 + t, n - 1)) * a.H * a.D];
+  __builtin_amdgcn_sched_barrier(0);                   // all of them, and the rows before them, are asked for first
 #pragma unroll
   for (int t = 0; t < 16; ++t) l[t] = (i < a.D && t0 + t < n) ? l[t] : 0.f;
 }
@@ -1973,10 +1973,11 @@ struct GlTile {
     for (int x = 0; x < 2; ++x) {
       const int u = threadIdx.x + 256 * x, t = u >> 3, i = 8 * (u & 7);
 #pragma unroll
-      for (int e = 0; e < 8; e += 4)
-        *reinterpret_cast<f32x4*>(tile + tile_at<GD>(t, i + e)) =
-            t < n ? f32x4{v[x][e], v[x][e + 1], v[x][e + 2], v[x][e + 3]} * scale
-                  : f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int e = 0; e < 8; e += 4) {
+        f32x4 f = f32x4{v[x][e], v[x][e + 1], v[x][e + 2], v[x][e + 3]} * scale;
+        asm volatile("" : "+v"(f));                    // (else some rows are asked for behind the choice, and waited for)
+        *reinterpret_cast<f32x4*>(tile + tile_at<GD>(t, i + e)) = t < n ? f : f32x4{0.f, 0.f, 0.f, 0.f};
+      }
     }
   }
 };
@@ -1985,7 +1986,7 @@ struct GlTile {
 template <typename T, bool VEC, int NV>
 struct GlValues {
   static constexpr int E = VEC ? 16 / (int)sizeof(T) : 1, W = 64 * NV, N = GC * W / (256 * E);
-  T v[N][E];
+  alignas(16) T v[N][E];
   EIA_DEV void load(const ScanArgs& a, int row0, int n, int h) {
     const T* X = static_cast<const T*>(a.x) + a.v_off + (long)h * a.Dv;
 #pragma unroll
@@ -1997,18 +1998,21 @@ struct GlValues {
     }
   }
   EIA_DEV void store(float* tile, int n, int Dv) const {
+    typedef __attribute__((ext_vector_type(4))) int i32x4;
 #pragma unroll
     for (int x = 0; x < N; ++x) {
       const int u = threadIdx.x + 256 * x, t = u / (W / E), i = E * (u % (W / E));
-      const bool ok = t < n && i < Dv;
-      if constexpr (VEC) {
+      const int keep = t < n && i < Dv ? -1 : 0;
+      if constexpr (VEC && sizeof(T) == 2) {
+        const i32x4 q = *reinterpret_cast<const i32x4*>(v[x]) & keep;
 #pragma unroll
-        for (int e = 0; e < E; e += 4)
-          *reinterpret_cast<f32x4*>(tile + tile_at<W>(t, i + e)) =
-              ok ? f32x4{(float)v[x][e], (float)v[x][e + 1], (float)v[x][e + 2], (float)v[x][e + 3]}
-                 : f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int e = 0; e < 4; e += 2)
+          *reinterpret_cast<i32x4*>(tile + tile_at<W>(t, i + 2 * e)) =
+              i32x4{q[e] << 16, q[e] & (int)0xffff0000, q[e + 1] << 16, q[e + 1] & (int)0xffff0000};
+      } else if constexpr (VEC) {
+        *reinterpret_cast<i32x4*>(tile + tile_at<W>(t, i)) = *reinterpret_cast<const i32x4*>(v[x]) & keep;
       } else {
-        tile[tile_at<W>(t, i)] = ok ? (float)v[x][0] : 0.f;
+        tile[tile_at<W>(t, i)] = __int_as_float(__float_as_int((float)v[x][0]) & keep);
       }
     }
   }
@@ -2124,9 +2128,9 @@ gl_out_kernel(ScanArgs a, KChunkArgs c) {
   GlValues<T, VEC, NV> tv;
   tq.load(a, c, row0, n, a.q_off + (long)h * a.D);
   tk.load(a, c, row0, n, a.k_off + (long)h * a.D);
+  tv.load(a, row0, n, h);
   float l[16];
   gl_decays(a, c, h, row0, n, t0, lane, l);
-  tv.load(a, row0, n, h);
   tq.store(sq, n, a.qscale);
   tk.store(sk, n, a.kscale);
 #pragma unroll
@@ -2179,6 +2183,16 @@ gl_out_kernel(ScanArgs a, KChunkArgs c) {
   for (int j = 0; j < 4 * NV; ++j) o[j] = f32x4{0.f, 0.f, 0.f, 0.f};
   // (weights are formed transposed, keys x queries: their registers are the A operand of P v)
   if (l16 >= 8 && g4 < 2) p += pq;                     // second 8 queries, first 8 keys
+  // the first quarter of the state is on its way during the weights' products, the next during those of the one before
+  const float* S = c.U + ((long)chunk_number() * a.H + h) * GD * W + (long)4 * g4 * W + 4 * l16;
+  f32x4 sq4[2][NV][4];
+  auto ask = [&](int x) {
+#pragma unroll
+    for (int z = 0; z < NV; ++z)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sq4[x & 1][z][e] = *reinterpret_cast<const f32x4*>(S + (16 * x + e) * W + 64 * z);
+  };
+  ask(0);
   for (int b = w;;) {
     f32x4 vb[4 * NV];
 #pragma unroll
@@ -2212,68 +2226,82 @@ gl_out_kernel(ScanArgs a, KChunkArgs c) {
 #pragma unroll
     for (int z = 0; z < NV; ++z) {
       const int d = 64 * z + 4 * l16;
-      if (c.wide) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          gv[i][z] = *reinterpret_cast<const T4*>(G + (row0 + min(t0 + 4 * g4 + i, n - 1)) * a.ld + min(d, Dv - 4));
-        if (a.norm_w) nw[z] = *reinterpret_cast<const T4*>(NW + min(d, Dv - 4));
-      } else {
+      for (int i = 0; i < 4; ++i) {
+        const T* q = G + (row0 + min(t0 + 4 * g4 + i, n - 1)) * a.ld;
+        if constexpr (VEC) {
+          gv[i][z] = *reinterpret_cast<const T4*>(q + min(d, Dv - 4));
+        } else {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int dj = min(d + j, Dv - 1);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) gv[i][z][j] = G[(row0 + min(t0 + 4 * g4 + i, n - 1)) * a.ld + dj];
-          if (a.norm_w) nw[z][j] = NW[dj];
+          for (int j = 0; j < 4; ++j) gv[i][z][j] = q[min(d + j, Dv - 1)];
         }
       }
-      if (!a.norm_w) nw[z] = T4{(T)1.f, (T)1.f, (T)1.f, (T)1.f};
+    }
+    if (a.norm_w) {
+#pragma unroll
+      for (int z = 0; z < NV; ++z) {
+        const int d = 64 * z + 4 * l16;
+        if constexpr (VEC) {
+          nw[z] = *reinterpret_cast<const T4*>(NW + min(d, Dv - 4));
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) nw[z][j] = NW[min(d + j, Dv - 1)];
+        }
+      }
+    } else {
+#pragma unroll
+      for (int z = 0; z < NV; ++z) nw[z] = T4{(T)1.f, (T)1.f, (T)1.f, (T)1.f};
     }
   }
   if (row0 != a.cu[s] || a.positions[a.cu[s]] != 0) {  // (a fresh sequence's first chunk: S = 0)
-    const float* S = c.U + ((long)chunk_number() * a.H + h) * GD * W + (long)4 * g4 * W + 4 * l16;
 #pragma unroll
-    for (int x = 0; x < 4; ++x)
+    for (int x = 0; x < 4; ++x) {
+      if (x < 3) ask(x + 1);
 #pragma unroll
       for (int z = 0; z < NV; ++z) {
         f32x4 sb[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const f32x4 q = *reinterpret_cast<const f32x4*>(S + (16 * x + e) * W + 64 * z);
+        for (int e = 0; e < 4; ++e)
 #pragma unroll
-          for (int j = 0; j < 4; ++j) sb[j][e] = q[j];
-        }
+          for (int j = 0; j < 4; ++j) sb[j][e] = sq4[x & 1][z][e][j];
 #pragma unroll
         for (int j = 0; j < 4; ++j) o[4 * z + j] = mfma_f32_k16(rt[x], sb[j], o[4 * z + j]);
       }
+    }
   }
   mfma_settle(o);
-  T* Y = static_cast<T*>(a.y);
+  T4 yv[4][NV];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {                        // head RMS norm (zeros past Dv), weight, gate
-    const int t = t0 + 4 * g4 + i;
     float ss = 0.f;
 #pragma unroll
     for (int j = 0; j < 4 * NV; ++j) ss += o[j][i] * o[j][i];
-    ss = row16_sum(ss);
-    if (t >= n) continue;
-    const float inv = a.out_scale / sqrtf(ss / (float)Dv + a.eps);
+    const float ms = row16_sum(ss) / (float)Dv + a.eps;
+    const float inv = a.out_scale * (sizeof(T) == 2 ? __builtin_amdgcn_rsqf(ms) : 1.0f / sqrtf(ms));
 #pragma unroll
     for (int z = 0; z < NV; ++z) {
-      const int d = 64 * z + 4 * l16;
-      T* y = Y + (long)(row0 + t) * a.ldy + (long)h * Dv + d;
-      T4 yv;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const float g = (float)gv[i][z][j];
         const float sig = sizeof(T) == 2 ? __builtin_amdgcn_rcpf(1.0f + __expf(-g)) : 1.0f / (1.0f + expf(-g));
-        yv[j] = (T)(o[4 * z + j][i] * inv * (float)nw[z][j] * (a.gate_act == 0 ? g * sig : sig));
+        yv[i][z][j] = (T)(o[4 * z + j][i] * inv * (float)nw[z][j] * (a.gate_act == 0 ? g * sig : sig));
       }
-      if (c.wide) {
-        if (d < Dv) *reinterpret_cast<T4*>(y) = yv;
+      asm volatile("" : "+v"(yv[i][z]));               // (formed before the branches of the stores)
+    }
+  }
+  T* Y = static_cast<T*>(a.y) + (long)(row0 + t0 + 4 * g4) * a.ldy + (long)h * Dv;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (t0 + 4 * g4 + i >= n) break;
+#pragma unroll
+    for (int z = 0; z < NV; ++z) {
+      const int d = 64 * z + 4 * l16;
+      if constexpr (VEC) {
+        if (d < Dv) *reinterpret_cast<T4*>(Y + i * a.ldy + d) = yv[i][z];
       } else {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          if (d + j < Dv) y[j] = yv[j];
+          if (d + j < Dv) Y[i * a.ldy + d + j] = yv[i][z][j];
       }
     }
   }
@@ -2293,14 +2321,14 @@ static void gl_launch(const ScanArgs& a, const KChunkArgs& c, hipStream_t st) {
 }
 
 template <typename T>
-static void gl_forms(const ScanArgs& a, KChunkArgs c, hipStream_t st) {
+static void gl_forms(const ScanArgs& a, const KChunkArgs& c, hipStream_t st) {
   constexpr int A = 16 / (int)sizeof(T);               // elements in 16 bytes
-  const uintptr_t io = reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.y) | reinterpret_cast<uintptr_t>(a.norm_w);
-  c.wide = io % (4 * sizeof(T)) == 0 && (a.ld | a.ldy | a.g_off | a.Dv | a.norm_h) % 4 == 0;
+  // gates, weights and outputs move four at a time where rows of q, k and v move by 16 bytes
+  const uintptr_t io = reinterpret_cast<uintptr_t>(a.y) | reinterpret_cast<uintptr_t>(a.norm_w);
   const int rot8 = a.rot_dims ? (a.rot_half ? a.rot_dims / 2 : a.rot_dims) : 0;
   const bool vec = reinterpret_cast<uintptr_t>(a.x) % 16 == 0 &&
                    (a.ld | a.q_off | a.k_off | a.v_off) % A == 0 && a.D % 8 == 0 && a.Dv % 8 == 0 &&
-                   rot8 % 8 == 0;
+                   rot8 % 8 == 0 && io % (4 * sizeof(T)) == 0 && (a.ldy | a.g_off | a.norm_h) % 4 == 0;
   const bool wide = a.Dv > 64, rot = a.rot_dims > 0;
 #define GL_GO(V, R) \
   do { if (wide) gl_launch<T, V, R, 2>(a, c, st); else gl_launch<T, V, R, 1>(a, c, st); } while (0)

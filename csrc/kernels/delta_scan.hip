@@ -246,7 +246,6 @@ struct DeltaChunkArgs {
   int ncu, nseq;                            // units of 32 state columns
   int whole, parts;                         // the workgroups of (1): dn_solve
   DeltaSpread spread;                       // the workgroups of (2) over the XCDs
-  int vec;                                  // out, gate and weight rows can be taken 4 at a time
 };
 
 EIA_DEV f32x4 mm(f32x4 a, f32x4 b, f32x4 c) { return mfma_f32_k16(a, b, c); }
@@ -969,65 +968,65 @@ delta_chunk_scan_kernel(DeltaArgs a, DeltaChunkArgs c) {
 // grid, so that those of a key head run on the XCD that formed them where G is eight.  Bound by memory.  (Four heads, chunks
 // first: three prompts of 155 tokens, 8 heads 32.9 -> 30.8 us, three of up to 1500, 16 heads 146.0 -> 145.2.)  Of bf16
 // outputs, whose rounding is 2^-9, the root and silu take the instructions' own reciprocal and exponential (1 ulp, some
-// 2^-21): with divisions and expf vector instructions filled 13 of 19.2 us, now the kernel takes 16.6; error of the
-// outputs against 64 bits 1.7e-3 as before.
+// 2^-21): with divisions and expf vector instructions filled 13 of 19.2 us, without the kernel takes 16.6; error of the
+// outputs against 64 bits 1.7e-3 as before.  All five reads of a thread are in flight together (the second head's behind
+// the first one's gate: the op 128.6 us instead of 125).
 constexpr int DN_HEADS = 2;
-template <typename T, int LN>
+template <typename T, int LN, bool VEC>
 __global__ void __launch_bounds__(256)
 delta_chunk_norm_kernel(DeltaArgs a, DeltaChunkArgs c) {
   constexpr int NH = DN_HEADS;
+  typedef T T4 __attribute__((ext_vector_type(4)));
   const int ch = blockIdx.y, sub = threadIdx.x % LN, t = blockIdx.z * (256 / LN) + threadIdx.x / LN;
   // no branch before the store: the outputs are asked for beside the chunk, the gates beside its slot
   const int row0 = c.chunks[4 * ch + 1], n = c.chunks[4 * ch + 2], slot = a.slots[c.chunks[4 * ch]];
   const int col = 4 * sub, Dv = a.Dv, VQ = 32 * c.ncu;
   const long r = row0 + min(t, n - 1);
   f32x4 o[NH];
-  float gv[NH][4], nw[4];
-  const T* GT = static_cast<const T*>(a.g) + r * a.ldg;
+  T4 gv[NH], nw;
+  const T *GT = static_cast<const T*>(a.g) + r * a.ldg, *NW = static_cast<const T*>(a.norm_w);
+  auto four = [&](const T* p) {
+    if constexpr (VEC) return *reinterpret_cast<const T4*>(p + min(col, Dv - 4));
+    T4 v;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = p[min(col + j, Dv - 1)];
+    return v;
+  };
 #pragma unroll
   for (int x = 0; x < NH; ++x) {
     const int h = min((int)blockIdx.x * NH + x, a.H - 1);
     o[x] = *reinterpret_cast<const f32x4*>(c.O + (((long)ch * DC + t) * a.H + h) * VQ + min(col, VQ - 4));
-    if (c.vec) {
-      typedef T T4 __attribute__((ext_vector_type(4)));
-      const T4 z = *reinterpret_cast<const T4*>(GT + (long)h * Dv + min(col, Dv - 4));
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const T zj = z[j];
-        gv[x][j] = ld_f32<T>(&zj, 0);
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) gv[x][j] = ld_f32<T>(GT, (long)h * Dv + min(col + j, Dv - 1));
-    }
+    gv[x] = four(GT + (long)h * Dv);
   }
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-    nw[j] = ld_f32<T>(static_cast<const T*>(a.norm_w), min(col + j, Dv - 1)) * a.out_scale;
+  nw = four(NW);
+  T4 v[NH];
 #pragma unroll
   for (int x = 0; x < NH; ++x) {
-    const int h = (int)blockIdx.x * NH + x;
     float sq = 0.f;
 #pragma unroll
     for (int j = 0; j < 4; ++j) sq += col + j < Dv ? o[x][j] * o[x][j] : 0.f;
 #pragma unroll
     for (int b = 1; b < LN; b <<= 1) sq += __shfl_xor(sq, b, 64);
     const float ms = sq / (float)Dv + a.eps, inv = sizeof(T) == 2 ? __builtin_amdgcn_rsqf(ms) : 1.0f / sqrtf(ms);
-    if (slot < 0 || t >= n || h >= a.H || col >= Dv) continue;
-    T* yp = static_cast<T*>(a.y) + r * a.ldy + (long)h * Dv + col;
-    T v[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const float z = gv[x][j], silu = sizeof(T) == 2 ? z * __builtin_amdgcn_rcpf(1.0f + __expf(-z)) : dl_silu(z);
-      st_f32<T>(v, j, o[x][j] * inv * nw[j] * silu);
+      const float z = (float)gv[x][j], silu = sizeof(T) == 2 ? z * __builtin_amdgcn_rcpf(1.0f + __expf(-z)) : dl_silu(z);
+      v[x][j] = (T)(o[x][j] * inv * ((float)nw[j] * a.out_scale) * silu);
     }
-    if (c.vec) {
-      typedef T T4 __attribute__((ext_vector_type(4)));
-      *reinterpret_cast<T4*>(yp) = T4{v[0], v[1], v[2], v[3]};
+    asm volatile("" : "+v"(v[x]));                     // (formed here: else the gates are asked for behind the branch)
+  }
+  if (slot < 0 || t >= n || col >= Dv) return;
+#pragma unroll
+  for (int x = 0; x < NH; ++x) {
+    const int h = (int)blockIdx.x * NH + x;
+    if (h >= a.H) break;
+    T* yp = static_cast<T*>(a.y) + r * a.ldy + (long)h * Dv + col;
+    if constexpr (VEC) {
+      *reinterpret_cast<T4*>(yp) = v[x];
     } else {
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        if (col + j < Dv) yp[j] = v[j];
+        if (col + j < Dv) yp[j] = v[x][j];
     }
   }
 }
@@ -1059,10 +1058,11 @@ EIA_API int eia_delta_scan_chunked(const float* q, const float* k, const float* 
   if (nseq == 0 || nchunk == 0) return EIA_OK;
   const int ndg = (DP + 63) / 64, ncu = (VP + 31) / 32, es = is_bf16 ? 2 : 4;
   const bool vec = Dv % 4 == 0 && ldy % 4 == 0 && ldg % 4 == 0 &&
-                   (reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(g)) % (4 * es) == 0;
+                   (reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(g) |
+                    reinterpret_cast<uintptr_t>(norm_w)) % (4 * es) == 0;
   const DeltaSolve solve = dn_solve(G, nchunk, H / G);
   DeltaChunkArgs c{chunks, seq_first, static_cast<bf16_t*>(Y), static_cast<bf16_t*>(Kt), static_cast<bf16_t*>(Qt),
-                   static_cast<bf16_t*>(P), X, O, cA, ncu, nseq, solve.whole, solve.parts, {}, vec};
+                   static_cast<bf16_t*>(P), X, O, cA, ncu, nseq, solve.whole, solve.parts, {}};
   const dim3 gc((unsigned)solve.blocks), b(256);
   const int nc = dn_columns(nseq * H * ncu);
   c.spread = dn_spread(G, 2 * ncu / nc * (H / G));
@@ -1074,12 +1074,14 @@ EIA_API int eia_delta_scan_chunked(const float* q, const float* k, const float* 
     hipLaunchKernelGGL(delta_chunk_solve_kernel<A>, gc, dim3(512), 0, st, a, c);                           \
     if (nc == 2) DO_SCAN(A, 2); else DO_SCAN(A, 1);                                                \
   } while (0)
-#define DO_NORM(TT, LN)                                                                            \
-  hipLaunchKernelGGL((delta_chunk_norm_kernel<TT, LN>), dim3((H + DN_HEADS - 1) / DN_HEADS, nchunk, DC * LN / 256), b, 0, st, a, c)
+#define DO_NORM_V(TT, LN, V)                                                                       \
+  hipLaunchKernelGGL((delta_chunk_norm_kernel<TT, LN, V>), dim3((H + DN_HEADS - 1) / DN_HEADS, nchunk, DC * LN / 256), b, 0, st, a, c)
+#define DO_NORM(TT, LN) do { if (vec) DO_NORM_V(TT, LN, true); else DO_NORM_V(TT, LN, false); } while (0)
   if (ndg == 2) DO_DIMS(2); else DO_DIMS(1);
   if (is_bf16) { if (VP > 64) DO_NORM(bf16_t, 32); else DO_NORM(bf16_t, 16); }
   else { if (VP > 64) DO_NORM(float, 32); else DO_NORM(float, 16); }
 #undef DO_NORM
+#undef DO_NORM_V
 #undef DO_DIMS
 #undef DO_SCAN
   EIA_LAUNCH_CHECK();

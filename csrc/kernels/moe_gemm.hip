@@ -229,47 +229,54 @@ __global__ void __launch_bounds__(256, OCC)
 moe_grouped_mfma_kernel(GroupedArgs a) {
   __shared__ __align__(16) bf16_t lds[(XS * MAXMU + WS * NU) * UNIT];
   const int lane = threadIdx.x & 63, E = a.E, NT = a.NT;
-  auto tiles = [&](int e) {                                // M tiles of expert e
-    return e < E ? moe_slice_tiles(a.offs[e + 1] - a.offs[e], MAXMU) : 0;
-  };
-  // blockIdx.x -> tile -> (expert, N tile, M tile); every wave for itself
-  int total = 0;
-  for (int e0 = 0; e0 < E; e0 += 64) {
-    int nt = tiles(e0 + lane);
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) nt += __shfl_xor(nt, o, 64);
-    total += nt;
-  }
-  total *= NT;
-  const int share = (total + 7) / 8, at = blockIdx.x >> 3;
-  const int tile = (blockIdx.x & 7) * share + at;
-  if (at >= share || tile >= total) return;                // surplus workgroup (uniform)
-  int ex = 0, n_tile = 0, m_tile = 0, m_tiles = 1;
-  for (int e0 = 0, base = 0; e0 < E; e0 += 64) {
-    const int nt = tiles(e0 + lane);
-    int incl = nt;
+  // blockIdx.x -> tile -> (expert, N tile, M tile); every wave for itself, a lane for each of 64 experts.  The first 64
+  // come last, so that their slices, read once, serve the search as well (read anew, and the tile's expert by itself
+  // once more, three trips to the L2 and twelve more shuffles stood before the first load)
+  int lo = 0, hi = 0, nt = 0, incl = 0;                    // the expert's rows, its M tiles, those up to and with it
+  auto slices = [&](int e0) {
+    const int e = e0 + lane;
+    lo = a.offs[min(e, E)];
+    hi = a.offs[min(e + 1, E)];
+    nt = e < E ? moe_slice_tiles(hi - lo, MAXMU) : 0;
+    incl = nt;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
       const int v = __shfl_up(incl, o, 64);
       if (lane >= o) incl += v;
     }
+  };
+  int total = 0;
+  for (int e0 = (E - 1) & ~63; e0 >= 0; e0 -= 64) {
+    slices(e0);
+    total += __builtin_amdgcn_readlane(incl, 63);
+  }
+  total *= NT;
+  const int share = (total + 7) / 8, at = blockIdx.x >> 3;
+  const int tile = (blockIdx.x & 7) * share + at;
+  if (at >= share || tile >= total) return;                // surplus workgroup (uniform)
+  int ex = 0, n_tile = 0, m_tile = 0, m_tiles = 1, rb = 0, rows = 0;
+  for (int e0 = 0, base = 0; e0 < E; e0 += 64) {
+    if (e0) slices(e0);
     const int q = tile - (base + incl - nt) * NT;
     const unsigned long long hit = __ballot(q >= 0 && q < nt * NT);
     if (hit) {
-      const int src = __ffsll(hit) - 1, qe = __shfl(q, src, 64);
-      m_tiles = __shfl(nt, src, 64);
+      const int src = __ffsll(hit) - 1, qe = __builtin_amdgcn_readlane(q, src);
+      m_tiles = __builtin_amdgcn_readlane(nt, src);
+      rb = __builtin_amdgcn_readlane(lo, src);
+      rows = __builtin_amdgcn_readlane(hi, src) - rb;
       ex = e0 + src;
       n_tile = qe / m_tiles;
       m_tile = qe - n_tile * m_tiles;
       break;
     }
-    base += __shfl(incl, 63, 64);
+    base += __builtin_amdgcn_readlane(incl, 63);
   }
   ex = __builtin_amdgcn_readfirstlane(ex);
   n_tile = __builtin_amdgcn_readfirstlane(n_tile);
   m_tile = __builtin_amdgcn_readfirstlane(m_tile);
   m_tiles = __builtin_amdgcn_readfirstlane(m_tiles);
-  const int rb = a.offs[ex], rows = a.offs[ex + 1] - rb;
+  rb = __builtin_amdgcn_readfirstlane(rb);
+  rows = __builtin_amdgcn_readfirstlane(rows);
   const bf16_t* We = a.W + (long)ex * a.w_estride;
   // Where weights come first (FRONT), tiles of 64 rows fall behind ones of 128 in long K loops: the op with 8 experts
   // of 4096 x 14336, 50 and 55 rows an expert: shares 578 and 573 us, whole tiles 555 and 557; not in short ones: 16

@@ -51,10 +51,9 @@ struct GroupedArgs {
 };
 
 // One tile: MU x 64 rows from row m0 of the slice [rb, rb + rows) of expert weights We, N tile n_tile.
-// TURN: tiles begin at different K steps.
-template <bool SWIGLU, int MU, int NU, int MAXMU, bool FRONT, bool TURN>
+template <bool SWIGLU, int MU, int NU, int MAXMU, bool FRONT>
 EIA_DEV void grouped_tile(const GroupedArgs& a, bf16_t* lds, const bf16_t* We, int rb, int rows, int m0,
-                          int n_tile, int ex) {
+                          int n_tile) {
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r32 = lane & 31, h = lane >> 5;
   // Access i of a step stands behind product i * RATE, with FRONT before all products.  Small tiles wait for memory rather than for the
@@ -83,23 +82,20 @@ EIA_DEV void grouped_tile(const GroupedArgs& a, bf16_t* lds, const bf16_t* We, i
     wsrc[i] = We + (long)wr * a.K + 8 * c;
   }
   const int nk = a.K / BK;
-  // where step kt of the tile begins in a row: at K step first + kt, from the last one on to the start
-  const int first = TURN ? (5 * n_tile + 3 * ex) % nk : 0;
-  auto from = [&](int kt) { return (!TURN || first + kt < nk ? first + kt : first + kt - nk) * BK; };
   auto put = [&](const bf16_t* src, bf16_t* dst) { glds16(src, lds_offset(dst)); };
-  auto fetch_x = [&](int i, int k, int slot) {
-    put(xsrc[i] + k, xlds + slot * MAXMU * UNIT + (32 * i + 8 * w) * BK);
+  auto fetch_x = [&](int i, int kt, int slot) {
+    put(xsrc[i] + kt * BK, xlds + slot * MAXMU * UNIT + (32 * i + 8 * w) * BK);
   };
-  auto fetch_w = [&](int i, int k, int slot) {
-    put(wsrc[i] + k, wlds + slot * NU * UNIT + (32 * i + 8 * w) * BK);
+  auto fetch_w = [&](int i, int kt, int slot) {
+    put(wsrc[i] + kt * BK, wlds + slot * NU * UNIT + (32 * i + 8 * w) * BK);
   };
-  auto all_x = [&](int k, int slot) {
+  auto all_x = [&](int kt, int slot) {
 #pragma unroll
-    for (int i = 0; i < 2 * MU; ++i) fetch_x(i, k, slot);
+    for (int i = 0; i < 2 * MU; ++i) fetch_x(i, kt, slot);
   };
-  auto all_w = [&](int k, int slot) {
+  auto all_w = [&](int kt, int slot) {
 #pragma unroll
-    for (int i = 0; i < 2 * NU; ++i) fetch_w(i, k, slot);
+    for (int i = 0; i < 2 * NU; ++i) fetch_w(i, kt, slot);
   };
 
   // wave (wm, wn): rows [32 MU wm, + 32 MU) of the X tile; W tile rows of N sub-tile nt: plain
@@ -141,18 +137,18 @@ EIA_DEV void grouped_tile(const GroupedArgs& a, bf16_t* lds, const bf16_t* We, i
     asm volatile("" ::: "memory");
   };
 
-  all_x(from(0), 0);
-  all_w(from(0), 0);
-  if (nk > 1) all_w(from(1), 1);
+  all_x(0, 0);
+  all_w(0, 0);
+  if (nk > 1) all_w(1, 1);
   arrive(nk > 1);
-  if (nk > 1) all_x(from(1), 1);
-  if (nk > 2) all_w(from(2), 2);
+  if (nk > 1) all_x(1, 1);
+  if (nk > 2) all_w(2, 2);
   // quarter kk of a step's products, its fragments in registers; between them accesses to
-  // X(xk) and then W(wk); done: products of the step before these
-  auto products = [&](int kk, int done, bool fx, int xk, int xslot, bool fw, int wk, int wslot) {
+  // X(xk) and then W(wk); `from`: products of the step before these
+  auto products = [&](int kk, int from, bool fx, int xk, int xslot, bool fw, int wk, int wslot) {
 #pragma unroll
     for (int j = 0; j < NU * MU; ++j) {
-      const int nt = j / MU, mt = j % MU, at = done + j, i = at / RATE;
+      const int nt = j / MU, mt = j % MU, at = from + j, i = at / RATE;
       acc[nt][mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[kk & 1][nt], xf[kk & 1][mt], acc[nt][mt], 0,
                                                             0, 0);
       if (at % RATE == 0) {
@@ -176,17 +172,17 @@ EIA_DEV void grouped_tile(const GroupedArgs& a, bf16_t* lds, const bf16_t* We, i
   // from step kt to kt + 1: X(kt + 2) goes where X(kt) was, W(kt + 3) where W(kt) was
   int ws = 0;
   auto advance = [&](int kt, auto fx, auto fw) {
-    const int xs = kt & 1, wn1 = ws + 1 < WS ? ws + 1 : 0, xk = from(kt + 2), wk = from(kt + 3);
+    const int xs = kt & 1, wn1 = ws + 1 < WS ? ws + 1 : 0;
     arrive(fx);
     if constexpr (FRONT) {
-      if (fx) all_x(xk, xs);
-      if (fw) all_w(wk, ws);
+      if (fx) all_x(kt + 2, xs);
+      if (fw) all_w(kt + 3, ws);
     }
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       frags(q, xs ^ 1, wn1);
       __builtin_amdgcn_sched_barrier(0);                   // the next fragments before these products
-      products((q + 3) & 3, q * NU * MU, fx && !FRONT, xk, xs, fw && !FRONT, wk, ws);
+      products((q + 3) & 3, q * NU * MU, fx && !FRONT, kt + 2, xs, fw && !FRONT, kt + 3, ws);
     }
     ws = wn1;
   };
@@ -224,7 +220,7 @@ EIA_DEV void grouped_tile(const GroupedArgs& a, bf16_t* lds, const bf16_t* We, i
   }
 }
 
-template <bool SWIGLU, int NU, int MAXMU, int OCC, bool FRONT, bool TURN>
+template <bool SWIGLU, int NU, int MAXMU, int OCC, bool FRONT>
 __global__ void __launch_bounds__(256, OCC)
 moe_grouped_mfma_kernel(GroupedArgs a) {
   __shared__ __align__(16) bf16_t lds[(XS * MAXMU + WS * NU) * UNIT];
@@ -284,7 +280,7 @@ moe_grouped_mfma_kernel(GroupedArgs a) {
   const MoeTile m = moe_slice_tile(rows, m_tiles, m_tile, FRONT && a.K > 2048, MAXMU);
 #define GG_TILE(M)                                                                            \
   case M:                                                                                     \
-    if constexpr (M <= MAXMU) grouped_tile<SWIGLU, M, NU, MAXMU, FRONT, TURN>(a, lds, We, rb, rows, 64 * m.lo, n_tile, ex); \
+    if constexpr (M <= MAXMU) grouped_tile<SWIGLU, M, NU, MAXMU, FRONT>(a, lds, We, rb, rows, 64 * m.lo, n_tile); \
     break
   switch (m.mu) { GG_TILE(1); GG_TILE(2); GG_TILE(3); GG_TILE(4); GG_TILE(5); }
 #undef GG_TILE
@@ -349,34 +345,20 @@ EIA_API int eia_moe_grouped_gemm(const void* X, long ldx, const int* row_idx, co
   // better, while beyond it holds the products up.  The op, spread / in front, us, cold weights: 8 experts of 4096 x
   // 14336, 64 rows 558 / 545; 16 of 2048 x 1024, 112 rows 70.6 / 69.8; 8 of 1024 x 512, 512 rows (form 0) 44.5 / 47.7.
   const bool front = max_rows <= 128L * E;
-  // Tiles that all run at once ask for the same place of their rows at the same time, whose lines lie on few of the
-  // memory's channels where rows are a power of two long; beginning at different K steps they do not, but read the
-  // rows of X again from farther off where an expert's do not stay in the L2.  So in one round of tiles (two
-  // workgroups a CU) and up to 7/8 MB of X an expert.  The op, together / apart, us: 16 experts of 2048 x 1024, 31 rows
-  // 57.8 / 49.6, 50 60.3 / 51.4, 75 65.0 / 55.0, 125 70.0 / 65.2, 187 83.3 / 78.7; beyond the line (1 MB) the down GEMM with 500
-  // rows 50.3 / 52.2, of 8 of 1024 x 512 with 1000 rows 18.6 / 19.8; 8 of 4096 x 14336, 125 rows 630 / 645.
-  // (A form of the kernel: the steps' places cost large tiles 1 %.)
-  auto turn = [&](int nt, int mm) {
-    const long tiles = (long)E * nt * ((max_rows + 64L * mm * E - 1) / (64L * mm * E));
-    return tiles <= 512 && (long)max_rows * K <= 448L * 1024 * E;
-  };
-#define GG_GO(SW, NU, MM, OCC, FRONT, TURN)                                                               \
+#define GG_GO(SW, NU, MM, OCC, FRONT)                                                               \
   do {                                                                                              \
     const int nt = N / (64 * NU);                                                                   \
     GroupedArgs a{(const bf16_t*)X, ldx, row_idx, (const bf16_t*)W, (long)N * K, offs, E, N / 2, K, \
                   nt, (bf16_t*)out, ldo, relu2};                                                    \
     const dim3 grid((unsigned)((((max_rows + 64 * MM - 1) / (64 * MM) + E) * (long)nt + 7) / 8 * 8)); \
-    if (TURN && turn(nt, MM))                                                                       \
-      hipLaunchKernelGGL((moe_grouped_mfma_kernel<SW, NU, MM, OCC, FRONT, TURN>), grid, dim3(256), 0, st, a);  \
-    else                                                                                            \
-      hipLaunchKernelGGL((moe_grouped_mfma_kernel<SW, NU, MM, OCC, FRONT, false>), grid, dim3(256), 0, st, a); \
+    hipLaunchKernelGGL((moe_grouped_mfma_kernel<SW, NU, MM, OCC, FRONT>), grid, dim3(256), 0, st, a);      \
   } while (0)
 #define GG_FORM(SW) \
   do {                                                                                              \
-    if (form == 0 && front) GG_GO(SW, 2, 2, 2, true, true);                                             \
-    else if (form == 0) GG_GO(SW, 2, 2, 2, false, true);                                                \
-    else if (form == 1) GG_GO(SW, 2, 5, 1, false, true);                                                \
-    else GG_GO(SW, 4, 4, 1, false, false);                                                               \
+    if (form == 0 && front) GG_GO(SW, 2, 2, 2, true);                                               \
+    else if (form == 0) GG_GO(SW, 2, 2, 2, false);                                                  \
+    else if (form == 1) GG_GO(SW, 2, 5, 1, false);                                                  \
+    else GG_GO(SW, 4, 4, 1, false);                                                                 \
   } while (0)
   if (swiglu) GG_FORM(true); else GG_FORM(false);
 #undef GG_FORM

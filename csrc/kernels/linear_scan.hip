@@ -629,21 +629,24 @@ EIA_DEV float2 ls_log_gates(const ScanArgs& a, int n, LsGates g, float m0, float
     }
     return q;
   };
+  // a token that forgets everything and adds nothing (f = i = -inf) leaves no number, in the state as in its outputs
+  auto shut = [](float f, float i) { return !(f > -INFINITY) && !(i > -INFINITY); };
+  auto pair = [&](float f, float i) { return make_float2(shut(f, i) ? __builtin_nanf("") : f, i); };
   const float2 none = make_float2(0.f, -INFINITY);
   const float gi = soft(value(g.xi[0])), gf = ls_logsigmoid(soft(value(g.xf[0])));
   float2 first = none;                      // of the 64 tokens before the second wave's
   if (t >= 64) {
-    first = scan(lane < n ? make_float2(ls_logsigmoid(soft(value(g.xf[1]))), soft(value(g.xi[1]))) : none);
+    first = scan(lane < n ? pair(ls_logsigmoid(soft(value(g.xf[1]))), soft(value(g.xi[1]))) : none);
     first = make_float2(__shfl(first.x, 63, 64), __shfl(first.y, 63, 64));
   }
-  const float2 p = join(first, scan(t < n ? make_float2(gf, gi) : none));
+  const float2 p = join(first, scan(t < n ? pair(gf, gi) : none));
   m = fmaxf(m0 + p.x, p.y);
   const float up = __shfl_up(m, 1, 64), before = lane ? up : fmaxf(m0 + first.x, first.y);
   // (not gf + before - m: where nothing new is met the maximum moves with the decays, and the roundings of its
   // steps would add up.  S against 64 bits 2.5e-7 instead of 1.6e-7)
-  const float fm = gf + before;
+  const float fm = pair(gf, gi).x + before;
   l = t >= n || before == -INFINITY || fm >= gi ? 0.f : fm - gi;
-  b = t >= n ? 0.f : m > -INFINITY ? gi - m : -INFINITY;
+  b = t >= n ? 0.f : shut(gf, gi) ? __builtin_nanf("") : m > -INFINITY ? gi - m : -INFINITY;
   return p;
 }
 // Sums of l over 16-token blocks: pre up to and with a token, suf behind it, tot of whole blocks;

@@ -155,23 +155,59 @@ def test_gates_that_shut(lens, dtype, monkeypatch):
         x[lo:lo + 2, at[4]:at[5]] = float("-inf")          # nor do the first two
     x[cu[0] + 128:cu[0] + 256, at[4] + 2] = float("-inf")  # nor does a chunk of the first sequence, head 2
     x = x.to(dtype)
-
-    def run(dev):
-        spec = ls.ScanSpec(H, D, Dv, "exp_gates", kscale=D ** -0.5, eps=1e-5)
-        st = ls.ScanState.allocate(n, spec, "cpu")
-        gs = torch.Generator().manual_seed(1)
-        for t in (st.S, st.n, st.m):
-            t.copy_(torch.randn(t.shape, generator=gs))
-        st = ls.ScanState(*(t.to(dev) for t in (st.S, st.n, st.m)))
-        plan = ls.chunk_plan(lens, dev) if dev == "cuda" else None
-        y = ls.linear_scan(x.to(dev), at[0], at[1], at[2], at[3], spec, st, slots.to(dev), cu.to(dev), n, pos.to(dev),
-                           None, None, at[4], at[5], plan=plan)
-        return y.cpu(), st
-
-    (y, a), (z, b) = run("cpu"), run("cuda")
+    (y, a), (z, b) = (_gated(dev, x, lens, cu, pos, slots, H, D, Dv) for dev in ("cpu", "cuda"))
     assert torch.isfinite(y).all() and _rel(z, y) < (1e-5 if dtype == torch.float32 else 4e-3)      # as above
     for u, v in ((a.S, b.S), (a.n, b.n), (a.m, b.m)):
         assert _rel(v, u) < 2e-6
+
+
+def _gated(dev, x, lens, cu, pos, slots, H, D, Dv):
+    """Matrix memory without a cap over rows of queries, keys, values, output gates and the two gates of each head."""
+    from enterprise_inference_amd.ops import linear_scan as ls
+    spec = ls.ScanSpec(H, D, Dv, "exp_gates", kscale=D ** -0.5, eps=1e-5)
+    st = ls.ScanState.allocate(len(lens), spec, "cpu")
+    gs = torch.Generator().manual_seed(1)
+    for t in (st.S, st.n, st.m):
+        t.copy_(torch.randn(t.shape, generator=gs))
+    st = ls.ScanState(*(t.to(dev) for t in (st.S, st.n, st.m)))
+    plan = ls.chunk_plan(lens, dev) if dev == "cuda" else None
+    HD = H * D
+    y = ls.linear_scan(x.to(dev), 0, HD, 2 * HD, 2 * HD + H * Dv, spec, st, slots.to(dev), cu.to(dev), len(lens),
+                       pos.to(dev), None, None, 2 * H * (D + Dv), 2 * H * (D + Dv) + H, plan=plan)
+    return y.cpu(), st
+
+
+# first and last rows of a chunk, of the half that a wave takes, of a block of sixteen, of the sequence
+@pytest.mark.parametrize("row", [0, 1, 63, 64, 127, 128, 130, 299])
+@pytest.mark.parametrize("past", [0, 5])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("i,f,lead", [(float("-inf"), float("-inf"), 0), (float("-inf"), float("-inf"), 2),
+                                      (0.5, float("-inf"), 0)])
+def test_gates_that_are_not_finite(i, f, lead, dtype, past, row, monkeypatch):
+    """One token's gates of head 1, behind ``lead`` tokens that add nothing.  A token that forgets everything and adds
+    nothing leaves no number, as in the recurrence, in its own and all later outputs and in the state."""
+    from enterprise_inference_amd.ops import linear_scan as ls
+    monkeypatch.setattr(ls, "FORCE_CHUNKED", True)
+    H, D, Dv, lens = 3, 32, 64, [300, 150]
+    cu, pos, slots = _step(lens, [past, 5], False)
+    at = 2 * H * (D + Dv)
+    x = torch.randn(sum(lens), at + 2 * H, generator=torch.Generator().manual_seed(row))
+    x[:, at + H:] += 3.0
+    x[max(0, row - lead):row, at + 1] = float("-inf")
+    x[row, at + 1], x[row, at + H + 1] = i, f
+    x = x.to(dtype)
+    (y, a), (z, b) = (_gated(dev, x, lens, cu, pos, slots, H, D, Dv) for dev in ("cpu", "cuda"))
+    bad = torch.zeros(sum(lens), H, Dv, dtype=torch.bool)
+    same = ~bad
+    if i != 0.5:
+        bad[row:lens[0], 1] = True
+        same[row // 16 * 16:lens[0], 1] = False            # (a block of sixteen is one product)
+    bad, same = bad.view(y.shape), same.view(y.shape)
+    assert torch.equal(torch.isfinite(y), ~bad) and not torch.isfinite(z[bad]).any()
+    assert torch.isfinite(z[same]).all() and _rel(z[same], y[same]) < (1e-5 if dtype == torch.float32 else 4e-3)  # as above
+    for u, v in ((a.S, b.S), (a.n, b.n), (a.m, b.m)):
+        v, ok = v.cpu(), torch.isfinite(u)
+        assert torch.equal(torch.isfinite(v), ok) and _rel(v[ok], u[ok]) < 2e-6
 
 
 def _stays_not_finite(y, z, H, col, hit):

@@ -629,8 +629,9 @@ EIA_DEV float2 ls_log_gates(const ScanArgs& a, int n, LsGates g, float m0, float
     }
     return q;
   };
-  // a token that forgets everything and adds nothing (f = i = -inf) leaves no number, in the state as in its outputs
-  auto shut = [](float f, float i) { return !(f > -INFINITY) && !(i > -INFINITY); };
+  // a token that forgets everything and adds nothing (f = i = -inf), or whose f is no number, leaves none, in the state
+  // as in its outputs
+  auto shut = [](float f, float i) { return !(f > -INFINITY) && !(f == -INFINITY && i > -INFINITY); };
   auto pair = [&](float f, float i) { return make_float2(shut(f, i) ? __builtin_nanf("") : f, i); };
   const float2 none = make_float2(0.f, -INFINITY);
   const float gi = soft(value(g.xi[0])), gf = ls_logsigmoid(soft(value(g.xf[0])));
@@ -646,7 +647,7 @@ EIA_DEV float2 ls_log_gates(const ScanArgs& a, int n, LsGates g, float m0, float
   // steps would add up.  S against 64 bits 2.5e-7 instead of 1.6e-7)
   const float fm = pair(gf, gi).x + before;
   l = t >= n || before == -INFINITY || fm >= gi ? 0.f : fm - gi;
-  b = t >= n ? 0.f : shut(gf, gi) ? __builtin_nanf("") : m > -INFINITY ? gi - m : -INFINITY;
+  b = t >= n ? 0.f : shut(gf, gi) ? __builtin_nanf("") : m > -INFINITY ? gi - m : gi;      // (gi: -inf or no number)
   return p;
 }
 // Sums of l over 16-token blocks: pre up to and with a token, suf behind it, tot of whole blocks;

@@ -161,7 +161,7 @@ def fa_parts(wgs: int, tiles: int, mean: float, tile_us: float = 1.65, merge_us:
     16 on 4: 32 of 24, 20: 45.2, 5: 23.2, 2: 31.1; 52 of 26, 25: 48.1, 7: 27.8, 6: 34; 128 of 32, 16: 58.2, 13: 38.6, 8: 47.7;
     236 of 24, 14: 47, 16: 50; 252 of 64, 33: 116, 34: 108, 22: 97, 16: 124.  28 on 4: 112 of 22, 16: 46.2, 11: 36.3, 8: 41;
     168 of 48, 36: 98, 24: 90, 16: 92, 15: 107; 224 of 30, 27: 66.2, 15: 81.7."""
-    if wgs > FA_SLOTS or tile_us * tiles < 9:
+    if wgs < 1 or wgs > FA_SLOTS or tile_us * tiles < 9:
         return 1, tiles
     work = wgs * max(1.0, mean)
     least = max(1, math.ceil(tiles * wgs / 1024))
@@ -354,7 +354,7 @@ def paged_prefill(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
     if code & PREFILL_FA:
         wgs, ws = n_work * (Hq // hpw), None
         parts = per = 1
-        if wgs <= FA_SLOTS and block_tables.shape[1] * bs >= 6 * 64:
+        if 0 < wgs <= FA_SLOTS and block_tables.shape[1] * bs >= 6 * 64:
             rows = PREFILL_FA_QB * (4 // hpw)
             tiles = block_tables.shape[1] * bs / 64          # (of the longest sequence)
             mean = tiles - T / (128 * (cu_q.numel() - 1)) if causal else tiles

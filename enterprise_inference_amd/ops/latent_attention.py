@@ -190,7 +190,7 @@ def flash_parts(wgs: int, lens, context: int, tiles: int, KT: int, window: int, 
     P, per = split_keys(wgs, tiles, tiles if window > 0 else tiles - max(lens) // (2 * KT),
                         512 if two else 256, 12 * 64 // KT, 11 if two else 3 * 64 // KT)
     if wgs <= 64 or (P == 1 and not two):
-        mean = (context - max(lens) + sum(n * n for n in lens) / (2 * sum(lens))) / KT
+        mean = (context - max(lens) + sum(n * n for n in lens) / (2 * max(1, sum(lens)))) / KT
         P, per = fa_parts(wgs, tiles, min(mean, tiles), 1.85 if two else 3.6, 6.5, 0.02, 1)
     return P, per
 

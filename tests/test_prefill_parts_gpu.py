@@ -30,6 +30,28 @@ def test_latent_parts_cover(lens, past, window, KT, two):
         assert parts == 1 or wgs * parts <= max(1024, 3 * 512)
 
 
+def test_launches_without_work_are_not_cut():
+    from enterprise_inference_amd.ops import latent_attention as la
+    from enterprise_inference_amd.ops import window_attention as wa
+    from enterprise_inference_amd.ops.attention import fa_parts
+    spec = wa.WindowSpec(8, 2, 1, 128, 128, 0, 0, mult=None)
+    assert fa_parts(0, 32, 32.0) == wa.pair_parts(0, spec, 64, 2048) == wa.flash_parts(0, spec, 64, 1, 2048) == (1, 32)
+    for lens in ([1], [0], [0, 0]):
+        assert la.flash_parts(0, lens, 2048, 32, 64, 0, True) == (1, 32)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cu", [[0], [0, 0]])
+def test_flash_prefill_without_work(cu):
+    """No sequences, and one without tokens, beside a block table of many pages."""
+    from enterprise_inference_amd.ops import attention
+    i32 = lambda *v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    q = torch.empty(0, 8, 128, dtype=BF, device="cuda")
+    k, v = torch.zeros(1, 2, 128, 128, dtype=BF, device="cuda"), torch.zeros(1, 2, 128, 128, dtype=BF, device="cuda")
+    bt, sl = torch.zeros(len(cu) - 1, 16, dtype=torch.int32, device="cuda"), i32(*[0] * (len(cu) - 1))
+    assert attention.paged_prefill(q, k, v, bt, sl, i32(*cu), i32(), 0, 0.1).shape == q.shape
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("Hq,Hkv", [(8, 2), (6, 3), (3, 1)])
 @pytest.mark.parametrize("qlens,ctxs", [([1, 33, 64, 127], [700, 5, 70, 0]), ([255, 40], [63, 600]), ([300], [0])])

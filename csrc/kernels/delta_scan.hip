@@ -966,11 +966,10 @@ delta_chunk_scan_kernel(DeltaArgs a, DeltaChunkArgs c) {
 
 // (3) Norm, weight and gate of the outputs: LN lanes per token and head, two heads each; the heads come first in the
 // grid, so that those of a key head run on the XCD that formed them where G is eight.  Bound by memory.  (Four heads, chunks
-// first: three prompts of 155 tokens, 8 heads 32.9 -> 30.8 us, three of up to 1500, 16 heads 146.0 -> 145.2.)  Of bf16
-// outputs, whose rounding is 2^-9, the root and silu take the instructions' own reciprocal and exponential (1 ulp, some
-// 2^-21): with divisions and expf vector instructions filled 13 of 19.2 us, without the kernel takes 16.6; error of the
-// outputs against 64 bits 1.7e-3 as before.  All five reads of a thread are in flight together (the second head's behind
-// the first one's gate: the op 128.6 us instead of 125).
+// first: three prompts of 155 tokens, 8 heads 32.9 -> 30.8 us, three of up to 1500, 16 heads 146.0 -> 145.2.)  All five
+// reads of a thread are in flight together (the second head's behind the first one's gate: the op 128.6 us instead of 125,
+// both with the instructions' own reciprocals).  Root and silu are formed with divisions and expf also of bf16 outputs:
+// with v_rsq, v_rcp and __expf the op takes 128.0 instead of 130.6 us, but of gates below -87.3 v_rcp leaves zero.
 constexpr int DN_HEADS = 2;
 template <typename T, int LN, bool VEC>
 __global__ void __launch_bounds__(256)
@@ -1007,12 +1006,10 @@ delta_chunk_norm_kernel(DeltaArgs a, DeltaChunkArgs c) {
     for (int j = 0; j < 4; ++j) sq += col + j < Dv ? o[x][j] * o[x][j] : 0.f;
 #pragma unroll
     for (int b = 1; b < LN; b <<= 1) sq += __shfl_xor(sq, b, 64);
-    const float ms = sq / (float)Dv + a.eps, inv = sizeof(T) == 2 ? __builtin_amdgcn_rsqf(ms) : 1.0f / sqrtf(ms);
+    const float inv = 1.0f / sqrtf(sq / (float)Dv + a.eps);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float z = (float)gv[x][j], silu = sizeof(T) == 2 ? z * __builtin_amdgcn_rcpf(1.0f + __expf(-z)) : dl_silu(z);
-      v[x][j] = (T)(o[x][j] * inv * ((float)nw[j] * a.out_scale) * silu);
-    }
+    for (int j = 0; j < 4; ++j)
+      v[x][j] = (T)(o[x][j] * inv * ((float)nw[j] * a.out_scale) * dl_silu((float)gv[x][j]));
     asm volatile("" : "+v"(v[x]));                     // (formed here: else the gates are asked for behind the branch)
   }
   if (slot < 0 || t >= n || col >= Dv) return;

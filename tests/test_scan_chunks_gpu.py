@@ -372,6 +372,21 @@ def _delta_chunks(lens, H, G, D, Dv, dtype, monkeypatch, plant=lambda rows, S: N
     return y, S, z, Z, live
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_delta_gates_that_are_nearly_shut(dtype, monkeypatch):
+    """silu(-88) is -5e-37: the output is small, and not zero, though 1 / (1 + exp(88)) is below the smallest normal number."""
+    cols = [0, 1, 70, 200]
+
+    def plant(rows, S):
+        rows[5][:, cols] = torch.tensor([-88.5, -88.0, -87.5, -60.0]).to(dtype)
+
+    y, _, z, _, live = _delta_chunks([100, 64, 3], 2, 1, 128, 128, dtype, monkeypatch, plant)
+    for c in cols:                                         # the bounds of test_delta_chunks
+        u, v = y[live][:, c], z[live][:, c]
+        ok = u.abs() > 2.0 ** -125                         # (the kernels flush numbers below 2^-126 to zero)
+        assert ok.sum() > 100 and _rel(v[ok], u[ok]) < (1e-5 if dtype == torch.float32 else 4e-3)
+
+
 @pytest.mark.parametrize("H,G,D,Dv", [(4, 2, 128, 128), (3, 3, 64, 72), (32, 8, 128, 128)])
 @pytest.mark.parametrize("where,value", [("v", float("inf")), ("v", float("nan")), ("k", float("nan")),
                                          ("q", float("inf")), ("q", float("nan")), ("S", float("-inf")),

@@ -583,8 +583,7 @@ wkv_chunk_out_kernel(WkvArgs a, WkvChunkArgs c) {
     float ss = 0.f;
 #pragma unroll
     for (int j = 0; j < 4; ++j) ss += o[j][i] * o[j][i];
-    const float ms = row16_sum(ss) / (float)D + a.eps;
-    const float inv = sizeof(T) == 2 ? __builtin_amdgcn_rsqf(ms) : 1.0f / sqrtf(ms);
+    const float inv = 1.0f / sqrtf(row16_sum(ss) / (float)D + a.eps);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const float g = (float)gv[i][j];

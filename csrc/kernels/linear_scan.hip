@@ -2280,8 +2280,7 @@ gl_out_kernel(ScanArgs a, KChunkArgs c) {
     float ss = 0.f;
 #pragma unroll
     for (int j = 0; j < 4 * NV; ++j) ss += o[j][i] * o[j][i];
-    const float ms = row16_sum(ss) / (float)Dv + a.eps;
-    const float inv = a.out_scale * (sizeof(T) == 2 ? __builtin_amdgcn_rsqf(ms) : 1.0f / sqrtf(ms));
+    const float inv = a.out_scale / sqrtf(row16_sum(ss) / (float)Dv + a.eps);
 #pragma unroll
     for (int z = 0; z < NV; ++z) {
 #pragma unroll

@@ -261,7 +261,7 @@ EIA_DEV bool wkv_chunk(const WkvArgs& a, int nseq, int x, int& s, int& row0, int
 }
 
 // A chunk's [WC][WD] tile of r, k or v on its way to LDS, zero past the chunk and past D: requested
-// by load, stored as fp32 by store.  VEC: 16-byte loads (D == WD, rows on 16-byte addresses; then the others' rows too).
+// by load, stored as fp32 by store.  VEC: 16-byte loads (D == WD, rows on 16-byte addresses).
 template <typename T, bool VEC>
 struct WkvTile {
   typedef __attribute__((ext_vector_type(4))) int i32x4;
@@ -415,7 +415,8 @@ wkv_chunk_scan_kernel(WkvArgs a, WkvChunkArgs c) {
 
 // (3) Wave w forms the outputs of tokens 16 w .. (later tokens meet more keys: which wave takes them
 // rotates with the chunk, so that no SIMD gets all of them).  50 KiB of LDS: three workgroups per CU.
-template <typename T, bool VEC>
+// WIDE: gate, weight and output rows can be taken four at a time.
+template <typename T, bool VEC, bool WIDE>
 __global__ void __launch_bounds__(256, 3)
 wkv_chunk_out_kernel(WkvArgs a, WkvChunkArgs c) {
   __shared__ __align__(16) float sr[WC * WD], sk[WC * WD], sAv[WC * WD];
@@ -550,14 +551,14 @@ wkv_chunk_out_kernel(WkvArgs a, WkvChunkArgs c) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const T* q = G + (long)(row0 + min(t0 + 4 * g4 + i, n - 1)) * a.ld;
-      if constexpr (VEC) {
+      if constexpr (WIDE) {
         gv[i] = *reinterpret_cast<const T4*>(q + 4 * l16);
       } else {
 #pragma unroll
         for (int j = 0; j < 4; ++j) gv[i][j] = q[min(4 * l16 + j, D - 1)];
       }
     }
-    if constexpr (VEC) {
+    if constexpr (WIDE) {
       nw = *reinterpret_cast<const T4*>(NW + 4 * l16);
     } else {
 #pragma unroll
@@ -597,7 +598,7 @@ wkv_chunk_out_kernel(WkvArgs a, WkvChunkArgs c) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     if (t0 + 4 * g4 + i >= n) break;
-    if constexpr (VEC) {
+    if constexpr (WIDE) {
       *reinterpret_cast<T4*>(Y + i * a.ldy) = yv[i];
     } else {
 #pragma unroll
@@ -607,12 +608,12 @@ wkv_chunk_out_kernel(WkvArgs a, WkvChunkArgs c) {
   }
 }
 
-template <typename T, bool VEC>
+template <typename T, bool VEC, bool WIDE>
 static void wkv_chunked(const WkvArgs& a, const WkvChunkArgs& c, int rows, hipStream_t st) {
   const dim3 gc = chunk_grid(rows / WC + c.nseq, a.H), gs = chunk_grid(c.nseq, a.H * (WD * WD / 1024));
   hipLaunchKernelGGL((wkv_chunk_state_kernel<T, VEC>), gc, dim3(256), 0, st, a, c);
   hipLaunchKernelGGL(wkv_chunk_scan_kernel, gs, dim3(256), 0, st, a, c);
-  hipLaunchKernelGGL((wkv_chunk_out_kernel<T, VEC>), gc, dim3(256), 0, st, a, c);
+  hipLaunchKernelGGL((wkv_chunk_out_kernel<T, VEC, WIDE>), gc, dim3(256), 0, st, a, c);
 }
 
 // As eia_wkv_scan for D <= 64 with cu given, for the sequences of split rows or more; rows: cu[nseq] at most; workspaces U
@@ -631,14 +632,20 @@ EIA_API int eia_wkv_scan_chunked(const void* r, const void* k, const void* v, co
   WkvArgs a{r, k, v, g, ld, dec, ld_dec, w0, u, norm_w, S, prev, x, W, slots, cu, positions,
             seq_lens, y, ldy, eps, H, D, split};
   const WkvChunkArgs c{U, L, nseq};
-  // 16-byte rows of r, k and v, gates, weights and outputs four at a time
+  // rows of r, k and v by 16 bytes, gates, weights and outputs four at a time, each where they lie so: one flag for both
+  // took a prompt of 4096 tokens, 32 heads of 64, with weights off 8 bytes from 101 to 108 us
   const int es = is_bf16 ? 2 : 4;
   const uintptr_t any = (uintptr_t)r | (uintptr_t)k | (uintptr_t)v | (uintptr_t)(ld * es);
-  const uintptr_t io = (uintptr_t)g | (uintptr_t)y | (uintptr_t)norm_w | (uintptr_t)(ldy * es);
-  const bool vec = D == WD && any % 16 == 0 && io % (4 * es) == 0;
-  if (is_bf16 && vec) wkv_chunked<bf16_t, true>(a, c, rows, st);
-  else if (is_bf16) wkv_chunked<bf16_t, false>(a, c, rows, st);
-  else if (vec) wkv_chunked<float, true>(a, c, rows, st);
-  else wkv_chunked<float, false>(a, c, rows, st);
+  const uintptr_t io = (uintptr_t)g | (uintptr_t)y | (uintptr_t)norm_w | (uintptr_t)(ld * es) | (uintptr_t)(ldy * es);
+  const bool vec = D == WD && any % 16 == 0, wide = D == WD && io % (4 * es) == 0;
+#define WKV_GO(T)                                                                                   \
+  do {                                                                                              \
+    if (vec && wide) wkv_chunked<T, true, true>(a, c, rows, st);                                    \
+    else if (vec) wkv_chunked<T, true, false>(a, c, rows, st);                                      \
+    else if (wide) wkv_chunked<T, false, true>(a, c, rows, st);                                     \
+    else wkv_chunked<T, false, false>(a, c, rows, st);                                              \
+  } while (0)
+  if (is_bf16) WKV_GO(bf16_t); else WKV_GO(float);
+#undef WKV_GO
   EIA_LAUNCH_CHECK();
 }

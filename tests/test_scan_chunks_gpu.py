@@ -741,3 +741,23 @@ def test_wkv_rows_of_any_alignment(dtype):
         out.append((y, S))
     # the same fp32 sums, whichever way their factors came
     assert _rel(out[1][0], out[0][0]) < (1e-6 if dtype == torch.float32 else 1e-3) and _rel(out[1][1], out[0][1]) < 1e-6
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("off,weight_off", [(0, 1), (4, 0), (4, 1), (2, 0)])
+def test_wkv_rows_and_weights_aligned_apart(off, weight_off, dtype):
+    """Rows that lie on 16 bytes beside weights that do not lie on four elements, and rows that do so the other way."""
+    from enterprise_inference_amd.ops import wkv
+    lens, H, D = [130, 64, 300], 2, 64
+    T, HD = sum(lens), H * D
+    cu, pos, slots = (t.cuda() for t in _step(lens, [0, 5, 0], False))
+    args = [t.cuda() for t in _wkv_args(torch.Generator().manual_seed(off), T, 3, H, D, dtype)]
+    S0, out = args[8].clone(), []
+    for o, w in ((0, 0), (off, weight_off)):
+        a = list(args)
+        a[8] = S0.clone()
+        a[:4] = (torch.empty(T, HD + 2 * o, device="cuda", dtype=dtype)[:, o:o + HD].copy_(t) for t in args[:4])
+        a[7] = torch.empty(HD + w, device="cuda", dtype=dtype)[w:].copy_(args[7])
+        out.append((wkv.wkv_scan(*a, slots, cu, 3, pos, None, 1e-5, H), a[8]))
+    # the same fp32 sums, whichever way their factors came
+    assert _rel(out[1][0], out[0][0]) < (1e-6 if dtype == torch.float32 else 1e-3) and _rel(out[1][1], out[0][1]) < 1e-6

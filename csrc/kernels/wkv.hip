@@ -308,15 +308,16 @@ struct WkvTile {
 
 // Base-2 log decays of channel i, tokens t0 .. t0 + 15 (0 past the chunk and past D): a weight then
 // costs one v_exp_f32.
-// ask: requests of the caller that go out behind the decays' own.
-template <typename T, typename Ask>
+// ask: requests of the caller that go out behind the decays' own.  HOLD: nothing is waited for before all of them are out;
+// else the compiler chooses.
+template <typename T, bool HOLD, typename Ask>
 EIA_DEV void wkv_decays(const WkvArgs& a, long hc, int row0, int n, int t0, int i, float (&l)[16], Ask&& ask) {
   const int ic = min(i, a.D - 1);
   const float w0 = ld_f32<T>(static_cast<const T*>(a.w0), hc + ic);
 #pragma unroll
   for (int t = 0; t < 16; ++t) l[t] = a.dec[(long)(row0 + min(t0 + t, n - 1)) * a.ld_dec + hc + ic];
   ask();
-  __builtin_amdgcn_sched_barrier(0);                   // (else the second half of them behind the first's exponentials)
+  if constexpr (HOLD) __builtin_amdgcn_sched_barrier(0);                   // (else the second half of them behind the first's exponentials)
 #pragma unroll
   for (int t = 0; t < 16; ++t)
     l[t] = (i < a.D && t0 + t < n) ? -1.4426950408889634f * expf(l[t] + w0) : 0.f;
@@ -336,10 +337,13 @@ wkv_chunk_state_kernel(WkvArgs a, WkvChunkArgs c) {
   const long hc = (long)h * a.D;
   WkvTile<T, VEC> tk, tv;
   float l[16];
-  wkv_decays<T>(a, hc, row0, n, 16 * w, lane, l, [&] {
+  auto rows = [&] {
     tk.load(a.k, a.ld, hc, row0, n, a.D);
     tv.load(a.v, a.ld, hc, row0, n, a.D);
-  });
+  };
+  // (rows by elements: 32 registers more, and two workgroups a CU, where they come behind the decays)
+  if constexpr (!VEC) rows();
+  wkv_decays<T, VEC>(a, hc, row0, n, 16 * w, lane, l, [&] { if constexpr (VEC) rows(); });
   float tot = 0.f;
 #pragma unroll
   for (int t = 0; t < 16; ++t) tot += l[t];
@@ -429,9 +433,9 @@ wkv_chunk_out_kernel(WkvArgs a, WkvChunkArgs c) {
   const long hc = (long)h * D;
   WkvTile<T, VEC> tr, tk, tv;
   const T u = static_cast<const T*>(a.u)[hc + min(lane, D - 1)];
-  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (VEC) __builtin_amdgcn_sched_barrier(0);
   float l[16];
-  wkv_decays<T>(a, hc, row0, n, t0, lane, l, [&] {
+  wkv_decays<T, VEC>(a, hc, row0, n, t0, lane, l, [&] {
     tr.load(a.r, a.ld, hc, row0, n, D);
     tk.load(a.k, a.ld, hc, row0, n, D);
     tv.load(a.v, a.ld, hc, row0, n, D);

@@ -761,3 +761,33 @@ def test_wkv_rows_and_weights_aligned_apart(off, weight_off, dtype):
         out.append((wkv.wkv_scan(*a, slots, cu, 3, pos, None, 1e-5, H), a[8]))
     # the same fp32 sums, whichever way their factors came
     assert _rel(out[1][0], out[0][0]) < (1e-6 if dtype == torch.float32 else 1e-3) and _rel(out[1][1], out[0][1]) < 1e-6
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("Dv", [128, 64])
+@pytest.mark.parametrize("off,weight_off,out_off", [(0, 1, 0), (0, 0, 2), (4, 0, 0), (4, 1, 4), (1, 0, 0)])
+def test_channel_rows_and_weights_aligned_apart(off, weight_off, out_off, Dv, dtype, monkeypatch):
+    """Rows that lie on 16 bytes beside weights or outputs that do not lie on four elements, and rows the other way."""
+    from enterprise_inference_amd.ops import linear_scan as ls
+    monkeypatch.setattr(ls, "FORCE_CHUNKED", True)
+    lens, H, D, R = [130, 64, 200], 2, 64, 8
+    T, W, at = sum(lens), H * Dv, [0, H * D, 2 * H * D, 2 * H * D + H * Dv, 2 * H * (D + Dv)]
+    g = torch.Generator(device="cuda").manual_seed(Dv)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    rows, nw = rnd(T, at[-1] + R).to(dtype), (1 + 0.1 * rnd(W)).to(dtype)
+    spec = ls.ScanSpec(H, D, Dv, "channel", kscale=D ** -0.5, eps=1e-5, a2t=rnd(R, H * D), tau=8.0)
+    cu, pos, slots = (t.cuda() for t in _step(lens, [0, 5, 0], False))
+
+    def run(o, w, b):
+        x = torch.empty(T, rows.shape[1] + 2 * o, device="cuda", dtype=dtype)[:, o:o + rows.shape[1]].copy_(rows)
+        weight = torch.empty(W + w, device="cuda", dtype=dtype)[w:].copy_(nw)
+        out = torch.empty(T, W + b, device="cuda", dtype=dtype)[:, b:]
+        st = ls.ScanState.allocate(3, spec, "cuda")
+        st.S.fill_(0.3)
+        y = ls.linear_scan(x, at[0], at[1], at[2], at[3], spec, st, slots, cu, 3, pos, None, weight, out=out,
+                           plan=ls.chunk_plan(lens, "cuda"), lo_off=at[4])
+        return y, st.S
+
+    (y, S), (z, Z) = run(0, 0, 0), run(off, weight_off, out_off)
+    # the same fp32 sums, whichever way their factors came
+    assert _rel(z, y) < (1e-6 if dtype == torch.float32 else 1e-3) and _rel(Z, S) < 1e-6

@@ -97,9 +97,10 @@ EIA_DEV KeyTiles key_tiles(int q0, int queries, int qlen, int L, int causal, int
 // Where the keys of query blocks are cut: at most `per` tiles a part, `most` parts a block.  A wave's part of
 // O^T lies in o as its lanes hold it ([part][16 registers of four][64 lanes]), maxima and sums of its 32
 // queries in ml.
+// apart: the parts of a block do not stand together in the grid, whose slowest places they are.
 struct KeyParts {
   float* o; float2* ml;
-  int per, most;
+  int per, most, apart;
 };
 
 EIA_DEV int parts_of(int tiles, const KeyParts& cut) { return max(1, min((tiles + cut.per - 1) / cut.per, cut.most)); }
@@ -139,8 +140,8 @@ paged_prefill_fa_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __r
   const int r32 = lane & 31, h = lane >> 5;
   // grid (head groups, work items): the heads of one query block are dispatched together and
   // the work list is latest-block-first, so the dispatch order is longest-first over the
-  // whole grid (causal blocks grow with their position), not per head; parts of a block stay together
-  const int item = CUT ? blockIdx.z : blockIdx.y;
+  // whole grid (causal blocks grow with their position), not per head
+  const int item = CUT && !cut.apart ? blockIdx.z : blockIdx.y, part = cut.apart ? blockIdx.z : blockIdx.y;
   const int s = work[2 * item], q0 = work[2 * item + 1];
   constexpr int FQB = FROWS / HPW;
   const int G = Hq / Hkv, NHG = G / HPW;
@@ -174,7 +175,7 @@ paged_prefill_fa_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __r
   int ntile = (hi - lo + FKB - 1) / FKB, parts = 1;
   if constexpr (CUT) {
     parts = parts_of(ntile, cut);
-    const int part = blockIdx.y, each = (ntile + parts - 1) / parts;
+    const int each = (ntile + parts - 1) / parts;
     if (part >= parts) return;
     lo += FKB * each * part;
     ntile = min(each, ntile - each * part);
@@ -350,7 +351,7 @@ paged_prefill_fa_kernel(const bf16_t* __restrict__ q, long q_stride, bf16_t* __r
   const float lt = pair_sum(l_run);
   if (CUT && parts > 1) {
     if (!wave_live) return;
-    const long at = (((long)item * cut.most + blockIdx.y) * gridDim.x + blockIdx.x) * (FTHREADS / 64) + w;
+    const long at = (((long)item * cut.most + part) * gridDim.x + blockIdx.x) * (FTHREADS / 64) + w;
     f32x4* po = reinterpret_cast<f32x4*>(cut.o) + at * (FD / 8 * 64) + lane;
 #pragma unroll
     for (int dt = 0; dt < FD / 32; ++dt)
@@ -442,16 +443,22 @@ EIA_API int eia_paged_prefill_fa(const void* q, long q_stride, void* out, long o
   if (D != FD || bs % FKB != 0 || out_stride % 8 != 0) return EIA_UNSUPPORTED;   // (16-B output stores)
   if (n_work == 0) return EIA_OK;
   const int G = Hq / Hkv, hpw = G % 4 == 0 ? 4 : G % 2 == 0 ? 2 : 1;
-  if (parts > 1 && (per < 1 || !ws || n_work > 65535)) return EIA_BAD_SHAPE;
-  KeyParts cut{nullptr, nullptr, per, parts};
+  if (parts > 1 && (per < 1 || !ws || n_work > 65535 || parts > 65535)) return EIA_BAD_SHAPE;
+  // Workgroups go to XCDs, and to the parts of one, in turn.  Where an even number of parts stand together, the first parts
+  // of all blocks, of which there are most, meet in some places, and launches of several rounds wait for those: 1350
+  // launches of 4 to 256 blocks, in all numbers of parts, apart against together beyond 256 parts: even numbers 0.88 to
+  // 0.97 of the time, odd ones 0.98.  16 heads on 4, 3754 tokens 118 -> 95 us, two of 1639 55.7 -> 47.7; 28 on 4, two of 766
+  // 37.6 -> 35.5.  In one round those that stand together read fewer keys on an XCD: 4 on 1, 2023 tokens 27.9 -> 24.9.
+  const int groups = Hq / hpw;
+  KeyParts cut{nullptr, nullptr, per, parts, parts > 1 && (long)n_work * groups * parts > 256};
   if (parts > 1) {
     cut.o = ws;
-    cut.ml = reinterpret_cast<float2*>(ws + (long)n_work * parts * (Hq / hpw) * FROWS * FD);
+    cut.ml = reinterpret_cast<float2*>(ws + (long)n_work * parts * groups * FROWS * FD);
   }
 #define FA_GO(HPW)                                                                                  \
   do {                                                                                              \
     const float sl = scale * 1.4426950408889634f;                                                   \
-    const dim3 grid = parts > 1 ? dim3(Hq / HPW, parts, n_work) : dim3(Hq / HPW, n_work);           \
+    const dim3 grid = cut.apart ? dim3(groups, n_work, parts) : parts > 1 ? dim3(groups, parts, n_work) : dim3(groups, n_work);   \
     auto* f = parts > 1 ? paged_prefill_fa_kernel<HPW, true> : paged_prefill_fa_kernel<HPW, false>; \
     hipLaunchKernelGGL(f, grid, dim3(FTHREADS), 0, st, (const bf16_t*)q, q_stride, (bf16_t*)out,    \
                        out_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables,    \

@@ -86,3 +86,14 @@ def test_flash_prefill_parts(Hq, Hkv, qlens, ctxs, causal, window, chunk, parts,
     # weights and outputs rounded to bf16 (2^-9 each, relative), fp32 sums
     err = (o.double().cpu() - r.double()).norm() / r.double().norm()
     assert err < 4e-3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Hq,Hkv,qlens,ctxs", [(24, 8, [300, 40], [0, 500]), (16, 4, [640, 90], [300, 5]), (4, 1, [1500], [100])])
+@pytest.mark.parametrize("parts,per", [(12, 1), (15, 1)])
+def test_flash_prefill_parts_of_several_rounds(Hq, Hkv, qlens, ctxs, parts, per, monkeypatch):
+    """More than 256 parts: those of a block do not stand together in the grid."""
+    from enterprise_inference_amd.ops import attention as a
+    blocks = sum(-(-n // a.prefill_query_block(Hq, Hkv, 128, block_size=128)) for n in qlens)
+    assert blocks * (Hq // a.heads_per_workgroup(Hq, Hkv)) * parts > 256
+    test_flash_prefill_parts(Hq, Hkv, qlens, ctxs, True, None, None, parts, per, monkeypatch)

@@ -153,14 +153,15 @@ def fa_parts(wgs: int, tiles: int, mean: float, tile_us: float = 1.65, merge_us:
     (of the whole chip).  Parts run in one round (232 of them: not every XCD gets the same number), or in two where short
     ones fill the gaps.  1024 are at most 136 MB.  More workgroups than run at a time even themselves out.
 
-    MI355X, workgroups of up to so many tiles, mean: tiles per part: us.  Heads 32 on 8: 16 of 12, 11: uncut 24.8, 6:
-    19.7, 3: 15.6, 2: 15.4, 1: 17.8; 16 of 34, 33: 58.6, 9: 25.4, 4: 20.9, 3: 21.3; 64 of 8, 4: 19.4, 3: 17.8, 1: 26.3;
-    64 of 258, 254: 425, 129: 224, 65: 138, 52: 197; 104 of 28, 27: 51.4, 14: 38.9, 12: 47.3, 5: 56.8; 128 of 6, 4: 15.6, 3:
-    17.7; 128 of 16, 8: 34.4, 9: 29.2, 7: 27.3, 5: 37.2, 2: 45; 128 of 48, 40: 85.4, 36: 75.4, 24: 59.1, 16: 67.8; 192 of
-    24, 12: 47.4, 12: 44.6, 6: 56.5; 256 of 32, 16: 61.1, 16: 63.5, 11: 61.1, 8: 82.5; 504 of 64, 33: 155, 32: 179.
-    16 on 4: 32 of 24, 20: 45.2, 5: 23.2, 2: 31.1; 52 of 26, 25: 48.1, 7: 27.8, 6: 34; 128 of 32, 16: 58.2, 13: 38.6, 8: 47.7;
-    236 of 24, 14: 47, 16: 50; 252 of 64, 33: 116, 34: 108, 22: 97, 16: 124.  28 on 4: 112 of 22, 16: 46.2, 11: 36.3, 8: 41;
-    168 of 48, 36: 98, 24: 90, 16: 92, 15: 107; 224 of 30, 27: 66.2, 15: 81.7."""
+    MI355X, workgroups of up to so many tiles, mean: tiles per part: us.  Heads 32 on 8: 16 of 12, 12: uncut 24.7, 6:
+    18.3, 3: 14.6, 2: 14.4, 1: 17.6; 24 of 34, 33: 59, 17: 36, 9: 25.2, 5: 21.3, 3: 27.1; 120 of 16, 9: 30.6, 9: 26.7, 6:
+    24.3, 3: 34.2; 128 of 18, 10: 35.4, 12: 31.9, 8: 27.6, 6: 36.4; 128 of 78, 70: 131, 39: 88.4, 26: 107, 20: 95.3; 200 of
+    26, 14: 45.5, 22: 46.3, 15: 39, 8: 49.2; 240 of 32, 17: 57.2, 24: 53.2, 16: 56.6, 8: 68.2.
+    16 on 4: 52 of 28, 26: 48.4, 14: 33, 7: 26.5, 5: 33; 120 of 32, 17: 57.3, 24: 50.4, 13: 35.8, 11: 34.1, 8: 45.5; 164 of
+    44, 24: 76.8, 26: 57.5, 22: 52.8, 12: 62.9; 208 of 52, 26: 88.9, 30: 67.9, 18: 77.5, 14: 78.8; 208 of 54, 48: 95.3, 27: 104.
+    28 on 4: 112 of 16, 9: 33.8, 12: 34, 6: 26.1, 4: 34.4; 168 of 40, 29: 77.9, 19: 67.4, 14: 66.3, 10: 74.7.  24 on 8: 192 of
+    36, 21: 71.5, 22: 70.7, 14: 65.2, 8: 75.4; 192 of 36, 36: 55.5, 18: 66.1.  8 on 2: 104 of 26, 13: 47.2, 16: 38.3, 8: 29.5, 6:
+    38.7.  4 on 1: 56 of 8, 5: 16.3, 4: 17.6, 3: 18.1."""
     if wgs < 1 or wgs > FA_SLOTS or tile_us * tiles < 9:
         return 1, tiles
     work = wgs * max(1.0, mean)
@@ -185,7 +186,10 @@ def fa_parts(wgs: int, tiles: int, mean: float, tile_us: float = 1.65, merge_us:
         two = cost(half, 2.3)
         if two < took:
             per, took = half, two
-    return (-(-tiles // per), per) if took < tile_us * tiles else (1, tiles)
+    # of 1350 launches of 1 to 256 workgroups, uneven ones that seem to save less than 8 % or 2 us lost as often as they won, by
+    # up to 16 %; with this line 1 lost (24 heads on 8, 47 tokens behind 362: 13.6 -> 14.2), all together 0.81 of the time
+    uncut = tile_us * tiles
+    return (-(-tiles // per), per) if took < (uncut if even else min(0.92 * uncut, uncut - 2)) else (1, tiles)
 
 
 def decode_partitions(batch: int, num_kv_heads: int, num_heads: int, max_len: int,

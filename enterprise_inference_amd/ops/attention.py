@@ -146,12 +146,13 @@ FA_SLOTS = 256        # workgroups of the flash form that run at a time: one a C
 
 @functools.lru_cache(maxsize=1024)            # (numbers to numbers; a step's layers ask the same)
 def fa_parts(wgs: int, tiles: int, mean: float, tile_us: float = 1.65, merge_us: float = 4.0,
-             rows_us: float = 1 / 28, rounds: int = 2):
+             rows_us: float = 1 / 28, rounds: int = 2, fit: int = 232):
     """(parts, tiles per part) of a launch of the flash form: ``wgs`` workgroups that walk up to ``tiles``
     and on average ``mean`` key tiles, of lengths spread evenly about the mean.  A tile takes ``tile_us`` (with fewer
     than four heads a workgroup 1.95), the merge's launch ``merge_us`` and a part's rows, written and read, ``rows_us``
-    (of the whole chip).  Parts run in one round (232 of them: not every XCD gets the same number), or in two where short
-    ones fill the gaps.  1024 are at most 136 MB.  More workgroups than run at a time even themselves out.
+    (of the whole chip).  Parts run in one round (``fit`` of them where they are uneven: not every XCD gets the same number),
+    or, ``rounds`` 2, in two where short ones fill the gaps.  1024 are at most 136 MB.  More workgroups than run at a time
+    even themselves out.
 
     MI355X, workgroups of up to so many tiles, mean: tiles per part: us.  Heads 32 on 8: 16 of 12, 12: uncut 24.7, 6:
     18.3, 3: 14.6, 2: 14.4, 1: 17.6; 24 of 34, 33: 59, 17: 36, 9: 25.2, 5: 21.3, 3: 27.1; 120 of 16, 9: 30.6, 9: 26.7, 6:
@@ -171,7 +172,7 @@ def fa_parts(wgs: int, tiles: int, mean: float, tile_us: float = 1.65, merge_us:
     if even:
         per = -(-tiles // (FA_SLOTS // wgs))
     else:
-        share = 232 / wgs - 0.5
+        share = fit / wgs - 0.5
         per = math.ceil(mean / share) if share > 0 else tiles
     per = min(tiles, max(per, least, math.ceil(math.sqrt(1.28 * work * rows_us / tile_us))))
     shortest = max(0.0, 2 * mean - tiles)
@@ -189,7 +190,7 @@ def fa_parts(wgs: int, tiles: int, mean: float, tile_us: float = 1.65, merge_us:
     # of 1350 launches of 1 to 256 workgroups, uneven ones that seem to save less than 8 % or 2 us lost as often as they won, by
     # up to 16 %; with this line 1 lost (24 heads on 8, 47 tokens behind 362: 13.6 -> 14.2), all together 0.81 of the time
     uncut = tile_us * tiles
-    return (-(-tiles // per), per) if took < (uncut if even else min(0.92 * uncut, uncut - 2)) else (1, tiles)
+    return (-(-tiles // per), per) if took < (uncut if even and rounds == 2 else min(0.92 * uncut, uncut - 2)) else (1, tiles)
 
 
 def decode_partitions(batch: int, num_kv_heads: int, num_heads: int, max_len: int,

@@ -191,7 +191,11 @@ def flash_parts(wgs: int, lens, context: int, tiles: int, KT: int, window: int, 
                         512 if two else 256, 12 * 64 // KT, 11 if two else 3 * 64 // KT)
     if wgs <= 64 or (P == 1 and not two):
         mean = (context - max(lens) + sum(n * n for n in lens) / (2 * max(1, sum(lens)))) / KT
-        P, per = fa_parts(wgs, tiles, min(mean, tiles), 1.85 if two else 3.6, 6.5, 0.02, 1)
+        # the parts of a workgroup run on its XCD, 32 of wide rows at a time
+        cut = (fa_parts(wgs, tiles, min(mean, tiles), 1.85, 6.5, 0.02, 1) if two else
+               fa_parts(-(-wgs // 8) * 8, tiles, min(mean, tiles), 3.6, 6.5, 0.02, 1, 220))
+        if cut[0] > 1 or not wgs:
+            return cut
     return P, per
 
 

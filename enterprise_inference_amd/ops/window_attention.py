@@ -171,7 +171,9 @@ def flash_parts(n_items: int, spec: WindowSpec, queries: int, longest: int, cont
     wgs = n_items * (spec.heads * queries // 128)
     if wgs <= 64:
         mean = tiles if spec.window > 0 else tiles - longest / 128
-        return fa_parts(wgs, tiles, mean, 1.1 if narrow else 1.6, 4.5, 0.015, 1)
+        parts, per = fa_parts(wgs, tiles, mean, 1.1 if narrow else 1.6, 4.5, 0.015, 1)
+        if parts > 1 or not wgs:
+            return parts, per
     return split_keys(wgs, tiles,
                       tiles if spec.window > 0 else tiles - longest // 128, (3 if narrow else 2) * cus,
                       merge=7 if narrow else 6)

@@ -50,6 +50,28 @@ def test_a_cut_is_not_slower(launch, us):
     assert parts > 1 or min(us.values()) > 0.85 * us[0]
 
 
+# times in us by tiles per part, as measured, and the one that split_keys' rule took
+@pytest.mark.parametrize("wgs,lens,context,tiles,KT,window,us,most", [
+    (55, [871], 896, 14, 64, 1024, {2: 50.6, 3: 35.6, 4: 36.8, 6: 43.9, 14: 65.8}, 43.9),
+    (56, [891], 896, 14, 64, 0, {2: 51.7, 3: 35.6, 4: 36.9, 6: 42.6, 14: 66.1}, 42.6),
+    (26, [108, 90, 80, 100], 1472, 18, 64, 1024, {2: 54.3, 3: 34.5, 4: 36.7, 6: 42.0}, 42.0),
+    (128, [261, 230, 190, 180, 140], 384, 6, 64, 1024, {2: 27.8, 3: 29.5, 6: 27.3}, 27.3),
+    (41, [162], 768, 24, 32, 0, {4: 61.9, 5: 41.0, 6: 42.0, 12: 58.6}, 58.6)])
+def test_latent_cuts_are_not_slower(wgs, lens, context, tiles, KT, window, us, most):
+    """The parts of a workgroup run on one XCD: 26 of nine parts are 36 on some, which run 32 at a time."""
+    from enterprise_inference_amd.ops.latent_attention import flash_parts
+    assert us[flash_parts(wgs, lens, context, tiles, KT, window, False)[1]] <= most
+
+
+def test_short_window_launches_are_not_cut():
+    """Up to 6 tiles, us uncut and in parts of two: 14.0 / 15.9, 16.5 / 18.0, 16.1 / 17.0."""
+    from enterprise_inference_amd.ops import window_attention as wa
+    spec = lambda heads, kv, maps, dim, vdim, window: wa.WindowSpec(heads, kv, maps, dim, vdim, window, 0, None)
+    assert wa.flash_parts(11, spec(16, 4, 1, 96, 96, 0), 32, 328, 384) == (1, 6)
+    assert wa.pair_parts(16, spec(8, 2, 2, 64, 128, 1024), 32, 384) == (1, 6)
+    assert wa.flash_parts(16, spec(8, 2, 1, 128, 128, 1024), 32, 260, 384) == (1, 6)
+
+
 def test_launches_without_work_are_not_cut():
     from enterprise_inference_amd.ops import latent_attention as la
     from enterprise_inference_amd.ops import window_attention as wa

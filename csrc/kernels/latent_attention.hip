@@ -432,7 +432,10 @@ latent_decode_kernel(LatentAttnArgs a) {
     }
   };
   look(k_begin);
-  // what the queries are formed from is asked for before the first rows, of whose arrival nothing then waits
+  // What the queries are formed from is asked for before the first rows, of whose arrival nothing then waits, where a
+  // workgroup has a CU to itself.  Others wait less for their rows than they lose to the longer start: 57 rows of 64
+  // heads, 256 + 32, window 1024 31.5 -> 32.6 us, of 32 heads, 128 + 32 17.6 -> 19.1.
+  constexpr bool AHEAD = NW == 8;
   const int hp = a.rot_dims >> 1, npass = a.rd - a.rot_dims;
   const bf16_t* qrb = static_cast<const bf16_t*>(a.qr) + (long)row * a.qr_st + (long)h0 * a.qr_sh;
   auto pair = [&](int e, int& m, int& ia, int& ib) {    // pair e of the rotary parts: head, places
@@ -442,56 +445,58 @@ latent_decode_kernel(LatentAttnArgs a) {
     ib = a.rot_half ? i + hp : 2 * i + 1;
     return i;
   };
-  const float turn = tid < hp ? a.inv_freq[tid] : 0.f;
+  float turn = 0.f;
   unsigned pu = 0, pv = 0;                              // (as they lie in memory: a conversion here would wait for them)
-  if (tid < nh * hp) {
-    int m, ia, ib;
-    pair(tid, m, ia, ib);
-    const unsigned short* src = reinterpret_cast<const unsigned short*>(qrb) + (long)m * a.qr_sh;
-    pu = src[ia];
-    pv = src[ib];
+  if constexpr (AHEAD) {
+    turn = tid < hp ? a.inv_freq[tid] : 0.f;
+    if (tid < nh * hp) {
+      int m, ia, ib;
+      pair(tid, m, ia, ib);
+      const unsigned short* src = reinterpret_cast<const unsigned short*>(qrb) + (long)m * a.qr_sh;
+      pu = src[ia];
+      pv = src[ib];
+    }
   }
   const bool ok = l16 < nh;                             // this lane's head
   const int h = h0 + (ok ? l16 : 0);
   const int kg = w & 3, s0 = NS * (w >> 2);             // the wave's keys of a tile, and steps of their rows
   bf16x8 qf[NS];
-  {
-    // R % 8 == 0 and rd % 8 == 0: a lane's eight entries lie wholly in one of the two parts
-    const bf16_t* qa = static_cast<const bf16_t*>(a.qa) + (long)row * a.qa_st + (long)h * a.qa_sh;
-    if (((reinterpret_cast<uintptr_t>(a.qa) | (uintptr_t)(a.qa_st * 2) | (uintptr_t)(a.qa_sh * 2)) & 15) == 0) {
+  // R % 8 == 0 and rd % 8 == 0: a lane's eight entries lie wholly in one of the two parts
+  const bf16_t* qa = static_cast<const bf16_t*>(a.qa) + (long)row * a.qa_st + (long)h * a.qa_sh;
+  const bool vec = ((reinterpret_cast<uintptr_t>(a.qa) | (uintptr_t)(a.qa_st * 2) | (uintptr_t)(a.qa_sh * 2)) & 15) == 0;
+  auto query = [&](int d) {
+    if (vec) return *reinterpret_cast<const bf16x8*>(qa + d);
+    bf16x8 v;
 #pragma unroll
-      for (int s = 0; s < NS; ++s) {
-        const int d = 32 * (s0 + s) + 8 * g4;
-        qf[s] = *reinterpret_cast<const bf16x8*>(qa + (d < R ? d : 0));
-      }
-    } else {
+    for (int e = 0; e < 8; ++e) v[e] = qa[d + e];
+    return v;
+  };
+  if constexpr (AHEAD) {
 #pragma unroll
-      for (int s = 0; s < NS; ++s) {
-        const int d = 32 * (s0 + s) + 8 * g4;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) qf[s][e] = qa[(d < R ? d : 0) + e];
-      }
+    for (int s = 0; s < NS; ++s) {
+      const int d = 32 * (s0 + s) + 8 * g4;
+      qf[s] = query(d < R ? d : 0);
     }
+    __builtin_amdgcn_sched_barrier(0);
   }
-  __builtin_amdgcn_sched_barrier(0);
   fetch(k_begin);
   look(k_begin + KT);
 
   // the rotary query parts, rotated once into LDS: the heads of a row turn by the same angles
   for (int i = tid; i < hp; i += NT) {
     float sn, cs;
-    sincosf((float)qpos * (i == tid ? turn : a.inv_freq[i]), &sn, &cs);
+    sincosf((float)qpos * (AHEAD && i == tid ? turn : a.inv_freq[i]), &sn, &cs);
     rot[i] = make_float2(cs * a.rot_amp, sn * a.rot_amp);
   }
   __syncthreads();
   bf16_t* qrs = tiles;                                  // [16][rd]
-  asm volatile("" : "+v"(pu), "+v"(pv));
+  if constexpr (AHEAD) asm volatile("" : "+v"(pu), "+v"(pv));
   for (int e = tid; e < nh * hp; e += NT) {
     int m, ia, ib;
     const int i = pair(e, m, ia, ib);
     const bf16_t* src = qrb + (long)m * a.qr_sh;
-    const float u = e == tid ? __uint_as_float(pu << 16) : bf2f(src[ia]);
-    const float v = e == tid ? __uint_as_float(pv << 16) : bf2f(src[ib]);
+    const float u = AHEAD && e == tid ? __uint_as_float(pu << 16) : bf2f(src[ia]);
+    const float v = AHEAD && e == tid ? __uint_as_float(pv << 16) : bf2f(src[ib]);
     const float2 cs = rot[i];
     qrs[m * a.rd + ia] = f2bf(u * cs.x - v * cs.y);
     qrs[m * a.rd + ib] = f2bf(v * cs.x + u * cs.y);
@@ -504,8 +509,16 @@ latent_decode_kernel(LatentAttnArgs a) {
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
     const int d = 32 * (s0 + s) + 8 * g4;
-    if (!ok || d >= Dk) qf[s] = zero8;
-    else if (d >= R) qf[s] = *reinterpret_cast<const bf16x8*>(qrs + l16 * a.rd + (d - R));
+    if constexpr (AHEAD) {
+      if (!ok || d >= Dk) qf[s] = zero8;
+      else if (d >= R) qf[s] = *reinterpret_cast<const bf16x8*>(qrs + l16 * a.rd + (d - R));
+    } else {
+      bf16x8 v = zero8;
+      if (ok && d < Dk) {
+        v = d >= R ? *reinterpret_cast<const bf16x8*>(qrs + l16 * a.rd + (d - R)) : query(d);
+      }
+      qf[s] = v;
+    }
   }
   __syncthreads();                                      // the rotary parts make room for tiles
   stash(0, k_begin);

@@ -364,7 +364,7 @@ def paged_prefill(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
             tiles = block_tables.shape[1] * bs / 64          # (of the longest sequence)
             mean = tiles - T / (128 * (cu_q.numel() - 1)) if causal else tiles
             span = sliding_window or chunk_size
-            if span:
+            if span and causal:                              # (else keys behind the queries are walked too)
                 tiles = min(tiles, (span + rows) / 64 + 1)
             parts, per = fa_parts(wgs, math.ceil(tiles), min(mean, tiles), 1.65 if hpw == 4 else 1.95)
             if parts > 1:

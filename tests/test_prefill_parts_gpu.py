@@ -122,9 +122,11 @@ def test_flash_prefill_parts(Hq, Hkv, qlens, ctxs, causal, window, chunk, parts,
                                     window, chunk)
     work = torch.tensor(attention.build_prefill_work(
         qlens, attention.prefill_query_block(Hq, Hkv, D, block_size=bs)), dtype=torch.int32)
-    monkeypatch.setattr(attention, "fa_parts", lambda *a: (parts, per))
+    asked = []
+    monkeypatch.setattr(attention, "fa_parts", lambda *a: asked.append(a) or (parts, per))
     d = [t.cuda() for t in (q, k, v, bt, sl, cu, work)]
     o = attention.paged_prefill(*d[:6], d[6], work.numel() // 2, D ** -0.5, causal, window, chunk)
+    assert asked                                           # (it was cut)
     # weights and outputs rounded to bf16 (2^-9 each, relative), fp32 sums
     err = (o.double().cpu() - r.double()).norm() / r.double().norm()
     assert err < 4e-3
@@ -139,3 +141,18 @@ def test_flash_prefill_parts_of_several_rounds(Hq, Hkv, qlens, ctxs, parts, per,
     blocks = sum(-(-n // a.prefill_query_block(Hq, Hkv, 128, block_size=128)) for n in qlens)
     assert blocks * (Hq // a.heads_per_workgroup(Hq, Hkv)) * parts > 256
     test_flash_prefill_parts(Hq, Hkv, qlens, ctxs, True, None, None, parts, per, monkeypatch)
+
+
+@pytest.mark.gpu
+def test_flash_prefill_counts_the_keys_behind_a_query(monkeypatch):
+    """Without a causal mask a window does not bound what a block walks."""
+    from enterprise_inference_amd.ops import attention
+    asked = []
+    monkeypatch.setattr(attention, "fa_parts", lambda *a: asked.append(a) or (1, a[1]))
+    i32 = lambda *v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    q = torch.zeros(64, 8, 128, dtype=BF, device="cuda")
+    k, v = torch.zeros(16, 2, 128, 128, dtype=BF, device="cuda"), torch.zeros(16, 2, 128, 128, dtype=BF, device="cuda")
+    bt = torch.arange(16, dtype=torch.int32, device="cuda")[None]
+    for causal, tiles in ((True, 6), (False, 32)):
+        attention.paged_prefill(q, k, v, bt, i32(2048), i32(0, 64), i32(0, 0), 1, 0.1, causal, 200)
+        assert asked[-1][1] == tiles

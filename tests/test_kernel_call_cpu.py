@@ -77,12 +77,12 @@ def test_what_is_not_plain(echo):
             _native.runtime().KernelCall(*bad)
 
 
-@pytest.mark.parametrize("sizes", [(1,), (0, 4, 0, 513), (512, 511, 1), (4096, 0)])
+@pytest.mark.parametrize("sizes", [(1,), (0, 4, 0, 513), (512, 511, 1), (4096, 0), (4, 1 << 21, 5, (1 << 21) + 1, 7)])
 def test_workspace_places(sizes):
-    """The places of one allocation lie apart, on 512-byte steps of it, inside it."""
+    """The places of one allocation lie apart, on 512-byte steps of it, large ones on 2 MiB steps, inside it."""
     from enterprise_inference_amd.ops._dispatch import workspace
     ws, at = workspace("cpu", *sizes)
     base = ws.data_ptr()
     for a, n, b in zip(at, sizes, at[1:] + [base + ws.numel()]):
-        assert (a - base) % 512 == 0 and a + n <= b
+        assert (a - base) % (512 if n < 1 << 21 else 1 << 21) == 0 and a + n <= b
     assert ws.numel() >= sum(sizes)

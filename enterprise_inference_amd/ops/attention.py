@@ -151,15 +151,16 @@ def fa_parts(wgs: int, tiles: int, mean: float, tile_us: float = 1.65, merge_us:
     and on average ``mean`` key tiles, of lengths spread evenly about the mean.  A tile takes ``tile_us`` (with fewer
     than four heads a workgroup 1.95), the merge's launch ``merge_us`` and a part's rows, written and read, ``rows_us``
     (of the whole chip).  Parts run in one round (``fit`` of them where they are uneven: not every XCD gets the same number),
-    or, ``rounds`` 2, in two where short ones fill the gaps.  1024 are at most 136 MB.  More workgroups than run at a time
+    or, ``rounds`` 2, are halves where short ones fill the gaps.  1024 are at most 136 MB.  More workgroups than run at a time
     even themselves out.
 
     MI355X, workgroups of up to so many tiles, mean: tiles per part: us.  Heads 32 on 8: 16 of 12, 12: uncut 24.7, 6:
     18.3, 3: 14.6, 2: 14.4, 1: 17.6; 24 of 34, 33: 59, 17: 36, 9: 25.2, 5: 21.3, 3: 27.1; 120 of 16, 9: 30.6, 9: 26.7, 6:
     24.3, 3: 34.2; 128 of 18, 10: 35.4, 12: 31.9, 8: 27.6, 6: 36.4; 128 of 78, 70: 131, 39: 88.4, 26: 107, 20: 95.3; 200 of
-    26, 14: 45.5, 22: 46.3, 15: 39, 8: 49.2; 240 of 32, 17: 57.2, 24: 53.2, 16: 56.6, 8: 68.2.
+    26, 14: 45.5, 22: 46.3, 13: 39.8, 8: 49.2; 240 of 32, 17: 57.2, 24: 53.2, 16: 56.6, 8: 68.2.
     16 on 4: 52 of 28, 26: 48.4, 14: 33, 7: 26.5, 5: 33; 120 of 32, 17: 57.3, 24: 50.4, 13: 35.8, 11: 34.1, 8: 45.5; 164 of
-    44, 24: 76.8, 26: 57.5, 22: 52.8, 12: 62.9; 208 of 52, 26: 88.9, 30: 67.9, 18: 77.5, 14: 78.8; 208 of 54, 48: 95.3, 27: 104.
+    44, 24: 76.8, 26: 57.5, 22: 52.8, 12: 62.9; 208 of 52, 26: 88.9, 26: 71.2, 18: 77.5, 14: 78.8; 236 of
+    60, 31: 104.5, 30: 87, 20: 91.6; 208 of 54, 48: 95.3, 27: 104.
     28 on 4: 112 of 16, 9: 33.8, 12: 34, 6: 26.1, 4: 34.4; 168 of 40, 29: 77.9, 19: 67.4, 14: 66.3, 10: 74.7.  24 on 8: 192 of
     36, 21: 71.5, 22: 70.7, 14: 65.2, 8: 75.4; 192 of 36, 36: 55.5, 18: 66.1.  8 on 2: 104 of 26, 13: 47.2, 16: 38.3, 8: 29.5, 6:
     38.7.  4 on 1: 56 of 8, 5: 16.3, 4: 17.6, 3: 18.1."""
@@ -177,20 +178,22 @@ def fa_parts(wgs: int, tiles: int, mean: float, tile_us: float = 1.65, merge_us:
     per = min(tiles, max(per, least, math.ceil(math.sqrt(1.28 * work * rows_us / tile_us))))
     shortest = max(0.0, 2 * mean - tiles)
 
-    def cost(per, factor=1.0):                               # (workgroups of up to ``per`` tiles stay whole)
-        whole = max(0.0, (per - shortest) / (tiles - shortest)) if per > shortest else 0.0
-        return factor * tile_us * per + merge_us + (work / per + wgs * (0.5 - whole)) * rows_us
+    uncut = tile_us * tiles
 
-    took = cost(per)
-    if rounds == 2 and not even:                                             # two rounds; 0.15: they do not meet everywhere
-        half = min(tiles, max(least, math.ceil(mean / (500 / wgs - 0.5))))
-        two = cost(half, 2.3)
-        if two < took:
-            per, took = half, two
+    def handed(per):                                         # the merge and its rows; up to ``per`` tiles stay whole
+        whole = max(0.0, (per - shortest) / (tiles - shortest)) if per > shortest else 0.0
+        return merge_us + (work / per + wgs * (0.5 - whole)) * rows_us
+
     # of 1350 launches of 1 to 256 workgroups, uneven ones that seem to save less than 8 % or 2 us lost as often as they won, by
     # up to 16 %; with this line 1 lost (24 heads on 8, 47 tokens behind 362: 13.6 -> 14.2), all together 0.81 of the time
-    uncut = tile_us * tiles
-    return (-(-tiles // per), per) if took < (uncut if even and rounds == 2 else min(0.92 * uncut, uncut - 2)) else (1, tiles)
+    took = tile_us * per + handed(per)
+    if took >= (uncut if even and rounds == 2 else min(0.92 * uncut, uncut - 2)):
+        per, took = tiles, uncut - 2
+    # halves, of which two thirds of one are left when the CUs run dry
+    half = -(-tiles // 2)
+    if rounds == 2 and not even and tile_us * (work / FA_SLOTS + 0.65 * half) + handed(half) < took:
+        per = half
+    return -(-tiles // per), per
 
 
 def decode_partitions(batch: int, num_kv_heads: int, num_heads: int, max_len: int,

@@ -23,7 +23,9 @@ inline int dn_parts(long nwg, int rep) {
   return parts;
 }
 // Beyond 512 the chunks that fill whole rounds of 512 keep a key head's heads together, and those of the last round are
-// spread as above: 66 chunks of 16 heads of 128 on 8, 528 workgroups, the solve 58.5 -> 51.5 us on an MI355X.
+// spread as above: 66 chunks of 16 heads of 128 on 8, 528 workgroups, the solve 58.5 -> 51.5 us on an MI355X.  The whole
+// op against one without the spread, 8, 16 and 32 heads: 8 to 104 workgroups in the last round 3 to 7 % faster, more of them
+// the same (1 %, as runs differ).
 struct DeltaSolve {
   int whole, parts;                                    // chunks whose heads stay together; parts of a key head of the others
   long blocks;                                         // workgroups

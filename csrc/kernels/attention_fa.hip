@@ -48,9 +48,9 @@
 //
 // Launches of fewer workgroups than CUs wait for their longest one (a tile of 64 keys takes 1.65 us): there blocks
 // are cut along the keys (CUT; attention.py fa_parts says where), parts hand over fp32 sums as their lanes hold
-// them, and a second kernel puts them together.  32 heads on 8, 100 tokens behind 2000: 59.5 -> 21 us, 1000 behind
-// 2000 85 -> 61, 1 x 1000 34 -> 28; 16 on 4, 500 behind 1000 45.5 -> 22.6, 1 x 4000 110 -> 97.5; error against 64
-// bits 2.35e-3 -> 2.29e-3.  Uncut launches run as before (1 x 8192 537, 4 x 300 15.7).
+// them, and a second kernel puts them together.  32 heads on 8, 100 tokens behind 2000: 58.9 -> 20.6 us, 1000 behind
+// 2000 80.8 -> 59.4, 1 x 1000 31.6 -> 25; 16 on 4, 500 behind 1000 44.1 -> 21.6, 1 x 4000 109 -> 94; error against 64
+// bits 2.35e-3 -> 2.29e-3.  Uncut launches run as before (1 x 8192 522, 4 x 300 14.6).
 #include "eia_common.h"
 
 namespace {

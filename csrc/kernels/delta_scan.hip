@@ -230,10 +230,10 @@ EIA_API int eia_delta_scan(const float* q, const float* k, const float* v, const
 //   X  [chunk, H, 4 token tiles, VP / 16 tiles]       fp32, B operand, rows tokens
 //   O  [chunk, 64, H, VP]                             fp32, outputs before their norm
 // with DP rounded up to 64 and VP to 32; tile j of 32 columns holds columns 2 x + j.
-// MI355X, 16 heads of 128 x 128 on 8, three prompts of 750 to 1500 tokens: 51 + 69 + 17 us
+// MI355X, 16 heads of 128 x 128 on 8, three prompts of 750 to 1500 tokens: 50 + 69 + 15 us
 // ((1), (2), (3)).  Before, with fp32 products and the states between chunks and u in memory for a kernel that formed
 // the outputs, 48 + 77 + 83 (the op: 197 -> 147).  S against 64 bits: 1.2e-7 .. 1.5e-7 where fp32 products left 1.3e-7 .. 1.6e-7.
-// (1) and (3) are bound by their writes and reads (3.0, 3.4 TB/s), (2) by the chain of its chunks: 6000 cycles
+// (1) and (3) are bound by their writes and reads (3.1, 4.4 TB/s), (2) by the chain of its chunks: 6000 cycles
 // each, of which matrix products take 2700 of a SIMD's.
 constexpr int DC = 64;                      // tokens per chunk
 constexpr int DL = DC + 4;                  // LDS row pitch of the triangular blocks

@@ -454,9 +454,9 @@ EIA_API int eia_linear_scan(const void* x, long ld, int q_off, int k_off, int v_
 // 128-token chunks: the states between chunks are the larger part of the memory
 // traffic (4 passes over chunks x H x dk x dv floats), and halving their number costs less than the
 // longer sums inside a chunk add.
-// Four prompts of 1000 .. 2000 tokens (6688 rows), 16 heads of 128, mode 1, bf16 take 35 + 21 +
-// 57 us on an MI355X ((1), (2), (3)); in fp32 products (1) and (3) took 57 + 103 us.  Bound by the
-// workspace and the rows, which (1), (2) and (3) move at 3.3, 5.4 and 3.4 TB/s, and by the steps of
+// Four prompts of 1000 .. 2000 tokens (6688 rows), 16 heads of 128, mode 1, bf16 take 34 + 21 +
+// 54 us on an MI355X ((1), (2), (3)); in fp32 products (1) and (3) took 57 + 103 us.  Bound by the
+// workspace and the rows, which (1), (2) and (3) move at 3.4, 5.5 and 3.6 TB/s, and by the steps of
 // a workgroup, which reads, splits and multiplies in turn: half of (3)'s wave cycles wait, and vector instructions
 // fill 0.4 of the others.  All heads of a chunk run side by side in (1) and (3), so
 // that whole rows are read together, and (3) asks for its queries before it waits for the gates: 135 -> 129 us for the
@@ -1904,8 +1904,8 @@ EIA_API int eia_linear_scan_channels(const void* x, long ld, int q_off, int k_of
 // cover; pairs of different 8-token blocks meet through the edges of the blocks between them, for those
 // inside a block see eia_chunks.h.  Products are fp32 matrix-core products.  Bound by instruction issue
 // (exponentials, operand rows through LDS), as there.
-// Four prompts of 490 to 977 tokens, 16 heads of 64 x 128, bf16: 21 + 22 + 11 + 48 us on an MI355X (l, (1),
-// (2), (3)); in the 32-token chunks of vector FMAs above 38 + 71 + 21 + 235 us, which remain for keys
+// Four prompts of 556 to 977 tokens, 16 heads of 64 x 128, bf16: 21 + 21 + 11 + 45 us on an MI355X (l, (1),
+// (2), (3)); in the 32-token chunks of vector FMAs above, of 490 to 977, 38 + 71 + 21 + 235 us, which remain for keys
 // wider than 64.
 constexpr int GC = 64;                      // tokens per chunk
 constexpr int GD = 64;                      // widest key head

@@ -241,8 +241,8 @@ EIA_API int eia_wkv_scan(const void* r, const void* k, const void* v, const void
 // instead of 1.2e-7 against 64 bits where every second token forgets, in the same time.)
 //
 // Bound by instruction issue (exponentials, conversions, fp32 products; 31 us of vector and 15 us of
-// matrix issue in (3)), not by memory: one 4096-token prompt, 32 heads of 64, bf16 takes 97 us on an
-// MI355X (25 + 16 + 60 in a trace), 2091 us token by token.  All that a workgroup reads is asked for before
+// matrix issue in (3)), not by memory: one 4096-token prompt, 32 heads of 64, bf16 takes 98 us on an
+// MI355X (25 + 17 + 62 in a trace), 2091 us token by token.  All that a workgroup reads is asked for before
 // it waits for any: with a row of r, u and half the decays behind branches and conversions, the state at
 // its products and a wait for each stored row 105 us (27 + 15 + 64).
 constexpr int WC = 64;                      // tokens per chunk

@@ -35,8 +35,8 @@ def ptr(t):
 
 
 def workspace(device, *sizes: int):
-    """One allocation of so many bytes each, at multiples of 512 bytes, large ones of 2 MiB as allocations of their own
-    would lie (expert layers of 2000 to 4000 rows without: 2 % slower) -> (the tensor that owns it, addresses).  An
+    """One allocation of so many bytes each, at multiples of 512 bytes from its start, large ones of 2 MiB (8 experts of
+    1024 x 512, 2000 rows 41.4 -> 40.4 us, other ops and sizes the same) -> (the tensor that owns it, addresses).  An
     allocation costs the host 1.3 us, and small steps are bound by their launches."""
     at, total = [], 0
     for n in sizes:
